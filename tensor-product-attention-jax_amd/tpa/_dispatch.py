@@ -7,6 +7,8 @@ through the C ABI.  There is no CPU fallback: a missing library raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -204,7 +206,10 @@ class TpaError(RuntimeError):
         self.code = code
 
 
+HOST_CALLS_PATH = os.path.join(os.path.dirname(_PKG_DIR), "lib", "tpa_host_calls.so")
+
 _lib = None
+_host = None
 _lib_lock = threading.Lock()
 
 
@@ -258,6 +263,25 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
         if path is None:
             _lib = lib
         return lib
+
+
+def host_calls():
+    """The module whose functions check an operator's operands, allocate its outputs and workspace and make the call
+    into the C ABI (csrc/host_calls.cc), loaded once and bound to the library of `load_library()`."""
+    global _host
+    if _host is not None:
+        return _host
+    load_library()
+    with _lib_lock:
+        if _host is None:
+            if not os.path.exists(HOST_CALLS_PATH):
+                raise RuntimeError(f"{HOST_CALLS_PATH} is not built: run `make -C {os.path.join(os.path.dirname(_PKG_DIR), 'csrc')}`")
+            loader = importlib.machinery.ExtensionFileLoader("tpa_host_calls", HOST_CALLS_PATH)
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("tpa_host_calls", loader))
+            loader.exec_module(module)
+            module.bind(LIB_PATH, TpaError)
+            _host = module
+    return _host
 
 
 def check(func: str, code: int) -> None:

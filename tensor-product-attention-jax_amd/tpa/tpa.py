@@ -130,6 +130,15 @@ def _lengths(kv_lengths, batch: int, device) -> torch.Tensor | None:
     return t
 
 
+def _call(native, arrays, *rest):
+    """One native call per operator (csrc/host_calls.cc); operands that are not GPU tensors yet are copied there first."""
+    out = native(*arrays, *rest)
+    if out is NotImplemented:
+        device = _pick_device(*arrays)
+        out = native(*(None if x is None else _as_device_tensor(x, device) for x in arrays), *rest)
+    return out
+
+
 def tpa_factors(
     qa, qb, ka, kb, va, vb,
     q_segment_ids=None,
@@ -162,64 +171,11 @@ def tpa_factors(
     """
     if use_workspace is None:
         use_workspace = USE_WORKSPACE
-    device = _pick_device(qa, qb, ka, kb, va, vb)
-    qa, qb, ka, kb, va, vb = (_as_device_tensor(x, device) for x in (qa, qb, ka, kb, va, vb))
-    dtype = qa.dtype
-    for name, t in (("qb", qb), ("ka", ka), ("kb", kb), ("va", va), ("vb", vb)):
-        if t.dtype != dtype:
-            raise TypeError(f"{name} has dtype {t.dtype}, expected {dtype}")
-    b, lq, rq, h = qa.shape
-    _, lk, rk, dv = vb.shape
-    dk = qb.shape[-1]
-    # shape rules of tpa/tpa.py:474-475: k and v share length and rank, q and k share h + dk
-    assert tuple(qb.shape) == (b, lq, rq, dk), qb.shape
-    assert tuple(ka.shape) == (b, lk, rk, h), ka.shape
-    assert tuple(kb.shape) == (b, lk, rk, dk), kb.shape
-    assert tuple(va.shape) == (b, lk, rk, h), va.shape
-    qseg = _segment_ids(q_segment_ids, b, lq, device)
-    kvseg = _segment_ids(kv_segment_ids, b, lk, device)
-    if (qseg is None) != (kvseg is None):
-        raise ValueError("q_segment_ids and kv_segment_ids must be given together")
-
-    kvlen = _lengths(kv_lengths, b, device)
-    o = torch.empty((b, lq, h, dv), dtype=dtype, device=device)
-    lse = torch.empty((b, h, lq), dtype=torch.float32, device=device) if return_lse else None
-    lib = _d.load_library()
-    # hand the library the workspace with which it can pick its fastest kernel (split partials for
-    # a decode through this entry point, dense Q, K and V for prefills that are long enough); it decides whether
-    # the problem qualifies
-    ws, ws_ptr, ws_bytes = None, None, 0
-    # (fp32 inputs: only the split-key decode kernel takes a workspace)
     nomat = NOMAT_RANK_PAIRS if nomat in ("pairs", NOMAT_RANK_PAIRS) and nomat is not True else int(bool(nomat))
-    if nomat == NOMAT_RANK_PAIRS:
-        pass  # one launch, no workspace
-    elif nomat:
-        # the split partials of the non-materialising kernels: required, not optional
-        need = lib.tpa_fwd_nomat_workspace_bytes(b, lq, lk, h, dk, dv, rq, rk) if kernel != _d.KERNEL_GENERIC else 0
-        if need:
-            ws = torch.empty(need + 256, dtype=torch.uint8, device=device)
-            pad = (-ws.data_ptr()) % 256
-            ws_ptr, ws_bytes = ws.data_ptr() + pad, need
-    elif use_workspace and kernel != _d.KERNEL_GENERIC and (dtype == torch.bfloat16 or lq <= 16):
-        need = lib.tpa_fwd_workspace_bytes(b, lq, lk, h, dk, dv, rq, rk)
-        if need:
-            ws = torch.empty(need + 256, dtype=torch.uint8, device=device)
-            pad = (-ws.data_ptr()) % 256
-            ws_ptr, ws_bytes = ws.data_ptr() + pad, need
-    args = _d.TpaFwdArgs(
-        qa=_d.factor(qa), qb=_d.factor(qb), ka=_d.factor(ka), kb=_d.factor(kb), va=_d.factor(va), vb=_d.factor(vb),
-        q_segment_ids=qseg.data_ptr() if qseg is not None else None,
-        kv_segment_ids=kvseg.data_ptr() if kvseg is not None else None,
-        o=o.data_ptr(), lse=lse.data_ptr() if lse is not None else None,
-        B=b, lq=lq, lk=lk, H=h, dk=dk, dv=dv, rq=rq, rk=rk,
-        dtype=_d.dtype_code(dtype), sm_scale=float(sm_scale), causal=_causal_code(causal), kernel=int(kernel),
-        workspace=ws_ptr, workspace_bytes=ws_bytes, num_splits=0,
-        kv_lengths=kvlen.data_ptr() if kvlen is not None else None,
-        causal_offset=int(causal_offset), nomat=nomat,
+    return _call(
+        _d.host_calls().factors, (qa, qb, ka, kb, va, vb, q_segment_ids, kv_segment_ids, kv_lengths),
+        sm_scale, _causal_code(causal), int(kernel), bool(return_lse), bool(use_workspace), int(causal_offset), nomat,
     )
-    with torch.cuda.device(device):
-        _d.check("tpa_fwd", lib.tpa_fwd(args, _d.current_stream_ptr(device)))
-    return o, lse
 
 
 def tpa_decode(
@@ -248,45 +204,10 @@ def tpa_decode(
     (causal_offset = lk - lq); segment ids are not taken here.
     Returns (o[b,lq,h,dv], lse[b,h,lq]).
     """
-    device = _pick_device(qa, qb, ka, kb, va, vb)
-    qa, qb, ka, kb, va, vb = (_as_device_tensor(x, device) for x in (qa, qb, ka, kb, va, vb))
-    dtype = qa.dtype
-    b, lq, rq, h = qa.shape
-    dk = qb.shape[-1]
-    pt, page_size, pages_per_seq = None, 0, 0
-    if page_table is None:
-        _, lk, rk, dv = vb.shape
-        assert tuple(kb.shape) == (b, lk, rk, dk), kb.shape
-        assert tuple(ka.shape) == (b, lk, rk, h) and tuple(va.shape) == (b, lk, rk, h)
-    else:
-        pt = _as_device_tensor(page_table, device).to(torch.int32).contiguous()
-        assert pt.dim() == 2 and pt.shape[0] == b, pt.shape
-        npages, page_size, rk, dv = vb.shape
-        pages_per_seq = pt.shape[1]
-        lk = pages_per_seq * page_size
-        assert tuple(kb.shape) == (npages, page_size, rk, dk), kb.shape
-        assert tuple(ka.shape) == (npages, page_size, rk, h) and tuple(va.shape) == (npages, page_size, rk, h)
-    kvlen = _lengths(kv_lengths, b, device)
-    lib = _d.load_library()
-    need = lib.tpa_decode_workspace_bytes(b, lq, lk, h, dv, num_splits)
-    if workspace is None:
-        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=device)
-    o = torch.empty((b, lq, h, dv), dtype=dtype, device=device)
-    lse = torch.empty((b, h, lq), dtype=torch.float32, device=device)
-    args = _d.TpaFwdArgs(
-        qa=_d.factor(qa), qb=_d.factor(qb), ka=_d.factor(ka), kb=_d.factor(kb), va=_d.factor(va), vb=_d.factor(vb),
-        q_segment_ids=None, kv_segment_ids=None, o=o.data_ptr(), lse=lse.data_ptr(),
-        B=b, lq=lq, lk=lk, H=h, dk=dk, dv=dv, rq=rq, rk=rk,
-        dtype=_d.dtype_code(dtype), sm_scale=float(sm_scale), causal=_causal_code(causal), kernel=int(kernel),
-        workspace=workspace.data_ptr(), workspace_bytes=workspace.numel() * workspace.element_size(),
-        num_splits=int(num_splits),
-        kv_lengths=kvlen.data_ptr() if kvlen is not None else None,
-        page_table=pt.data_ptr() if pt is not None else None, page_size=int(page_size), pages_per_seq=int(pages_per_seq),
-        causal_offset=int(causal_offset),
+    return _call(
+        _d.host_calls().decode, (qa, qb, ka, kb, va, vb, kv_lengths, page_table, workspace),
+        sm_scale, int(num_splits), int(kernel), _causal_code(causal), int(causal_offset),
     )
-    with torch.cuda.device(device):
-        _d.check("tpa_decode", lib.tpa_decode(args, _d.current_stream_ptr(device)))
-    return o, lse
 
 
 def tpa_cache_append(
@@ -313,62 +234,12 @@ def tpa_cache_append(
     `cache_append_workspace_bytes(...)`; a serving loop passes the same one every step) or, with
     `use_workspace` (default: the module's `USE_WORKSPACE`), one allocated here.
     Returns (qa[b, n, rq, h], qb[b, n, rq, d], new_kv_lengths[b])."""
-    device = _pick_device(x, w, ka, kb, va, vb)
-    x, w, ka, kb, va, vb = (_as_device_tensor(t, device) for t in (x, w, ka, kb, va, vb))
-    dtype = x.dtype
-    for name, t in (("w", w), ("ka", ka), ("kb", kb), ("va", va), ("vb", vb)):
-        if t.dtype != dtype:
-            raise TypeError(f"{name} has dtype {t.dtype}, expected {dtype}")
-    b, n, d_model = x.shape
-    rk, h = ka.shape[2], ka.shape[3]
-    d = kb.shape[3]
-    rq = int(rank_q)
-    assert tuple(w.shape) == (rq * (h + d) + 2 * rk * (h + d), d_model), w.shape
-    assert kb.shape[:3] == ka.shape[:3] and va.shape == ka.shape and vb.shape == kb.shape, (ka.shape, kb.shape, va.shape, vb.shape)
-    cos = _as_device_tensor(rope_cos, device).to(torch.float32).contiguous()
-    sin = _as_device_tensor(rope_sin, device).to(torch.float32).contiguous()
-    assert cos.shape == sin.shape and cos.dim() == 2 and cos.shape[1] == d // 2, (cos.shape, d)
-    pt, page_size, pages_per_seq = None, 0, 0
-    if page_table is None:
-        assert ka.shape[0] == b, ka.shape
-        cache_len = ka.shape[1]
-    else:
-        pt = _as_device_tensor(page_table, device).to(torch.int32).contiguous()
-        assert pt.dim() == 2 and pt.shape[0] == b, pt.shape
-        page_size, pages_per_seq = ka.shape[1], pt.shape[1]
-        cache_len = pages_per_seq * page_size
-    kvlen = _lengths(kv_lengths, b, device)
-    pos = None
-    if positions is not None:
-        pos = _as_device_tensor(positions, device).to(torch.int32).contiguous()
-        assert tuple(pos.shape) == (b, n), pos.shape
-    x, w = x.contiguous(), w.contiguous()
-    qa = torch.empty((b, n, rq, h), dtype=dtype, device=device)
-    qb = torch.empty((b, n, rq, d), dtype=dtype, device=device)
-    new_len = torch.empty((b,), dtype=torch.int32, device=device)
-    lib = _d.load_library()
-    ws_ptr, ws_bytes = None, 0
     if use_workspace is None:
         use_workspace = USE_WORKSPACE
-    if workspace is None and use_workspace and kernel != _d.KERNEL_GENERIC:
-        need = lib.tpa_cache_append_workspace_bytes(b, n, d_model, h, d, rq, rk, _d.dtype_code(dtype))
-        if need:
-            workspace = torch.empty(need + 16, dtype=torch.uint8, device=device)
-    if workspace is not None:
-        pad = (-workspace.data_ptr()) % 16
-        ws_ptr, ws_bytes = workspace.data_ptr() + pad, workspace.numel() * workspace.element_size() - pad
-    args = _d.TpaAppendArgs(
-        x=x.data_ptr(), w=w.data_ptr(), rope_cos=cos.data_ptr(), rope_sin=sin.data_ptr(),
-        positions=None if pos is None else pos.data_ptr(), kv_lengths=None if kvlen is None else kvlen.data_ptr(),
-        new_kv_lengths=new_len.data_ptr(),
-        qa=_d.factor(qa), qb=_d.factor(qb), ka=_d.factor(ka), kb=_d.factor(kb), va=_d.factor(va), vb=_d.factor(vb),
-        page_table=None if pt is None else pt.data_ptr(), page_size=int(page_size), pages_per_seq=int(pages_per_seq),
-        B=b, n=n, d_model=d_model, H=h, D=d, rq=rq, rk=rk, cache_len=int(cache_len), rope_len=int(cos.shape[0]),
-        dtype=_d.dtype_code(dtype), kernel=int(kernel), workspace=ws_ptr, workspace_bytes=ws_bytes,
+    return _call(
+        _d.host_calls().append, (x, w, rope_cos, rope_sin, ka, kb, va, vb, kv_lengths, positions, page_table, workspace),
+        int(rank_q), int(kernel), bool(use_workspace),
     )
-    with torch.cuda.device(device):
-        _d.check("tpa_cache_append", lib.tpa_cache_append(args, _d.current_stream_ptr(device)))
-    return qa, qb, new_len
 
 
 def cache_append_workspace_bytes(b: int, n: int, d_model: int, h: int, d: int, rq: int, rk: int, dtype=torch.bfloat16) -> int:
@@ -457,38 +328,12 @@ def bwd_workspace_bytes(b: int, lq: int, lk: int, h: int, dk: int, dv: int) -> i
     return int(_d.load_library().tpa_bwd_workspace_bytes(b, lq, lk, h, dk, dv))
 
 
-def _bwd_concat(q, k, v, qseg, kvseg, o, lse_bhl, do, num_heads, sm_scale, causal, causal_offset=0):
-    """Gradients in the concatenated layout of q, k, v (fp32), written in place by the kernels."""
-    h = num_heads
-    dq, dk, dv = (torch.empty(t.shape, dtype=torch.float32, device=t.device) for t in (q, k, v))
-    views = (dq[..., :h], dq[..., h:], dk[..., :h], dk[..., h:], dv[..., :h], dv[..., h:])
-    tpa_factors_bwd(
-        q[..., :h], q[..., h:], k[..., :h], k[..., h:], v[..., :h], v[..., h:],
-        qseg, kvseg, o, lse_bhl, do, sm_scale, causal, grads=views, causal_offset=causal_offset,
+def _operator(q, k, v, num_heads, q_segment_ids, kv_segment_ids, sm_scale, causal, nomat, interpret, causal_offset):
+    """(o, lse[b, h, lq]) with the vjp of tpa/tpa.py:217 (`Operator` in csrc/host_calls.cc) where an input asks for gradients."""
+    return _call(
+        _d.host_calls().tpa, (q, k, v, q_segment_ids, kv_segment_ids), int(num_heads), sm_scale, _causal_code(causal),
+        _d.KERNEL_GENERIC if interpret else _d.KERNEL_AUTO, USE_WORKSPACE, int(causal_offset), int(bool(nomat)),
     )
-    return dq, dk, dv
-
-
-class _TpaFunction(torch.autograd.Function):
-    """The operator with its vjp, as tpa.defvjp(_tpa_fwd, _tpa_bwd) registers it (tpa/tpa.py:217)."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, num_heads, qseg, kvseg, sm_scale, causal, kernel, causal_offset=0, nomat=False):
-        qa, qb = q[..., :num_heads], q[..., num_heads:]
-        ka, kb = k[..., :num_heads], k[..., num_heads:]
-        va, vb = v[..., :num_heads], v[..., num_heads:]
-        o, lse = tpa_factors(qa, qb, ka, kb, va, vb, qseg, kvseg, sm_scale, causal, kernel, causal_offset=causal_offset, nomat=nomat)
-        ctx.mark_non_differentiable(lse)
-        ctx.save_for_backward(q, k, v, o, lse)
-        ctx.statics = (num_heads, qseg, kvseg, sm_scale, causal, causal_offset)
-        return o, lse
-
-    @staticmethod
-    def backward(ctx, do, _dlse):
-        q, k, v, o, lse = ctx.saved_tensors
-        num_heads, qseg, kvseg, sm_scale, causal, causal_offset = ctx.statics
-        dq, dk, dv = _bwd_concat(q, k, v, qseg, kvseg, o, lse, do, num_heads, sm_scale, causal, causal_offset)
-        return dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), None, None, None, None, None, None, None, None
 
 
 def _tpa_fwd(
@@ -500,14 +345,7 @@ def _tpa_fwd(
     del block_sizes, debug
     device = _pick_device(q, k, v)
     q, k, v = (_as_device_tensor(x, device) for x in (q, k, v))
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-        raise ValueError("q, k, v must be [b, l, r, h + d]")
-    b, lq, rq, h_dk = q.shape
-    _, lk, rk, _ = v.shape  # rank and length of the keys are read from v (tpa/tpa.py:474)
-    assert tuple(k.shape) == (b, lk, rk, h_dk), k.shape  # tpa/tpa.py:475
-    assert 0 < num_heads < h_dk and num_heads < v.shape[-1], (num_heads, q.shape, v.shape)
-    kernel = _d.KERNEL_GENERIC if interpret else _d.KERNEL_AUTO
-    o, lse = _TpaFunction.apply(q, k, v, int(num_heads), q_segment_ids, kv_segment_ids, float(sm_scale), _causal_code(causal), kernel, int(causal_offset), bool(nomat))
+    o, lse = _operator(q, k, v, num_heads, q_segment_ids, kv_segment_ids, sm_scale, causal, nomat, interpret, causal_offset)
     l = lse.permute(0, 2, 1)
     return o, (q, k, v, q_segment_ids, kv_segment_ids, o, l)
 
@@ -533,11 +371,9 @@ def tpa(
     numpy result.  `causal_offset` (an addition, differentiable like the rest): with `causal`,
     query i sees keys up to i + causal_offset instead of i (see `tpa_factors`).
     """
+    del block_sizes, debug
     was_numpy = not isinstance(q, torch.Tensor)
-    o, _ = _tpa_fwd(
-        q, k, v, num_heads, q_segment_ids, kv_segment_ids, sm_scale, causal, block_sizes, nomat, debug, interpret,
-        causal_offset=causal_offset,
-    )
+    o, _ = _operator(q, k, v, num_heads, q_segment_ids, kv_segment_ids, sm_scale, causal, nomat, interpret, causal_offset)
     return o.cpu().numpy() if was_numpy and o.dtype != torch.bfloat16 else o
 
 
@@ -562,9 +398,11 @@ def _tpa_bwd(num_heads, sm_scale, causal, block_sizes, nomat, debug, interpret, 
     q, k, v, q_segment_ids, kv_segment_ids, o, l = residuals
     device = _pick_device(q, k, v)
     q, k, v, o, l, do = (_as_device_tensor(x, device) for x in (q, k, v, o, l, do))
-    dq, dk, dv = _bwd_concat(q, k, v, q_segment_ids, kv_segment_ids, o, l.permute(0, 2, 1), do, int(num_heads), float(sm_scale), _causal_code(causal),
-                             int(causal_offset))
-    return dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), None, None
+    dq, dk, dv = _call(
+        _d.host_calls().backward, (q, k, v, q_segment_ids, kv_segment_ids, o, l.permute(0, 2, 1), do), int(num_heads), sm_scale,
+        _causal_code(causal), int(causal_offset),
+    )
+    return dq, dk, dv, None, None
 
 
 def _bwd(
