@@ -161,9 +161,15 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dq_kernel(BwdF32Params p) {
   const int q0 = blk * kBlock, wrow0 = q0 + 32 * w, qrow = wrow0 + i, qrow_ld = min(qrow, p.lq - 1);
   const int64_t hd = (int64_t)p.H * D;
 
-  const int kend = p.causal ? max(1, min(p.lk, q0 + kBlock + p.coff)) : p.lk;  // at least one (then fully masked) tile
-  const int ntiles = (kend + kTile - 1) / kTile;
-  const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + p.coff + 31, 0) / kTile) : ntiles - 1;
+  int kend = p.causal ? max(1, min(p.lk, q0 + kBlock + p.coff)) : p.lk, kbeg = 0;  // at least one (then fully masked) tile
+  if constexpr (SEG) {  // only tiles that hold keys with ids of these rows
+    int first, last;
+    id_window<kThreads>(p.qseg + (int64_t)b * p.lq + q0, min(kBlock, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
+    kbeg = last < 0 ? 0 : first / kTile * kTile;
+    kend = last < 0 ? 1 : last + 1;
+  }
+  const int ntiles = (kend - kbeg + kTile - 1) / kTile;
+  const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + p.coff + 31 - kbeg, 0) / kTile) : ntiles - 1;
 
   float qf[D / 2], gf[D / 2];
   load_own_row<D>(p.q + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, p.sm_scale * kLog2e, false, qf);
@@ -186,10 +192,10 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dq_kernel(BwdF32Params p) {
   TileRegs<D> kreg, vreg;
   int32_t seg_reg = 0;
   auto issue = [&](int tile) __attribute__((always_inline)) {
-    kreg.issue(kbase, hd, tile * kTile, kend, false);
-    vreg.issue(vbase, hd, tile * kTile, kend, false);
+    kreg.issue(kbase, hd, kbeg + tile * kTile, kend, false);
+    vreg.issue(vbase, hd, kbeg + tile * kTile, kend, false);
     if constexpr (SEG)
-      if (tid < kTile) seg_reg = p.kvseg[(int64_t)b * p.lk + min(tile * kTile + tid, p.lk - 1)];
+      if (tid < kTile) seg_reg = p.kvseg[(int64_t)b * p.lk + min(kbeg + tile * kTile + tid, p.lk - 1)];
   };
   auto commit = [&](int tile) __attribute__((always_inline)) {
     kreg.store(lds_k + (tile & 1) * kMat);
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dq_kernel(BwdF32Params p) {
   auto compute = [&](int tile) __attribute__((always_inline)) {
     const float* const ks = lds_k + (tile & 1) * kMat;
     const float* const vs = lds_v + (tile & 1) * kMat;
-    const int k0 = tile * kTile;
+    const int k0 = kbeg + tile * kTile;
     f32x16 s[2], dp[2];
     rows_dot<D>(ks, i, g, qf, s[0], s[1]);    // x * log2(e)
     rows_dot<D>(vs, i, g, gf, dp[0], dp[1]);  // dP
@@ -256,8 +262,15 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dkv_kernel(BwdF32Params p) {
   const int64_t hd = (int64_t)p.H * D;
 
   // under the causal mask only rows at or after a key see it
-  const int first_tile = p.causal ? max(k0 - p.coff, 0) / kTile : 0;
-  const int ntiles = (p.lq + kTile - 1) / kTile;
+  int first_tile = p.causal ? max(k0 - p.coff, 0) / kTile : 0;
+  int ntiles = (p.lq + kTile - 1) / kTile;
+  if constexpr (SEG) {  // only tiles that hold rows with ids of these keys
+    int first, last;
+    const int rbeg = min(first_tile * kTile, p.lq);
+    id_window<kThreads>(p.kvseg + (int64_t)b * p.lk + k0, min(kBlock, p.lk - k0), p.qseg + (int64_t)b * p.lq + rbeg, p.lq - rbeg, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
+    ntiles = last < 0 ? 0 : (rbeg + last) / kTile + 1;
+    if (last >= 0) first_tile = (rbeg + first) / kTile;
+  }
   const int wave_first_tile = p.causal ? max(wkey0 - p.coff, 0) / kTile : 0;
 
   float kf[D / 2], vf[D / 2];
@@ -346,29 +359,311 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dkv_kernel(BwdF32Params p) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same two kernels for problems with few blocks of 128 rows (or keys), whose launch leaves most of the chip idle and
+// takes as long as one workgroup walking the whole sequence (2 sequences of 1000 tokens, 8 heads of 64: 128 workgroups,
+// 112 and 160 us).  A workgroup owns 32 rows (keys) and its four waves split the streamed tiles, 32 rows each: wave w
+// takes tiles w, w + 4, ... into LDS of its own (no barrier in the loop; the next tile's rows are in flight in registers
+// meanwhile, one matrix at a time), and the four partial sums are added through LDS in a fixed order.
+template <int D>
+struct SplitLds {
+  static constexpr int RS = D + 4;
+  static constexpr int kMat = 32 * RS;
+  static constexpr int kPerWave = 2 * kMat + 3 * 32;  // two matrices, then lse2 | delta | segment id of the tile's rows
+  static constexpr size_t kBytes = (size_t)kWaves * kPerWave * 4;
+};
+
+// 32 rows of dense X[b, row0 .., h, :] on their way to a wave's LDS; rows past the end read as zero
+template <int D>
+struct WaveTile {
+  static constexpr int CPR = D / 4, RPI = 64 / CPR, NST = 32 / RPI;
+  typedef f32x4 Regs[NST];
+  __amdgpu_buffer_rsrc_t rs;
+  int voff, row_bytes;
+  __device__ __forceinline__ void describe(const float* base, int64_t hd, int nrows, int l) {
+    rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)(((int64_t)(nrows - 1) * hd + D) * 4), 0x00020000);
+    voff = (int)(((l / CPR) * hd + 4 * (l % CPR)) * 4);
+    row_bytes = (int)(hd * 4);
+  }
+  __device__ __forceinline__ void issue(int row0, Regs& r) const {
+#pragma unroll
+    for (int q = 0; q < NST; ++q)
+      r[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, (row0 + q * RPI) * row_bytes, 0));
+  }
+  static __device__ __forceinline__ void store(const Regs& r, float* dst, int l, bool scrub_nan) {
+#pragma unroll
+    for (int q = 0; q < NST; ++q) {
+      f32x4 x = r[q];
+      if (scrub_nan) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = x[e] == x[e] ? x[e] : 0.f;
+      }
+      *reinterpret_cast<f32x4*>(dst + (q * RPI + l / CPR) * SplitLds<D>::RS + 4 * (l % CPR)) = x;
+    }
+  }
+};
+
+// a = A-tile rows . own row, b = B-tile rows . own row, both over d: two chains that alternate
+template <int D>
+__device__ __forceinline__ void rows_dot_pair(const float* ta, const float* tb, int i, int g, const float (&oa)[D / 2], const float (&ob)[D / 2], f32x16& a, f32x16& b) {
+  constexpr int RS = SplitLds<D>::RS;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) { a[v] = 0.f; b[v] = 0.f; }
+#pragma unroll
+  for (int m = 0; m < D / 8; ++m) {
+    const f32x4 fa = *reinterpret_cast<const f32x4*>(ta + i * RS + 8 * m + 4 * g);
+    const f32x4 fb = *reinterpret_cast<const f32x4*>(tb + i * RS + 8 * m + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      a = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], oa[4 * m + e], a, 0, 0, 0);
+      b = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[e], ob[4 * m + e], b, 0, 0, 0);
+    }
+  }
+}
+
+template <int D>
+__device__ __forceinline__ void cols_accumulate32(const float* tile, int i, int g, const f32x16& wgt, f32x16 (&out)[D / 32]) {
+  constexpr int RS = SplitLds<D>::RS, NDB = D / 32;
+  typedef __attribute__((ext_vector_type(NDB))) float f32xN;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const f32xN a = *reinterpret_cast<const f32xN*>(tile + (8 * (v >> 2) + 4 * g + (v & 3)) * RS + NDB * i);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) out[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[db], wgt[v], out[db], 0, 0, 0);
+  }
+}
+
+// a wave's accumulator as rows of 32 own rows x D in LDS
+template <int D>
+__device__ __forceinline__ void park(float* dst, int i, int g, const f32x16 (&acc)[D / 32]) { store_own_row<D>(dst + i * SplitLds<D>::RS, g, acc); }
+
+// dst[row0 + r, h, :] = sum over the waves of what they parked at `at`
+template <int D>
+__device__ __forceinline__ void add_waves(const float* at, float* dst, int row0, int nrows, int64_t hd, int tid) {
+  constexpr int CPR = D / 4;
+  for (int idx = tid; idx < 32 * CPR; idx += kThreads) {
+    const int r = idx / CPR, cc = idx % CPR;
+    if (row0 + r >= nrows) break;
+    f32x4 x = *reinterpret_cast<const f32x4*>(at + r * SplitLds<D>::RS + 4 * cc);
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) x += *reinterpret_cast<const f32x4*>(at + w * SplitLds<D>::kPerWave + r * SplitLds<D>::RS + 4 * cc);
+    *reinterpret_cast<f32x4*>(dst + (int64_t)(row0 + r) * hd + 4 * cc) = x;
+  }
+}
+
 template <int D, bool SEG>
-int launch_pair(const BwdF32Params& base, hipStream_t stream) {
-  static bool configured_q[kMaxDevices] = {}, configured_kv[kMaxDevices] = {};
-  const size_t smem = BwdLds<D>::kBytes;
-  {
-    BwdF32Params p = base;
-    p.nblk = (p.lq + kBlock - 1) / kBlock;
-    p.npairs = p.nblk * p.B;
-    auto kern = bwd_f32_dq_kernel<D, SEG>;
-    if (int rc = raise_lds_limit(configured_q, reinterpret_cast<const void*>(kern), smem); rc != TPA_OK) return rc;
-    hipLaunchKernelGGL(kern, dim3(((p.npairs + 7) / 8) * 8 * p.H), dim3(kThreads), smem, stream, p);
-    if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
+__global__ __launch_bounds__(kThreads, 1) void bwd_f32_dq_split_kernel(BwdF32Params p) {
+  constexpr int NDB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
+  int pair, h;
+  if (!decode_block(p.npairs, p.H, p.B, pair, h)) return;
+  const int blk = p.nblk - 1 - pair / p.B, b = pair % p.B;  // heaviest causal blocks first
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  const int q0 = blk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
+  const int64_t hd = (int64_t)p.H * D;
+  float* const lds_k = smem_bwd_f32 + w * SplitLds<D>::kPerWave;
+  float* const lds_v = lds_k + SplitLds<D>::kMat;
+  int32_t* const lds_seg = reinterpret_cast<int32_t*>(lds_v + SplitLds<D>::kMat);
+
+  int kbeg = 0, kend = p.causal ? max(0, min(p.lk, q0 + 32 + p.coff)) : p.lk;
+  int32_t qseg = 0;
+  if constexpr (SEG) {
+    qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
+    int first, last;
+    id_window<kThreads>(p.qseg + (int64_t)b * p.lq + q0, min(32, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
+    kbeg = last < 0 ? 0 : first / 32 * 32;
+    kend = last < 0 ? 0 : last + 1;
   }
-  {
-    BwdF32Params p = base;
-    p.nblk = (p.lk + kBlock - 1) / kBlock;
-    p.npairs = p.nblk * p.B;
-    auto kern = bwd_f32_dkv_kernel<D, SEG>;
-    if (int rc = raise_lds_limit(configured_kv, reinterpret_cast<const void*>(kern), smem); rc != TPA_OK) return rc;
-    hipLaunchKernelGGL(kern, dim3(((p.npairs + 7) / 8) * 8 * p.H), dim3(kThreads), smem, stream, p);
-    if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
+  const int ntiles = (max(0, kend - kbeg) + 31) / 32;
+  WaveTile<D> kt, vt;
+  kt.describe(p.k + (int64_t)b * p.lk * hd + (int64_t)h * D, hd, max(kend, 1), l);
+  vt.describe(p.v + (int64_t)b * p.lk * hd + (int64_t)h * D, hd, max(kend, 1), l);
+  // one matrix is in flight at a time: V's tile is free after the first two products, K's after the third
+  typename WaveTile<D>::Regs in;
+  int32_t seg_in = 0;
+  if (w < ntiles) vt.issue(kbeg + 32 * w, in);
+
+  float qf[D / 2], gf[D / 2];
+  load_own_row<D>(p.q + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, p.sm_scale * kLog2e, false, qf);
+  load_own_row<D>(p.d_o + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, 1.f, true, gf);
+  const float lse = p.lse[((int64_t)b * p.H + h) * p.lq + qrow_ld];
+  // a row without a visible key (lse = -inf) has no gradient: +inf makes every p of the row zero
+  const float lse2 = (qrow < p.lq && lse > -INFINITY) ? lse * kLog2e : INFINITY;
+  const float delta = p.delta[((int64_t)b * p.H + h) * p.lq + qrow_ld];
+  f32x16 dq[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) dq[db][v] = 0.f;
+
+  auto next_k = [&](int tile) __attribute__((always_inline)) {
+    WaveTile<D>::store(in, lds_v, l, false);
+    kt.issue(kbeg + 32 * tile, in);
+    if constexpr (SEG) seg_in = p.kvseg[(int64_t)b * p.lk + min(kbeg + 32 * tile + i, p.lk - 1)];
+  };
+  auto arrive_k = [&]() __attribute__((always_inline)) {
+    WaveTile<D>::store(in, lds_k, l, false);
+    if constexpr (SEG) lds_seg[i] = seg_in;
+  };
+  if (w < ntiles) {
+    next_k(w);
+    arrive_k();
   }
-  return TPA_OK;
+  for (int tile = w; tile < ntiles; tile += kWaves) {
+    const bool more = tile + kWaves < ntiles;
+    if (more) vt.issue(kbeg + 32 * (tile + kWaves), in);
+    const int k0 = kbeg + 32 * tile;
+    f32x16 s, dp;
+    rows_dot_pair<D>(lds_k, lds_v, i, g, qf, gf, s, dp);
+    if (more) next_k(tile + kWaves);
+    const int limit = p.causal ? min(qrow + p.coff, kend - 1) : kend - 1;  // largest visible key index
+#pragma unroll
+    for (int vq = 0; vq < 4; ++vq) {
+      int4 ids = {0, 0, 0, 0};
+      if constexpr (SEG) ids = *reinterpret_cast<const int4*>(lds_seg + 8 * vq + 4 * g);
+      const int idv[4] = {ids.x, ids.y, ids.z, ids.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int v = 4 * vq + e;
+        bool keep = k0 + 8 * vq + 4 * g + e <= limit;
+        if constexpr (SEG) keep = keep && idv[e] == qseg;
+        const float pt = keep ? __builtin_amdgcn_exp2f(s[v] - lse2) : 0.f;
+        s[v] = p.sm_scale * pt * (dp[v] - delta);  // dS
+      }
+    }
+    cols_accumulate32<D>(lds_k, i, g, s, dq);
+    if (more) arrive_k();
+  }
+  park<D>(lds_k, i, g, dq);
+  __syncthreads();
+  add_waves<D>(smem_bwd_f32, p.dq + (int64_t)b * p.lq * hd + (int64_t)h * D, q0, p.lq, hd, tid);
+}
+
+template <int D, bool SEG>
+__global__ __launch_bounds__(kThreads, 1) void bwd_f32_dkv_split_kernel(BwdF32Params p) {
+  constexpr int NDB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
+  int pair, h;
+  if (!decode_block(p.npairs, p.H, p.B, pair, h)) return;
+  const int blk = pair / p.B, b = pair % p.B;  // under the causal mask the first key blocks see the most rows: heaviest first
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  const int k0 = blk * 32, key = k0 + i, key_ld = min(key, p.lk - 1);
+  const int64_t hd = (int64_t)p.H * D;
+  float* const lds_q = smem_bwd_f32 + w * SplitLds<D>::kPerWave;
+  float* const lds_g = lds_q + SplitLds<D>::kMat;
+  float* const lds_row = lds_g + SplitLds<D>::kMat;  // [lse2 | delta | segment id][32]
+
+  // under the causal mask only rows at or after a key see it
+  int rbeg = p.causal ? min(p.lq, max(k0 - p.coff, 0)) / 32 * 32 : 0, rend = p.lq;
+  int32_t kseg = 0;
+  if constexpr (SEG) {
+    kseg = p.kvseg[(int64_t)b * p.lk + key_ld];
+    int first, last;
+    id_window<kThreads>(p.kvseg + (int64_t)b * p.lk + k0, min(32, p.lk - k0), p.qseg + (int64_t)b * p.lq + rbeg, p.lq - rbeg, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
+    rend = last < 0 ? rbeg : rbeg + last + 1;
+    if (last >= 0) rbeg = (rbeg + first) / 32 * 32;
+  }
+  const int ntiles = (max(0, rend - rbeg) + 31) / 32;
+  const float* const lse_b = p.lse + ((int64_t)b * p.H + h) * p.lq;
+  const float* const delta_b = p.delta + ((int64_t)b * p.H + h) * p.lq;
+  WaveTile<D> qt, gt;
+  qt.describe(p.q + (int64_t)b * p.lq * hd + (int64_t)h * D, hd, max(rend, 1), l);
+  gt.describe(p.d_o + (int64_t)b * p.lq * hd + (int64_t)h * D, hd, max(rend, 1), l);
+  // one matrix is in flight at a time: dO's tile is free after dV's product, Q's after dK's
+  typename WaveTile<D>::Regs in;
+  float row_in = 0.f;  // lanes 0-31: lse2, lanes 32-63: delta of one row of the tile
+  int32_t seg_in = 0;
+  if (w < ntiles) gt.issue(rbeg + 32 * w, in);
+  auto next_q = [&](int tile) __attribute__((always_inline)) {
+    const int row0 = rbeg + 32 * tile, r = row0 + i;
+    WaveTile<D>::store(in, lds_g, l, true);
+    qt.issue(row0, in);
+    const float x = (g ? delta_b : lse_b)[min(r, p.lq - 1)];
+    // rows past the end and rows without a visible key (lse = -inf): +inf makes every p of the row zero
+    row_in = g ? x : (r < rend && x > -INFINITY) ? x * kLog2e : INFINITY;
+    if constexpr (SEG) seg_in = p.qseg[(int64_t)b * p.lq + min(r, p.lq - 1)];
+  };
+  auto arrive_q = [&]() __attribute__((always_inline)) {
+    WaveTile<D>::store(in, lds_q, l, false);
+    lds_row[l] = row_in;
+    if constexpr (SEG) reinterpret_cast<int32_t*>(lds_row)[64 + i] = seg_in;
+  };
+
+  float kf[D / 2], vf[D / 2];
+  load_own_row<D>(p.k + ((int64_t)b * p.lk + key_ld) * hd + (int64_t)h * D, g, p.sm_scale * kLog2e, false, kf);
+  load_own_row<D>(p.v + ((int64_t)b * p.lk + key_ld) * hd + (int64_t)h * D, g, 1.f, false, vf);
+  f32x16 dk[NDB], dv[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { dk[db][v] = 0.f; dv[db][v] = 0.f; }
+
+  if (w < ntiles) {
+    next_q(w);
+    arrive_q();
+  }
+  for (int tile = w; tile < ntiles; tile += kWaves) {
+    const bool more = tile + kWaves < ntiles;
+    if (more) gt.issue(rbeg + 32 * (tile + kWaves), in);
+    const int r0 = rbeg + 32 * tile;
+    f32x16 s, dp;
+    rows_dot_pair<D>(lds_q, lds_g, i, g, kf, vf, s, dp);  // lane = key, registers = rows of the tile
+#pragma unroll
+    for (int vq = 0; vq < 4; ++vq) {
+      const int off = 8 * vq + 4 * g;
+      const f32x4 lse2 = *reinterpret_cast<const f32x4*>(lds_row + off);
+      const f32x4 dl = *reinterpret_cast<const f32x4*>(lds_row + 32 + off);
+      int4 ids = {0, 0, 0, 0};
+      if constexpr (SEG) ids = *reinterpret_cast<const int4*>(lds_row + 64 + off);
+      const int idv[4] = {ids.x, ids.y, ids.z, ids.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int v = 4 * vq + e;
+        bool keep = !p.causal || key - p.coff <= r0 + off + e;
+        if constexpr (SEG) keep = keep && idv[e] == kseg;
+        const float pt = keep ? __builtin_amdgcn_exp2f(s[v] - lse2[e]) : 0.f;
+        s[v] = pt;                                 // p
+        dp[v] = p.sm_scale * pt * (dp[v] - dl[e]);  // dS
+      }
+    }
+    cols_accumulate32<D>(lds_g, i, g, s, dv);
+    if (more) next_q(tile + kWaves);
+    cols_accumulate32<D>(lds_q, i, g, dp, dk);
+    if (more) arrive_q();
+  }
+  park<D>(lds_q, i, g, dk);
+  park<D>(lds_g, i, g, dv);
+  __syncthreads();
+  add_waves<D>(smem_bwd_f32, p.dk + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
+  add_waves<D>(smem_bwd_f32 + SplitLds<D>::kMat, p.dv + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
+}
+
+// Whether 32-row workgroups pay: the launch of 128-row ones leaves half of the 256 compute units idle, or fills them once
+// with causal blocks, of which the heaviest is twice the average.  (Forward and backward, us, 128 / 32 rows, 8 heads of
+// 64: 2 x 1000 tokens causal 384 / 215, not causal 434 / 313; 4 x 1000 causal 461 / 387, not causal 470 / 511; 8 x 1000
+// causal 562 / 617.)  The split kernels' buffer offsets take a batch entry below 2 GiB.
+bool few_blocks(const BwdF32Params& p, int rows, int D) {
+  const int64_t big = p.lq > p.lk ? p.lq : p.lk;
+  return (int64_t)((rows + kBlock - 1) / kBlock) * p.B * p.H <= (p.causal ? 256 : 128) && (big + 64) * p.H * D * 4 < (int64_t(1) << 31);
+}
+
+template <typename K>
+int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int block, size_t lds, BwdF32Params p, hipStream_t stream) {
+  p.nblk = (rows + block - 1) / block;
+  p.npairs = p.nblk * p.B;
+  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(((p.npairs + 7) / 8) * 8 * p.H), dim3(kThreads), lds, stream, p);
+  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+}
+
+template <int D, bool SEG>
+int launch_pair(const BwdF32Params& p, hipStream_t stream) {
+  static bool configured[4][kMaxDevices] = {};
+  int rc = few_blocks(p, p.lq, D) ? launch_kernel(bwd_f32_dq_split_kernel<D, SEG>, configured[0], p.lq, 32, SplitLds<D>::kBytes, p, stream)
+                                  : launch_kernel(bwd_f32_dq_kernel<D, SEG>, configured[1], p.lq, kBlock, BwdLds<D>::kBytes, p, stream);
+  if (rc != TPA_OK) return rc;
+  return few_blocks(p, p.lk, D) ? launch_kernel(bwd_f32_dkv_split_kernel<D, SEG>, configured[2], p.lk, 32, SplitLds<D>::kBytes, p, stream)
+                                : launch_kernel(bwd_f32_dkv_kernel<D, SEG>, configured[3], p.lk, kBlock, BwdLds<D>::kBytes, p, stream);
 }
 
 }  // namespace

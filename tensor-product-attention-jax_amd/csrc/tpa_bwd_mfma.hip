@@ -114,47 +114,6 @@ __device__ __forceinline__ f32x16 splat16(float x) {
   return r;
 }
 
-
-// Packed sequences (tpa/tpa.py:369-375 compares ids pairwise): an element of `other` can only
-// pair with this workgroup's elements if its id lies within [min, max] of the workgroup's own ids
-// `mine[0 .. n_mine)`.  Returns the first and last such index of other[0 .. n_other) (last = -1 if
-// there is none): exact for ids that do not decrease along the sequence, conservative otherwise
-// (the per-pair mask still decides).  `red` = 4 ints of LDS; every thread of the workgroup calls.
-template <int NT>
-__device__ __forceinline__ void id_window(const int32_t* mine, int n_mine, const int32_t* other, int n_other, int32_t* red,
-                                          int tid, int& first, int& last) {
-  if (tid == 0) { red[0] = INT32_MAX; red[1] = INT32_MIN; red[2] = INT32_MAX; red[3] = -1; }
-  __syncthreads();
-  {  // one atomic per wave: the lanes' values are reduced in registers first
-    int32_t smin = INT32_MAX, smax = INT32_MIN;
-    for (int t = tid; t < n_mine; t += NT) {
-      const int32_t sid = mine[t];
-      smin = min(smin, sid); smax = max(smax, sid);
-    }
-    smin = wave_min(smin); smax = wave_max(smax);
-    if ((tid & 63) == 0 && smin <= smax) {
-      __hip_atomic_fetch_min(&red[0], smin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_max(&red[1], smax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-  }
-  __syncthreads();
-  const int32_t lo_id = red[0], hi_id = red[1];
-  int lo = INT32_MAX, hi = -1;
-  for (int t = tid; t < n_other; t += NT) {
-    const int32_t sid = other[t];
-    if (sid >= lo_id && sid <= hi_id) { lo = min(lo, t); hi = max(hi, t); }
-  }
-  lo = wave_min(lo); hi = wave_max(hi);
-  if ((tid & 63) == 0 && hi >= 0) {
-    __hip_atomic_fetch_min(&red[2], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_max(&red[3], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  __syncthreads();
-  first = red[2];
-  last = red[3];
-  __syncthreads();  // the tiles reuse this memory
-}
-
 // ============================================================================================
 // dQ
 // ============================================================================================

@@ -24,8 +24,7 @@ namespace tpa {
 namespace {
 
 constexpr int kTK = 64;   // keys per tile
-constexpr int kNW = 8;    // waves per workgroup
-constexpr int kBQ = 256;  // query rows per workgroup (32 per wave)
+constexpr int kNW = 8;    // waves per workgroup (32 query rows each); half as many where 256-row blocks are too few
 
 struct F32Params {
   TpaFactor qa, qb, ka, kb, va, vb;  // dense: a pointers null, b = q/k/v with stride_l = H*D
@@ -46,9 +45,9 @@ struct LdsF32 {
   static constexpr size_t kBytes = (size_t)(4 * kTile + 2 * kTK) * 4;  // K and V double buffered + key segment ids
 };
 
-template <int D, bool SEG>
-__global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
-  constexpr int NT = kNW * 64;
+template <int D, int NW, bool SEG>
+__global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
+  constexpr int NT = NW * 64, kBQ = NW * 32;
   constexpr int RS = LdsF32<D>::RS, kTile = LdsF32<D>::kTile;
   constexpr int NDB = D / 32;         // 32-row blocks of O^T
   constexpr int NQ = D / 2;           // Q values per lane
@@ -90,7 +89,15 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
   // ---- key range
   const int len_b = p.kvlen ? max(0, min(p.kvlen[b], p.lk)) : p.lk;
   const int coff = p.coff + (p.causal == TPA_CAUSAL_BOTTOM_RIGHT ? len_b - p.lq : 0);  // bottom-right alignment counts from the end of this entry's keys
-  const int kend = p.causal ? min(len_b, min(q0 + kBQ, p.lq) + coff) : len_b;
+  int kend = p.causal ? min(len_b, min(q0 + kBQ, p.lq) + coff) : len_b, kbeg = 0;
+  if constexpr (SEG) {  // only tiles that hold keys with ids of these rows
+    if (kend > 0) {
+      int first, last;
+      id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kBQ, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem_f32), tid, first, last);
+      kbeg = last < 0 ? 0 : first / kTK * kTK;
+      kend = last + 1;
+    }
+  }
   float* const orow = p.o + (((int64_t)b * p.lq + qrow) * p.H + h) * D;
   if (kend <= 0) {  // no key at all: the rows end as NaN / -inf (tpa/tpa.py:437-439)
     if (qrow < p.lq) {
@@ -101,8 +108,8 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
     }
     return;
   }
-  const int ntiles = (kend + kTK - 1) / kTK;
-  const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + coff + 31, 0) / kTK) : ntiles - 1;
+  const int ntiles = (kend - kbeg + kTK - 1) / kTK;
+  const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + coff + 31 - kbeg, 0) / kTK) : ntiles - 1;
 
   // ---- Q (B operand of S^T = K Q^T), scaled: qf[4m + e] = c * Q[qrow][8m + 4g + e]
   float qf[NQ];
@@ -137,7 +144,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
 #pragma unroll
     for (int q = 0; q < CH; ++q) {
       const int chunk = q * NT + tid, t = chunk / CPR, cc = chunk % CPR;
-      const int tok = tile * kTK + t;
+      const int tok = kbeg + tile * kTK + t;
       f32x4 ak = {0.f, 0.f, 0.f, 0.f}, av = {0.f, 0.f, 0.f, 0.f};
       if (tok < kend) {  // rows past the end stay zero: they are masked, and 0 * padding must not make NaN
         for (int r = 0; r < p.rk; ++r) {
@@ -153,7 +160,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
       *reinterpret_cast<f32x4*>(vd + t * RS + 4 * cc) = av * inv_r;
     }
     if constexpr (SEG)
-      if (tid < kTK) lds_seg[(tile & 1) * kTK + tid] = p.kvseg[(int64_t)b * p.lk + min(tile * kTK + tid, p.lk - 1)];
+      if (tid < kTK) lds_seg[(tile & 1) * kTK + tid] = p.kvseg[(int64_t)b * p.lk + min(kbeg + tile * kTK + tid, p.lk - 1)];
   };
 
   // ---- per-wave state
@@ -170,7 +177,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
   f32x16 s[2];  // logits, then probabilities, of the tile in flight: two 32-key blocks
   auto logits_softmax = [&](int tile) __attribute__((always_inline)) {
     const float* const ks = lds_k + (tile & 1) * kTile;
-    const int k0 = tile * kTK;
+    const int k0 = kbeg + tile * kTK;
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -256,7 +263,7 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
   // The next tile may be rebuilt anywhere between two barriers.  Waves w and w + 4 share a SIMD:
   // one of them rebuilds (waiting for its factor loads) before its matrix work, the other in the
   // middle of it, so the SIMD always has a wave with matrix work and both end the tile together.
-  const bool rebuild_first = w < kNW / 2;
+  const bool rebuild_first = w < NW / 2;
   for (int j = 0; j < ntiles; ++j) {
     const bool more = j + 1 < ntiles, mine = j <= wave_last_tile && wrow0 < p.lq;  // waves past the last row only help rebuild
     if (rebuild_first && more) rebuild(j + 1);
@@ -282,14 +289,305 @@ __global__ __launch_bounds__(kNW * 64) void prefill_f32_kernel(F32Params pp) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same for problems with few blocks of 256 query rows.  Such a launch leaves most of the chip idle and its time is
+// that of one workgroup walking all keys (one sequence of 512 tokens, 8 heads of 64: 16 workgroups, 75 us).  Here a
+// workgroup owns 32 query rows and its four waves split the keys: wave w takes the tiles of 32 keys w, w + 4, ...,
+// rebuilds each into LDS of its own (no barrier in the loop) with the next tile's factors on their way while the matrix
+// pipe works on this one, and the four partial results are merged through LDS with the rule of _lse_accum
+// (tpa/tpa.py:228-242).  Every workgroup rebuilds its tiles for 32 rows instead of 256, which is why the kernel above
+// stays the one for launches that fill the chip (`few_rows_pay` below).
+constexpr int kSplitWaves = 4;
+template <int D>
+struct SplitLdsF32 {
+  static constexpr int RS = D + 4;
+  static constexpr int kPerWave = 2 * 32 * RS;  // K and V tile; the merge reuses the K tile (O), its last columns (m, l)
+  static constexpr size_t kBytes = (size_t)(kSplitWaves * kPerWave + 4) * 4;
+};
+
+template <int D, bool SEG>
+__global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(F32Params p) {
+  constexpr int RS = SplitLdsF32<D>::RS;
+  constexpr int NDB = D / 32, CPR = D / 4, RPI = 64 / CPR, NST = 32 / RPI;  // a load instruction of the wave takes RPI rows
+  typedef __attribute__((ext_vector_type(NDB))) float f32xN;
+
+  extern __shared__ __attribute__((aligned(16))) float smem_f32_split[];
+  const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
+  const int round = slot / p.H;
+  const int pair = round * 8 + xcd_pair_slot(round, xcd, p.B);
+  const int h = slot % p.H;
+  if (pair >= p.npairs) return;
+  const int qblk = p.nqb - 1 - pair / p.B;  // heaviest causal blocks first
+  const int b = pair % p.B;
+
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  const int q0 = qblk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
+  const bool dense = p.ka.ptr == nullptr;  // dense q, k, v: weight 1, the head's slice of the row
+  float* const lds_k = smem_f32_split + w * SplitLdsF32<D>::kPerWave;  // [32][RS]
+  float* const lds_v = lds_k + 32 * RS;
+
+  const int len_b = p.kvlen ? max(0, min(p.kvlen[b], p.lk)) : p.lk;
+  const int coff = !p.causal ? 0 : p.coff + (p.causal == TPA_CAUSAL_BOTTOM_RIGHT ? len_b - p.lq : 0);
+  int kend = p.causal ? min(len_b, min(q0 + 32, p.lq) + coff) : len_b, kbeg = 0;
+  int32_t qseg = 0;
+  if constexpr (SEG) {
+    qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
+    if (kend > 0) {
+      int first, last;
+      id_window<kSplitWaves * 64>(p.qseg + (int64_t)b * p.lq + q0, min(32, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend,
+                                  reinterpret_cast<int32_t*>(smem_f32_split), tid, first, last);
+      kbeg = last < 0 ? 0 : first / 32 * 32;
+      kend = last < 0 ? 0 : last + 1;
+    }
+  }
+  const int ntiles = kend > kbeg ? (kend - kbeg + 31) / 32 : 0;
+
+  // Factor rows as raw buffer loads: per array one lane offset that never changes and a scalar one per load (with 64-bit
+  // addresses per lane and load the kernel spilled 240 registers).  Tokens from kend on are inside the array or read as
+  // zero; the last tile clears them (padding rows may hold anything, and 0 * NaN must not reach the sums).
+  const float inv_r = 1.f / (float)p.rk;
+  const int lrow = l / CPR, lc = l % CPR;
+  struct Rows { __amdgpu_buffer_rsrc_t rs; int voff, sl, sr; };  // byte offset of the lane, bytes between tokens and ranks
+  auto rows_of = [&](const TpaFactor& f, int64_t first, int lane_elem, int width) {
+    const float* base = static_cast<const float*>(f.ptr) + b * f.stride_b + first;
+    const int64_t bytes = ((int64_t)(p.lk - 1) * f.stride_l + (int64_t)(p.rk - 1) * f.stride_r + width) * 4;
+    return Rows{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)bytes, 0x00020000),
+                (int)((lrow * f.stride_l + lane_elem) * 4), (int)(f.stride_l * 4), (int)(f.stride_r * 4)};
+  };
+  const Rows kb_r = rows_of(p.kb, dense ? (int64_t)h * D : 0, 4 * lc, D), vb_r = rows_of(p.vb, dense ? (int64_t)h * D : 0, 4 * lc, D);
+  const Rows ka_r = dense ? kb_r : rows_of(p.ka, h, 0, 1), va_r = dense ? vb_r : rows_of(p.va, h, 0, 1);
+  f32x4 in[NST], vac[NST];  // the rows in flight (K's or V's, one rank), the sum over V's ranks
+  float wt[NST];
+  int32_t seg_in = 0, seg_id = 0;  // ids of key (this lane's i) of the next tile and of this one
+  auto issue = [&](const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NST; ++q) {
+      const int t = kbeg + tile * 32 + q * RPI;
+      in[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb.rs, rb.voff, t * rb.sl + r * rb.sr, 0));
+      wt[q] = 1.f;
+      if (!dense) wt[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra.rs, ra.voff, t * ra.sl + r * ra.sr, 0));
+    }
+  };
+  auto row_in = [&](int tile, int q) __attribute__((always_inline)) -> f32x4 {
+    const f32x4 x = wt[q] * inv_r * in[q];
+    return q * RPI + lrow < kend - kbeg - tile * 32 ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  // K is added up in its LDS tile (free once the logits are done), V in registers until its tile has been used
+  auto take_k = [&](int tile, bool first) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NST; ++q) {
+      f32x4* const at = reinterpret_cast<f32x4*>(lds_k + (q * RPI + lrow) * RS + 4 * lc);
+      const f32x4 x = row_in(tile, q);
+      *at = first ? x : *at + x;
+    }
+  };
+  auto take_v = [&](int tile, bool first) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NST; ++q) {
+      const f32x4 x = row_in(tile, q);
+      vac[q] = first ? x : vac[q] + x;
+    }
+  };
+  auto store_v = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NST; ++q) *reinterpret_cast<f32x4*>(lds_v + (q * RPI + lrow) * RS + 4 * lc) = vac[q];
+  };
+  // all ranks but the last of one array: the first is on its way already, the last one is when this returns
+  auto ranks = [&](const Rows& rb, const Rows& ra, int tile, auto&& take) __attribute__((always_inline)) {
+    take(tile, true);
+    for (int r = 1; r + 1 < p.rk; ++r) {
+      issue(rb, ra, tile, r);
+      take(tile, false);
+    }
+    if (p.rk > 1) issue(rb, ra, tile, p.rk - 1);
+  };
+
+  if (w < ntiles) issue(vb_r, va_r, w, 0);
+  // ---- Q (B operand of S^T = K Q^T), scaled: qf[4m + e] = c * Q[qrow][8m + 4g + e]
+  float qf[D / 2];
+#pragma unroll
+  for (int j = 0; j < D / 2; ++j) qf[j] = 0.f;
+  {
+    const float* qb = static_cast<const float*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qrow_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * g;
+    const float* qa = dense ? nullptr : static_cast<const float*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qrow_ld * p.qa.stride_l + h;
+    for (int r0 = 0; r0 < p.rq; r0 += 3) {  // three ranks in flight: the loads of one would expose their latency rank by rank
+      f32x4 bv[3][D / 8];
+      float a[3];
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        const int r = min(r0 + u, p.rq - 1);
+        a[u] = r0 + u >= p.rq ? 0.f : dense ? 1.f : qa[r * p.qa.stride_r];
+#pragma unroll
+        for (int m = 0; m < D / 8; ++m) bv[u][m] = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r + 8 * m);
+      }
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (r0 + u < p.rq)
+#pragma unroll
+          for (int m = 0; m < D / 8; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qf[4 * m + e] += a[u] * bv[u][m][e];
+    }
+    const float scale = p.sm_scale * kLog2e / (float)p.rq;
+#pragma unroll
+    for (int j = 0; j < D / 2; ++j) qf[j] *= scale;
+  }
+
+  f32x16 o[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[db][v] = 0.f;
+  float m_run = -INFINITY, lsum = 0.f;
+
+  if (w < ntiles) {
+    ranks(vb_r, va_r, w, take_v);
+    if (p.rk > 1) take_v(w, false);
+    store_v();
+    issue(kb_r, ka_r, w, 0);
+    ranks(kb_r, ka_r, w, take_k);
+    if (p.rk > 1) take_k(w, false);
+    if constexpr (SEG) seg_id = p.kvseg[(int64_t)b * p.lk + min(kbeg + w * 32 + i, p.lk - 1)];
+  }
+  for (int tile = w; tile < ntiles; tile += kSplitWaves) {
+    const int next = tile + kSplitWaves;
+    const bool more = next < ntiles;
+    if (more) issue(vb_r, va_r, next, 0);
+    f32x16 s, s2;  // two accumulation chains, added at the end
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { s[v] = 0.f; s2[v] = 0.f; }
+#pragma unroll
+    for (int m = 0; m < D / 8; ++m) {
+      if (m == D / 16 && more) ranks(vb_r, va_r, next, take_v);
+      const f32x4 kf = *reinterpret_cast<const f32x4*>(lds_k + i * RS + 8 * m + 4 * g);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[0], qf[4 * m], s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[1], qf[4 * m + 1], s2, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[2], qf[4 * m + 2], s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[3], qf[4 * m + 3], s2, 0, 0, 0);
+    }
+    if (more) {
+      if (p.rk > 1) take_v(next, false);
+      issue(kb_r, ka_r, next, 0);
+      if constexpr (SEG) seg_in = p.kvseg[(int64_t)b * p.lk + min(kbeg + next * 32 + i, p.lk - 1)];
+    }
+    // register v, wave half g  <->  key k0 + 8 (v / 4) + 4 g + v % 4
+    const int k0 = kbeg + tile * 32;
+    const int limit = p.causal ? min(qrow + coff, kend - 1) : kend - 1;  // largest visible key index
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int t = 8 * (v >> 2) + 4 * g + (v & 3);
+      bool keep = k0 + t <= limit;
+      if constexpr (SEG) {
+        const int32_t id_t = __shfl(seg_id, t, 64);  // by every lane, whatever it keeps
+        keep = keep && id_t == qseg;
+      }
+      s[v] = keep ? s[v] + s2[v] : -INFINITY;
+      tmax = fmaxf(tmax, s[v]);
+    }
+    tmax = halves_max(tmax);
+    const float m_new = fmaxf(m_run, tmax);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // a row that has met no visible key yet
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    m_run = m_new;
+    if (__any(alpha != 1.f)) {
+      lsum *= alpha;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      s[v] = __builtin_amdgcn_exp2f(s[v] - m_use);
+      lsum += s[v];
+    }
+    // O^T += V^T P^T: the step of register v takes, in wave half g, the key that register belongs to
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      if (v == 8 && more) ranks(kb_r, ka_r, next, take_k);
+      const f32xN vf = *reinterpret_cast<const f32xN*>(lds_v + (8 * (v >> 2) + 4 * g + (v & 3)) * RS + NDB * i);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db], s[v], o[db], 0, 0, 0);
+    }
+    if (more) {
+      if (p.rk > 1) take_k(next, false);
+      store_v();
+      if constexpr (SEG) seg_id = seg_in;
+    }
+  }
+
+  // ---- merge the waves: row i of a wave's O at lds_k + i RS, its m and l in the four padding columns
+  const float ltot = halves_sum(lsum);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int row = 8 * (v >> 2) + 4 * g + (v & 3);  // of block db: d = NDB row + db
+    f32xN out;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) out[db] = o[db][v];
+    *reinterpret_cast<f32xN*>(lds_k + i * RS + NDB * row) = out;
+  }
+  if (g == 0) {
+    lds_k[i * RS + D] = m_run;
+    lds_k[i * RS + D + 1] = ltot;
+  }
+  __syncthreads();
+  for (int idx = tid; idx < 32 * CPR; idx += kSplitWaves * 64) {
+    const int row = idx / CPR, cc = idx % CPR;
+    if (q0 + row >= p.lq) continue;
+    const float* const at = smem_f32_split + row * RS;
+    float mmax = -INFINITY, lacc = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < kSplitWaves; ++ww) mmax = fmaxf(mmax, at[ww * SplitLdsF32<D>::kPerWave + D]);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ww = 0; ww < kSplitWaves; ++ww) {
+      const float mw = at[ww * SplitLdsF32<D>::kPerWave + D];
+      const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mmax);
+      acc += f * *reinterpret_cast<const f32x4*>(at + ww * SplitLdsF32<D>::kPerWave + 4 * cc);
+      lacc += f * at[ww * SplitLdsF32<D>::kPerWave + D + 1];
+    }
+    const float inv = 1.f / lacc;  // no visible key: 0 * inf = NaN, as in tpa/tpa.py:437-439
+    *reinterpret_cast<f32x4*>(p.o + (((int64_t)b * p.lq + q0 + row) * p.H + h) * D + 4 * cc) = acc * inv;
+    if (p.lse && cc == 0) p.lse[((int64_t)b * p.H + h) * p.lq + q0 + row] = (mmax + __builtin_amdgcn_logf(lacc)) * kLn2;
+  }
+}
+
+// The split kernel's buffer offsets take keys of one batch entry below 2 GiB.
+bool split_supported(const F32Params& p) {
+  const TpaFactor* fs[4] = {&p.ka, &p.kb, &p.va, &p.vb};
+  for (const TpaFactor* f : fs)
+    if (f->stride_l < 0 || f->stride_r < 0 || (p.lk * f->stride_l + p.rk * f->stride_r + 256) * 4 >= (int64_t(1) << 31)) return false;
+  return true;
+}
+
+// Rows of a workgroup: 32 (keys split over its waves), 128 or 256.  A launch of 256-row workgroups that does not fill the
+// 256 compute units takes as long as one workgroup; with 128 rows (one wave per SIMD) a tile takes half the time, which
+// pays as long as they all fit the chip at once - under the causal mask, whose heaviest workgroup is twice the average,
+// up to two rounds.  Measured, us with 256 / 128 / 32 rows: 1 x 512 tokens, 8 heads of 64 causal 75 / 41 / 32; 2 x 1000
+// 144 / 69 / 68; 4 x 1000 146 / 112 / 134, not causal 155 / 113 / 222; 8 x 1000 not causal 157 / 191 / 441.
+int rows_per_workgroup(const F32Params& p) {
+  auto wgs = [&](int rows) { return (int64_t)((p.lq + rows - 1) / rows) * p.B * p.H; };
+  if (wgs(32) <= 512 && split_supported(p)) return 32;
+  return wgs(128) <= 256 || (p.causal && wgs(256) <= 256) ? 128 : 256;
+}
+
+template <typename K>
+int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int threads, size_t lds, F32Params p, hipStream_t stream) {
+  p.nqb = (p.lq + rows - 1) / rows;
+  p.npairs = p.nqb * p.B;
+  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3((p.npairs + 7) / 8 * 8 * p.H), dim3(threads), lds, stream, p);
+  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+}
+
 template <int D, bool SEG>
 int launch_f32(const F32Params& p, hipStream_t stream) {
-  auto kern = prefill_f32_kernel<D, SEG>;
-  static bool configured[kMaxDevices] = {};
-  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), LdsF32<D>::kBytes); rc != TPA_OK) return rc;
-  const int groups = (p.npairs + 7) / 8;
-  hipLaunchKernelGGL(kern, dim3(groups * 8 * p.H), dim3(kNW * 64), LdsF32<D>::kBytes, stream, p);
-  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+  static bool configured[3][kMaxDevices] = {};
+  const int rows = rows_per_workgroup(p);
+  if (rows == 32) return launch_kernel(prefill_f32_split_kernel<D, SEG>, configured[0], 32, kSplitWaves * 64, SplitLdsF32<D>::kBytes, p, stream);
+  if (rows == 128) return launch_kernel(prefill_f32_kernel<D, kNW / 2, SEG>, configured[1], 128, kNW * 32, LdsF32<D>::kBytes, p, stream);
+  return launch_kernel(prefill_f32_kernel<D, kNW, SEG>, configured[2], 256, kNW * 64, LdsF32<D>::kBytes, p, stream);
 }
 
 int launch_any(const F32Params& p, int d, hipStream_t stream) {
@@ -319,8 +617,6 @@ int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
   p.o = static_cast<float*>(a->o); p.lse = a->lse;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq; p.rk = a->rk;
   p.sm_scale = a->sm_scale; p.causal = a->causal; p.coff = causal_offset_of(a);
-  p.nqb = (a->lq + kBQ - 1) / kBQ;
-  p.npairs = p.nqb * a->B;
   return launch_any(p, a->dk, stream);
 }
 
@@ -343,7 +639,5 @@ int mha_prefill_f32_launch(const MhaFwdArgs* a, hipStream_t stream) {
   p.o = static_cast<float*>(a->o); p.lse = a->lse;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = 1; p.rk = 1;
   p.sm_scale = a->sm_scale; p.causal = a->causal ? TPA_CAUSAL_TOP_LEFT : TPA_CAUSAL_NONE;
-  p.nqb = (a->lq + kBQ - 1) / kBQ;
-  p.npairs = p.nqb * a->B;
   return launch_any(p, a->dk, stream);
 }
