@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define TPA_ABI_VERSION 9
+#define TPA_ABI_VERSION 10
 
 /* element types of the factor / output arrays */
 enum { TPA_DTYPE_F32 = 0, TPA_DTYPE_BF16 = 1 };
@@ -171,7 +171,7 @@ typedef struct MhaFwdArgs {
 } MhaFwdArgs;
 
 /*
- * One gradient array, fp32 whatever the element type of the inputs is: same indexing as the
+ * One gradient array, fp32 unless TpaBwdArgs.grad_dtype says otherwise (`ptr` is then cast): same indexing as the
  * TpaFactor it is the gradient of (innermost dimension contiguous, ELEMENT strides), so the
  * concatenated dq[b, lq, rq, h+dk] that _tpa_bwd returns (tpa/tpa.py:960-962) is written in place
  * (A part = base, B part = base + h, rank stride h+dk).
@@ -201,7 +201,7 @@ typedef struct TpaBwdArgs {
   const void* o;     /* [B, lq, H, dv] forward output, element type = dtype */
   const float* lse;  /* [B, H, lq] forward logsumexp (fp32) */
   const void* d_o;   /* [B, lq, H, dv] gradient of the loss with respect to o, element type = dtype */
-  TpaGrad dqa, dqb, dka, dkb, dva, dvb; /* outputs, fp32 */
+  TpaGrad dqa, dqb, dka, dkb, dva, dvb; /* outputs, element type = grad_dtype */
   int32_t B, lq, lk, H, dk, dv, rq, rk;
   int32_t dtype;
   float sm_scale;
@@ -210,6 +210,8 @@ typedef struct TpaBwdArgs {
   void* workspace;        /* required: at least tpa_bwd_workspace_bytes(...) bytes, 256-byte aligned */
   size_t workspace_bytes;
   int32_t causal_offset;  /* as in TpaFwdArgs: the value the forward call was made with */
+  int32_t grad_dtype;     /* TPA_DTYPE_F32 (0), or TPA_DTYPE_BF16 with bf16 inputs: element type of the six gradient arrays
+                             (fp32 sums, rounded once) */
 } TpaBwdArgs;
 
 /*

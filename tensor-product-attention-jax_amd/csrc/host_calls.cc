@@ -406,7 +406,7 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ------------------------------------------------------------------------------------------------ backward
-// Gradients of the six factors into the concatenated fp32 arrays dq, dk, dv (tpa/tpa.py:960-962); `lse` is [b, h, lq].
+// Gradients of the six factors into concatenated arrays dq, dk, dv of the inputs' type (tpa/tpa.py:960-962); `lse` is [b, h, lq].
 struct BwdCall {
   Tensor q, k, v, qseg, kvseg, o, lse, d_o;
   int64_t heads = 0;
@@ -432,7 +432,7 @@ void run_bwd(const BwdCall& c, Tensor* grads) {
   expect(is_shape(d_o, {a.B, a.lq, a.H, a.dv}), d_o);
   expect(is_shape(lse, {a.B, a.H, a.lq}), lse);
   const Tensor* in[3] = {&c.q, &c.k, &c.v};
-  for (int i = 0; i < 3; ++i) grads[i] = at::empty(in[i]->sizes(), at::TensorOptions().device(device).dtype(at::kFloat));
+  for (int i = 0; i < 3; ++i) grads[i] = at::empty(in[i]->sizes(), at::TensorOptions().device(device).dtype(dtype));
   a.dqa = factor_of<TpaGrad>(grads[0]); a.dqb = factor_of<TpaGrad>(grads[0], h);
   a.dka = factor_of<TpaGrad>(grads[1]); a.dkb = factor_of<TpaGrad>(grads[1], h);
   a.dva = factor_of<TpaGrad>(grads[2]); a.dvb = factor_of<TpaGrad>(grads[2], h);
@@ -444,12 +444,12 @@ void run_bwd(const BwdCall& c, Tensor* grads) {
   a.sm_scale = (float)c.sm_scale;
   a.causal = c.causal;
   a.causal_offset = c.causal_offset;
+  a.grad_dtype = a.dtype;
   const size_t need = lib.tpa_bwd_workspace_bytes(a.B, a.lq, a.lk, a.H, a.dk, a.dv);
   const Tensor ws = bytes_on(device, need + 256);
   a.workspace = aligned(ws, 256);
   a.workspace_bytes = need;
   check("tpa_bwd", lib.tpa_bwd(&a, stream_of(device)));
-  for (int i = 0; i < 3; ++i) grads[i] = grads[i].to(dtype);
 }
 
 // backward(q, k, v, q_segment_ids, kv_segment_ids, o, lse, do, num_heads, sm_scale, causal, causal_offset)

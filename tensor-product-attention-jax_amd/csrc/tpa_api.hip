@@ -173,6 +173,7 @@ int mha_fwd(const MhaFwdArgs* a, void* stream) {
 int tpa_bwd(const TpaBwdArgs* a, void* stream) {
   if (!a) return TPA_ERR_NULL;
   if (a->dtype != TPA_DTYPE_F32 && a->dtype != TPA_DTYPE_BF16) return TPA_ERR_DTYPE;
+  if (a->grad_dtype != TPA_DTYPE_F32 && a->grad_dtype != a->dtype) return TPA_ERR_DTYPE;
   if (a->B <= 0 || a->lq <= 0 || a->lk <= 0 || a->H <= 0 || a->dk <= 0 || a->dv <= 0 || a->rq <= 0 || a->rk <= 0)
     return TPA_ERR_SHAPE;
   if (a->dk > 256 || a->dv > 256) return TPA_ERR_SHAPE;

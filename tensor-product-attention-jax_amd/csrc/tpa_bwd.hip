@@ -90,12 +90,82 @@ __global__ __launch_bounds__(256) void recon_bf16_kernel(TpaFactor fa, TpaFactor
 // (token, 16-byte piece of D, group of 8 heads) and reads, per rank, one 16-byte piece of b and
 // the 8 head factors as one 16-byte piece of a - 64 multiply-adds per two loads.  Pieces are the
 // fastest thread index, so the 16 threads of a (token, head group) store whole rows of D.
-struct ReconJob { TpaFactor fa, fb; uint16_t* out; int L, R; float scale; };
-struct ReconJobs { ReconJob job[3]; };  // blockIdx.z picks one: several arrays in one launch
+struct ReconJob { TpaFactor fa, fb; void* out; int L, R; float scale; };
+// The backward's delta in the same launch (blockIdx.z = 3): delta[b, h, i] = sum_d o * do, NaN products (an empty row's o)
+// skipped; a thread takes the same piece of 8 heads of one row, the sum over d runs across the lanes that share them.
+struct DeltaJob { const void *o, *d_o; float* delta; int lq; };
+struct ReconJobs { ReconJob job[3]; DeltaJob delta; };  // blockIdx.z picks one: several arrays in one launch
+template <typename T>
+__device__ __forceinline__ void delta_h8(const DeltaJob& j, int64_t t, int g, int cc, int cpr, int b, int H, int D) {
+  constexpr int N = 16 / sizeof(T);  // elements of a 16-byte piece
+  const bool live = t < j.lq;
+  const int64_t at = (((int64_t)b * j.lq + (live ? t : j.lq - 1)) * H + 8 * g) * D + N * cc;
+  u32x4 ov[8], gv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    ov[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const T*>(j.o) + at + (int64_t)i * D));
+    gv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const T*>(j.d_o) + at + (int64_t)i * D));
+  }
+  float mine = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float acc = 0.f;
+    auto add = [&](float x) { if (x == x) acc += x; };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (sizeof(T) == 2) {
+        add(bf16lo_to_f32(ov[i][e]) * bf16lo_to_f32(gv[i][e]));
+        add(bf16hi_to_f32(ov[i][e]) * bf16hi_to_f32(gv[i][e]));
+      } else {
+        add(__uint_as_float(ov[i][e]) * __uint_as_float(gv[i][e]));
+      }
+    }
+    for (int m = 1; m < cpr; m <<= 1) acc += __shfl_xor(acc, m, 64);
+    if (cc == i) mine = acc;
+  }
+  if (live && cc < 8) j.delta[((int64_t)b * H + 8 * g + cc) * j.lq + t] = mine;
+}
+
+// fp32 factors -> dense fp32, in the same way: a thread owns 4 elements of D for 8 heads of a token
+__global__ __launch_bounds__(256) void recon_f32_h8_kernel(ReconJobs jobs, int H, int D) {
+  const int cpr = D / 4, hg = H / 8;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int cc = (int)(idx % cpr), g = (int)(idx / cpr % hg), b = blockIdx.y;
+  const int64_t t = idx / ((int64_t)cpr * hg);
+  if (blockIdx.z == 3) return delta_h8<float>(jobs.delta, t, g, cc, cpr, b, H, D);
+  const ReconJob job = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
+  if (t >= job.L) return;
+  const float* ap = static_cast<const float*>(job.fa.ptr) + b * job.fa.stride_b + t * job.fa.stride_l + 8 * g;
+  const float* bp = static_cast<const float*>(job.fb.ptr) + b * job.fb.stride_b + t * job.fb.stride_l + 4 * cc;
+  f32x4 acc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int G = 2;  // ranks whose loads are in flight together
+  for (int r0 = 0; r0 < job.R; r0 += G) {
+    f32x4 av[G][2], bv[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const int r = min(r0 + u, job.R - 1);
+      av[u][0] = *reinterpret_cast<const f32x4*>(ap + (int64_t)r * job.fa.stride_r);
+      av[u][1] = *reinterpret_cast<const f32x4*>(ap + (int64_t)r * job.fa.stride_r + 4);
+      bv[u] = *reinterpret_cast<const f32x4*>(bp + (int64_t)r * job.fb.stride_r);
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u)
+      if (r0 + u < job.R)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] += av[u][i / 4][i % 4] * bv[u];
+  }
+  const float inv = job.scale / (float)job.R;
+  float* op = reinterpret_cast<float*>(job.out) + (((int64_t)b * job.L + t) * H + 8 * g) * D + 4 * cc;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(op + (int64_t)i * D) = acc[i] * inv;
+}
+
 __global__ __launch_bounds__(256) void recon_bf16_h8_kernel(ReconJobs jobs, int H, int D) {
   const TpaFactor fa = blockIdx.z == 0 ? jobs.job[0].fa : blockIdx.z == 1 ? jobs.job[1].fa : jobs.job[2].fa;
   const TpaFactor fb = blockIdx.z == 0 ? jobs.job[0].fb : blockIdx.z == 1 ? jobs.job[1].fb : jobs.job[2].fb;
-  uint16_t* const out = blockIdx.z == 0 ? jobs.job[0].out : blockIdx.z == 1 ? jobs.job[1].out : jobs.job[2].out;
+  uint16_t* const out = static_cast<uint16_t*>(blockIdx.z == 0 ? jobs.job[0].out : blockIdx.z == 1 ? jobs.job[1].out : jobs.job[2].out);
   const int L = blockIdx.z == 0 ? jobs.job[0].L : blockIdx.z == 1 ? jobs.job[1].L : jobs.job[2].L;
   const int R = blockIdx.z == 0 ? jobs.job[0].R : blockIdx.z == 1 ? jobs.job[1].R : jobs.job[2].R;
   const float scale = blockIdx.z == 0 ? jobs.job[0].scale : blockIdx.z == 1 ? jobs.job[1].scale : jobs.job[2].scale;
@@ -105,6 +175,7 @@ __global__ __launch_bounds__(256) void recon_bf16_h8_kernel(ReconJobs jobs, int 
   const int g = (int)(idx / cpr % hg);
   const int64_t t = idx / ((int64_t)cpr * hg);
   const int b = blockIdx.y;
+  if (blockIdx.z == 3) return delta_h8<uint16_t>(jobs.delta, t, g, cc, cpr, b, H, D);
   if (t >= L) return;
   const uint16_t* ap = static_cast<const uint16_t*>(fa.ptr) + b * fa.stride_b + t * fa.stride_l + 8 * g;
   const uint16_t* bp = static_cast<const uint16_t*>(fb.ptr) + b * fb.stride_b + t * fb.stride_l + 8 * cc;
@@ -396,15 +467,15 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(DenseParams p) {
 // One workgroup (256 threads) per token: da[r, h] and db[r, d] from the token's dense gradient
 // dX[h, d].  With STAGE the token's dX (row stride D + 1), a and b sit in LDS; each da output is
 // shared by `ns` neighbouring lanes that split the sum over d and combine with lane shuffles.
-template <typename T, bool STAGE>
+template <typename T, typename TO, bool STAGE>
 __global__ __launch_bounds__(256) void project_kernel(const float* dx, TpaFactor fa, TpaFactor fb, TpaGrad ga, TpaGrad gb, int L, int H,
                                                        int D, int R, int dsh, int nsh) {
   const int t = blockIdx.x, b = blockIdx.y;
   const float* xp = dx + ((int64_t)b * L + t) * H * D;
   const T* ap = static_cast<const T*>(fa.ptr) + b * fa.stride_b + t * fa.stride_l;
   const T* bp = static_cast<const T*>(fb.ptr) + b * fb.stride_b + t * fb.stride_l;
-  float* oa = ga.ptr + b * ga.stride_b + t * ga.stride_l;
-  float* ob = gb.ptr + b * gb.stride_b + t * gb.stride_l;
+  TO* oa = reinterpret_cast<TO*>(ga.ptr) + b * ga.stride_b + t * ga.stride_l;
+  TO* ob = reinterpret_cast<TO*>(gb.ptr) + b * gb.stride_b + t * gb.stride_l;
   const float inv = 1.f / (float)R;
   extern __shared__ __attribute__((aligned(16))) float xs[];  // [H][XS], then b[R][D], then a[R][H]
   if constexpr (STAGE) {
@@ -437,7 +508,7 @@ __global__ __launch_bounds__(256) void project_kernel(const float* dx, TpaFactor
         for (int e = 0; e < 4; ++e) acc[e] += xv[e] * av;
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ob[r * gb.stride_r + 4 * d4 + e] = acc[e] * inv;
+      for (int e = 0; e < 4; ++e) store_from_f32(ob + r * gb.stride_r + 4 * d4 + e, acc[e] * inv);
     }
     // da: ns = 1 << nsh neighbouring lanes share an output
     const int per_pass = 256 >> nsh, sub = threadIdx.x & ((1 << nsh) - 1);
@@ -452,25 +523,25 @@ __global__ __launch_bounds__(256) void project_kernel(const float* dx, TpaFactor
         acc += xv[0] * bv[0] + xv[1] * bv[1] + xv[2] * bv[2] + xv[3] * bv[3];
       }
       for (int m = (1 << nsh) >> 1; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, 64);
-      if (ok && sub == 0) oa[r * ga.stride_r + h] = acc * inv;
+      if (ok && sub == 0) store_from_f32(oa + r * ga.stride_r + h, acc * inv);
     }
   } else {
     for (int idx = threadIdx.x; idx < R * D; idx += 256) {
       const int r = idx / D, d = idx - r * D;
       float acc = 0.f;
       for (int h = 0; h < H; ++h) acc += xp[h * D + d] * load_as_f32(ap + r * fa.stride_r + h);
-      ob[r * gb.stride_r + d] = acc * inv;
+      store_from_f32(ob + r * gb.stride_r + d, acc * inv);
     }
     for (int idx = threadIdx.x; idx < R * H; idx += 256) {
       const int r = idx / H, h = idx - r * H;
       float acc = 0.f;
       for (int d = 0; d < D; ++d) acc += xp[h * D + d] * load_as_f32(bp + r * fb.stride_r + d);
-      oa[r * ga.stride_r + h] = acc * inv;
+      store_from_f32(oa + r * ga.stride_r + h, acc * inv);
     }
   }
 }
 
-// The same projections for bf16 factors with H % 8 == 0 and (D / 8) (H / 8) a power of two up to 64,
+// The same projections for factors with H % 8 == 0 and (D / 8) (H / 8) a power of two up to 64,
 // without LDS: a thread owns an 8 x 8 piece of one token's dX, rows 8 hg .. 8 hg + 7, columns 4 cc .. 4 cc + 3 of
 // the lower and of the upper half of D (pieces of D are the fastest thread index, so each of the 16 loads of a
 // piece reads whole contiguous half rows across the lanes: 12 % faster than 8 consecutive columns per thread,
@@ -482,19 +553,42 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
   return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }
-__global__ __launch_bounds__(256) void project_h8_kernel(const float* dx, TpaFactor fa, TpaFactor fb, TpaGrad ga, TpaGrad gb, int L, int H,
-                                                         int D, int R) {
+// All three arrays in one launch (blockIdx.z): at short lengths a launch of its own leaves each of them waiting for the
+// one before.  The gradients are written in the type the caller wants them in (rounded once, from the fp32 sums).
+struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R; };
+struct ProjectJobs { ProjectJob job[3]; };
+template <typename T>
+__device__ __forceinline__ f32x4 four_as_f32(const T* p) {
+  if constexpr (sizeof(T) == 2) {
+    const u32x2 x = *reinterpret_cast<const u32x2*>(p);
+    return f32x4{bf16lo_to_f32(x[0]), bf16hi_to_f32(x[0]), bf16lo_to_f32(x[1]), bf16hi_to_f32(x[1])};
+  } else {
+    return *reinterpret_cast<const f32x4*>(p);
+  }
+}
+template <typename TO>
+__device__ __forceinline__ void store_four(TO* p, f32x4 x) {
+  if constexpr (sizeof(TO) == 2) *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])};
+  else *reinterpret_cast<f32x4*>(p) = x;
+}
+template <typename T, typename TO>
+__global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H, int D) {
+  const ProjectJob j = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
+  const TpaFactor &fa = j.fa, &fb = j.fb;
+  const TpaGrad &ga = j.ga, &gb = j.gb;
+  const int L = j.L, R = j.R;
   const int cpr = D / 8, hgs = H / 8, tt = cpr * hgs;  // threads per token
   const int64_t gtid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int cc = (int)(gtid % cpr), hg = (int)(gtid / cpr % hgs);
   const int64_t tok = gtid / tt;
   const bool live = tok < L;
+  if ((int64_t)blockIdx.x * 256 / tt >= L) return;  // a whole workgroup past the end of a shorter array
   const int64_t t = live ? tok : L - 1;  // lanes past the end idle along: the reductions need whole waves
   const int b = blockIdx.y;
   const int dh = D / 2;  // a thread's eight columns: 4 cc .. 4 cc + 3 and the same in the upper half of the row
-  const float* xp = dx + (((int64_t)b * L + t) * H + 8 * hg) * D + 4 * cc;
-  const uint16_t* ap = static_cast<const uint16_t*>(fa.ptr) + b * fa.stride_b + t * fa.stride_l + 8 * hg;
-  const uint16_t* bp = static_cast<const uint16_t*>(fb.ptr) + b * fb.stride_b + t * fb.stride_l + 4 * cc;
+  const float* xp = j.dx + (((int64_t)b * L + t) * H + 8 * hg) * D + 4 * cc;
+  const T* ap = static_cast<const T*>(fa.ptr) + b * fa.stride_b + t * fa.stride_l + 8 * hg;
+  const T* bp = static_cast<const T*>(fb.ptr) + b * fb.stride_b + t * fb.stride_l + 4 * cc;
   float x[8][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -504,19 +598,14 @@ __global__ __launch_bounds__(256) void project_h8_kernel(const float* dx, TpaFac
     for (int j = 0; j < 4; ++j) { x[i][j] = lo[j]; x[i][4 + j] = hi[j]; }
   }
   const float inv = 1.f / (float)R;
-  float* oa = ga.ptr + b * ga.stride_b + t * ga.stride_l + 8 * hg;
-  float* ob = gb.ptr + b * gb.stride_b + t * gb.stride_l + 4 * cc;
+  TO* oa = reinterpret_cast<TO*>(ga.ptr) + b * ga.stride_b + t * ga.stride_l + 8 * hg;
+  TO* ob = reinterpret_cast<TO*>(gb.ptr) + b * gb.stride_b + t * gb.stride_l + 4 * cc;
   for (int r = 0; r < R; ++r) {
-    const u32x4 av = *reinterpret_cast<const u32x4*>(ap + (int64_t)r * fa.stride_r);
-    const u32x2 bl = *reinterpret_cast<const u32x2*>(bp + (int64_t)r * fb.stride_r);
-    const u32x2 bh = *reinterpret_cast<const u32x2*>(bp + (int64_t)r * fb.stride_r + dh);
-    const u32x4 bv = u32x4{bl[0], bl[1], bh[0], bh[1]};
+    const f32x4 al = four_as_f32(ap + (int64_t)r * fa.stride_r), ah = four_as_f32(ap + (int64_t)r * fa.stride_r + 4);
+    const f32x4 bl = four_as_f32(bp + (int64_t)r * fb.stride_r), bh = four_as_f32(bp + (int64_t)r * fb.stride_r + dh);
     float af[8], bf[8];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      af[2 * j] = bf16lo_to_f32(av[j]); af[2 * j + 1] = bf16hi_to_f32(av[j]);
-      bf[2 * j] = bf16lo_to_f32(bv[j]); bf[2 * j + 1] = bf16hi_to_f32(bv[j]);
-    }
+    for (int j = 0; j < 4; ++j) { af[j] = al[j]; af[4 + j] = ah[j]; bf[j] = bl[j]; bf[4 + j] = bh[j]; }
     float da[8], db[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -550,41 +639,52 @@ __global__ __launch_bounds__(256) void project_h8_kernel(const float* dx, TpaFac
       db[j] = v;
     }
     if (live && cc == 0) {
-      *reinterpret_cast<f32x4*>(oa + (int64_t)r * ga.stride_r) = f32x4{da[0] * inv, da[1] * inv, da[2] * inv, da[3] * inv};
-      *reinterpret_cast<f32x4*>(oa + (int64_t)r * ga.stride_r + 4) = f32x4{da[4] * inv, da[5] * inv, da[6] * inv, da[7] * inv};
+      store_four(oa + (int64_t)r * ga.stride_r, f32x4{da[0] * inv, da[1] * inv, da[2] * inv, da[3] * inv});
+      store_four(oa + (int64_t)r * ga.stride_r + 4, f32x4{da[4] * inv, da[5] * inv, da[6] * inv, da[7] * inv});
     }
     if (live && hg == 0) {
-      *reinterpret_cast<f32x4*>(ob + (int64_t)r * gb.stride_r) = f32x4{db[0] * inv, db[1] * inv, db[2] * inv, db[3] * inv};
-      *reinterpret_cast<f32x4*>(ob + (int64_t)r * gb.stride_r + dh) = f32x4{db[4] * inv, db[5] * inv, db[6] * inv, db[7] * inv};
+      store_four(ob + (int64_t)r * gb.stride_r, f32x4{db[0] * inv, db[1] * inv, db[2] * inv, db[3] * inv});
+      store_four(ob + (int64_t)r * gb.stride_r + dh, f32x4{db[4] * inv, db[5] * inv, db[6] * inv, db[7] * inv});
     }
   }
 }
 
+inline bool al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+// rows of whole 16-byte pieces
 template <typename T>
-void launch_project(const float* dx, const TpaFactor& fa, const TpaFactor& fb, const TpaGrad& ga, const TpaGrad& gb, int B, int L,
-                    int H, int D, int R, hipStream_t stream) {
-  if constexpr (sizeof(T) == 2) {
-    const int cpr = D / 8, hgs = H / 8, tt = cpr * hgs;
-    auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
-    const bool fast = D % 8 == 0 && H % 8 == 0 && (cpr == 8 || cpr == 16) && tt <= 64 && (tt & (tt - 1)) == 0 && al16(dx) && al16(fa.ptr) &&
-                      al16(fb.ptr) && al16(ga.ptr) && al16(gb.ptr) && fa.stride_b % 8 == 0 && fa.stride_l % 8 == 0 && fa.stride_r % 8 == 0 &&
-                      fb.stride_b % 8 == 0 && fb.stride_l % 8 == 0 && fb.stride_r % 8 == 0 && ga.stride_b % 4 == 0 && ga.stride_l % 4 == 0 &&
-                      ga.stride_r % 4 == 0 && gb.stride_b % 4 == 0 && gb.stride_l % 4 == 0 && gb.stride_r % 4 == 0;
-    const int64_t blocks = ((int64_t)L * tt + 255) / 256;
-    if (fast && blocks <= 2147483647LL) {
-      hipLaunchKernelGGL(project_h8_kernel, dim3((unsigned)blocks, B), dim3(256), 0, stream, dx, fa, fb, ga, gb, L, H, D, R);
-      return;
-    }
+bool rows16(const TpaFactor& f) {
+  constexpr int N = 16 / sizeof(T);
+  return al16(f.ptr) && f.stride_b % N == 0 && f.stride_l % N == 0 && f.stride_r % N == 0;
+}
+
+template <typename T, typename TO>
+void launch_project(const ProjectJobs& jobs, int B, int H, int dk, int dv, hipStream_t stream) {
+  const int cpr = dk / 8, hgs = H / 8, tt = cpr * hgs;
+  bool fast = dk == dv && dk % 8 == 0 && H % 8 == 0 && (cpr == 8 || cpr == 16) && tt <= 64 && (tt & (tt - 1)) == 0;
+  int lmax = 0;
+  for (const ProjectJob& j : jobs.job) {
+    const TpaFactor ga{j.ga.ptr, j.ga.stride_b, j.ga.stride_l, j.ga.stride_r}, gb{j.gb.ptr, j.gb.stride_b, j.gb.stride_l, j.gb.stride_r};
+    fast = fast && al16(j.dx) && rows16<T>(j.fa) && rows16<T>(j.fb) && rows16<TO>(ga) && rows16<TO>(gb);
+    lmax = j.L > lmax ? j.L : lmax;
   }
-  const size_t smem = ((size_t)H * (D + 4) + (size_t)R * D + (size_t)R * H) * sizeof(float);
-  int dsh = 0;
-  while ((1 << dsh) < D) ++dsh;
-  int nsh = 0;  // lanes per da output: a power of two, at most a wave, so that one pass covers the outputs if it can
-  while (nsh < 6 && (4 << nsh) * R * H <= 512 && (16 << nsh) <= D) ++nsh;
-  if (smem <= 60 * 1024 && (1 << dsh) == D && D >= 4)
-    hipLaunchKernelGGL((project_kernel<T, true>), dim3(L, B), dim3(256), smem, stream, dx, fa, fb, ga, gb, L, H, D, R, dsh, nsh);
-  else
-    hipLaunchKernelGGL((project_kernel<T, false>), dim3(L, B), dim3(256), 0, stream, dx, fa, fb, ga, gb, L, H, D, R, dsh, nsh);
+  const int64_t blocks = ((int64_t)lmax * tt + 255) / 256;
+  if (fast && blocks <= 2147483647LL) {
+    hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, 3), dim3(256), 0, stream, jobs, H, dk);
+    return;
+  }
+  for (int n = 0; n < 3; ++n) {
+    const ProjectJob& j = jobs.job[n];
+    const int D = n == 2 ? dv : dk;
+    const size_t smem = ((size_t)H * (D + 4) + (size_t)j.R * D + (size_t)j.R * H) * sizeof(float);
+    int dsh = 0;
+    while ((1 << dsh) < D) ++dsh;
+    int nsh = 0;  // lanes per da output: a power of two, at most a wave, so that one pass covers the outputs if it can
+    while (nsh < 6 && (4 << nsh) * j.R * H <= 512 && (16 << nsh) <= D) ++nsh;
+    if (smem <= 60 * 1024 && (1 << dsh) == D && D >= 4)
+      hipLaunchKernelGGL((project_kernel<T, TO, true>), dim3(j.L, B), dim3(256), smem, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, D, j.R, dsh, nsh);
+    else
+      hipLaunchKernelGGL((project_kernel<T, TO, false>), dim3(j.L, B), dim3(256), 0, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, D, j.R, dsh, nsh);
+  }
 }
 
 template <typename T, int DMAX>
@@ -624,41 +724,41 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
   // the matrix-core kernels: bf16 ones on bf16 copies of Q, K, V; fp32 ones on the fp32 copies
   const bool mfma32 = mfma && sizeof(T) == sizeof(float);
   mfma = mfma && !mfma32;
-  if (mfma) {
-    uint16_t *q16 = reinterpret_cast<uint16_t*>(qd), *k16 = reinterpret_cast<uint16_t*>(kd), *v16 = reinterpret_cast<uint16_t*>(vd);
-    auto recon16 = [&](const TpaFactor& fa, const TpaFactor& fb, uint16_t* out, int L, int D, int R) {
-      const bool vec = sizeof(T) == 2 && !(reinterpret_cast<uintptr_t>(fb.ptr) & 15) && fb.stride_b % 8 == 0 && fb.stride_l % 8 == 0 &&
-                       fb.stride_r % 8 == 0;
-      if (vec)
-        hipLaunchKernelGGL(recon_bf16_kernel, dim3((L + kReconTokens - 1) / kReconTokens, a->B), dim3(threads), 0, stream, fa, fb, out, L, a->H, D, R, 1.f);
-      else
-        hipLaunchKernelGGL((recon_kernel<T, uint16_t>), dim3(L, a->B), dim3(threads), 0, stream, fa, fb, out, L, a->H, D, R);
-    };
-    // all three in one launch where the vectorised kernel applies (16-byte aligned factors, H % 8 == 0)
-    bool one_launch = sizeof(T) == 2 && a->H % 8 == 0 && a->dk % 8 == 0 && a->dk == a->dv;
-    const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
-    for (const TpaFactor* f : fs)
-      one_launch = one_launch && !(reinterpret_cast<uintptr_t>(f->ptr) & 15) && f->stride_b % 8 == 0 && f->stride_l % 8 == 0 && f->stride_r % 8 == 0;
-    const int lmax = a->lq > a->lk ? a->lq : a->lk;
-    const int64_t blocks = ((int64_t)lmax * (a->dk / 8) * (a->H / 8) + 255) / 256;
-    if (one_launch && blocks <= 2147483647LL) {
-      ReconJobs jobs{};
-      jobs.job[0] = ReconJob{a->qa, a->qb, q16, a->lq, a->rq, 1.f};
-      jobs.job[1] = ReconJob{a->ka, a->kb, k16, a->lk, a->rk, 1.f};
-      jobs.job[2] = ReconJob{a->va, a->vb, v16, a->lk, a->rk, 1.f};
-      hipLaunchKernelGGL(recon_bf16_h8_kernel, dim3((unsigned)blocks, a->B, 3), dim3(256), 0, stream, jobs, a->H, a->dk);
-    } else {
-      recon16(a->qa, a->qb, q16, a->lq, a->dk, a->rq);
-      recon16(a->ka, a->kb, k16, a->lk, a->dk, a->rk);
-      recon16(a->va, a->vb, v16, a->lk, a->dv, a->rk);
-    }
+  // dense Q, K, V and delta in one launch where the vectorised kernels apply (16-byte aligned arrays, H % 8 == 0, a row
+  // of D on 8, 16 or 32 lanes)
+  const int cpr = a->dk * (int)sizeof(T) / 16;
+  bool one_launch = (mfma || mfma32) && a->H % 8 == 0 && a->dk == a->dv && cpr >= 8 && cpr <= 32 && (cpr & (cpr - 1)) == 0 &&
+                    a->dk * sizeof(T) % 16 == 0 && al16(a->o) && al16(a->d_o);
+  const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
+  for (const TpaFactor* f : fs) one_launch = one_launch && rows16<T>(*f);
+  const int lmax = a->lq > a->lk ? a->lq : a->lk;
+  const int64_t blocks = ((int64_t)lmax * cpr * (a->H / 8) + 255) / 256;
+  if (one_launch && blocks <= 2147483647LL) {
+    ReconJobs jobs{};
+    jobs.job[0] = ReconJob{a->qa, a->qb, qd, a->lq, a->rq, 1.f};
+    jobs.job[1] = ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
+    jobs.job[2] = ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
+    jobs.delta = DeltaJob{a->o, a->d_o, delta, a->lq};
+    if constexpr (sizeof(T) == 2) hipLaunchKernelGGL(recon_bf16_h8_kernel, dim3((unsigned)blocks, a->B, 4), dim3(256), 0, stream, jobs, a->H, a->dk);
+    else hipLaunchKernelGGL(recon_f32_h8_kernel, dim3((unsigned)blocks, a->B, 4), dim3(256), 0, stream, jobs, a->H, a->dk);
   } else {
-    hipLaunchKernelGGL((recon_kernel<T, float>), dim3(a->lq, a->B), dim3(threads), 0, stream, a->qa, a->qb, qd, a->lq, a->H, a->dk, a->rq);
-    hipLaunchKernelGGL((recon_kernel<T, float>), dim3(a->lk, a->B), dim3(threads), 0, stream, a->ka, a->kb, kd, a->lk, a->H, a->dk, a->rk);
-    hipLaunchKernelGGL((recon_kernel<T, float>), dim3(a->lk, a->B), dim3(threads), 0, stream, a->va, a->vb, vd, a->lk, a->H, a->dv, a->rk);
-  }
-  {
-    const int vec = a->dv % 8 == 0 && !(reinterpret_cast<uintptr_t>(a->o) & 15) && !(reinterpret_cast<uintptr_t>(a->d_o) & 15);
+    if (mfma) {
+      auto recon16 = [&](const TpaFactor& fa, const TpaFactor& fb, float* slot, int L, int D, int R) {
+        uint16_t* out = reinterpret_cast<uint16_t*>(slot);
+        if (sizeof(T) == 2 && rows16<uint16_t>(fb))
+          hipLaunchKernelGGL(recon_bf16_kernel, dim3((L + kReconTokens - 1) / kReconTokens, a->B), dim3(threads), 0, stream, fa, fb, out, L, a->H, D, R, 1.f);
+        else
+          hipLaunchKernelGGL((recon_kernel<T, uint16_t>), dim3(L, a->B), dim3(threads), 0, stream, fa, fb, out, L, a->H, D, R);
+      };
+      recon16(a->qa, a->qb, qd, a->lq, a->dk, a->rq);
+      recon16(a->ka, a->kb, kd, a->lk, a->dk, a->rk);
+      recon16(a->va, a->vb, vd, a->lk, a->dv, a->rk);
+    } else {
+      hipLaunchKernelGGL((recon_kernel<T, float>), dim3(a->lq, a->B), dim3(threads), 0, stream, a->qa, a->qb, qd, a->lq, a->H, a->dk, a->rq);
+      hipLaunchKernelGGL((recon_kernel<T, float>), dim3(a->lk, a->B), dim3(threads), 0, stream, a->ka, a->kb, kd, a->lk, a->H, a->dk, a->rk);
+      hipLaunchKernelGGL((recon_kernel<T, float>), dim3(a->lk, a->B), dim3(threads), 0, stream, a->va, a->vb, vd, a->lk, a->H, a->dv, a->rk);
+    }
+    const int vec = a->dv % 8 == 0 && al16(a->o) && al16(a->d_o);
     hipLaunchKernelGGL((delta_kernel<T>), dim3((unsigned)((nd * 16 + threads - 1) / threads)), dim3(threads), 0, stream,
                        static_cast<const T*>(a->o), static_cast<const T*>(a->d_o), delta, a->B, a->lq, a->H, a->dv, vec);
   }
@@ -682,9 +782,14 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
   }
   if (rc != TPA_OK) return rc;
 
-  launch_project<T>(dqd, a->qa, a->qb, a->dqa, a->dqb, a->B, a->lq, a->H, a->dk, a->rq, stream);
-  launch_project<T>(dkd, a->ka, a->kb, a->dka, a->dkb, a->B, a->lk, a->H, a->dk, a->rk, stream);
-  launch_project<T>(dvd, a->va, a->vb, a->dva, a->dvb, a->B, a->lk, a->H, a->dv, a->rk, stream);
+  const ProjectJobs jobs{{{dqd, a->qa, a->qb, a->dqa, a->dqb, a->lq, a->rq},
+                          {dkd, a->ka, a->kb, a->dka, a->dkb, a->lk, a->rk},
+                          {dvd, a->va, a->vb, a->dva, a->dvb, a->lk, a->rk}}};
+  if (sizeof(T) == 2 && a->grad_dtype == TPA_DTYPE_BF16) {
+    if constexpr (sizeof(T) == 2) launch_project<T, uint16_t>(jobs, a->B, a->H, a->dk, a->dv, stream);
+  } else {
+    launch_project<T, float>(jobs, a->B, a->H, a->dk, a->dv, stream);
+  }
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 

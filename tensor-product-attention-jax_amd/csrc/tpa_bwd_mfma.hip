@@ -7,13 +7,13 @@
 // roles of the MFMA operands chosen so that nothing ever goes through LDS between two
 // contractions (v_mfma_f32_32x32x16_bf16; "lane" = the accumulator column a lane owns):
 //
-//   bwd_dq_kernel   one workgroup = 256 query rows of one head, a wave owns 32 rows, lane = row
+//   dq_block        one workgroup = 256 query rows of one head, a wave owns 32 rows, lane = row
 //     S^T  = K Q^T            A = K rows (LDS),      B = Q (registers, pre-scaled), addend -lse
 //     dP^T = V dO^T           A = V rows (LDS),      B = dO (registers),            addend -delta
 //     dS^T = exp2(S^T) * dP^T  in registers, packed to bf16 in place
 //     dQ^T += K^T dS^T        A = K^T (transposed LDS reads), B = dS^T
 //
-//   bwd_dkv_kernel  one workgroup = 32 keys per wave of one head, lane = key
+//   dkv_block       one workgroup = 32 keys per wave of one head, lane = key
 //     S  = Q K^T              A = Q rows (LDS),      B = K (registers, pre-scaled), addend -lse[row]
 //     dP = dO V^T             A = dO rows (LDS),     B = V (registers; at D = 128 a per-lane LDS slot), addend -delta[row]
 //     dV^T += dO^T P          A = dO^T (transposed LDS reads), B = P
@@ -118,7 +118,7 @@ __device__ __forceinline__ f32x16 splat16(float x) {
 // dQ
 // ============================================================================================
 template <int D, int NW, int NB, bool SEG>
-__global__ __launch_bounds__(NW * 64) void bwd_dq_kernel(BwdParams p) {
+__device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
   // a wave owns NB blocks of 32 query rows: every operand fragment read from LDS feeds NB MFMAs
   constexpr int NT = NW * 64, S = tile_stride(D), CPR = D / 8, TPP = NT / CPR, NPASS = kTile / TPP;
   constexpr int NKS = D / 16, NDB = D / 32, kWQ = 32 * NB, kBQ = NW * kWQ;
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dq_kernel(BwdParams p) {
   // about the same time and find them in that XCD's L2.
   // Pairs are taken in groups of `pair_group` (launch_dq): with every pair of an XCD side by side and many pairs the
   // resident workgroups would all belong to different pairs and share nothing.
-  const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
+  const int xcd = id & 7, slot = id >> 3;
   const int per_xcd = (p.B * p.H + 7) / 8, per_group = p.pair_group * p.nblk;
   const int grp = slot / per_group, rem = slot - grp * per_group;
   const int pair_local = grp * p.pair_group + rem % p.pair_group;
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dq_kernel(BwdParams p) {
 // dK, dV
 // ============================================================================================
 template <int D, int NW, int NB, bool SEG>
-__global__ __launch_bounds__(NW * 64) void bwd_dkv_kernel(BwdParams p) {
+__device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
   // a wave owns NB blocks of 32 keys: every operand fragment read from LDS feeds NB MFMAs
   constexpr int NT = NW * 64, S = tile_stride(D), CPR = D / 8, TPP = NT / CPR, NPASS = kTile / TPP;
   constexpr int NKS = D / 16, NDB = D / 32, kWK = 32 * NB, kBK = NW * kWK;
@@ -339,8 +339,8 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkv_kernel(BwdParams p) {
   int32_t* const lds_seg = reinterpret_cast<int32_t*>(lds_ndel + 2 * kTile);  // [2][64]
   u32x4* const lds_vf = reinterpret_cast<u32x4*>(lds_seg + 2 * kTile);  // [NW][NB][NKS][64 lanes]: V of the wave's keys as B operands
 
-  // (batch, head) pairs per XCD, blocks heaviest first: see bwd_dq_kernel
-  const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
+  // (batch, head) pairs per XCD, blocks heaviest first: see dq_block
+  const int xcd = id & 7, slot = id >> 3;
   const int per_xcd = (p.B * p.H + 7) / 8, per_group = p.pair_group * p.nblk;
   const int grp = slot / per_group, rem = slot - grp * per_group;
   const int pair_local = grp * p.pair_group + rem % p.pair_group;
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkv_kernel(BwdParams p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) { s[nb][4 * vq + e] = a[e]; dp[nb][4 * vq + e] = d4[e]; }
       }
-      // the two independent chains alternate with their operands requested ahead, in a pinned order (see bwd_dq_kernel);
+      // the two independent chains alternate with their operands requested ahead, in a pinned order (see dq_block);
       // the index of the parked V fragments passes through an empty asm per row block: the compiler would otherwise keep
       // the first block's fragments for the second, which is the register pressure parking them is meant to take away
       int vf_idx = w * NB * NKS * 64 + l;  // (the index, not the pointer: a pointer out of an asm has lost its address space)
@@ -590,57 +590,45 @@ inline int pair_group_of(int per_xcd, int nblk) {
   return g < per_xcd ? g : per_xcd;
 }
 
+// Both in one launch: the dK/dV workgroups first (four products per tile against three), then the dQ ones, so that the
+// second fills the compute units that the tail of the first leaves idle.  Against two launches, forward and backward:
+// 1 x 1000 tokens, 16 heads of 128, 168 -> 127 us; 4 x 1000 194 -> 170; 4 x 4096 and longer unchanged.
+struct BwdPair { BwdParams kv, q; int n_kv; };
 template <int D, int NW, int NB, bool SEG>
-int launch_dq(const BwdParams& base, hipStream_t stream) {
-  BwdParams p = base;
-  p.nblk = (p.lq + NW * NB * 32 - 1) / (NW * NB * 32);
+__global__ __launch_bounds__(NW * 64) void bwd_dq_dkv_kernel(BwdPair p) {
+  if ((int)blockIdx.x < p.n_kv) dkv_block<D, NW, NB, SEG>(p.kv, blockIdx.x);
+  else dq_block<D, NW, NB, SEG>(p.q, blockIdx.x - p.n_kv);
+}
+
+// fills in the decomposition of `rows` rows (or keys) in blocks of `block`; the number of workgroups
+inline int64_t decompose(BwdParams& p, int rows, int block) {
+  p.nblk = (rows + block - 1) / block;
   p.npairs = p.nblk * p.B;
   const int per_xcd = (p.B * p.H + 7) / 8;
   p.pair_group = pair_group_of(per_xcd, p.nblk);
-  const int64_t nwg = (int64_t)((per_xcd + p.pair_group - 1) / p.pair_group) * p.pair_group * p.nblk * 8;
-  if (nwg > 2147483647LL) return TPA_ERR_SHAPE;
-  auto kern = bwd_dq_kernel<D, NW, NB, SEG>;
-  const size_t smem = (size_t)4 * kTile * tile_stride(D) * 2 + 2 * kTile * 4;
-  static bool configured[kMaxDevices] = {};
-  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), smem); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(NW * 64), smem, stream, p);
-  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+  return (int64_t)((per_xcd + p.pair_group - 1) / p.pair_group) * p.pair_group * p.nblk * 8;
 }
 
 template <int D, int NW, int NB, bool SEG>
-int launch_dkv(const BwdParams& base, hipStream_t stream) {
-  BwdParams p = base;
-  p.nblk = (p.lk + NW * NB * 32 - 1) / (NW * NB * 32);
-  p.npairs = p.nblk * p.B;
-  const int per_xcd = (p.B * p.H + 7) / 8;
-  p.pair_group = pair_group_of(per_xcd, p.nblk);
-  const int64_t nwg = (int64_t)((per_xcd + p.pair_group - 1) / p.pair_group) * p.pair_group * p.nblk * 8;
-  if (nwg > 2147483647LL) return TPA_ERR_SHAPE;
-  auto kern = bwd_dkv_kernel<D, NW, NB, SEG>;
+int launch(const BwdParams& base, hipStream_t stream) {
+  BwdPair p{base, base, 0};
+  const int64_t n_kv = decompose(p.kv, base.lk, NW * NB * 32), n_q = decompose(p.q, base.lq, NW * NB * 32);
+  if (n_kv + n_q > 2147483647LL) return TPA_ERR_SHAPE;
+  p.n_kv = (int)n_kv;
+  auto kern = bwd_dq_dkv_kernel<D, NW, NB, SEG>;
   const size_t smem = (size_t)4 * kTile * tile_stride(D) * 2 + 6 * kTile * 4 + (dkv_v_in_lds(D) ? (size_t)NW * NB * (D / 16) * 64 * 16 : 0);
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), smem); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(NW * 64), smem, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_kv + n_q)), dim3(NW * 64), smem, stream, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
 template <int D>
 int launch_both(const BwdParams& p, hipStream_t stream) {
-  // dK/dV: 8 waves of 32 keys.  (64 keys per wave would halve the LDS reads per MFMA, but its 384
-  // stationary registers at D = 128 leave the compiler spilling.)
-  // (measured at D = 128: the dQ kernel with 4 waves of 64 rows, one wave per SIMD and 512 registers, takes
-  // 922 us where 8 waves of 32 rows take 401 us)
-  constexpr int NW = 8, NB = 1;
-  constexpr int QNW = 8, QNB = 1;
-  int rc;
-  if (p.qseg) {
-    rc = launch_dq<D, QNW, QNB, true>(p, stream);
-    if (rc == TPA_OK) rc = launch_dkv<D, NW, NB, true>(p, stream);
-  } else {
-    rc = launch_dq<D, QNW, QNB, false>(p, stream);
-    if (rc == TPA_OK) rc = launch_dkv<D, NW, NB, false>(p, stream);
-  }
-  return rc;
+  // 8 waves of 32 rows or keys.  (64 keys per wave would halve the LDS reads per MFMA, but its 384
+  // stationary registers at D = 128 leave the compiler spilling; the dQ kernel with 4 waves of 64 rows, one
+  // wave per SIMD and 512 registers, takes 922 us where 8 waves of 32 rows take 401 us.)
+  return p.qseg ? launch<D, 8, 1, true>(p, stream) : launch<D, 8, 1, false>(p, stream);
 }
 
 }  // namespace

@@ -24,7 +24,7 @@ KERNEL_AUTO = 0
 KERNEL_GENERIC = 1
 KERNEL_MFMA = 2
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 
 class TpaFactor(ctypes.Structure):
@@ -134,6 +134,7 @@ class TpaBwdArgs(ctypes.Structure):
         ("workspace", ctypes.c_void_p),
         ("workspace_bytes", ctypes.c_size_t),
         ("causal_offset", ctypes.c_int32),
+        ("grad_dtype", ctypes.c_int32),
     ]
 
 
