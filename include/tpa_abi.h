@@ -107,7 +107,7 @@ typedef struct TpaFwdArgs {
   int32_t kernel; /* TPA_KERNEL_* */
   void* workspace;        /* required by tpa_decode (split partials); optional for tpa_fwd (tpa_fwd_workspace_bytes) */
   size_t workspace_bytes; /* size of workspace */
-  int32_t num_splits;     /* tpa_decode only: 0 = choose; otherwise the number of key ranges */
+  int32_t num_splits;     /* 0 = choose; otherwise the number of key ranges (tpa_decode; tpa_fwd where it splits the keys) */
   const int32_t* kv_lengths; /* [B] or NULL: batch entry b attends to its first min(kv_lengths[b], lk) keys only,
                                 the rest of its k / v arrays is not read (sequences of different lengths in one
                                 padded cache; 0 = no key: o = NaN, lse = -inf).  No counterpart in the reference,
@@ -318,6 +318,13 @@ int tpa_fwd(const TpaFwdArgs* args, void* stream);
  * reconstructs them per pair of blocks, tpa/tpa.py:317,364,417).
  */
 size_t tpa_fwd_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk);
+
+/*
+ * Bytes of optional workspace (256-byte aligned) that leave tpa_fwd every route it has for this problem: at least
+ * tpa_fwd_workspace_bytes(...), plus room for the partial results of key ranges where the blocks of 256 query rows
+ * alone would leave the chip partly idle (bf16, no segment ids).
+ */
+size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk);
 
 /*
  * Bytes of workspace (256-byte aligned) tpa_fwd needs with args.nomat != 0 for the split-key kernels to serve

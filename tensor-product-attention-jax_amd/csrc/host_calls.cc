@@ -30,7 +30,7 @@ using at::Tensor;
 
 // ------------------------------------------------------------------------------------------------ the C ABI, by name
 #define TPA_CALLS(X)                                                                                             \
-  X(tpa_fwd) X(tpa_decode) X(tpa_cache_append) X(tpa_bwd) X(tpa_strerror) X(tpa_fwd_workspace_bytes)             \
+  X(tpa_fwd) X(tpa_decode) X(tpa_cache_append) X(tpa_bwd) X(tpa_strerror) X(tpa_fwd_workspace_bytes) X(tpa_fwd_best_workspace_bytes) \
   X(tpa_fwd_nomat_workspace_bytes) X(tpa_decode_workspace_bytes) X(tpa_cache_append_workspace_bytes) X(tpa_bwd_workspace_bytes)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -179,7 +179,7 @@ std::pair<Tensor, Tensor> run_fwd(TpaFwdArgs& a, const FwdCall& c, const at::Dev
   if (c.nomat == kNomatRankPairs || c.kernel == TPA_KERNEL_GENERIC) need = 0;
   else if (c.nomat) need = lib.tpa_fwd_nomat_workspace_bytes(a.B, a.lq, a.lk, a.H, a.dk, a.dv, a.rq, a.rk);
   else if (c.use_workspace && (dtype == at::kBFloat16 || a.lq <= 16))
-    need = lib.tpa_fwd_workspace_bytes(a.B, a.lq, a.lk, a.H, a.dk, a.dv, a.rq, a.rk);
+    need = (dtype == at::kBFloat16 ? lib.tpa_fwd_best_workspace_bytes : lib.tpa_fwd_workspace_bytes)(a.B, a.lq, a.lk, a.H, a.dk, a.dv, a.rq, a.rk);
   if (need) {
     ws = bytes_on(device, need + 256);
     a.workspace = aligned(ws, 256);

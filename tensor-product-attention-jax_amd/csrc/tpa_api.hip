@@ -138,11 +138,18 @@ size_t tpa_fwd_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int
   if (dk != dv || (dk != 64 && dk != 128)) return 0;  // the kernels that use a workspace take these head sizes only
   size_t need = 0;
   if (lq <= 16 && lk >= 1024) need = tpa_decode_workspace_bytes(B, lq, lk, H, dv, 0);
-  if (tpa_prefill_wants_dense(lq, rk)) {
+  if (tpa_prefill_wants_dense(lq, lk, rk)) {
     const size_t dense = tpa_prefill_dense_bytes(B, lq, lk, H, dk);
     if (dense > need) need = dense;
   }
   return need;
+}
+
+size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk) {
+  const size_t base = tpa_fwd_workspace_bytes(B, lq, lk, H, dk, dv, rq, rk);
+  if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0 || rk <= 0 || dk != dv || (dk != 64 && dk != 128)) return base;
+  const size_t best = tpa_prefill_best_bytes(B, lq, lk, H, dk, rk);
+  return best > base ? best : base;
 }
 
 int tpa_decode(const TpaFwdArgs* a, void* stream) {

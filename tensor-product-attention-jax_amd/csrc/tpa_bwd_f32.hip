@@ -32,7 +32,7 @@ struct BwdF32Params {
   float *dq, *dk, *dv;
   int B, lq, lk, H;
   float sm_scale;
-  int causal, coff, nblk, npairs;  // coff: with causal, row i sees keys <= i + coff
+  int causal, coff, nblk, npairs, groups;  // coff: with causal, row i sees keys <= i + coff; groups: see pair_of_workgroup
 };
 
 template <int D>
@@ -42,15 +42,6 @@ struct BwdLds {
   // two matrices double buffered, then per buffer: lse2[64], delta[64], segment ids[64]
   static constexpr size_t kBytes = (size_t)(4 * kMat + 2 * 3 * kTile) * 4;
 };
-
-// which (block, batch, head): heads of one (block, batch) pair on one XCD, pairs in launch order
-__device__ __forceinline__ bool decode_block(int npairs, int H, int B, int& pair, int& h) {
-  const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-  const int round = slot / H;
-  pair = round * 8 + xcd_pair_slot(round, xcd, B);
-  h = slot % H;
-  return pair < npairs;
-}
 
 // The 64 x D tile of dense X[b, row0 .., h, :] that `issue` fetched, into LDS; rows >= nrows as zeros.
 template <int D>
@@ -154,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dq_kernel(BwdF32Params p) {
   int32_t* const lds_seg = reinterpret_cast<int32_t*>(smem_bwd_f32 + 4 * kMat);  // [2][kTile] key segment ids
 
   int pair, h;
-  if (!decode_block(p.npairs, p.H, p.B, pair, h)) return;
+  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int blk = p.nblk - 1 - pair / p.B;  // heaviest causal blocks first
   const int b = pair % p.B;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
@@ -254,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dkv_kernel(BwdF32Params p) {
   float* const lds_row = smem_bwd_f32 + 4 * kMat;  // [2][lse2 | delta | segment id][kTile]
 
   int pair, h;
-  if (!decode_block(p.npairs, p.H, p.B, pair, h)) return;
+  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int blk = pair / p.B;  // under the causal mask the first key blocks see the most rows: heaviest first
   const int b = pair % p.B;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
@@ -456,7 +447,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dq_split_kernel(BwdF32Par
   constexpr int NDB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
   int pair, h;
-  if (!decode_block(p.npairs, p.H, p.B, pair, h)) return;
+  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int blk = p.nblk - 1 - pair / p.B, b = pair % p.B;  // heaviest causal blocks first
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = blk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
@@ -544,7 +535,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dkv_split_kernel(BwdF32Pa
   constexpr int NDB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
   int pair, h;
-  if (!decode_block(p.npairs, p.H, p.B, pair, h)) return;
+  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int blk = pair / p.B, b = pair % p.B;  // under the causal mask the first key blocks see the most rows: heaviest first
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int k0 = blk * 32, key = k0 + i, key_ld = min(key, p.lk - 1);
@@ -651,8 +642,9 @@ template <typename K>
 int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int block, size_t lds, BwdF32Params p, hipStream_t stream) {
   p.nblk = (rows + block - 1) / block;
   p.npairs = p.nblk * p.B;
+  p.groups = head_groups(p.npairs, p.H);
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(((p.npairs + 7) / 8) * 8 * p.H), dim3(kThreads), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)workgroups_of(p.npairs, p.H, p.groups)), dim3(kThreads), lds, stream, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 

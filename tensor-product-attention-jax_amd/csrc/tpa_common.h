@@ -184,6 +184,28 @@ __device__ __forceinline__ int xcd_pair_slot(int round, int xcd, int B) {
   return 7 - xcd;
 }
 
+// Workgroup id -> (block, batch) pair and head for the kernels whose heads share the pair's B factors: the heads of a
+// pair sit on one XCD (workgroup ids are dealt round-robin to the eight) and find the factors in its L2.  With fewer than
+// eight pairs, or a number that leaves some XCDs a round more than others, that would idle XCDs - one pair of 64 heads ran
+// on 32 of 256 compute units - so the heads then go in `groups` groups that are placed like pairs of their own.
+__device__ __forceinline__ bool pair_of_workgroup(int id, int npairs, int H, int B, int groups, int& pair, int& h) {
+  const int xcd = id & 7, slot = id >> 3, per_group = H / groups;
+  const int round = slot / per_group, x = round * 8 + xcd_pair_slot(round, xcd, B * groups);
+  pair = x / groups;
+  h = x % groups * per_group + slot % per_group;
+  return x < npairs * groups;
+}
+inline int head_groups(int64_t npairs, int H) {
+  if (npairs >= 64) return 1;  // the last round is a small part of the launch
+  int groups = 1;
+  for (int g = 1; g <= 8 && H % g == 0; g *= 2) {
+    groups = g;
+    if (npairs * g % 8 == 0) break;
+  }
+  return groups;
+}
+inline int64_t workgroups_of(int64_t npairs, int H, int groups) { return (npairs * groups + 7) / 8 * 8 * (H / groups); }
+
 // Causal offset of a forward call as the kernels take it: row i sees keys <= i + offset.  Offsets
 // of lk and more mask nothing and offsets of -lq and less mask everything, so the value is clamped
 // to that range (keeps the kernels' index arithmetic far from overflow); 0 without the causal mask.
@@ -254,7 +276,8 @@ int dense_bwd_f32_launch(const float* q, const float* k, const float* v, const f
 size_t tpa_bwd_workspace_size(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t dk, int64_t dv);
 size_t mha_bwd_workspace_size(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t dk, int64_t dv, int dtype);
 size_t tpa_prefill_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D);
-int tpa_prefill_wants_dense(int64_t lq, int64_t rk);
+int tpa_prefill_wants_dense(int64_t lq, int64_t lk, int64_t rk);
+size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk);
 // dense bf16 X[B, L, H, D] = (scale/R) sum_r a_r (x) b_r from bf16 factors
 int tpa_recon_dense_bf16(const TpaFactor* fa, const TpaFactor* fb, uint16_t* out, int B, int L, int H, int D, int R, float scale, hipStream_t stream);
 // dense Q (times q_scale), K, V of a forward call in one launch; TPA_ERR_UNSUPPORTED where the vectorised kernel does not apply

@@ -55,6 +55,12 @@ struct PrefillParams {
   int npairs;  // nqb * B
   int q_scaled;   // dense loader only: 1 = q already holds sm_scale * log2(e) * Q (it was reconstructed with that factor)
   int pair_group; // dense loader only: (batch, head) pairs of an XCD whose query blocks run side by side (see the kernel)
+  int head_groups; // factor loaders only: see pair_of_workgroup
+  // key ranges per query block (1: none).  nqb then counts (query block, range) and a workgroup's result goes, not
+  // normalised, to part_o [S][B, lq, H, D] with the reference (log2 domain; -inf: no key seen) and the sum in part_ml
+  int S;
+  float* part_o;
+  float2* part_ml;  // [S][B, lq, H]
 };
 
 // LDS: three buffers of a K tile (tile j is read while tile j+1 is already there for waves that run
@@ -102,7 +108,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int V>
 using IC = std::integral_constant<int, V>;
 
-template <int D, int LOADER, bool SEG>
+template <int D, int LOADER, bool SEG, bool SPLIT>
 __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // row blocks per wave: the per-wave state below is indexed by row block, and one is what fits 256 registers
   // (two per wave on four waves of 512 registers were slower: one wave per SIMD issues too slowly)
@@ -122,9 +128,9 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // scalars out of the argument block (never take the address of the block itself)
   struct Fac { const uint16_t* ptr; int64_t stride_b; int stride_l, stride_r; };
   auto fac = [](const TpaFactor& f) { return Fac{static_cast<const uint16_t*>(f.ptr), f.stride_b, (int)f.stride_l, (int)f.stride_r}; };
-  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; uint16_t* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs, q_scaled, pair_group; } const p = {
+  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; uint16_t* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs, q_scaled, pair_group, head_groups, S; } const p = {
       fac(pp.qa), fac(pp.qb), fac(pp.ka), fac(pp.kb), fac(pp.va), fac(pp.vb), pp.qseg, pp.kvseg, pp.kvlen, pp.o, pp.lse, pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk,
-      pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.q_scaled, pp.pair_group};
+      pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.q_scaled, pp.pair_group, pp.head_groups, SPLIT ? pp.S : 1};
 
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   auto lds_k = [&](int buf) __attribute__((always_inline)) { return smem + L::k_off(buf); };    // [kTK][KS]
@@ -132,11 +138,8 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   auto lds_a = [&](int buf) __attribute__((always_inline)) { return smem + L::a_off(buf); };    // [K|V][kTK][2]
   auto lds_seg = [&](int buf) __attribute__((always_inline)) { return reinterpret_cast<int32_t*>(smem + L::seg_off(buf)); };  // [kTK]
 
-  // ---- which (query block, batch, head): heads of one (block, batch) pair sit on one XCD
-  // (workgroup ids are dealt round-robin to the 8 XCDs) so they share the B-factor tiles in
-  // that XCD's L2; pairs are ordered heaviest (last causal block) first.
+  // ---- which (query block, batch, head); (block, batch) pairs are ordered heaviest (last causal block) first
   const int id = blockIdx.x;
-  const int xcd = id & 7, slot = id >> 3;
   int h, b, qblk;
   if constexpr (LOADER == LOAD_DENSE) {
     // Dense K and V belong to one (batch, head): what workgroups can share is the K/V stream of
@@ -146,6 +149,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     // neighbouring query blocks of a few pairs, which walk the same tiles at about the same time and
     // find them in that XCD's L2 (with every pair of the XCD in one group and many pairs, the resident
     // workgroups would all belong to different pairs and every tile would come from memory).
+    const int xcd = id & 7, slot = id >> 3;
     const int per_xcd = (p.B * p.H + 7) / 8;
     const int per_group = p.pair_group * p.nqb;
     const int grp = slot / per_group, rem = slot - grp * per_group;
@@ -156,12 +160,16 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     b = bh / p.H;
     h = bh % p.H;
   } else {
-    const int round = slot / p.H;
-    const int pair = round * 8 + xcd_pair_slot(round, xcd, p.B);
-    h = slot % p.H;
-    if (pair >= p.npairs) return;
+    int pair;
+    if (!pair_of_workgroup(id, p.npairs, p.H, p.B, p.head_groups, pair, h)) return;
     qblk = p.nqb - 1 - pair / p.B;
     b = pair % p.B;
+  }
+
+  int range = 0;
+  if constexpr (SPLIT) {
+    range = qblk % p.S;
+    qblk /= p.S;
   }
 
   const int tid = threadIdx.x;
@@ -276,7 +284,16 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // query with the last key
   const int coff = p.coff + (p.causal == TPA_CAUSAL_BOTTOM_RIGHT ? len_b - p.lq : 0);
   int kend = p.causal ? min(len_b, min(q0 + kBQ, p.lq) + coff) : len_b;
-  if (kend <= 0) {  // no key at all: the rows end as NaN / -inf (tpa/tpa.py:437-439)
+  if constexpr (SPLIT) {  // this workgroup's share of the block's tiles
+    const int all = kend > 0 ? (kend + kTK - 1) / kTK : 0;
+    const int t0 = (int)((int64_t)all * range / p.S), t1 = (int)((int64_t)all * (range + 1) / p.S);
+    if (t0 == t1) {
+      if (tid < kBQ && q0 + tid < p.lq) pp.part_ml[(((int64_t)range * p.B + b) * p.lq + q0 + tid) * p.H + h] = float2{-INFINITY, 0.f};
+      return;
+    }
+    kpos0 = t0 * kTK;
+    kend = min(kend, t1 * kTK);
+  } else if (kend <= 0) {  // no key at all: the rows end as NaN / -inf (tpa/tpa.py:437-439)
 #pragma unroll
     for (int r = 0; r < RB; ++r)
       if (qrow[r] < p.lq) {
@@ -1026,6 +1043,19 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   static_for<RB>([&](auto r_c) __attribute__((always_inline)) {
     constexpr int r = decltype(r_c)::value;
     const float ltot = halves_sum(lsum[r]);
+    if constexpr (SPLIT) {
+      if (qrow[r] < p.lq) {
+        const int64_t row = (((int64_t)range * p.B + b) * p.lq + qrow[r]) * p.H + h;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int vq = 0; vq < 4; ++vq)
+            *reinterpret_cast<f32x4*>(pp.part_o + row * D + 32 * db + 8 * vq + 4 * g) =
+                f32x4{o[r][db][4 * vq], o[r][db][4 * vq + 1], o[r][db][4 * vq + 2], o[r][db][4 * vq + 3]};
+        if (g == 0) pp.part_ml[row] = float2{seen[r] ? mref[r] : -INFINITY, ltot};
+      }
+      return;
+    }
     const float inv = 1.f / ltot;
     constexpr int OS = D + 8;  // row stride (elements)
     uint16_t* const ot = smem + w * 32 * OS;
@@ -1057,6 +1087,40 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   });
 }
 
+// Merges the key ranges of a split launch: o = sum_s 2^(m_s - max m) O_s / sum_s 2^(m_s - max m) l_s, lse = ln of the
+// total (the rule of _lse_accum, tpa/tpa.py:228-242).  A thread takes 8 elements of one (row, head); all references are
+// whole numbers, so every factor is an exact power of two and the split changes no rounding but that of the fp32 sums.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const float* part_o, const float2* part_ml, uint16_t* o, float* lse, int S, int64_t rows, int lq, int H) {
+  constexpr int CPR = D / 8;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x, row = idx / CPR;  // row over (b, query row, h)
+  const int cc = (int)(idx % CPR);
+  if (row >= rows) return;
+  float m = -INFINITY;
+  for (int s = 0; s < S; ++s) m = fmaxf(m, part_ml[s * rows + row].x);
+  float acc[8] = {}, l = 0.f;
+  for (int s = 0; s < S; ++s) {
+    const float2 ml = part_ml[s * rows + row];
+    if (ml.x == -INFINITY) continue;  // this range held no key of the row: nothing was stored for it
+    const float f = __builtin_amdgcn_exp2f(ml.x - m);
+    const f32x4* at = reinterpret_cast<const f32x4*>(part_o + (s * rows + row) * D + 8 * cc);
+    const f32x4 x0 = at[0], x1 = at[1];
+    l += f * ml.y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { acc[e] += f * x0[e]; acc[4 + e] += f * x1[e]; }
+  }
+  const float inv = 1.f / l;  // no visible key: 0 * inf = NaN, as in tpa/tpa.py:437-439
+  u32x4 pk;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) pk[j] = pack_bf16(acc[2 * j] * inv, acc[2 * j + 1] * inv);
+  *reinterpret_cast<u32x4*>(o + row * D + 8 * cc) = pk;
+  if (lse && cc == 0) {
+    const int h = (int)(row % H);
+    const int64_t bi = row / H;
+    lse[(bi / lq * H + h) * lq + bi % lq] = (m + __builtin_amdgcn_logf(l)) * kLn2;
+  }
+}
+
 // (batch, head) pairs of an XCD that run side by side (dense loader): enough of them for about 64 workgroups (two
 // rounds of an XCD's 32 compute units, so that the heaviest query blocks of a group start together), as few as that
 // allows (so that the workgroups resident together are neighbouring blocks of the same pairs).  Measured, dense
@@ -1068,9 +1132,11 @@ inline int dense_pair_group(int per_xcd, int nqb) {
   return g < 1 ? 1 : g < per_xcd ? g : per_xcd;
 }
 
-template <int D, int LOADER, bool SEG = false>
+template <int D, int LOADER, bool SEG = false, bool SPLIT = false>
 int launch_prefill(const PrefillParams& p, hipStream_t stream) {
-  auto kern = prefill_kernel<D, LOADER, SEG>;
+  if constexpr (!SEG && !SPLIT)
+    if (p.S > 1) return launch_prefill<D, LOADER, SEG, true>(p, stream);
+  auto kern = prefill_kernel<D, LOADER, SEG, SPLIT>;
   constexpr size_t lds_bytes = Lds<D>::kBytes;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds_bytes); rc != TPA_OK) return rc;
@@ -1082,13 +1148,42 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
     q.pair_group = dense_pair_group(per_xcd, p.nqb);
     n = (int64_t)((per_xcd + q.pair_group - 1) / q.pair_group) * q.pair_group * p.nqb * 8;
   } else {
-    n = (int64_t)((p.npairs + 7) / 8) * 8 * p.H;
+    q.head_groups = head_groups(p.npairs, p.H);
+    n = workgroups_of(p.npairs, p.H, q.head_groups);
   }
   if (n > 2147483647LL) return TPA_ERR_SHAPE;
   dim3 grid((unsigned)n);
   hipLaunchKernelGGL(kern, grid, dim3(512), lds_bytes, stream, q);
+  if constexpr (SPLIT) {
+    if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
+    const int64_t rows = (int64_t)p.B * p.lq * p.H;
+    hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned)((rows * (D / 8) + 255) / 256)), dim3(256), 0, stream, p.part_o, p.part_ml, p.o, p.lse, p.S, rows, p.lq, p.H);
+  }
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
+
+// Key ranges per query block.  Without them a launch of fewer workgroups than compute units takes as long as the block
+// with the most tiles; with them the partial results make a trip through memory and every workgroup pays its prologue
+// again.  The choice minimises an estimate in us: 1.7 per tile (D = 128; 1.3 at D = 64), 7 per workgroup, 7 for the merge
+// and the partial results at 4 TB/s; the launch takes its rounds of 256 average workgroups, or the heaviest workgroup.
+// Measured, us without / with ranges: a chunk of 331 tokens over 2258 keys, 16 heads of 128: 97 / 73; 608 over 11433, 8
+// heads of 64: 182 / 76; one sequence of 4096 tokens, 8 heads of 64, causal: 70 / 47.
+int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, bool causal) {
+  const int64_t blocks = (lq + kBQ - 1) / kBQ, wgs = blocks * B * H;
+  const double per_tile = D == 128 ? 1.7 : 1.3, per_wg = 7.0, most = (double)((lk + kTK - 1) / kTK);
+  // tiles of an average block: under the causal mask the first one sees (lk - lq + 256) keys, the last one all
+  const double least = lk > lq ? (double)(lk - lq) / kTK : 0.0, avg = causal ? 0.5 * (least + most) + 2.0 : most;
+  if (most < 24) return 1;  // a block's own tiles take 40 us at most: little to win over the merge
+  int best = 1;
+  double best_us = 0.0;
+  for (int S = 1; S <= 16 && wgs * S <= 1024 && (S == 1 || most >= 2 * S); ++S) {
+    const double heaviest = per_wg + per_tile * (double)(((int64_t)most + S - 1) / S), all = (double)((wgs * S + 255) / 256) * (per_wg + per_tile * avg / S);
+    const double us = (heaviest > all ? heaviest : all) + (S > 1 ? 7.0 + (double)S * B * lq * H * D * 8.0 / 4e6 : 0.0);
+    if (S == 1 || us < (best == 1 ? 0.92 : 1.0) * best_us) { best = S; best_us = us; }
+  }
+  return best;
+}
+size_t split_bytes(int64_t B, int64_t lq, int64_t H, int64_t D, int64_t S) { return S > 1 ? (size_t)(S * B * lq * H * (D + 2) * 4) : 0; }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 bool factor_ok(const TpaFactor& f) {
@@ -1131,10 +1226,17 @@ size_t tpa_prefill_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int
 // reconstruction grows with the length only.  Rank 2 has a tuned rebuild in the fused kernel:
 // measured at B * H = 64, D = 128 the two routes meet at 1024 rows (51 against 52 us) and the dense
 // one wins from 2048 on (105 against 115 us; 4096: 0.32 against 0.38 ms).  Other ranks loop over
-// the ranks per tile in the fused kernel: dense from the second query block on.
-int tpa_prefill_wants_dense(int64_t lq, int64_t rk) {
-  if (rk != 2) return lq > tpa::kBQ;
+// the ranks per tile in the fused kernel: dense from the second query block on, and for one block over many keys
+// (6 x 242 rows over 14228 keys, rank 8, 32 heads of 128: 3.89 ms fused).
+int tpa_prefill_wants_dense(int64_t lq, int64_t lk, int64_t rk) {
+  if (rk != 2) return lq > tpa::kBQ || (lq > 16 && lk >= 1024);
   return lq >= 2048;
+}
+
+size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
+  const size_t dense = tpa_prefill_wants_dense(lq, lk, rk) ? tpa_prefill_dense_bytes(B, lq, lk, H, D) : 0;
+  const int s0 = tpa::choose_splits(B, lq, lk, H, D, false), s1 = tpa::choose_splits(B, lq, lk, H, D, true);
+  return dense + tpa::split_bytes(B, lq, H, D, s0 > s1 ? s0 : s1);
 }
 
 int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
@@ -1150,9 +1252,21 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
   // With a workspace Q (times sm_scale * log2 e), K and V are reconstructed once as dense bf16 and
   // the kernel runs with its plain tile loader: no workgroup rebuilds tiles from the rank factors
   // (the fused kernel does that once per 256 query rows and head).
-  const size_t dense_bytes = tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk);
-  if (tpa_prefill_wants_dense(a->lq, a->rk) && a->workspace && dense_bytes && a->workspace_bytes >= dense_bytes &&
-      !(reinterpret_cast<uintptr_t>(a->workspace) & 255)) {
+  const bool usable = a->workspace && !(reinterpret_cast<uintptr_t>(a->workspace) & 255);
+  const size_t dense_bytes = tpa_prefill_wants_dense(a->lq, a->lk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0;
+  const bool dense = usable && dense_bytes && a->workspace_bytes >= dense_bytes;
+  // what the workspace has beyond that can take the partial results of key ranges
+  p.S = 1;
+  const size_t used = dense ? dense_bytes : 0;
+  const int S = a->num_splits > 0 ? a->num_splits : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0);
+  if (usable && !p.kvseg && S > 1 && a->workspace_bytes >= used + split_bytes(a->B, a->lq, a->H, a->dk, S)) {
+    p.S = S;
+    p.part_o = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + used);
+    p.part_ml = reinterpret_cast<float2*>(p.part_o + (size_t)S * a->B * a->lq * a->H * a->dk);
+    p.nqb *= S;
+    p.npairs *= S;
+  }
+  if (dense) {
     const int64_t hd = (int64_t)a->H * a->dk;
     const size_t kv_slot = ((size_t)a->B * a->lk * hd * 2 + 255) / 256 * 256;
     uint16_t* kd = static_cast<uint16_t*>(a->workspace);
@@ -1215,6 +1329,7 @@ int mha_prefill_mfma_launch(const MhaFwdArgs* a, hipStream_t stream) {
   p.sm_scale = a->sm_scale; p.causal = a->causal ? TPA_CAUSAL_TOP_LEFT : TPA_CAUSAL_NONE; p.coff = 0;
   p.nqb = (a->lq + kBQ - 1) / kBQ;
   p.npairs = p.nqb * a->B;
+  p.S = 1;
   if (a->dk == 128) return launch_prefill<128, LOAD_DENSE>(p, stream);
   return launch_prefill<64, LOAD_DENSE>(p, stream);
 }

@@ -35,7 +35,7 @@ struct F32Params {
   float* lse;
   int B, lq, lk, H, rq, rk;
   float sm_scale;
-  int causal, coff, nqb, npairs;  // coff: with causal, row i sees keys <= i + coff
+  int causal, coff, nqb, npairs, groups;  // coff: with causal, row i sees keys <= i + coff; groups: see pair_of_workgroup
 };
 
 template <int D>
@@ -58,23 +58,17 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
 
   struct Fac { const float* ptr; int64_t stride_b, stride_l, stride_r; };
   auto fac = [](const TpaFactor& f) { return Fac{static_cast<const float*>(f.ptr), f.stride_b, f.stride_l, f.stride_r}; };
-  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; float* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs; } const p = {
+  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; float* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs, groups; } const p = {
       fac(pp.qa), fac(pp.qb), fac(pp.ka), fac(pp.kb), fac(pp.va), fac(pp.vb), pp.qseg, pp.kvseg, pp.kvlen, pp.o, pp.lse,
-      pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk, pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs};
+      pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk, pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.groups};
 
   extern __shared__ __attribute__((aligned(16))) float smem_f32[];
   float* const lds_k = smem_f32;                                         // [2][kTK][RS]
   float* const lds_v = smem_f32 + 2 * kTile;                             // [2][kTK][RS]
   int32_t* const lds_seg = reinterpret_cast<int32_t*>(smem_f32 + 4 * kTile);  // [2][kTK]
 
-  // heads of one (query block, batch) pair on one XCD (they share the B factors in its L2),
-  // heaviest causal blocks first
-  const int id = blockIdx.x;
-  const int xcd = id & 7, slot = id >> 3;
-  const int round = slot / p.H;
-  const int pair = round * 8 + xcd_pair_slot(round, xcd, p.B);
-  const int h = slot % p.H;
-  if (pair >= p.npairs) return;
+  int pair, h;
+  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;  // heaviest causal blocks first
   const int qblk = p.nqb - 1 - pair / p.B;
   const int b = pair % p.B;
 
@@ -312,11 +306,8 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
   typedef __attribute__((ext_vector_type(NDB))) float f32xN;
 
   extern __shared__ __attribute__((aligned(16))) float smem_f32_split[];
-  const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-  const int round = slot / p.H;
-  const int pair = round * 8 + xcd_pair_slot(round, xcd, p.B);
-  const int h = slot % p.H;
-  if (pair >= p.npairs) return;
+  int pair, h;
+  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int qblk = p.nqb - 1 - pair / p.B;  // heaviest causal blocks first
   const int b = pair % p.B;
 
@@ -576,8 +567,9 @@ template <typename K>
 int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int threads, size_t lds, F32Params p, hipStream_t stream) {
   p.nqb = (p.lq + rows - 1) / rows;
   p.npairs = p.nqb * p.B;
+  p.groups = head_groups(p.npairs, p.H);
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((p.npairs + 7) / 8 * 8 * p.H), dim3(threads), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)workgroups_of(p.npairs, p.H, p.groups)), dim3(threads), lds, stream, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 

@@ -249,6 +249,8 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
         lib.mha_fwd_workspace_bytes.argtypes = [ctypes.c_int32] * 6
         lib.tpa_fwd_workspace_bytes.restype = ctypes.c_size_t
         lib.tpa_fwd_workspace_bytes.argtypes = [ctypes.c_int32] * 8
+        lib.tpa_fwd_best_workspace_bytes.restype = ctypes.c_size_t
+        lib.tpa_fwd_best_workspace_bytes.argtypes = [ctypes.c_int32] * 8
         lib.tpa_fwd_nomat_workspace_bytes.restype = ctypes.c_size_t
         lib.tpa_fwd_nomat_workspace_bytes.argtypes = [ctypes.c_int32] * 8
         lib.tpa_bwd.restype = ctypes.c_int
