@@ -362,9 +362,9 @@ int tpa_decode_noalloc(const TpaFwdArgs* args, void* stream);
 /* Bytes of workspace tpa_decode needs for this problem (num_splits = 0: the default choice). */
 size_t tpa_decode_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dv, int32_t num_splits);
 
-/* Number of key ranges tpa_decode_workspace_bytes sizes the workspace for when num_splits == 0: what
-   the bf16 kernel uses, and an upper bound on what the fp32 kernel uses (it serves one query row per
-   workgroup and so asks for at most as many ranges). */
+/* Number of key ranges per batch entry that tpa_decode_workspace_bytes sizes the workspace for when
+   num_splits == 0.  An upper bound on what the kernels use: with kv_lengths (B <= 64) up to B times as many
+   ranges are dealt to the entries by their lengths; otherwise every entry gets as many as fill the chip once. */
 int32_t tpa_decode_default_splits(int32_t B, int32_t lq, int32_t lk, int32_t H);
 
 /* Dense attention forward with the layouts of tpa/mha.py:11-17 (see MhaFwdArgs). */

@@ -15,6 +15,7 @@
 // online softmax (tpa/tpa.py:389-424).  The waves are merged through LDS, the key ranges
 // through a workspace and a small second kernel, both with the rule of _lse_accum
 // (tpa/tpa.py:228-242).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -25,13 +26,17 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kRowsPerBlock = 32;
+constexpr int kMinKeys = kWaves * kRowsPerBlock / 2;  // keys of a range with one block of rank 2 per wave
+// Several query rows make the partials and their merge dearer: ranges of two blocks per wave then (step of 6 sequences of
+// 1022 .. 2048 tokens, four query tokens each: 31.9 us; 33.4 with ranges of one block).
+inline int min_keys(int lq) { return lq >= 2 ? 2 * kMinKeys : kMinKeys; }
 
 
 struct DecodeParams {
   TpaFactor qa, qb, ka, kb, va, vb;
-  float* part_o;  // [B, lq, S, H, D] fp32, unnormalised
-  float* part_m;  // [B, lq, S, H] running max (log2 domain)
-  float* part_l;  // [B, lq, S, H] sum of exp2
+  float* part_o;  // [range, lq, H, D] fp32, unnormalised; the ranges of a batch entry are neighbours
+  float* part_m;  // [range, lq, H] running max (log2 domain)
+  float* part_l;  // [range, lq, H] sum of exp2
   const int32_t* kvlen;  // [B] keys per batch entry, or null (= lk)
   const int32_t* page_table;  // paged cache: [B, pages_per_seq] physical page of each logical page
   int page_size, pages_per_seq;  // tokens per page; table row length
@@ -40,9 +45,124 @@ struct DecodeParams {
   int cbr;         // causal, last query aligned with the last key of each batch entry: climit counts from len - lq_total
   int row0;        // this call serves query rows row0 .. row0 + lq - 1 of lq_total (outputs are indexed with them)
   int lq_total;
-  int S;           // key ranges
+  int S;           // key ranges per batch entry (slots == 0)
+  int slots;       // > 0: the ranges are dealt by the batch entries' lengths, this many at most (plan_ranges)
+  int min_keys;    // slots > 0: no range shorter than this while it can be helped
   float qscale;    // sm_scale * log2(e) / (rq * rk)
 };
+
+// Key ranges dealt by length.  With one count for all batch entries a launch lasts as long as the longest entry takes,
+// and shorter ones leave their compute units early; so every entry gets as many ranges as its length asks for at one
+// common range length, the shortest one that needs no more than `slots` ranges (one workgroup per compute unit).  The
+// lengths are known on the device only, so each wave works the plan out for itself: lane = batch entry (B <= 64) for the
+// lengths, lane = candidate range length for the search.  What rounding does to a count only moves the balance: an
+// entry's blocks are dealt round-robin to whatever number of ranges it has, at least one.
+// 48 paged sequences of 2047 .. 4096 tokens (32 heads of 128, rank 2): 67.7 us with equal counts (288 workgroups), 43.4 so.
+constexpr int kMaxPlanEntries = 64;
+struct RangePlan { int S, first; };  // of batch entry `lane`: its number of ranges and the first one's index
+__device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, int min_keys) {
+  const int lane = threadIdx.x & 63;
+  const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
+  int total = len;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
+  const float shortest = fmaxf((float)total / (float)slots, (float)min_keys);
+  const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
+  const float inv = 1.f / (shortest + (longest - shortest) * (float)lane * (1.f / 63.f));
+  int count = 0;
+  for (int j = 0; j < B; ++j) count += max(1, (int)ceilf((float)__builtin_amdgcn_readlane(len, j) * inv));
+  const uint64_t fits = __ballot(count <= slots);
+  RangePlan r;
+  r.S = lane < B ? 1 : 0;
+  if (fits) {
+    const float pick = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), __builtin_ctzll(fits)));
+    if (lane < B) r.S = max(1, (int)ceilf((float)len * pick));
+  }
+  r.first = r.S;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    const int below = __shfl_up(r.first, m, 64);
+    if (lane >= m) r.first += below;
+  }
+  r.first -= r.S;
+  return r;
+}
+
+// Range index -> batch entry, its range and its number of ranges; false past the last range.
+__device__ __forceinline__ bool range_of(const DecodeParams& p, int x, int& b, int& split, int& S) {
+  if (p.slots == 0) {
+    S = p.S;
+    b = x / S;
+    split = x - b * S;
+    return x < p.B * S;
+  }
+  const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.min_keys);
+  const int lane = threadIdx.x & 63;
+  b = __popcll(__ballot(lane < p.B && plan.first <= x)) - 1;
+  S = __builtin_amdgcn_readlane(plan.S, b);
+  split = x - __builtin_amdgcn_readlane(plan.first, b);
+  return split < S;
+}
+
+// Qm^T fragments (B operand of S'^T = B_k Qm^T): lane (h, g) holds Qm[h][16 ks + 8 g + 0..7] with
+// Qm[h, :] = scale * sum_r qa[r, h] qb[r, :], itself a product of the matrix cores (rows d, columns h, contraction over
+// the ranks in steps of 16, zeros past the last).  `QRaw` holds the operands of one step as loaded, so that the loads can
+// be issued ahead of the cache's.  An accumulator column has d = 8 q + 4 g + e of its block; exchanging halves between
+// the packed words of neighbouring q gives the order of the fragments.
+// (On the vector ALU this took 8 600 of the 35 800 cycles of a decode of 1500 keys, half of them the conversions; with this
+// form and the merge of the waves in 16-byte words, 64 x 8192 keys: 112.1 -> 107.3 us.)
+template <int NDB>
+struct QRaw { uint16_t a[8], b[NDB][8]; };
+template <int NDB>
+__device__ __forceinline__ QRaw<NDB> load_q_factors(const uint16_t* ap, int64_t a_stride, const uint16_t* bp, int64_t b_stride, int r0, int rq, int g) {
+  QRaw<NDB> raw;
+  const uint16_t* pa = ap + min(r0 + 8 * g, rq - 1) * a_stride;
+  const uint16_t* pb = bp + min(r0 + 8 * g, rq - 1) * b_stride;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    raw.a[j] = *pa;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) raw.b[db][j] = pb[32 * db];
+    const bool more = r0 + 8 * g + j + 1 < rq;  // reads past the last rank repeat it and count as zero
+    pa += more ? a_stride : 0;
+    pb += more ? b_stride : 0;
+  }
+  return raw;
+}
+template <int NKS>
+__device__ __forceinline__ void finish_q_fragments(QRaw<NKS / 2> raw, const uint16_t* ap, int64_t a_stride, const uint16_t* bp, int64_t b_stride,
+                                                   int rq, float scale, int g, bf16x8 (&qf)[NKS]) {
+  constexpr int NDB = NKS / 2;
+  f32x16 acc[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[db][v] = 0.f;
+  for (int r0 = 0;;) {
+    auto operand = [&](const uint16_t (&x)[8]) {
+      u32x4 w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        w[j] = (r0 + 8 * g + 2 * j < rq ? (uint32_t)x[2 * j] : 0u) | (r0 + 8 * g + 2 * j + 1 < rq ? (uint32_t)x[2 * j + 1] << 16 : 0u);
+      return __builtin_bit_cast(bf16x8, w);
+    };
+    const bf16x8 a = operand(raw.a);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(raw.b[db]), a, acc[db], 0, 0, 0);
+    r0 += 16;
+    if (r0 >= rq) break;
+    raw = load_q_factors<NDB>(ap, a_stride, bp, b_stride, r0, rq, g);
+  }
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) {
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = pack_bf16(acc[ks / 2][8 * (ks & 1) + 2 * j] * scale, acc[ks / 2][8 * (ks & 1) + 2 * j + 1] * scale);
+    const auto even = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+    const auto odd = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    qf[ks] = __builtin_bit_cast(bf16x8, u32x4{even[0], odd[0], even[1], odd[1]});
+  }
+}
 
 template <int D>
 struct DecodeLds {
@@ -70,7 +190,6 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
 
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
 
-  const int S = p.S;
   // workgroup id -> (key range x, query row qi): ids are dealt to the 8 XCDs round-robin, and the
   // rows of one query token group read the same cache slice, so they get ids that are 8 apart
   // (same XCD, same L2) and next to each other in launch order (resident together)
@@ -80,11 +199,11 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   const int nqg = (p.lq + NQ - 1) / NQ;  // groups of NQ query rows
   const int gid = blockIdx.x, grp = gid / (8 * nqg), rem = gid - grp * 8 * nqg;
   const int qi0 = NQ * (rem >> 3), x = grp * 8 + (rem & 7);
-  if (x >= p.B * S) return;  // the grid is rounded up to whole groups of 8 ranges
-  const int b = x / S, split = x % S;
+  int b, split, S;
+  if (!range_of(p, x, b, split, S)) return;  // the grid is rounded up to whole groups of 8 ranges
   const int h0 = blockIdx.y * 32;
   const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int hl = min(h0 + i, p.H - 1);  // this lane's head (clamped: lanes past H idle along)
 
   uint16_t* lds = smem + w * DecodeLds<D>::kPerWave;
@@ -93,24 +212,23 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   uint16_t* lds_ak = lds + 2 * DecodeLds<D>::kB;
   uint16_t* lds_av = lds_ak + DecodeLds<D>::kA;
 
-  // ---- Qm^T fragments (B operand of S'^T = B_k Qm^T): lane (h, g) holds Qm[h][16ks + 8g + 0..7].
-  // Called after the first cache loads are in flight so that their latency is not exposed.
+  // ---- Qm^T fragments: requested ahead of the cache's first blocks, finished while those are in flight.
   // With one query row they stay in registers; with NQ rows wave r builds row r's fragments once
   // and parks them in LDS behind the waves' staging regions (fragment (r, ks) of lane l at
   // [(r NKS + ks) 64 + l]), from where every wave reads them as it needs them: the registers go to
   // the NQ accumulator sets instead.
   bf16x8 qf[NQ == 1 ? NKS : 1];
   u32x4* const lds_q = reinterpret_cast<u32x4*>(smem + kWaves * DecodeLds<D>::kPerWave);
-  auto build_q = [&]() {
-    const int qi = NQ == 1 ? qi0 : min(qi0 + w, p.lq - 1);
-    const uint16_t* ap = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qi * p.qa.stride_l + hl;
-    const uint16_t* bp = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qi * p.qb.stride_l + 8 * g;
+  const int qi_build = NQ == 1 ? qi0 : min(qi0 + w, p.lq - 1);
+  const uint16_t* const qa_row = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qi_build * p.qa.stride_l + hl;
+  const uint16_t* const qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qi_build * p.qb.stride_l + i;
+  auto build_q = [&](const QRaw<NDB>& raw) __attribute__((always_inline)) {
     if constexpr (NQ == 1) {
-      build_q_fragments<NKS, 6>(ap, p.qa.stride_r, bp, p.qb.stride_r, p.rq, p.qscale, qf);
+      finish_q_fragments<NKS>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, g, qf);
     } else {
       if (w < NQ) {
         bf16x8 tmp[NKS];
-        build_q_fragments<NKS, 6>(ap, p.qa.stride_r, bp, p.qb.stride_r, p.rq, p.qscale, tmp);
+        finish_q_fragments<NKS>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, g, tmp);
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) lds_q[(w * NKS + ks) * 64 + l] = __builtin_bit_cast(u32x4, tmp[ks]);
       }
@@ -242,11 +360,12 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   using Set1 = std::integral_constant<int, 1>;
   page_ahead[0] = lookup(blk_begin);
   if constexpr (NSETS == 2) page_ahead[1] = lookup(blk_begin + blk_step);
+  const QRaw<NDB> q_raw = load_q_factors<NDB>(qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, 0, p.rq, g);
   if (blk_begin < blk_end) issue(Set0{}, blk_begin);
   if constexpr (NSETS == 2) {
     if (blk_begin + blk_step < blk_end) issue(Set1{}, blk_begin + blk_step);
   }
-  build_q();
+  build_q(q_raw);
 
   auto compute = [&](int blk) {
     // ---- a_k / a_v of this lane's head for its 16 rows (rows 8q + 4g + 0..3, q = 0..3)
@@ -402,24 +521,25 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
     }
     __syncthreads();
 
-    const int64_t pbase = (((int64_t)b * p.lq + qi0 + r) * S + split) * p.H + h0;
-    for (int idx = tid; idx < nh * D; idx += kWaves * 64) {
-      const int hh = idx / D, d = idx % D;
+    const int64_t pbase = ((int64_t)x * p.lq + qi0 + r) * p.H + h0;
+    for (int idx = tid; idx < nh * (D / 4); idx += kWaves * 64) {
+      const int hh = idx / (D / 4), d = 4 * (idx % (D / 4));
       float mw[kWaves], mmax = -INFINITY;
 #pragma unroll
       for (int ww = 0; ww < kWaves; ++ww) {
         mw[ww] = reinterpret_cast<const float*>(smem + ww * DecodeLds<D>::kPerWave)[32 * RS + hh];
         mmax = fmaxf(mmax, mw[ww]);
       }
-      float acc = 0.f, lacc = 0.f;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      float lacc = 0.f;
 #pragma unroll
       for (int ww = 0; ww < kWaves; ++ww) {
         const float* ro = reinterpret_cast<const float*>(smem + ww * DecodeLds<D>::kPerWave);
         const float f = mw[ww] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[ww] - mmax);
-        acc += f * ro[hh * RS + d];
+        acc += f * *reinterpret_cast<const f32x4*>(ro + hh * RS + d);
         lacc += f * ro[32 * RS + 32 + hh];
       }
-      p.part_o[(pbase + hh) * D + d] = acc;
+      *reinterpret_cast<f32x4*>(p.part_o + (pbase + hh) * D + d) = acc;
       if (d == 0) {
         p.part_m[pbase + hh] = mmax;
         p.part_l[pbase + hh] = lacc;
@@ -459,14 +579,13 @@ __global__ __launch_bounds__(kWaves * 64) void decode_f32_kernel(DecodeParams p)
 
   extern __shared__ __attribute__((aligned(16))) float smem_dec_f32[];
 
-  const int S = p.S;
   // workgroup id -> (key range x, query row qi): ids are dealt to the 8 XCDs round-robin, and the
   // rows of one query token group read the same cache slice, so they get ids that are 8 apart
   // (same XCD, same L2) and next to each other in launch order (resident together)
   const int gid = blockIdx.x, grp = gid / (8 * p.lq), rem = gid - grp * 8 * p.lq;
   const int qi = rem >> 3, x = grp * 8 + (rem & 7);
-  if (x >= p.B * S) return;  // the grid is rounded up to whole groups of 8 ranges
-  const int b = x / S, split = x % S;
+  int b, split, S;
+  if (!range_of(p, x, b, split, S)) return;  // the grid is rounded up to whole groups of 8 ranges
   const int h0 = blockIdx.y * 32;
   const int tid = threadIdx.x;
   const int w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
@@ -664,7 +783,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_f32_kernel(DecodeParams p)
   __syncthreads();
 
   const int nh = min(32, p.H - h0);
-  const int64_t pbase = (((int64_t)b * p.lq + qi) * S + split) * p.H + h0;
+  const int64_t pbase = ((int64_t)x * p.lq + qi) * p.H + h0;
   for (int idx = tid; idx < nh * D; idx += kWaves * 64) {
     const int hh = idx / D, d = idx % D;
     float mw[kWaves], mmax = -INFINITY;
@@ -691,11 +810,16 @@ __global__ __launch_bounds__(kWaves * 64) void decode_f32_kernel(DecodeParams p)
 
 // Merge the key ranges: o = sum_s f_s O_s / (Rk sum_s f_s l_s), f_s = 2^(m_s - max m); lse = ln of the total.
 template <int D, typename TO>
-__global__ __launch_bounds__(D) void decode_merge_kernel(const float* part_o, const float* part_m, const float* part_l,
-                                                         TO* o, float* lse, int S, int H, int lq, float inv_rk, int row0, int lq_total) {
-  const int bq = blockIdx.x;  // b * lq + qi
-  const int h = blockIdx.y;
+__global__ __launch_bounds__(D) void decode_merge_kernel(DecodeParams p, TO* o, float* lse, float inv_rk) {
+  const int h = blockIdx.y, H = p.H;
   const int d = threadIdx.x;
+  const int b = blockIdx.x / p.lq, qi = blockIdx.x % p.lq;
+  int S = p.S, first = b * S;  // the batch entry's ranges
+  if (p.slots > 0) {
+    const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.min_keys);
+    S = __builtin_amdgcn_readlane(plan.S, b);
+    first = __builtin_amdgcn_readlane(plan.first, b);
+  }
   // ranges are taken eight at a time with all their loads in flight together (one round trip
   // to memory for the usual S <= 8); a running (max, sum, acc) triple carries across groups
   float mmax = -INFINITY, acc = 0.f, lacc = 0.f;
@@ -704,10 +828,10 @@ __global__ __launch_bounds__(D) void decode_merge_kernel(const float* part_o, co
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       const int s = min(s0 + q, S - 1);
-      const int64_t idx = ((int64_t)bq * S + s) * H + h;
-      ms[q] = s0 + q < S ? part_m[idx] : -INFINITY;
-      ls[q] = part_l[idx];
-      os[q] = part_o[idx * D + d];
+      const int64_t idx = ((int64_t)(first + s) * p.lq + qi) * H + h;
+      ms[q] = s0 + q < S ? p.part_m[idx] : -INFINITY;
+      ls[q] = p.part_l[idx];
+      os[q] = p.part_o[idx * D + d];
     }
     float gmax = mmax;
 #pragma unroll
@@ -724,9 +848,8 @@ __global__ __launch_bounds__(D) void decode_merge_kernel(const float* part_o, co
     mmax = gmax;
   }
   // this call's rows are row0 .. row0 + lq - 1 of the lq_total rows of o and lse
-  const int b = bq / lq, qi = bq % lq;
-  store_from_f32(o + (((int64_t)b * lq_total + row0 + qi) * H + h) * D + d, acc * inv_rk / lacc);
-  if (lse && d == 0) lse[((int64_t)b * H + h) * lq_total + row0 + qi] = (mmax + __builtin_amdgcn_logf(lacc)) * kLn2;
+  store_from_f32(o + (((int64_t)b * p.lq_total + p.row0 + qi) * H + h) * D + d, acc * inv_rk / lacc);
+  if (lse && d == 0) lse[((int64_t)b * H + h) * p.lq_total + p.row0 + qi] = (mmax + __builtin_amdgcn_logf(lacc)) * kLn2;
 }
 
 size_t workspace_bytes(int B, int lq, int H, int D, int S) {
@@ -737,95 +860,110 @@ size_t workspace_bytes(int B, int lq, int H, int D, int S) {
 // row row0; a->o and a->lse at row 0); a plain call has {0, a->lq}
 struct RowWindow { int row0, lq_total; };
 
-template <int D, int RK, bool PAGED, int NQ>
-int launch_decode_t(const TpaFwdArgs* a, int S, hipStream_t stream, RowWindow rows) {
+// How the keys are split: `S` ranges per batch entry, or (slots > 0) up to `slots` ranges dealt by length
+struct KeyRanges {
+  int S, slots;
+  int count(int B) const { return slots > 0 ? slots : B * S; }
+};
+
+template <int RK>
+DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows) {
   DecodeParams p{};
   p.qa = a->qa; p.qb = a->qb; p.ka = a->ka; p.kb = a->kb; p.va = a->va; p.vb = a->vb;
   float* ws = static_cast<float*>(a->workspace);
-  const size_t no = (size_t)a->B * a->lq * S * a->H * D;
-  const size_t nm = (size_t)a->B * a->lq * S * a->H;
+  const size_t nm = (size_t)ranges.count(a->B) * a->lq * a->H, no = nm * a->dv;
   p.part_o = ws; p.part_m = ws + no; p.part_l = ws + no + nm;
-  p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq; p.S = S;
+  p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq;
+  p.S = ranges.S; p.slots = ranges.slots;
+  p.min_keys = min_keys(a->lq);
   p.kvlen = a->kv_lengths;
   p.climit = a->causal ? causal_offset_of(a) + 1 + rows.row0 : a->lk;
   p.cbr = a->causal == TPA_CAUSAL_BOTTOM_RIGHT;
   p.row0 = rows.row0; p.lq_total = rows.lq_total;
   p.page_table = a->page_table; p.page_size = a->page_size; p.pages_per_seq = a->pages_per_seq;
   p.qscale = a->sm_scale * kLog2e / ((float)a->rq * (float)RK);
+  return p;
+}
+
+template <int D, int RK, bool PAGED, int NQ>
+int launch_decode_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
+  const DecodeParams p = decode_params<RK>(a, ranges, rows);
   auto kern = decode_kernel<D, RK, PAGED, NQ>;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), DecodeLds<D>::bytes(NQ)); rc != TPA_OK) return rc;
-  dim3 grid((a->B * S + 7) / 8 * 8 * ((a->lq + NQ - 1) / NQ), (a->H + 31) / 32);
+  dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * ((a->lq + NQ - 1) / NQ), (a->H + 31) / 32);
   hipLaunchKernelGGL(kern, grid, dim3(kWaves * 64), DecodeLds<D>::bytes(NQ), stream, p);
   if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
-  hipLaunchKernelGGL((decode_merge_kernel<D, uint16_t>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p.part_o, p.part_m, p.part_l,
-                     static_cast<uint16_t*>(a->o), a->lse, S, a->H, a->lq, 1.f / (float)RK, rows.row0, rows.lq_total);
+  hipLaunchKernelGGL((decode_merge_kernel<D, uint16_t>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p, static_cast<uint16_t*>(a->o), a->lse, 1.f / (float)RK);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
 template <int D, int RK, bool PAGED>
-int launch_decode_f32_t(const TpaFwdArgs* a, int S, hipStream_t stream, RowWindow rows) {
-  DecodeParams p{};
-  p.qa = a->qa; p.qb = a->qb; p.ka = a->ka; p.kb = a->kb; p.va = a->va; p.vb = a->vb;
-  float* ws = static_cast<float*>(a->workspace);
-  const size_t no = (size_t)a->B * a->lq * S * a->H * D, nm = (size_t)a->B * a->lq * S * a->H;
-  p.part_o = ws; p.part_m = ws + no; p.part_l = ws + no + nm;
-  p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq; p.S = S;
-  p.kvlen = a->kv_lengths;
-  p.climit = a->causal ? causal_offset_of(a) + 1 + rows.row0 : a->lk;
-  p.cbr = a->causal == TPA_CAUSAL_BOTTOM_RIGHT;
-  p.row0 = rows.row0; p.lq_total = rows.lq_total;
-  p.page_table = a->page_table; p.page_size = a->page_size; p.pages_per_seq = a->pages_per_seq;
-  p.qscale = a->sm_scale * kLog2e / ((float)a->rq * (float)RK);
+int launch_decode_f32_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
+  const DecodeParams p = decode_params<RK>(a, ranges, rows);
   auto kern = decode_f32_kernel<D, RK, PAGED>;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), DecodeF32Lds<D>::kBytes); rc != TPA_OK) return rc;
-  dim3 grid((a->B * S + 7) / 8 * 8 * a->lq, (a->H + 31) / 32);
+  dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * a->lq, (a->H + 31) / 32);
   hipLaunchKernelGGL(kern, grid, dim3(kWaves * 64), DecodeF32Lds<D>::kBytes, stream, p);
   if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
-  hipLaunchKernelGGL((decode_merge_kernel<D, float>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p.part_o, p.part_m, p.part_l,
-                     static_cast<float*>(a->o), a->lse, S, a->H, a->lq, 1.f / (float)RK, rows.row0, rows.lq_total);
+  hipLaunchKernelGGL((decode_merge_kernel<D, float>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p, static_cast<float*>(a->o), a->lse, 1.f / (float)RK);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
 template <int D, int RK>
-int launch_decode_f32(const TpaFwdArgs* a, int S, hipStream_t stream, RowWindow rows) {
+int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   if (a->page_table) {
     if (a->page_size <= 0 || (a->page_size * RK) % kRowsPerBlock != 0 ||
         (int64_t)a->pages_per_seq * a->page_size < a->lk)
       return TPA_ERR_SHAPE;
-    return launch_decode_f32_t<D, RK, true>(a, S, stream, rows);
+    return launch_decode_f32_t<D, RK, true>(a, ranges, stream, rows);
   }
-  return launch_decode_f32_t<D, RK, false>(a, S, stream, rows);
+  return launch_decode_f32_t<D, RK, false>(a, ranges, stream, rows);
 }
 
 template <int D, int RK>
-int launch_decode(const TpaFwdArgs* a, int S, hipStream_t stream, RowWindow rows) {
+int launch_decode(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   if (a->page_table) {
     // a block of 32 (token, rank) rows must not straddle pages, and the table must cover lk
     if (a->page_size <= 0 || (a->page_size * RK) % kRowsPerBlock != 0 ||
         (int64_t)a->pages_per_seq * a->page_size < a->lk)
       return TPA_ERR_SHAPE;
-    return a->lq >= 2 ? launch_decode_t<D, RK, true, 2>(a, S, stream, rows) : launch_decode_t<D, RK, true, 1>(a, S, stream, rows);
+    return a->lq >= 2 ? launch_decode_t<D, RK, true, 2>(a, ranges, stream, rows) : launch_decode_t<D, RK, true, 1>(a, ranges, stream, rows);
   }
-  return a->lq >= 2 ? launch_decode_t<D, RK, false, 2>(a, S, stream, rows) : launch_decode_t<D, RK, false, 1>(a, S, stream, rows);
+  return a->lq >= 2 ? launch_decode_t<D, RK, false, 2>(a, ranges, stream, rows) : launch_decode_t<D, RK, false, 1>(a, ranges, stream, rows);
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
+// Key ranges per batch entry that the workspace is sized for.  One workgroup per compute unit is resident (the kernel
+// keeps two blocks of loads in flight in registers), so there are as many as fill 256 of them.  A wave then has at
+// least one block of rank 2; where that would take more partials than four blocks per wave
+// and more than the fixed array of tpa_decode_noalloc holds (at head size 128), it has four.
+// (One sequence of 1500 keys, 16 heads of 128, with the merge: 17.3 us with 6 ranges of four blocks per wave, 14.1 with
+// 12 of two, 12.3 with 24 of one.)
+// The bf16 kernel serves two query rows per workgroup, which is what callers are told to size
+// the workspace for; the fp32 kernel serves one, launches twice the workgroups per range and so
+// asks for at most as many ranges (and never more workspace).
 int default_splits(int B, int lq, int lk, int H, int rows_per_group = 2) {
-  // one workgroup per CU is resident (the kernel keeps a block of loads in flight in registers),
-  // so aim for a whole number of waves of 256 workgroups and at least 4 blocks per wave.
-  // The bf16 kernel serves two query rows per workgroup, which is what callers are told to size
-  // the workspace for; the fp32 kernel serves one, launches twice the workgroups per range and so
-  // asks for at most as many ranges (and never more workspace).
-  const int groups = B * ((lq + rows_per_group - 1) / rows_per_group) * ((H + 31) / 32);
-  int S = (256 + groups - 1) / groups;
-  if (groups >= 256) S = 1;
-  const int max_s = (lk + 4 * kWaves * 16 - 1) / (4 * kWaves * 16);
-  if (S > max_s) S = max_s;
-  if (S < 1) S = 1;
-  return S;
+  const int64_t groups = (int64_t)B * ((lq + rows_per_group - 1) / rows_per_group) * ((H + 31) / 32);
+  if (groups >= 256) return 1;
+  const int want = (int)((256 + groups - 1) / groups);
+  const int few = std::min(want, (lk + 4 * kMinKeys - 1) / (4 * kMinKeys));
+  const int room = (int)(TPA_DECODE_NOALLOC_SCRATCH_BYTES / workspace_bytes(B, lq, H, 128, 1));
+  return std::max({1, few, std::min({want, (lk + kMinKeys - 1) / kMinKeys, room})});
+}
+
+// How a launch splits the keys if the caller leaves it to us, with partials for B * default_splits ranges at hand.
+// With lengths per batch entry the ranges are dealt by them; otherwise all entries get one count, which fills the chip
+// at most once: 288 workgroups take two rounds, the second nearly empty (48 x 4096 keys, 32 heads of 128: 6 ranges each 69.5 us, 5 48.6).
+KeyRanges choose_ranges(const TpaFwdArgs* a, int rows_per_group) {
+  const int S = default_splits(a->B, a->lq, a->lk, a->H, rows_per_group);
+  const int per_range = (a->lq + rows_per_group - 1) / rows_per_group * ((a->H + 31) / 32);  // workgroups of one range
+  if (a->kv_lengths && a->B <= kMaxPlanEntries)
+    return KeyRanges{S, std::min(std::max(a->B, 256 / per_range), a->B * S)};
+  const int most = (a->lk + min_keys(a->lq) - 1) / min_keys(a->lq);
+  return KeyRanges{std::max(1, (int)std::min<int64_t>(std::min(S, most), 256 / ((int64_t)a->B * per_range))), 0};
 }
 
 }  // namespace
@@ -867,25 +1005,26 @@ int tpa_decode_mfma_launch_rows(const TpaFwdArgs* a, hipStream_t stream, int row
   const RowWindow rows{row0, lq_total};
   const int S = a->num_splits > 0 ? a->num_splits : default_splits(a->B, a->lq, a->lk, a->H);
   if (S > 65535 || (int64_t)a->B * S > 2147483647LL) return TPA_ERR_SHAPE;
+  const KeyRanges ranges = a->num_splits > 0 ? KeyRanges{S, 0} : choose_ranges(a, 2);
   if (!a->workspace || a->workspace_bytes < workspace_bytes(a->B, a->lq, a->H, a->dv, S)) return TPA_ERR_WORKSPACE;
   if (!aligned16(a->workspace)) return TPA_ERR_ALIGN;
   if (a->dk == 128) {
     switch (a->rk) {
-      case 1: return launch_decode<128, 1>(a, S, stream, rows);
-      case 2: return launch_decode<128, 2>(a, S, stream, rows);
-      case 4: return launch_decode<128, 4>(a, S, stream, rows);
-      case 8: return launch_decode<128, 8>(a, S, stream, rows);
-      case 16: return launch_decode<128, 16>(a, S, stream, rows);
-      default: return launch_decode<128, 32>(a, S, stream, rows);
+      case 1: return launch_decode<128, 1>(a, ranges, stream, rows);
+      case 2: return launch_decode<128, 2>(a, ranges, stream, rows);
+      case 4: return launch_decode<128, 4>(a, ranges, stream, rows);
+      case 8: return launch_decode<128, 8>(a, ranges, stream, rows);
+      case 16: return launch_decode<128, 16>(a, ranges, stream, rows);
+      default: return launch_decode<128, 32>(a, ranges, stream, rows);
     }
   }
   switch (a->rk) {
-    case 1: return launch_decode<64, 1>(a, S, stream, rows);
-    case 2: return launch_decode<64, 2>(a, S, stream, rows);
-    case 4: return launch_decode<64, 4>(a, S, stream, rows);
-    case 8: return launch_decode<64, 8>(a, S, stream, rows);
-    case 16: return launch_decode<64, 16>(a, S, stream, rows);
-    default: return launch_decode<64, 32>(a, S, stream, rows);
+    case 1: return launch_decode<64, 1>(a, ranges, stream, rows);
+    case 2: return launch_decode<64, 2>(a, ranges, stream, rows);
+    case 4: return launch_decode<64, 4>(a, ranges, stream, rows);
+    case 8: return launch_decode<64, 8>(a, ranges, stream, rows);
+    case 16: return launch_decode<64, 16>(a, ranges, stream, rows);
+    default: return launch_decode<64, 32>(a, ranges, stream, rows);
   }
 }
 
@@ -913,25 +1052,26 @@ int tpa_decode_f32_launch_rows(const TpaFwdArgs* a, hipStream_t stream, int row0
   const RowWindow rows{row0, lq_total};
   const int S = a->num_splits > 0 ? a->num_splits : default_splits(a->B, a->lq, a->lk, a->H, 1);
   if (S > 65535 || (int64_t)a->B * S > 2147483647LL) return TPA_ERR_SHAPE;
+  const KeyRanges ranges = a->num_splits > 0 ? KeyRanges{S, 0} : choose_ranges(a, 1);
   if (!a->workspace || a->workspace_bytes < workspace_bytes(a->B, a->lq, a->H, a->dv, S)) return TPA_ERR_WORKSPACE;
   if (!aligned16(a->workspace)) return TPA_ERR_ALIGN;
   if (a->dk == 128) {
     switch (a->rk) {
-      case 1: return launch_decode_f32<128, 1>(a, S, stream, rows);
-      case 2: return launch_decode_f32<128, 2>(a, S, stream, rows);
-      case 4: return launch_decode_f32<128, 4>(a, S, stream, rows);
-      case 8: return launch_decode_f32<128, 8>(a, S, stream, rows);
-      case 16: return launch_decode_f32<128, 16>(a, S, stream, rows);
-      default: return launch_decode_f32<128, 32>(a, S, stream, rows);
+      case 1: return launch_decode_f32<128, 1>(a, ranges, stream, rows);
+      case 2: return launch_decode_f32<128, 2>(a, ranges, stream, rows);
+      case 4: return launch_decode_f32<128, 4>(a, ranges, stream, rows);
+      case 8: return launch_decode_f32<128, 8>(a, ranges, stream, rows);
+      case 16: return launch_decode_f32<128, 16>(a, ranges, stream, rows);
+      default: return launch_decode_f32<128, 32>(a, ranges, stream, rows);
     }
   }
   switch (a->rk) {
-    case 1: return launch_decode_f32<64, 1>(a, S, stream, rows);
-    case 2: return launch_decode_f32<64, 2>(a, S, stream, rows);
-    case 4: return launch_decode_f32<64, 4>(a, S, stream, rows);
-    case 8: return launch_decode_f32<64, 8>(a, S, stream, rows);
-    case 16: return launch_decode_f32<64, 16>(a, S, stream, rows);
-    default: return launch_decode_f32<64, 32>(a, S, stream, rows);
+    case 1: return launch_decode_f32<64, 1>(a, ranges, stream, rows);
+    case 2: return launch_decode_f32<64, 2>(a, ranges, stream, rows);
+    case 4: return launch_decode_f32<64, 4>(a, ranges, stream, rows);
+    case 8: return launch_decode_f32<64, 8>(a, ranges, stream, rows);
+    case 16: return launch_decode_f32<64, 16>(a, ranges, stream, rows);
+    default: return launch_decode_f32<64, 32>(a, ranges, stream, rows);
   }
 }
 
@@ -984,6 +1124,5 @@ extern "C" int tpa_decode_noalloc(const TpaFwdArgs* a, void* stream) {
   TpaFwdArgs b = *a;
   b.workspace = ptr;
   b.workspace_bytes = TPA_DECODE_NOALLOC_SCRATCH_BYTES;
-  b.num_splits = S;
   return bf16 ? tpa_decode_mfma_launch(&b, static_cast<hipStream_t>(stream)) : tpa_decode_f32_launch(&b, static_cast<hipStream_t>(stream));
 }
