@@ -353,15 +353,15 @@ __global__ __launch_bounds__(kThreads) void bwd_f32_dkv_kernel(BwdF32Params p) {
 // ---------------------------------------------------------------------------------------------
 // The same two kernels for problems with few blocks of 128 rows (or keys), whose launch leaves most of the chip idle and
 // takes as long as one workgroup walking the whole sequence (2 sequences of 1000 tokens, 8 heads of 64: 128 workgroups,
-// 112 and 160 us).  A workgroup owns 32 rows (keys) and its four waves split the streamed tiles, 32 rows each: wave w
-// takes tiles w, w + 4, ... into LDS of its own (no barrier in the loop; the next tile's rows are in flight in registers
-// meanwhile, one matrix at a time), and the four partial sums are added through LDS in a fixed order.
+// 112 and 160 us).  A workgroup owns 32 rows (keys) and its NW waves split the streamed tiles, 32 rows each: wave w
+// takes tiles w, w + NW, ... into LDS of its own (no barrier in the loop; the next tile's rows are in flight in registers
+// meanwhile, one matrix at a time), and the partial sums are added through LDS in a fixed order.
 template <int D>
 struct SplitLds {
   static constexpr int RS = D + 4;
   static constexpr int kMat = 32 * RS;
   static constexpr int kPerWave = 2 * kMat + 3 * 32;  // two matrices, then lse2 | delta | segment id of the tile's rows
-  static constexpr size_t kBytes = (size_t)kWaves * kPerWave * 4;
+  static constexpr size_t bytes(int nw) { return (size_t)nw * kPerWave * 4; }
 };
 
 // 32 rows of dense X[b, row0 .., h, :] on their way to a wave's LDS; rows past the end read as zero
@@ -429,21 +429,21 @@ template <int D>
 __device__ __forceinline__ void park(float* dst, int i, int g, const f32x16 (&acc)[D / 32]) { store_own_row<D>(dst + i * SplitLds<D>::RS, g, acc); }
 
 // dst[row0 + r, h, :] = sum over the waves of what they parked at `at`
-template <int D>
+template <int D, int NW>
 __device__ __forceinline__ void add_waves(const float* at, float* dst, int row0, int nrows, int64_t hd, int tid) {
   constexpr int CPR = D / 4;
-  for (int idx = tid; idx < 32 * CPR; idx += kThreads) {
+  for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
     const int r = idx / CPR, cc = idx % CPR;
     if (row0 + r >= nrows) break;
     f32x4 x = *reinterpret_cast<const f32x4*>(at + r * SplitLds<D>::RS + 4 * cc);
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) x += *reinterpret_cast<const f32x4*>(at + w * SplitLds<D>::kPerWave + r * SplitLds<D>::RS + 4 * cc);
+    for (int w = 1; w < NW; ++w) x += *reinterpret_cast<const f32x4*>(at + w * SplitLds<D>::kPerWave + r * SplitLds<D>::RS + 4 * cc);
     *reinterpret_cast<f32x4*>(dst + (int64_t)(row0 + r) * hd + 4 * cc) = x;
   }
 }
 
-template <int D, bool SEG>
-__global__ __launch_bounds__(kThreads, 1) void bwd_f32_dq_split_kernel(BwdF32Params p) {
+template <int D, int NW, bool SEG>
+__global__ __launch_bounds__(NW * 64, 1) void bwd_f32_dq_split_kernel(BwdF32Params p) {
   constexpr int NDB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
   int pair, h;
@@ -461,7 +461,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dq_split_kernel(BwdF32Par
   if constexpr (SEG) {
     qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
     int first, last;
-    id_window<kThreads>(p.qseg + (int64_t)b * p.lq + q0, min(32, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
+    id_window<NW * 64>(p.qseg + (int64_t)b * p.lq + q0, min(32, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
     kbeg = last < 0 ? 0 : first / 32 * 32;
     kend = last < 0 ? 0 : last + 1;
   }
@@ -500,13 +500,13 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dq_split_kernel(BwdF32Par
     next_k(w);
     arrive_k();
   }
-  for (int tile = w; tile < ntiles; tile += kWaves) {
-    const bool more = tile + kWaves < ntiles;
-    if (more) vt.issue(kbeg + 32 * (tile + kWaves), in);
+  for (int tile = w; tile < ntiles; tile += NW) {
+    const bool more = tile + NW < ntiles;
+    if (more) vt.issue(kbeg + 32 * (tile + NW), in);
     const int k0 = kbeg + 32 * tile;
     f32x16 s, dp;
     rows_dot_pair<D>(lds_k, lds_v, i, g, qf, gf, s, dp);
-    if (more) next_k(tile + kWaves);
+    if (more) next_k(tile + NW);
     const int limit = p.causal ? min(qrow + p.coff, kend - 1) : kend - 1;  // largest visible key index
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq) {
@@ -527,11 +527,11 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dq_split_kernel(BwdF32Par
   }
   park<D>(lds_k, i, g, dq);
   __syncthreads();
-  add_waves<D>(smem_bwd_f32, p.dq + (int64_t)b * p.lq * hd + (int64_t)h * D, q0, p.lq, hd, tid);
+  add_waves<D, NW>(smem_bwd_f32, p.dq + (int64_t)b * p.lq * hd + (int64_t)h * D, q0, p.lq, hd, tid);
 }
 
-template <int D, bool SEG>
-__global__ __launch_bounds__(kThreads, 1) void bwd_f32_dkv_split_kernel(BwdF32Params p) {
+template <int D, int NW, bool SEG>
+__global__ __launch_bounds__(NW * 64, 1) void bwd_f32_dkv_split_kernel(BwdF32Params p) {
   constexpr int NDB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
   int pair, h;
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dkv_split_kernel(BwdF32Pa
   if constexpr (SEG) {
     kseg = p.kvseg[(int64_t)b * p.lk + key_ld];
     int first, last;
-    id_window<kThreads>(p.kvseg + (int64_t)b * p.lk + k0, min(32, p.lk - k0), p.qseg + (int64_t)b * p.lq + rbeg, p.lq - rbeg, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
+    id_window<NW * 64>(p.kvseg + (int64_t)b * p.lk + k0, min(32, p.lk - k0), p.qseg + (int64_t)b * p.lq + rbeg, p.lq - rbeg, reinterpret_cast<int32_t*>(smem_bwd_f32), tid, first, last);
     rend = last < 0 ? rbeg : rbeg + last + 1;
     if (last >= 0) rbeg = (rbeg + first) / 32 * 32;
   }
@@ -593,9 +593,9 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dkv_split_kernel(BwdF32Pa
     next_q(w);
     arrive_q();
   }
-  for (int tile = w; tile < ntiles; tile += kWaves) {
-    const bool more = tile + kWaves < ntiles;
-    if (more) gt.issue(rbeg + 32 * (tile + kWaves), in);
+  for (int tile = w; tile < ntiles; tile += NW) {
+    const bool more = tile + NW < ntiles;
+    if (more) gt.issue(rbeg + 32 * (tile + NW), in);
     const int r0 = rbeg + 32 * tile;
     f32x16 s, dp;
     rows_dot_pair<D>(lds_q, lds_g, i, g, kf, vf, s, dp);  // lane = key, registers = rows of the tile
@@ -618,15 +618,15 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32_dkv_split_kernel(BwdF32Pa
       }
     }
     cols_accumulate32<D>(lds_g, i, g, s, dv);
-    if (more) next_q(tile + kWaves);
+    if (more) next_q(tile + NW);
     cols_accumulate32<D>(lds_q, i, g, dp, dk);
     if (more) arrive_q();
   }
   park<D>(lds_q, i, g, dk);
   park<D>(lds_g, i, g, dv);
   __syncthreads();
-  add_waves<D>(smem_bwd_f32, p.dk + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
-  add_waves<D>(smem_bwd_f32 + SplitLds<D>::kMat, p.dv + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
+  add_waves<D, NW>(smem_bwd_f32, p.dk + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
+  add_waves<D, NW>(smem_bwd_f32 + SplitLds<D>::kMat, p.dv + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
 }
 
 // Whether 32-row workgroups pay: the launch of 128-row ones leaves half of the 256 compute units idle, or fills them once
@@ -638,24 +638,38 @@ bool few_blocks(const BwdF32Params& p, int rows, int D) {
   return (int64_t)((rows + kBlock - 1) / kBlock) * p.B * p.H <= (p.causal ? 256 : 128) && (big + 64) * p.H * D * 4 < (int64_t(1) << 31);
 }
 
+// Eight waves instead of four, as in the forward (tpa_prefill_f32.hip): head size 64, a tile and a half per wave.  Forward
+// and backward, us, causal, 8 heads of 64: 1 x 400 tokens 93 -> 81, 2 x 1000 198 -> 167, 2 x 2000 622 -> 500.
+template <int D>
+bool eight_waves_pay(int streamed) { return D == 64 && streamed >= 384; }
+
 template <typename K>
-int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int block, size_t lds, BwdF32Params p, hipStream_t stream) {
+int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int block, int threads, size_t lds, BwdF32Params p, hipStream_t stream) {
   p.nblk = (rows + block - 1) / block;
   p.npairs = p.nblk * p.B;
   p.groups = head_groups(p.npairs, p.H);
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)workgroups_of(p.npairs, p.H, p.groups)), dim3(kThreads), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)workgroups_of(p.npairs, p.H, p.groups)), dim3(threads), lds, stream, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
 template <int D, bool SEG>
 int launch_pair(const BwdF32Params& p, hipStream_t stream) {
-  static bool configured[4][kMaxDevices] = {};
-  int rc = few_blocks(p, p.lq, D) ? launch_kernel(bwd_f32_dq_split_kernel<D, SEG>, configured[0], p.lq, 32, SplitLds<D>::kBytes, p, stream)
-                                  : launch_kernel(bwd_f32_dq_kernel<D, SEG>, configured[1], p.lq, kBlock, BwdLds<D>::kBytes, p, stream);
-  if (rc != TPA_OK) return rc;
-  return few_blocks(p, p.lk, D) ? launch_kernel(bwd_f32_dkv_split_kernel<D, SEG>, configured[2], p.lk, 32, SplitLds<D>::kBytes, p, stream)
-                                : launch_kernel(bwd_f32_dkv_kernel<D, SEG>, configured[3], p.lk, kBlock, BwdLds<D>::kBytes, p, stream);
+  static bool configured[6][kMaxDevices] = {};
+  auto dq = [&]() {
+    if (!few_blocks(p, p.lq, D)) return launch_kernel(bwd_f32_dq_kernel<D, SEG>, configured[1], p.lq, kBlock, kThreads, BwdLds<D>::kBytes, p, stream);
+    if constexpr (D == 64)
+      if (eight_waves_pay<D>(p.lk)) return launch_kernel(bwd_f32_dq_split_kernel<D, 8, SEG>, configured[4], p.lq, 32, 512, SplitLds<D>::bytes(8), p, stream);
+    return launch_kernel(bwd_f32_dq_split_kernel<D, 4, SEG>, configured[0], p.lq, 32, 256, SplitLds<D>::bytes(4), p, stream);
+  };
+  auto dkv = [&]() {
+    if (!few_blocks(p, p.lk, D)) return launch_kernel(bwd_f32_dkv_kernel<D, SEG>, configured[3], p.lk, kBlock, kThreads, BwdLds<D>::kBytes, p, stream);
+    if constexpr (D == 64)
+      if (eight_waves_pay<D>(p.lq)) return launch_kernel(bwd_f32_dkv_split_kernel<D, 8, SEG>, configured[5], p.lk, 32, 512, SplitLds<D>::bytes(8), p, stream);
+    return launch_kernel(bwd_f32_dkv_split_kernel<D, 4, SEG>, configured[2], p.lk, 32, 256, SplitLds<D>::bytes(4), p, stream);
+  };
+  if (int rc = dq(); rc != TPA_OK) return rc;
+  return dkv();
 }
 
 }  // namespace

@@ -286,22 +286,21 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
 // ---------------------------------------------------------------------------------------------
 // The same for problems with few blocks of 256 query rows.  Such a launch leaves most of the chip idle and its time is
 // that of one workgroup walking all keys (one sequence of 512 tokens, 8 heads of 64: 16 workgroups, 75 us).  Here a
-// workgroup owns 32 query rows and its four waves split the keys: wave w takes the tiles of 32 keys w, w + 4, ...,
+// workgroup owns 32 query rows and its NW waves split the keys: wave w takes the tiles of 32 keys w, w + NW, ...,
 // rebuilds each into LDS of its own (no barrier in the loop) with the next tile's factors on their way while the matrix
-// pipe works on this one, and the four partial results are merged through LDS with the rule of _lse_accum
+// pipe works on this one, and the partial results are merged through LDS with the rule of _lse_accum
 // (tpa/tpa.py:228-242).  Every workgroup rebuilds its tiles for 32 rows instead of 256, which is why the kernel above
 // stays the one for launches that fill the chip (`few_rows_pay` below).
-constexpr int kSplitWaves = 4;
-template <int D>
+template <int D, int NW>
 struct SplitLdsF32 {
   static constexpr int RS = D + 4;
   static constexpr int kPerWave = 2 * 32 * RS;  // K and V tile; the merge reuses the K tile (O), its last columns (m, l)
-  static constexpr size_t kBytes = (size_t)(kSplitWaves * kPerWave + 4) * 4;
+  static constexpr size_t kBytes = (size_t)(NW * kPerWave + 4) * 4;
 };
 
-template <int D, bool SEG>
-__global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(F32Params p) {
-  constexpr int RS = SplitLdsF32<D>::RS;
+template <int D, int NW, bool SEG>
+__global__ __launch_bounds__(NW * 64, 1) void prefill_f32_split_kernel(F32Params p) {
+  constexpr int RS = SplitLdsF32<D, NW>::RS;
   constexpr int NDB = D / 32, CPR = D / 4, RPI = 64 / CPR, NST = 32 / RPI;  // a load instruction of the wave takes RPI rows
   typedef __attribute__((ext_vector_type(NDB))) float f32xN;
 
@@ -314,7 +313,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = qblk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
   const bool dense = p.ka.ptr == nullptr;  // dense q, k, v: weight 1, the head's slice of the row
-  float* const lds_k = smem_f32_split + w * SplitLdsF32<D>::kPerWave;  // [32][RS]
+  float* const lds_k = smem_f32_split + w * SplitLdsF32<D, NW>::kPerWave;  // [32][RS]
   float* const lds_v = lds_k + 32 * RS;
 
   const int len_b = p.kvlen ? max(0, min(p.kvlen[b], p.lk)) : p.lk;
@@ -325,7 +324,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
     qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
     if (kend > 0) {
       int first, last;
-      id_window<kSplitWaves * 64>(p.qseg + (int64_t)b * p.lq + q0, min(32, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend,
+      id_window<NW * 64>(p.qseg + (int64_t)b * p.lq + q0, min(32, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend,
                                   reinterpret_cast<int32_t*>(smem_f32_split), tid, first, last);
       kbeg = last < 0 ? 0 : first / 32 * 32;
       kend = last < 0 ? 0 : last + 1;
@@ -347,35 +346,38 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
   };
   const Rows kb_r = rows_of(p.kb, dense ? (int64_t)h * D : 0, 4 * lc, D), vb_r = rows_of(p.vb, dense ? (int64_t)h * D : 0, 4 * lc, D);
   const Rows ka_r = dense ? kb_r : rows_of(p.ka, h, 0, 1), va_r = dense ? vb_r : rows_of(p.va, h, 0, 1);
-  f32x4 in[NST], vac[NST];  // the rows in flight (K's or V's, one rank), the sum over V's ranks
-  float wt[NST];
+  struct Flight { f32x4 x[NST]; float wt[NST]; };  // rows in flight and their weights (K's or V's, one rank)
+  Flight in;
+  f32x4 vac[NST];  // the sum over V's ranks
   int32_t seg_in = 0, seg_id = 0;  // ids of key (this lane's i) of the next tile and of this one
-  auto issue = [&](const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) {
+  auto issue_to = [&](Flight& in, const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
       const int t = kbeg + tile * 32 + q * RPI;
-      in[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb.rs, rb.voff, t * rb.sl + r * rb.sr, 0));
-      wt[q] = 1.f;
-      if (!dense) wt[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra.rs, ra.voff, t * ra.sl + r * ra.sr, 0));
+      in.x[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb.rs, rb.voff, t * rb.sl + r * rb.sr, 0));
+      in.wt[q] = 1.f;
+      if (!dense) in.wt[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra.rs, ra.voff, t * ra.sl + r * ra.sr, 0));
     }
   };
-  auto row_in = [&](int tile, int q) __attribute__((always_inline)) -> f32x4 {
-    const f32x4 x = wt[q] * inv_r * in[q];
+  auto issue = [&](const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) { issue_to(in, rb, ra, tile, r); };
+  auto row_of = [&](const Flight& in, int tile, int q) __attribute__((always_inline)) -> f32x4 {
+    const f32x4 x = in.wt[q] * inv_r * in.x[q];
     return q * RPI + lrow < kend - kbeg - tile * 32 ? x : f32x4{0.f, 0.f, 0.f, 0.f};
   };
   // K is added up in its LDS tile (free once the logits are done), V in registers until its tile has been used
-  auto take_k = [&](int tile, bool first) __attribute__((always_inline)) {
+  auto take_k_of = [&](const Flight& in, int tile, bool first) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
       f32x4* const at = reinterpret_cast<f32x4*>(lds_k + (q * RPI + lrow) * RS + 4 * lc);
-      const f32x4 x = row_in(tile, q);
+      const f32x4 x = row_of(in, tile, q);
       *at = first ? x : *at + x;
     }
   };
+  auto take_k = [&](int tile, bool first) __attribute__((always_inline)) { take_k_of(in, tile, first); };
   auto take_v = [&](int tile, bool first) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
-      const f32x4 x = row_in(tile, q);
+      const f32x4 x = row_of(in, tile, q);
       vac[q] = first ? x : vac[q] + x;
     }
   };
@@ -393,36 +395,44 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
     if (p.rk > 1) issue(rb, ra, tile, p.rk - 1);
   };
 
-  if (w < ntiles) issue(vb_r, va_r, w, 0);
-  // ---- Q (B operand of S^T = K Q^T), scaled: qf[4m + e] = c * Q[qrow][8m + 4g + e]
-  float qf[D / 2];
+  Flight in_k;  // of the first tile only: its first ranks of V and of K travel together, ahead of Q's
+  if (w < ntiles) {
+    issue(vb_r, va_r, w, 0);
+    issue_to(in_k, kb_r, ka_r, w, 0);
+  }
+  // ---- Q, scaled, through LDS (the waves' tiles are not in use yet): the 32 rows are the same for all waves, and read in the
+  // layout of the operand every load of every wave would touch 32 cache lines
+  for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
+    const int row = idx / CPR, cc = idx % CPR, row_ld = min(q0 + row, p.lq - 1);
+    const float* qb = static_cast<const float*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)row_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * cc;
+    const float* qa = dense ? nullptr : static_cast<const float*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)row_ld * p.qa.stride_l + h;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int G = 6;  // ranks whose loads are in flight together
+    for (int r0 = 0; r0 < p.rq; r0 += G) {
+      f32x4 bv[G];
+      float a[G];
 #pragma unroll
-  for (int j = 0; j < D / 2; ++j) qf[j] = 0.f;
-  {
-    const float* qb = static_cast<const float*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qrow_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * g;
-    const float* qa = dense ? nullptr : static_cast<const float*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qrow_ld * p.qa.stride_l + h;
-    for (int r0 = 0; r0 < p.rq; r0 += 3) {  // three ranks in flight: the loads of one would expose their latency rank by rank
-      f32x4 bv[3][D / 8];
-      float a[3];
-#pragma unroll
-      for (int u = 0; u < 3; ++u) {
+      for (int u = 0; u < G; ++u) {
         const int r = min(r0 + u, p.rq - 1);
-        a[u] = r0 + u >= p.rq ? 0.f : dense ? 1.f : qa[r * p.qa.stride_r];
-#pragma unroll
-        for (int m = 0; m < D / 8; ++m) bv[u][m] = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r + 8 * m);
+        a[u] = dense ? 1.f : qa[r * p.qa.stride_r];
+        bv[u] = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r);
       }
 #pragma unroll
-      for (int u = 0; u < 3; ++u)
-        if (r0 + u < p.rq)
-#pragma unroll
-          for (int m = 0; m < D / 8; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) qf[4 * m + e] += a[u] * bv[u][m][e];
+      for (int u = 0; u < G; ++u)
+        if (r0 + u < p.rq) acc += a[u] * bv[u];
     }
-    const float scale = p.sm_scale * kLog2e / (float)p.rq;
-#pragma unroll
-    for (int j = 0; j < D / 2; ++j) qf[j] *= scale;
+    *reinterpret_cast<f32x4*>(smem_f32_split + row * RS + 4 * cc) = acc * (p.sm_scale * kLog2e / (float)p.rq);
   }
+  __syncthreads();
+  // B operand of S^T = K Q^T: qf[4m + e] = Q[qrow][8m + 4g + e]
+  float qf[D / 2];
+#pragma unroll
+  for (int m = 0; m < D / 8; ++m) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(smem_f32_split + i * RS + 8 * m + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qf[4 * m + e] = x[e];
+  }
+  __syncthreads();
 
   f32x16 o[NDB];
 #pragma unroll
@@ -433,15 +443,20 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
 
   if (w < ntiles) {
     ranks(vb_r, va_r, w, take_v);
-    if (p.rk > 1) take_v(w, false);
-    store_v();
-    issue(kb_r, ka_r, w, 0);
-    ranks(kb_r, ka_r, w, take_k);
-    if (p.rk > 1) take_k(w, false);
+    take_k_of(in_k, w, true);
+    for (int r = 1; r < p.rk; ++r) {
+      issue_to(in_k, kb_r, ka_r, w, r);
+      if (r == 1) {
+        take_v(w, false);
+        store_v();
+      }
+      take_k_of(in_k, w, false);
+    }
+    if (p.rk == 1) store_v();
     if constexpr (SEG) seg_id = p.kvseg[(int64_t)b * p.lk + min(kbeg + w * 32 + i, p.lk - 1)];
   }
-  for (int tile = w; tile < ntiles; tile += kSplitWaves) {
-    const int next = tile + kSplitWaves;
+  for (int tile = w; tile < ntiles; tile += NW) {
+    const int next = tile + NW;
     const bool more = next < ntiles;
     if (more) issue(vb_r, va_r, next, 0);
     f32x16 s, s2;  // two accumulation chains, added at the end
@@ -523,20 +538,20 @@ __global__ __launch_bounds__(kSplitWaves * 64, 1) void prefill_f32_split_kernel(
     lds_k[i * RS + D + 1] = ltot;
   }
   __syncthreads();
-  for (int idx = tid; idx < 32 * CPR; idx += kSplitWaves * 64) {
+  for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
     const int row = idx / CPR, cc = idx % CPR;
     if (q0 + row >= p.lq) continue;
     const float* const at = smem_f32_split + row * RS;
     float mmax = -INFINITY, lacc = 0.f;
 #pragma unroll
-    for (int ww = 0; ww < kSplitWaves; ++ww) mmax = fmaxf(mmax, at[ww * SplitLdsF32<D>::kPerWave + D]);
+    for (int ww = 0; ww < NW; ++ww) mmax = fmaxf(mmax, at[ww * SplitLdsF32<D, NW>::kPerWave + D]);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ww = 0; ww < kSplitWaves; ++ww) {
-      const float mw = at[ww * SplitLdsF32<D>::kPerWave + D];
+    for (int ww = 0; ww < NW; ++ww) {
+      const float mw = at[ww * SplitLdsF32<D, NW>::kPerWave + D];
       const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mmax);
-      acc += f * *reinterpret_cast<const f32x4*>(at + ww * SplitLdsF32<D>::kPerWave + 4 * cc);
-      lacc += f * at[ww * SplitLdsF32<D>::kPerWave + D + 1];
+      acc += f * *reinterpret_cast<const f32x4*>(at + ww * SplitLdsF32<D, NW>::kPerWave + 4 * cc);
+      lacc += f * at[ww * SplitLdsF32<D, NW>::kPerWave + D + 1];
     }
     const float inv = 1.f / lacc;  // no visible key: 0 * inf = NaN, as in tpa/tpa.py:437-439
     *reinterpret_cast<f32x4*>(p.o + (((int64_t)b * p.lq + q0 + row) * p.H + h) * D + 4 * cc) = acc * inv;
@@ -552,14 +567,23 @@ bool split_supported(const F32Params& p) {
   return true;
 }
 
+// Eight waves instead of four where a wave then still has a tile and a half: two per SIMD cover each other's waits (four
+// hold 276 registers each, so that only one fits).  At head size 64 only: at 128 the tiles of eight waves exceed the LDS.
+// Measured, us, causal, heads of 64: 1 x 400
+// tokens, 16 heads 32.1 / 23.9; 1 x 512, 8 heads 32.1 / 23.1; 2 x 1000, 8 heads 69.3 / 51.4 (a quarter of it from Q
+// through LDS); 1 x 200, 8 heads 17.6 with four.
+bool eight_waves_pay(const F32Params& p) { return p.lk >= 384; }
+
 // Rows of a workgroup: 32 (keys split over its waves), 128 or 256.  A launch of 256-row workgroups that does not fill the
 // 256 compute units takes as long as one workgroup; with 128 rows (one wave per SIMD) a tile takes half the time, which
 // pays as long as they all fit the chip at once - under the causal mask, whose heaviest workgroup is twice the average,
-// up to two rounds.  Measured, us with 256 / 128 / 32 rows: 1 x 512 tokens, 8 heads of 64 causal 75 / 41 / 32; 2 x 1000
-// 144 / 69 / 68; 4 x 1000 146 / 112 / 134, not causal 155 / 113 / 222; 8 x 1000 not causal 157 / 191 / 441.
-int rows_per_workgroup(const F32Params& p) {
+// up to two rounds.  Measured, us with 256 / 128 / 32 rows: 1 x 512 tokens, 8 heads of 64 causal 75 / 41 / 23; 2 x 1000
+// 144 / 69 / 51; not causal 4 x 1000 155 / 113 / 222, 8 x 1000 157 / 191 / 441.  32 causal rows at head size 64 also pay
+// for up to four rounds of long sequences, whose heaviest workgroup is twice the average however few there are: 4 x 1000
+// 146 / 113 / 102, 1 x 4000 489 with 256 / 294; but 1 x 512, 64 heads 64 / 65, and eight rounds: 8 x 1000 149 / 195.
+int rows_per_workgroup(const F32Params& p, int D) {
   auto wgs = [&](int rows) { return (int64_t)((p.lq + rows - 1) / rows) * p.B * p.H; };
-  if (wgs(32) <= 512 && split_supported(p)) return 32;
+  if (wgs(32) <= (D == 64 && p.causal && p.lk >= 768 ? 1024 : 512) && split_supported(p)) return 32;
   return wgs(128) <= 256 || (p.causal && wgs(256) <= 256) ? 128 : 256;
 }
 
@@ -575,9 +599,13 @@ int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int threads
 
 template <int D, bool SEG>
 int launch_f32(const F32Params& p, hipStream_t stream) {
-  static bool configured[3][kMaxDevices] = {};
-  const int rows = rows_per_workgroup(p);
-  if (rows == 32) return launch_kernel(prefill_f32_split_kernel<D, SEG>, configured[0], 32, kSplitWaves * 64, SplitLdsF32<D>::kBytes, p, stream);
+  static bool configured[4][kMaxDevices] = {};
+  const int rows = rows_per_workgroup(p, D);
+  if (rows == 32) {
+    if constexpr (D == 64)
+      if (eight_waves_pay(p)) return launch_kernel(prefill_f32_split_kernel<D, 8, SEG>, configured[3], 32, 512, SplitLdsF32<D, 8>::kBytes, p, stream);
+    return launch_kernel(prefill_f32_split_kernel<D, 4, SEG>, configured[0], 32, 256, SplitLdsF32<D, 4>::kBytes, p, stream);
+  }
   if (rows == 128) return launch_kernel(prefill_f32_kernel<D, kNW / 2, SEG>, configured[1], 128, kNW * 32, LdsF32<D>::kBytes, p, stream);
   return launch_kernel(prefill_f32_kernel<D, kNW, SEG>, configured[2], 256, kNW * 64, LdsF32<D>::kBytes, p, stream);
 }
