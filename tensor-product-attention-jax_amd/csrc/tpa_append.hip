@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256) void append_mfma_kernel(AppendParams p) {
 // that are 8 apart (same XCD: its L2 serves their x tiles).
 // WB = blocks of 32 per wave and dimension: 4 (the tile described above) or 2 (128 x 128 tiles, a wave owns
 // 64 x 64, 4 fragment reads per 4 MFMAs) for chunks too small to fill the chip with the large tiles.
-// KS = groups of four waves that share the contraction of one tile.  The small tiles leave a compute unit one workgroup, and
+// KS = groups of four waves that share the contraction of one tile.  Up to 256 small tiles leave a compute unit one workgroup, and
 // a k step of theirs is shorter than the way of a load from the L2 (0.87 us per step of 0.2 us of matrix work): two groups
 // take half of the steps each, side by side in their own buffers, the sums meet in LDS, and loads are two steps ahead
 // instead of one.  2048 tokens x 1600 columns, d_model 4096: 56 -> 45.5 us.
@@ -707,8 +707,11 @@ extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
   } else if (mfma && gemm_tiles_pay<4>(p, a)) {
     if (int rc = launch_gemm<4, 1>(p, s); rc != TPA_OK) return rc;
   } else if (mfma && gemm_tiles_pay<2>(p, a)) {
-    // two groups of waves need an even number of k steps
-    if (int rc = p.K % (2 * kGK) == 0 ? launch_gemm<2, 2>(p, s) : launch_gemm<2, 1>(p, s); rc != TPA_OK) return rc;
+    // Two groups of waves need an even number of k steps, and an XCD that holds all its tiles at once (whole rows of column
+    // tiles on 32 compute units): with their buffers a compute unit holds one tile, with those of one group two.  d_model
+    // 4096, us with one / two groups: 2048 tokens x 1600 columns (26 tiles per XCD) 56 / 45.5, 3178 x 1120 (36) 69 / 75.
+    const int per_xcd = ((p.M + 127) / 128 + 7) / 8 * ((p.N + 127) / 128);
+    if (int rc = p.K % (2 * kGK) == 0 && per_xcd <= 32 ? launch_gemm<2, 2>(p, s) : launch_gemm<2, 1>(p, s); rc != TPA_OK) return rc;
   } else if (mfma) {
     dim3 grid((p.N + kBN - 1) / kBN, (p.M + kBM - 1) / kBM);
     if (grid.y > 65535) return TPA_ERR_SHAPE;
