@@ -69,9 +69,13 @@ __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, in
   const float shortest = fmaxf((float)total / (float)slots, (float)min_keys);
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
   const float inv = 1.f / (shortest + (longest - shortest) * (float)lane * (1.f / 63.f));
-  int count = 0;
-  for (int j = 0; j < B; ++j) count += max(1, (int)ceilf((float)__builtin_amdgcn_readlane(len, j) * inv));
-  const uint64_t fits = __ballot(count <= slots);
+  // eight entries at a time, their chains side by side (lanes past the last entry hold length 0 and count 1)
+  int count[8] = {}, j0 = 0;
+  for (; j0 < B; j0 += 8)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) count[j] += max(1, (int)ceilf((float)__builtin_amdgcn_readlane(len, j0 + j) * inv));
+  const int total_count = ((count[0] + count[1]) + (count[2] + count[3])) + ((count[4] + count[5]) + (count[6] + count[7])) - (j0 - B);
+  const uint64_t fits = __ballot(total_count <= slots);
   RangePlan r;
   r.S = lane < B ? 1 : 0;
   if (fits) {
@@ -820,33 +824,40 @@ __global__ __launch_bounds__(D) void decode_merge_kernel(DecodeParams p, TO* o, 
     S = __builtin_amdgcn_readlane(plan.S, b);
     first = __builtin_amdgcn_readlane(plan.first, b);
   }
-  // ranges are taken eight at a time with all their loads in flight together (one round trip
-  // to memory for the usual S <= 8); a running (max, sum, acc) triple carries across groups
+  // ranges are taken eight at a time with all their loads in flight together (one round trip to memory), or 24 at a
+  // time where all entries have the same number of more than eight (one sequence of 1500 keys in 24 ranges, with the decode:
+  // 11.6 -> 10.6 us; ranges dealt by length, 6 x 4 rows of about 21: 4.5 us eight at a time, 5.4 by 24);
+  // a running (max, sum, acc) triple carries across groups
   float mmax = -INFINITY, acc = 0.f, lacc = 0.f;
-  for (int s0 = 0; s0 < S; s0 += 8) {
-    float ms[8], ls[8], os[8];
+  auto merge = [&](auto group_c) __attribute__((always_inline)) {
+    constexpr int G = decltype(group_c)::value;
+    for (int s0 = 0; s0 < S; s0 += G) {
+      float ms[G], ls[G], os[G];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int s = min(s0 + q, S - 1);
-      const int64_t idx = ((int64_t)(first + s) * p.lq + qi) * H + h;
-      ms[q] = s0 + q < S ? p.part_m[idx] : -INFINITY;
-      ls[q] = p.part_l[idx];
-      os[q] = p.part_o[idx * D + d];
+      for (int q = 0; q < G; ++q) {
+        const int s = min(s0 + q, S - 1);
+        const int64_t idx = ((int64_t)(first + s) * p.lq + qi) * H + h;
+        ms[q] = s0 + q < S ? p.part_m[idx] : -INFINITY;
+        ls[q] = p.part_l[idx];
+        os[q] = p.part_o[idx * D + d];
+      }
+      float gmax = mmax;
+#pragma unroll
+      for (int q = 0; q < G; ++q) gmax = fmaxf(gmax, ms[q]);
+      const float carry = mmax == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mmax - gmax);
+      acc *= carry;
+      lacc *= carry;
+#pragma unroll
+      for (int q = 0; q < G; ++q) {
+        const float f = ms[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[q] - gmax);
+        acc += f * os[q];
+        lacc += f * ls[q];
+      }
+      mmax = gmax;
     }
-    float gmax = mmax;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) gmax = fmaxf(gmax, ms[q]);
-    const float carry = mmax == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mmax - gmax);
-    acc *= carry;
-    lacc *= carry;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float f = ms[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[q] - gmax);
-      acc += f * os[q];
-      lacc += f * ls[q];
-    }
-    mmax = gmax;
-  }
+  };
+  if (S <= 8 || p.slots > 0) merge(std::integral_constant<int, 8>{});
+  else merge(std::integral_constant<int, 24>{});
   // this call's rows are row0 .. row0 + lq - 1 of the lq_total rows of o and lse
   store_from_f32(o + (((int64_t)b * p.lq_total + p.row0 + qi) * H + h) * D + d, acc * inv_rk / lacc);
   if (lse && d == 0) lse[((int64_t)b * H + h) * p.lq_total + p.row0 + qi] = (mmax + __builtin_amdgcn_logf(lacc)) * kLn2;
