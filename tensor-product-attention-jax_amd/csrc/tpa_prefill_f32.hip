@@ -290,7 +290,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
 // rebuilds each into LDS of its own (no barrier in the loop) with the next tile's factors on their way while the matrix
 // pipe works on this one, and the partial results are merged through LDS with the rule of _lse_accum
 // (tpa/tpa.py:228-242).  Every workgroup rebuilds its tiles for 32 rows instead of 256, which is why the kernel above
-// stays the one for launches that fill the chip (`few_rows_pay` below).
+// stays the one for launches that fill the chip (`rows_per_workgroup` below).
 template <int D, int NW>
 struct SplitLdsF32 {
   static constexpr int RS = D + 4;
