@@ -205,6 +205,19 @@ void check_dtypes(const Tensor* t, const char* const* names, int n) {
       throw Raise{PyExc_TypeError, std::string(names[i]) + " has dtype " + c10::toString(t[i].scalar_type()) + ", expected " + c10::toString(t[0].scalar_type())};
 }
 
+// q[b, lq, rq, h + dk], k[b, lk, rk, h + dk], v[b, lk, rk, h + dv] of one type: what the operator and its gradient take
+void check_concatenated(const Tensor& q, const Tensor& k, const Tensor& v, int64_t h) {
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) throw Raise{PyExc_ValueError, "q, k, v must be [b, l, r, h + d]"};
+  // rank and length of the keys are read from v (tpa/tpa.py:474-475)
+  expect(is_shape(k, {q.size(0), v.size(1), v.size(2), q.size(3)}), k);
+  expect(v.size(0) == q.size(0), v);
+  if (!(0 < h && h < q.size(3) && h < v.size(3)))
+    throw Raise{PyExc_AssertionError, "num_heads = " + std::to_string(h) + ", " + sizes_of(q) + ", " + sizes_of(v)};
+  const Tensor three[3] = {q, k, v};
+  static const char* const names[3] = {"q", "k", "v"};
+  check_dtypes(three, names, 3);
+}
+
 void unpack_six(PyObject* const* args, Tensor* t) {
   static const char* const names[6] = {"qa", "qb", "ka", "kb", "va", "vb"};
   for (int i = 0; i < 6; ++i) t[i] = THPVariable_Unpack(args[i]);
@@ -462,6 +475,7 @@ PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   c.qseg = tensor_or_none(args[3]); c.kvseg = tensor_or_none(args[4]);
   c.o = THPVariable_Unpack(args[5]); c.lse = THPVariable_Unpack(args[6]); c.d_o = THPVariable_Unpack(args[7]);
   c.heads = integer(args[8]);
+  check_concatenated(c.q, c.k, c.v, c.heads);
   c.sm_scale = real(args[9]);
   c.causal = (int)integer(args[10]); c.causal_offset = (int)integer(args[11]);
   Tensor grads[3];
@@ -537,15 +551,7 @@ PyObject* tpa(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!gpu_tensors(args, 3) || !none_or_gpu(args[3]) || !none_or_gpu(args[4])) Py_RETURN_NOTIMPLEMENTED;
   const Tensor q = THPVariable_Unpack(args[0]), k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]);
   const int64_t h = integer(args[5]);
-  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) throw Raise{PyExc_ValueError, "q, k, v must be [b, l, r, h + d]"};
-  // rank and length of the keys are read from v (tpa/tpa.py:474-475)
-  expect(is_shape(k, {q.size(0), v.size(1), v.size(2), q.size(3)}), k);
-  expect(v.size(0) == q.size(0), v);
-  if (!(0 < h && h < q.size(3) && h < v.size(3)))
-    throw Raise{PyExc_AssertionError, "num_heads = " + std::to_string(h) + ", " + sizes_of(q) + ", " + sizes_of(v)};
-  const Tensor three[3] = {q, k, v};
-  static const char* const names[3] = {"q", "k", "v"};
-  check_dtypes(three, names, 3);
+  check_concatenated(q, k, v, h);
   FwdCall c;
   c.qseg = tensor_or_none(args[3]); c.kvseg = tensor_or_none(args[4]);
   c.sm_scale = real(args[6]);

@@ -1,0 +1,59 @@
+"""Refusals of the native host layer (csrc/host_calls.cc) that need no GPU: shape-only tensors that claim to live on one
+reach the checks of its functions and nothing behind them."""
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+BF16, F32 = torch.bfloat16, torch.float32
+B, LQ, LK, RQ, RK, H, D = 2, 8, 16, 6, 2, 8, 64
+
+
+@pytest.fixture
+def shapes():
+    with FakeTensorMode():
+        yield lambda *s, dtype=BF16: torch.empty(s, device="cuda", dtype=dtype)
+
+
+def _concatenated(new, **changed):
+    x = dict(q=new(B, LQ, RQ, H + D), k=new(B, LK, RK, H + D), v=new(B, LK, RK, H + D), heads=H)
+    x.update(changed)
+    return x["q"], x["k"], x["v"], x["heads"]
+
+
+CONCATENATED = [
+    (AssertionError, lambda new: dict(k=new(B, LK - 1, RK, H + D))),  # fewer tokens than v
+    (AssertionError, lambda new: dict(k=new(B, LK, RK - 1, H + D))),
+    (AssertionError, lambda new: dict(k=new(B, LK, RK, H + D - 8))),
+    (AssertionError, lambda new: dict(k=new(B - 1, LK, RK, H + D))),
+    (AssertionError, lambda new: dict(k=new(B - 1, LK, RK, H + D), v=new(B - 1, LK, RK, H + D))),
+    (AssertionError, lambda new: dict(v=new(B - 1, LK, RK, H + D))),
+    (AssertionError, lambda new: dict(heads=0)),
+    (AssertionError, lambda new: dict(heads=-1)),
+    (AssertionError, lambda new: dict(heads=H + D)),
+    (TypeError, lambda new: dict(k=new(B, LK, RK, H + D, dtype=F32))),
+    (TypeError, lambda new: dict(v=new(B, LK, RK, H + D, dtype=F32))),
+    (ValueError, lambda new: dict(k=new(B, LK * RK, H + D))),
+]
+
+
+@pytest.mark.parametrize("call", ["tpa", "_tpa_bwd"])
+@pytest.mark.parametrize("error,changed", CONCATENATED)
+def test_the_operator_and_its_gradient_refuse_operands_that_do_not_fit(shapes, call, error, changed):
+    from tpa import tpa
+
+    q, k, v, heads = _concatenated(shapes, **changed(shapes))
+    with pytest.raises(error):
+        if call == "tpa":
+            tpa.tpa(q, k, v, heads)
+        else:
+            o, l = shapes(B, LQ, H, D), shapes(B, LQ, H, dtype=F32)
+            tpa._tpa_bwd(heads, 1.0, False, None, False, False, False, (q, k, v, None, None, o, l), o)
+
+
+def test_the_gradient_of_one_entry_refuses_them_too(shapes):
+    from tpa import tpa
+
+    q, k, v, o, l = shapes(LQ, RQ, H + D), shapes(LK - 1, RK, H + D), shapes(LK, RK, H + D), shapes(LQ, H, D), shapes(LQ, H, dtype=F32)
+    with pytest.raises(AssertionError):
+        tpa._bwd(q, k, v, None, None, o, l, o, H, 1.0, False, None, False, False, False)
