@@ -236,6 +236,7 @@ void describe(const Tensor* t, Args& a) {
   expect(is_shape(t[2], {a.B, a.lk, a.rk, a.H}), t[2]);
   expect(is_shape(t[3], {a.B, a.lk, a.rk, a.dk}), t[3]);
   expect(is_shape(t[4], {a.B, a.lk, a.rk, a.H}), t[4]);
+  expect(t[5].size(0) == a.B, t[5]);
   a.qa = factor_of<TpaFactor>(t[0]); a.qb = factor_of<TpaFactor>(t[1]);
   a.ka = factor_of<TpaFactor>(t[2]); a.kb = factor_of<TpaFactor>(t[3]);
   a.va = factor_of<TpaFactor>(t[4]); a.vb = factor_of<TpaFactor>(t[5]);

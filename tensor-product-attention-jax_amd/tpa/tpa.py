@@ -281,7 +281,14 @@ def tpa_factors_bwd(
     b, lq, rq, h = qa.shape
     _, lk, rk, dv = vb.shape
     dk = qb.shape[-1]
+    for name, t in (("qb", qb), ("ka", ka), ("kb", kb), ("va", va), ("vb", vb)):
+        if t.dtype != dtype:
+            raise TypeError(f"{name} has dtype {t.dtype}, expected {dtype}")
+    assert tuple(qb.shape) == (b, lq, rq, dk), qb.shape
+    assert tuple(ka.shape) == (b, lk, rk, h), ka.shape
     assert tuple(kb.shape) == (b, lk, rk, dk), kb.shape
+    assert tuple(va.shape) == (b, lk, rk, h), va.shape
+    assert vb.shape[0] == b, vb.shape
     assert tuple(o.shape) == (b, lq, h, dv) and tuple(do.shape) == (b, lq, h, dv), (o.shape, do.shape)
     assert tuple(lse.shape) == (b, h, lq), lse.shape
     qseg = _segment_ids(q_segment_ids, b, lq, device)
@@ -302,6 +309,8 @@ def tpa_factors_bwd(
     lse = lse.to(torch.float32).contiguous()
     if grads is None:
         grads = tuple(torch.empty(t.shape, dtype=torch.float32, device=device) for t in (qa, qb, ka, kb, va, vb))
+    for g, t in zip(grads, (qa, qb, ka, kb, va, vb)):
+        assert g.shape == t.shape, (g.shape, t.shape)
     lib = _d.load_library()
     need = lib.tpa_bwd_workspace_bytes(b, lq, lk, h, dk, dv)
     if workspace is None:

@@ -57,3 +57,30 @@ def test_the_gradient_of_one_entry_refuses_them_too(shapes):
     q, k, v, o, l = shapes(LQ, RQ, H + D), shapes(LK - 1, RK, H + D), shapes(LK, RK, H + D), shapes(LQ, H, D), shapes(LQ, H, dtype=F32)
     with pytest.raises(AssertionError):
         tpa._bwd(q, k, v, None, None, o, l, o, H, 1.0, False, None, False, False, False)
+
+
+@pytest.mark.parametrize("call", ["tpa_factors", "tpa_decode", "tpa_factors_bwd"])
+@pytest.mark.parametrize(
+    "changed",
+    [
+        dict(qb=(B, LQ, RQ - 1, D)), dict(ka=(B, LK - 1, RK, H)), dict(ka=(B, LK, RK, H - 1)), dict(kb=(B, LK, RK - 1, D)),
+        dict(va=(B - 1, LK, RK, H)), dict(va=(B, LK, RK - 1, H)), dict(vb=(B - 1, LK, RK, D)), dict(vb=(B, LK + 1, RK, D)),
+        dict(grads=4),
+    ],
+)
+def test_the_split_forms_refuse_factors_that_do_not_fit(shapes, call, changed):
+    from tpa import tpa
+
+    sizes = dict(qa=(B, LQ, RQ, H), qb=(B, LQ, RQ, D), ka=(B, LK, RK, H), kb=(B, LK, RK, D), va=(B, LK, RK, H), vb=(B, LK, RK, D))
+    if "grads" in changed and call != "tpa_factors_bwd":
+        pytest.skip("takes no gradient arrays")
+    x = [shapes(*{**sizes, **changed}[name]) for name in sizes]
+    with pytest.raises(AssertionError):
+        if call == "tpa_factors_bwd":
+            o, lse = shapes(B, LQ, H, x[5].shape[3]), shapes(B, H, LQ, dtype=F32)
+            grads = [shapes(*t.shape, dtype=F32) for t in x]
+            if "grads" in changed:
+                grads[changed["grads"]] = shapes(B, LK - 1, RK, H, dtype=F32)
+            tpa.tpa_factors_bwd(*x, None, None, o, lse, o, grads=grads)
+        else:
+            getattr(tpa, call)(*x)
