@@ -553,6 +553,10 @@ PyObject* tpa(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor q = THPVariable_Unpack(args[0]), k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]);
   const int64_t h = integer(args[5]);
   check_concatenated(q, k, v, h);
+  // a dual tensor need not ask for gradients, so the autograd node below, which refuses a tangent, may never see it
+  for (const Tensor* t : {&q, &k, &v})
+    if (t->_fw_grad(/*level=*/0).defined())
+      throw Raise{PyExc_NotImplementedError, "tpa has no forward-mode derivative: an input carries a tangent"};
   FwdCall c;
   c.qseg = tensor_or_none(args[3]); c.kvseg = tensor_or_none(args[4]);
   c.sm_scale = real(args[6]);

@@ -84,3 +84,14 @@ def test_the_split_forms_refuse_factors_that_do_not_fit(shapes, call, changed):
             tpa.tpa_factors_bwd(*x, None, None, o, lse, o, grads=grads)
         else:
             getattr(tpa, call)(*x)
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_forward_mode_raises_instead_of_dropping_the_tangent(shapes, which):
+    import torch.autograd.forward_ad as fwd
+    from tpa import tpa
+
+    qkv = [shapes(B, LQ, RQ, H + D), shapes(B, LK, RK, H + D), shapes(B, LK, RK, H + D)]
+    with fwd.dual_level(), pytest.raises(NotImplementedError):
+        qkv[which] = fwd.make_dual(qkv[which], shapes(*qkv[which].shape))
+        tpa.tpa(*qkv, H)
