@@ -303,7 +303,8 @@ const char* tpa_strerror(int code);
  * If `workspace` holds at least tpa_decode_workspace_bytes(...) bytes and the problem is a
  * decode (lq <= 16, lk >= 1024, no segment ids) that tpa_decode's kernel takes, the call is served by
  * it; if `workspace` holds tpa_fwd_workspace_bytes(...) bytes and the problem is long enough for it to
- * pay (rank 2: 2048 query rows and more; other ranks: more than 256), dense bf16 Q (times
+ * pay (rank 2: 2048 query rows and more; other ranks: more than 256, and from rank 3 on more than 16 over
+ * 1024 keys or more), dense bf16 Q (times
  * sm_scale * log2 e), K and V are reconstructed into it once and the prefill kernel runs its loop over
  * dense tiles.  Without a workspace the same problems run on the fused prefill kernel, which rebuilds
  * K / V tiles from the rank factors inside its loop.  The two routes round at the same points (Q, K, V,

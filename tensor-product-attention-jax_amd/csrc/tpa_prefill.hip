@@ -1226,11 +1226,15 @@ size_t tpa_prefill_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int
 // reconstruction grows with the length only.  Rank 2 has a tuned rebuild in the fused kernel:
 // measured at B * H = 64, D = 128 the two routes meet at 1024 rows (51 against 52 us) and the dense
 // one wins from 2048 on (105 against 115 us; 4096: 0.32 against 0.38 ms).  Other ranks loop over
-// the ranks per tile in the fused kernel: dense from the second query block on, and for one block over many keys
-// (6 x 242 rows over 14228 keys, rank 8, 32 heads of 128: 3.89 ms fused).
+// the ranks per tile in the fused kernel: dense from the second query block on.
+// One query block rebuilds every tile once on either route, so there the rebuild itself decides.  Fused over dense time
+// at 17 to 256 rows over 1024 to 16384 keys, 1 to 8 sequences of 8 to 64 heads of 64 and 128, keys split where that pays:
+// rank 1 0.65 - 1.37 (over 1 only up to 1024 keys and for small batches of up to 4096; 8 sequences of 32 heads over 4096 keys
+// 170 against 253 us), rank 3 0.94 - 1.8, rank 4 0.99 - 2.0, rank 8 1.25 - 5.5, rank 16 1.4 - 9.5.  So from rank 3 on
+// dense, which takes 4 lk H D bytes per sequence for K and V where the fused kernel takes none.
 int tpa_prefill_wants_dense(int64_t lq, int64_t lk, int64_t rk) {
-  if (rk != 2) return lq > tpa::kBQ || (lq > 16 && lk >= 1024);
-  return lq >= 2048;
+  if (rk == 2) return lq >= 2048;
+  return lq > tpa::kBQ || (rk > 2 && lq > 16 && lk >= 1024);
 }
 
 size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {

@@ -177,3 +177,12 @@ def test_missing_library_fails_loudly(tmp_path):
 
     with pytest.raises(RuntimeError, match="not built"):
         _dispatch.load_library(str(tmp_path / "nope.so"))
+
+
+@pytest.mark.parametrize("rk,lq,lk,dense", [(1, 17, 16384, False), (1, 256, 1024, False), (1, 257, 1024, True), (2, 256, 16384, False),
+                                            (3, 17, 1024, True), (4, 256, 4096, True), (8, 17, 1023, False), (8, 16, 1000, False)])
+def test_few_query_rows_rebuild_dense_keys_only_where_that_is_faster(rk, lq, lk, dense):
+    from tpa import _dispatch
+
+    want = 2 * 4 * (lq + 2 * lk) * 16 * 128 if dense else 0
+    assert _dispatch.load_library().tpa_fwd_workspace_bytes(4, lq, lk, 16, 128, 128, 6, rk) == want
