@@ -181,7 +181,13 @@ std::pair<Tensor, Tensor> run_fwd(TpaFwdArgs& a, const FwdCall& c, const at::Dev
   else if (c.use_workspace && (dtype == at::kBFloat16 || a.lq <= 16))
     need = (dtype == at::kBFloat16 ? lib.tpa_fwd_best_workspace_bytes : lib.tpa_fwd_workspace_bytes)(a.B, a.lq, a.lk, a.H, a.dk, a.dv, a.rq, a.rk);
   if (need) {
-    ws = bytes_on(device, need + 256);
+    try {
+      ws = bytes_on(device, need + 256);
+    } catch (const c10::OutOfMemoryError&) {
+      if (c.nomat) throw;  // otherwise it is optional: on a card too full for it the kernels that take none serve the call
+    }
+  }
+  if (ws.defined()) {
     a.workspace = aligned(ws, 256);
     a.workspace_bytes = need;
   }
