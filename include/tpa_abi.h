@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define TPA_ABI_VERSION 10
+#define TPA_ABI_VERSION 11
 
 /* element types of the factor / output arrays */
 enum { TPA_DTYPE_F32 = 0, TPA_DTYPE_BF16 = 1 };
@@ -326,6 +326,14 @@ size_t tpa_fwd_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int
  * alone would leave the chip partly idle (bf16, no segment ids).
  */
 size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk);
+
+/*
+ * Bytes of workspace (256-byte aligned) that tpa_fwd would use for this very call: its sizes, mask, segment ids, strides,
+ * alignment, kernel, num_splits and nomat; 0 if none, or if tpa_fwd would refuse the call.  `workspace` and
+ * `workspace_bytes` of the arguments are not looked at.  Never more than tpa_fwd_best_workspace_bytes(...) unless
+ * num_splits or nomat is set.
+ */
+size_t tpa_fwd_call_workspace_bytes(const TpaFwdArgs* args);
 
 /*
  * Bytes of workspace (256-byte aligned) tpa_fwd needs with args.nomat != 0 for the split-key kernels to serve

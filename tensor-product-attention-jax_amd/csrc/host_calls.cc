@@ -30,8 +30,8 @@ using at::Tensor;
 
 // ------------------------------------------------------------------------------------------------ the C ABI, by name
 #define TPA_CALLS(X)                                                                                             \
-  X(tpa_fwd) X(tpa_decode) X(tpa_cache_append) X(tpa_bwd) X(tpa_strerror) X(tpa_fwd_workspace_bytes) X(tpa_fwd_best_workspace_bytes) \
-  X(tpa_fwd_nomat_workspace_bytes) X(tpa_decode_workspace_bytes) X(tpa_cache_append_workspace_bytes) X(tpa_bwd_workspace_bytes)
+  X(tpa_fwd) X(tpa_decode) X(tpa_cache_append) X(tpa_bwd) X(tpa_strerror) X(tpa_fwd_call_workspace_bytes) \
+  X(tpa_decode_workspace_bytes) X(tpa_cache_append_workspace_bytes) X(tpa_bwd_workspace_bytes)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
   TPA_CALLS(X)
@@ -155,8 +155,6 @@ void* aligned(const Tensor& t, size_t to) {
 void* stream_of(const at::Device& device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
 
 // ------------------------------------------------------------------------------------------------ forward
-constexpr int kNomatRankPairs = TPA_NOMAT_RANK_PAIRS;
-
 struct FwdCall {
   Tensor qseg, kvseg, kvlen;
   double sm_scale = 1.0;
@@ -173,13 +171,18 @@ std::pair<Tensor, Tensor> run_fwd(TpaFwdArgs& a, const FwdCall& c, const at::Dev
   const auto options = at::TensorOptions().device(device);
   Tensor o = at::empty({a.B, a.lq, a.H, a.dv}, options.dtype(dtype)), lse, ws;
   if (c.return_lse) lse = at::empty({a.B, a.H, a.lq}, options.dtype(at::kFloat));
-  // the workspace with which the library can pick its fastest kernel (nomat: the split partials, required); it decides
-  // whether the problem qualifies.  fp32 inputs: only the split-key decode kernel takes one.
-  size_t need = 0;
-  if (c.nomat == kNomatRankPairs || c.kernel == TPA_KERNEL_GENERIC) need = 0;
-  else if (c.nomat) need = lib.tpa_fwd_nomat_workspace_bytes(a.B, a.lq, a.lk, a.H, a.dk, a.dv, a.rq, a.rk);
-  else if (c.use_workspace && (dtype == at::kBFloat16 || a.lq <= 16))
-    need = (dtype == at::kBFloat16 ? lib.tpa_fwd_best_workspace_bytes : lib.tpa_fwd_workspace_bytes)(a.B, a.lq, a.lk, a.H, a.dk, a.dv, a.rq, a.rk);
+  a.q_segment_ids = ids_ptr(qseg);
+  a.kv_segment_ids = ids_ptr(kvseg);
+  a.kv_lengths = ids_ptr(kvlen);
+  a.o = o.data_ptr();
+  a.lse = f32_ptr(lse);
+  a.sm_scale = (float)c.sm_scale;
+  a.causal = c.causal;
+  a.kernel = c.kernel;
+  a.causal_offset = c.causal_offset;
+  a.nomat = c.nomat;
+  // the workspace with which the library can pick its fastest kernel (nomat: the split partials, required)
+  const size_t need = c.use_workspace || c.nomat ? lib.tpa_fwd_call_workspace_bytes(&a) : 0;
   if (need) {
     try {
       ws = bytes_on(device, need + 256);
@@ -191,16 +194,6 @@ std::pair<Tensor, Tensor> run_fwd(TpaFwdArgs& a, const FwdCall& c, const at::Dev
     a.workspace = aligned(ws, 256);
     a.workspace_bytes = need;
   }
-  a.q_segment_ids = ids_ptr(qseg);
-  a.kv_segment_ids = ids_ptr(kvseg);
-  a.kv_lengths = ids_ptr(kvlen);
-  a.o = o.data_ptr();
-  a.lse = f32_ptr(lse);
-  a.sm_scale = (float)c.sm_scale;
-  a.causal = c.causal;
-  a.kernel = c.kernel;
-  a.causal_offset = c.causal_offset;
-  a.nomat = c.nomat;
   check("tpa_fwd", lib.tpa_fwd(&a, stream_of(device)));
   return {o, lse};
 }

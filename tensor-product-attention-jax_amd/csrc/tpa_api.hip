@@ -67,21 +67,29 @@ bool nomat_rank_and_heads(int dk, int dv, int rk) {
   return dk == dv && (dk == 64 || dk == 128) && rk >= 1 && rk <= 32 && (rk & (rk - 1)) == 0;
 }
 
-// tpa_fwd with nomat: the split-key kernels, which never form K or V, over windows of query rows.  Every window
-// shares the workspace; they run one after the other on the stream.
-int tpa_fwd_nomat(const TpaFwdArgs* a, hipStream_t s) {
+// the first window of query rows of a nomat call
+TpaFwdArgs nomat_window(const TpaFwdArgs* a) {
   TpaFwdArgs w = *a;
   w.lq = a->lq < kNomatWindow ? a->lq : kNomatWindow;
   w.nomat = 0;
+  return w;
+}
+size_t nomat_bytes(const TpaFwdArgs* a, const TpaFwdArgs& w) {
+  return a->num_splits > 0 ? tpa_decode_workspace_bytes(a->B, w.lq, a->lk, a->H, a->dv, a->num_splits)
+                           : tpa_fwd_nomat_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->dv, a->rq, a->rk);
+}
+
+// tpa_fwd with nomat: the split-key kernels, which never form K or V, over windows of query rows.  Every window
+// shares the workspace; they run one after the other on the stream.
+int tpa_fwd_nomat(const TpaFwdArgs* a, hipStream_t s) {
+  TpaFwdArgs w = nomat_window(a);
   const bool bf16 = a->kernel != TPA_KERNEL_GENERIC && tpa_decode_mfma_supported(&w);
   const bool f32 = a->kernel != TPA_KERNEL_GENERIC && !bf16 && tpa_decode_f32_supported(&w);
   if (!bf16 && !f32) {
     if (a->kernel == TPA_KERNEL_MFMA) return TPA_ERR_UNSUPPORTED;
     return tpa_generic_launch(a, s);
   }
-  const size_t need = a->num_splits > 0 ? tpa_decode_workspace_bytes(a->B, w.lq, a->lk, a->H, a->dv, a->num_splits)
-                                        : tpa_fwd_nomat_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->dv, a->rq, a->rk);
-  if (!a->workspace || a->workspace_bytes < need) return TPA_ERR_WORKSPACE;
+  if (!a->workspace || a->workspace_bytes < nomat_bytes(a, w)) return TPA_ERR_WORKSPACE;
   const size_t esz = a->dtype == TPA_DTYPE_BF16 ? 2 : 4;
   for (int row0 = 0; row0 < a->lq; row0 += kNomatWindow) {
     w.lq = a->lq - row0 < kNomatWindow ? a->lq - row0 : kNomatWindow;
@@ -92,6 +100,9 @@ int tpa_fwd_nomat(const TpaFwdArgs* a, hipStream_t s) {
   }
   return TPA_OK;
 }
+
+// few query tokens over a long cache (the reference's decode is this same call with lq = 1, tpa/tpa.py:485)
+bool is_decode(const TpaFwdArgs* a) { return a->kernel != TPA_KERNEL_GENERIC && a->lq <= 16 && a->lk >= 1024 && !a->q_segment_ids; }
 
 }  // namespace
 
@@ -119,10 +130,8 @@ int tpa_fwd(const TpaFwdArgs* a, void* stream) {
     return tpa_generic_launch(a, s);
   }
   if (a->nomat) return tpa_fwd_nomat(a, s);
-  // few query tokens over a long cache (the reference's decode is this same call with lq = 1,
-  // tpa/tpa.py:485): split over keys, if the caller brought the workspace for it
-  if (a->kernel != TPA_KERNEL_GENERIC && a->workspace && a->lq <= 16 && a->lk >= 1024 &&
-      !a->q_segment_ids && a->workspace_bytes >= tpa_decode_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->num_splits)) {
+  // a decode is split over keys, if the caller brought the workspace for it
+  if (is_decode(a) && a->workspace && a->workspace_bytes >= tpa_decode_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->num_splits)) {
     if (tpa_decode_mfma_supported(a)) return tpa_decode_mfma_launch(a, s);
     if (tpa_decode_f32_supported(a)) return tpa_decode_f32_launch(a, s);
   }
@@ -150,6 +159,17 @@ size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H
   if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0 || rk <= 0 || dk != dv || (dk != 64 && dk != 128)) return base;
   const size_t best = tpa_prefill_best_bytes(B, lq, lk, H, dk, rk);
   return best > base ? best : base;
+}
+
+size_t tpa_fwd_call_workspace_bytes(const TpaFwdArgs* a) {
+  if (tpa_validate_fwd_args(a) != TPA_OK || a->page_table || a->kernel == TPA_KERNEL_GENERIC || a->nomat == TPA_NOMAT_RANK_PAIRS) return 0;
+  if (a->nomat) {
+    const TpaFwdArgs w = nomat_window(a);
+    return tpa_decode_mfma_supported(&w) || tpa_decode_f32_supported(&w) ? nomat_bytes(a, w) : 0;
+  }
+  if (is_decode(a) && (tpa_decode_mfma_supported(a) || tpa_decode_f32_supported(a)))
+    return tpa_decode_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->num_splits);
+  return tpa_prefill_mfma_supported(a) ? tpa_prefill_call_bytes(a) : 0;
 }
 
 int tpa_decode(const TpaFwdArgs* a, void* stream) {

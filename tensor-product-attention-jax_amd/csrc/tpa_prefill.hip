@@ -1243,6 +1243,28 @@ size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int6
   return dense + tpa::split_bytes(B, lq, H, D, s0 > s1 ? s0 : s1);
 }
 
+namespace tpa {
+namespace {
+
+// What a call wants of a workspace: dense Q, K and V (0: the fused kernel), and behind them the partial results of S key
+// ranges per query block (the kernels with segment ids do not split the keys).
+struct PrefillRoute {
+  size_t dense;
+  int S;
+};
+PrefillRoute route_of(const TpaFwdArgs* a) {
+  return {tpa_prefill_wants_dense(a->lq, a->lk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
+          a->kv_segment_ids ? 1 : a->num_splits > 0 ? a->num_splits : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0)};
+}
+
+}  // namespace
+}  // namespace tpa
+
+size_t tpa_prefill_call_bytes(const TpaFwdArgs* a) {
+  const tpa::PrefillRoute route = tpa::route_of(a);
+  return route.dense + tpa::split_bytes(a->B, a->lq, a->H, a->dk, route.S);
+}
+
 int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
   using namespace tpa;
   PrefillParams p{};
@@ -1257,13 +1279,13 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
   // the kernel runs with its plain tile loader: no workgroup rebuilds tiles from the rank factors
   // (the fused kernel does that once per 256 query rows and head).
   const bool usable = a->workspace && !(reinterpret_cast<uintptr_t>(a->workspace) & 255);
-  const size_t dense_bytes = tpa_prefill_wants_dense(a->lq, a->lk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0;
-  const bool dense = usable && dense_bytes && a->workspace_bytes >= dense_bytes;
+  const PrefillRoute route = route_of(a);
+  const bool dense = usable && route.dense && a->workspace_bytes >= route.dense;
   // what the workspace has beyond that can take the partial results of key ranges
   p.S = 1;
-  const size_t used = dense ? dense_bytes : 0;
-  const int S = a->num_splits > 0 ? a->num_splits : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0);
-  if (usable && !p.kvseg && S > 1 && a->workspace_bytes >= used + split_bytes(a->B, a->lq, a->H, a->dk, S)) {
+  const size_t used = dense ? route.dense : 0;
+  const int S = route.S;
+  if (usable && S > 1 && a->workspace_bytes >= used + split_bytes(a->B, a->lq, a->H, a->dk, S)) {
     p.S = S;
     p.part_o = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + used);
     p.part_ml = reinterpret_cast<float2*>(p.part_o + (size_t)S * a->B * a->lq * a->H * a->dk);

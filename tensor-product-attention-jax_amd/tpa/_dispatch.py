@@ -24,7 +24,7 @@ KERNEL_AUTO = 0
 KERNEL_GENERIC = 1
 KERNEL_MFMA = 2
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 
 class TpaFactor(ctypes.Structure):
@@ -251,6 +251,8 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
         lib.tpa_fwd_workspace_bytes.argtypes = [ctypes.c_int32] * 8
         lib.tpa_fwd_best_workspace_bytes.restype = ctypes.c_size_t
         lib.tpa_fwd_best_workspace_bytes.argtypes = [ctypes.c_int32] * 8
+        lib.tpa_fwd_call_workspace_bytes.restype = ctypes.c_size_t
+        lib.tpa_fwd_call_workspace_bytes.argtypes = [ctypes.POINTER(TpaFwdArgs)]
         lib.tpa_fwd_nomat_workspace_bytes.restype = ctypes.c_size_t
         lib.tpa_fwd_nomat_workspace_bytes.argtypes = [ctypes.c_int32] * 8
         lib.tpa_bwd.restype = ctypes.c_int

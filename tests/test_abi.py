@@ -2,6 +2,7 @@
 declares, and the ctypes structures have the layout the C compiler gives the header's."""
 
 import ctypes
+import itertools
 import os
 import re
 import subprocess
@@ -186,3 +187,42 @@ def test_few_query_rows_rebuild_dense_keys_only_where_that_is_faster(rk, lq, lk,
 
     want = 2 * 4 * (lq + 2 * lk) * 16 * 128 if dense else 0
     assert _dispatch.load_library().tpa_fwd_workspace_bytes(4, lq, lk, 16, 128, 128, 6, rk) == want
+
+
+def _forward_call(B=1, lq=331, lk=2258, H=16, D=128, rk=2, **changed):
+    from tpa import _dispatch as d
+
+    fake = d.TpaFactor(256, 8, 8, 8)  # aligned, never read: these calls only ask for sizes
+    if lq <= 16:
+        fake = d.TpaFactor(256, 8, 8 * rk, 8)
+    x = dict(qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, o=256, B=B, lq=lq, lk=lk, H=H, dk=D, dv=D, rq=6, rk=rk,
+             dtype=d.TPA_DTYPE_BF16, sm_scale=1.0, causal=0, kernel=d.KERNEL_AUTO)
+    x.update(changed)
+    return d.TpaFwdArgs(**x)
+
+
+def test_a_call_asks_for_the_workspace_that_it_can_use():
+    """The partial results of key ranges are asked for by calls that split their keys and at the size of their mask's choice:
+    packed documents never split, a call without a mask needs fewer ranges, the generic kernel uses nothing."""
+    from tpa import _dispatch as d
+
+    lib = d.load_library()
+    need = lambda **kw: lib.tpa_fwd_call_workspace_bytes(ctypes.byref(_forward_call(**kw)))
+    ids = dict(q_segment_ids=256, kv_segment_ids=256)
+    part = 331 * 16 * (128 + 2) * 4  # one range's partial results
+    assert need() > 0 and need() % part == 0
+    assert need(num_splits=3) == 3 * part
+    assert need(**ids) == 0
+    assert need(kernel=d.KERNEL_GENERIC) == 0 and need(sm_scale=-1.0) == 0 and need(lk=0) == 0
+    assert need(dtype=d.TPA_DTYPE_F32) == 0
+    # dense Q, K and V, and nothing behind them
+    assert need(B=4, lq=4096, lk=4096, **ids) == need(B=4, lq=4096, lk=4096) == 3 * 4 * 4096 * 16 * 128 * 2
+    # the causal mask leaves blocks of different lengths and takes more ranges to level them
+    wide, causal = (need(B=1, lq=3000, lk=3000, H=8, D=64, causal=c) for c in (0, 1))
+    assert wide < causal == lib.tpa_fwd_best_workspace_bytes(1, 3000, 3000, 8, 64, 64, 6, 2)
+    # the split-key decode kernels, and the calls that never form K or V
+    assert need(lq=1, lk=8192) == lib.tpa_decode_workspace_bytes(1, 1, 8192, 16, 128, 0)
+    assert need(lq=1, lk=8192, **ids) == 0
+    assert need(lq=1, lk=8192, num_splits=5) == lib.tpa_decode_workspace_bytes(1, 1, 8192, 16, 128, 5)
+    for B, lq, lk, H, D, rk, c in itertools.product((1, 6), (40, 300, 2500), (900, 5000), (8, 32), (64, 128), (1, 2, 4), (0, 1)):
+        assert need(B=B, lq=lq, lk=lk, H=H, D=D, rk=rk, causal=c) <= lib.tpa_fwd_best_workspace_bytes(B, lq, lk, H, D, D, 6, rk)
