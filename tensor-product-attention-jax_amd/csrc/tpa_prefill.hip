@@ -1253,8 +1253,9 @@ struct PrefillRoute {
   int S;
 };
 PrefillRoute route_of(const TpaFwdArgs* a) {
+  const int tiles = (int)(((int64_t)a->lk + kTK - 1) / kTK);  // a caller's count beyond that only adds empty ranges
   return {tpa_prefill_wants_dense(a->lq, a->lk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
-          a->kv_segment_ids ? 1 : a->num_splits > 0 ? a->num_splits : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0)};
+          a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0)};
 }
 
 }  // namespace

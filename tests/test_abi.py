@@ -212,6 +212,7 @@ def test_a_call_asks_for_the_workspace_that_it_can_use():
     part = 331 * 16 * (128 + 2) * 4  # one range's partial results
     assert need() > 0 and need() % part == 0
     assert need(num_splits=3) == 3 * part
+    assert need(num_splits=2**31 - 1) == (2258 + 63) // 64 * part  # no more ranges than tiles of 64 keys
     assert need(**ids) == 0
     assert need(kernel=d.KERNEL_GENERIC) == 0 and need(sm_scale=-1.0) == 0 and need(lk=0) == 0
     assert need(dtype=d.TPA_DTYPE_F32) == 0
