@@ -56,11 +56,14 @@ struct DecodeParams {
 // common range length, the shortest one that needs no more than `slots` ranges (one workgroup per compute unit).  The
 // lengths are known on the device only, so each wave works the plan out for itself: lane = batch entry (B <= 64) for the
 // lengths, lane = candidate range length for the search.  What rounding does to a count only moves the balance: an
-// entry's blocks are dealt round-robin to whatever number of ranges it has, at least one.
+// entry's blocks are dealt round-robin to whatever number of ranges it has, at least one.  But the decode kernel and the
+// merge each work the plan out and must arrive at the same one, so nothing in it is left to the compiler: the products
+// and sums are not contracted but where `fmaf` says so, and conversions, quotients and `ceilf` are exact or round once.
 // 48 paged sequences of 2047 .. 4096 tokens (32 heads of 128, rank 2): 67.7 us with equal counts (288 workgroups), 43.4 so.
 constexpr int kMaxPlanEntries = 64;
 struct RangePlan { int S, first; };  // of batch entry `lane`: its number of ranges and the first one's index
 __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, int min_keys) {
+#pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
   int total = len;
@@ -68,7 +71,7 @@ __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, in
   for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
   const float shortest = fmaxf((float)total / (float)slots, (float)min_keys);
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
-  const float inv = 1.f / (shortest + (longest - shortest) * (float)lane * (1.f / 63.f));
+  const float inv = 1.f / fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
   // eight entries at a time, their chains side by side (lanes past the last entry hold length 0 and count 1)
   int count[8] = {}, j0 = 0;
   for (; j0 < B; j0 += 8)

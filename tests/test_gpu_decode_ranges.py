@@ -2,6 +2,7 @@
 CPU oracle: one entry and as many as a wave has lanes (and one more, where all entries get one count again), lengths
 from none to the whole cache, two row groups, ranks of the queries past one matrix instruction (16)."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -57,3 +58,45 @@ def test_several_rows_are_the_rows_alone(gpu, lq):
         ends = [n - lq + 1 + i for n in lengths]
         o_ref, l_ref = _varlen_reference(as_f64(tq[:, i : i + 1]), as_f64(tk), as_f64(tv), ends, h, d**-0.5, False)
         check(o[:, i : i + 1], lse[:, :, i : i + 1], o_ref, l_ref, BF16_TOL, tuple(x[:, i : i + 1] for x in bounds))
+
+
+def _planned_ranges(lengths, lk, slots, min_keys):
+    """Ranges per entry as the kernels plan them, in the same fp32 steps."""
+    f = np.float32
+    n = np.minimum(np.maximum(np.asarray(lengths), 0), lk)
+    total = f(n.sum())
+    shortest = max(total / f(slots), f(min_keys))
+    longest = max(total / f(slots - len(n)) + f(1), shortest) if slots > len(n) else f(lk)
+    for lane in range(64):  # the product and the sum round once, together: long double holds the product exactly
+        length = f(np.longdouble((longest - shortest) * f(lane)) * np.longdouble(f(1) / f(63)) + np.longdouble(shortest))
+        ranges = np.maximum(1, np.ceil(n.astype(f) * (f(1) / length))).astype(int)
+        if ranges.sum() <= slots:
+            return ranges
+    return np.ones(len(n), int)
+
+
+@pytest.mark.parametrize("seed", range(12))
+def test_both_kernels_follow_the_stated_plan(gpu, seed):
+    """The decode kernel and the merge work the plan out separately.  A workspace of NaN shows the first one's ranges (those
+    that were written); a merge that takes others reads NaN."""
+    from tpa import tpa
+
+    rng = np.random.default_rng(seed)
+    b, lk, h, d = int(rng.integers(1, 65)), int(rng.integers(300, 9000)), 8, 64
+    lengths = rng.integers(0 if seed % 2 else lk // 2, lk + 1, b)
+    lengths[0] = max(1, lengths[0])
+    q, k, v = make_factors(97 + seed, b, 1, lk, h, d, d, 2, 2, scale_by_rank=True)
+    parts = tpa_split(*(to_gpu(x, torch.bfloat16, gpu) for x in (q, k, v)), h)
+    kvl = torch.tensor(lengths, dtype=torch.int32, device=gpu)
+    default = tpa._d.load_library().tpa_decode_default_splits(b, 1, lk, h)
+    slots = min(max(b, 256), b * default)
+    ws = torch.full((tpa.decode_workspace_bytes(b, 1, lk, h, d),), 0xFF, dtype=torch.uint8, device=gpu)
+    got = tpa.tpa_decode(*parts, sm_scale=d**-0.5, kv_lengths=kvl, kernel=2, workspace=ws)
+    maxima = ws.view(torch.float32)[slots * h * d :][: slots * h].view(slots, h)
+    written = (~maxima.isnan()).all(1).sum().item()
+    assert written == _planned_ranges(lengths, lk, slots, 64).sum(), (b, lk, slots)
+    want = tpa.tpa_decode(*parts, sm_scale=d**-0.5, kv_lengths=kvl, kernel=1)
+    some = torch.from_numpy(lengths > 0).to(gpu)
+    for x, y in zip(got, want):
+        assert x[some].isfinite().all()
+        torch.testing.assert_close(x[some].float(), y[some].float(), rtol=2e-2, atol=2e-2)
