@@ -15,6 +15,8 @@
 //                for X in {Q, K, V}                                            (tpa/tpa.py:767-768,776-777,782-783)
 // Rows without a visible key (lse = -inf) contribute nothing (tpa/tpa.py:675-676).
 // Gradients are written as fp32 whatever the input type is.
+#include <algorithm>
+
 #include "tpa_common.h"
 
 namespace tpa {
@@ -553,9 +555,9 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
   return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }
-// All three arrays in one launch (blockIdx.z): at short lengths a launch of its own leaves each of them waiting for the
-// one before.  The gradients are written in the type the caller wants them in (rounded once, from the fp32 sums).
-struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R; };
+// All arrays that this kernel takes in one launch (blockIdx.z): at short lengths a launch of its own leaves each of them
+// waiting for the one before.  The gradients are written in the type the caller wants them in (rounded once, from the fp32 sums).
+struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R, D; };
 struct ProjectJobs { ProjectJob job[3]; };
 template <typename T>
 __device__ __forceinline__ f32x4 four_as_f32(const T* p) {
@@ -572,11 +574,11 @@ __device__ __forceinline__ void store_four(TO* p, f32x4 x) {
   else *reinterpret_cast<f32x4*>(p) = x;
 }
 template <typename T, typename TO>
-__global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H, int D) {
+__global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H) {
   const ProjectJob j = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
   const TpaFactor &fa = j.fa, &fb = j.fb;
   const TpaGrad &ga = j.ga, &gb = j.gb;
-  const int L = j.L, R = j.R;
+  const int L = j.L, R = j.R, D = j.D;
   const int cpr = D / 8, hgs = H / 8, tt = cpr * hgs;  // threads per token
   const int64_t gtid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int cc = (int)(gtid % cpr), hg = (int)(gtid / cpr % hgs);
@@ -657,34 +659,38 @@ bool rows16(const TpaFactor& f) {
   return al16(f.ptr) && f.stride_b % N == 0 && f.stride_l % N == 0 && f.stride_r % N == 0;
 }
 
+// Whether project_h8_kernel takes an array: each is judged by itself, so that one that it cannot take (an unaligned view,
+// another head size) does not send the others to the kernel of one workgroup per token.
 template <typename T, typename TO>
-void launch_project(const ProjectJobs& jobs, int B, int H, int dk, int dv, hipStream_t stream) {
-  const int cpr = dk / 8, hgs = H / 8, tt = cpr * hgs;
-  bool fast = dk == dv && dk % 8 == 0 && H % 8 == 0 && (cpr == 8 || cpr == 16) && tt <= 64 && (tt & (tt - 1)) == 0;
-  int lmax = 0;
+bool projects_by_h8(const ProjectJob& j, int H) {
+  const int cpr = j.D / 8, tt = cpr * (H / 8);
+  const TpaFactor ga{j.ga.ptr, j.ga.stride_b, j.ga.stride_l, j.ga.stride_r}, gb{j.gb.ptr, j.gb.stride_b, j.gb.stride_l, j.gb.stride_r};
+  return j.D % 8 == 0 && H % 8 == 0 && (cpr == 8 || cpr == 16) && tt <= 64 && (tt & (tt - 1)) == 0 && ((int64_t)j.L * tt + 255) / 256 <= 2147483647LL &&
+         al16(j.dx) && rows16<T>(j.fa) && rows16<T>(j.fb) && rows16<TO>(ga) && rows16<TO>(gb);
+}
+
+template <typename T, typename TO>
+void launch_project(const ProjectJobs& jobs, int B, int H, hipStream_t stream) {
+  ProjectJobs h8{};
+  int64_t blocks = 0;
+  unsigned n = 0;
   for (const ProjectJob& j : jobs.job) {
-    const TpaFactor ga{j.ga.ptr, j.ga.stride_b, j.ga.stride_l, j.ga.stride_r}, gb{j.gb.ptr, j.gb.stride_b, j.gb.stride_l, j.gb.stride_r};
-    fast = fast && al16(j.dx) && rows16<T>(j.fa) && rows16<T>(j.fb) && rows16<TO>(ga) && rows16<TO>(gb);
-    lmax = j.L > lmax ? j.L : lmax;
-  }
-  const int64_t blocks = ((int64_t)lmax * tt + 255) / 256;
-  if (fast && blocks <= 2147483647LL) {
-    hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, 3), dim3(256), 0, stream, jobs, H, dk);
-    return;
-  }
-  for (int n = 0; n < 3; ++n) {
-    const ProjectJob& j = jobs.job[n];
-    const int D = n == 2 ? dv : dk;
-    const size_t smem = ((size_t)H * (D + 4) + (size_t)j.R * D + (size_t)j.R * H) * sizeof(float);
+    if (projects_by_h8<T, TO>(j, H)) {
+      h8.job[n++] = j;
+      blocks = std::max(blocks, ((int64_t)j.L * (j.D / 8) * (H / 8) + 255) / 256);
+      continue;
+    }
+    const size_t smem = ((size_t)H * (j.D + 4) + (size_t)j.R * j.D + (size_t)j.R * H) * sizeof(float);
     int dsh = 0;
-    while ((1 << dsh) < D) ++dsh;
+    while ((1 << dsh) < j.D) ++dsh;
     int nsh = 0;  // lanes per da output: a power of two, at most a wave, so that one pass covers the outputs if it can
-    while (nsh < 6 && (4 << nsh) * j.R * H <= 512 && (16 << nsh) <= D) ++nsh;
-    if (smem <= 60 * 1024 && (1 << dsh) == D && D >= 4)
-      hipLaunchKernelGGL((project_kernel<T, TO, true>), dim3(j.L, B), dim3(256), smem, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, D, j.R, dsh, nsh);
+    while (nsh < 6 && (4 << nsh) * j.R * H <= 512 && (16 << nsh) <= j.D) ++nsh;
+    if (smem <= 60 * 1024 && (1 << dsh) == j.D && j.D >= 4)
+      hipLaunchKernelGGL((project_kernel<T, TO, true>), dim3(j.L, B), dim3(256), smem, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, j.D, j.R, dsh, nsh);
     else
-      hipLaunchKernelGGL((project_kernel<T, TO, false>), dim3(j.L, B), dim3(256), 0, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, D, j.R, dsh, nsh);
+      hipLaunchKernelGGL((project_kernel<T, TO, false>), dim3(j.L, B), dim3(256), 0, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, j.D, j.R, dsh, nsh);
   }
+  if (n) hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, n), dim3(256), 0, stream, h8, H);
 }
 
 template <typename T, int DMAX>
@@ -782,13 +788,13 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
   }
   if (rc != TPA_OK) return rc;
 
-  const ProjectJobs jobs{{{dqd, a->qa, a->qb, a->dqa, a->dqb, a->lq, a->rq},
-                          {dkd, a->ka, a->kb, a->dka, a->dkb, a->lk, a->rk},
-                          {dvd, a->va, a->vb, a->dva, a->dvb, a->lk, a->rk}}};
+  const ProjectJobs jobs{{{dqd, a->qa, a->qb, a->dqa, a->dqb, a->lq, a->rq, a->dk},
+                          {dkd, a->ka, a->kb, a->dka, a->dkb, a->lk, a->rk, a->dk},
+                          {dvd, a->va, a->vb, a->dva, a->dvb, a->lk, a->rk, a->dv}}};
   if (sizeof(T) == 2 && a->grad_dtype == TPA_DTYPE_BF16) {
-    if constexpr (sizeof(T) == 2) launch_project<T, uint16_t>(jobs, a->B, a->H, a->dk, a->dv, stream);
+    if constexpr (sizeof(T) == 2) launch_project<T, uint16_t>(jobs, a->B, a->H, stream);
   } else {
-    launch_project<T, float>(jobs, a->B, a->H, a->dk, a->dv, stream);
+    launch_project<T, float>(jobs, a->B, a->H, stream);
   }
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
