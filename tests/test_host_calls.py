@@ -95,3 +95,16 @@ def test_forward_mode_raises_instead_of_dropping_the_tangent(shapes, which):
     with fwd.dual_level(), pytest.raises(NotImplementedError):
         qkv[which] = fwd.make_dual(qkv[which], shapes(*qkv[which].shape))
         tpa.tpa(*qkv, H)
+
+
+@pytest.mark.parametrize("transform", ["vmap", "grad", "vjp", "jvp"])
+def test_function_transforms_are_refused(shapes, transform):
+    """The node has no rule for them: an error, never a result that ignores the transform."""
+    from tpa import tpa
+
+    q, k, v = shapes(B, LQ, RQ, H + D), shapes(B, LK, RK, H + D), shapes(B, LK, RK, H + D)
+    f = lambda x: tpa.tpa(x, k, v, H)
+    calls = dict(vmap=lambda: torch.vmap(f)(shapes(3, B, LQ, RQ, H + D)), grad=lambda: torch.func.grad(lambda x: f(x).sum())(q),
+                 vjp=lambda: torch.func.vjp(f, q), jvp=lambda: torch.func.jvp(f, (q,), (q,)))
+    with pytest.raises(RuntimeError, match="forward-mode|functorch|data pointer"):
+        calls[transform]()
