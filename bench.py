@@ -535,7 +535,7 @@ def main():
                 metric="TPA causal prefill backward throughput", value=bw["tflops_wall"], unit="TFLOP/s", ms_per_step=bw["wall_ms"],
                 roofline=dict(bound="mfma", achieved=bw["tflops_kernel"], peak=PEAK_BF16_TFLOPS, unit="TFLOP/s",
                               frac=bw["tflops_kernel"] / PEAK_BF16_TFLOPS, traffic=None,
-                              kernel="recon + delta + bwd_dq_kernel + bwd_dkv_kernel + project (whole call)",
+                              kernel="recon with delta + bwd_dq_dkv_kernel + project (whole call)",
                               **launch_times(bw),
                               algorithmic_flops_per_launch=bw["flops"]),
                 config=dict(workload="c2b: TPA backward", **bw["shape"]),
@@ -588,8 +588,8 @@ def main():
             metric="TPA causal prefill backward throughput", value=r["tflops_wall"], unit="TFLOP/s", ms_per_step=r["wall_ms"],
             roofline=dict(bound="mfma", achieved=r["tflops_kernel"], peak=peak, unit="TFLOP/s",
                           frac=r["tflops_kernel"] / peak, traffic=None,
-                          kernel=("recon + delta + bwd_f32_dq_kernel + bwd_f32_dkv_kernel + project (whole call)" if f32 else
-                                  "recon + delta + bwd_dq_kernel + bwd_dkv_kernel + project (whole call)"),
+                          kernel=("recon with delta + fp32 dq kernel + fp32 dk/dv kernel + project (whole call)" if f32 else
+                                  "recon with delta + bwd_dq_dkv_kernel + project (whole call)"),
                           **launch_times(r),
                           algorithmic_flops_per_launch=r["flops"]),
             config=dict(workload=f"{args.workload}: TPA backward" + (", fp32 inputs" if f32 else ""), **r["shape"]),

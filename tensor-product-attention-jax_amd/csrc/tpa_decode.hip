@@ -828,9 +828,12 @@ __global__ __launch_bounds__(D) void decode_merge_kernel(DecodeParams p, TO* o, 
     first = __builtin_amdgcn_readlane(plan.first, b);
   }
   // ranges are taken eight at a time with all their loads in flight together (one round trip to memory), or 24 at a
-  // time where all entries have the same number of more than eight (one sequence of 1500 keys in 24 ranges, with the decode:
-  // 11.6 -> 10.6 us; ranges dealt by length, 6 x 4 rows of about 21: 4.5 us eight at a time, 5.4 by 24);
-  // a running (max, sum, acc) triple carries across groups
+  // time where all entries have the same number of more than eight.  Decode and merge by 8 / 16 / 24 / 32, us, one sequence,
+  // 16 heads of 128, 64 keys per range: 9 to 16 ranges 10.6 / 9.8 / 10.4 / 11.0, 17 to 24 11.7 / 11.3 / 10.5 / 11.0, 25 to 32
+  // 12.9 / 11.4 / 12.4 / 11.1, 40 and 48 15.0 / 13.3 / 12.8 / 13.8, 64 17.4 / 14.9 / 14.8 / 14.0; the same order for 32 heads,
+  // four sequences, head size 64, four query rows and fp32.  With ranges dealt by length, where entries of few ranges pay for
+  // the empty places (6 x 4 rows of about 21 ranges), 24 lose: 4.5 us by eight, 5.4 by 24.
+  // A running (max, sum, acc) triple carries across groups
   float mmax = -INFINITY, acc = 0.f, lacc = 0.f;
   auto merge = [&](auto group_c) __attribute__((always_inline)) {
     constexpr int G = decltype(group_c)::value;
