@@ -40,6 +40,12 @@ void split(const ffi::AnyBuffer& x, int h, int code, TpaFactor* a, TpaFactor* b)
 
 ffi::Error fail(int rc) { return ffi::Error::InvalidArgument(std::string("libtpa_gfx950: ") + tpa_strerror(rc)); }
 
+// shape rules of tpa/tpa.py:475 on q[b, lq, rq, h + dk], k[b, lk, rk, h + dk], v[b, lk, rk, h + dv]
+template <typename Dims>
+bool shapes_fit(const Dims& qd, const Dims& kd, const Dims& vd, int32_t num_heads) {
+  return kd[0] == qd[0] && vd[0] == qd[0] && kd[1] == vd[1] && kd[2] == vd[2] && kd[3] == qd[3] && num_heads > 0 && qd[3] > num_heads && vd[3] > num_heads;
+}
+
 ffi::Error fill(TpaFwdArgs* a, const ffi::AnyBuffer& q, const ffi::AnyBuffer& k, const ffi::AnyBuffer& v,
                 ffi::Result<ffi::AnyBuffer>& o, ffi::Result<ffi::AnyBuffer>& lse, int32_t num_heads, float sm_scale,
                 bool causal) {
@@ -48,10 +54,7 @@ ffi::Error fill(TpaFwdArgs* a, const ffi::AnyBuffer& q, const ffi::AnyBuffer& k,
   const int code = dtype_code(q.element_type());
   if (code < 0 || k.element_type() != q.element_type() || v.element_type() != q.element_type())
     return ffi::Error::InvalidArgument("q, k, v must share one of f32 / bf16");
-  // shape rules of tpa/tpa.py:475
-  if (kd[0] != qd[0] || vd[0] != qd[0] || kd[1] != vd[1] || kd[2] != vd[2] || kd[3] != qd[3] || num_heads <= 0 ||
-      qd[3] <= num_heads || vd[3] <= num_heads)
-    return ffi::Error::InvalidArgument("inconsistent q / k / v shapes");
+  if (!shapes_fit(qd, kd, vd, num_heads)) return ffi::Error::InvalidArgument("inconsistent q / k / v shapes");
   // results: o[b, lq, h, dv] in the input type, lse[b, h, lq] fp32 (NOT the reference's l[b, lq, h] in
   // the input type, tpa/tpa.py:530: a caller that declares that shape for bf16 would be written past)
   const auto od = o->dimensions(), ld = lse->dimensions();
@@ -136,6 +139,8 @@ ffi::Error MhaFwdImpl(hipStream_t stream, ffi::AnyBuffer q, ffi::AnyBuffer k, ff
                       ffi::Result<ffi::AnyBuffer> workspace, float sm_scale, bool causal) {
   const auto qd = q.dimensions(), kd = k.dimensions(), vd = v.dimensions();
   if (qd.size() != 4 || kd.size() != 4 || vd.size() != 4) return ffi::Error::InvalidArgument("q, k, v must be [b, l, h, d]");
+  if (kd[0] != qd[0] || vd[0] != qd[0] || kd[1] != vd[1] || kd[2] != qd[2] || vd[2] != qd[2] || kd[3] != qd[3])
+    return ffi::Error::InvalidArgument("inconsistent q / k / v shapes");
   const auto od = o->dimensions(), ld = lse->dimensions();
   if (k.element_type() != q.element_type() || v.element_type() != q.element_type() || o->element_type() != q.element_type() ||
       od.size() != 4 || od[0] != qd[0] || od[1] != qd[1] || od[2] != qd[2] || od[3] != vd[3])
@@ -180,7 +185,10 @@ ffi::Error TpaBwdCommon(hipStream_t stream, const ffi::AnyBuffer& q, const ffi::
   if (lse.element_type() != ffi::DataType::F32 || dq->element_type() != ffi::DataType::F32 ||
       dk->element_type() != ffi::DataType::F32 || dv->element_type() != ffi::DataType::F32)
     return ffi::Error::InvalidArgument("lse and the gradients are f32");
-  const auto ld = lse.dimensions();
+  if (!shapes_fit(qd, kd, vd, num_heads)) return ffi::Error::InvalidArgument("inconsistent q / k / v shapes");
+  const auto od = o.dimensions(), ld = lse.dimensions();
+  if (od.size() != 4 || od[0] != qd[0] || od[1] != qd[1] || od[2] != num_heads || od[3] != vd[3] - num_heads)
+    return ffi::Error::InvalidArgument("o must be [b, lq, h, dv]");
   if (ld.size() != 3 || ld[0] != qd[0] || ld[1] != num_heads || ld[2] != qd[1]) return ffi::Error::InvalidArgument("lse must be [b, h, lq]");
   if (dq->dimensions() != qd || dk->dimensions() != kd || dv->dimensions() != vd || o.dimensions() != d_o.dimensions())
     return ffi::Error::InvalidArgument("gradients are shaped like q, k, v; do like o");
