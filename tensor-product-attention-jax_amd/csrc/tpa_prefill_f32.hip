@@ -1,29 +1,29 @@
-// Flash-style prefill for fp32 inputs on gfx950: fp32 MFMA contractions, fp32 online softmax.
+// Flash-style prefill for fp32 inputs on gfx950: fp32 contractions as split bf16 products, fp32 online softmax.
 //
 // Same decomposition as the bf16 kernel: one workgroup = one (batch, head, block of 256 query
-// rows), eight waves of 32 rows; per tile of 64 keys the workgroup rebuilds the head's K and V
-// tile from the rank factors (K = (1/R) sum_r a_r (x) b_r, tpa/tpa.py:364,417) into LDS, as fp32,
-// and each wave computes
-//     S^T = K Q^T      v_mfma_f32_32x32x2_f32; Q stays in registers, pre-scaled by
-//                      sm_scale*log2(e); each lane ends up with 32 logits of ONE query row
+// rows), eight waves of 32 rows; per tile of keys the workgroup rebuilds the head's K and V
+// tile from the rank factors (K = (1/R) sum_r a_r (x) b_r, tpa/tpa.py:364,417) in fp32, splits every
+// value into three bf16 parts (tpa_split3.h) and stages them as three planes in LDS; each wave computes
+//     S^T = K Q^T      six v_mfma_f32_32x32x16_bf16 per 16 values of d; Q stays in registers, pre-scaled by
+//                      sm_scale*log2(e) and split; each lane ends up with the logits of ONE query row
 //     online softmax   the recurrence of tpa/tpa.py:389-424 with the normalisation deferred
-//     O^T += V^T P^T   the S^T accumulator, turned into P in place, is the B operand
-// A 32x32x2 step takes two contraction indices, one per half of the wave.  Neither contraction
-// cares about the order of its index, so the halves walk it in the order that makes every LDS
-// operand read a 16-byte one: over d, half g takes d = 8m + 4g + e (m outer, e = 0..3 from one
-// read); over keys, half g takes the key its S^T register already belongs to; and the rows of a
-// 32-row block of O^T are d = (D/32) i + block, so one read of V[key][(D/32) i ...] feeds all
-// blocks and the epilogue stores whole vectors.
-// The matrix pipe is the bound by a wide margin (256 MFMAs of 64 cycles per wave and tile against
-// a few hundred vector instructions), so the loop is plain: rebuild the next tile, compute this
-// one, one barrier.  The dense baseline (tpa/mha.py:23-37) is the same kernel with rank 1 and
-// weight 1.
+//     O^T += V^T P^T   P is split in the registers of the logits it was made from
+// The contraction over keys does not care about their order, so the B operand of a step of 16 keys is the accumulator
+// as it is - half g of the wave holds keys 8q + 4g + 0..3 of two neighbouring q - and V is read transposed to match.
+// The fp32 matrix instruction, which this kernel used to be made of, takes 64 cycles for 2 contraction indices where the
+// six of a split take 192 for 16: 4 x 4096 tokens, 16 heads of 128 causal 2497 -> 1593 us (174 TFLOP/s where the fp32
+// instruction peaks at 157), 2 x 2000, 64 heads of 64 712 -> 487.  It is left for workgroups that meet values that do not
+// split (tpa_split3.h): these walk their tiles a second time.
+// The loop is plain: rebuild the next tile, compute this one, one barrier.  The dense baseline (tpa/mha.py:23-37) is the
+// same kernel with rank 1 and weight 1.
+#include <type_traits>
+
 #include "tpa_common.h"
+#include "tpa_split3.h"
 
 namespace tpa {
 namespace {
 
-constexpr int kTK = 64;   // keys per tile
 constexpr int kNW = 8;    // waves per workgroup (32 query rows each); half as many where 256-row blocks are too few
 
 struct F32Params {
@@ -40,21 +40,23 @@ struct F32Params {
 
 template <int D>
 struct LdsF32 {
-  static constexpr int RS = D + 4;        // row stride (floats): 16-byte reads of 16 rows hit distinct banks
-  static constexpr int kTile = kTK * RS;  // floats of one tile
-  static constexpr size_t kBytes = (size_t)(4 * kTile + 2 * kTK) * 4;  // K and V double buffered + key segment ids
+  static constexpr int kTK = D == 128 ? 32 : 64;  // keys per tile: two buffers of six planes fit the LDS
+  static constexpr int KS = D + 8, VS = D + 32;   // row strides (bf16): spread the banks for the row reads of K and the transposed ones of V
+  static constexpr int kKPlane = kTK * KS, kVPlane = kTK * VS;
+  static constexpr int kBuffer = 3 * (kKPlane + kVPlane);  // bf16 elements of one buffer
+  static constexpr size_t kBytes = (size_t)2 * kBuffer * 2 + 2 * kTK * 4;  // two buffers, key segment ids
 };
 
 template <int D, int NW, bool SEG>
 __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   constexpr int NT = NW * 64, kBQ = NW * 32;
-  constexpr int RS = LdsF32<D>::RS, kTile = LdsF32<D>::kTile;
+  typedef LdsF32<D> L;
+  constexpr int kTK = L::kTK, NMB = kTK / 32;  // keys of a tile, 32-key blocks
   constexpr int NDB = D / 32;         // 32-row blocks of O^T
-  constexpr int NQ = D / 2;           // Q values per lane
+  constexpr int NKS = D / 16;         // steps of the contraction over d
   constexpr int CPR = D / 4;          // 16-byte chunks per row
   constexpr int CH = kTK * CPR / NT;  // chunks per thread, tile and matrix
   static_assert(CH >= 1 && kTK * CPR % NT == 0, "loader shape");
-  typedef __attribute__((ext_vector_type(NDB))) float f32xN;
 
   struct Fac { const float* ptr; int64_t stride_b, stride_l, stride_r; };
   auto fac = [](const TpaFactor& f) { return Fac{static_cast<const float*>(f.ptr), f.stride_b, f.stride_l, f.stride_r}; };
@@ -63,9 +65,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
       pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk, pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.groups};
 
   extern __shared__ __attribute__((aligned(16))) float smem_f32[];
-  float* const lds_k = smem_f32;                                         // [2][kTK][RS]
-  float* const lds_v = smem_f32 + 2 * kTile;                             // [2][kTK][RS]
-  int32_t* const lds_seg = reinterpret_cast<int32_t*>(smem_f32 + 4 * kTile);  // [2][kTK]
+  uint16_t* const planes = reinterpret_cast<uint16_t*>(smem_f32);  // [2][K h, m, l; V h, m, l]
+  int32_t* const lds_seg = reinterpret_cast<int32_t*>(planes + 2 * L::kBuffer);  // [2][kTK]
 
   int pair, h;
   if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;  // heaviest causal blocks first
@@ -105,25 +106,42 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   const int ntiles = (kend - kbeg + kTK - 1) / kTK;
   const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + coff + 31 - kbeg, 0) / kTK) : ntiles - 1;
 
-  // ---- Q (B operand of S^T = K Q^T), scaled: qf[4m + e] = c * Q[qrow][8m + 4g + e]
-  float qf[NQ];
-#pragma unroll
-  for (int j = 0; j < NQ; ++j) qf[j] = 0.f;
+  // ---- Q (B operand of S^T = K Q^T), scaled and split: lane (i, g) holds Q[qrow][16 ks + 8 g + 0..7]
+  Split3 qf[NKS];
+  bool bad = false;  // this thread has met values that do not split
   {
-    const float* qb = p.qb.ptr + b * p.qb.stride_b + (int64_t)qrow_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * g;
-    const float* qa = dense ? nullptr : p.qa.ptr + b * p.qa.stride_b + (int64_t)qrow_ld * p.qa.stride_l + h;
-    for (int r = 0; r < p.rq; ++r) {
-      const float a = dense ? 1.f : qa[r * p.qa.stride_r];
-#pragma unroll
-      for (int m = 0; m < D / 8; ++m) {
-        const f32x4 bv = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r + 8 * m);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) qf[4 * m + e] += a * bv[e];
-      }
-    }
+    const float* const qb = p.qb.ptr + b * p.qb.stride_b + (int64_t)qrow_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 8 * g;
+    const float* const qa = dense ? nullptr : p.qa.ptr + b * p.qa.stride_b + (int64_t)qrow_ld * p.qa.stride_l + h;
     const float scale = p.sm_scale * kLog2e / (float)p.rq;
+    float top = 0.f;
+    constexpr int NH = NKS < 4 ? NKS : 4;  // steps at a time
 #pragma unroll
-    for (int j = 0; j < NQ; ++j) qf[j] *= scale;
+    for (int k0 = 0; k0 < NKS; k0 += NH) {
+      float q[NH][8];
+#pragma unroll
+      for (int ks = 0; ks < NH; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[ks][e] = 0.f;
+      for (int r = 0; r < p.rq; ++r) {
+        const float a = dense ? 1.f : qa[r * p.qa.stride_r];
+#pragma unroll
+        for (int j = 0; j < 2 * NH; ++j) {
+          const f32x4 bv = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r + 16 * (k0 + (j >> 1)) + 4 * (j & 1));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[j >> 1][4 * (j & 1) + e] += a * bv[e];
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < NH; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[ks][e] *= scale;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) top = largest(top, q[ks][e], q[ks][e + 1]);
+        qf[k0 + ks] = split8<true>(q[ks]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    bad = irregular(top);
   }
 
   // ---- tile rebuild: thread -> CH chunks of 4 floats per matrix
@@ -132,9 +150,24 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   const float* const ka_b = dense ? nullptr : p.ka.ptr + b * p.ka.stride_b + h;
   const float* const va_b = dense ? nullptr : p.va.ptr + b * p.va.stride_b + h;
   const float inv_r = 1.f / (float)p.rk;
-  auto rebuild = [&](int tile) __attribute__((always_inline)) {
-    float* const kd = lds_k + (tile & 1) * kTile;
-    float* const vd = lds_v + (tile & 1) * kTile;
+  // `fp32` is a compile-time flag here and below: the walk over the tiles that uses the fp32 instruction
+  auto stage = [&](auto fp32, uint16_t* at, int plane, const f32x4& x) __attribute__((always_inline)) {
+    Pair3 a, c;
+    if constexpr (decltype(fp32)::value) {
+      a = split_pair_any(x[0], x[1]);
+      c = split_pair_any(x[2], x[3]);
+    } else {
+      a = split_pair(x[0], x[1]);
+      c = split_pair(x[2], x[3]);
+      bad |= irregular(largest(largest(0.f, x[0], x[1]), x[2], x[3]));
+    }
+    *reinterpret_cast<u32x2*>(at) = u32x2{a.h, c.h};
+    *reinterpret_cast<u32x2*>(at + plane) = u32x2{a.m, c.m};
+    *reinterpret_cast<u32x2*>(at + 2 * plane) = u32x2{a.l, c.l};
+  };
+  auto rebuild = [&](auto fp32, int tile) __attribute__((always_inline)) {
+    uint16_t* const kd = planes + (tile & 1) * L::kBuffer;
+    uint16_t* const vd = kd + 3 * L::kKPlane;
 #pragma unroll
     for (int q = 0; q < CH; ++q) {
       const int chunk = q * NT + tid, t = chunk / CPR, cc = chunk % CPR;
@@ -150,49 +183,58 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
           av += wv * bv;
         }
       }
-      *reinterpret_cast<f32x4*>(kd + t * RS + 4 * cc) = ak * inv_r;
-      *reinterpret_cast<f32x4*>(vd + t * RS + 4 * cc) = av * inv_r;
+      stage(fp32, kd + t * L::KS + 4 * cc, L::kKPlane, ak * inv_r);
+      stage(fp32, vd + t * L::VS + 4 * cc, L::kVPlane, av * inv_r);
     }
     if constexpr (SEG)
       if (tid < kTK) lds_seg[(tile & 1) * kTK + tid] = p.kvseg[(int64_t)b * p.lk + min(kbeg + tile * kTK + tid, p.lk - 1)];
   };
+  auto row_operand = [&](const uint16_t* at) __attribute__((always_inline)) -> Split3 {  // eight values of a row of K
+    return {*reinterpret_cast<const bf16x8*>(at), *reinterpret_cast<const bf16x8*>(at + L::kKPlane), *reinterpret_cast<const bf16x8*>(at + 2 * L::kKPlane)};
+  };
 
   // ---- per-wave state
   f32x16 o[NDB];
-#pragma unroll
-  for (int db = 0; db < NDB; ++db)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) o[db][v] = 0.f;
-  float m_run = -INFINITY;  // running max of row qrow (log2 domain, scale included)
-  float lsum = 0.f;         // this lane's share of sum exp2(x - m_run)
+  float m_run, lsum;  // running max of row qrow (log2 domain, scale included); this lane's share of sum exp2(x - m_run)
   int32_t qseg = 0;
   if constexpr (SEG) qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
 
-  f32x16 s[2];  // logits, then probabilities, of the tile in flight: two 32-key blocks
-  auto logits_softmax = [&](int tile) __attribute__((always_inline)) {
-    const float* const ks = lds_k + (tile & 1) * kTile;
+  f32x16 s[NMB];  // logits, then probabilities, of the tile in flight
+  auto logits_softmax = [&](auto fp32, int tile) __attribute__((always_inline)) {
+    const uint16_t* const kt = planes + (tile & 1) * L::kBuffer + i * L::KS + 8 * g;
     const int k0 = kbeg + tile * kTK;
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) s[mb][v] = 0.f;
-    // the two blocks' accumulation chains alternate, so no MFMA waits for the one just issued
+    if constexpr (!decltype(fp32)::value) {
 #pragma unroll
-    for (int m = 0; m < D / 8; ++m) {
-      const f32x4 kf0 = *reinterpret_cast<const f32x4*>(ks + i * RS + 8 * m + 4 * g);
-      const f32x4 kf1 = *reinterpret_cast<const f32x4*>(ks + (32 + i) * RS + 8 * m + 4 * g);
+      for (int mb = 0; mb < NMB; ++mb) {
+        f32x16 small;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf0[e], qf[4 * m + e], s[0], 0, 0, 0);
-        s[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf1[e], qf[4 * m + e], s[1], 0, 0, 0);
+        for (int v = 0; v < 16; ++v) small[v] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+          const Split3 kf = row_operand(kt + 32 * mb * L::KS + 16 * ks);
+          mfma_small(kf, qf[ks], small);
+          s[mb] = mfma_bf16(kf.h, qf[ks].h, s[mb]);
+          if constexpr (D == 128) __builtin_amdgcn_sched_barrier(0);  // the operands of one step at a time: more do not fit the registers
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s[mb][v] += small[v];
       }
+    } else {
+#pragma unroll
+      for (int mb = 0; mb < NMB; ++mb)
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) mfma_joined(row_operand(kt + 32 * mb * L::KS + 16 * ks), qf[ks], s[mb]);
     }
     // register v of block mb, wave half g  <->  key k0 + 32 mb + 8 (v / 4) + 4 g + v % 4
     const bool need_mask = (k0 + kTK > kend) || (p.causal && (k0 + kTK - 1 > wrow0 + coff));
     if (need_mask) {
       const int limit = p.causal ? min(qrow + coff, kend - 1) : kend - 1;  // largest visible key index
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int t = k0 + 32 * mb + 8 * (v >> 2) + 4 * g + (v & 3);
@@ -202,7 +244,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
     if constexpr (SEG) {  // keys of another segment (tpa/tpa.py:369-375)
       const int32_t* idslot = lds_seg + (tile & 1) * kTK;
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq) {
           const int4 ids = *reinterpret_cast<const int4*>(idslot + 32 * mb + 8 * vq + 4 * g);
@@ -214,7 +256,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
     }
     float tmax = s[0][0];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) tmax = fmaxf(tmax, s[mb][v]);
     tmax = halves_max(tmax);
@@ -230,7 +272,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
         for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
     }
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const float pv = __builtin_amdgcn_exp2f(s[mb][v] - m_use);
@@ -238,69 +280,125 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
         s[mb][v] = pv;
       }
   };
-  // O^T += V^T P^T: the step of register v takes, in wave half g, the key that register belongs to
-  auto accumulate = [&](int tile) __attribute__((always_inline)) {
-    const float* const vs = lds_v + (tile & 1) * kTile;
+  // O^T += V^T P^T, 16 keys at a time: registers 8t .. 8t + 7 of a block are keys 8 (2t + u) + 4 g + 0..3 for u = 0, 1
+  const int lp = l & 15, dhalf = (l >> 4) & 1;
+  auto accumulate = [&](auto fp32, int tile) __attribute__((always_inline)) {
+    const uint16_t* const vt = planes + (tile & 1) * L::kBuffer + 3 * L::kKPlane + (4 * g + (lp >> 2)) * L::VS + 16 * dhalf + 4 * (lp & 3);
+    auto column_operand = [&](int mb, int t, int db) __attribute__((always_inline)) -> Split3 {
+      bf16x8 part[3];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+      for (int pl = 0; pl < 3; ++pl) {
+        const uint16_t* const at = vt + pl * L::kVPlane + (32 * mb + 16 * t) * L::VS + 32 * db;
+        const s16x4 u0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)at);
+        const s16x4 u1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(at + 8 * L::VS));
+        part[pl] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(u0, u1, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+      return {part[0], part[1], part[2]};
+    };
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int kr = 32 * mb + 8 * (v >> 2) + 4 * g + (v & 3);
-        const f32xN vf = *reinterpret_cast<const f32xN*>(vs + kr * RS + NDB * i);
+    for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db], s[mb][v], o[db], 0, 0, 0);
+      for (int t = 0; t < 2; ++t) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = s[mb][8 * t + e];
+        if constexpr (!decltype(fp32)::value) {
+          const Split3 pf = split8(x);
+#pragma unroll
+          for (int db = 0; db < NDB; db += 2) {  // the accumulation chains of two blocks alternate
+            const Split3 v0 = column_operand(mb, t, db), v1 = column_operand(mb, t, db + 1);
+            o[db] = mfma_bf16(v0.l, pf.h, o[db]);
+            o[db + 1] = mfma_bf16(v1.l, pf.h, o[db + 1]);
+            o[db] = mfma_bf16(v0.h, pf.l, o[db]);
+            o[db + 1] = mfma_bf16(v1.h, pf.l, o[db + 1]);
+            o[db] = mfma_bf16(v0.m, pf.m, o[db]);
+            o[db + 1] = mfma_bf16(v1.m, pf.m, o[db + 1]);
+            o[db] = mfma_bf16(v0.m, pf.h, o[db]);
+            o[db + 1] = mfma_bf16(v1.m, pf.h, o[db + 1]);
+            o[db] = mfma_bf16(v0.h, pf.m, o[db]);
+            o[db + 1] = mfma_bf16(v1.h, pf.m, o[db + 1]);
+            o[db] = mfma_bf16(v0.h, pf.h, o[db]);
+            o[db + 1] = mfma_bf16(v1.h, pf.h, o[db + 1]);
+            if constexpr (D == 128) __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            const Split3 vf = column_operand(mb, t, db);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(join(vf, e), x[e], o[db], 0, 0, 0);
+          }
+        }
       }
   };
 
-  rebuild(0);
-  __syncthreads();
-  // The next tile may be rebuilt anywhere between two barriers.  Waves w and w + 4 share a SIMD:
-  // one of them rebuilds (waiting for its factor loads) before its matrix work, the other in the
-  // middle of it, so the SIMD always has a wave with matrix work and both end the tile together.
-  const bool rebuild_first = w < NW / 2;
-  for (int j = 0; j < ntiles; ++j) {
-    const bool more = j + 1 < ntiles, mine = j <= wave_last_tile && wrow0 < p.lq;  // waves past the last row only help rebuild
-    if (rebuild_first && more) rebuild(j + 1);
-    if (mine) logits_softmax(j);
-    if (!rebuild_first && more) rebuild(j + 1);
-    if (mine) accumulate(j);
+  auto walk = [&](auto fp32) __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[db][v] = 0.f;
+    m_run = -INFINITY;
+    lsum = 0.f;
+    rebuild(fp32, 0);
     __syncthreads();
-  }
+    // The next tile may be rebuilt anywhere between two barriers.  Waves w and w + 4 share a SIMD:
+    // one of them rebuilds (waiting for its factor loads) before its matrix work, the other in the
+    // middle of it, so the SIMD always has a wave with matrix work and both end the tile together.
+    const bool rebuild_first = w < NW / 2;
+    for (int j = 0; j < ntiles; ++j) {
+      const bool more = j + 1 < ntiles, mine = j <= wave_last_tile && wrow0 < p.lq;  // waves past the last row only help rebuild
+      if (rebuild_first && more) rebuild(fp32, j + 1);
+      if (mine) logits_softmax(fp32, j);
+      if (!rebuild_first && more) rebuild(fp32, j + 1);
+      if (mine) accumulate(fp32, j);
+      __syncthreads();
+    }
+  };
+  walk(std::false_type{});
+  if (__builtin_expect(__syncthreads_or(bad), 0)) walk(std::true_type{});
 
-  // ---- epilogue: row 8 (v / 4) + 4 g + v % 4 of block db is d = NDB * row + db
+  // ---- epilogue: register v of block db is d = 32 db + 8 (v / 4) + 4 g + v % 4
   const float ltot = halves_sum(lsum);
   const float inv = 1.f / ltot;  // no visible key: 0 * inf = NaN, as in tpa/tpa.py:437-439
   if (qrow < p.lq) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int row = 8 * (v >> 2) + 4 * g + (v & 3);
-      f32xN out;
+    for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) out[db] = o[db][v] * inv;
-      *reinterpret_cast<f32xN*>(orow + NDB * row) = out;
-    }
+      for (int vq = 0; vq < 4; ++vq) {
+        f32x4 out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = o[db][4 * vq + e] * inv;
+        *reinterpret_cast<f32x4*>(orow + 32 * db + 8 * vq + 4 * g) = out;
+      }
     if (p.lse && g == 0) p.lse[((int64_t)b * p.H + h) * p.lq + qrow] = (m_run + __builtin_amdgcn_logf(ltot)) * kLn2;
   }
 }
 
 // ---------------------------------------------------------------------------------------------
 // The same for problems with few blocks of 256 query rows.  Such a launch leaves most of the chip idle and its time is
-// that of one workgroup walking all keys (one sequence of 512 tokens, 8 heads of 64: 16 workgroups, 75 us).  Here a
+// that of one workgroup walking all keys (one sequence of 512 tokens, 8 heads of 64: 16 workgroups, 53 us).  Here a
 // workgroup owns 32 query rows and its NW waves split the keys: wave w takes the tiles of 32 keys w, w + NW, ...,
-// rebuilds each into LDS of its own (no barrier in the loop) with the next tile's factors on their way while the matrix
-// pipe works on this one, and the partial results are merged through LDS with the rule of _lse_accum
-// (tpa/tpa.py:228-242).  Every workgroup rebuilds its tiles for 32 rows instead of 256, which is why the kernel above
+// rebuilds each into LDS of its own (no barrier in the loop; fp32, split on the way to the matrix cores: a value has one
+// reader) with the next tile's factors on their way while they work on this one, and the partial results are merged
+// through LDS with the rule of _lse_accum (tpa/tpa.py:228-242).  One workgroup's chain of loads, rebuild and two
+// contractions is the bound: 1 x 512 tokens, 8 heads of 64 causal 23.4 us with the fp32 instruction and offsets that the
+// compiler did not know to be scalar (a loop around every load), 17.1 so; 2 x 1000 51 -> 37.  Every workgroup rebuilds its tiles for 32 rows instead of 256, which is why the kernel above
 // stays the one for launches that fill the chip (`rows_per_workgroup` below).
-template <int D, int NW>
+template <int D>
 struct SplitLdsF32 {
+  // waves: two per SIMD cover each other's waits (four or eight, us, heads of 64: 1 x 128 tokens, 8 heads 9.6 / 8.6, 1 x 384
+  // 18.3 / 13.9, 4 x 448 27.5 / 22.5); at head size 128 the tiles of eight exceed the LDS
+  static constexpr int NW = D == 64 ? 8 : 4;
   static constexpr int RS = D + 4;
   static constexpr int kPerWave = 2 * 32 * RS;  // K and V tile; the merge reuses the K tile (O), its last columns (m, l)
-  static constexpr size_t kBytes = (size_t)(NW * kPerWave + 4) * 4;
+  static constexpr int QS = D + 8;              // row stride (bf16) of the parts of Q, which all waves read
+  static constexpr int kQPlane = 32 * QS;
+  static constexpr size_t kBytes = (size_t)NW * kPerWave * 4 + (size_t)3 * kQPlane * 2;
 };
 
-template <int D, int NW, bool SEG>
-__global__ __launch_bounds__(NW * 64, 1) void prefill_f32_split_kernel(F32Params p) {
-  constexpr int RS = SplitLdsF32<D, NW>::RS;
+template <int D, bool SEG, int RK>  // RK: rank of K and V, 0 = any
+__global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_kernel(F32Params p) {
+  constexpr int RS = SplitLdsF32<D>::RS, NW = SplitLdsF32<D>::NW;
   constexpr int NDB = D / 32, CPR = D / 4, RPI = 64 / CPR, NST = 32 / RPI;  // a load instruction of the wave takes RPI rows
   typedef __attribute__((ext_vector_type(NDB))) float f32xN;
 
@@ -310,10 +408,12 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_f32_split_kernel(F32Params
   const int qblk = p.nqb - 1 - pair / p.B;  // heaviest causal blocks first
   const int b = pair % p.B;
 
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  // the wave's index is a scalar: the scalar offsets of its buffer loads are made from it
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = qblk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
-  const bool dense = p.ka.ptr == nullptr;  // dense q, k, v: weight 1, the head's slice of the row
-  float* const lds_k = smem_f32_split + w * SplitLdsF32<D, NW>::kPerWave;  // [32][RS]
+  const int rk = RK ? RK : p.rk;
+  const bool dense = RK == 1 && p.ka.ptr == nullptr;  // dense q, k, v: weight 1, the head's slice of the row
+  float* const lds_k = smem_f32_split + w * SplitLdsF32<D>::kPerWave;  // [32][RS]
   float* const lds_v = lds_k + 32 * RS;
 
   const int len_b = p.kvlen ? max(0, min(p.kvlen[b], p.lk)) : p.lk;
@@ -330,42 +430,45 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_f32_split_kernel(F32Params
       kend = last < 0 ? 0 : last + 1;
     }
   }
+  kbeg = __builtin_amdgcn_readfirstlane(kbeg);
+  kend = __builtin_amdgcn_readfirstlane(kend);
   const int ntiles = kend > kbeg ? (kend - kbeg + 31) / 32 : 0;
 
   // Factor rows as raw buffer loads: per array one lane offset that never changes and a scalar one per load (with 64-bit
   // addresses per lane and load the kernel spilled 240 registers).  Tokens from kend on are inside the array or read as
   // zero; the last tile clears them (padding rows may hold anything, and 0 * NaN must not reach the sums).
-  const float inv_r = 1.f / (float)p.rk;
+  const float inv_r = 1.f / (float)rk;
   const int lrow = l / CPR, lc = l % CPR;
   struct Rows { __amdgpu_buffer_rsrc_t rs; int voff, sl, sr; };  // byte offset of the lane, bytes between tokens and ranks
   auto rows_of = [&](const TpaFactor& f, int64_t first, int lane_elem, int width) {
     const float* base = static_cast<const float*>(f.ptr) + b * f.stride_b + first;
-    const int64_t bytes = ((int64_t)(p.lk - 1) * f.stride_l + (int64_t)(p.rk - 1) * f.stride_r + width) * 4;
+    const int64_t bytes = ((int64_t)(p.lk - 1) * f.stride_l + (int64_t)(rk - 1) * f.stride_r + width) * 4;
     return Rows{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)bytes, 0x00020000),
                 (int)((lrow * f.stride_l + lane_elem) * 4), (int)(f.stride_l * 4), (int)(f.stride_r * 4)};
   };
   const Rows kb_r = rows_of(p.kb, dense ? (int64_t)h * D : 0, 4 * lc, D), vb_r = rows_of(p.vb, dense ? (int64_t)h * D : 0, 4 * lc, D);
   const Rows ka_r = dense ? kb_r : rows_of(p.ka, h, 0, 1), va_r = dense ? vb_r : rows_of(p.va, h, 0, 1);
   struct Flight { f32x4 x[NST]; float wt[NST]; };  // rows in flight and their weights (K's or V's, one rank)
-  Flight in;
   f32x4 vac[NST];  // the sum over V's ranks
   int32_t seg_in = 0, seg_id = 0;  // ids of key (this lane's i) of the next tile and of this one
-  auto issue_to = [&](Flight& in, const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) {
+  auto issue = [&](Flight& in, const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
       const int t = kbeg + tile * 32 + q * RPI;
       in.x[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb.rs, rb.voff, t * rb.sl + r * rb.sr, 0));
-      in.wt[q] = 1.f;
-      if (!dense) in.wt[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra.rs, ra.voff, t * ra.sl + r * ra.sr, 0));
+    }
+#pragma unroll
+    for (int q = 0; q < NST; ++q) {
+      const int t = kbeg + tile * 32 + q * RPI;
+      in.wt[q] = dense ? 1.f : __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra.rs, ra.voff, t * ra.sl + r * ra.sr, 0));
     }
   };
-  auto issue = [&](const Rows& rb, const Rows& ra, int tile, int r) __attribute__((always_inline)) { issue_to(in, rb, ra, tile, r); };
   auto row_of = [&](const Flight& in, int tile, int q) __attribute__((always_inline)) -> f32x4 {
     const f32x4 x = in.wt[q] * inv_r * in.x[q];
     return q * RPI + lrow < kend - kbeg - tile * 32 ? x : f32x4{0.f, 0.f, 0.f, 0.f};
   };
   // K is added up in its LDS tile (free once the logits are done), V in registers until its tile has been used
-  auto take_k_of = [&](const Flight& in, int tile, bool first) __attribute__((always_inline)) {
+  auto take_k = [&](const Flight& in, int tile, bool first) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
       f32x4* const at = reinterpret_cast<f32x4*>(lds_k + (q * RPI + lrow) * RS + 4 * lc);
@@ -373,35 +476,64 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_f32_split_kernel(F32Params
       *at = first ? x : *at + x;
     }
   };
-  auto take_k = [&](int tile, bool first) __attribute__((always_inline)) { take_k_of(in, tile, first); };
-  auto take_v = [&](int tile, bool first) __attribute__((always_inline)) {
+  auto take_v = [&](const Flight& in, int tile, bool first) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
       const f32x4 x = row_of(in, tile, q);
       vac[q] = first ? x : vac[q] + x;
     }
   };
-  auto store_v = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < NST; ++q) *reinterpret_cast<f32x4*>(lds_v + (q * RPI + lrow) * RS + 4 * lc) = vac[q];
-  };
   // all ranks but the last of one array: the first is on its way already, the last one is when this returns
-  auto ranks = [&](const Rows& rb, const Rows& ra, int tile, auto&& take) __attribute__((always_inline)) {
-    take(tile, true);
-    for (int r = 1; r + 1 < p.rk; ++r) {
-      issue(rb, ra, tile, r);
-      take(tile, false);
+  auto but_last = [&](Flight& in, const Rows& rb, const Rows& ra, int tile, auto&& take) __attribute__((always_inline)) {
+    if (rk == 1) return;
+    take(in, tile, true);
+    issue(in, rb, ra, tile, 1);
+    for (int r = 2; r < rk; ++r) {
+      take(in, tile, false);
+      issue(in, rb, ra, tile, r);
     }
-    if (p.rk > 1) issue(rb, ra, tile, p.rk - 1);
+  };
+  // the last ones; `bad`: this lane has met values that do not split
+  bool bad = false;
+  auto last_v = [&](const Flight& in, int tile) __attribute__((always_inline)) {
+    if (rk == 1) take_v(in, tile, true);
+    else take_v(in, tile, false);
+    float top = 0.f;
+#pragma unroll
+    for (int q = 0; q < NST; ++q) {
+      top = largest(largest(top, vac[q][0], vac[q][1]), vac[q][2], vac[q][3]);
+      *reinterpret_cast<f32x4*>(lds_v + (q * RPI + lrow) * RS + 4 * lc) = vac[q];
+    }
+    bad |= irregular(top);
+  };
+  auto last_k = [&](const Flight& in, int tile) __attribute__((always_inline)) {
+    float top = 0.f;
+    auto finish = [&](bool first) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < NST; ++q) {
+        f32x4* const at = reinterpret_cast<f32x4*>(lds_k + (q * RPI + lrow) * RS + 4 * lc);
+        f32x4 x = row_of(in, tile, q);
+        if (!first) x += *at;
+        top = largest(largest(top, x[0], x[1]), x[2], x[3]);
+        *at = x;
+      }
+    };
+    if (rk == 1) finish(true);
+    else finish(false);
+    bad |= irregular(top);
   };
 
-  Flight in_k;  // of the first tile only: its first ranks of V and of K travel together, ahead of Q's
-  if (w < ntiles) {
-    issue(vb_r, va_r, w, 0);
-    issue_to(in_k, kb_r, ka_r, w, 0);
-  }
-  // ---- Q, scaled, through LDS (the waves' tiles are not in use yet): the 32 rows are the same for all waves, and read in the
-  // layout of the operand every load of every wave would touch 32 cache lines
+  Flight in_v, in_k;
+  auto request_first = [&]() __attribute__((always_inline)) {
+    if (w < ntiles) {
+      issue(in_v, vb_r, va_r, w, 0);
+      issue(in_k, kb_r, ka_r, w, 0);
+    }
+  };
+  request_first();  // ahead of Q
+  // ---- Q, scaled and split (B operand of S^T = K Q^T): the 32 rows are the same for all waves, which read them from LDS
+  uint16_t* const lds_q = reinterpret_cast<uint16_t*>(smem_f32_split + NW * SplitLdsF32<D>::kPerWave);
+  float q_top = 0.f;
   for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
     const int row = idx / CPR, cc = idx % CPR, row_ld = min(q0 + row, p.lq - 1);
     const float* qb = static_cast<const float*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)row_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * cc;
@@ -421,137 +553,184 @@ __global__ __launch_bounds__(NW * 64, 1) void prefill_f32_split_kernel(F32Params
       for (int u = 0; u < G; ++u)
         if (r0 + u < p.rq) acc += a[u] * bv[u];
     }
-    *reinterpret_cast<f32x4*>(smem_f32_split + row * RS + 4 * cc) = acc * (p.sm_scale * kLog2e / (float)p.rq);
+    acc *= p.sm_scale * kLog2e / (float)p.rq;
+    q_top = largest(largest(q_top, acc[0], acc[1]), acc[2], acc[3]);
+    const Pair3 x = split_pair_any(acc[0], acc[1]), y = split_pair_any(acc[2], acc[3]);
+    uint16_t* const at = lds_q + row * SplitLdsF32<D>::QS + 4 * cc;
+    *reinterpret_cast<u32x2*>(at) = u32x2{x.h, y.h};
+    *reinterpret_cast<u32x2*>(at + SplitLdsF32<D>::kQPlane) = u32x2{x.m, y.m};
+    *reinterpret_cast<u32x2*>(at + 2 * SplitLdsF32<D>::kQPlane) = u32x2{x.l, y.l};
   }
+  bad = irregular(q_top);
   __syncthreads();
-  // B operand of S^T = K Q^T: qf[4m + e] = Q[qrow][8m + 4g + e]
-  float qf[D / 2];
-#pragma unroll
-  for (int m = 0; m < D / 8; ++m) {
-    const f32x4 x = *reinterpret_cast<const f32x4*>(smem_f32_split + i * RS + 8 * m + 4 * g);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) qf[4 * m + e] = x[e];
-  }
-  __syncthreads();
+  int q_offset = i * SplitLdsF32<D>::QS + 8 * g;
+  auto q_operand = [&](int ks) __attribute__((always_inline)) -> Split3 {
+    const uint16_t* const at = lds_q + q_offset + 16 * ks;
+    return {*reinterpret_cast<const bf16x8*>(at), *reinterpret_cast<const bf16x8*>(at + SplitLdsF32<D>::kQPlane),
+            *reinterpret_cast<const bf16x8*>(at + 2 * SplitLdsF32<D>::kQPlane)};
+  };
 
   f32x16 o[NDB];
+  float m_run, lsum;
+  auto walk = [&](auto fp32) __attribute__((always_inline)) {
 #pragma unroll
-  for (int db = 0; db < NDB; ++db)
+    for (int db = 0; db < NDB; ++db)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) o[db][v] = 0.f;
-  float m_run = -INFINITY, lsum = 0.f;
-
-  if (w < ntiles) {
-    ranks(vb_r, va_r, w, take_v);
-    take_k_of(in_k, w, true);
-    for (int r = 1; r < p.rk; ++r) {
-      issue_to(in_k, kb_r, ka_r, w, r);
-      if (r == 1) {
-        take_v(w, false);
-        store_v();
+      for (int v = 0; v < 16; ++v) o[db][v] = 0.f;
+    m_run = -INFINITY;
+    lsum = 0.f;
+    if (w < ntiles) {
+      but_last(in_v, vb_r, va_r, w, take_v);
+      but_last(in_k, kb_r, ka_r, w, take_k);
+      last_v(in_v, w);
+      last_k(in_k, w);
+      if constexpr (SEG) seg_id = p.kvseg[(int64_t)b * p.lk + min(kbeg + w * 32 + i, p.lk - 1)];
+    }
+    for (int tile = w; tile < ntiles; tile += NW) {
+      const int next = tile + NW;
+      const bool more = next < ntiles;
+      if (more) issue(in_v, vb_r, va_r, next, 0);
+      f32x16 s, s2;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) { s[v] = 0.f; s2[v] = 0.f; }
+      asm volatile("" : "+v"(q_offset));  // Q is read again for every tile: held in registers it would not fit
+      if constexpr (!decltype(fp32)::value) {
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) {
+          float x[8];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const f32x4 kf = *reinterpret_cast<const f32x4*>(lds_k + i * RS + 16 * ks + 8 * g + 4 * u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[4 * u + e] = kf[e];
+          }
+          const Split3 kf = split8(x), qf = q_operand(ks);
+          mfma_small(kf, qf, s2);
+          s = mfma_bf16(kf.h, qf.h, s);
+          __builtin_amdgcn_sched_barrier(0);  // the operands of one step at a time: more do not fit the registers
+        }
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) {
+          const Split3 qf = q_operand(ks);
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(lds_k[i * RS + 16 * ks + 8 * g + e], join(qf, e), s, 0, 0, 0);
+        }
       }
-      take_k_of(in_k, w, false);
-    }
-    if (p.rk == 1) store_v();
-    if constexpr (SEG) seg_id = p.kvseg[(int64_t)b * p.lk + min(kbeg + w * 32 + i, p.lk - 1)];
-  }
-  for (int tile = w; tile < ntiles; tile += NW) {
-    const int next = tile + NW;
-    const bool more = next < ntiles;
-    if (more) issue(vb_r, va_r, next, 0);
-    f32x16 s, s2;  // two accumulation chains, added at the end
-#pragma unroll
-    for (int v = 0; v < 16; ++v) { s[v] = 0.f; s2[v] = 0.f; }
-#pragma unroll
-    for (int m = 0; m < D / 8; ++m) {
-      if (m == D / 16 && more) ranks(vb_r, va_r, next, take_v);
-      const f32x4 kf = *reinterpret_cast<const f32x4*>(lds_k + i * RS + 8 * m + 4 * g);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[0], qf[4 * m], s, 0, 0, 0);
-      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[1], qf[4 * m + 1], s2, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[2], qf[4 * m + 2], s, 0, 0, 0);
-      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[3], qf[4 * m + 3], s2, 0, 0, 0);
-    }
-    if (more) {
-      if (p.rk > 1) take_v(next, false);
-      issue(kb_r, ka_r, next, 0);
-      if constexpr (SEG) seg_in = p.kvseg[(int64_t)b * p.lk + min(kbeg + next * 32 + i, p.lk - 1)];
-    }
-    // register v, wave half g  <->  key k0 + 8 (v / 4) + 4 g + v % 4
-    const int k0 = kbeg + tile * 32;
-    const int limit = p.causal ? min(qrow + coff, kend - 1) : kend - 1;  // largest visible key index
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int t = 8 * (v >> 2) + 4 * g + (v & 3);
-      bool keep = k0 + t <= limit;
-      if constexpr (SEG) {
-        const int32_t id_t = __shfl(seg_id, t, 64);  // by every lane, whatever it keeps
-        keep = keep && id_t == qseg;
+      if (more) {
+        but_last(in_v, vb_r, va_r, next, take_v);
+        issue(in_k, kb_r, ka_r, next, 0);
+        if constexpr (SEG) seg_in = p.kvseg[(int64_t)b * p.lk + min(kbeg + next * 32 + i, p.lk - 1)];
       }
-      s[v] = keep ? s[v] + s2[v] : -INFINITY;
-      tmax = fmaxf(tmax, s[v]);
-    }
-    tmax = halves_max(tmax);
-    const float m_new = fmaxf(m_run, tmax);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // a row that has met no visible key yet
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-    m_run = m_new;
-    if (__any(alpha != 1.f)) {
-      lsum *= alpha;
+      // register v, wave half g  <->  key k0 + 8 (v / 4) + 4 g + v % 4
+      const int k0 = kbeg + tile * 32;
+      const int limit = p.causal ? min(qrow + coff, kend - 1) : kend - 1;  // largest visible key index
+      float tmax = -INFINITY;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
+      for (int v = 0; v < 16; ++v) {
+        const int t = 8 * (v >> 2) + 4 * g + (v & 3);
+        bool keep = k0 + t <= limit;
+        if constexpr (SEG) {
+          const int32_t id_t = __shfl(seg_id, t, 64);  // by every lane, whatever it keeps
+          keep = keep && id_t == qseg;
+        }
+        s[v] = keep ? s[v] + s2[v] : -INFINITY;
+        tmax = fmaxf(tmax, s[v]);
+      }
+      tmax = halves_max(tmax);
+      const float m_new = fmaxf(m_run, tmax);
+      const float m_use = m_new == -INFINITY ? 0.f : m_new;  // a row that has met no visible key yet
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+      m_run = m_new;
+      if (__any(alpha != 1.f)) {
+        lsum *= alpha;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        s[v] = __builtin_amdgcn_exp2f(s[v] - m_use);
+        lsum += s[v];
+      }
+      // O^T += V^T P^T: 16 keys a step, in wave half g those its registers 8t .. 8t + 7 belong to
+      auto v_rows = [&](int v) __attribute__((always_inline)) -> f32xN {
+        return *reinterpret_cast<const f32xN*>(lds_v + (8 * (v >> 2) + 4 * g + (v & 3)) * RS + NDB * i);
+      };
+      if constexpr (!decltype(fp32)::value) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          if (t == 1 && more) but_last(in_k, kb_r, ka_r, next, take_k);
+          float x[8], y[NDB][8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            x[e] = s[8 * t + e];
+            const f32xN vf = v_rows(8 * t + e);
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) y[db][e] = vf[db];
+          }
+          const Split3 pf = split8(x);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            const Split3 vf = split8(y[db]);
+            mfma_small(vf, pf, o[db]);
+            o[db] = mfma_bf16(vf.h, pf.h, o[db]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          if (v == 8 && more) but_last(in_k, kb_r, ka_r, next, take_k);
+          const f32xN vf = v_rows(v);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db], s[v], o[db], 0, 0, 0);
+        }
+      }
+      if (more) {
+        last_v(in_v, next);
+        last_k(in_k, next);
+        if constexpr (SEG) seg_id = seg_in;
+      }
     }
+    // ---- for the merge of the waves: row i of a wave's O at lds_k + i RS, its m and l in the four padding columns
+    const float ltot = halves_sum(lsum);
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      s[v] = __builtin_amdgcn_exp2f(s[v] - m_use);
-      lsum += s[v];
+      const int row = 8 * (v >> 2) + 4 * g + (v & 3);  // of block db: d = NDB row + db
+      f32xN out;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) out[db] = o[db][v];
+      *reinterpret_cast<f32xN*>(lds_k + i * RS + NDB * row) = out;
     }
-    // O^T += V^T P^T: the step of register v takes, in wave half g, the key that register belongs to
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      if (v == 8 && more) ranks(kb_r, ka_r, next, take_k);
-      const f32xN vf = *reinterpret_cast<const f32xN*>(lds_v + (8 * (v >> 2) + 4 * g + (v & 3)) * RS + NDB * i);
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db], s[v], o[db], 0, 0, 0);
+    if (g == 0) {
+      lds_k[i * RS + D] = m_run;
+      lds_k[i * RS + D + 1] = ltot;
     }
-    if (more) {
-      if (p.rk > 1) take_k(next, false);
-      store_v();
-      if constexpr (SEG) seg_id = seg_in;
-    }
+  };
+  walk(std::false_type{});
+  if (__builtin_expect(__syncthreads_or(bad), 0)) {
+    request_first();
+    walk(std::true_type{});
+    __syncthreads();
   }
-
-  // ---- merge the waves: row i of a wave's O at lds_k + i RS, its m and l in the four padding columns
-  const float ltot = halves_sum(lsum);
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = 8 * (v >> 2) + 4 * g + (v & 3);  // of block db: d = NDB row + db
-    f32xN out;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) out[db] = o[db][v];
-    *reinterpret_cast<f32xN*>(lds_k + i * RS + NDB * row) = out;
-  }
-  if (g == 0) {
-    lds_k[i * RS + D] = m_run;
-    lds_k[i * RS + D + 1] = ltot;
-  }
-  __syncthreads();
+  // ---- merge the waves
   for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
     const int row = idx / CPR, cc = idx % CPR;
     if (q0 + row >= p.lq) continue;
     const float* const at = smem_f32_split + row * RS;
     float mmax = -INFINITY, lacc = 0.f;
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) mmax = fmaxf(mmax, at[ww * SplitLdsF32<D, NW>::kPerWave + D]);
+    for (int ww = 0; ww < NW; ++ww) mmax = fmaxf(mmax, at[ww * SplitLdsF32<D>::kPerWave + D]);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ww = 0; ww < NW; ++ww) {
-      const float mw = at[ww * SplitLdsF32<D, NW>::kPerWave + D];
+      const float mw = at[ww * SplitLdsF32<D>::kPerWave + D];
       const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mmax);
-      acc += f * *reinterpret_cast<const f32x4*>(at + ww * SplitLdsF32<D, NW>::kPerWave + 4 * cc);
-      lacc += f * at[ww * SplitLdsF32<D, NW>::kPerWave + D + 1];
+      acc += f * *reinterpret_cast<const f32x4*>(at + ww * SplitLdsF32<D>::kPerWave + 4 * cc);
+      lacc += f * at[ww * SplitLdsF32<D>::kPerWave + D + 1];
     }
     const float inv = 1.f / lacc;  // no visible key: 0 * inf = NaN, as in tpa/tpa.py:437-439
     *reinterpret_cast<f32x4*>(p.o + (((int64_t)b * p.lq + q0 + row) * p.H + h) * D + 4 * cc) = acc * inv;
@@ -567,24 +746,19 @@ bool split_supported(const F32Params& p) {
   return true;
 }
 
-// Eight waves instead of four where a wave then still has a tile and a half: two per SIMD cover each other's waits (four
-// hold 276 registers each, so that only one fits).  At head size 64 only: at 128 the tiles of eight waves exceed the LDS.
-// Measured, us, causal, heads of 64: 1 x 400
-// tokens, 16 heads 32.1 / 23.9; 1 x 512, 8 heads 32.1 / 23.1; 2 x 1000, 8 heads 69.3 / 51.4 (a quarter of it from Q
-// through LDS); 1 x 200, 8 heads 17.6 with four.
-bool eight_waves_pay(const F32Params& p) { return p.lk >= 384; }
-
 // Rows of a workgroup: 32 (keys split over its waves), 128 or 256.  A launch of 256-row workgroups that does not fill the
-// 256 compute units takes as long as one workgroup; with 128 rows (one wave per SIMD) a tile takes half the time, which
-// pays as long as they all fit the chip at once - under the causal mask, whose heaviest workgroup is twice the average,
-// up to two rounds.  Measured, us with 256 / 128 / 32 rows: 1 x 512 tokens, 8 heads of 64 causal 75 / 41 / 23; 2 x 1000
-// 144 / 69 / 51; not causal 4 x 1000 155 / 113 / 222, 8 x 1000 157 / 191 / 441.  32 causal rows at head size 64 also pay
-// for up to four rounds of long sequences, whose heaviest workgroup is twice the average however few there are: 4 x 1000
-// 146 / 113 / 102, 1 x 4000 489 with 256 / 294; but 1 x 512, 64 heads 64 / 65, and eight rounds: 8 x 1000 149 / 195.
+// 256 compute units takes as long as one workgroup walking all keys.  Measured, us with 256 / 128 / 32 rows:
+//   two rounds of 32-row workgroups at most: 1 x 512 tokens, 8 heads of 64 causal 53 / 52 / 17, 2 x 1000 95 / 97 / 38, not
+//   causal 100 / 98 / 57; 2 x 512, 16 heads of 128 causal 109 / 105 / 60
+//   up to four under the causal mask, whose heaviest workgroup is twice the average: 8 heads of 64, 8 x 512 56 / 55 / 51,
+//   4 x 1000 97 / 97 / 70, 1 x 4000 360 / 429 / 200, but eight rounds 8 x 1000 103 / 118 / 138; with heads of 128 only long
+//   sequences: 16 heads, 1 x 2000 360 / 422 / 332, 2 x 1000 188 / 209 / 188, 4 x 512 111 / 108 / 115
+//   short sequences whose 128-row workgroups fit the chip at once: 16 heads of 128, 8 x 256 71 / 66 / 78, 4 x 512 not
+//   causal 115 / 110 / 170, but 1 x 2000 371 / 435
 int rows_per_workgroup(const F32Params& p, int D) {
   auto wgs = [&](int rows) { return (int64_t)((p.lq + rows - 1) / rows) * p.B * p.H; };
-  if (wgs(32) <= (D == 64 && p.causal && p.lk >= 768 ? 1024 : 512) && split_supported(p)) return 32;
-  return wgs(128) <= 256 || (p.causal && wgs(256) <= 256) ? 128 : 256;
+  if (wgs(32) <= (p.causal && (D == 64 || p.lk >= 1536) ? 1024 : 512) && split_supported(p)) return 32;
+  return wgs(128) <= 256 && p.lk <= (p.causal ? 512 : 1024) ? 128 : 256;
 }
 
 template <typename K>
@@ -597,17 +771,23 @@ int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int threads
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
+template <int D, bool SEG, int RK>
+int launch_split(const F32Params& p, hipStream_t stream) {
+  static bool configured[kMaxDevices] = {};
+  constexpr int NW = SplitLdsF32<D>::NW;
+  return launch_kernel(prefill_f32_split_kernel<D, SEG, RK>, configured, 32, NW * 64, SplitLdsF32<D>::kBytes, p, stream);
+}
+
 template <int D, bool SEG>
 int launch_f32(const F32Params& p, hipStream_t stream) {
-  static bool configured[4][kMaxDevices] = {};
+  static bool configured[2][kMaxDevices] = {};
   const int rows = rows_per_workgroup(p, D);
   if (rows == 32) {
-    if constexpr (D == 64)
-      if (eight_waves_pay(p)) return launch_kernel(prefill_f32_split_kernel<D, 8, SEG>, configured[3], 32, 512, SplitLdsF32<D, 8>::kBytes, p, stream);
-    return launch_kernel(prefill_f32_split_kernel<D, 4, SEG>, configured[0], 32, 256, SplitLdsF32<D, 4>::kBytes, p, stream);
+    if (p.rk == 1) return launch_split<D, SEG, 1>(p, stream);
+    return p.rk == 2 ? launch_split<D, SEG, 2>(p, stream) : launch_split<D, SEG, 0>(p, stream);
   }
-  if (rows == 128) return launch_kernel(prefill_f32_kernel<D, kNW / 2, SEG>, configured[1], 128, kNW * 32, LdsF32<D>::kBytes, p, stream);
-  return launch_kernel(prefill_f32_kernel<D, kNW, SEG>, configured[2], 256, kNW * 64, LdsF32<D>::kBytes, p, stream);
+  if (rows == 128) return launch_kernel(prefill_f32_kernel<D, kNW / 2, SEG>, configured[0], 128, kNW * 32, LdsF32<D>::kBytes, p, stream);
+  return launch_kernel(prefill_f32_kernel<D, kNW, SEG>, configured[1], 256, kNW * 64, LdsF32<D>::kBytes, p, stream);
 }
 
 int launch_any(const F32Params& p, int d, hipStream_t stream) {
