@@ -59,6 +59,11 @@ __device__ __forceinline__ void store_from_f32<uint16_t>(uint16_t* p, float v) {
   *p = __builtin_bit_cast(uint16_t, b);
 }
 
+// A value that is the same in all lanes of a wave, as a scalar.  The compiler takes whatever is made from threadIdx.x or read
+// from LDS for a vector: branches on it mask lanes, and a buffer load whose scalar offset or resource is made from it
+// becomes a loop over the lanes' values.
+__device__ __forceinline__ int scalar(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
 // Combine a value with the one held by lane ^ 32.  v_permlane32_swap hands every lane both its
 // own value and its partner's (which of the two results holds which depends on the half the
 // lane is in), so order-independent reductions need no select.
@@ -126,8 +131,8 @@ __device__ __forceinline__ void id_window(const int32_t* mine, int n_mine, const
     __hip_atomic_fetch_max(&red[3], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
   __syncthreads();
-  first = red[2];
-  last = red[3];
+  first = scalar(red[2]);
+  last = scalar(red[3]);
   __syncthreads();  // the tiles reuse this memory
 }
 

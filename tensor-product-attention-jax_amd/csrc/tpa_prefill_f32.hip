@@ -74,7 +74,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   const int b = pair % p.B;
 
   const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  const int w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = qblk * kBQ;
   const int wrow0 = q0 + 32 * w;
   const int qrow = wrow0 + i;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
   const int b = pair % p.B;
 
   // the wave's index is a scalar: the scalar offsets of its buffer loads are made from it
-  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
+  const int tid = threadIdx.x, w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = qblk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
   const int rk = RK ? RK : p.rk;
   const bool dense = RK == 1 && p.ka.ptr == nullptr;  // dense q, k, v: weight 1, the head's slice of the row

@@ -1,4 +1,4 @@
-"""fp32 attention on the bf16 matrix cores (products of three-way splits): values that do not split - infinities, NaN, numbers
+"""fp32 attention, forward and backward, on the bf16 matrix cores (products of three-way splits): values that do not split - infinities, NaN, numbers
 that round up to infinity in bf16, numbers whose parts would be denormal - in each of the workgroup forms, against float64.
 
 Tolerance: the kernels' own error on ordinary values is below 1e-6 of the result's norm; 1e-5 leaves ten times that, and
@@ -78,3 +78,40 @@ def test_forward_values_that_do_not_split(gpu, b, t, h, d, rk, kind):
         if x.size:
             top = np.abs(y).max()
             assert np.linalg.norm((x - y) / top) <= 1e-5 * np.linalg.norm(y / top), c
+
+
+@pytest.mark.parametrize("kind", ["ordinary", "tiny gradient", "rounds to infinity", "large gradient"])
+@pytest.mark.parametrize(
+    "b,t,h,d,causal",
+    [
+        (1, 70, 2, 64, True),     # 32 rows, waves split the streamed tiles
+        (1, 70, 2, 128, False),
+        (1, 300, 64, 64, False),  # 192 blocks of 128 rows, four waves
+        (2, 300, 64, 64, False),  # 256 blocks of 256 rows, eight waves
+        (4, 390, 64, 64, True),   # 512 of them, causal
+        (2, 300, 32, 128, False),
+    ],
+)
+def test_backward_values_that_do_not_split(gpu, b, t, h, d, causal, kind):
+    from tpa import tpa
+
+    q, k, v = make_factors(83, b, t, t, h, d, d, 2, 2, scale_by_rank=True)
+    do = np.random.default_rng(84).standard_normal((b, t, h, d)).astype(np.float32)
+    if kind == "tiny gradient":
+        do *= np.float32(1e-28)
+    elif kind == "large gradient":  # dP and dS near the largest float
+        do *= np.float32(1e16)
+        v[..., h:] *= np.float32(1e20)
+    elif kind == "rounds to infinity":
+        _spoil(kind, q, k, v, h)
+        do[..., 7] *= np.float32(1e-30)
+    scale = d**-0.5
+    sp = lambda x: (torch.from_numpy(x[..., :h].copy()).to(gpu), torch.from_numpy(x[..., h:].copy()).to(gpu))
+    o, lse = tpa.tpa_factors(*sp(q), *sp(k), *sp(v), None, None, scale, causal, kernel=2)
+    grads = tpa.tpa_factors_bwd(*sp(q), *sp(k), *sp(v), None, None, o, lse, torch.from_numpy(do).to(gpu), scale, causal, kernel=2)
+    want = orc.tpa_backward(q, k, v, None, None, h, do, sm_scale=scale, causal=causal)
+    for n, w in enumerate(want):
+        got = np.concatenate([x.cpu().numpy() for x in grads[2 * n : 2 * n + 2]], axis=-1).astype(np.float64)
+        for x, y in ((got[..., :h], w[..., :h]), (got[..., h:], w[..., h:])):
+            top = np.abs(y).max()
+            assert np.linalg.norm((x - y) / top) <= 1e-5 * np.linalg.norm(y / top), "qkv"[n]
