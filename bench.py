@@ -374,11 +374,8 @@ def run_append(torch, tpa, device, name, steps, warmup):
     caches = [torch.zeros((B, cache_len, rk, inner), dtype=torch.bfloat16, device=device) for inner in (H, D, H, D)]
     lengths = torch.full((B,), cache_len - n - 1, dtype=torch.int32, device=device)
 
-    ws_bytes = tpa.cache_append_workspace_bytes(B, n, dm, H, D, rq, rk)  # decode steps split the contraction over workgroups
-    ws = torch.empty(ws_bytes + 16, dtype=torch.uint8, device=device) if ws_bytes else None
-
     def step(i):
-        tpa.tpa_cache_append(x, w, cos, sin, *caches, lengths, rank_q=rq, kernel=2, workspace=ws)
+        tpa.tpa_cache_append(x, w, cos, sin, *caches, lengths, rank_q=rq, kernel=2)
 
     t = time_steps(torch, step, steps, warmup)
     wall_ms, ev_ms, ev_min, ev_med = t["wall_ms"], t["kernel_ms"], t["kernel_ms_min"], t["kernel_ms_median"]
@@ -574,7 +571,7 @@ def main():
             unit="GB/s" if hbm else "TFLOP/s", ms_per_step=r["wall_ms"],
             roofline=dict(bound="hbm" if hbm else "mfma", achieved=ach, peak=PEAK_HBM_GBS if hbm else PEAK_BF16_TFLOPS,
                           unit="GB/s" if hbm else "TFLOP/s", frac=ach / (PEAK_HBM_GBS if hbm else PEAK_BF16_TFLOPS), traffic=None,
-                          kernel="append_fewrows_kernel + append_finish_kernel" if hbm else ("append_gemm_kernel<2>" if args.workload == "ap3" else "append_gemm_kernel<4>"), **launch_times(r),
+                          kernel="append_rows_kernel" if hbm else ("append_gemm_kernel<2>" if args.workload == "ap3" else "append_gemm_kernel<4>"), **launch_times(r),
                           algorithmic_flops_per_launch=r["flops"], algorithmic_bytes_per_launch=r["bytes"]),
             config=dict(workload=f"{args.workload}: TPA cache append", **r["shape"]),
         )

@@ -360,7 +360,7 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n) {
   a.rk = (int)ka.size(2); a.H = (int)ka.size(3); a.D = (int)kb.size(3); a.rq = (int)integer(args[12]);
   a.dtype = dtype_code(x.scalar_type());
   a.kernel = (int)integer(args[13]);
-  const bool use_workspace = integer(args[14]);
+  (void)integer(args[14]);  // use_workspace: no append kernel takes scratch memory any more
   expect(is_shape(w, {(int64_t)(a.rq + 2 * a.rk) * (a.H + a.D), a.d_model}), w);
   expect(kb.sizes().slice(0, 3) == ka.sizes().slice(0, 3) && va.sizes() == ka.sizes() && vb.sizes() == kb.sizes(), kb);
   expect(cos.sizes() == sin.sizes() && cos.dim() == 2 && cos.size(1) == a.D / 2, cos);
@@ -395,10 +395,6 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n) {
     qa = at::empty({a.B, a.n, a.rq, a.H}, options.dtype(x.scalar_type()));
     qb = at::empty({a.B, a.n, a.rq, a.D}, options.dtype(x.scalar_type()));
     new_len = at::empty({a.B}, options.dtype(at::kInt));
-    if (!ws.defined() && use_workspace && a.kernel != TPA_KERNEL_GENERIC) {
-      const size_t need = lib.tpa_cache_append_workspace_bytes(a.B, a.n, a.d_model, a.H, a.D, a.rq, a.rk, a.dtype);
-      if (need) ws = bytes_on(device, need + 16);
-    }
     if (ws.defined()) {
       a.workspace = aligned(ws, 16);
       a.workspace_bytes = ws.numel() * ws.element_size() - (static_cast<char*>(a.workspace) - static_cast<char*>(ws.data_ptr()));

@@ -4,9 +4,9 @@
 // prefill kernels read.  The reference has no such step (its tests draw the factors at random,
 // tpa/tpa_test.py:86-91); the arithmetic follows arXiv 2501.06425, section 3.
 //
-// bf16, three kernels by the number of new tokens: 256 x 256 tiles once they fill the chip (a prefill
-// chunk), 64 x 64 tiles below that, and for a decode step (at most 64 tokens in all) a kernel that
-// splits the contraction instead of the tokens.  All of them compute with v_mfma_f32_*_bf16, stage the
+// bf16, three kernels by the number of new tokens: 256 x 256 or 128 x 128 tiles once they fill the chip (a prefill
+// chunk), 64 x 64 tiles below that, and for a decode step and other few tokens a kernel whose workgroups own 16 columns
+// and split the contraction over their waves.  All of them compute with v_mfma_f32_*_bf16, stage the
 // fp32 results in LDS, and finish whole 16-byte chunks of eight columns: a chunk lies inside one rank
 // row of one factor (H and D are multiples of 8), so the rotation partners (2j, 2j+1) are inside it.
 // Any other dtype / shape: one thread per chunk of eight columns, fp32 arithmetic.
@@ -48,8 +48,6 @@ struct AppendParams {
   int B, n, K, H, D, rq, rk, cache_len, rope_len;
   int M, N;          // tokens (B * n), output columns
   int seg[7];        // first column of qa, qb, ka, kb, va, vb, and N
-  float* partial;    // decode-step kernel with the contraction split over workgroups: [slabs][kFewTokens][N] fp32
-  int slabs;
 };
 
 // Where chunk (token m, columns c0 .. c0 + 7) of y goes: the factor it belongs to, and the address
@@ -456,124 +454,139 @@ __global__ __launch_bounds__(256 * KS) void append_gemm_kernel(AppendParams p) {
   }
 }
 
-// ---- bf16, at most 64 new tokens in all (a decode step): the call is one read of W, and 64 x 64 tiles
-// would leave most of the chip idle.  Operands go from global memory straight into
-// v_mfma_f32_16x16x32_bf16 fragments (a lane holds 8 consecutive k of one token / one row of W, which
-// is how both arrays lie in memory); the eight waves of a workgroup split its share of k, their partial
-// tiles meet in LDS and one thread per chunk of eight columns finishes.
-// What bounds it: a wave ingests fragments as half cache lines (16 rows x 64 bytes per load
-// instruction), about 18 bytes per clock and CU, and every workgroup needs all 64 tokens of x for its
-// share of k.  Without a workspace a workgroup owns 16 columns and all of k (100 workgroups at 1600
-// columns; x alone is 512 KB per workgroup, 14 of the kernel's 22 us at d_model = 4096).  With a
-// workspace the contraction is also split over `slabs` workgroups (blockIdx.y) that own 64 columns
-// each: x is then read once per 64 columns and slab, the fp32 partial tiles go to the workspace and
-// append_finish_kernel adds them up and finishes.
-// U = k steps of 32 whose loads are in flight together, NCB = blocks of 16 columns per workgroup.
-constexpr int kFewTokens = 64, kFewWaves = 8;
-template <int U, int NCB>
-__global__ __launch_bounds__(kFewWaves * 64) void append_fewrows_kernel(AppendParams p) {
-  constexpr int kCols = 16 * NCB;
-  extern __shared__ __attribute__((aligned(16))) float part_mem[];  // [kFewWaves][kFewTokens][kCols + 4]
-  auto part = [&](int ww, int m, int c) -> float& { return part_mem[(ww * kFewTokens + m) * (kCols + 4) + c]; };
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r16 = l & 15, kg = l >> 4;
-  const int n0 = blockIdx.x * kCols;
-  const uint16_t* x = static_cast<const uint16_t*>(p.x);
-  const uint16_t* wt = static_cast<const uint16_t*>(p.w);
-  const int kw = p.K / (kFewWaves * p.slabs), k_begin = (blockIdx.y * kFewWaves + w) * kw;  // this wave's share of the contraction
-  const uint16_t* wrow[NCB];
+// ---- bf16, few tokens (a decode step): the call is one read of W, and tiles of 64 columns would leave most of the chip idle.
+// A workgroup owns 16 columns, up to 64 tokens and all of k: its eight waves deal the chunks of 64 k round robin, each stages
+// its own chunk (16 rows of W and the tokens' rows, whole cache lines in 16-byte pieces, kept in flight in registers several
+// chunks ahead) in LDS of its own, swizzled, and multiplies it with v_mfma_f32_16x16x32_bf16 - no barrier before the end,
+// where a ninth wave, which has looked up destinations and angles meanwhile, adds the eight partial tiles and stores.
+// What bounds it: bytes through the compute unit, 128 KB of W (d_model 4096) and 8 KB per token, at some 40 bytes a clock
+// behind the first one's way from HBM; hence the tokens are dealt to more workgroups while there are idle ones.
+// (Until now operands were read as fragments, half a cache line per row, and the contraction was split over workgroups with
+// a second kernel to add the parts.  d_model 4096, us before / now: 1 token x 1600 columns 10.9 / 7.2, 24 x 1440 11.6 / 7.6,
+// 48 x 1600 13.5 / 9.5, 64 x 4096 23.5 / 15.3; above 64 tokens against 64 x 64 tiles: 128 x 1600 50 / 13.6, 256 x 1600
+// 50 / 22, 256 x 4096 50 / 44.)
+template <int MB>
+struct RowsTile {
+  static constexpr int kTok = 16 * MB;
+  static constexpr int kRows = 16 + kTok;           // staged rows: 16 of W, then the tokens
+  static constexpr int kStage = kRows * 64;         // elements of a wave's stage, one chunk of 64 k
+  static constexpr int kPS = 20;                    // row stride (floats) of the partial tile, which reuses the stage
+  static constexpr int NLD = kRows / 8;             // load instructions of a chunk: 8 rows x 128 bytes each
+  static constexpr int NSET = MB >= 4 ? 2 : MB == 2 ? 4 : 6;  // chunks in flight in registers
+  static_assert(kTok * kPS * 4 <= kStage * 2, "the partial tile fits the stage");
+};
+constexpr int kRowWaves = 8;
+template <int MB>
+__global__ __launch_bounds__((kRowWaves + 1) * 64) void append_rows_kernel(AppendParams p, int nct, int ntb) {
+  typedef RowsTile<MB> T;
+  constexpr int NLD = T::NLD, NSET = T::NSET;
+  extern __shared__ __attribute__((aligned(16))) uint16_t stage_mem[];  // [kRowWaves][kStage]
+  const int tid = threadIdx.x, w = scalar(tid >> 6), l = tid & 63;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int ct = slot / ntb * 8 + xcd, tb = slot % ntb;
+  if (ct >= nct) return;  // the grid is rounded up to whole groups of 8 column blocks
+  const int n0 = 16 * ct, m0 = T::kTok * tb;
+  if (w < kRowWaves) {
+    const int nchunks = p.K / 64, lrow = l >> 3, lc = l & 7;
+    // buffer loads: the resource ends with the last row of the block that exists, rows past it read as zero
+    constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
+    const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.w) + (int64_t)n0 * p.K), 0, min(16, p.N - n0) * p.K * 2, kRsrcFlags);
+    const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.x) + (int64_t)m0 * p.K), 0, min(T::kTok, p.M - m0) * p.K * 2, kRsrcFlags);
+    const int voff = (lrow * p.K + 8 * lc) * 2;
+    uint16_t* const st = stage_mem + w * T::kStage;
+    u32x4 in[NSET][NLD];
+    auto load = [&](auto set_c, int chunk) __attribute__((always_inline)) {
+      constexpr int set = decltype(set_c)::value;
 #pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) wrow[cb] = wt + (int64_t)min(n0 + 16 * cb + r16, p.N - 1) * p.K + k_begin + 8 * kg;
-  const uint16_t* xrow[4];
+      for (int q = 0; q < NLD; ++q)
+        in[set][q] = __builtin_amdgcn_raw_buffer_load_b128(q < 2 ? w_rs : x_rs, voff, ((q < 2 ? q : q - 2) * 8 * p.K + 64 * chunk) * 2, 0);
+    };
+    f32x4 acc[MB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) xrow[mb] = x + (int64_t)min(16 * mb + r16, p.M - 1) * p.K + k_begin + 8 * kg;
-  // (all four blocks of 16 tokens are always computed: rows past the last token repeat it and are dropped
-  // at the end - branches around the loads would keep them from being in flight together)
-  f32x4 acc[4][NCB];
+    for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int r16 = l & 15, kg = l >> 4;
+    auto take = [&](auto set_c) __attribute__((always_inline)) {
+      constexpr int set = decltype(set_c)::value;
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+      for (int q = 0; q < NLD; ++q) *reinterpret_cast<u32x4*>(st + (8 * q + lrow) * 64 + 8 * (lc ^ lrow)) = in[set][q];
+    };
+    auto multiply = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) acc[mb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < kw; k0 += 32 * U) {
-    bf16x8 bq[U][NCB], a[U][4];
+      for (int ks = 0; ks < 2; ++ks) {
+        const int at = r16 * 64 + 8 * ((4 * ks + kg) ^ (r16 & 7));
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(st + at);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+        for (int mb = 0; mb < MB; ++mb)
+          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(st + (16 + 16 * mb) * 64 + at), b, acc[mb], 0, 0, 0);
+      }
+    };
+    static_for<NSET>([&](auto n) __attribute__((always_inline)) {
+      if (w + kRowWaves * decltype(n)::value < nchunks) load(n, w + kRowWaves * decltype(n)::value);
+    });
+    for (int c0 = w; c0 < nchunks; c0 += kRowWaves * NSET)
+      static_for<NSET>([&](auto n) __attribute__((always_inline)) {
+        const int c = c0 + kRowWaves * decltype(n)::value;
+        if (c < nchunks) {
+          take(n);
+          if (c + kRowWaves * NSET < nchunks) load(n, c + kRowWaves * NSET);
+          multiply();
+        }
+      });
+    // acc[mb][v] = partial y[token m0 + 16 mb + 4 kg + v][column n0 + r16]
+    float* const part = reinterpret_cast<float*>(st);
 #pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) bq[u][cb] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wrow[cb] + k0 + 32 * u));
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) a[u][mb] = *reinterpret_cast<const bf16x8*>(xrow[mb] + k0 + 32 * u);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // every load of the group is issued before the first matrix instruction waits
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) acc[mb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][mb], bq[u][cb], acc[mb][cb], 0, 0, 0);
+      for (int v = 0; v < 4; ++v) part[(16 * mb + 4 * kg + v) * T::kPS + r16] = acc[mb][v];
+    __syncthreads();
+    if (blockIdx.x == 0 && w == 0 && p.new_kvlen)
+      for (int b = l; b < p.B; b += 64) p.new_kvlen[b] = min((p.kvlen ? max(0, min(p.kvlen[b], p.cache_len)) : 0) + p.n, p.cache_len);
+    return;
   }
-  // acc[mb][cb][v] = partial y[token 16 mb + 4 kg + v][column n0 + 16 cb + r16]
+  // the last wave looks up where the results go and their angles while the others multiply, then adds and stores
+  constexpr int NC = (2 * T::kTok + 63) / 64;  // chunks of eight columns per lane
+  uint16_t* dst[NC];
+  float cs[NC][4], sn[NC][4];
+  bool rotate[NC];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int u = 0; u < NC; ++u) {
+    const int t = (64 * u + l) >> 1, c0 = n0 + 8 * (l & 1);
+    const bool live = t < T::kTok && m0 + t < p.M && c0 < p.N;
+    int j0 = 0, pos = 0;
+    dst[u] = nullptr;
+    rotate[u] = false;
+    if (live) dst[u] = chunk_destination<uint16_t>(p, m0 + t, c0, rotate[u], j0, pos);
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) part(w, 16 * mb + 4 * kg + v, 16 * cb + r16) = acc[mb][cb][v];
+    for (int j = 0; j < 4; ++j) {
+      cs[u][j] = rotate[u] ? p.cosv[(int64_t)pos * (p.D / 2) + j0 + j] : 1.f;
+      sn[u][j] = rotate[u] ? p.sinv[(int64_t)pos * (p.D / 2) + j0 + j] : 0.f;
+    }
+  }
   __syncthreads();
-  for (int idx = tid; idx < kFewTokens * (kCols / 8); idx += kFewWaves * 64) {
-    const int m = idx / (kCols / 8), cc = idx % (kCols / 8), c0 = n0 + 8 * cc;
-    if (m >= p.M || c0 >= p.N) continue;
+#pragma unroll
+  for (int u = 0; u < NC; ++u) {
+    if (!dst[u]) continue;
+    const int t = (64 * u + l) >> 1;
     float y[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) y[j] = 0.f;
 #pragma unroll
-    for (int ww = 0; ww < kFewWaves; ++ww) {
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(&part(ww, m, 8 * cc)), hi = *reinterpret_cast<const f32x4*>(&part(ww, m, 8 * cc + 4));
+    for (int ww = 0; ww < kRowWaves; ++ww) {
+      const float* const src = reinterpret_cast<const float*>(stage_mem + ww * T::kStage) + t * T::kPS + 8 * (l & 1);
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) { y[j] += lo[j]; y[4 + j] += hi[j]; }
     }
-    if (p.partial) {  // this slab's share of the chunk; append_finish_kernel takes it from there
-      float* dst = p.partial + ((int64_t)blockIdx.y * kFewTokens + m) * p.N + c0;
-      *reinterpret_cast<f32x4*>(dst) = f32x4{y[0], y[1], y[2], y[3]};
-      *reinterpret_cast<f32x4*>(dst + 4) = f32x4{y[4], y[5], y[6], y[7]};
-      continue;
+    if (rotate[u]) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float a = y[2 * j], b = y[2 * j + 1];
+        y[2 * j] = a * cs[u][j] - b * sn[u][j];
+        y[2 * j + 1] = b * cs[u][j] + a * sn[u][j];
+      }
     }
-    bool rotate; int j0, pos;
-    uint16_t* dst = chunk_destination<uint16_t>(p, m, c0, rotate, j0, pos);
-    if (dst) {
-      if (rotate) rotate_chunk(p, y, pos, j0);
-      store_chunk(dst, y);
-    }
+    store_chunk(dst[u], y);
   }
-  if (!p.partial) write_new_lengths(p);  // (with partial sums the finishing kernel writes them)
-}
-
-// second kernel of the split decode step: eight lanes per chunk of eight columns, one per slab of k; they add
-// their partial sums with three exchanges and the first of them finishes the chunk
-__global__ __launch_bounds__(256) void append_finish_kernel(AppendParams p) {
-  const int idx = (blockIdx.x * 256 + threadIdx.x) >> 3, sl = threadIdx.x & 7, nchunks = p.N / 8;
-  const bool live = idx < p.M * nchunks;
-  const int m = live ? idx / nchunks : 0, c0 = live ? 8 * (idx % nchunks) : 0;
-  float y[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) y[j] = 0.f;
-  if (live && sl < p.slabs) {
-    const float* src = p.partial + ((int64_t)sl * kFewTokens + m) * p.N + c0;
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { y[j] = lo[j]; y[4 + j] = hi[j]; }
-  }
-#pragma unroll
-  for (int off = 1; off < 8; off <<= 1)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] += __shfl_xor(y[j], off);
-  if (live && sl == 0) {
-    bool rotate; int j0, pos;
-    uint16_t* dst = chunk_destination<uint16_t>(p, m, c0, rotate, j0, pos);
-    if (dst) {
-      if (rotate) rotate_chunk(p, y, pos, j0);
-      store_chunk(dst, y);
-    }
-  }
-  write_new_lengths(p);
 }
 
 // ---- any dtype and shape: one thread per chunk of eight columns
@@ -627,20 +640,19 @@ int launch_gemm(const AppendParams& p, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
-// slabs of k that a split decode step uses: as many as 8, each a whole number of k steps per wave
-int few_slabs(int d_model) {
-  for (int sl = 8; sl > 1; sl >>= 1)
-    if (d_model % (32 * kFewWaves * sl) == 0) return sl;
-  return 1;
-}
+// The few-token kernel serves calls of at most three rounds of its workgroups of 64 tokens (d_model 4096, us against 64 x 64
+// tiles: 768 tokens x 960 columns, 720 workgroups, 31 / 43; 1024 x 720, 720, 35 / 37; 1200 x 720, 855, 48 / 37; 1024 x 960,
+// 960, 45 / 38).
+bool few_tokens(const AppendParams& p) { return (int64_t)((p.N + 15) / 16) * ((p.M + 63) / 64) <= 768; }
 
-template <int U, int NCB>
-int launch_fewrows(const AppendParams& p, hipStream_t s) {
-  auto kern = append_fewrows_kernel<U, NCB>;
-  const size_t lds = (size_t)kFewWaves * kFewTokens * (16 * NCB + 4) * sizeof(float);
+template <int MB>
+int launch_rows(const AppendParams& p, hipStream_t s) {
+  const int nct = (p.N + 15) / 16, ntb = (p.M + 16 * MB - 1) / (16 * MB);
+  const size_t lds = (size_t)kRowWaves * RowsTile<MB>::kStage * sizeof(uint16_t);
+  auto kern = append_rows_kernel<MB>;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((p.N + 16 * NCB - 1) / (16 * NCB), p.slabs), dim3(kFewWaves * 64), lds, s, p);
+  hipLaunchKernelGGL(kern, dim3((nct + 7) / 8 * 8 * ntb), dim3((kRowWaves + 1) * 64), lds, s, p, nct, ntb);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 bool chunk_ok(const TpaFactor& f) { return aligned16(f.ptr) && f.stride_b % 8 == 0 && f.stride_l % 8 == 0 && f.stride_r % 8 == 0; }
@@ -648,14 +660,13 @@ bool chunk_ok(const TpaFactor& f) { return aligned16(f.ptr) && f.stride_b % 8 ==
 }  // namespace
 }  // namespace tpa
 
+// (The size that the decode step's two kernels needed while there were two.)
 extern "C" size_t tpa_cache_append_workspace_bytes(int32_t B, int32_t n, int32_t d_model, int32_t H, int32_t D, int32_t rq, int32_t rk, int32_t dtype) {
-  using namespace tpa;
   if (B <= 0 || n <= 0 || d_model <= 0 || H <= 0 || D <= 0 || rq <= 0 || rk <= 0 || dtype != TPA_DTYPE_BF16) return 0;
-  if ((int64_t)B * n > kFewTokens || H % 8 != 0 || D % 8 != 0) return 0;
-  const int slabs = few_slabs(d_model);
-  if (slabs == 1) return 0;
-  const int64_t n_out = (int64_t)(rq + 2 * rk) * (H + D);
-  return (size_t)slabs * kFewTokens * n_out * sizeof(float);
+  if ((int64_t)B * n > 64 || H % 8 != 0 || D % 8 != 0) return 0;
+  for (int slabs = 8; slabs > 1; slabs >>= 1)
+    if (d_model % (256 * slabs) == 0) return (size_t)slabs * 64 * (rq + 2 * rk) * (H + D) * sizeof(float);
+  return 0;
 }
 
 extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
@@ -693,17 +704,12 @@ extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
   bool mfma = a->kernel != TPA_KERNEL_GENERIC && a->dtype == TPA_DTYPE_BF16 && a->d_model % kBK == 0 && aligned16(a->x) && aligned16(a->w);
   for (const TpaFactor* f : fs) mfma = mfma && chunk_ok(*f);
   if (a->kernel == TPA_KERNEL_MFMA && !mfma) return TPA_ERR_UNSUPPORTED;
-  if (mfma && p.M <= kFewTokens && a->d_model % (32 * kFewWaves) == 0) {
-    const size_t need = tpa_cache_append_workspace_bytes(a->B, a->n, a->d_model, a->H, a->D, a->rq, a->rk, a->dtype);
-    const bool split = need && a->workspace && a->workspace_bytes >= need && aligned16(a->workspace);
-    p.slabs = split ? few_slabs(a->d_model) : 1;
-    p.partial = split ? static_cast<float*>(a->workspace) : nullptr;
-    const int steps = a->d_model / (32 * kFewWaves * p.slabs);  // k steps of 32 per wave
-    int rc;
-    if (split) rc = steps % 4 == 0 ? launch_fewrows<4, 4>(p, s) : steps % 2 == 0 ? launch_fewrows<2, 4>(p, s) : launch_fewrows<1, 4>(p, s);
-    else rc = steps % 4 == 0 ? launch_fewrows<4, 1>(p, s) : launch_fewrows<1, 1>(p, s);
+  if (mfma && few_tokens(p)) {
+    // as many tokens per workgroup as let the call fit the 256 compute units at once (d_model 4096, us with 16 / 32 / 64: 32
+    // tokens x 1600 columns 8.2 / 10.7 / 11.2, 64 x 1600 11.5 / 10.7 / 14.0, 128 x 1600 20 / 16 / 13.6, 64 x 4096 24 / 19 / 15)
+    const int nct = (p.N + 15) / 16;
+    const int rc = nct * ((p.M + 15) / 16) <= 256 ? launch_rows<1>(p, s) : nct * ((p.M + 31) / 32) <= 256 ? launch_rows<2>(p, s) : launch_rows<4>(p, s);
     if (rc != TPA_OK) return rc;
-    if (split) hipLaunchKernelGGL(append_finish_kernel, dim3((p.M * (p.N / 8) * 8 + 255) / 256), dim3(256), 0, s, p);
   } else if (mfma && gemm_tiles_pay<4>(p, a)) {
     if (int rc = launch_gemm<4, 1>(p, s); rc != TPA_OK) return rc;
   } else if (mfma && gemm_tiles_pay<2>(p, a)) {

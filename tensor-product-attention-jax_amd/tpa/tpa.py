@@ -229,10 +229,8 @@ def tpa_cache_append(
     x[b, n, d_model]; w[rq*(h+d) + 2*rk*(h+d), d_model] (rows in the order qa, qb, ka, kb, va, vb,
     as torch.nn.Linear keeps its weight); rope_cos, rope_sin[rope_len, d/2] fp32; the cache arrays
     [b, cache_len, rk, h|d], or page pools [pages, page_size, rk, h|d] with `page_table`
-    [b, pages_per_seq]; `positions` [b, n] defaults to kv_lengths[b] + i.  A decode step (at most 64 new
-    tokens in all) is faster with scratch memory for partial sums: `workspace` (uint8, at least
-    `cache_append_workspace_bytes(...)`; a serving loop passes the same one every step) or, with
-    `use_workspace` (default: the module's `USE_WORKSPACE`), one allocated here.
+    [b, pages_per_seq]; `positions` [b, n] defaults to kv_lengths[b] + i.  `workspace` (uint8) and
+    `use_workspace` are accepted and change nothing: no kernel of this call takes scratch memory.
     Returns (qa[b, n, rq, h], qb[b, n, rq, d], new_kv_lengths[b])."""
     if use_workspace is None:
         use_workspace = USE_WORKSPACE

@@ -50,8 +50,7 @@ def make_layer(seed, b, n, dm, h, d, rq, rk, dtype, gpu):
 )
 @pytest.mark.parametrize("use_workspace", [False, True])
 def test_append_matches_the_oracle(gpu, dtype, kernel, b, n, dm, h, d, rq, rk, use_workspace):
-    """With `use_workspace` a decode step whose d_model is a multiple of 512 runs as two kernels (partial sums of
-    2, 4 or 8 slabs of k in the workspace, then a finishing kernel); every other case ignores it."""
+    """`use_workspace` is accepted and changes nothing; the size that a workspace may have stays what it was."""
     x, w = make_layer(1, b, n, dm, h, d, rq, rk, dtype, gpu)
     if use_workspace and kernel == 2 and b * n <= 64 and dm % 512 == 0:
         slabs = next(sl for sl in (8, 4, 2) if dm % (256 * sl) == 0)

@@ -1,0 +1,26 @@
+"""The append kernel for few tokens (16 columns and up to 64 tokens per workgroup, the contraction dealt to eight waves in
+chunks of 64): numbers of tokens around its blocks of 16, 32 and 64, contractions of fewer chunks than waves and of odd
+numbers of chunks, ragged column blocks, and calls on either side of the line to the 64 x 64 tiles, against the CPU oracle."""
+
+import pytest
+import torch
+
+from test_gpu_append import test_append_matches_the_oracle as check_append
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+    "b,n,dm,h,d,rq,rk",
+    [
+        (1, 1, 4096, 32, 128, 6, 2),   # blocks of 16 tokens, 15 of them past the end
+        (17, 1, 192, 8, 64, 2, 1),     # three chunks of k: five waves have none; a second block of one token
+        (11, 3, 1088, 32, 128, 6, 2),  # 17 chunks; 33 tokens x 100 column blocks: blocks of 32
+        (13, 5, 64, 32, 128, 6, 2),    # one chunk; 65 tokens: blocks of 64, the last of one token
+        (3, 30, 2112, 8, 64, 1, 1),    # 33 chunks; 216 columns: the last block owns 8 of its 16
+        (2, 83, 512, 64, 64, 16, 8),   # 166 tokens x 256 column blocks: 768 workgroups, the most it serves
+        (3, 71, 512, 64, 64, 16, 8),   # 213 tokens, 1024: tiles
+    ],
+)
+def test_append_few_tokens(gpu, b, n, dm, h, d, rq, rk):
+    check_append(gpu, torch.bfloat16, 2, b, n, dm, h, d, rq, rk, False)
