@@ -173,7 +173,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   }
 
   const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  const int w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = qblk * kBQ;
   // row block r of this wave within the workgroup's eight
   int rblk[RB], wrow0[RB], qrow[RB], qrow_ld[RB];
@@ -361,11 +361,13 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     if (hi >= 0) {
       kpos0 = lo / kTK * kTK;
       kend = hi + 1;
-      seg_pure = qmin == qmax && cnt == hi - lo + 1;
+      seg_pure = scalar(qmin == qmax && cnt == hi - lo + 1);
     } else {
       kend = min(kend, kTK);  // nothing visible: one (fully masked) tile, the rows end as NaN / -inf
     }
   }
+  kpos0 = scalar(kpos0);
+  kend = scalar(kend);
   const int lk_r = kend - kpos0;          // keys counted from kpos0
   const int ntiles = (lk_r + kTK - 1) / kTK;
   const int last = ntiles - 1;
@@ -425,7 +427,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // values to the same addresses), so that the eight waves run one instruction stream.
   uint32_t a_pending = 0;
   const int a_idx = tid & (4 * kTK - 1);
-  const int a_mat = a_idx / (2 * kTK), a_tok = (a_idx >> 1) % kTK, a_rank = a_idx & 1;
+  const int a_mat = scalar(a_idx / (2 * kTK)), a_tok = (a_idx >> 1) % kTK, a_rank = a_idx & 1;
   const int ka_bytes = ((lk_r - 1) * p.ka.stride_l + p.ka.stride_r + 1) * 2, va_bytes = ((lk_r - 1) * p.va.stride_l + p.va.stride_r + 1) * 2;
   const __amdgpu_buffer_rsrc_t ka_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ka_b), 0, ka_bytes, kRsrcFlags);
   const __amdgpu_buffer_rsrc_t va_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(va_b), 0, va_bytes, kRsrcFlags);
