@@ -583,11 +583,14 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
 // kernels wait for LDS more than for memory: with fewer pairs side by side they lose 1 % at B = 4, T = 4096, H = 16),
 // but not all pairs of the XCD where they are many (the workgroups resident together would all belong to different
 // pairs and share nothing: B = 16, T = 1024, H = 16 takes 0.574 ms with 16 of its 32 pairs side by side, 0.620 with all;
-// B = 8, T = 2048, H = 64, D = 64 not causal 2.25 against 2.44 ms)
+// B = 8, T = 2048, H = 64, D = 64 not causal 2.25 against 2.44 ms).  Groups of one size, as in the forward: a short last
+// one leaves compute units idle (72 pairs, whole backward, us, short last group / equal groups: T = 2040, D = 64 causal
+// 292 / 249, D = 128 513 / 450, T = 4000 827 / 688 and 1478 / 1260; 192 pairs, T = 1500 368 / 350)
 inline int pair_group_of(int per_xcd, int nblk) {
   int g = (64 + nblk - 1) / nblk;
   if (g < 8) g = 8;
-  return g < per_xcd ? g : per_xcd;
+  const int n = per_xcd / g;
+  return n < 1 ? per_xcd : (per_xcd + n - 1) / n;
 }
 
 // Both in one launch: the dK/dV workgroups first (four products per tile against three), then the dQ ones, so that the

@@ -1129,9 +1129,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* part_o,
 // attention: B = 8, T = 2048, H = 64, D = 64 (64 pairs per XCD, 8 blocks each) 0.654 ms with all pairs side by
 // side, 0.601 - 0.603 with 1 to 8; B = 4, T = 4096, H = 16 (8 pairs, 16 blocks) 0.250 with 4 or 8, 0.256 with 2,
 // 0.291 with 1 (the last group's heavy blocks start late); T = 32768, H = 32 (4 pairs, 128 blocks) 7.04 with 1, 7.21 with 4.
+// The groups are of one size, give or take a pair: a short last one would start its heavy blocks late and leave compute
+// units idle (with the reconstruction, us, short last group / equal groups, causal, 72 pairs: T = 2040, D = 64 89 / 70, D =
+// 128 136 / 109, T = 4000 238 / 200 and 377 / 322; 48 pairs, T = 4000, not causal 268 / 222; 192 pairs, T = 1500 118 / 104).
 inline int dense_pair_group(int per_xcd, int nqb) {
   const int g = (64 + nqb - 1) / nqb;
-  return g < 1 ? 1 : g < per_xcd ? g : per_xcd;
+  const int n = per_xcd / (g < 1 ? 1 : g);
+  return n < 1 ? per_xcd : (per_xcd + n - 1) / n;
 }
 
 template <int D, int LOADER, bool SEG = false, bool SPLIT = false>
