@@ -1227,7 +1227,7 @@ size_t tpa_prefill_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int
 }
 
 // Whether reconstructing dense Q, K and V once (one HBM-bound launch) and running the plain tile
-// loader beats rebuilding every tile in the flash loop.  The loop over dense tiles overlaps the
+// loader beats rebuilding every tile in the flash loop, by the lengths and the rank alone.  The loop over dense tiles overlaps the
 // logits of one tile with the softmax of the one before and has no rebuild in it; the
 // reconstruction grows with the length only.  Rank 2 has a tuned rebuild in the fused kernel:
 // measured at B * H = 64, D = 128 the two routes meet at 1024 rows (51 against 52 us) and the dense
@@ -1243,8 +1243,27 @@ int tpa_prefill_wants_dense(int64_t lq, int64_t lk, int64_t rk) {
   return lq > tpa::kBQ || (rk > 2 && lq > 16 && lk >= 1024);
 }
 
+namespace tpa {
+namespace {
+// The same for one call, of which the number of workgroups is known.  Rank 2 below 2048 rows, dense over fused time, no mask /
+// causal / packed documents, 8 to 400 (batch, head) pairs of 257 to 2040 rows each, one to five times as many keys:
+//   at most 64 workgroups: the prologue with its loads and Q is most of the time, and shorter without the factors.  D = 128
+//     0.76 - 1.01 (8 pairs of 512 rows 27 / 23 us); D = 64 0.89 - 1.16, not taken
+//   65 to 256: every compute unit rebuilds for itself and the reconstruction is a launch more.  0.84 - 1.40, from 0.97 on for
+//     most; 128 pairs of 512 rows 22 / 29 us, but 24 pairs of 2040 rows, D = 128 75 / 66
+//   more, from 1000 rows on: 0.77 - 1.07 (48 pairs of 1777, D = 64, documents of 421 tokens 46 / 41 us)
+//   more, of fewer rows: 0.83 - 1.04, with more keys than rows up to 1.32
+bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
+  if (tpa_prefill_wants_dense(lq, lk, rk)) return true;
+  if (rk != 2 || lq <= kBQ || lk > 5 * lq) return false;
+  const int64_t wgs = B * H * ((lq + kBQ - 1) / kBQ);
+  return wgs <= 64 ? D == 128 : wgs > 256 && lq >= 1000;
+}
+}  // namespace
+}  // namespace tpa
+
 size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
-  const size_t dense = tpa_prefill_wants_dense(lq, lk, rk) ? tpa_prefill_dense_bytes(B, lq, lk, H, D) : 0;
+  const size_t dense = tpa::dense_pays(B, lq, lk, H, D, rk) ? tpa_prefill_dense_bytes(B, lq, lk, H, D) : 0;
   const int s0 = tpa::choose_splits(B, lq, lk, H, D, false), s1 = tpa::choose_splits(B, lq, lk, H, D, true);
   return dense + tpa::split_bytes(B, lq, H, D, s0 > s1 ? s0 : s1);
 }
@@ -1260,7 +1279,7 @@ struct PrefillRoute {
 };
 PrefillRoute route_of(const TpaFwdArgs* a) {
   const int tiles = (int)(((int64_t)a->lk + kTK - 1) / kTK);  // a caller's count beyond that only adds empty ranges
-  return {tpa_prefill_wants_dense(a->lq, a->lk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
+  return {dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
           a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0)};
 }
 
