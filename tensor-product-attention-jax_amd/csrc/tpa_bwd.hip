@@ -560,14 +560,9 @@ __device__ __forceinline__ float dpp_add(float v) {
 struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R, D; };
 struct ProjectJobs { ProjectJob job[3]; };
 template <typename T>
-__device__ __forceinline__ f32x4 four_as_f32(const T* p) {
-  if constexpr (sizeof(T) == 2) {
-    const u32x2 x = *reinterpret_cast<const u32x2*>(p);
-    return f32x4{bf16lo_to_f32(x[0]), bf16hi_to_f32(x[0]), bf16lo_to_f32(x[1]), bf16hi_to_f32(x[1])};
-  } else {
-    return *reinterpret_cast<const f32x4*>(p);
-  }
-}
+using Four = std::conditional_t<sizeof(T) == 2, u32x2, f32x4>;  // four values as they lie in memory
+__device__ __forceinline__ f32x4 as_f32(const u32x2& x) { return f32x4{bf16lo_to_f32(x[0]), bf16hi_to_f32(x[0]), bf16lo_to_f32(x[1]), bf16hi_to_f32(x[1])}; }
+__device__ __forceinline__ f32x4 as_f32(const f32x4& x) { return x; }
 template <typename TO>
 __device__ __forceinline__ void store_four(TO* p, f32x4 x) {
   if constexpr (sizeof(TO) == 2) *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])};
@@ -602,9 +597,20 @@ __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H
   const float inv = 1.f / (float)R;
   TO* oa = reinterpret_cast<TO*>(ga.ptr) + b * ga.stride_b + t * ga.stride_l + 8 * hg;
   TO* ob = reinterpret_cast<TO*>(gb.ptr) + b * gb.stride_b + t * gb.stride_l + 4 * cc;
+  // a rank's factors are requested while the one before is worked on
+  Four<T> next[4];
+  auto request = [&](int r) __attribute__((always_inline)) {
+    const T* const a = ap + (int64_t)r * fa.stride_r;
+    const T* const b = bp + (int64_t)r * fb.stride_r;
+    next[0] = *reinterpret_cast<const Four<T>*>(a);
+    next[1] = *reinterpret_cast<const Four<T>*>(a + 4);
+    next[2] = *reinterpret_cast<const Four<T>*>(b);
+    next[3] = *reinterpret_cast<const Four<T>*>(b + dh);
+  };
+  request(0);
   for (int r = 0; r < R; ++r) {
-    const f32x4 al = four_as_f32(ap + (int64_t)r * fa.stride_r), ah = four_as_f32(ap + (int64_t)r * fa.stride_r + 4);
-    const f32x4 bl = four_as_f32(bp + (int64_t)r * fb.stride_r), bh = four_as_f32(bp + (int64_t)r * fb.stride_r + dh);
+    const f32x4 al = as_f32(next[0]), ah = as_f32(next[1]), bl = as_f32(next[2]), bh = as_f32(next[3]);
+    if (r + 1 < R) request(r + 1);
     float af[8], bf[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) { af[j] = al[j]; af[4 + j] = ah[j]; bf[j] = bl[j]; bf[4 + j] = bh[j]; }

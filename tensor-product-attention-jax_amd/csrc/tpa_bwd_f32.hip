@@ -616,12 +616,12 @@ __device__ __forceinline__ void add_waves(const float* at, float* dst, int row0,
 }
 
 template <int D, bool SEG>
-__global__ __launch_bounds__(SplitLds<D>::NW * 64, 1) void bwd_f32_dq_split_kernel(BwdF32Params p) {
+__device__ __forceinline__ void dq_split(const BwdF32Params& p, int id) {
   typedef SplitLds<D> L;
   constexpr int NDB = D / 32, NKS = D / 16, NW = L::NW;
   extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
   int pair, h;
-  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
+  if (!pair_of_workgroup(id, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int blk = p.nblk - 1 - pair / p.B, b = pair % p.B;  // heaviest causal blocks first
   const int tid = threadIdx.x, w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = blk * 32, qrow = q0 + i, qrow_ld = min(qrow, p.lq - 1);
@@ -721,12 +721,12 @@ __global__ __launch_bounds__(SplitLds<D>::NW * 64, 1) void bwd_f32_dq_split_kern
 }
 
 template <int D, bool SEG>
-__global__ __launch_bounds__(SplitLds<D>::NW * 64, 1) void bwd_f32_dkv_split_kernel(BwdF32Params p) {
+__device__ __forceinline__ void dkv_split(const BwdF32Params& p, int id) {
   typedef SplitLds<D> L;
   constexpr int NDB = D / 32, NKS = D / 16, NW = L::NW;
   extern __shared__ __attribute__((aligned(16))) float smem_bwd_f32[];
   int pair, h;
-  if (!pair_of_workgroup(blockIdx.x, p.npairs, p.H, p.B, p.groups, pair, h)) return;
+  if (!pair_of_workgroup(id, p.npairs, p.H, p.B, p.groups, pair, h)) return;
   const int blk = pair / p.B, b = pair % p.B;  // under the causal mask the first key blocks see the most rows: heaviest first
   const int tid = threadIdx.x, w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int k0 = blk * 32, key = k0 + i, key_ld = min(key, p.lk - 1);
@@ -839,6 +839,16 @@ __global__ __launch_bounds__(SplitLds<D>::NW * 64, 1) void bwd_f32_dkv_split_ker
   add_waves<D>(smem_bwd_f32 + SplitLds<D>::kMat, p.dv + (int64_t)b * p.lk * hd + (int64_t)h * D, k0, p.lk, hd, tid);
 }
 
+// Both in one launch: the dK/dV workgroups first (four products per tile against three), then the dQ ones, which fill the
+// compute units that the tail of the first leaves idle: a launch and its gap less (2 x 1000 tokens, 8 heads of 64, whole
+// training step 133.3 -> 131.3 us with the factors of the projections requested a rank ahead).
+struct BwdF32Pair { BwdF32Params kv, q; int n_kv; };
+template <int D, bool SEG>
+__global__ __launch_bounds__(SplitLds<D>::NW * 64, 1) void bwd_f32_split_kernel(BwdF32Pair p) {
+  if ((int)blockIdx.x < p.n_kv) dkv_split<D, SEG>(p.kv, blockIdx.x);
+  else dq_split<D, SEG>(p.q, blockIdx.x - p.n_kv);
+}
+
 // Whether 32-row workgroups pay: the launch of 128-row ones leaves half of the 256 compute units idle, or fills them once
 // with causal blocks of long sequences, of which the heaviest is twice the average.  Backward, us, 32 / 128 rows: 8 heads of
 // 64, 2 x 1000 tokens causal 98 / 201, 4 x 1000 177 / 207, 8 x 1000 343 / 261, not causal 2 x 1000 143 / 205, 4 x 1000
@@ -854,37 +864,50 @@ bool few_blocks(const BwdF32Params& p, int rows, int D) {
 // 569 / 427, 8 x 1000 not causal 359 / 411, 4 x 1000 308 / 217.  At head size 128 their registers do not hold the operands.
 bool many_blocks(const BwdF32Params& p, int rows) { return (int64_t)((rows + 255) / 256) * p.B * p.H >= (p.causal ? 512 : 256); }
 
-template <typename K>
-int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int block, int threads, size_t lds, BwdF32Params p, hipStream_t stream) {
+// fills in the decomposition of `rows` rows (or keys) in blocks of `block`; the number of workgroups
+int64_t decompose(BwdF32Params& p, int rows, int block) {
   p.nblk = (rows + block - 1) / block;
   p.npairs = p.nblk * p.B;
   p.groups = head_groups(p.npairs, p.H);
+  return workgroups_of(p.npairs, p.H, p.groups);
+}
+
+template <typename K>
+int launch_kernel(K kern, bool (&configured)[kMaxDevices], int rows, int waves, size_t lds, BwdF32Params p, hipStream_t stream) {
+  const int64_t n = decompose(p, rows, 32 * waves);
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)workgroups_of(p.npairs, p.H, p.groups)), dim3(threads), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * waves), lds, stream, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
 template <int D, bool SEG>
-int launch_dq(const BwdF32Params& p, hipStream_t stream) {
-  static bool configured[3][kMaxDevices] = {};
-  if (few_blocks(p, p.lq, D)) return launch_kernel(bwd_f32_dq_split_kernel<D, SEG>, configured[0], p.lq, 32, SplitLds<D>::NW * 64, SplitLds<D>::kBytes, p, stream);
-  if constexpr (D == 64)
-    if (many_blocks(p, p.lq)) return launch_kernel(bwd_f32_dq_kernel<D, 8, SEG>, configured[1], p.lq, 256, 512, BwdLds<D>::kBytes, p, stream);
-  return launch_kernel(bwd_f32_dq_kernel<D, 4, SEG>, configured[2], p.lq, 128, 256, BwdLds<D>::kBytes, p, stream);
-}
-template <int D, bool SEG>
-int launch_dkv(const BwdF32Params& p, hipStream_t stream) {
-  static bool configured[3][kMaxDevices] = {};
-  if (few_blocks(p, p.lk, D)) return launch_kernel(bwd_f32_dkv_split_kernel<D, SEG>, configured[0], p.lk, 32, SplitLds<D>::NW * 64, SplitLds<D>::kBytes, p, stream);
-  if constexpr (D == 64)
-    if (many_blocks(p, p.lk)) return launch_kernel(bwd_f32_dkv_kernel<D, 8, SEG>, configured[1], p.lk, 256, 512, BwdLds<D>::kBytes, p, stream);
-  return launch_kernel(bwd_f32_dkv_kernel<D, 4, SEG>, configured[2], p.lk, 128, 256, BwdLds<D>::kBytes, p, stream);
+int launch_split(const BwdF32Params& p, bool dq, bool dkv, hipStream_t stream) {
+  static bool configured[kMaxDevices] = {};
+  auto kern = bwd_f32_split_kernel<D, SEG>;
+  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), SplitLds<D>::kBytes); rc != TPA_OK) return rc;
+  BwdF32Pair pair{p, p, 0};
+  const int64_t nk = decompose(pair.kv, p.lk, 32), nq = decompose(pair.q, p.lq, 32);
+  pair.n_kv = dkv ? (int)nk : 0;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(pair.n_kv + (dq ? nq : 0))), dim3(SplitLds<D>::NW * 64), SplitLds<D>::kBytes, stream, pair);
+  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
 template <int D, bool SEG>
 int launch_pair(const BwdF32Params& p, hipStream_t stream) {
-  if (int rc = launch_dq<D, SEG>(p, stream); rc != TPA_OK) return rc;
-  return launch_dkv<D, SEG>(p, stream);
+  static bool configured[4][kMaxDevices] = {};
+  const bool split_dq = few_blocks(p, p.lq, D), split_dkv = few_blocks(p, p.lk, D);
+  if (split_dq || split_dkv)
+    if (int rc = launch_split<D, SEG>(p, split_dq, split_dkv, stream); rc != TPA_OK) return rc;
+  int rc = TPA_OK;
+  if (!split_dq) {
+    if constexpr (D == 64) rc = many_blocks(p, p.lq) ? launch_kernel(bwd_f32_dq_kernel<D, 8, SEG>, configured[0], p.lq, 8, BwdLds<D>::kBytes, p, stream)
+                                                     : launch_kernel(bwd_f32_dq_kernel<D, 4, SEG>, configured[1], p.lq, 4, BwdLds<D>::kBytes, p, stream);
+    else rc = launch_kernel(bwd_f32_dq_kernel<D, 4, SEG>, configured[1], p.lq, 4, BwdLds<D>::kBytes, p, stream);
+  }
+  if (rc != TPA_OK || split_dkv) return rc;
+  if constexpr (D == 64)
+    if (many_blocks(p, p.lk)) return launch_kernel(bwd_f32_dkv_kernel<D, 8, SEG>, configured[2], p.lk, 8, BwdLds<D>::kBytes, p, stream);
+  return launch_kernel(bwd_f32_dkv_kernel<D, 4, SEG>, configured[3], p.lk, 4, BwdLds<D>::kBytes, p, stream);
 }
 
 }  // namespace
