@@ -61,23 +61,37 @@ struct DecodeParams {
 // and sums are not contracted but where `fmaf` says so, and conversions, quotients and `ceilf` are exact or round once.
 // 48 paged sequences of 2047 .. 4096 tokens (32 heads of 128, rank 2): 67.7 us with equal counts (288 workgroups), 43.4 so.
 constexpr int kMaxPlanEntries = 64;
+// What costs time in it is latency, twice per call (here and in the merge): sums over the lanes go through DPP adds (through
+// the LDS permute they were 1 400 cycles), and the search takes four instructions per entry.  With both, append, decode and
+// merge of the step above 57.1 -> 54.1 us, of 6 sequences of 1022 .. 2048 tokens with four query tokens each 26.1 -> 24.8.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int add_from(int x) { return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false); }
+__device__ __forceinline__ int wave_prefix_sum(int x) {  // lane i: sum of lanes 0 .. i
+  x = add_from<0x111, 0xf>(x);  // row_shr 1, 2, 4, 8: inside rows of 16 lanes
+  x = add_from<0x112, 0xf>(x);
+  x = add_from<0x114, 0xf>(x);
+  x = add_from<0x118, 0xf>(x);
+  x = add_from<0x142, 0xa>(x);  // row_bcast 15: the last lane of rows 0 and 2 to rows 1 and 3
+  return add_from<0x143, 0xc>(x);  // row_bcast 31: lane 31 to rows 2 and 3
+}
 struct RangePlan { int S, first; };  // of batch entry `lane`: its number of ranges and the first one's index
 __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, int min_keys) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
-  int total = len;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
+  const int total = __builtin_amdgcn_readlane(wave_prefix_sum(len), 63);
   const float shortest = fmaxf((float)total / (float)slots, (float)min_keys);
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
   const float inv = 1.f / fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
-  // eight entries at a time, their chains side by side (lanes past the last entry hold length 0 and count 1)
-  int count[8] = {}, j0 = 0;
+  // eight entries at a time, their chains side by side; an entry without keys counts as one of one key (one range), and so do
+  // the lanes past the last entry, which are taken off again
+  const uint32_t keys = __float_as_uint((float)max(len, 1));
+  float count[8] = {};
+  int j0 = 0;
   for (; j0 < B; j0 += 8)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) count[j] += max(1, (int)ceilf((float)__builtin_amdgcn_readlane(len, j0 + j) * inv));
-  const int total_count = ((count[0] + count[1]) + (count[2] + count[3])) + ((count[4] + count[5]) + (count[6] + count[7])) - (j0 - B);
+    for (int j = 0; j < 8; ++j) count[j] += ceilf(__uint_as_float(__builtin_amdgcn_readlane(keys, j0 + j)) * inv);
+  const int total_count = (int)(((count[0] + count[1]) + (count[2] + count[3])) + ((count[4] + count[5]) + (count[6] + count[7]))) - (j0 - B);
   const uint64_t fits = __ballot(total_count <= slots);
   RangePlan r;
   r.S = lane < B ? 1 : 0;
@@ -85,13 +99,7 @@ __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, in
     const float pick = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), __builtin_ctzll(fits)));
     if (lane < B) r.S = max(1, (int)ceilf((float)len * pick));
   }
-  r.first = r.S;
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) {
-    const int below = __shfl_up(r.first, m, 64);
-    if (lane >= m) r.first += below;
-  }
-  r.first -= r.S;
+  r.first = wave_prefix_sum(r.S) - r.S;
   return r;
 }
 
