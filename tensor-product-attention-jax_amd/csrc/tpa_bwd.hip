@@ -88,6 +88,10 @@ __global__ __launch_bounds__(256) void recon_bf16_kernel(TpaFactor fa, TpaFactor
   }
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
 // The same for head counts that are multiples of 8 with 16-byte aligned a rows: a thread owns one
 // (token, 16-byte piece of D, group of 8 heads) and reads, per rank, one 16-byte piece of b and
 // the 8 head factors as one 16-byte piece of a - 64 multiply-adds per two loads.  Pieces are the
@@ -122,18 +126,39 @@ __device__ __forceinline__ void delta_h8(const DeltaJob& j, int64_t t, int g, in
         add(__uint_as_float(ov[i][e]) * __uint_as_float(gv[i][e]));
       }
     }
-    for (int m = 1; m < cpr; m <<= 1) acc += __shfl_xor(acc, m, 64);
+    acc = dpp_add<0xB1>(acc);
+    acc = dpp_add<0x4E>(acc);
+    acc = dpp_add<0x141>(acc);
+    if (cpr >= 16) acc = dpp_add<0x140>(acc);
+    if (cpr == 32) acc += __shfl_xor(acc, 16, 64);
     if (cc == i) mine = acc;
   }
   if (live && cc < 8) j.delta[((int64_t)b * H + 8 * g + cc) * j.lq + t] = mine;
 }
 
+// This thread's token t, group g of 8 heads and piece cc of D: shifts where the counts are powers of two (three divisions of 64 bits
+// are a microsecond before the first load: 1340 tokens x 16 heads x 128 with the delta 10.6 us, with shifts and its sums by DPP 7.8)
+__device__ __forceinline__ void piece_of(int cpr, int hg, int64_t& t, int& g, int& cc) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (((cpr & (cpr - 1)) | (hg & (hg - 1))) == 0) {
+    const int s = __builtin_ctz(cpr);
+    cc = (int)idx & (cpr - 1);
+    g = (int)(idx >> s) & (hg - 1);
+    t = idx >> (s + __builtin_ctz(hg));
+  } else {
+    cc = (int)(idx % cpr);
+    g = (int)(idx / cpr % hg);
+    t = idx / ((int64_t)cpr * hg);
+  }
+}
+
 // fp32 factors -> dense fp32, in the same way: a thread owns 4 elements of D for 8 heads of a token
 __global__ __launch_bounds__(256) void recon_f32_h8_kernel(ReconJobs jobs, int H, int D) {
   const int cpr = D / 4, hg = H / 8;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int cc = (int)(idx % cpr), g = (int)(idx / cpr % hg), b = blockIdx.y;
-  const int64_t t = idx / ((int64_t)cpr * hg);
+  int cc, g;
+  int64_t t;
+  piece_of(cpr, hg, t, g, cc);
+  const int b = blockIdx.y;
   if (blockIdx.z == 3) return delta_h8<float>(jobs.delta, t, g, cc, cpr, b, H, D);
   const ReconJob job = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
   if (t >= job.L) return;
@@ -172,10 +197,9 @@ __global__ __launch_bounds__(256) void recon_bf16_h8_kernel(ReconJobs jobs, int 
   const int R = blockIdx.z == 0 ? jobs.job[0].R : blockIdx.z == 1 ? jobs.job[1].R : jobs.job[2].R;
   const float scale = blockIdx.z == 0 ? jobs.job[0].scale : blockIdx.z == 1 ? jobs.job[1].scale : jobs.job[2].scale;
   const int cpr = D / 8, hg = H / 8;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int cc = (int)(idx % cpr);
-  const int g = (int)(idx / cpr % hg);
-  const int64_t t = idx / ((int64_t)cpr * hg);
+  int cc, g;
+  int64_t t;
+  piece_of(cpr, hg, t, g, cc);
   const int b = blockIdx.y;
   if (blockIdx.z == 3) return delta_h8<uint16_t>(jobs.delta, t, g, cc, cpr, b, H, D);
   if (t >= L) return;
@@ -550,11 +574,10 @@ __global__ __launch_bounds__(256) void project_kernel(const float* dx, TpaFactor
 // where one load instruction touched every other 16 bytes), multiplies it
 // with its 8 values of b (for da) and of a (for db) rank by rank, and the sums over d and over h are
 // reductions across the lanes that share a token: over the D / 8 neighbouring lanes with DPP adds,
-// over the H / 8 groups above them with lane exchanges.  Several tokens share a wave.
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
+// over the H / 8 groups above them with DPP adds and exchanges of rows of lanes, in registers throughout: through the LDS
+// (ds_bpermute, eight or more per rank) the kernel waited for them, 1340 tokens x 16 heads x 128 with ranks 6, 2, 2 took 14.7 us
+// instead of 11.1 us, 16 384 x 32 x 64 93 instead of 79 (403 MB read, 5 TB/s: at that size the memory is what bounds it).
+// Several tokens share a wave.
 // All arrays that this kernel takes in one launch (blockIdx.z): at short lengths a launch of its own leaves each of them
 // waiting for the one before.  The gradients are written in the type the caller wants them in (rounded once, from the fp32 sums).
 struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R, D; };
@@ -568,6 +591,27 @@ __device__ __forceinline__ void store_four(TO* p, f32x4 x) {
   if constexpr (sizeof(TO) == 2) *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])};
   else *reinterpret_cast<f32x4*>(p) = x;
 }
+template <typename TO>
+__device__ __forceinline__ void store_two(TO* p, float x, float y) {
+  if constexpr (sizeof(TO) == 2) *reinterpret_cast<uint32_t*>(p) = pack_bf16(x, y);
+  else p[0] = x, p[1] = y;
+}
+template <typename TO>
+__device__ __forceinline__ void store_eight(TO* p, const float* x) {
+  if constexpr (sizeof(TO) == 2) {
+    *reinterpret_cast<u32x4*>(p) = u32x4{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]), pack_bf16(x[6], x[7])};
+  } else {
+    *reinterpret_cast<f32x4*>(p) = f32x4{x[0], x[1], x[2], x[3]};
+    *reinterpret_cast<f32x4*>(p + 4) = f32x4{x[4], x[5], x[6], x[7]};
+  }
+}
+// x and y of the lanes N apart: the lanes of the lower side get the sum of the two x, those of the upper side that of the two y
+template <int N>
+__device__ __forceinline__ float swap_add(float x, float y) {
+  const unsigned a = __float_as_uint(x), b = __float_as_uint(y);
+  auto s = N == 16 ? __builtin_amdgcn_permlane16_swap(a, b, false, false) : __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
 template <typename T, typename TO>
 __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H) {
   const ProjectJob j = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
@@ -575,11 +619,11 @@ __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H
   const TpaGrad &ga = j.ga, &gb = j.gb;
   const int L = j.L, R = j.R, D = j.D;
   const int cpr = D / 8, hgs = H / 8, tt = cpr * hgs;  // threads per token
-  const int64_t gtid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int cc = (int)(gtid % cpr), hg = (int)(gtid / cpr % hgs);
-  const int64_t tok = gtid / tt;
+  int cc, hg;
+  int64_t tok;
+  piece_of(cpr, hgs, tok, hg, cc);
   const bool live = tok < L;
-  if ((int64_t)blockIdx.x * 256 / tt >= L) return;  // a whole workgroup past the end of a shorter array
+  if ((int64_t)blockIdx.x * (256 >> __builtin_ctz(tt)) >= L) return;  // a whole workgroup past the end of a shorter array
   const int64_t t = live ? tok : L - 1;  // lanes past the end idle along: the reductions need whole waves
   const int b = blockIdx.y;
   const int dh = D / 2;  // a thread's eight columns: 4 cc .. 4 cc + 3 and the same in the upper half of the row
@@ -595,9 +639,14 @@ __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H
     for (int j = 0; j < 4; ++j) { x[i][j] = lo[j]; x[i][4 + j] = hi[j]; }
   }
   const float inv = 1.f / (float)R;
+  // which of the lanes that share a (token, piece of D) write which of its columns, see db below
+  const int swaps = (tt > 16) + (tt > 32), lane = threadIdx.x & 63;
+  const bool writes = live && (cpr == 16 || (lane & 8) == 0);
+  const int column = (lane & 16 ? dh : 0) + (swaps == 2 && (lane & 32) ? 2 : 0);
   TO* oa = reinterpret_cast<TO*>(ga.ptr) + b * ga.stride_b + t * ga.stride_l + 8 * hg;
   TO* ob = reinterpret_cast<TO*>(gb.ptr) + b * gb.stride_b + t * gb.stride_l + 4 * cc;
-  // a rank's factors are requested while the one before is worked on
+  // a rank's factors are requested while the one before is worked on (two ranks ahead: the small sizes gain 0.3 us, but the
+  // registers cost a wave per SIMD and 16 384 tokens x 32 heads x 64 go from 81 to 84 us)
   Four<T> next[4];
   auto request = [&](int r) __attribute__((always_inline)) {
     const T* const a = ap + (int64_t)r * fa.stride_r;
@@ -637,23 +686,32 @@ __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H
       v = dpp_add<0x4E>(v);   // quad_perm [2, 3, 0, 1]
       v = dpp_add<0x141>(v);  // row_half_mirror: the other quad of the same eight lanes
       if (cpr == 16) v = dpp_add<0x140>(v);  // row_mirror: the other eight lanes of the row
-      da[i] = v;
+      da[i] = v * inv;
     }
-    // db: sum over the head groups, which lie cpr lanes apart
+    if (live && cc == 0) store_eight(oa + (int64_t)r * ga.stride_r, da);
+    // db: sum over the head groups, which lie cpr lanes apart.  The exchange of two rows of 16 lanes (or of the two halves of
+    // the wave) takes a pair of values and leaves each side the sum of one of them, so that the lanes share out the columns
+    if (cpr == 8 && hgs > 1) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = db[j];
-      for (int m = cpr; m < tt; m <<= 1) v += __shfl_xor(v, m, 64);
-      db[j] = v;
+      for (int j = 0; j < 8; ++j) db[j] = dpp_add<0x128>(db[j]);  // row_ror 8: the other eight lanes of the row
     }
-    if (live && cc == 0) {
-      store_four(oa + (int64_t)r * ga.stride_r, f32x4{da[0] * inv, da[1] * inv, da[2] * inv, da[3] * inv});
-      store_four(oa + (int64_t)r * ga.stride_r + 4, f32x4{da[4] * inv, da[5] * inv, da[6] * inv, da[7] * inv});
+    TO* const o = ob + (int64_t)r * gb.stride_r;
+    if (swaps == 0) {
+      if (live && hg == 0) {
+        store_four(o, f32x4{db[0] * inv, db[1] * inv, db[2] * inv, db[3] * inv});
+        store_four(o + dh, f32x4{db[4] * inv, db[5] * inv, db[6] * inv, db[7] * inv});
+      }
+      continue;
     }
-    if (live && hg == 0) {
-      store_four(ob + (int64_t)r * gb.stride_r, f32x4{db[0] * inv, db[1] * inv, db[2] * inv, db[3] * inv});
-      store_four(ob + (int64_t)r * gb.stride_r + dh, f32x4{db[4] * inv, db[5] * inv, db[6] * inv, db[7] * inv});
+    float h4[4];  // odd rows of the wave: columns of the upper half
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h4[j] = swap_add<16>(db[j], db[j + 4]);
+    if (swaps == 1) {
+      if (writes) store_four(o + column, f32x4{h4[0] * inv, h4[1] * inv, h4[2] * inv, h4[3] * inv});
+      continue;
     }
+    const float lo = swap_add<32>(h4[0], h4[2]), hi = swap_add<32>(h4[1], h4[3]);  // upper half of the wave: columns 2, 3 of the four
+    if (writes) store_two(o + column, lo * inv, hi * inv);
   }
 }
 

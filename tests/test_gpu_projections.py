@@ -57,3 +57,22 @@ def test_head_sizes_that_differ(gpu, dt, tol, dk, dv):
     want = orc.tpa_backward(as_f64(q), as_f64(k), as_f64(v), None, None, h, as_f64(do), sm_scale=dk**-0.5, causal=True)
     for name, g, w in zip("qkv", got, want):
         assert rel_err(as_f64(g), w) <= tol, name
+
+
+@pytest.mark.parametrize("dt,tol", [(torch.float32, 2e-4), (torch.bfloat16, 1.5e-2)])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("h", [8, 16, 24, 32, 64])
+def test_every_number_of_lanes_that_share_a_token(gpu, dt, tol, h, d):
+    """One to eight groups of heads: each number of exchanges between the lanes, 24 heads (no power of two: indices by division,
+    the staged projection) and 64 x 128 (more than a wave per token); token counts that end inside a wave.  Tolerances as above."""
+    from tpa import tpa
+
+    b, lq, lk = 2, 37, 91
+    q, k, v = (to_gpu(x, dt, gpu) for x in make_factors(105, b, lq, lk, h, d, d, 3, 2, scale_by_rank=True))
+    o, res = tpa._tpa_fwd(q, k, v, h, None, None, d**-0.5, True, None, False, False, False)
+    do = to_gpu(np.random.default_rng(10).standard_normal((b, lq, h, d)).astype(np.float32), dt, gpu)
+    got = tpa._tpa_bwd(h, d**-0.5, True, None, False, False, False, res, do)
+    want = orc.tpa_backward(as_f64(q), as_f64(k), as_f64(v), None, None, h, as_f64(do), sm_scale=d**-0.5, causal=True)
+    for name, g, w in zip("qkv", got, want):
+        assert rel_err(as_f64(g), w) <= tol, name
+        assert rel_err(as_f64(g)[..., :h], w[..., :h]) <= tol and rel_err(as_f64(g)[..., h:], w[..., h:]) <= tol, name
