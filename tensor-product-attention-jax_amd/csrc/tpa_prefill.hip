@@ -313,51 +313,9 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     // decrease along the sequence; any other id pattern just visits more tiles, the mask itself
     // is applied per key as before).  If the rows share one id and the keys with that id form one
     // contiguous run, the tiles inside the run need no segment mask at all.
-    int32_t* const red = reinterpret_cast<int32_t*>(smem);
-    if (tid == 0) { red[0] = INT32_MAX; red[1] = INT32_MIN; red[2] = INT32_MAX; red[3] = -1; red[4] = 0; }
-    __syncthreads();
-    {  // one atomic per wave: the lanes' values are reduced in registers first
-      const bool mine = tid < kBQ && q0 + tid < p.lq;
-      const int32_t sid = mine ? p.qseg[(int64_t)b * p.lq + q0 + tid] : 0;
-      const int32_t smin = wave_min(mine ? sid : INT32_MAX), smax = wave_max(mine ? sid : INT32_MIN);
-      if ((tid & 63) == 0 && smin <= smax) {
-        __hip_atomic_fetch_min(&red[0], smin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __hip_atomic_fetch_max(&red[1], smax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-    }
-    __syncthreads();
-    const int32_t qmin = red[0], qmax = red[1];
-    int lo = INT32_MAX, hi = -1, cnt = 0;
-    auto visit = [&](int t, int32_t sid) __attribute__((always_inline)) {
-      if (sid >= qmin && sid <= qmax) { lo = min(lo, t); hi = max(hi, t); ++cnt; }
-    };
-    const int32_t* const kid = p.kvseg + (int64_t)b * p.lk;
-    // four ids per load and four loads in flight per thread where the row of ids is 16-byte aligned
-    const int kv4 = (reinterpret_cast<uintptr_t>(kid) & 15) == 0 ? (kend & ~3) : 0;
-    constexpr int U = 4;
-    for (int base = 4 * tid; base < kv4; base += 4 * NT * U) {
-      int4 ids[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int t = base + 4 * NT * u;
-        ids[u] = *reinterpret_cast<const int4*>(kid + (t < kv4 ? t : 0));
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int t = base + 4 * NT * u;
-        if (t < kv4) { visit(t, ids[u].x); visit(t + 1, ids[u].y); visit(t + 2, ids[u].z); visit(t + 3, ids[u].w); }
-      }
-    }
-    for (int t = kv4 + tid; t < kend; t += NT) visit(t, kid[t]);
-    lo = wave_min(lo); hi = wave_max(hi); cnt = wave_sum(cnt);
-    if ((tid & 63) == 0 && cnt) {
-      __hip_atomic_fetch_min(&red[2], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_max(&red[3], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_add(&red[4], cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __syncthreads();
-    lo = red[2]; hi = red[3]; cnt = red[4];
-    __syncthreads();  // the staging below reuses this memory
+    int lo, hi, cnt;
+    int32_t qmin, qmax;
+    id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kBQ, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem), tid, lo, hi, cnt, qmin, qmax);
     if (hi >= 0) {
       kpos0 = lo / kTK * kTK;
       kend = hi + 1;
