@@ -4,8 +4,8 @@
 // prefill kernels read.  The reference has no such step (its tests draw the factors at random,
 // tpa/tpa_test.py:86-91); the arithmetic follows arXiv 2501.06425, section 3.
 //
-// bf16, three kernels by the number of new tokens: 256 x 256 or 128 x 128 tiles once they fill the chip (a prefill
-// chunk), 64 x 64 tiles below that, and for a decode step and other few tokens a kernel whose workgroups own 16 columns
+// bf16, three kernels by the number of new tokens: 256 x 256 or 128 x 128 tiles for a large prefill chunk, 64 x 64 tiles
+// below that, and for a decode step and other few tokens a kernel whose workgroups own 16 columns
 // and split the contraction over their waves.  All of them compute with v_mfma_f32_*_bf16, stage the
 // fp32 results in LDS, and finish whole 16-byte chunks of eight columns: a chunk lies inside one rank
 // row of one factor (H and D are multiples of 8), so the rotation partners (2j, 2j+1) are inside it.
@@ -115,71 +115,99 @@ __device__ __forceinline__ void write_new_lengths(const AppendParams& p) {
     }
 }
 
-// ---- bf16, 64 x 64 tiles: four waves, one 32 x 32 block each; x and W tiles of 64 x 64 double buffered in LDS,
-// the next tiles in registers while the current ones are multiplied
-__global__ __launch_bounds__(256) void append_mfma_kernel(AppendParams p) {
-  __shared__ __attribute__((aligned(16))) uint16_t xs[2][kBM * kXS];
-  __shared__ __attribute__((aligned(16))) uint16_t ws[2][kBN * kXS];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
-  const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
-  const int wm = w >> 1, wn = w & 1;       // this wave's 32 x 32 block of the tile
-  const uint16_t* x = static_cast<const uint16_t*>(p.x);
-  const uint16_t* wt = static_cast<const uint16_t*>(p.w);
+// Workgroup id -> tile of y.  Ids are dealt to the 8 XCDs round robin; each XCD takes an eighth of the tiles, walking along the
+// shorter side of the matrix of tiles, so that what its L2 has to fetch of x and W is least.  False: past its share.
+// (Whole rows of tiles per XCD left XCDs idle below eight rows and unequal above: 600 tokens x 5120 columns 71 -> 41 us,
+// 1200 x 5120 125 -> 73, 4352 x 1600 110 -> 75.)
+__device__ __forceinline__ bool tile_of_workgroup(int id, int ntm, int ntn, int& tm, int& tn) {
+  const int64_t tiles = (int64_t)ntm * ntn;
+  const int xcd = id & 7, t = (int)((tiles * xcd + 7) / 8) + (id >> 3);  // (workgroup 0 always has one)
+  if (ntn <= ntm) { tm = t / ntn; tn = t % ntn; }
+  else { tn = t / ntm; tm = t % ntm; }
+  return t < (int)((tiles * (xcd + 1) + 7) / 8);
+}
+inline unsigned tile_workgroups(int ntm, int ntn) { return (unsigned)(((int64_t)ntm * ntn + 7) / 8 * 8); }
 
-  // loader: a 64 x 64 tile is 512 chunks of 16 bytes, two per thread (rows past the end repeat the last)
+// ---- bf16, 64 x 64 tiles: four waves, one 32 x 32 block each; x and W tiles of 64 x 64 double buffered in LDS,
+// the next tiles in registers while the current ones are multiplied.  One tile on a compute unit waits for its loads (0.6 us a
+// step for 0.06 us of matrix work), so KS groups of four waves deal the steps among themselves, each with buffers of its own, and
+// their sums meet in LDS: d_model 4096, 600 tokens x 1600 columns 38 -> 20 us, 1000 x 1600 with two groups 39 -> 28.  With four
+// groups the LDS is what bounds a step (192 KB, 0.7 of 1 us); loads two steps ahead change nothing.
+constexpr int kTileStage = (kBM + kBN) * kXS;
+template <int KS>
+__global__ __launch_bounds__(256 * KS) void append_mfma_kernel(AppendParams p, int ntm, int ntn) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t tile_mem[];  // [KS][2][x | W][64][kXS]
+  const int grp = KS > 1 ? scalar(threadIdx.x >> 8) : 0;
+  uint16_t* const mem = tile_mem + grp * 2 * kTileStage;
+  const int tid = threadIdx.x & 255, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
+  int tm, tn;
+  if (!tile_of_workgroup(blockIdx.x, ntm, ntn, tm, tn)) return;
+  const int m0 = tm * kBM, n0 = tn * kBN;
+  const int wm = w >> 1, wn = w & 1;       // this wave's 32 x 32 block of the tile
+
+  // loader: a 64 x 64 tile is 512 chunks of 16 bytes, two per thread (rows past the end read as zero)
+  constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
+  const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.x) + (int64_t)m0 * p.K), 0, min(kBM, p.M - m0) * p.K * 2, kRsrcFlags);
+  const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.w) + (int64_t)n0 * p.K), 0, min(kBN, p.N - n0) * p.K * 2, kRsrcFlags);
+  const int lrow = tid >> 3, lc = tid & 7, voff = (lrow * p.K + 8 * lc) * 2;
+  const int nk = p.K / kBK, steps = (nk + KS - 1) / KS, mine = (nk - grp + KS - 1) / KS;  // this group takes steps grp, grp + KS, ..
   u32x4 xr[2], wr[2];
-  auto load = [&](int k0) {
+  auto load = [&](int kt) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      const int c = q * 256 + tid, row = c >> 3, cc = c & 7;
-      xr[q] = *reinterpret_cast<const u32x4*>(x + (int64_t)min(m0 + row, p.M - 1) * p.K + k0 + 8 * cc);
-      wr[q] = *reinterpret_cast<const u32x4*>(wt + (int64_t)min(n0 + row, p.N - 1) * p.K + k0 + 8 * cc);
+      const int at = (32 * q * p.K + (grp + KS * kt) * kBK) * 2;
+      xr[q] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, voff, at, 0);
+      wr[q] = __builtin_amdgcn_raw_buffer_load_b128(w_rs, voff, at, 0);
     }
   };
   auto stage = [&](int buf) {
+    uint16_t* const xs = mem + buf * kTileStage + lrow * kXS + 8 * lc;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      const int c = q * 256 + tid, row = c >> 3, cc = c & 7;
-      *reinterpret_cast<u32x4*>(&xs[buf][row * kXS + 8 * cc]) = xr[q];
-      *reinterpret_cast<u32x4*>(&ws[buf][row * kXS + 8 * cc]) = wr[q];
+      *reinterpret_cast<u32x4*>(xs + 32 * q * kXS) = xr[q];
+      *reinterpret_cast<u32x4*>(xs + (kBM + 32 * q) * kXS) = wr[q];
     }
   };
   f32x16 acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  const int nk = p.K / kBK;
-  load(0);
-  stage(0);
+  if (mine > 0) { load(0); stage(0); }
   __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk) load((kt + 1) * kBK);
-    const uint16_t* xb = xs[kt & 1] + (32 * wm + i) * kXS + 8 * g;
-    const uint16_t* wb = ws[kt & 1] + (32 * wn + i) * kXS + 8 * g;
+  for (int kt = 0; kt < steps; ++kt) {
+    if (kt + 1 < mine) load(kt + 1);
+    if (kt < mine) {
+      const uint16_t* xb = mem + (kt & 1) * kTileStage + (32 * wm + i) * kXS + 8 * g;
+      const uint16_t* wb = mem + (kt & 1) * kTileStage + (kBM + 32 * wn + i) * kXS + 8 * g;
 #pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
-      // A = 32 tokens x 16, B = 16 x 32 output columns (rows of W): acc[v] = y[token 8(v/4) + 4g + v%4][column i]
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(xb + 16 * ks);
-      const bf16x8 bq = *reinterpret_cast<const bf16x8*>(wb + 16 * ks);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bq, acc, 0, 0, 0);
+      for (int ks = 0; ks < kBK / 16; ++ks) {
+        // A = 32 tokens x 16, B = 16 x 32 output columns (rows of W): acc[v] = y[token 8(v/4) + 4g + v%4][column i]
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(xb + 16 * ks);
+        const bf16x8 bq = *reinterpret_cast<const bf16x8*>(wb + 16 * ks);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bq, acc, 0, 0, 0);
+      }
     }
-    if (kt + 1 < nk) stage((kt + 1) & 1);
+    if (kt + 1 < mine) stage((kt + 1) & 1);
     __syncthreads();
   }
-  // ---- stage the fp32 tile (it reuses the x / W buffers, which every wave has finished reading)
-  float* cs = reinterpret_cast<float*>(&xs[0][0]);
-  static_assert(sizeof(xs) >= kBM * kCS * sizeof(float), "the staged tile fits the x buffers");
+  // ---- stage the fp32 tiles (each reuses its group's buffers, which every wave has finished reading) and add them
+  constexpr int kGroupFloats = 2 * kTileStage / 2;
+  float* const all = reinterpret_cast<float*>(tile_mem);
+  static_assert(kGroupFloats >= kBM * kCS, "the staged tile fits a group's buffers");
 #pragma unroll
-  for (int v = 0; v < 16; ++v) cs[(32 * wm + 8 * (v >> 2) + 4 * g + (v & 3)) * kCS + 32 * wn + i] = acc[v];
+  for (int v = 0; v < 16; ++v) all[grp * kGroupFloats + (32 * wm + 8 * (v >> 2) + 4 * g + (v & 3)) * kCS + 32 * wn + i] = acc[v];
   __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int c = q * 256 + tid, row = c >> 3, cc = c & 7;
+  for (int c = threadIdx.x; c < kBM * kBN / 8; c += 256 * KS) {
+    const int row = c >> 3, cc = c & 7;
     const int m = m0 + row, c0 = n0 + 8 * cc;
     if (m >= p.M || c0 >= p.N) continue;
-    float y[8];
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(cs + row * kCS + 8 * cc), hi = *reinterpret_cast<const f32x4*>(cs + row * kCS + 8 * cc + 4);
+    float y[8] = {};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) { y[j] = lo[j]; y[4 + j] = hi[j]; }
+    for (int k = 0; k < KS; ++k) {
+      const float* const src = all + k * kGroupFloats + row * kCS + 8 * cc;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { y[j] += lo[j]; y[4 + j] += hi[j]; }
+    }
     bool rotate; int j0, pos;
     uint16_t* dst = chunk_destination<uint16_t>(p, m, c0, rotate, j0, pos);
     if (!dst) continue;
@@ -193,7 +221,7 @@ __global__ __launch_bounds__(256) void append_mfma_kernel(AppendParams p) {
 // (one per SIMD, 512 registers each: the 256 accumulators sit in AGPRs).  A wave owns 128 tokens x 128
 // columns = 4 x 4 blocks of v_mfma_f32_32x32x16_bf16, computed transposed (A = rows of W, B = tokens), so
 // that a lane ends up with runs of four consecutive columns of one token.  A k step reads 8 fragments for
-// 16 MFMAs (the 64 x 64 tiles above read 2 for 1, which is what bounds them; eight waves of 64 x 128 read
+// 16 MFMAs (the 64 x 64 tiles above read 2 for 1; eight waves of 64 x 128 read
 // 6 for 8 and measured the same time as this form).  x and W tiles of 256 rows x 64 k are double buffered
 // in LDS (row stride 72 elements), raw buffer loads over the tile's rows only (rows past the end read as
 // zeros and are never stored).
@@ -206,8 +234,6 @@ __global__ __launch_bounds__(256) void append_mfma_kernel(AppendParams p) {
 // columns at a time, and finishes 16-byte chunks; everything that depends on the token alone (sequence,
 // position, cache row or page) is worked out once per workgroup into a small LDS table, everything that
 // depends on the column alone once per lane and piece.
-// Grid: linear ids are dealt to the 8 XCDs round robin, so the column tiles of one token tile get ids
-// that are 8 apart (same XCD: its L2 serves their x tiles).
 // WB = blocks of 32 per wave and dimension: 4 (the tile described above) or 2 (128 x 128 tiles, a wave owns
 // 64 x 64, 4 fragment reads per 4 MFMAs) for chunks too small to fill the chip with the large tiles.
 // KS = groups of four waves that share the contraction of one tile.  Up to 256 small tiles leave a compute unit one workgroup, and
@@ -235,9 +261,8 @@ __global__ __launch_bounds__(256 * KS) void append_gemm_kernel(AppendParams p) {
   const int tid = threadIdx.x & 255, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int wm = w >> 1, wn = w & 1;
   const int ntn = (p.N + kGN - 1) / kGN, ntm = (p.M + kGM - 1) / kGM;
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int tm = (slot / ntn) * 8 + xcd, tn = slot % ntn;
-  if (tm >= ntm) return;  // the grid is rounded up to whole groups of 8 token tiles
+  int tm, tn;
+  if (!tile_of_workgroup(blockIdx.x, ntm, ntn, tm, tn)) return;
   const int m0 = tm * kGM, n0 = tn * kGN;
   const uint16_t* x = static_cast<const uint16_t*>(p.x);
   const uint16_t* wt = static_cast<const uint16_t*>(p.w);
@@ -463,8 +488,8 @@ __global__ __launch_bounds__(256 * KS) void append_gemm_kernel(AppendParams p) {
 // behind the first one's way from HBM; hence the tokens are dealt to more workgroups while there are idle ones.
 // (Until now operands were read as fragments, half a cache line per row, and the contraction was split over workgroups with
 // a second kernel to add the parts.  d_model 4096, us before / now: 1 token x 1600 columns 10.9 / 7.2, 24 x 1440 11.6 / 7.6,
-// 48 x 1600 13.5 / 9.5, 64 x 4096 23.5 / 15.3; above 64 tokens against 64 x 64 tiles: 128 x 1600 50 / 13.6, 256 x 1600
-// 50 / 22, 256 x 4096 50 / 44.)
+// 48 x 1600 13.5 / 9.5, 64 x 4096 23.5 / 15.3; above 64 tokens against 64 x 64 tiles of one group: 128 x 1600 38 /
+// 13.6.)
 template <int MB>
 struct RowsTile {
   static constexpr int kTok = 16 * MB;
@@ -619,13 +644,12 @@ __global__ __launch_bounds__(256) void append_generic_kernel(AppendParams p) {
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
-// 256 x 256 tiles (WB = 4) pay once they fill three quarters of the chip (256 CUs, one workgroup each), 128 x 128
-// tiles (WB = 2) from half of it; the rotation tables must allow 16-byte reads of four angles
-template <int WB>
+// The tiles of 256 x 256 and 128 x 128 read the rotation tables four angles at a time, and take what is more than one round of
+// the 64 x 64 tiles with their contraction in two groups (512 of them).  d_model 4096, us of 64 x 64 / 128 x 128: 1200 tokens x
+// 1600 columns (475) 29.9 / 37.2, 416 x 4608 (504) 33 / 38, 1536 x 1440 (552) 39.6 / 37.4, 600 x 4096 (640) 42.8 / 37.2.
 bool gemm_tiles_pay(const AppendParams& p, const TpaAppendArgs* a) {
-  constexpr int kM = GemmTile<WB, 1>::kM, kN = GemmTile<WB, 1>::kN;
-  const int64_t tiles = (int64_t)((p.M + kM - 1) / kM) * ((p.N + kN - 1) / kN);
-  return tiles >= (WB == 4 ? 192 : 128) && tiles < (1 << 28) && p.D % 8 == 0 && aligned16(a->rope_cos) && aligned16(a->rope_sin);
+  const int64_t tiles = (int64_t)((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
+  return tiles > 512 && tiles < (1 << 28) && p.D % 8 == 0 && aligned16(a->rope_cos) && aligned16(a->rope_sin);
 }
 
 template <int WB, int KS>
@@ -636,14 +660,25 @@ int launch_gemm(const AppendParams& p, hipStream_t s) {
   auto kern = append_gemm_kernel<WB, KS>;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), Tile::kLds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((ntm + 7) / 8 * 8 * ntn), dim3(256 * KS), Tile::kLds, s, p);
+  hipLaunchKernelGGL(kern, dim3(tile_workgroups(ntm, ntn)), dim3(256 * KS), Tile::kLds, s, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
-// The few-token kernel serves calls of at most three rounds of its workgroups of 64 tokens (d_model 4096, us against 64 x 64
-// tiles: 768 tokens x 960 columns, 720 workgroups, 31 / 43; 1024 x 720, 720, 35 / 37; 1200 x 720, 855, 48 / 37; 1024 x 960,
-// 960, 45 / 38).
-bool few_tokens(const AppendParams& p) { return (int64_t)((p.N + 15) / 16) * ((p.M + 63) / 64) <= 768; }
+template <int KS>
+int launch_tiles(const AppendParams& p, hipStream_t s) {
+  const int ntm = (p.M + kBM - 1) / kBM, ntn = (p.N + kBN - 1) / kBN;
+  constexpr size_t lds = (size_t)KS * 2 * kTileStage * sizeof(uint16_t);
+  auto kern = append_mfma_kernel<KS>;
+  static bool configured[kMaxDevices] = {};
+  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(tile_workgroups(ntm, ntn)), dim3(256 * KS), lds, s, p, ntm, ntn);
+  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+}
+
+// The few-token kernel serves up to 400 of its workgroups of 64 tokens (d_model 4096, us against 64 x 64 tiles: 300 tokens x 720
+// columns, 225 workgroups, 11.5 / 19.3; 300 x 1280, 400, 18.1 / 18.8; 600 x 720, 450, 20.6 / 19.7; 300 x 1600, 500, 24.5 / 19.1;
+// 416 x 1440, 630, 26.2 / 19.4; 1000 x 720, 720, 34.6 / 20.1).
+bool few_tokens(const AppendParams& p) { return (int64_t)((p.N + 15) / 16) * ((p.M + 63) / 64) <= 400; }
 
 template <int MB>
 int launch_rows(const AppendParams& p, hipStream_t s) {
@@ -710,18 +745,23 @@ extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
     const int nct = (p.N + 15) / 16;
     const int rc = nct * ((p.M + 15) / 16) <= 256 ? launch_rows<1>(p, s) : nct * ((p.M + 31) / 32) <= 256 ? launch_rows<2>(p, s) : launch_rows<4>(p, s);
     if (rc != TPA_OK) return rc;
-  } else if (mfma && gemm_tiles_pay<4>(p, a)) {
-    if (int rc = launch_gemm<4, 1>(p, s); rc != TPA_OK) return rc;
-  } else if (mfma && gemm_tiles_pay<2>(p, a)) {
-    // Two groups of waves need an even number of k steps, and an XCD that holds all its tiles at once (whole rows of column
-    // tiles on 32 compute units): with their buffers a compute unit holds one tile, with those of one group two.  d_model
-    // 4096, us with one / two groups: 2048 tokens x 1600 columns (26 tiles per XCD) 56 / 45.5, 3178 x 1120 (36) 69 / 75.
-    const int per_xcd = ((p.M + 127) / 128 + 7) / 8 * ((p.N + 127) / 128);
-    if (int rc = p.K % (2 * kGK) == 0 && per_xcd <= 32 ? launch_gemm<2, 2>(p, s) : launch_gemm<2, 1>(p, s); rc != TPA_OK) return rc;
+  } else if (mfma && gemm_tiles_pay(p, a)) {
+    // With t tiles of 128 x 128 these take 0.155 t + 25 us (from 512 on; d_model 4096) and rounds of 256 tiles of 256 x 256 122 us each.
+    // Measured, 128 / 256: 6600 tokens x 1440 columns (624) 133 / 128, 2048 x 5120 (640) 139 / 129, 6600 x 1600 (676) 137 / 124,
+    // 3264 x 4608 (936) 153 / 135, 3264 x 5120 (1040) 184 / 237, 4352 x 4608 (1224) 214 / 240, 6600 x 4096 (1664) 277 / 254.
+    const int64_t small = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128), large = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
+    // Two groups of waves need an even number of k steps and one round of tiles: with their buffers a compute unit holds one
+    // tile, with those of one group two.  d_model 4096, us with one / two groups: 2048 x 1600 (208) 56 / 40, 3178 x 1120 (225,
+    // then 36 on one XCD) 69 / 75.
+    const int rc = small + 180 > (large + 255) / 256 * 790 ? launch_gemm<4, 1>(p, s)
+                   : p.K % (2 * kGK) == 0 && small <= 256  ? launch_gemm<2, 2>(p, s)
+                                                           : launch_gemm<2, 1>(p, s);
+    if (rc != TPA_OK) return rc;
   } else if (mfma) {
-    dim3 grid((p.N + kBN - 1) / kBN, (p.M + kBM - 1) / kBM);
-    if (grid.y > 65535) return TPA_ERR_SHAPE;
-    hipLaunchKernelGGL(append_mfma_kernel, grid, dim3(256), 0, s, p);
+    const int64_t ntm = (p.M + kBM - 1) / kBM, tiles = ntm * ((p.N + kBN - 1) / kBN);
+    if (ntm > 65535 || tiles > 2147483640) return TPA_ERR_SHAPE;
+    const int rc = tiles <= 256 ? launch_tiles<4>(p, s) : tiles <= 512 ? launch_tiles<2>(p, s) : launch_tiles<1>(p, s);
+    if (rc != TPA_OK) return rc;
   } else {
     const int64_t chunks = (int64_t)p.M * (p.N / 8);
     const int64_t blocks = (chunks + 255) / 256;

@@ -18,8 +18,9 @@ pytestmark = pytest.mark.gpu
         (11, 3, 1088, 32, 128, 6, 2),  # 17 chunks; 33 tokens x 100 column blocks: blocks of 32
         (13, 5, 64, 32, 128, 6, 2),    # one chunk; 65 tokens: blocks of 64, the last of one token
         (3, 30, 2112, 8, 64, 1, 1),    # 33 chunks; 216 columns: the last block owns 8 of its 16
-        (2, 83, 512, 64, 64, 16, 8),   # 166 tokens x 256 column blocks: 768 workgroups, the most it serves
+        (2, 83, 512, 64, 64, 16, 8),   # 166 tokens x 256 column blocks: 768 workgroups: tiles
         (3, 71, 512, 64, 64, 16, 8),   # 213 tokens, 1024: tiles
+        (4, 63, 512, 32, 128, 6, 2),   # 252 tokens x 100 column blocks: 400 workgroups, the most it serves
     ],
 )
 def test_append_few_tokens(gpu, b, n, dm, h, d, rq, rk):
