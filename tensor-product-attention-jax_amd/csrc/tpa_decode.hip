@@ -26,6 +26,8 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kRowsPerBlock = 32;
+constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
+constexpr int64_t kFarthestRow = 1 << 25;  // elements between neighbouring rows of the cache, at most: 31 of them in a block, offsets of 32 bits
 constexpr int kMinKeys = kWaves * kRowsPerBlock / 2;  // keys of a range with one block of rank 2 per wave
 // Several query rows make the partials and their merge dearer: ranges of two blocks per wave then (step of 6 sequences of
 // 1022 .. 2048 tokens, four query tokens each: 31.9 us; 33.4 with ranges of one block).
@@ -40,6 +42,7 @@ struct DecodeParams {
   const int32_t* kvlen;  // [B] keys per batch entry, or null (= lk)
   const int32_t* page_table;  // paged cache: [B, pages_per_seq] physical page of each logical page
   int page_size, pages_per_seq;  // tokens per page; table row length
+  int page_shift;  // log2 of the rows (token, rank) of a page, or -1: no power of two
   int B, lq, lk, H, rq;
   int climit;      // query row qi sees its first qi + climit keys (causal: offset + 1; otherwise lk, no limit)
   int cbr;         // causal, last query aligned with the last key of each batch entry: climit counts from len - lq_total
@@ -126,47 +129,85 @@ __device__ __forceinline__ bool range_of(const DecodeParams& p, int x, int& b, i
 // the packed words of neighbouring q gives the order of the fragments.
 // (On the vector ALU this took 8 600 of the 35 800 cycles of a decode of 1500 keys, half of them the conversions; with this
 // form and the merge of the waves in 16-byte words, 64 x 8192 keys: 112.1 -> 107.3 us.)
-template <int NDB>
-struct QRaw { uint16_t a[8], b[NDB][8]; };
-template <int NDB>
-__device__ __forceinline__ QRaw<NDB> load_q_factors(const uint16_t* ap, int64_t a_stride, const uint16_t* bp, int64_t b_stride, int r0, int rq, int g) {
-  QRaw<NDB> raw;
-  const uint16_t* pa = ap + min(r0 + 8 * g, rq - 1) * a_stride;
-  const uint16_t* pb = bp + min(r0 + 8 * g, rq - 1) * b_stride;
+// Both operands have the ranks innermost, which memory has not: the token factors come as whole rows, 16 bytes a lane, and are
+// transposed by the reads of the wave's LDS region (laid out as the cache's rows are, in `lds`), the head factors two bytes at a
+// time: 6 loads a lane for a rank of 6 where two bytes at a time for both took 40.  Slot (g, j) of a fragment is rank 8 (j / 4) + 4 g + j % 4 of the step, in both; steps of up to 8 ranks load half of it.
+template <int D>
+struct QRaw { uint16_t a[8]; u32x4 b[D / 32]; };
+template <int D>
+__device__ __forceinline__ QRaw<D> load_q_factors(const uint16_t* ap, int64_t a_stride, const uint16_t* bp, int64_t b_stride, int r0, int rq, int l) {
+  constexpr int CPR = D / 8, RPI = 64 / CPR;
+  const int g = l >> 5;
+  QRaw<D> raw = {};
+  // reads past the last rank repeat it and count as zero
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    raw.a[j] = *pa;
+  for (int half = 0; half < 2; ++half) {
+    if (half && r0 + 8 >= rq) break;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) raw.b[db][j] = pb[32 * db];
-    const bool more = r0 + 8 * g + j + 1 < rq;  // reads past the last rank repeat it and count as zero
-    pa += more ? a_stride : 0;
-    pb += more ? b_stride : 0;
+    for (int n = half * D / 64; n < (half + 1) * D / 64; ++n)
+      raw.b[n] = *reinterpret_cast<const u32x4*>(bp + min(r0 + n * RPI + l / CPR, rq - 1) * b_stride + 8 * (l % CPR));
+    const uint16_t* pa = ap + min(r0 + 8 * half + 4 * g, rq - 1) * a_stride;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      raw.a[4 * half + j] = *pa;
+      pa += r0 + 8 * half + 4 * g + j + 1 < rq ? a_stride : 0;
+    }
   }
   return raw;
 }
-template <int NKS>
-__device__ __forceinline__ void finish_q_fragments(QRaw<NKS / 2> raw, const uint16_t* ap, int64_t a_stride, const uint16_t* bp, int64_t b_stride,
-                                                   int rq, float scale, int g, bf16x8 (&qf)[NKS]) {
-  constexpr int NDB = NKS / 2;
+
+// Where a lane's pieces of a tile of rows of D lie in LDS (elements; 16-byte chunk c of row r at chunk c ^ (r mod chunks)): one
+// address each, from which the others differ by an exclusive or with a constant, a constant, or both.
+template <int D>
+struct TileAt {
+  static constexpr int CPR = D / 8, RPI = 64 / CPR;
+  int wr, row, tr;
+  __device__ __forceinline__ explicit TileAt(int l) {
+    const int i = l & 31, g = l >> 5, lp = l & 15, dhalf = (l >> 4) & 1, r = 4 * g + (lp >> 2);
+    wr = (l / CPR) * D + 8 * ((l % CPR) ^ (l / CPR));
+    row = i * D + 8 * (g ^ (i & (CPR - 1)));
+    tr = r * D + 8 * ((2 * dhalf + ((lp & 3) >> 1)) ^ r) + 4 * (lp & 1);
+  }
+  __device__ __forceinline__ int write(int n) const { return (wr ^ (8 * ((n * RPI) & (CPR - 1)))) + n * RPI * D; }  // row n RPI + l / CPR, chunk l % CPR
+  __device__ __forceinline__ int read(int ks) const { return row ^ (16 * ks); }                                    // row i, chunk 2 ks + g
+  // transposed: rows 16 kk + 8 hi + 4 g + 0..3, columns 32 db + 0..31
+  __device__ __forceinline__ int read_tr(int kk, int hi, int db) const { return (tr ^ (32 * db) ^ (hi && CPR == 16 ? 64 : 0)) + (16 * kk + 8 * hi) * D; }
+};
+template <int D>
+__device__ __forceinline__ bf16x8 tile_tr(const uint16_t* tile, const TileAt<D>& at, int kk, int db) {
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + at.read_tr(kk, 0, db)));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + at.read_tr(kk, 1, db)));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int D>
+__device__ __forceinline__ void finish_q_fragments(QRaw<D> raw, const uint16_t* ap, int64_t a_stride, const uint16_t* bp, int64_t b_stride,
+                                                   int rq, float scale, int l, uint16_t* lds, const TileAt<D>& at, bf16x8 (&qf)[D / 16]) {
+  constexpr int NDB = D / 32, NKS = D / 16, CPR = D / 8, RPI = 64 / CPR;
+  const int g = l >> 5;
   f32x16 acc[NDB];
+  auto step = [&](int r0, auto first_c) __attribute__((always_inline)) {
 #pragma unroll
-  for (int db = 0; db < NDB; ++db)
+    for (int n = 0; n < D / 32; ++n)
+      *reinterpret_cast<u32x4*>(lds + at.write(n)) = r0 + n * RPI + l / CPR < rq ? raw.b[n] : u32x4{0, 0, 0, 0};
+    u32x4 aw;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[db][v] = 0.f;
-  for (int r0 = 0;;) {
-    auto operand = [&](const uint16_t (&x)[8]) {
-      u32x4 w;
+    for (int j = 0; j < 4; ++j) {
+      const int r = r0 + 8 * (j >> 1) + 4 * g + 2 * (j & 1);
+      aw[j] = (r < rq ? (uint32_t)raw.a[2 * j] : 0u) | (r + 1 < rq ? (uint32_t)raw.a[2 * j + 1] << 16 : 0u);
+    }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        w[j] = (r0 + 8 * g + 2 * j < rq ? (uint32_t)x[2 * j] : 0u) | (r0 + 8 * g + 2 * j + 1 < rq ? (uint32_t)x[2 * j + 1] << 16 : 0u);
-      return __builtin_bit_cast(bf16x8, w);
-    };
-    const bf16x8 a = operand(raw.a);
+    for (int db = 0; db < NDB; ++db) {
+      f32x16 c;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(raw.b[db]), a, acc[db], 0, 0, 0);
-    r0 += 16;
-    if (r0 >= rq) break;
-    raw = load_q_factors<NDB>(ap, a_stride, bp, b_stride, r0, rq, g);
+      for (int v = 0; v < 16; ++v) c[v] = decltype(first_c)::value ? 0.f : acc[db][v];
+      acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tile_tr<D>(lds, at, 0, db), __builtin_bit_cast(bf16x8, aw), c, 0, 0, 0);
+    }
+  };
+  step(0, std::true_type{});
+  for (int r0 = 16; r0 < rq; r0 += 16) {
+    raw = load_q_factors<D>(ap, a_stride, bp, b_stride, r0, rq, l);
+    step(r0, std::false_type{});
   }
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) {
@@ -192,7 +233,7 @@ struct DecodeLds {
   static constexpr size_t bytes(int nq) { return kBytes + (nq > 1 ? (size_t)nq * (D / 16) * 64 * 16 : 0); }
 };
 
-template <int D, int RK, bool PAGED, int NQ>
+template <int D, int RK, bool PAGED, int NQ, bool STREAM>
 __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   constexpr int CPR = D / 8;               // 16-byte chunks per B row
   constexpr int RPI = 64 / CPR;            // B rows per load instruction
@@ -227,6 +268,8 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   uint16_t* lds_ak = lds + 2 * DecodeLds<D>::kB;
   uint16_t* lds_av = lds_ak + DecodeLds<D>::kA;
 
+  const TileAt<D> at(l);
+
   // ---- Qm^T fragments: requested ahead of the cache's first blocks, finished while those are in flight.
   // With one query row they stay in registers; with NQ rows wave r builds row r's fragments once
   // and parks them in LDS behind the waves' staging regions (fragment (r, ks) of lane l at
@@ -236,18 +279,18 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   u32x4* const lds_q = reinterpret_cast<u32x4*>(smem + kWaves * DecodeLds<D>::kPerWave);
   const int qi_build = NQ == 1 ? qi0 : min(qi0 + w, p.lq - 1);
   const uint16_t* const qa_row = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qi_build * p.qa.stride_l + hl;
-  const uint16_t* const qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qi_build * p.qb.stride_l + i;
-  auto build_q = [&](const QRaw<NDB>& raw) __attribute__((always_inline)) {
+  const uint16_t* const qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qi_build * p.qb.stride_l;
+  auto build_q = [&](const QRaw<D>& raw) __attribute__((always_inline)) {
     if constexpr (NQ == 1) {
-      finish_q_fragments<NKS>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, g, qf);
+      finish_q_fragments<D>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, l, lds, at, qf);
     } else {
       if (w < NQ) {
         bf16x8 tmp[NKS];
-        finish_q_fragments<NKS>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, g, tmp);
+        finish_q_fragments<D>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, l, lds, at, tmp);
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) lds_q[(w * NKS + ks) * 64 + l] = __builtin_bit_cast(u32x4, tmp[ks]);
       }
-      __syncthreads();
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the cache's loads stay in flight
     }
   };
 
@@ -286,68 +329,68 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
 
   // two register sets: while one block is staged and consumed, two more are in flight (one set
   // with NQ rows, whose accumulators take the room and whose blocks take NQ times as long to
-  // consume).  The cache is read exactly once per call, so the loads are marked non-temporal
-  // (measured on the whole call: 5.1 -> 5.75 TB/s)
+  // consume)
   constexpr int NSETS = NQ == 1 ? 2 : 1;
   u32x4 rbk[NSETS][NLB], rbv[NSETS][NLB], rak[NSETS][2], rav[NSETS][2];
-  // Paged cache: the page a block lies in is looked up one visit of its register set ahead (when the set's
-  // previous block is requested), so that no request waits for a page-table entry
-  int32_t page_ahead[NSETS] = {};
-  auto lookup = [&](int blk) __attribute__((always_inline)) -> int32_t {
-    return PAGED && blk < blk_end ? p.page_table[(int64_t)b * p.pages_per_seq + blk * kRowsPerBlock / rpp] : 0;
+  // Paged cache: the place of a block (its page, the row in it) is looked up one visit of its register set ahead (when the
+  // set's previous block is requested), so that no request waits for a page-table entry
+  struct Place { int32_t page; int row; };  // the page as loaded: made a scalar only where it is used, which waits for it
+  Place ahead[NSETS] = {};
+  auto lookup = [&](int blk) __attribute__((always_inline)) -> Place {
+    if constexpr (!PAGED) return Place{0, 0};
+    const int row0 = max(min(blk, blk_end - 1), 0) * kRowsPerBlock, page = p.page_shift >= 0 ? row0 >> p.page_shift : row0 / rpp;
+    return Place{p.page_table[(int64_t)b * p.pages_per_seq + page], row0 - page * rpp};
   };
-  // One row group per cache slice: each byte is used once and the loads are marked non-temporal.  Several
-  // (more query rows than a workgroup serves): the groups' workgroups run side by side on one XCD and the
-  // later one is meant to find the slice in its L2, so the loads stay ordinary (four rows at the c4 shape:
-  // 1022 MB fetched with non-temporal loads, 676 MB = the cache once with ordinary ones).
-  auto load16 = [&](const uint16_t* ptr, auto nt_c) __attribute__((always_inline)) -> u32x4 {
-    if constexpr (decltype(nt_c)::value) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ptr));
-    else return *reinterpret_cast<const u32x4*>(ptr);
-  };
-  auto issue_as = [&](auto set_c, int blk, auto nt_c) __attribute__((always_inline)) {
+  // A block's rows are read through buffer resources that end with its last valid row (what lies past it reads as zero): the
+  // lane's offset in a block never changes and the rest of an address is scalar.  Offsets inside a block have 32 bits
+  // (kFarthestRow).
+  // Every request is made whether or not its block is there (a block past the last one has no rows: its resource is empty), and
+  // there is no branch around a load: each path through the loop then has the same number of loads in flight, and the wait in
+  // front of `stage` counts past the other set's.  Behind a branch they are waited for by the count of the path without them: to
+  // the last one, and the second set is in flight in name only.
+  // us per call, addresses per lane and load behind branches / this, 32 heads of 128, rank 2: 90 sequences of 6000 keys, two
+  // rows, 136 / 125; 300 of 1000, one row, 100 / 95; 16 heads of 64: 20 of 12 345 31.8 / 30.7.  64 x 8192 keys (108 us) is bound
+  // by HBM and has them alike; 40 paged sequences of 4800 - 9600 keys, 64 heads of 64, lose 2 % (77.7 / 79.4).
+  const int kb_sr = 2 * (int)p.kb.stride_r, vb_sr = 2 * (int)p.vb.stride_r, ka_sr = 2 * (int)p.ka.stride_r, va_sr = 2 * (int)p.va.stride_r;
+  const int kb_voff = lb_row * kb_sr + 16 * lb_c, vb_voff = lb_row * vb_sr + 16 * lb_c;
+  const int ka_voff = la_row * ka_sr + 16 * la_c, va_voff = la_row * va_sr + 16 * la_c;
+  auto issue = [&](auto set_c, int blk) __attribute__((always_inline)) {
     constexpr int set = decltype(set_c)::value;
     const int row0 = blk * kRowsPerBlock;
-    // element offsets that take a logical row of this block to its place in the page pool
-    int64_t pkb = 0, pvb = 0, pka = 0, pva = 0;
+    const int rows = max(0, min(kRowsPerBlock, last_row + 1 - row0));
+    int64_t page = 0, first = row0;  // of a page pool: the page and the row in it
     if constexpr (PAGED) {
-      const int page = row0 / rpp;
-      const int64_t phys = page_ahead[set];
-      page_ahead[set] = lookup(blk + NSETS * blk_step);
-      const int64_t first = (int64_t)page * rpp;  // first logical row of the page
-      pkb = phys * p.kb.stride_b - first * p.kb.stride_r;
-      pvb = phys * p.vb.stride_b - first * p.vb.stride_r;
-      pka = phys * p.ka.stride_b - first * p.ka.stride_r;
-      pva = phys * p.va.stride_b - first * p.va.stride_r;
+      page = last_row < 0 ? 0 : scalar(ahead[set].page);
+      first = ahead[set].row;
+      ahead[set] = lookup(blk + NSETS * blk_step);
     }
+    const uint16_t* const kb = kb_base + page * p.kb.stride_b + first * p.kb.stride_r;
+    const uint16_t* const vb = vb_base + page * p.vb.stride_b + first * p.vb.stride_r;
+    const uint16_t* const ka = ka_base + page * p.ka.stride_b + first * p.ka.stride_r;
+    const uint16_t* const va = va_base + page * p.va.stride_b + first * p.va.stride_r;
+    auto rows_of = [&](const uint16_t* base, int sr, int width) __attribute__((always_inline)) {
+      return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, rows > 0 ? (rows - 1) * sr + 2 * width : 0, kRsrcFlags);
+    };
+    const __amdgpu_buffer_rsrc_t kb_rs = rows_of(kb, kb_sr, D), vb_rs = rows_of(vb, vb_sr, D);
+    const __amdgpu_buffer_rsrc_t ka_rs = rows_of(ka, ka_sr, 8 * a_chunks), va_rs = rows_of(va, va_sr, 8 * a_chunks);
+    constexpr int aux = STREAM ? 2 : 0;  // bit 1: non-temporal
 #pragma unroll
     for (int n = 0; n < NLB; ++n) {
-      const int row = min(row0 + n * RPI + lb_row, last_row);
-      rbk[set][n] = load16(kb_base + pkb + (int64_t)row * p.kb.stride_r + 8 * lb_c, nt_c);
-      rbv[set][n] = load16(vb_base + pvb + (int64_t)row * p.vb.stride_r + 8 * lb_c, nt_c);
+      rbk[set][n] = __builtin_amdgcn_raw_buffer_load_b128(kb_rs, kb_voff, n * RPI * kb_sr, aux);
+      rbv[set][n] = __builtin_amdgcn_raw_buffer_load_b128(vb_rs, vb_voff, n * RPI * vb_sr, aux);
     }
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      const int row = min(row0 + 16 * n + la_row, last_row);
-      rak[set][n] = load16(ka_base + pka + (int64_t)row * p.ka.stride_r + 8 * la_c, nt_c);
-      rav[set][n] = load16(va_base + pva + (int64_t)row * p.va.stride_r + 8 * la_c, nt_c);
-    }
-  };
-  auto issue = [&](auto set_c, int blk) {
-    if constexpr (NQ == 1) {
-      issue_as(set_c, blk, std::true_type{});
-    } else {
-      if (nqg == 1) issue_as(set_c, blk, std::true_type{});
-      else issue_as(set_c, blk, std::false_type{});
+      rak[set][n] = __builtin_amdgcn_raw_buffer_load_b128(ka_rs, ka_voff, 16 * n * ka_sr, aux);
+      rav[set][n] = __builtin_amdgcn_raw_buffer_load_b128(va_rs, va_voff, 16 * n * va_sr, aux);
     }
   };
   auto stage = [&](auto set_c) {
     constexpr int set = decltype(set_c)::value;
 #pragma unroll
     for (int n = 0; n < NLB; ++n) {
-      const int row = n * RPI + lb_row;
-      const int pos = lb_c ^ (row & (CPR - 1));
-      *reinterpret_cast<u32x4*>(lds_bk + row * D + 8 * pos) = rbk[set][n];
-      *reinterpret_cast<u32x4*>(lds_bv + row * D + 8 * pos) = rbv[set][n];
+      *reinterpret_cast<u32x4*>(lds_bk + at.write(n)) = rbk[set][n];
+      *reinterpret_cast<u32x4*>(lds_bv + at.write(n)) = rbv[set][n];
     }
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
@@ -373,13 +416,14 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
 
   using Set0 = std::integral_constant<int, 0>;
   using Set1 = std::integral_constant<int, 1>;
-  page_ahead[0] = lookup(blk_begin);
-  if constexpr (NSETS == 2) page_ahead[1] = lookup(blk_begin + blk_step);
-  const QRaw<NDB> q_raw = load_q_factors<NDB>(qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, 0, p.rq, g);
-  if (blk_begin < blk_end) issue(Set0{}, blk_begin);
-  if constexpr (NSETS == 2) {
-    if (blk_begin + blk_step < blk_end) issue(Set1{}, blk_begin + blk_step);
-  }
+  ahead[0] = lookup(blk_begin);
+  if constexpr (NSETS == 2) ahead[1] = lookup(blk_begin + blk_step);
+  const QRaw<D> q_raw = load_q_factors<D>(qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, 0, p.rq, l);
+  __builtin_amdgcn_sched_barrier(0);  // in the order of their use, as in the loop: what is waited for is counted from the last one
+  issue(Set0{}, blk_begin);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NSETS == 2) issue(Set1{}, blk_begin + blk_step);
+  __builtin_amdgcn_sched_barrier(0);
   build_q(q_raw);
 
   auto compute = [&](int blk) {
@@ -410,8 +454,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
       for (int v = 0; v < 16; ++v) sp[v] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
-        const int pos = (2 * ks + g) ^ (i & (CPR - 1));
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(lds_bk + i * D + 8 * pos);
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(lds_bk + at.read(ks));
         if constexpr (NQ == 1) {
           sp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], sp, 0, 0, 0);
         } else {
@@ -446,7 +489,9 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
       // the key ranges) is an exact power of two
       const float m_new = fmaxf(m[r], __builtin_ceilf(tmax));
       const float m_use = NQ > 1 && m_new == -INFINITY ? 0.f : m_new;
-      if (__any(m_new > m[r])) {
+      if (NQ == 1 && blk == blk_begin) {
+        m[r] = m_new;  // nothing to rescale yet
+      } else if (__any(m_new > m[r])) {
         const float alpha = __builtin_amdgcn_exp2f(m[r] - m_use);
         lsum[r] *= alpha;
 #pragma unroll
@@ -477,38 +522,31 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
       // ---- O^T[d, h] += sum_row B_v[row, d] P'^T[row, h]; slot (g, j) = row 16kk + 8(j/4) + 4g + j%4
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const int r_lo = 16 * kk + 4 * g + (lp >> 2);
-        const int r_hi = r_lo + 8;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          const int chunk = 4 * db + 2 * dhalf + ((lp & 3) >> 1);
-          const int sub = 4 * (lp & 1);
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (s16x4 __attribute__((address_space(3)))*)(lds_bv + r_lo * D + 8 * (chunk ^ (r_lo & (CPR - 1))) + sub));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (s16x4 __attribute__((address_space(3)))*)(lds_bv + r_hi * D + 8 * (chunk ^ (r_hi & (CPR - 1))) + sub));
-          const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-          o[r][db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[kk], o[r][db], 0, 0, 0);
-        }
+        for (int db = 0; db < NDB; ++db)
+          o[r][db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tile_tr<D>(lds_bv, at, kk, db), pf[kk], o[r][db], 0, 0, 0);
       }
     }
   };
 
   if constexpr (NSETS == 2) {
-    for (int blk = blk_begin; blk < blk_end; blk += 2 * blk_step) {
-      stage(Set0{});  // waits for this block's loads only; its registers are then free again
-      if (blk + 2 * blk_step < blk_end) issue(Set0{}, blk + 2 * blk_step);
+    int blk = blk_begin;
+    for (; blk + blk_step < blk_end; blk += 2 * blk_step) {  // left in one place, for the same reason
+      stage(Set0{});
+      issue(Set0{}, blk + 2 * blk_step);
       compute(blk);
-      if (blk + blk_step < blk_end) {
-        stage(Set1{});
-        if (blk + 3 * blk_step < blk_end) issue(Set1{}, blk + 3 * blk_step);
-        compute(blk + blk_step);
-      }
+      stage(Set1{});
+      issue(Set1{}, blk + 3 * blk_step);
+      compute(blk + blk_step);
+    }
+    if (blk < blk_end) {
+      stage(Set0{});
+      compute(blk);
     }
   } else {
     for (int blk = blk_begin; blk < blk_end; blk += blk_step) {
       stage(Set0{});
-      if (blk + blk_step < blk_end) issue(Set0{}, blk + blk_step);
+      issue(Set0{}, blk + blk_step);
       compute(blk);
     }
   }
@@ -537,6 +575,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
     __syncthreads();
 
     const int64_t pbase = ((int64_t)x * p.lq + qi0 + r) * p.H + h0;
+#pragma unroll(NQ == 1 ? 4 : 1)
     for (int idx = tid; idx < nh * (D / 4); idx += kWaves * 64) {
       const int hh = idx / (D / 4), d = 4 * (idx % (D / 4));
       float mw[kWaves], mmax = -INFINITY;
@@ -906,14 +945,16 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   p.cbr = a->causal == TPA_CAUSAL_BOTTOM_RIGHT;
   p.row0 = rows.row0; p.lq_total = rows.lq_total;
   p.page_table = a->page_table; p.page_size = a->page_size; p.pages_per_seq = a->pages_per_seq;
+  const int page_rows = a->page_size * RK;
+  p.page_shift = page_rows > 0 && (page_rows & (page_rows - 1)) == 0 ? __builtin_ctz(page_rows) : -1;
   p.qscale = a->sm_scale * kLog2e / ((float)a->rq * (float)RK);
   return p;
 }
 
-template <int D, int RK, bool PAGED, int NQ>
+template <int D, int RK, bool PAGED, int NQ, bool STREAM>
 int launch_decode_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   const DecodeParams p = decode_params<RK>(a, ranges, rows);
-  auto kern = decode_kernel<D, RK, PAGED, NQ>;
+  auto kern = decode_kernel<D, RK, PAGED, NQ, STREAM>;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), DecodeLds<D>::bytes(NQ)); rc != TPA_OK) return rc;
   dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * ((a->lq + NQ - 1) / NQ), (a->H + 31) / 32);
@@ -947,6 +988,19 @@ int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream,
   return launch_decode_f32_t<D, RK, false>(a, ranges, stream, rows);
 }
 
+// One row group per cache slice: each byte is used once and the loads are marked non-temporal (the whole call 5.1 -> 5.75 TB/s).
+// Several (more query rows than a workgroup serves): the groups' workgroups run side by side on one XCD and the later one is
+// meant to find the slice in its L2, so the loads stay ordinary (four rows at the c4 shape: 1022 MB fetched with non-temporal
+// loads, 676 MB = the cache once with ordinary ones).  Two head blocks read the same token rows as well; with two rows and from
+// rank 4 on that decides (3 x 9000 keys, 64 heads of 64, rank 4: 24.1 us non-temporal, 22.5 ordinary; rank 2 19.1 / 19.2, paged
+// 52.0 / 54.3), with one row the second block of loads hides it.
+template <int D, int RK, bool PAGED>
+int launch_decode_rows(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
+  if (a->lq == 1) return launch_decode_t<D, RK, PAGED, 1, true>(a, ranges, stream, rows);
+  if (a->lq == 2 && (a->H <= 32 || RK < 4)) return launch_decode_t<D, RK, PAGED, 2, true>(a, ranges, stream, rows);
+  return launch_decode_t<D, RK, PAGED, 2, false>(a, ranges, stream, rows);
+}
+
 template <int D, int RK>
 int launch_decode(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   if (a->page_table) {
@@ -954,9 +1008,9 @@ int launch_decode(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, Row
     if (a->page_size <= 0 || (a->page_size * RK) % kRowsPerBlock != 0 ||
         (int64_t)a->pages_per_seq * a->page_size < a->lk)
       return TPA_ERR_SHAPE;
-    return a->lq >= 2 ? launch_decode_t<D, RK, true, 2>(a, ranges, stream, rows) : launch_decode_t<D, RK, true, 1>(a, ranges, stream, rows);
+    return launch_decode_rows<D, RK, true>(a, ranges, stream, rows);
   }
-  return a->lq >= 2 ? launch_decode_t<D, RK, false, 2>(a, ranges, stream, rows) : launch_decode_t<D, RK, false, 1>(a, ranges, stream, rows);
+  return launch_decode_rows<D, RK, false>(a, ranges, stream, rows);
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
@@ -1017,7 +1071,7 @@ int tpa_decode_mfma_supported(const TpaFwdArgs* a) {
   const TpaFactor* fs[4] = {&a->ka, &a->kb, &a->va, &a->vb};
   for (const TpaFactor* f : fs) {
     if (f->stride_l != (int64_t)a->rk * f->stride_r) return 0;
-    if (!aligned16(f->ptr) || f->stride_r % 8 != 0 || f->stride_b % 8 != 0) return 0;
+    if (!aligned16(f->ptr) || f->stride_r % 8 != 0 || f->stride_b % 8 != 0 || f->stride_r < 0 || f->stride_r > kFarthestRow) return 0;
   }
   if (!aligned16(a->qb.ptr) || a->qb.stride_r % 8 != 0 || a->qb.stride_l % 8 != 0 || a->qb.stride_b % 8 != 0) return 0;
   return 1;

@@ -1,0 +1,50 @@
+"""The split-key decode kernels where their loop and the query's ranks change form: no, one, two, three and four blocks per wave
+with rows left over, ranks of the queries around half an operand (8) and a whole one (16), pages of a size that is and is not
+a power of two, against the CPU oracle."""
+
+import pytest
+import torch
+
+from conftest import make_factors
+from test_gpu_parity import BF16_TOL, _varlen_reference, as_f64, bf16_bounds, check, to_gpu, tpa_split
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("h,d,rk", [(16, 128, 2), (40, 64, 4)])
+@pytest.mark.parametrize("rq", [1, 8, 9, 16, 17, 33])
+@pytest.mark.parametrize("lq", [1, 2, 3])
+@pytest.mark.parametrize("page", [0, 48, 64])
+def test_blocks_per_wave(gpu, h, d, rk, rq, lq, page):
+    from tpa import tpa
+
+    per_wave = 4 * 32 // rk  # keys of one block per wave of a range
+    lengths = [0, 1, per_wave // 4, per_wave - 1, per_wave + 1, 2 * per_wave, 3 * per_wave - 5, 4 * per_wave]
+    b, lk = len(lengths), 4 * per_wave
+    q, k, v = make_factors(97, b, lq, lk, h, d, d, rq, rk, scale_by_rank=True)
+    tq, tk, tv = (to_gpu(x, torch.bfloat16, gpu) for x in (q, k, v))
+    o_ref, l_ref = _varlen_reference(as_f64(tq), as_f64(tk), as_f64(tv), lengths, h, d**-0.5, False)
+    bounds = bf16_bounds(tq, tk, tv, h, d**-0.5, form="factored")
+    qa, qb, *kv = tpa_split(tq, tk, tv, h)
+    table = None
+    for bi, n in enumerate(lengths):  # nothing past the end of an entry is used
+        for x in kv:
+            x[bi, n:] = float("nan")
+    if page:
+        per_seq = -(-lk // page)
+        order = torch.randperm(b * per_seq, generator=torch.Generator().manual_seed(5))
+        table = order.to(torch.int32).view(b, per_seq)
+        pools = []
+        for x in kv:
+            pool = torch.full((b * per_seq, page, *x.shape[2:]), float("nan"), dtype=x.dtype, device=x.device)
+            for bi in range(b):
+                for pi in range(per_seq):
+                    part = x[bi, pi * page : (pi + 1) * page]
+                    pool[int(table[bi, pi]), : part.shape[0]] = part
+            pools.append(pool)
+        kv, table = pools, table.to(gpu)
+        for bi, n in enumerate(lengths):  # entries of the table past an entry's last page are not followed
+            table[bi, max(0, -(-n // page)) :] = -(1 << 30)
+    kvl = torch.tensor(lengths, dtype=torch.int32)
+    o, lse = tpa.tpa_decode(qa, qb, *kv, sm_scale=d**-0.5, num_splits=1, kv_lengths=kvl, page_table=table, kernel=2)
+    check(o, lse, o_ref, l_ref, BF16_TOL, bounds)
