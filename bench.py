@@ -129,7 +129,7 @@ def add_hbm_sustained(roof):
 TRAFFIC_KERNELS = {  # workload -> the kernels of one step, as rocprofv3 prints the start of their names
     "c2": ["recon_bf16_h8_kernel", "prefill_kernel<128, 2, false>"],
     "c2u": ["prefill_kernel<128, 0, false>"],
-    "c4": ["decode_kernel<128, 2, false, 1>", "decode_merge_kernel<128, bf16"],
+    "c4": ["decode_kernel<128, 2, false, 1", "decode_merge_kernel<128, bf16"],
 }
 
 
