@@ -210,14 +210,6 @@ __device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {
     for (int v = 0; v < 16; ++v) acc[db][v] = 0.f;
 }
 
-// the largest magnitude of an accumulator's values: they are split only where that is not too large
-__device__ __forceinline__ bool too_large(const f32x16& x) {
-  float top = 0.f;
-#pragma unroll
-  for (int v = 0; v < 16; v += 2) top = largest(top, x[v], x[v + 1]);
-  return !(top < 0x1p127f);
-}
-
 // ------------------------------------------------------------------------------------- dQ
 template <int D, int NW, bool SEG>
 __global__ __launch_bounds__(NW * 64) void bwd_f32_dq_kernel(BwdF32Params p) {

@@ -222,6 +222,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
         }
 #pragma unroll
         for (int v = 0; v < 16; ++v) s[mb][v] += small[v];
+        bad |= too_large(s[mb]);  // -inf + inf is NaN where the fp32 instruction has -inf: the key drops out
       }
     } else {
 #pragma unroll
@@ -590,11 +591,14 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
       const int next = tile + NW;
       const bool more = next < ntiles;
       if (more) issue(in_v, vb_r, va_r, next, 0);
-      f32x16 s, s2;
+      f32x16 s;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) { s[v] = 0.f; s2[v] = 0.f; }
+      for (int v = 0; v < 16; ++v) s[v] = 0.f;
       asm volatile("" : "+v"(q_offset));  // Q is read again for every tile: held in registers it would not fit
       if constexpr (!decltype(fp32)::value) {
+        f32x16 s2;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s2[v] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) {
           float x[8];
@@ -609,6 +613,9 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
           s = mfma_bf16(kf.h, qf.h, s);
           __builtin_amdgcn_sched_barrier(0);  // the operands of one step at a time: more do not fit the registers
         }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s[v] += s2[v];
+        bad |= too_large(s);  // -inf + inf is NaN where the fp32 instruction has -inf: the key drops out
       } else {
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) {
@@ -635,7 +642,7 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
           const int32_t id_t = __shfl(seg_id, t, 64);  // by every lane, whatever it keeps
           keep = keep && id_t == qseg;
         }
-        s[v] = keep ? s[v] + s2[v] : -INFINITY;
+        s[v] = keep ? s[v] : -INFINITY;
         tmax = fmaxf(tmax, s[v]);
       }
       tmax = halves_max(tmax);

@@ -73,6 +73,13 @@ __device__ __forceinline__ float largest(float so_far, float a, float b) {
 __device__ __forceinline__ bool irregular(float largest_magnitude) {
   return !(largest_magnitude < 0x1p127f) || (largest_magnitude < 0x1p-50f && largest_magnitude != 0.f);
 }
+// of sums of products: one that left the range of floats on the way, of whose parts one may be -inf and another +inf
+__device__ __forceinline__ bool too_large(const f32x16& x) {
+  float top = 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; v += 2) top = largest(top, x[v], x[v + 1]);
+  return !(top < 0x1p127f);
+}
 
 __device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 // c_small takes the five small terms, c the large one (they may be the same)

@@ -49,12 +49,18 @@ def _spoil(kind, q, k, v, h):
         v[:, key, 1:, h + 7] = 0.0
     elif kind == "tiny values":
         v[:, :, :, h:] *= 1e-33
+    elif kind == "logit below the range":  # finite operands, products around -2^140 of which the parts have both signs
+        q[:, :, :, :h] = np.abs(q[:, :, :, :h]) + 0.5
+        k[:, key, :, :h] = np.abs(k[:, key, :, :h]) + 0.5
+        q[:, :, :, h] = np.float32(1.302 * 2.0**70)
+        k[:, :, :, h] = 0.0
+        k[:, key, :, h] = np.float32(-1.302 * 2.0**70)
     elif kind == "tiny queries, large keys":
         q[:, :, :, h:] *= 1e-19
         k[:, :, :, h:] *= 1e19
 
 
-@pytest.mark.parametrize("kind", ["ordinary", "infinite key", "infinite query", "NaN value", "infinite value", "rounds to infinity", "tiny values", "tiny queries, large keys"])
+@pytest.mark.parametrize("kind", ["ordinary", "infinite key", "infinite query", "NaN value", "infinite value", "rounds to infinity", "tiny values", "tiny queries, large keys", "logit below the range"])
 @pytest.mark.parametrize("b,t,h,d,rk", SHAPES)
 def test_forward_values_that_do_not_split(gpu, b, t, h, d, rk, kind):
     from tpa import tpa
