@@ -27,7 +27,10 @@ namespace {
 constexpr int kWaves = 4;
 constexpr int kRowsPerBlock = 32;
 constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
-constexpr int64_t kFarthestRow = 1 << 25;  // elements between neighbouring rows of the cache, at most: 31 of them in a block, offsets of 32 bits
+// How the cache is read: through buffer resources with or without the non-temporal hint, or, where the rows lie too far apart for
+// the 32-bit offsets of these (31 rows in a block) or in descending order, with an address per lane.
+enum class Reads { kOrdinary, kStreaming, kFar };
+constexpr int64_t kFarthestRow = 1 << 25;  // elements between neighbouring rows, at most, for the first two
 constexpr int kMinKeys = kWaves * kRowsPerBlock / 2;  // keys of a range with one block of rank 2 per wave
 // Several query rows make the partials and their merge dearer: ranges of two blocks per wave then (step of 6 sequences of
 // 1022 .. 2048 tokens, four query tokens each: 31.9 us; 33.4 with ranges of one block).
@@ -233,7 +236,7 @@ struct DecodeLds {
   static constexpr size_t bytes(int nq) { return kBytes + (nq > 1 ? (size_t)nq * (D / 16) * 64 * 16 : 0); }
 };
 
-template <int D, int RK, bool PAGED, int NQ, bool STREAM>
+template <int D, int RK, bool PAGED, int NQ, Reads READS>
 __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
   constexpr int CPR = D / 8;               // 16-byte chunks per B row
   constexpr int RPI = 64 / CPR;            // B rows per load instruction
@@ -342,8 +345,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
     return Place{p.page_table[(int64_t)b * p.pages_per_seq + page], row0 - page * rpp};
   };
   // A block's rows are read through buffer resources that end with its last valid row (what lies past it reads as zero): the
-  // lane's offset in a block never changes and the rest of an address is scalar.  Offsets inside a block have 32 bits
-  // (kFarthestRow).
+  // lane's offset in a block never changes and the rest of an address is scalar.
   // Every request is made whether or not its block is there (a block past the last one has no rows: its resource is empty), and
   // there is no branch around a load: each path through the loop then has the same number of loads in flight, and the wait in
   // front of `stage` counts past the other set's.  Behind a branch they are waited for by the count of the path without them: to
@@ -368,12 +370,28 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
     const uint16_t* const vb = vb_base + page * p.vb.stride_b + first * p.vb.stride_r;
     const uint16_t* const ka = ka_base + page * p.ka.stride_b + first * p.ka.stride_r;
     const uint16_t* const va = va_base + page * p.va.stride_b + first * p.va.stride_r;
+    if constexpr (READS == Reads::kFar) {
+      auto row_at = [&](const uint16_t* base, int row, int64_t stride, int c) __attribute__((always_inline)) {
+        return row < rows ? *reinterpret_cast<const u32x4*>(base + row * stride + 8 * c) : u32x4{0, 0, 0, 0};
+      };
+#pragma unroll
+      for (int n = 0; n < NLB; ++n) {
+        rbk[set][n] = row_at(kb, n * RPI + lb_row, p.kb.stride_r, lb_c);
+        rbv[set][n] = row_at(vb, n * RPI + lb_row, p.vb.stride_r, lb_c);
+      }
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        rak[set][n] = row_at(ka, 16 * n + la_row, p.ka.stride_r, la_c);
+        rav[set][n] = row_at(va, 16 * n + la_row, p.va.stride_r, la_c);
+      }
+      return;
+    }
     auto rows_of = [&](const uint16_t* base, int sr, int width) __attribute__((always_inline)) {
       return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, rows > 0 ? (rows - 1) * sr + 2 * width : 0, kRsrcFlags);
     };
     const __amdgpu_buffer_rsrc_t kb_rs = rows_of(kb, kb_sr, D), vb_rs = rows_of(vb, vb_sr, D);
     const __amdgpu_buffer_rsrc_t ka_rs = rows_of(ka, ka_sr, 8 * a_chunks), va_rs = rows_of(va, va_sr, 8 * a_chunks);
-    constexpr int aux = STREAM ? 2 : 0;  // bit 1: non-temporal
+    constexpr int aux = READS == Reads::kStreaming ? 2 : 0;  // bit 1: non-temporal
 #pragma unroll
     for (int n = 0; n < NLB; ++n) {
       rbk[set][n] = __builtin_amdgcn_raw_buffer_load_b128(kb_rs, kb_voff, n * RPI * kb_sr, aux);
@@ -951,10 +969,10 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   return p;
 }
 
-template <int D, int RK, bool PAGED, int NQ, bool STREAM>
+template <int D, int RK, bool PAGED, int NQ, Reads READS>
 int launch_decode_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   const DecodeParams p = decode_params<RK>(a, ranges, rows);
-  auto kern = decode_kernel<D, RK, PAGED, NQ, STREAM>;
+  auto kern = decode_kernel<D, RK, PAGED, NQ, READS>;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), DecodeLds<D>::bytes(NQ)); rc != TPA_OK) return rc;
   dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * ((a->lq + NQ - 1) / NQ), (a->H + 31) / 32);
@@ -996,9 +1014,11 @@ int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream,
 // 52.0 / 54.3), with one row the second block of loads hides it.
 template <int D, int RK, bool PAGED>
 int launch_decode_rows(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
-  if (a->lq == 1) return launch_decode_t<D, RK, PAGED, 1, true>(a, ranges, stream, rows);
-  if (a->lq == 2 && (a->H <= 32 || RK < 4)) return launch_decode_t<D, RK, PAGED, 2, true>(a, ranges, stream, rows);
-  return launch_decode_t<D, RK, PAGED, 2, false>(a, ranges, stream, rows);
+  for (const TpaFactor* f : {&a->ka, &a->kb, &a->va, &a->vb})
+    if (f->stride_r < 0 || f->stride_r > kFarthestRow) return launch_decode_t<D, RK, PAGED, 2, Reads::kFar>(a, ranges, stream, rows);
+  if (a->lq == 1) return launch_decode_t<D, RK, PAGED, 1, Reads::kStreaming>(a, ranges, stream, rows);
+  if (a->lq == 2 && (a->H <= 32 || RK < 4)) return launch_decode_t<D, RK, PAGED, 2, Reads::kStreaming>(a, ranges, stream, rows);
+  return launch_decode_t<D, RK, PAGED, 2, Reads::kOrdinary>(a, ranges, stream, rows);
 }
 
 template <int D, int RK>
@@ -1071,7 +1091,7 @@ int tpa_decode_mfma_supported(const TpaFwdArgs* a) {
   const TpaFactor* fs[4] = {&a->ka, &a->kb, &a->va, &a->vb};
   for (const TpaFactor* f : fs) {
     if (f->stride_l != (int64_t)a->rk * f->stride_r) return 0;
-    if (!aligned16(f->ptr) || f->stride_r % 8 != 0 || f->stride_b % 8 != 0 || f->stride_r < 0 || f->stride_r > kFarthestRow) return 0;
+    if (!aligned16(f->ptr) || f->stride_r % 8 != 0 || f->stride_b % 8 != 0) return 0;
   }
   if (!aligned16(a->qb.ptr) || a->qb.stride_r % 8 != 0 || a->qb.stride_l % 8 != 0 || a->qb.stride_b % 8 != 0) return 0;
   return 1;

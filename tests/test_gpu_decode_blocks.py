@@ -48,3 +48,52 @@ def test_blocks_per_wave(gpu, h, d, rk, rq, lq, page):
     kvl = torch.tensor(lengths, dtype=torch.int32)
     o, lse = tpa.tpa_decode(qa, qb, *kv, sm_scale=d**-0.5, num_splits=1, kv_lengths=kvl, page_table=table, kernel=2)
     check(o, lse, o_ref, l_ref, BF16_TOL, bounds)
+
+
+@pytest.mark.parametrize("lq", [1, 2, 3])
+@pytest.mark.parametrize("page", [0, 16])
+@pytest.mark.parametrize("order", ["far apart", "descending"])
+def test_rows_that_lie_far_apart_or_descend(gpu, order, page, lq):
+    """Rows of the cache more than 2^25 elements apart, or in descending order, give what the same rows next to each other give."""
+    from tpa import _dispatch as dd
+
+    b, lk, h, d, rq, rk, far = 2, 80, 16, 64, 6, 2, (1 << 25) + 8
+    q, k, v = (to_gpu(x, torch.bfloat16, gpu) for x in make_factors(98, b, lq, lk, h, d, d, rq, rk, scale_by_rank=True))
+    qa, qb, *kv = (x.contiguous() for x in tpa_split(q, k, v, h))
+    lengths = torch.tensor([lk, 37], dtype=torch.int32, device=gpu)
+    table = None
+    if page:
+        kv = [x.view(b * lk // page, page, rk, x.shape[-1]) for x in kv]
+        table = torch.arange(b * lk // page, dtype=torch.int32, device=gpu).view(b, -1)
+    lib = dd.load_library()
+    ws = torch.empty(1 << 24, dtype=torch.uint8, device=gpu)
+
+    def call(factors):
+        o = torch.empty((b, lq, h, d), dtype=torch.bfloat16, device=gpu)
+        lse = torch.empty((b, h, lq), dtype=torch.float32, device=gpu)
+        args = dd.TpaFwdArgs(
+            qa=dd.factor(qa), qb=dd.factor(qb), ka=factors[0], kb=factors[1], va=factors[2], vb=factors[3], o=o.data_ptr(), lse=lse.data_ptr(),
+            B=b, lq=lq, lk=lk, H=h, dk=d, dv=d, rq=rq, rk=rk, dtype=dd.dtype_code(torch.bfloat16), sm_scale=d**-0.5, kernel=dd.KERNEL_MFMA,
+            workspace=ws.data_ptr(), workspace_bytes=ws.numel(), num_splits=1, kv_lengths=lengths.data_ptr(),
+            page_table=table.data_ptr() if page else None, page_size=page, pages_per_seq=lk // page if page else 0)
+        dd.check("tpa_decode", lib.tpa_decode(args, dd.current_stream_ptr(gpu)))
+        torch.cuda.synchronize()
+        return o, lse
+
+    want = call([dd.factor(x) for x in kv])
+    moved = []
+    for n, x in enumerate(kv):
+        if order == "descending":
+            flipped = x.flip(1, 2).contiguous()
+            last = (x.shape[1] * rk - 1) * x.shape[3] * 2
+            moved.append((flipped, dd.TpaFactor(flipped.data_ptr() + last, x.stride(0), -x.stride(1), -x.stride(2))))
+        elif n == 1:  # one array is enough for the far form; batch entries (pages) lie between its rows
+            place = torch.empty((x.shape[1] * rk - 1) * far + x.shape[0] * d, dtype=x.dtype, device=gpu)
+            spread = place.as_strided(x.shape, (d, rk * far, far, 1))
+            spread.copy_(x)
+            moved.append((spread, dd.factor(spread)))
+        else:
+            moved.append((x, dd.factor(x)))
+    got = call([f for _, f in moved])
+    for x, y in zip(got, want):
+        torch.testing.assert_close(x, y, rtol=2.0**-7, atol=1e-3)
