@@ -5,6 +5,8 @@ numbers of chunks, ragged column blocks, and calls on either side of the line to
 import pytest
 import torch
 
+from tpa import tpa
+
 from test_gpu_append import test_append_matches_the_oracle as check_append
 
 pytestmark = pytest.mark.gpu
@@ -25,3 +27,23 @@ pytestmark = pytest.mark.gpu
 )
 def test_append_few_tokens(gpu, b, n, dm, h, d, rq, rk):
     check_append(gpu, torch.bfloat16, 2, b, n, dm, h, d, rq, rk, False)
+
+
+def test_results_are_the_roundings_of_exact_sums(gpu):
+    """Results of a long contraction that are not the bf16 rounding of the exact sum.  An fp32 sum that is off by e rounds to the
+    wrong side for a share of about 2 e / spacing of the results; with the chunks of 64 summed one by one that is 1.8e-4 here, with one
+    chain of matrix instructions per wave 3.2e-4 (1.8 million results: 320 and 590, give or take 25)."""
+    n, dm, h, d, rq, rk = 48, 16384, 32, 128, 6, 2
+    wrong = total = 0
+    for seed in range(24):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        x = torch.randn((1, n, dm), generator=g, device=gpu).to(torch.bfloat16)
+        w = (torch.randn(((rq + 2 * rk) * (h + d), dm), generator=g, device=gpu) * dm**-0.5).to(torch.bfloat16)
+        cos, sin = torch.ones((n, d // 2), device=gpu), torch.zeros((n, d // 2), device=gpu)
+        kv = [torch.zeros((1, n, rk, e), dtype=torch.bfloat16, device=gpu) for e in (h, d, h, d)]
+        qa, qb, _ = tpa.tpa_cache_append(x, w, cos, sin, *kv, torch.zeros(1, dtype=torch.int32, device=gpu), rank_q=rq, kernel=2)
+        got = torch.cat([t.reshape(n, -1) for t in (qa, qb, *kv)], dim=1)
+        want = (x[0].double() @ w.double().T).float().to(torch.bfloat16)
+        wrong += int((got != want).sum())
+        total += got.numel()
+    assert wrong <= 2.4e-4 * total, wrong / total
