@@ -10,6 +10,7 @@
 // fp32 results in LDS, and finish whole 16-byte chunks of eight columns: a chunk lies inside one rank
 // row of one factor (H and D are multiples of 8), so the rotation partners (2j, 2j+1) are inside it.
 // Any other dtype / shape: one thread per chunk of eight columns, fp32 arithmetic.
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -657,7 +658,7 @@ bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15)
 // 1600 columns (475) 29.9 / 37.2, 416 x 4608 (504) 33 / 38, 1536 x 1440 (552) 39.6 / 37.4, 600 x 4096 (640) 42.8 / 37.2.
 bool gemm_tiles_pay(const AppendParams& p, const TpaAppendArgs* a) {
   const int64_t tiles = (int64_t)((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
-  return tiles > 512 && tiles < (1 << 28) && p.D % 8 == 0 && aligned16(a->rope_cos) && aligned16(a->rope_sin);
+  return tiles > 512 && tiles < (1 << 28) && p.K < (1 << 22) && p.D % 8 == 0 && aligned16(a->rope_cos) && aligned16(a->rope_sin);
 }
 
 template <int WB, int KS>
@@ -683,10 +684,26 @@ int launch_tiles(const AppendParams& p, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
-// The few-token kernel serves up to 400 of its workgroups of 64 tokens (d_model 4096, us against 64 x 64 tiles: 300 tokens x 720
-// columns, 225 workgroups, 11.5 / 19.3; 300 x 1280, 400, 18.1 / 18.8; 600 x 720, 450, 20.6 / 19.7; 300 x 1600, 500, 24.5 / 19.1;
-// 416 x 1440, 630, 26.2 / 19.4; 1000 x 720, 720, 34.6 / 20.1).
-bool few_tokens(const AppendParams& p) { return (int64_t)((p.N + 15) / 16) * ((p.M + 63) / 64) <= 400; }
+// What a call of the few-token kernel costs is the bytes that a compute unit takes in: with `mb` blocks of 16 tokens per workgroup,
+// rows of W and x of the workgroups that share one, plus as much again as a block for a workgroup's own way.  d_model 4096, us with
+// 16 / 32 / 64 tokens per workgroup: 32 tokens x 1600 columns 8.2 / 10.7 / 11.2, 64 x 1600 11.5 / 10.7 / 14.0, 128 x 1600 20 / 16 /
+// 13.6, 150 x 800 14.5 / 13.5 / 10.7, 150 x 1440 - / 14.6 / 17.8, 64 x 4096 24 / 19 / 15, 16 x 5120 13.0 / 15.3 / 18.4.
+int rows_cost(const AppendParams& p, int mb) {
+  const int64_t per_xcd = (int64_t)(((p.N + 15) / 16 + 7) / 8) * ((p.M + 16 * mb - 1) / (16 * mb));
+  return (int)std::min<int64_t>((per_xcd + 31) / 32 * (32 + 16 * mb), 1 << 20);
+}
+// Blocks of 16 tokens per workgroup if the few-token kernel serves the call, 0 if the tiles do: their time is nearly the same from
+// one tile to 256, and less of it is proportional to d_model than of the few tokens'.  us of this kernel / 64 x 64 tiles: d_model
+// 256, 100 tokens x 1440 columns (cost 128) 6.6 / 6.3, 48 x 1440 (64) 6.0 / 6.3; 512, 150 x 1440 (128) 7.0 / 7.2, 200 x 1440 (192)
+// 9.2 / 7.2; 1024, 150 x 1440 7.8 / 8.8, 200 x 1440 10.4 / 8.9; 2048, 10.1 / 12.0 and 12.6 / 12.1; 4096, 14.6 / 18.8 and 19.1 / 19.0;
+// 8192, 23.5 / 35.0 and 32.6 / 35.2; 4096 with more than 400 workgroups of 64 tokens: 600 x 720 20.6 / 19.7, 300 x 1600 24.5 / 19.1.
+int few_tokens(const AppendParams& p) {
+  if ((int64_t)((p.N + 15) / 16) * ((p.M + 63) / 64) > 400) return 0;
+  int mb = 4;
+  for (int n : {2, 1})
+    if (rows_cost(p, n) < rows_cost(p, mb)) mb = n;
+  return (int64_t)rows_cost(p, mb) * (p.K + 320) <= (int64_t)208 * p.K ? mb : 0;
+}
 
 template <int MB>
 int launch_rows(const AppendParams& p, hipStream_t s) {
@@ -747,23 +764,24 @@ extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
   bool mfma = a->kernel != TPA_KERNEL_GENERIC && a->dtype == TPA_DTYPE_BF16 && a->d_model % kBK == 0 && aligned16(a->x) && aligned16(a->w);
   for (const TpaFactor* f : fs) mfma = mfma && chunk_ok(*f);
   if (a->kernel == TPA_KERNEL_MFMA && !mfma) return TPA_ERR_UNSUPPORTED;
-  if (mfma && few_tokens(p)) {
-    // as many tokens per workgroup as let the call fit the 256 compute units at once (d_model 4096, us with 16 / 32 / 64: 32
-    // tokens x 1600 columns 8.2 / 10.7 / 11.2, 64 x 1600 11.5 / 10.7 / 14.0, 128 x 1600 20 / 16 / 13.6, 64 x 4096 24 / 19 / 15)
-    const int nct = (p.N + 15) / 16;
-    const int rc = nct * ((p.M + 15) / 16) <= 256 ? launch_rows<1>(p, s) : nct * ((p.M + 31) / 32) <= 256 ? launch_rows<2>(p, s) : launch_rows<4>(p, s);
-    if (rc != TPA_OK) return rc;
+  mfma = mfma && p.K < (1 << 24);  // up to 64 rows are read with offsets of 32 bits
+  const int few = mfma ? few_tokens(p) : 0;
+  if (few) {
+    if (const int rc = few == 1 ? launch_rows<1>(p, s) : few == 2 ? launch_rows<2>(p, s) : launch_rows<4>(p, s); rc != TPA_OK) return rc;
   } else if (mfma && gemm_tiles_pay(p, a)) {
-    // With t tiles of 128 x 128 these take 0.155 t + 25 us (from 512 on; d_model 4096) and rounds of 256 tiles of 256 x 256 122 us each.
-    // Measured, 128 / 256: 6600 tokens x 1440 columns (624) 133 / 128, 2048 x 5120 (640) 139 / 129, 6600 x 1600 (676) 137 / 124,
-    // 3264 x 4608 (936) 153 / 135, 3264 x 5120 (1040) 184 / 237, 4352 x 4608 (1224) 214 / 240, 6600 x 4096 (1664) 277 / 254.
+    // What counts is the most tiles that a compute unit gets.  One of 256 x 256 takes 14 us and 23 per 1024 of d_model, four of
+    // 128 x 128 where a compute unit has as many take 9 and 35: the large ones are ahead where they save a quarter of
+    // the small ones, from d_model 1024 on, or the third of three small ones, above 2048.  us, 128 / 256:
+    //   d_model 512: 2600 tokens x 5120 columns (4 and 1 tiles) 31.4 / 32.8, 8192 x 5120 (10, 3) 81 / 89, 6600 x 1440 (3, 1) 25.5 / 31.6
+    //   1024: 47.7 / 45.0, 134 / 126, 38.3 / 43.9; 2048: 81 / 70, 233 / 206, 64 / 65; 4096: 149 / 121, 439 / 375, 116 / 109
+    //   three for two, 4352 x 5120 (6, 2): 2048 133 / 132, 4096 249 / 232, 8192 483 / 434; five for two, 3264 x 5120: 4096 190 / 229
     const int64_t small = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128), large = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
-    // Two groups of waves need an even number of k steps and one round of tiles: with their buffers a compute unit holds one
-    // tile, with those of one group two.  d_model 4096, us with one / two groups: 2048 x 1600 (208) 56 / 40, 3178 x 1120 (225,
-    // then 36 on one XCD) 69 / 75.
-    const int rc = small + 180 > (large + 255) / 256 * 790 ? launch_gemm<4, 1>(p, s)
-                   : p.K % (2 * kGK) == 0 && small <= 256  ? launch_gemm<2, 2>(p, s)
-                                                           : launch_gemm<2, 1>(p, s);
+    const int64_t smalls = (small + 255) / 256, larges = (large + 255) / 256;
+    // Two groups of waves need an even number of k steps and one tile per compute unit: with their buffers it holds one, with
+    // those of one group two.  us with one / two groups: 2048 x 1600 (208 tiles), d_model 4096 56 / 40, 2048 24 / 23, but 512 12.8 / 13.4.
+    const int rc = (smalls > 3 * larges ? p.K >= 1024 : smalls == 3 * larges && p.K > 2048) ? launch_gemm<4, 1>(p, s)
+                   : p.K % (2 * kGK) == 0 && smalls == 1                                    ? launch_gemm<2, 2>(p, s)
+                                                                                            : launch_gemm<2, 1>(p, s);
     if (rc != TPA_OK) return rc;
   } else if (mfma) {
     const int64_t ntm = (p.M + kBM - 1) / kBM, tiles = ntm * ((p.N + kBN - 1) / kBN);

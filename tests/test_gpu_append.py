@@ -37,15 +37,15 @@ def make_layer(seed, b, n, dm, h, d, rq, rk, dtype, gpu):
 @pytest.mark.parametrize(
     "b,n,dm,h,d,rq,rk",
     [
-        (3, 5, 256, 16, 64, 6, 2),     # 15 tokens: the decode-step kernel (k split over the waves), one k step per wave
+        (3, 5, 256, 16, 64, 6, 2),     # 15 tokens: the kernel for few tokens, four chunks of k: four of its waves have none
         (2, 70, 128, 8, 128, 3, 4),    # 140 tokens: 64 x 64 tiles
-        (1, 1, 64, 32, 128, 6, 2),     # d_model too short for the k split: tiles
-        (64, 1, 1024, 32, 128, 6, 2),  # a decode step of 64 sequences: all four blocks of 16 tokens
+        (1, 1, 64, 32, 128, 6, 2),     # one chunk of k: tiles
+        (64, 1, 1024, 32, 128, 6, 2),  # a decode step of 64 sequences: two blocks of 32 tokens
         (7, 3, 512, 8, 64, 2, 1),      # 21 tokens: the second block of 16 is ragged
         (5, 2, 256, 8, 64, 1, 1),      # 216 output columns: the last workgroup owns half a block of columns
-        (8, 2, 2048, 16, 128, 2, 2),   # with a workspace: 8 slabs of k, one k step per wave
-        (4, 9, 4096, 8, 64, 3, 1),     # 8 slabs, two k steps per wave; 200 columns: the last workgroup owns 8 of its 64
-        (2, 3, 1536, 8, 64, 2, 2),     # 2 slabs, three k steps per wave
+        (8, 2, 2048, 16, 128, 2, 2),   # 32 chunks of k, four per wave
+        (4, 9, 4096, 8, 64, 3, 1),     # 64 chunks; 200 columns: the last workgroup owns 8 of its 16
+        (2, 3, 1536, 8, 64, 2, 2),     # 24 chunks, three per wave
     ],
 )
 @pytest.mark.parametrize("use_workspace", [False, True])
@@ -160,10 +160,10 @@ def test_append_contiguous_and_paged_caches_hold_the_same_rows(gpu):
 @pytest.mark.parametrize(
     "b,n,dm,h,d,rq,rk",
     [
-        (3, 2731, 128, 32, 128, 6, 2),  # 8193 tokens: the last token tile holds one; 1600 columns: the last column tile a quarter
-        (2, 4900, 64, 32, 96, 6, 2),    # 1280 columns = five whole column tiles; one k step
+        (3, 2731, 128, 32, 128, 6, 2),  # 8193 tokens: the last token tile holds one; 1600 columns: the last column tile half
+        (2, 4900, 64, 32, 96, 6, 2),    # 1280 columns = ten whole column tiles; one k step
         (5, 2000, 192, 16, 128, 7, 1),  # 1296 columns: rank rows and factors change inside a wave's 64-column pieces
-        (2, 1025, 128, 32, 128, 6, 2),  # 2050 tokens: too few for the 256 x 256 tiles, enough for the 128 x 128 ones
+        (2, 1025, 128, 32, 128, 6, 2),  # 2050 tokens: the last token tile holds two
         (3, 700, 64, 16, 128, 6, 2),    # 128 x 128 tiles: 1440 columns (the last tile a quarter), one k step
     ],
 )
