@@ -49,7 +49,7 @@ struct BwdParams {
   int coff;  // with causal: row i sees keys <= i + coff
   int nblk;    // row blocks (dq) or key blocks (dkv) per (batch, head)
   int npairs;  // nblk * B
-  int pair_group;  // (batch, head) pairs of an XCD whose blocks run side by side
+  int pair_groups;  // groups of (batch, head) pairs of an XCD whose blocks run side by side
 };
 
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -132,15 +132,11 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
   // workgroups can share, so an XCD owns whole (batch, head) pairs and runs their blocks heaviest first,
   // the same block of all its pairs side by side: neighbouring blocks of a pair walk the same tiles at
   // about the same time and find them in that XCD's L2.
-  // Pairs are taken in groups of `pair_group` (launch_dq): with every pair of an XCD side by side and many pairs the
+  // Pairs are taken in groups (pair_groups_of): with every pair of an XCD side by side and many pairs the
   // resident workgroups would all belong to different pairs and share nothing.
-  const int xcd = id & 7, slot = id >> 3;
-  const int per_xcd = (p.B * p.H + 7) / 8, per_group = p.pair_group * p.nblk;
-  const int grp = slot / per_group, rem = slot - grp * per_group;
-  const int pair_local = grp * p.pair_group + rem % p.pair_group;
-  const int bh = pair_local * 8 + xcd;
-  if (pair_local >= per_xcd || bh >= p.B * p.H) return;
-  const int qblk = p.nblk - 1 - rem / p.pair_group, b = bh / p.H, h = bh % p.H;  // heaviest causal blocks first
+  int bh, rank;
+  if (!pair_in_group(id, p.B * p.H, p.pair_groups, p.nblk, bh, rank)) return;
+  const int qblk = p.nblk - 1 - rank, b = bh / p.H, h = bh % p.H;  // heaviest causal blocks first
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int lp = l & 15, dhalf = (l >> 4) & 1;
   const int q0 = qblk * kBQ, wrow0 = q0 + kWQ * w;
@@ -340,13 +336,9 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
   u32x4* const lds_vf = reinterpret_cast<u32x4*>(lds_seg + 2 * kTile);  // [NW][NB][NKS][64 lanes]: V of the wave's keys as B operands
 
   // (batch, head) pairs per XCD, blocks heaviest first: see dq_block
-  const int xcd = id & 7, slot = id >> 3;
-  const int per_xcd = (p.B * p.H + 7) / 8, per_group = p.pair_group * p.nblk;
-  const int grp = slot / per_group, rem = slot - grp * per_group;
-  const int pair_local = grp * p.pair_group + rem % p.pair_group;
-  const int bh = pair_local * 8 + xcd;
-  if (pair_local >= per_xcd || bh >= p.B * p.H) return;
-  const int kblk = rem / p.pair_group, b = bh / p.H, h = bh % p.H;  // under the causal mask the first key blocks are the heaviest
+  int bh, rank;
+  if (!pair_in_group(id, p.B * p.H, p.pair_groups, p.nblk, bh, rank)) return;
+  const int kblk = rank, b = bh / p.H, h = bh % p.H;  // under the causal mask the first key blocks are the heaviest
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int lp = l & 15, dhalf = (l >> 4) & 1;
   const int k0 = kblk * kBK, wkey0 = k0 + kWK * w;
@@ -583,14 +575,12 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
 // kernels wait for LDS more than for memory: with fewer pairs side by side they lose 1 % at B = 4, T = 4096, H = 16),
 // but not all pairs of the XCD where they are many (the workgroups resident together would all belong to different
 // pairs and share nothing: B = 16, T = 1024, H = 16 takes 0.574 ms with 16 of its 32 pairs side by side, 0.620 with all;
-// B = 8, T = 2048, H = 64, D = 64 not causal 2.25 against 2.44 ms).  Groups of one size, as in the forward: a short last
-// one leaves compute units idle (72 pairs, whole backward, us, short last group / equal groups: T = 2040, D = 64 causal
-// 292 / 249, D = 128 513 / 450, T = 4000 827 / 688 and 1478 / 1260; 192 pairs, T = 1500 368 / 350)
-inline int pair_group_of(int per_xcd, int nblk) {
-  int g = (64 + nblk - 1) / nblk;
-  if (g < 8) g = 8;
-  const int n = per_xcd / g;
-  return n < 1 ? per_xcd : (per_xcd + n - 1) / n;
+// B = 8, T = 2048, H = 64, D = 64 not causal 2.25 against 2.44 ms).  Groups of one size, give or take a pair, as in the
+// forward: a short last one leaves compute units idle (forward and backward, us, short last group / these, causal: 72 pairs, T =
+// 2048, D = 64 384 / 318, D = 128 669 / 575; 104, T = 4096, D = 128 2724 / 2555; 136, T = 1024, D = 64 301 / 240)
+inline int pair_groups_of(int npairs, int nblk) {
+  const int size = (64 + nblk - 1) / nblk;
+  return pair_groups(npairs, size < 8 ? 8 : size);
 }
 
 // Both in one launch: the dK/dV workgroups first (four products per tile against three), then the dQ ones, so that the
@@ -607,9 +597,8 @@ __global__ __launch_bounds__(NW * 64) void bwd_dq_dkv_kernel(BwdPair p) {
 inline int64_t decompose(BwdParams& p, int rows, int block) {
   p.nblk = (rows + block - 1) / block;
   p.npairs = p.nblk * p.B;
-  const int per_xcd = (p.B * p.H + 7) / 8;
-  p.pair_group = pair_group_of(per_xcd, p.nblk);
-  return (int64_t)((per_xcd + p.pair_group - 1) / p.pair_group) * p.pair_group * p.nblk * 8;
+  p.pair_groups = pair_groups_of(p.B * p.H, p.nblk);
+  return pair_group_workgroups(p.B * p.H, p.nblk);
 }
 
 template <int D, int NW, int NB, bool SEG>

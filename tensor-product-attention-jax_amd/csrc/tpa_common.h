@@ -207,6 +207,27 @@ inline int head_groups(int64_t npairs, int H) {
 }
 inline int64_t workgroups_of(int64_t npairs, int H, int groups) { return (npairs * groups + 7) / 8 * 8 * (H / groups); }
 
+// Workgroup id -> (batch, head) pair and block rank for the kernels over dense arrays, which belong to one pair: an XCD owns whole
+// pairs and runs them in `groups` groups, whose sizes differ by one at most; inside a group the blocks go in order of their
+// rank, the same block of all its pairs side by side.  False: the XCD has a pair less than the others.
+__device__ __forceinline__ bool pair_in_group(int id, int npairs, int groups, int nblk, int& pair, int& rank) {
+  const int xcd = id & 7, slot = id >> 3, per_xcd = (npairs + 7) / 8;
+  const int small = per_xcd / groups, larger = per_xcd - small * groups;  // pairs of a group; groups that have one more
+  const int first_small = larger * (small + 1);
+  const bool large = slot < first_small * nblk;
+  const int size = large ? small + 1 : small, at = large ? slot : slot - first_small * nblk;
+  const int grp = at / (size * nblk), rem = at - grp * size * nblk;
+  rank = rem / size;
+  pair = ((large ? 0 : first_small) + grp * size + rem - rank * size) * 8 + xcd;
+  return pair < npairs;
+}
+inline int64_t pair_group_workgroups(int npairs, int nblk) { return (int64_t)((npairs + 7) / 8) * nblk * 8; }
+// as many groups as come nearest to `size` pairs in each
+inline int pair_groups(int npairs, int size) {
+  const int per_xcd = (npairs + 7) / 8, n = (2 * per_xcd + size - 1) / (2 * size);
+  return n < 1 ? 1 : n;
+}
+
 // Causal offset of a forward call as the kernels take it: row i sees keys <= i + offset.  Offsets
 // of lk and more mask nothing and offsets of -lq and less mask everything, so the value is clamped
 // to that range (keeps the kernels' index arithmetic far from overflow); 0 without the causal mask.

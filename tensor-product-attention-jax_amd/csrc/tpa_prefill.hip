@@ -54,7 +54,7 @@ struct PrefillParams {
   int nqb;     // query blocks per (batch, head)
   int npairs;  // nqb * B
   int q_scaled;   // dense loader only: 1 = q already holds sm_scale * log2(e) * Q (it was reconstructed with that factor)
-  int pair_group; // dense loader only: (batch, head) pairs of an XCD whose query blocks run side by side (see the kernel)
+  int pair_groups; // dense loader only: groups of (batch, head) pairs of an XCD whose query blocks run side by side (see the kernel)
   int head_groups; // factor loaders only: see pair_of_workgroup
   // key ranges per query block (1: none).  nqb then counts (query block, range) and a workgroup's result goes, not
   // normalised, to part_o [S][B, lq, H, D] with the reference (log2 domain; -inf: no key seen) and the sum in part_ml
@@ -128,9 +128,9 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // scalars out of the argument block (never take the address of the block itself)
   struct Fac { const uint16_t* ptr; int64_t stride_b; int stride_l, stride_r; };
   auto fac = [](const TpaFactor& f) { return Fac{static_cast<const uint16_t*>(f.ptr), f.stride_b, (int)f.stride_l, (int)f.stride_r}; };
-  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; uint16_t* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs, q_scaled, pair_group, head_groups, S; } const p = {
+  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; uint16_t* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs, q_scaled, pair_groups, head_groups, S; } const p = {
       fac(pp.qa), fac(pp.qb), fac(pp.ka), fac(pp.kb), fac(pp.va), fac(pp.vb), pp.qseg, pp.kvseg, pp.kvlen, pp.o, pp.lse, pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk,
-      pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.q_scaled, pp.pair_group, pp.head_groups, SPLIT ? pp.S : 1};
+      pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.q_scaled, pp.pair_groups, pp.head_groups, SPLIT ? pp.S : 1};
 
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   auto lds_k = [&](int buf) __attribute__((always_inline)) { return smem + L::k_off(buf); };    // [kTK][KS]
@@ -144,19 +144,14 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   if constexpr (LOADER == LOAD_DENSE) {
     // Dense K and V belong to one (batch, head): what workgroups can share is the K/V stream of
     // their head.  An XCD therefore owns whole (batch, head) pairs and runs them in groups of
-    // `pair_group` pairs: the query blocks of a group heaviest first, the same block of the group's
+    // pairs: the query blocks of a group heaviest first, the same block of the group's
     // pairs side by side.  The 32 workgroups that are resident together on an XCD are then
     // neighbouring query blocks of a few pairs, which walk the same tiles at about the same time and
     // find them in that XCD's L2 (with every pair of the XCD in one group and many pairs, the resident
     // workgroups would all belong to different pairs and every tile would come from memory).
-    const int xcd = id & 7, slot = id >> 3;
-    const int per_xcd = (p.B * p.H + 7) / 8;
-    const int per_group = p.pair_group * p.nqb;
-    const int grp = slot / per_group, rem = slot - grp * per_group;
-    const int pair_local = grp * p.pair_group + rem % p.pair_group;
-    const int bh = pair_local * 8 + xcd;
-    if (pair_local >= per_xcd || bh >= p.B * p.H) return;
-    qblk = p.nqb - 1 - rem / p.pair_group;
+    int bh, rank;
+    if (!pair_in_group(id, p.B * p.H, p.pair_groups, p.nqb, bh, rank)) return;
+    qblk = p.nqb - 1 - rank;
     b = bh / p.H;
     h = bh % p.H;
   } else {
@@ -1087,14 +1082,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* part_o,
 // attention: B = 8, T = 2048, H = 64, D = 64 (64 pairs per XCD, 8 blocks each) 0.654 ms with all pairs side by
 // side, 0.601 - 0.603 with 1 to 8; B = 4, T = 4096, H = 16 (8 pairs, 16 blocks) 0.250 with 4 or 8, 0.256 with 2,
 // 0.291 with 1 (the last group's heavy blocks start late); T = 32768, H = 32 (4 pairs, 128 blocks) 7.04 with 1, 7.21 with 4.
-// The groups are of one size, give or take a pair: a short last one would start its heavy blocks late and leave compute
-// units idle (with the reconstruction, us, short last group / equal groups, causal, 72 pairs: T = 2040, D = 64 89 / 70, D =
-// 128 136 / 109, T = 4000 238 / 200 and 377 / 322; 48 pairs, T = 4000, not causal 268 / 222; 192 pairs, T = 1500 118 / 104).
-inline int dense_pair_group(int per_xcd, int nqb) {
-  const int g = (64 + nqb - 1) / nqb;
-  const int n = per_xcd / (g < 1 ? 1 : g);
-  return n < 1 ? per_xcd : (per_xcd + n - 1) / n;
-}
+// The sizes of an XCD's groups differ by one at most: a short last one would start its heavy blocks late and leave compute
+// units idle.  With the reconstruction, us, a short last group / these, causal: 72 pairs, T = 2048, D = 64 93 / 73, D = 128 140 /
+// 112; 80, T = 2048 94 / 78; 136, T = 1024 68 / 57; not causal 40, T = 4096, D = 128 429 / 343, 72 677 / 588, but 104, T = 2048 (of
+// eight and five; seven and six) 248 / 259.  The number of groups is the nearest: with 31 pairs per XCD of 4 blocks, causal, 88 us
+// in one group of all, 86 in two.
+inline int dense_pair_groups(int npairs, int nqb) { return pair_groups(npairs, (64 + nqb - 1) / nqb); }
 
 template <int D, int LOADER, bool SEG = false, bool SPLIT = false>
 int launch_prefill(const PrefillParams& p, hipStream_t stream) {
@@ -1108,9 +1101,8 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
   PrefillParams q = p;
   int64_t n;
   if (LOADER == LOAD_DENSE) {
-    const int per_xcd = (p.B * p.H + 7) / 8;
-    q.pair_group = dense_pair_group(per_xcd, p.nqb);
-    n = (int64_t)((per_xcd + q.pair_group - 1) / q.pair_group) * q.pair_group * p.nqb * 8;
+    q.pair_groups = dense_pair_groups(p.B * p.H, p.nqb);
+    n = pair_group_workgroups(p.B * p.H, p.nqb);
   } else {
     q.head_groups = head_groups(p.npairs, p.H);
     n = workgroups_of(p.npairs, p.H, q.head_groups);

@@ -1,10 +1,10 @@
 """Launches in which an XCD owns many (batch, head) pairs and runs them in groups.
 
 The dense-loader prefill kernel and the matrix-core backward kernels deal whole (batch, head) pairs
-to the eight XCDs and let an XCD run its pairs a group at a time; the grid is rounded up to whole
-groups, so the last group of an XCD can be short and an XCD can own fewer pairs than its neighbours.
+to the eight XCDs and let an XCD run its pairs a group at a time; the sizes of its groups can differ
+by one and an XCD can own fewer pairs than its neighbours.
 These shapes have such remainders: pair counts that are no multiple of 8, pairs per XCD that are no
-multiple of the group size.  What a pair receives must not depend on the other pairs of the launch:
+multiple of the number of groups.  What a pair receives must not depend on the other pairs of the launch:
 a call on a subset of the heads gives the same bits, and sampled rows meet the oracle.
 """
 
@@ -27,8 +27,7 @@ def _randn(gpu, seed, *shape):
 
 
 def test_prefill_sampled_rows_with_a_short_last_group(gpu):
-    """B=3, H=40 (120 pairs, 15 per XCD), 1536 rows = 6 query blocks: groups of 11 pairs, the second one
-    holds 4; sampled rows of every batch entry, all heads, against the oracle within the per-row bounds
+    """B=3, H=40 (120 pairs, 15 per XCD), 1536 rows = 6 query blocks: 15 is nearer to one group of 11 than to two; sampled rows of every batch entry, all heads, against the oracle within the per-row bounds
     of the kernels' rounding points (tests/error_model.py)."""
     b, t, h, d, scale = 3, 1536, 40, 64, 64**-0.5
     rows = np.array([0, 255, 256, 700, 1279, 1535])
