@@ -67,26 +67,28 @@ struct TileRegs {
   // returns whether a value of this thread's does not split
   template <bool FP32>
   __device__ __forceinline__ bool store(uint16_t* dst, std::integral_constant<bool, FP32>) const {
-    bool bad = false;
+    Magnitudes seen;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
       const int chunk = c * NT + threadIdx.x, t = chunk / CPR, cc = chunk % CPR;
       uint16_t* const at = dst + t * BwdLds<D>::RS + 4 * cc;
       const f32x4& x = r[c];
-      const Pair3 a = FP32 ? split_pair_any(x[0], x[1]) : split_pair(x[0], x[1]), b = FP32 ? split_pair_any(x[2], x[3]) : split_pair(x[2], x[3]);
-      if constexpr (!FP32) bad |= irregular(largest(largest(0.f, x[0], x[1]), x[2], x[3]));
+      const Pair3 a = FP32 ? halves_of_pair(x[0], x[1]) : split_pair(x[0], x[1]), b = FP32 ? halves_of_pair(x[2], x[3]) : split_pair(x[2], x[3]);
       *reinterpret_cast<u32x2*>(at) = u32x2{a.h, b.h};
       *reinterpret_cast<u32x2*>(at + BwdLds<D>::kPlane) = u32x2{a.m, b.m};
-      *reinterpret_cast<u32x2*>(at + 2 * BwdLds<D>::kPlane) = u32x2{a.l, b.l};
+      if constexpr (!FP32) {
+        *reinterpret_cast<u32x2*>(at + 2 * BwdLds<D>::kPlane) = u32x2{a.l, b.l};
+        seen.add(x);
+      }
     }
-    return bad;
+    return seen.irregular();
   }
 };
 
 // The wave's own row, scaled and split (B operand of the row-wise contractions): lane (i, g) holds X[row][16 ks + 8 g + 0..7]
-template <int D>
-__device__ __forceinline__ bool load_own_row(const float* rowp, int g, float scale, bool scrub_nan, Split3 (&out)[D / 16]) {
-  float top = 0.f;
+template <int D, bool FP32>
+__device__ __forceinline__ bool load_own_row(const float* rowp, int g, float scale, bool scrub_nan, Split3 (&out)[D / 16], std::integral_constant<bool, FP32>) {
+  Magnitudes seen;
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks) {
     float y[8];
@@ -97,10 +99,10 @@ __device__ __forceinline__ bool load_own_row(const float* rowp, int g, float sca
       for (int e = 0; e < 4; ++e) y[4 * u + e] = (scrub_nan && x[e] != x[e] ? 0.f : x[e]) * scale;
     }
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) top = largest(top, y[e], y[e + 1]);
-    out[ks] = split8<true>(y);
+    for (int e = 0; e < 8; e += 2) seen.add(y[e], y[e + 1]);
+    out[ks] = split8<FP32>(y);
   }
-  return irregular(top);
+  return seen.irregular();
 }
 
 // The same as floats, split anew for every tile, for a wave whose registers do not hold both operands' parts.
@@ -108,15 +110,15 @@ template <int D>
 struct OwnFloats {
   float x[D / 2];
   __device__ __forceinline__ bool load(const float* rowp, int g, float scale) {
-    float top = 0.f;
+    Magnitudes seen;
 #pragma unroll
     for (int j = 0; j < D / 8; ++j) {
       const f32x4 y = *reinterpret_cast<const f32x4*>(rowp + 16 * (j >> 1) + 8 * g + 4 * (j & 1)) * scale;
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[4 * j + e] = y[e];
-      top = largest(largest(top, y[0], y[1]), y[2], y[3]);
+      seen.add(y);
     }
-    return irregular(top);
+    return seen.irregular();
   }
 };
 
@@ -238,8 +240,12 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dq_kernel(BwdF32Params p) {
   const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + p.coff + 31 - kbeg, 0) / kTile) : ntiles - 1;
 
   Split3 qf[NKS], gf[NKS];
-  bool bad = load_own_row<D>(p.q + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, p.sm_scale * kLog2e, false, qf);
-  bad |= load_own_row<D>(p.d_o + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, 1.f, true, gf);
+  bool bad = false;
+  auto load_own = [&](auto fp32, const auto& p, int row) __attribute__((always_inline)) {
+    const int64_t at = ((int64_t)b * p.lq + row) * p.H * D + (int64_t)h * D;
+    bad |= load_own_row<D>(p.q + at, g, p.sm_scale * kLog2e, false, qf, fp32);
+    bad |= load_own_row<D>(p.d_o + at, g, 1.f, true, gf, fp32);
+  };
   const float lse = p.lse[((int64_t)b * p.H + h) * p.lq + qrow_ld];
   // a row without a visible key (lse = -inf) has no gradient: +inf makes every p of the row zero
   const float lse2 = (qrow < p.lq && lse > -INFINITY) ? lse * kLog2e : INFINITY;
@@ -296,6 +302,8 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dq_kernel(BwdF32Params p) {
 
   auto walk = [&](auto fp32) __attribute__((always_inline)) {
     clear<D>(dq);
+    if constexpr (decltype(fp32)::value) load_own(fp32, *arguments_again<BwdF32Params>(), again(qrow_ld));
+    else load_own(fp32, p, qrow_ld);
     issue(0);
     commit(fp32, 0);
     __syncthreads();
@@ -341,17 +349,18 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dkv_kernel(BwdF32Params p) {
   }
   const int wave_first_tile = p.causal ? max(wkey0 - p.coff, 0) / kTile : 0;
 
-  const float* const krow = p.k + ((int64_t)b * p.lk + key_ld) * hd + (int64_t)h * D;
-  const float* const vrow = p.v + ((int64_t)b * p.lk + key_ld) * hd + (int64_t)h * D;
   std::conditional_t<D == 128, OwnFloats<D>, Split3[NKS]> kf, vf;
-  bool bad;
-  if constexpr (D == 128) {  // with both accumulators the parts of both operands do not fit 512 registers
-    bad = kf.load(krow, g, p.sm_scale * kLog2e);
-    bad |= vf.load(vrow, g, 1.f);
-  } else {
-    bad = load_own_row<D>(krow, g, p.sm_scale * kLog2e, false, kf);
-    bad |= load_own_row<D>(vrow, g, 1.f, false, vf);
-  }
+  bool bad = false;
+  auto load_own = [&](auto fp32, const auto& p, int row) __attribute__((always_inline)) {
+    const int64_t at = ((int64_t)b * p.lk + row) * p.H * D + (int64_t)h * D;
+    if constexpr (D == 128) {  // with both accumulators the parts of both operands do not fit 512 registers
+      bad |= kf.load(p.k + at, g, p.sm_scale * kLog2e);
+      bad |= vf.load(p.v + at, g, 1.f);
+    } else {
+      bad |= load_own_row<D>(p.k + at, g, p.sm_scale * kLog2e, false, kf, fp32);
+      bad |= load_own_row<D>(p.v + at, g, 1.f, false, vf, fp32);
+    }
+  };
   int32_t kseg = 0;
   if constexpr (SEG) kseg = p.kvseg[(int64_t)b * p.lk + key_ld];
 
@@ -417,6 +426,8 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dkv_kernel(BwdF32Params p) {
   auto walk = [&](auto fp32) __attribute__((always_inline)) {
     clear<D>(dk);
     clear<D>(dv);
+    if constexpr (decltype(fp32)::value) load_own(fp32, *arguments_again<BwdF32Params>(), again(key_ld));
+    else load_own(fp32, p, key_ld);
     if (first_tile < ntiles) {
       issue(first_tile);
       commit(fp32, first_tile);
@@ -476,7 +487,7 @@ struct WaveTile {
   }
   // returns whether a value of this lane's does not split
   static __device__ __forceinline__ bool store(const Regs& r, float* dst, int l, bool scrub_nan) {
-    float top = 0.f;
+    Magnitudes seen;
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
       f32x4 x = r[q];
@@ -484,30 +495,30 @@ struct WaveTile {
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = x[e] == x[e] ? x[e] : 0.f;
       }
-      top = largest(largest(top, x[0], x[1]), x[2], x[3]);
+      seen.add(x);
       *reinterpret_cast<f32x4*>(dst + (q * RPI + l / CPR) * SplitLds<D>::RS + 4 * (l % CPR)) = x;
     }
-    return irregular(top);
+    return seen.irregular();
   }
 };
 
 // The 32 own rows of one operand, scaled, split and parked for all waves; returns whether a value does not split
-template <int D>
-__device__ __forceinline__ bool park_own(const float* base, int64_t hd, int row0, int nrows, float scale, uint16_t* lds, int tid) {
+template <int D, bool FP32>
+__device__ __forceinline__ bool park_own(const float* base, int64_t hd, int row0, int nrows, float scale, uint16_t* lds, int tid, std::integral_constant<bool, FP32>) {
   typedef SplitLds<D> L;
   constexpr int CPR = D / 4;
-  float top = 0.f;
+  Magnitudes seen;
   for (int idx = tid; idx < 32 * CPR; idx += L::NW * 64) {
     const int row = idx / CPR, cc = idx % CPR;
     const f32x4 x = *reinterpret_cast<const f32x4*>(base + (int64_t)min(row0 + row, nrows - 1) * hd + 4 * cc) * scale;
-    top = largest(largest(top, x[0], x[1]), x[2], x[3]);
-    const Pair3 a = split_pair_any(x[0], x[1]), b = split_pair_any(x[2], x[3]);
+    seen.add(x);
+    const Pair3 a = FP32 ? halves_of_pair(x[0], x[1]) : split_pair(x[0], x[1]), b = FP32 ? halves_of_pair(x[2], x[3]) : split_pair(x[2], x[3]);
     uint16_t* const at = lds + row * L::OS + 4 * cc;
     *reinterpret_cast<u32x2*>(at) = u32x2{a.h, b.h};
     *reinterpret_cast<u32x2*>(at + L::kOwnPlane) = u32x2{a.m, b.m};
     *reinterpret_cast<u32x2*>(at + 2 * L::kOwnPlane) = u32x2{a.l, b.l};
   }
-  return irregular(top);
+  return seen.irregular();
 }
 
 // acc = tile rows . own row over d; `own(ks)` hands out the own row's operand of a step
@@ -529,7 +540,7 @@ __device__ __forceinline__ f32x16 rows_dot32(const float* tile, int i, int g, Ow
     }
     if constexpr (FP32) {
       Split3 b = o;
-      asm volatile("" : "+v"(b.h), "+v"(b.m), "+v"(b.l));  // not summed ahead of the loop (tpa_split3.h)
+      asm volatile("" : "+v"(b.h), "+v"(b.m));  // not joined ahead of the loop (tpa_split3.h)
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], join(b, e), acc, 0, 0, 0);
     } else {
@@ -645,9 +656,13 @@ __device__ __forceinline__ void dq_split(const BwdF32Params& p, int id) {
 
   uint16_t* const lds_q = reinterpret_cast<uint16_t*>(smem_bwd_f32 + NW * L::kPerWave);
   Split3 gf[NKS];
-  bool bad = park_own<D>(p.q + (int64_t)b * p.lq * hd + (int64_t)h * D, hd, q0, p.lq, p.sm_scale * kLog2e, lds_q, tid);
-  bad |= load_own_row<D>(p.d_o + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, 1.f, true, gf);
-  __syncthreads();
+  bool bad = false;
+  auto load_own = [&](auto fp32) __attribute__((always_inline)) {
+    bad |= park_own<D>(p.q + (int64_t)b * p.lq * hd + (int64_t)h * D, hd, q0, p.lq, p.sm_scale * kLog2e, lds_q, tid, fp32);
+    bad |= load_own_row<D>(p.d_o + ((int64_t)b * p.lq + qrow_ld) * hd + (int64_t)h * D, g, 1.f, true, gf, fp32);
+    __syncthreads();
+  };
+  load_own(SplitProducts{});
   int own_at = i * L::OS + 8 * g;
   auto q_operand = [&](int ks) __attribute__((always_inline)) -> Split3 {
     const uint16_t* const at = lds_q + own_at + 16 * ks;
@@ -706,6 +721,7 @@ __device__ __forceinline__ void dq_split(const BwdF32Params& p, int id) {
   walk(SplitProducts{});
   if (__builtin_expect(__syncthreads_or(bad), 0)) {
     request_first();
+    load_own(Fp32Products{});
     walk(Fp32Products{});
     __syncthreads();
   }
@@ -769,9 +785,12 @@ __device__ __forceinline__ void dkv_split(const BwdF32Params& p, int id) {
 
   uint16_t* const lds_own = reinterpret_cast<uint16_t*>(smem_bwd_f32 + NW * L::kPerWave);
   Split3 vf[NKS];
-  bad |= park_own<D>(p.k + (int64_t)b * p.lk * hd + (int64_t)h * D, hd, k0, p.lk, p.sm_scale * kLog2e, lds_own, tid);
-  bad |= load_own_row<D>(p.v + ((int64_t)b * p.lk + key_ld) * hd + (int64_t)h * D, g, 1.f, false, vf);
-  __syncthreads();
+  auto load_own = [&](auto fp32) __attribute__((always_inline)) {
+    bad |= park_own<D>(p.k + (int64_t)b * p.lk * hd + (int64_t)h * D, hd, k0, p.lk, p.sm_scale * kLog2e, lds_own, tid, fp32);
+    bad |= load_own_row<D>(p.v + ((int64_t)b * p.lk + key_ld) * hd + (int64_t)h * D, g, 1.f, false, vf, fp32);
+    __syncthreads();
+  };
+  load_own(SplitProducts{});
   int own_at = i * L::OS + 8 * g;
   auto k_operand = [&](int ks) __attribute__((always_inline)) -> Split3 {
     const uint16_t* const at = lds_own + own_at + 16 * ks;
@@ -824,6 +843,7 @@ __device__ __forceinline__ void dkv_split(const BwdF32Params& p, int id) {
   walk(SplitProducts{});
   if (__builtin_expect(__syncthreads_or(bad), 0)) {
     request_first();
+    load_own(Fp32Products{});
     walk(Fp32Products{});
     __syncthreads();
   }

@@ -106,10 +106,11 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   const int ntiles = (kend - kbeg + kTK - 1) / kTK;
   const int wave_last_tile = p.causal ? min(ntiles - 1, max(wrow0 + coff + 31 - kbeg, 0) / kTK) : ntiles - 1;
 
-  // ---- Q (B operand of S^T = K Q^T), scaled and split: lane (i, g) holds Q[qrow][16 ks + 8 g + 0..7]
+  // ---- Q (B operand of S^T = K Q^T), scaled and split: lane (i, g) holds Q[qrow][16 ks + 8 g + 0..7].  `fp32` is a compile-time
+  // flag here and below: the walk over the tiles that uses the fp32 instruction
   Split3 qf[NKS];
   bool bad = false;  // this thread has met values that do not split
-  {
+  auto load_q = [&](auto fp32) __attribute__((always_inline)) {
     const float* const qb = p.qb.ptr + b * p.qb.stride_b + (int64_t)qrow_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 8 * g;
     const float* const qa = dense ? nullptr : p.qa.ptr + b * p.qa.stride_b + (int64_t)qrow_ld * p.qa.stride_l + h;
     const float scale = p.sm_scale * kLog2e / (float)p.rq;
@@ -137,12 +138,12 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
         for (int e = 0; e < 8; ++e) q[ks][e] *= scale;
 #pragma unroll
         for (int e = 0; e < 8; e += 2) top = largest(top, q[ks][e], q[ks][e + 1]);
-        qf[k0 + ks] = split8<true>(q[ks]);
+        qf[k0 + ks] = split8<decltype(fp32)::value>(q[ks]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    bad = irregular(top);
-  }
+    bad |= !(top < kLogitOperand);
+  };
 
   // ---- tile rebuild: thread -> CH chunks of 4 floats per matrix
   const float* const kb_b = p.kb.ptr + b * p.kb.stride_b + (dense ? (int64_t)h * D : 0);
@@ -150,24 +151,18 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   const float* const ka_b = dense ? nullptr : p.ka.ptr + b * p.ka.stride_b + h;
   const float* const va_b = dense ? nullptr : p.va.ptr + b * p.va.stride_b + h;
   const float inv_r = 1.f / (float)p.rk;
-  // `fp32` is a compile-time flag here and below: the walk over the tiles that uses the fp32 instruction
   auto stage = [&](auto fp32, uint16_t* at, int plane, const f32x4& x) __attribute__((always_inline)) {
-    Pair3 a, c;
-    if constexpr (decltype(fp32)::value) {
-      a = split_pair_any(x[0], x[1]);
-      c = split_pair_any(x[2], x[3]);
-    } else {
-      a = split_pair(x[0], x[1]);
-      c = split_pair(x[2], x[3]);
-      bad |= irregular(largest(largest(0.f, x[0], x[1]), x[2], x[3]));
-    }
+    constexpr bool whole = decltype(fp32)::value;
+    const Pair3 a = whole ? halves_of_pair(x[0], x[1]) : split_pair(x[0], x[1]), c = whole ? halves_of_pair(x[2], x[3]) : split_pair(x[2], x[3]);
     *reinterpret_cast<u32x2*>(at) = u32x2{a.h, c.h};
     *reinterpret_cast<u32x2*>(at + plane) = u32x2{a.m, c.m};
-    *reinterpret_cast<u32x2*>(at + 2 * plane) = u32x2{a.l, c.l};
+    if constexpr (!whole) *reinterpret_cast<u32x2*>(at + 2 * plane) = u32x2{a.l, c.l};
   };
   auto rebuild = [&](auto fp32, int tile) __attribute__((always_inline)) {
     uint16_t* const kd = planes + (tile & 1) * L::kBuffer;
     uint16_t* const vd = kd + 3 * L::kKPlane;
+    float k_top = 0.f;
+    Magnitudes v_seen;
 #pragma unroll
     for (int q = 0; q < CH; ++q) {
       const int chunk = q * NT + tid, t = chunk / CPR, cc = chunk % CPR;
@@ -183,9 +178,14 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
           av += wv * bv;
         }
       }
-      stage(fp32, kd + t * L::KS + 4 * cc, L::kKPlane, ak * inv_r);
-      stage(fp32, vd + t * L::VS + 4 * cc, L::kVPlane, av * inv_r);
+      ak *= inv_r;
+      av *= inv_r;
+      k_top = largest(k_top, ak);
+      v_seen.add(av);
+      stage(fp32, kd + t * L::KS + 4 * cc, L::kKPlane, ak);
+      stage(fp32, vd + t * L::VS + 4 * cc, L::kVPlane, av);
     }
+    if constexpr (!decltype(fp32)::value) bad |= !(k_top < kLogitOperand) | v_seen.irregular();
     if constexpr (SEG)
       if (tid < kTK) lds_seg[(tile & 1) * kTK + tid] = p.kvseg[(int64_t)b * p.lk + min(kbeg + tile * kTK + tid, p.lk - 1)];
   };
@@ -340,6 +340,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
       for (int v = 0; v < 16; ++v) o[db][v] = 0.f;
     m_run = -INFINITY;
     lsum = 0.f;
+    load_q(fp32);
     rebuild(fp32, 0);
     __syncthreads();
     // The next tile may be rebuilt anywhere between two barriers.  Waves w and w + 4 share a SIMD:
@@ -499,13 +500,20 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
   auto last_v = [&](const Flight& in, int tile) __attribute__((always_inline)) {
     if (rk == 1) take_v(in, tile, true);
     else take_v(in, tile, false);
-    float top = 0.f;
+    float top = 0.f, bottom = INFINITY;
 #pragma unroll
     for (int q = 0; q < NST; ++q) {
-      top = largest(largest(top, vac[q][0], vac[q][1]), vac[q][2], vac[q][3]);
+      top = largest(top, vac[q]);
+      bottom = smallest(bottom, vac[q]);
       *reinterpret_cast<f32x4*>(lds_v + (q * RPI + lrow) * RS + 4 * lc) = vac[q];
     }
-    bad |= irregular(top);
+    bad |= !(top < 0x1p127f);
+    if (bottom < 0x1p-90f) {  // zeros or small values
+      Magnitudes seen;
+#pragma unroll
+      for (int q = 0; q < NST; ++q) seen.add(vac[q]);
+      bad |= seen.irregular();
+    }
   };
   auto last_k = [&](const Flight& in, int tile) __attribute__((always_inline)) {
     float top = 0.f;
@@ -515,13 +523,13 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
         f32x4* const at = reinterpret_cast<f32x4*>(lds_k + (q * RPI + lrow) * RS + 4 * lc);
         f32x4 x = row_of(in, tile, q);
         if (!first) x += *at;
-        top = largest(largest(top, x[0], x[1]), x[2], x[3]);
+        top = largest(top, x);
         *at = x;
       }
     };
     if (rk == 1) finish(true);
     else finish(false);
-    bad |= irregular(top);
+    bad |= !(top < kLogitOperand);
   };
 
   Flight in_v, in_k;
@@ -534,36 +542,40 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
   request_first();  // ahead of Q
   // ---- Q, scaled and split (B operand of S^T = K Q^T): the 32 rows are the same for all waves, which read them from LDS
   uint16_t* const lds_q = reinterpret_cast<uint16_t*>(smem_f32_split + NW * SplitLdsF32<D>::kPerWave);
-  float q_top = 0.f;
-  for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
-    const int row = idx / CPR, cc = idx % CPR, row_ld = min(q0 + row, p.lq - 1);
-    const float* qb = static_cast<const float*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)row_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * cc;
-    const float* qa = dense ? nullptr : static_cast<const float*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)row_ld * p.qa.stride_l + h;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    constexpr int G = 6;  // ranks whose loads are in flight together
-    for (int r0 = 0; r0 < p.rq; r0 += G) {
-      f32x4 bv[G];
-      float a[G];
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const int r = min(r0 + u, p.rq - 1);
-        a[u] = dense ? 1.f : qa[r * p.qa.stride_r];
-        bv[u] = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r);
+  auto park_q = [&](auto fp32, const auto& p, int tid) __attribute__((always_inline)) {
+    constexpr bool whole = decltype(fp32)::value;
+    float top = 0.f;
+    for (int idx = tid; idx < 32 * CPR; idx += NW * 64) {
+      const int row = idx / CPR, cc = idx % CPR, row_ld = min(q0 + row, p.lq - 1);
+      const float* qb = static_cast<const float*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)row_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 4 * cc;
+      const float* qa = dense ? nullptr : static_cast<const float*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)row_ld * p.qa.stride_l + h;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      constexpr int G = 6;  // ranks whose loads are in flight together
+      for (int r0 = 0; r0 < p.rq; r0 += G) {
+        f32x4 bv[G];
+        float a[G];
+  #pragma unroll
+        for (int u = 0; u < G; ++u) {
+          const int r = min(r0 + u, p.rq - 1);
+          a[u] = dense ? 1.f : qa[r * p.qa.stride_r];
+          bv[u] = *reinterpret_cast<const f32x4*>(qb + r * p.qb.stride_r);
+        }
+  #pragma unroll
+        for (int u = 0; u < G; ++u)
+          if (r0 + u < p.rq) acc += a[u] * bv[u];
       }
-#pragma unroll
-      for (int u = 0; u < G; ++u)
-        if (r0 + u < p.rq) acc += a[u] * bv[u];
+      acc *= p.sm_scale * kLog2e / (float)p.rq;
+      top = largest(top, acc);
+      const Pair3 x = whole ? halves_of_pair(acc[0], acc[1]) : split_pair(acc[0], acc[1]), y = whole ? halves_of_pair(acc[2], acc[3]) : split_pair(acc[2], acc[3]);
+      uint16_t* const at = lds_q + row * SplitLdsF32<D>::QS + 4 * cc;
+      *reinterpret_cast<u32x2*>(at) = u32x2{x.h, y.h};
+      *reinterpret_cast<u32x2*>(at + SplitLdsF32<D>::kQPlane) = u32x2{x.m, y.m};
+      *reinterpret_cast<u32x2*>(at + 2 * SplitLdsF32<D>::kQPlane) = u32x2{x.l, y.l};
     }
-    acc *= p.sm_scale * kLog2e / (float)p.rq;
-    q_top = largest(largest(q_top, acc[0], acc[1]), acc[2], acc[3]);
-    const Pair3 x = split_pair_any(acc[0], acc[1]), y = split_pair_any(acc[2], acc[3]);
-    uint16_t* const at = lds_q + row * SplitLdsF32<D>::QS + 4 * cc;
-    *reinterpret_cast<u32x2*>(at) = u32x2{x.h, y.h};
-    *reinterpret_cast<u32x2*>(at + SplitLdsF32<D>::kQPlane) = u32x2{x.m, y.m};
-    *reinterpret_cast<u32x2*>(at + 2 * SplitLdsF32<D>::kQPlane) = u32x2{x.l, y.l};
-  }
-  bad = irregular(q_top);
-  __syncthreads();
+    bad |= !(top < kLogitOperand);
+    __syncthreads();
+  };
+  park_q(std::false_type{}, p, tid);
   int q_offset = i * SplitLdsF32<D>::QS + 8 * g;
   auto q_operand = [&](int ks) __attribute__((always_inline)) -> Split3 {
     const uint16_t* const at = lds_q + q_offset + 16 * ks;
@@ -589,8 +601,8 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
     }
     for (int tile = w; tile < ntiles; tile += NW) {
       const int next = tile + NW;
-      const bool more = next < ntiles;
-      if (more) issue(in_v, vb_r, va_r, next, 0);
+      const bool more = next < ntiles, ahead = more && !decltype(fp32)::value;  // the second walk fetches a tile when it is needed: it holds less
+      if (ahead) issue(in_v, vb_r, va_r, next, 0);
       f32x16 s;
 #pragma unroll
       for (int v = 0; v < 16; ++v) s[v] = 0.f;
@@ -623,9 +635,10 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             s = __builtin_amdgcn_mfma_f32_32x32x2f32(lds_k[i * RS + 16 * ks + 8 * g + e], join(qf, e), s, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
-      if (more) {
+      if (ahead) {
         but_last(in_v, vb_r, va_r, next, take_v);
         issue(in_k, kb_r, ka_r, next, 0);
         if constexpr (SEG) seg_in = p.kvseg[(int64_t)b * p.lk + min(kbeg + next * 32 + i, p.lk - 1)];
@@ -669,7 +682,7 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
       if constexpr (!decltype(fp32)::value) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          if (t == 1 && more) but_last(in_k, kb_r, ka_r, next, take_k);
+          if (t == 1 && ahead) but_last(in_k, kb_r, ka_r, next, take_k);
           float x[8], y[NDB][8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
@@ -690,11 +703,17 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
       } else {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          if (v == 8 && more) but_last(in_k, kb_r, ka_r, next, take_k);
           const f32xN vf = v_rows(v);
 #pragma unroll
           for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db], s[v], o[db], 0, 0, 0);
         }
+      }
+      if (more && !ahead) {
+        issue(in_v, vb_r, va_r, next, 0);
+        but_last(in_v, vb_r, va_r, next, take_v);
+        issue(in_k, kb_r, ka_r, next, 0);
+        but_last(in_k, kb_r, ka_r, next, take_k);
+        if constexpr (SEG) seg_in = p.kvseg[(int64_t)b * p.lk + min(kbeg + next * 32 + i, p.lk - 1)];
       }
       if (more) {
         last_v(in_v, next);
@@ -720,6 +739,7 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
   walk(std::false_type{});
   if (__builtin_expect(__syncthreads_or(bad), 0)) {
     request_first();
+    park_q(std::true_type{}, *arguments_again<F32Params>(), again(tid));
     walk(std::true_type{});
     __syncthreads();
   }

@@ -49,6 +49,15 @@ def _spoil(kind, q, k, v, h):
         v[:, key, 1:, h + 7] = 0.0
     elif kind == "tiny values":
         v[:, :, :, h:] *= 1e-33
+    elif kind == "one small column":  # below 2^-110, where the last bits of a value are below bf16's smallest number
+        v[:, :, :, h + 6] *= 1e-34
+    elif kind == "one small column beside an infinity":
+        v[:, :, :, h + 6] *= 1e-34
+        v[:, key, :, :h] = np.abs(v[:, key, :, :h])
+        v[:, key, 0, h + 7] = np.inf
+    elif kind == "small queries, large keys":  # products around 1 of parts whose last bits are below bf16's smallest number
+        q[:, :, :, h:] *= 1e-35
+        k[:, :, :, h:] *= 1e35
     elif kind == "logit below the range":  # finite operands, products around -2^140 of which the parts have both signs
         q[:, :, :, :h] = np.abs(q[:, :, :, :h]) + 0.5
         k[:, key, :, :h] = np.abs(k[:, key, :, :h]) + 0.5
@@ -60,7 +69,7 @@ def _spoil(kind, q, k, v, h):
         k[:, :, :, h:] *= 1e19
 
 
-@pytest.mark.parametrize("kind", ["ordinary", "infinite key", "infinite query", "NaN value", "infinite value", "rounds to infinity", "tiny values", "tiny queries, large keys", "logit below the range"])
+@pytest.mark.parametrize("kind", ["ordinary", "infinite key", "infinite query", "NaN value", "infinite value", "rounds to infinity", "tiny values", "tiny queries, large keys", "logit below the range", "one small column", "one small column beside an infinity", "small queries, large keys"])
 @pytest.mark.parametrize("b,t,h,d,rk", SHAPES)
 def test_forward_values_that_do_not_split(gpu, b, t, h, d, rk, kind):
     from tpa import tpa
@@ -86,7 +95,7 @@ def test_forward_values_that_do_not_split(gpu, b, t, h, d, rk, kind):
             assert np.linalg.norm((x - y) / top) <= 1e-5 * np.linalg.norm(y / top), c
 
 
-@pytest.mark.parametrize("kind", ["ordinary", "tiny gradient", "rounds to infinity", "large gradient"])
+@pytest.mark.parametrize("kind", ["ordinary", "small gradient", "tiny gradient", "one tiny column", "rounds to infinity", "large gradient"])
 @pytest.mark.parametrize(
     "b,t,h,d,causal",
     [
@@ -105,6 +114,11 @@ def test_backward_values_that_do_not_split(gpu, b, t, h, d, causal, kind):
     do = np.random.default_rng(84).standard_normal((b, t, h, d)).astype(np.float32)
     if kind == "tiny gradient":
         do *= np.float32(1e-28)
+    elif kind == "small gradient":  # small, but split
+        do *= np.float32(1e-20)
+    elif kind == "one tiny column":  # of the upstream gradient and of the values
+        do[..., 6] *= np.float32(1e-34)
+        v[..., h + 7] *= np.float32(1e-34)
     elif kind == "large gradient":  # dP and dS near the largest float
         do *= np.float32(1e16)
         v[..., h:] *= np.float32(1e20)
@@ -118,6 +132,7 @@ def test_backward_values_that_do_not_split(gpu, b, t, h, d, causal, kind):
     want = orc.tpa_backward(q, k, v, None, None, h, do, sm_scale=scale, causal=causal)
     for n, w in enumerate(want):
         got = np.concatenate([x.cpu().numpy() for x in grads[2 * n : 2 * n + 2]], axis=-1).astype(np.float64)
-        for x, y in ((got[..., :h], w[..., :h]), (got[..., h:], w[..., h:])):
+        # the head factors' gradients as a whole, the token factors' column by column
+        for x, y in [(got[..., :h], w[..., :h])] + [(got[..., h + c], w[..., h + c]) for c in range(d)]:
             top = np.abs(y).max()
             assert np.linalg.norm((x - y) / top) <= 1e-5 * np.linalg.norm(y / top), "qkv"[n]
