@@ -50,9 +50,9 @@ def _spoil(kind, q, k, v, h):
     elif kind == "tiny values":
         v[:, :, :, h:] *= 1e-33
     elif kind == "one small column":  # below 2^-110, where the last bits of a value are below bf16's smallest number
-        v[:, :, :, h + 6] *= 1e-34
+        v[:, :, :, h + 6] *= 2e-37
     elif kind == "one small column beside an infinity":
-        v[:, :, :, h + 6] *= 1e-34
+        v[:, :, :, h + 6] *= 2e-37
         v[:, key, :, :h] = np.abs(v[:, key, :, :h])
         v[:, key, 0, h + 7] = np.inf
     elif kind == "small queries, large keys":  # products around 1 of parts whose last bits are below bf16's smallest number
@@ -117,8 +117,8 @@ def test_backward_values_that_do_not_split(gpu, b, t, h, d, causal, kind):
     elif kind == "small gradient":  # small, but split
         do *= np.float32(1e-20)
     elif kind == "one tiny column":  # of the upstream gradient and of the values
-        do[..., 6] *= np.float32(1e-34)
-        v[..., h + 7] *= np.float32(1e-34)
+        do[..., 6] *= np.float32(2e-37)
+        v[..., h + 7] *= np.float32(2e-37)
     elif kind == "large gradient":  # dP and dS near the largest float
         do *= np.float32(1e16)
         v[..., h:] *= np.float32(1e20)
