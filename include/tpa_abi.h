@@ -300,8 +300,8 @@ const char* tpa_strerror(int code);
  * If `workspace` holds at least tpa_decode_workspace_bytes(...) bytes and the problem is a
  * decode (lq <= 16, lk >= 1024, no segment ids) that tpa_decode's kernel takes, the call is served by
  * it; if `workspace` holds tpa_fwd_workspace_bytes(...) bytes and the problem is long enough for it to
- * pay (rank 2: 2048 query rows and more; other ranks: more than 256, and from rank 3 on more than 16 over
- * 1024 keys or more), dense bf16 Q (times
+ * pay (rank 2: 2048 query rows and more, and fewer where tpa_fwd_call_workspace_bytes asks for the room; other
+ * ranks: more than 256, and from rank 3 on more than 16 over 1024 keys or more), dense bf16 Q (times
  * sm_scale * log2 e), K and V are reconstructed into it once and the prefill kernel runs its loop over
  * dense tiles.  Without a workspace the same problems run on the fused prefill kernel, which rebuilds
  * K / V tiles from the rank factors inside its loop.  The two routes round at the same points (Q, K, V,
@@ -320,7 +320,8 @@ size_t tpa_fwd_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int
 /*
  * Bytes of optional workspace (256-byte aligned) that leave tpa_fwd every route it has for this problem: at least
  * tpa_fwd_workspace_bytes(...), plus room for the partial results of key ranges where the blocks of 256 query rows
- * alone would leave the chip partly idle (bf16, no segment ids).
+ * alone would leave the chip partly idle (bf16, no segment ids), and for dense Q, K and V of calls of rank 2 below 2048
+ * query rows where these pay.
  */
 size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk);
 

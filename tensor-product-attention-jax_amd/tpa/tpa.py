@@ -21,7 +21,7 @@ reference, all on purpose:
   * `interpret=True` (the Pallas CPU interpreter upstream) selects the plain fp32-arithmetic
     kernel instead of the MFMA kernels; `debug` is ignored;
   * the backward pass (tpa/tpa.py:168-214,546-995) goes through dense Q, K, V and dense gradients
-    in a workspace (bf16 MFMA kernels for bf16 inputs and fp32 MFMA kernels for fp32 inputs of
+    in a workspace (matrix-core kernels for bf16 inputs and, on split values, for fp32 inputs of
     head sizes 64 and 128, fp32 vector-ALU kernels otherwise); gradients are accumulated in fp32
     and cast to the input dtype; torch.autograd reaches it through `tpa()`.
 """
