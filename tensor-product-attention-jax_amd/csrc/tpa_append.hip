@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256 * KS) void append_gemm_kernel(AppendParams p) {
 }
 
 // ---- bf16, few tokens (a decode step): the call is one read of W, and tiles of 64 columns would leave most of the chip idle.
-// A workgroup owns 16 columns, up to 64 tokens and all of k: its eight waves deal the chunks of 64 k round robin, each stages
+// A workgroup owns 16 columns, up to 64 tokens and all of k: each of its eight waves takes an eighth of the chunks of 64 k, stages
 // its own chunk (16 rows of W and the tokens' rows, whole cache lines in 16-byte pieces, kept in flight in registers several
 // chunks ahead) in LDS of its own, swizzled, and multiplies it with v_mfma_f32_16x16x32_bf16 - no barrier before the end,
 // where a ninth wave, which has looked up destinations and angles meanwhile, adds the eight partial tiles and stores.
@@ -538,7 +538,7 @@ __global__ __launch_bounds__((kRowWaves + 1) * 64) void append_rows_kernel(Appen
     };
     // Each chunk is summed by itself and then added: a chain of matrix instructions over all of a wave's chunks rounds against
     // the whole sum every time (d_model 4096 / 16 384, 48 tokens: 1.6e-4 / 3.2e-4 of the results missed the rounding of the exact
-    // sum, 1.2e-4 / 1.8e-4 so; 200 tokens x 1600 columns 19.0 / 19.9 us).
+    // sum, 1.2e-4 / 1.7e-4 so; 200 tokens x 1600 columns 19.0 / 19.9 us).
     auto multiply = [&]() __attribute__((always_inline)) {
       f32x4 part[MB];
 #pragma unroll
@@ -552,15 +552,16 @@ __global__ __launch_bounds__((kRowWaves + 1) * 64) void append_rows_kernel(Appen
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[mb] += part[mb];
     };
+    const int first = w * nchunks / kRowWaves, end = (w + 1) * nchunks / kRowWaves;  // this wave's chunks
     static_for<NSET>([&](auto n) __attribute__((always_inline)) {
-      if (w + kRowWaves * decltype(n)::value < nchunks) load(n, w + kRowWaves * decltype(n)::value);
+      if (first + decltype(n)::value < end) load(n, first + decltype(n)::value);
     });
-    for (int c0 = w; c0 < nchunks; c0 += kRowWaves * NSET)
+    for (int c0 = first; c0 < end; c0 += NSET)
       static_for<NSET>([&](auto n) __attribute__((always_inline)) {
-        const int c = c0 + kRowWaves * decltype(n)::value;
-        if (c < nchunks) {
+        const int c = c0 + decltype(n)::value;
+        if (c < end) {
           take(n);
-          if (c + kRowWaves * NSET < nchunks) load(n, c + kRowWaves * NSET);
+          if (c + NSET < end) load(n, c + NSET);
           multiply();
         }
       });
@@ -607,9 +608,9 @@ __global__ __launch_bounds__((kRowWaves + 1) * 64) void append_rows_kernel(Appen
       hi[ww] = *reinterpret_cast<const f32x4*>(src + 4);
     }
 #pragma unroll
-    for (int n = kRowWaves / 2; n > 0; n /= 2)
+    for (int n = 1; n < kRowWaves; n *= 2)
 #pragma unroll
-      for (int ww = 0; ww < n; ++ww) { lo[ww] += lo[ww + n]; hi[ww] += hi[ww + n]; }
+      for (int ww = 0; ww < kRowWaves; ww += 2 * n) { lo[ww] += lo[ww + n]; hi[ww] += hi[ww + n]; }
     float y[8] = {lo[0][0], lo[0][1], lo[0][2], lo[0][3], hi[0][0], hi[0][1], hi[0][2], hi[0][3]};
     if (rotate[u]) {
 #pragma unroll

@@ -1,4 +1,4 @@
-"""The append kernel for few tokens (16 columns and up to 64 tokens per workgroup, the contraction dealt to eight waves in
+"""The append kernel for few tokens (16 columns and up to 64 tokens per workgroup, the contraction in eight parts, one to a wave, in
 chunks of 64): numbers of tokens around its blocks of 16, 32 and 64, contractions of fewer chunks than waves and of odd
 numbers of chunks, ragged column blocks, and calls on either side of the line to the 64 x 64 tiles, against the CPU oracle."""
 
@@ -35,8 +35,8 @@ def test_append_few_tokens(gpu, b, n, dm, h, d, rq, rk):
 
 def test_results_are_the_roundings_of_exact_sums(gpu):
     """Results of a long contraction that are not the bf16 rounding of the exact sum.  An fp32 sum that is off by e rounds to the
-    wrong side for a share of about 2 e / spacing of the results; with the chunks of 64 summed one by one that is 1.8e-4 here, with one
-    chain of matrix instructions per wave 3.2e-4 (1.8 million results: 320 and 590, give or take 25)."""
+    wrong side for a share of about 2 e / spacing of the results; with the chunks of 64 summed one by one that is 1.7e-4 here, with one
+    chain of matrix instructions per wave 3.2e-4 (1.8 million results: 310 and 590, give or take 25)."""
     n, dm, h, d, rq, rk = 48, 16384, 32, 128, 6, 2
     wrong = total = 0
     for seed in range(24):
