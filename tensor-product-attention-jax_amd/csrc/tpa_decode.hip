@@ -236,8 +236,12 @@ struct DecodeLds {
   static constexpr size_t bytes(int nq) { return kBytes + (nq > 1 ? (size_t)nq * (D / 16) * 64 * 16 : 0); }
 };
 
+// At head size 64 and from rank 4 on two workgroups fit a compute unit, which the compiler has to be told: at 258 registers
+// instead of 256 rank 8 lost the second one (64 heads, two rows per workgroup: 48 x 4096 keys, eight rows 544 -> 707 us; 4 x 1024
+// rows and keys without K and V 2.42 -> 3.15 ms; 2.10 so, with 204).
+constexpr int min_waves(int d, int rk) { return d == 64 && rk >= 4 ? 2 : 1; }
 template <int D, int RK, bool PAGED, int NQ, Reads READS>
-__global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeParams p) {
+__global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(DecodeParams p) {
   constexpr int CPR = D / 8;               // 16-byte chunks per B row
   constexpr int RPI = 64 / CPR;            // B rows per load instruction
   constexpr int NLB = kRowsPerBlock / RPI; // load instructions per B tile
@@ -1011,12 +1015,17 @@ int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream,
 // meant to find the slice in its L2, so the loads stay ordinary (four rows at the c4 shape: 1022 MB fetched with non-temporal
 // loads, 676 MB = the cache once with ordinary ones).  Two head blocks read the same token rows as well; with two rows and from
 // rank 4 on that decides (3 x 9000 keys, 64 heads of 64, rank 4: 24.1 us non-temporal, 22.5 ordinary; rank 2 19.1 / 19.2, paged
-// 52.0 / 54.3), with one row the second block of loads hides it.
+// 52.0 / 54.3), with one row from rank 16 on (48 x 4096 keys, 64 heads of 64: rank 4 94 / 93, rank 8 180 / 179 - 187, paged
+// 140 / 133; 16 380 / 356 and 270 / 250; 32 831 / 700 and 557 / 468; with one block of loads in flight, non-temporal, 798 and 518).
 template <int D, int RK, bool PAGED>
 int launch_decode_rows(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   for (const TpaFactor* f : {&a->ka, &a->kb, &a->va, &a->vb})
     if (f->stride_r < 0 || f->stride_r > kFarthestRow) return launch_decode_t<D, RK, PAGED, 2, Reads::kFar>(a, ranges, stream, rows);
-  if (a->lq == 1) return launch_decode_t<D, RK, PAGED, 1, Reads::kStreaming>(a, ranges, stream, rows);
+  if (a->lq == 1) {
+    if constexpr (RK >= 16)
+      if (a->H > 32) return launch_decode_t<D, RK, PAGED, 1, Reads::kOrdinary>(a, ranges, stream, rows);
+    return launch_decode_t<D, RK, PAGED, 1, Reads::kStreaming>(a, ranges, stream, rows);
+  }
   if (a->lq == 2 && (a->H <= 32 || RK < 4)) return launch_decode_t<D, RK, PAGED, 2, Reads::kStreaming>(a, ranges, stream, rows);
   return launch_decode_t<D, RK, PAGED, 2, Reads::kOrdinary>(a, ranges, stream, rows);
 }

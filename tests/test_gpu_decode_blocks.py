@@ -11,7 +11,7 @@ from test_gpu_parity import BF16_TOL, _varlen_reference, as_f64, bf16_bounds, ch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("h,d,rk", [(16, 128, 2), (40, 64, 4)])
+@pytest.mark.parametrize("h,d,rk", [(16, 128, 2), (40, 64, 4), (40, 64, 8), (40, 64, 16)])
 @pytest.mark.parametrize("rq", [1, 8, 9, 16, 17, 33])
 @pytest.mark.parametrize("lq", [1, 2, 3])
 @pytest.mark.parametrize("page", [0, 48, 64])
