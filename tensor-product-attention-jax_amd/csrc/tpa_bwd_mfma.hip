@@ -169,6 +169,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
     }
     qseg[nb] = SEG ? p.qseg[(int64_t)b * p.lq + qrow_ld] : 0;
   }
+  const TileIds<SEG, NB> ids_of_wave(qseg);
 
   // keys [kpos0, kend) are visited; tiles and key positions below count from kpos0
   int kpos0 = 0, kend = p.causal ? max(1, min(p.lk, min(q0 + kBQ, p.lq) + p.coff)) : p.lk;  // at least one (then fully masked) tile
@@ -221,7 +222,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) acc[nb][db] = splat16(0.f);
 
-  auto compute = [&](int j) __attribute__((always_inline)) {
+  auto compute = [&](int j, bool masked_ids) __attribute__((always_inline)) {
     const uint16_t* ks = lds_k + (j & 1) * kTile * S;
     const uint16_t* vs = lds_v + (j & 1) * kTile * S;
     const int k0 = j * kTile;
@@ -263,7 +264,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
           for (int v = 0; v < 16; ++v)
             if (k0 + 32 * mb + 8 * (v >> 2) + 4 * g + (v & 3) > limit) s[nb][v] = -INFINITY;
         }
-        if constexpr (SEG) {
+        if (SEG && masked_ids) {
           const int32_t* ids_p = lds_seg + (j & 1) * kTile + 32 * mb + 4 * g;
 #pragma unroll
           for (int vq = 0; vq < 4; ++vq) {
@@ -292,7 +293,10 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
   issue(min(1, last));
   __syncthreads();
   for (int j = 0; j < ntiles; ++j) {
-    if (j <= wave_last_tile) compute(j);
+    if (j <= wave_last_tile) {
+      const int ids = ids_of_wave.look(lds_seg + (j & 1) * kTile, l);
+      if (ids != kNoneOfThem) compute(j, ids == kSomeOfThem);
+    }
     if (j + 1 < ntiles) {
       commit(j + 1);
       issue(min(j + 2, last));
@@ -364,6 +368,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
     }
     kseg[nb] = SEG ? p.kvseg[(int64_t)b * p.lk + key_ld] : 0;
   }
+  const TileIds<SEG, NB> ids_of_wave(kseg);
 
   // query tiles tile0 .. : under the causal mask rows before this block's first key see none of
   // its keys; rows from lq_r on are not visited
@@ -436,7 +441,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) { dk_acc[nb][db] = splat16(0.f); dv_acc[nb][db] = splat16(0.f); }
 
-  auto compute = [&](int j) __attribute__((always_inline)) {
+  auto compute = [&](int j, bool masked_ids) __attribute__((always_inline)) {
     const uint16_t* qs = lds_q + (j & 1) * kTile * S;
     const uint16_t* gs = lds_g + (j & 1) * kTile * S;
     const float* nl = lds_nlse + (j & 1) * kTile;
@@ -498,7 +503,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
           for (int v = 0; v < 16; ++v)
             if (r0 + 32 * mb + 8 * (v >> 2) + 4 * g + (v & 3) < key) s[nb][v] = -INFINITY;
         }
-        if constexpr (SEG) {
+        if (SEG && masked_ids) {
           const int32_t* ids_p = lds_seg + (j & 1) * kTile + 32 * mb + 4 * g;
 #pragma unroll
           for (int vq = 0; vq < 4; ++vq) {
@@ -538,7 +543,10 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
     issue(min(1, last));
     __syncthreads();
     for (int j = 0; j < ntiles; ++j) {
-      if (j >= wave_first_tile) compute(j);
+      if (j >= wave_first_tile) {
+        const int ids = ids_of_wave.look(lds_seg + (j & 1) * kTile, l);
+        if (ids != kNoneOfThem) compute(j, ids == kSomeOfThem);
+      }
       if (j + 1 < ntiles) {
         commit(j + 1);
         issue(min(j + 2, last));

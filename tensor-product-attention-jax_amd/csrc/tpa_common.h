@@ -173,6 +173,30 @@ __device__ __forceinline__ void id_window(const int32_t* mine, int n_mine, const
   id_window<NT>(mine, n_mine, other, n_other, red, tid, first, last, cnt, smin, smax);
 }
 
+// Segment ids inside the window.  A workgroup visits every tile that one of its rows needs, a wave owns 32 of them and often a
+// single document, so a wave looks at each tile's 64 ids itself: a tile without an id in the range of its own rows is left out, and
+// one that holds nothing but the one id of all of them needs no mask.  Both are exact for any order of the ids.
+enum { kNoneOfThem = 0, kSomeOfThem = 1, kAllOfThem = 2 };
+template <bool SEG, int NB>
+struct TileIds {
+  int32_t least, most;
+  __device__ __forceinline__ explicit TileIds(const int32_t (&own)[NB]) : least(0), most(0) {
+    if constexpr (SEG) {
+      least = most = own[0];
+#pragma unroll
+      for (int nb = 1; nb < NB; ++nb) { least = min(least, own[nb]); most = max(most, own[nb]); }
+      least = scalar(wave_min(least)); most = scalar(wave_max(most));
+    }
+  }
+  // `tile` = the tile's 64 ids in LDS
+  __device__ __forceinline__ int look(const int32_t* tile, int lane) const {
+    if constexpr (!SEG) return kAllOfThem;
+    const int32_t id = tile[lane];
+    if (__ballot(id >= least && id <= most) == 0) return kNoneOfThem;
+    return least == most && __ballot(id != least) == 0 ? kAllOfThem : kSomeOfThem;
+  }
+};
+
 // Which of the eight (block, batch) pairs of round `round` the workgroups on XCD `xcd` take, with
 // pair = block_rank * B + batch.  Workgroup ids map to XCDs statically, so with a fixed direction
 // one XCD would collect the heaviest causal block of every round; odd rounds therefore reverse the

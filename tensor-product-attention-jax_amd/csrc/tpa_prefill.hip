@@ -417,6 +417,8 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
 #pragma unroll
     for (int r = 0; r < RB; ++r) qseg[r] = p.qseg[(int64_t)b * p.lq + qrow_ld[r]];
   }
+  const TileIds<has_seg, RB> ids_of_wave(qseg);
+  bool masked_ids = false;  // tile j needs its segment mask for this wave's rows
 
   // (a0/2)*b0[d] + (a1/2)*b1[d] for 8 consecutive d; aa = packed (a0/2, a1/2): fetch_aa hands out
   // halved head factors.
@@ -598,9 +600,8 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
           if (t > limit) s[r][mb][v] = -INFINITY;
         }
     }
-    // keys of another segment (tpa/tpa.py:369-375); where the rows share one id and its keys form one run,
-    // only tile 0 can hold keys of another segment (the run's end is the end of the keys this workgroup visits)
-    if (has_seg && !(seg_pure && tile > 0)) {
+    // keys of another segment (tpa/tpa.py:369-375)
+    if (has_seg && masked_ids) {
       const int32_t* slot = lds_seg(tile & 1);
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb)
@@ -757,7 +758,13 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     }
   };
   auto cold_iteration = [&](int j) __attribute__((always_inline)) {
-    if (j <= wave_last_tile[0]) cold_compute(j, IC<1>{}, IC<0>{});
+    if (j <= wave_last_tile[0]) {
+      // where the rows share one id and its keys form one run, only tile 0 can hold keys of another segment (the run's
+      // end is the end of the keys this workgroup visits)
+      const int ids = has_seg && !(seg_pure && j > 0) ? ids_of_wave.look(lds_seg(j & 1), l) : kAllOfThem;
+      masked_ids = ids == kSomeOfThem;
+      if (ids != kNoneOfThem) cold_compute(j, IC<1>{}, IC<0>{});
+    }
     advance_tiles(j);
   };
 
@@ -825,6 +832,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     // iterations 1 .. hot_end - 2 and leaves the logits of tile hot_end - 1, which is finished
     // here.  The state goes in and comes back in operands pinned to the loop's registers.
     if (hot_end >= 3) {
+      masked_ids = false;
       cold_compute(1, IC<1>{}, IC<1>{});
       auto cat4 = [](const u32x4& a0, const u32x4& a1, const u32x4& a2, const u32x4& a3) __attribute__((always_inline)) -> f32x16 {
         const u32x8 lo = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -903,6 +911,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     // register assignment) runs iterations 1 .. hot_end - 2 - everything advance_tiles() and tail() do
     // included - and leaves the logits of the first 32 keys of tile hot_end - 1, which is finished here.
     if (hot_end >= 3) {
+      masked_ids = false;
       cold_compute(1, IC<1>{}, IC<3>{});
       auto cat4 = [](const u32x4& a0, const u32x4& a1, const u32x4& a2, const u32x4& a3) __attribute__((always_inline)) -> u32x16 {
         const u32x8 lo = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
