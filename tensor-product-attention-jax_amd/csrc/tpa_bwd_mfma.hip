@@ -596,7 +596,7 @@ inline int pair_groups_of(int npairs, int nblk) {
 // 1 x 1000 tokens, 16 heads of 128, 168 -> 127 us; 4 x 1000 194 -> 170; 4 x 4096 and longer unchanged.
 struct BwdPair { BwdParams kv, q; int n_kv; };
 template <int D, int NW, int NB, bool SEG>
-__global__ __launch_bounds__(NW * 64) void bwd_dq_dkv_kernel(BwdPair p) {
+__global__ __launch_bounds__(NW * 64, 2) void bwd_dq_dkv_kernel(BwdPair p) {
   if ((int)blockIdx.x < p.n_kv) dkv_block<D, NW, NB, SEG>(p.kv, blockIdx.x);
   else dq_block<D, NW, NB, SEG>(p.q, blockIdx.x - p.n_kv);
 }
@@ -623,12 +623,28 @@ int launch(const BwdParams& base, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
+// Rows (keys) per workgroup: eight waves of 32, or at head size 64 four waves of 32 with two workgroups on a compute unit (their
+// tiles take 37 KB; at head size 128 they and the parked V fragments take 110 KB and only one fits).  Two halves do not wait for
+// each other's barriers and fit documents and the diagonal more closely; both stage every tile for themselves, which is what
+// long blocks without documents lose by.  Training steps, us, eight waves / four (the compiler has to be held to two waves per
+// SIMD, or only one workgroup fits and everything is slower):
+//   documents: 3 x 1777, 16 heads, of 421 tokens 129 / 117; 2 x 9000, 8 heads, of 9000 684 / 590; 1 x 20 000, 8 heads, of 4000
+//     609 / 569; 4 x 3000, 16 heads, of 2900 401 / 377; without a mask 2 x 9000, 16 heads, of 3000 1216 / 1136
+//   causal: 16 x 512, 16 heads 163 / 146; 2 x 1300, 64 heads 265 / 252; 8 x 1024, 64 heads 681 / 657; 2 x 2300, 64 heads 560 /
+//     559; 8 x 3000, 16 heads 904 / 908; 1 x 8192, 16 heads 636 / 654
+//   no mask: 16 x 512, 16 heads 180 / 174; 4 x 1000, 64 heads 443 / 449; 4 x 2048, 16 heads 361 / 376
+// (64 keys per wave would halve the LDS reads per MFMA, but its 384 stationary registers at D = 128 leave the compiler
+// spilling; the dQ kernel with 4 waves of 64 rows, one wave per SIMD and 512 registers, takes 922 us where 8 waves of 32
+// rows take 401 us.)
 template <int D>
 int launch_both(const BwdParams& p, hipStream_t stream) {
-  // 8 waves of 32 rows or keys.  (64 keys per wave would halve the LDS reads per MFMA, but its 384
-  // stationary registers at D = 128 leave the compiler spilling; the dQ kernel with 4 waves of 64 rows, one
-  // wave per SIMD and 512 registers, takes 922 us where 8 waves of 32 rows take 401 us.)
-  return p.qseg ? launch<D, 8, 1, true>(p, stream) : launch<D, 8, 1, false>(p, stream);
+  if constexpr (D == 64) {
+    if (p.qseg) return launch<D, 4, 1, true>(p, stream);
+    if (p.causal && p.lq <= 2304 && p.lk <= 2304) return launch<D, 4, 1, false>(p, stream);
+    return launch<D, 8, 1, false>(p, stream);
+  } else {
+    return p.qseg ? launch<D, 8, 1, true>(p, stream) : launch<D, 8, 1, false>(p, stream);
+  }
 }
 
 }  // namespace
