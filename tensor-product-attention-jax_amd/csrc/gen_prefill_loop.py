@@ -9,7 +9,7 @@ softmax reads were finished one step earlier.
 dense loader (prefill_kernel<D, LOAD_DENSE, false>), one iteration j = one tile of 64 keys:
 
     S^T of tile j+1  (2 D/16 MFMAs, into the logit registers the previous iteration freed)
-    softmax of tile j (row maximum, exponentials, packing to bf16), spread behind those MFMAs
+    softmax of tile j (exponentials, row sums, packing to bf16), spread behind those MFMAs
     O^T += V^T P^T of tile j  (4 D/32 MFMAs)
     loader: K tile j+2 and V tile j+1 from registers to LDS, K tile j+3 and V tile j+2 requested
     one barrier
@@ -46,6 +46,8 @@ of gfx950 (results of matrix, dot and transcendental instructions, lane swaps, v
 matrix instructions) and inserts the s_waitcnt / s_nop instructions they need.
 
 usage: gen_prefill_loop.py <D: 128|64> <dense|r2> <output.inc>
+Beside the output it writes <output>_rare.inc (the rare paths; the asm statement includes them behind the loop) and
+<output>_clobbers.inc.
 """
 import re
 import sys
@@ -78,8 +80,8 @@ if not R2:
     RING_BUFS = [192, 196, 200]                       # v[192:203]: fragment buffers
     MREF, LSUM, KFRAG0, VFRAG, KW0, VW, KVOFF, VVOFF = range(204, 212)   # v[204:219]: state / address tuple
     STATE = range(204, 220)
-    TA, TB, T0A, T1A, KFRAG, KW, RD, RAL, T0B, T1B = range(220, 230)        # v[220:229]: temporaries
-    TEMPS = range(220, 230)
+    BS0, BS1, T0A, T1A, KFRAG, KW, T0B, T1B = range(220, 228)              # v[220:227]: temporaries
+    TEMPS = range(220, 228)
     # s[32:47] scalar tuple
     S_J, S_END, S_LAST, S_KTILE, S_VTILE, S_KPASS, S_VPASS, S_KR, S_KWB = range(32, 41)
     S_KB, S_VB = 48, 52                               # buffer resources s[48:51], s[52:55]
@@ -96,9 +98,9 @@ else:
     # v[188:203]: state / address tuple
     MREF, LSUM, KFRAG0, VFRAG, KW0, VW, KVOFF, VVOFF, A_RD, A_WR, A_VOFF, A_PEND = range(188, 200)
     STATE = range(188, 204)
-    # v[204:221]: temporaries
-    TA, TB, T0A, T1A, T0B, T1B, KFA, KFB, KW, RD, RAL, AAK0, AAK1, AAV0, AAV1, PT, PT2, AT = range(204, 222)
-    TEMPS = range(204, 222)
+    # v[204:219]: temporaries
+    BS0, BS1, T0A, T1A, T0B, T1B, KFA, KFB, KW, AAK0, AAK1, AAV0, AAV1, PT, PT2, AT = range(204, 220)
+    TEMPS = range(204, 220)
     # s[32:47] scalar tuple
     S_J, S_END, S_LAST, S_KTILE, S_VTILE, S_KPASS, S_VPASS, S_K0, S_K1, S_K2, S_KRANK, S_VRANK, S_ATILE, S_AAHEAD = range(32, 46)
     S_KB, S_VB, S_AB = 48, 52, 56                     # buffer resources s[48:51], s[52:55], s[56:59]
@@ -373,42 +375,46 @@ def issue_loads(e, is_v):
         if ps + 1 < NPASS:
             e.ins("s_add_u32", f"s{S_T1}", f"s{S_T1}", f"s{pss}")
 
-# ---- softmax of tile j (set p): one maximum over the tile's 32 logits of this lane's row
-def sm_max(e, p):
-    s = S(p, 0)
-    e.ins("v_max3_f32", f"v{TA}", f"v{s}", f"v{s + 1}", f"v{s + 2}")
-    e.ins("v_max3_f32", f"v{TB}", f"v{s + 3}", f"v{s + 4}", f"v{s + 5}")
-    for k in range(6, 32, 4):
-        e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{s + k}", f"v{s + k + 1}")
-        if k + 3 < 32:
-            e.ins("v_max3_f32", f"v{TB}", f"v{TB}", f"v{s + k + 2}", f"v{s + k + 3}")
-    e.ins("v_max_f32", f"v{TA}", f"v{TA}", f"v{TB}")
-    e.ins("v_mov_b32", f"v{TB}", f"v{TA}")
-    e.ins("v_permlane32_swap_b32", f"v{TA}", f"v{TB}", ndst=2)
-    e.ins("v_max_f32", f"v{TA}", f"v{TA}", f"v{TB}")
-    e.ins("v_cmp_lt_f32", "vcc", f"s{S_SLACK}", f"v{TA}")
-    e.raw(f"s_cbranch_vccnz .Lpf_rare_{p}_%=")
-    e.raw(f".Lpf_cont_{p}_%=:")
-
-def sm_exp_regs(e, s, q, T0, T1):
-    """exponentials, row sum and bf16 packing of logits 4q .. 4q+3 of the 16 in v[s:s+15]"""
+# ---- softmax
+# There is no row maximum in the loop.  The exponentials are taken against the running reference as it is; what says that the
+# reference must move is the sum of a group of them, which is needed anyway: a sum above 2^8 (or NaN) means that an exponent
+# may have left the range in which nothing is lost.  Up to there no bit depends on the reference (it is a whole number and every factor an exact
+# power of two).  The rare path then computes the group's logits again from K tile j, which stays in LDS until the iteration
+# ends, takes their maximum, moves the reference and repeats the group's exponentials, before any O^T instruction has
+# seen them.  A maximum of 32 logits is 20 vector instructions of the 139 an iteration of the dense loop had.
+def sm_exp_regs(e, s, q, T0, T1, BS, first):
+    """exponentials and bf16 packing of logits 4q .. 4q+3 of the 16 in v[s:s+15]; their sum goes to BS (`first`) or onto it"""
     for k in range(4):
         e.ins("v_exp_f32", f"v{s + 4 * q + k}", f"v{s + 4 * q + k}")
     e.ins("v_add_f32", f"v{T0}", f"v{s + 4 * q}", f"v{s + 4 * q + 1}")
     e.ins("v_add_f32", f"v{T1}", f"v{s + 4 * q + 2}", f"v{s + 4 * q + 3}")
     e.ins("v_cvt_pk_bf16_f32", f"v{s + 2 * q}", f"v{s + 4 * q}", f"v{s + 4 * q + 1}")
-    e.ins("v_add_f32", f"v{T0}", f"v{T0}", f"v{T1}")
+    e.ins("v_add_f32", f"v{BS if first else T0}", f"v{T0}", f"v{T1}")
     e.ins("v_cvt_pk_bf16_f32", f"v{s + 2 * q + 1}", f"v{s + 4 * q + 2}", f"v{s + 4 * q + 3}")
-    e.ins("v_add_f32", f"v{LSUM}", f"v{LSUM}", f"v{T0}")
+    if not first:
+        e.ins("v_add_f32", f"v{BS}", f"v{BS}", f"v{T0}")
 
-def sm_exp(e, p, mb, q):
-    T0, T1 = ((T0A, T1A), (T0B, T1B))[mb]   # the two blocks' instructions interleave: a pair of temporaries each
-    sm_exp_regs(e, S(p, mb), q, T0, T1)
+def sm_check(e, BS, name):
+    """the group's sum against the slack (a NaN takes the branch too), then onto the row sum"""
+    e.ins("v_cmp_nge_f32", "vcc", f"s{S_SLACK}", f"v{BS}")
+    e.raw(f"s_cbranch_vccnz .Lpf_rare_{name}_%=")
+    e.raw(f".Lpf_cont_{name}_%=:")
+    e.ins("v_add_f32", f"v{LSUM}", f"v{LSUM}", f"v{BS}")
 
-def rescale(e, sets):
+def row_max(e, regs, TA, TB):
+    """maximum of the listed logits of this lane's row, over both lanes that share it, into TA"""
+    regs = list(regs)
+    e.ins("v_max_f32", f"v{TA}", f"v{regs[0]}", f"v{regs[1]}")
+    for k in range(2, len(regs), 2):
+        e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{regs[k]}", f"v{regs[k + 1]}")
+    e.ins("v_mov_b32", f"v{TB}", f"v{TA}")
+    e.ins("v_permlane32_swap_b32", f"v{TA}", f"v{TB}", ndst=2)
+    e.ins("v_max_f32", f"v{TA}", f"v{TA}", f"v{TB}")
+
+def rescale(e, tmax, RD, RAL, sets):
     """the reference moves up by ceil(row maximum) (a whole number, so every factor is an exact power of
     two): O and the row sum shrink, the logit registers listed in `sets` move down"""
-    e.ins("v_ceil_f32", f"v{RD}", f"v{TA}")
+    e.ins("v_ceil_f32", f"v{RD}", f"v{tmax}")
     e.ins("v_max_f32", f"v{RD}", "0", f"v{RD}")               # delta = tmax > 0 ? ceil(tmax) : 0
     e.ins("v_exp_f32_e64", f"v{RAL}", f"-v{RD}")              # alpha = 2^-delta
     e.ins("v_add_f32", f"v{MREF}", f"v{MREF}", f"v{RD}")
@@ -422,18 +428,32 @@ def rescale(e, sets):
         for k in range(16):
             e.ins("v_sub_f32", f"v{s + k}", f"v{s + k}", f"v{RD}")
 
-def rare_path(p, started):
-    """Row maximum of tile j left the slack (rare): move the reference up by a whole number and
-    rescale what was accumulated against the old one (do_softmax() in tpa_prefill.hip).  `started`
-    = the blocks of tile j+1 whose first matrix instruction was issued before the branch: their
-    accumulation began at the old reference."""
+def rare_path(name, f, frag_load, set_address, temps, again, moved, redo):
+    """A group's sum left the slack behind matrix instruction f (do_softmax() in tpa_prefill.hip moves the reference by
+    the same rule).  `again` = (register, byte offset of its rows in a K buffer) of the blocks whose logits are computed again,
+    `moved` = the logits of later blocks whose accumulation began at the old reference, `redo` = the recorded exponentials that
+    were issued.  `temps` = the registers of the group's sum and its two temporaries, which `redo` writes anew.  The fragments that the
+    loop has read ahead are overwritten here and read again at the end."""
     e = Stream()
-    e.raw(f".Lpf_rare_{p}_%=:")
+    e.raw(f".Lpf_rare_{name}_%=:")
+    e.raw("s_waitcnt lgkmcnt(0)")
     e.nop(64)                        # matrix instructions in flight: their results and their operand reads
-    # nothing of tile j is packed yet: both its blocks move
-    rescale(e, [S(p, 0), S(p, 1)] + [S(1 - p, mb) for mb in started])
-    e.nop(4)
-    e.raw(f"s_branch .Lpf_cont_{p}_%=")
+    sum_, t0, t1 = temps
+    addr = set_address(e, t1)
+    for n in range(len(again) * NKS):
+        (s, off), kk = again[n // NKS], n % NKS
+        b = RING_BUFS[n % len(RING_BUFS)]
+        e.ins("ds_read_b128", vt(b), f"v{addr} offset:{off + kk * 32}")
+        e.ins("v_mfma_f32_32x32x16_bf16", vt(s, 16), vt(b), vt(Q(kk)), vt(NMREF, 16) if kk == 0 else vt(s, 16))
+    row_max(e, [s + k for s, _ in again for k in range(16)], t0, t1)
+    rescale(e, t0, sum_, t1, [s for s, _ in again] + moved)
+    for it in redo:
+        replay(e, it)
+    for n in range(f + 1, min(f + LA, NF - 1) + 1):
+        frag_load(e, n)
+    e.raw("s_waitcnt lgkmcnt(0)")
+    e.nop(16)
+    e.raw(f"s_branch .Lpf_cont_{name}_%=")
     return e.lines
 
 
@@ -445,31 +465,41 @@ def half(e, p, rare):
         emit_frag_load(e, f, p)
     slots = [[] for _ in range(NF)]
     N_QK = 2 * NKS
-    ga, gb, gc, gd = Rec(), Rec(), Rec(), Rec()
-    sm_max(ga, p)
-    n_max = len(ga.items)
-    for q in range(4):
-        sm_exp(ga, p, 0, q)
-    for q in range(4):
-        sm_exp(gb, p, 1, q)
+    sm, gc, gd = [Rec(), Rec()], Rec(), Rec()
+    for mb in range(2):              # the two blocks' instructions may interleave: a pair of temporaries each
+        for q in range(4):
+            sm_exp_regs(sm[mb], S(p, mb), q, (T0A, T0B)[mb], (T1A, T1B)[mb], (BS0, BS1)[mb], q == 0)
     write_tile(gc, False, p); issue_loads(gc, False)
     write_tile(gd, True, p); issue_loads(gd, True)
-    # P of keys 0-31 must be packed before the first O^T instruction, P of keys 32-63 before the
+    # P of keys 0-31 must be packed and its sum looked at before the first O^T instruction, P of keys 32-63 before the
     # O^T instructions of the second half of the tile
-    spread(ga.items, 0, N_QK - 1, slots)
-    spread(gb.items, N_QK // 2, N_QK + 2 * NDB - 1, slots)
+    end = N_QK + 2 * NDB
+    check = [end // 2 if end // 2 < N_QK else N_QK - 1, end - 1]
+    spread(sm[0].items, 0, check[0], slots)
+    spread(sm[1].items, check[0], check[1], slots)
+    for mb in range(2):
+        c = Rec()
+        sm_check(c, (BS0, BS1)[mb], f"{p}{mb}")
+        slots[check[mb]][0:0] = c.items if mb == 0 else []
+        slots[check[mb]] += c.items if mb == 1 else []
     spread(gc.items, N_QK, N_QK + 2 * NDB, slots)
     spread(gd.items, N_QK + 2 * NDB, NF, slots)
-    # the slot behind which the maximum's branch sits decides which blocks of tile j+1 have started
-    branch_slot = (n_max - 1) * (N_QK - 1) // len(ga.items)
-    assert branch_slot < N_QK // 2     # before the first exponential of block 1
-    rare[p] = sorted({qk_of(f)[0] for f in range(branch_slot + 1)})
     for f in range(NF):
         if f + LA < NF:
             emit_frag_load(e, f + LA, p)
         emit_mfma(e, f, p)
         for it in slots[f]:
             replay(e, it)
+    def address(e2, t):              # K tile j: the third buffer, beside the ones of tiles j+1 and j+2
+        e2.ins("s_sub_u32", "vcc_lo", f"0x{3 * KBUF:x}", f"s{S_KR}")
+        e2.ins("s_sub_u32", "vcc_lo", "vcc_lo", f"s{S_KWB}")
+        e2.ins("v_add_u32", f"v{t}", "vcc_lo", f"v{KFRAG0}")
+        return t
+    for mb in range(2):
+        # block 0's check comes before any exponential of block 1, whose logits only move; at block 1's, block 0 is in O
+        assert check[0] >= N_QK // 2 and check[0] < N_QK and check[1] == N_QK + 2 * NDB - 1
+        rare += rare_path(f"{p}{mb}", check[mb], lambda e2, n: emit_frag_load(e2, n, p), address, ((BS0, T0A, T1A), (BS1, T0B, T1B))[mb], [(S(p, mb), mb * 32 * KS * 2)],
+                          ([S(p, 1)] if mb == 0 else []) + [S(1 - p, 0), S(1 - p, 1)], sm[mb].items)
     # the K buffers rotate: next iteration reads what this one wrote beside, and writes the one after
     e.ins("s_mov_b32", f"s{S_KR}", f"s{S_KWB}")
     e.ins("s_add_u32", f"s{S_KWB}", f"s{S_KWB}", f"0x{KBUF:x}")
@@ -517,36 +547,6 @@ def r2_mfma(e, f, p):
         kk, db = divmod(k, NDB)
         pr = SET(ph // 2) + 4 * kk         # P fragment kk of the block lives in the registers of the logits it was made from
         e.ins("v_mfma_f32_32x32x16_bf16", vt(O(db), 16), vt(b), vt(pr), vt(O(db), 16))
-
-def r2_sm_max(e, p, blk):
-    """row maximum over the 16 logits of this lane's row in set blk, and the test against the slack"""
-    s = SET(blk)
-    e.ins("v_max3_f32", f"v{TA}", f"v{s}", f"v{s + 1}", f"v{s + 2}")
-    e.ins("v_max3_f32", f"v{TB}", f"v{s + 3}", f"v{s + 4}", f"v{s + 5}")
-    e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{s + 6}", f"v{s + 7}")
-    e.ins("v_max3_f32", f"v{TB}", f"v{TB}", f"v{s + 8}", f"v{s + 9}")
-    e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{s + 10}", f"v{s + 11}")
-    e.ins("v_max3_f32", f"v{TB}", f"v{TB}", f"v{s + 12}", f"v{s + 13}")
-    e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{s + 14}", f"v{s + 15}")
-    e.ins("v_max_f32", f"v{TA}", f"v{TA}", f"v{TB}")
-    e.ins("v_mov_b32", f"v{TB}", f"v{TA}")
-    e.ins("v_permlane32_swap_b32", f"v{TA}", f"v{TB}", ndst=2)
-    e.ins("v_max_f32", f"v{TA}", f"v{TA}", f"v{TB}")
-    e.ins("v_cmp_lt_f32", "vcc", f"s{S_SLACK}", f"v{TA}")
-    e.raw(f"s_cbranch_vccnz .Lpf_rare_{p}{blk}_%=")
-    e.raw(f".Lpf_cont_{p}{blk}_%=:")
-
-def r2_rare_path(p, blk):
-    """Row maximum of a block left the slack (rare).  The block's own logits are not packed yet; the
-    other set holds the partial sums of the next block, whose accumulation began at the old
-    reference (its first matrix instruction is always issued before the branch)."""
-    e = Stream()
-    e.raw(f".Lpf_rare_{p}{blk}_%=:")
-    e.nop(64)                        # matrix instructions in flight: their results and their operand reads
-    rescale(e, [SET(blk), SET(1 - blk)])
-    e.nop(4)
-    e.raw(f"s_branch .Lpf_cont_{p}{blk}_%=")
-    return e.lines
 
 def r2_rebuild(e, is_v, p):
     """K tile j+2 (into the buffer s_K2 names) or V tile j+1 (into buffer 1-p) from the B-factor rows
@@ -599,7 +599,7 @@ def r2_head_factors(e, p):
     e.ins("s_mul_i32", f"s{S_T1}", f"s{S_T0}", f"s{S_ATILE}")
     e.ins("buffer_load_ushort", f"v{A_PEND}", f"v{A_VOFF}", st(S_AB), f"s{S_T1} offen")
 
-def half_r2(e, p):
+def half_r2(e, p, rare):
     """iteration j with j & 1 == p"""
     e.ins("v_add_u32", f"v{KFA}", f"s{S_K0}", f"v{KFRAG0}")
     e.ins("v_add_u32", f"v{KFB}", f"s{S_K1}", f"v{KFRAG0}")
@@ -613,27 +613,30 @@ def half_r2(e, p):
         r2_frag_load(e, f, p)
     slots = [[] for _ in range(NF)]
     P1, P2, P3 = NKS, NKS + 2 * NDB, 2 * NKS + 2 * NDB     # first instruction of phases 1, 2, 3
-    g0, g0b, g1, g1b, gk, gv = Rec(), Rec(), Rec(), Rec(), Rec(), Rec()
-    # softmax of block 2j (set 0): maximum and the first 8 keys before the O^T instructions of keys
-    # 0-15 of the block, the other 8 keys before those of keys 16-31
-    r2_sm_max(g0, p, 0)
-    for q in range(2):
-        sm_exp_regs(g0, SET(0), q, T0A, T1A)
-    for q in range(2, 4):
-        sm_exp_regs(g0b, SET(0), q, T0B, T1B)
-    r2_sm_max(g1, p, 1)
-    for q in range(2):
-        sm_exp_regs(g1, SET(1), q, T0A, T1A)
-    for q in range(2, 4):
-        sm_exp_regs(g1b, SET(1), q, T0B, T1B)
+    # softmax of block 2j (set 0): the first 8 keys of a lane before the O^T instructions of keys 0-15 of the block, the
+    # other 8 keys before those of keys 16-31; each half with its sum and its look at it
+    sm = [[Rec(), Rec()], [Rec(), Rec()]]
+    gk, gv = Rec(), Rec()
+    for blk in range(2):
+        for q in range(4):
+            sm_exp_regs(sm[blk][q // 2], SET(blk), q, (T0A, T0B)[q // 2], (T1A, T1B)[q // 2], (BS0, BS1)[q // 2], q % 2 == 0)
     r2_rebuild(gk, False, p)
     r2_rebuild(gv, True, p)
     r2_head_factors(gv, p)
-    spread(g0.items, 0, P1, slots)
-    spread(g0b.items, P1 - NKS // 4, P1 + NDB, slots)
+    checks = []
+    for blk, (lo, hi) in enumerate(((0, P1), (P2, P3))):
+        first, second = hi - NKS // 4, hi + NDB - 1
+        spread(sm[blk][0].items, lo, first, slots)
+        spread(sm[blk][1].items, first, second, slots)
+        for hf, at in ((0, first), (1, second)):
+            c = Rec()
+            sm_check(c, (BS0, BS1)[hf], f"{p}{blk}{hf}")
+            if hf == 0:
+                slots[at][0:0] = c.items
+            else:
+                slots[at] += c.items
+            checks.append((blk, hf, at))
     spread(gk.items, P1, P2, slots)
-    spread(g1.items, P2, P3, slots)
-    spread(g1b.items, P3 - NKS // 4, P3 + NDB, slots)
     spread(gv.items, P3, NF, slots)
     for f in range(NF):
         if f + LA < NF:
@@ -641,6 +644,11 @@ def half_r2(e, p):
         r2_mfma(e, f, p)
         for it in slots[f]:
             replay(e, it)
+    for blk, hf, at in checks:
+        # the block is one half of K tile j; the other set holds the next block, begun at the old reference
+        rare += rare_path(f"{p}{blk}{hf}", at, lambda e2, n: r2_frag_load(e2, n, p), lambda e2, t: KFA, ((BS0, T0A, T1A), (BS1, T0B, T1B))[hf],
+                          [(SET(blk), blk * 32 * KS * 2)],
+                          [SET(1 - blk)], sm[blk][hf].items)
     # the K buffers rotate: (tile j, tile j+1, free) -> (tile j+1, tile j+2, free)
     e.ins("s_mov_b32", f"s{S_T0}", f"s{S_K0}")
     e.ins("s_mov_b32", f"s{S_K0}", f"s{S_K1}")
@@ -652,7 +660,7 @@ def half_r2(e, p):
 
 def main():
     e = Stream()
-    e.raw(f"s_mov_b32 s{S_SLACK}, 0x41000000")       # 8.0: the slack of the reference
+    e.raw(f"s_mov_b32 s{S_SLACK}, 0x43800000")       # 2^8: the slack of a group's sum
     if R2:
         e.raw(f"s_mov_b32 s{S_SELLO}, 0x05040100")   # v_perm_b32 selectors: low halves / high halves of two registers
         e.raw(f"s_mov_b32 s{S_SELHI}, 0x07060302")
@@ -662,36 +670,27 @@ def main():
     e.prime_vm(load_groups())
     n_vm = len(e.vm)
     rare_lines = []
-    if R2:
-        half_r2(e, 1)                                 # entry with an odd tile
-        e.raw(f"s_cmp_lt_u32 s{S_J}, s{S_END}")
-        e.raw("s_cbranch_scc0 .Lpf_done_%=")
-        half_r2(e, 0)
-        for p in (0, 1):
-            for blk in (0, 1):
-                rare_lines += r2_rare_path(p, blk)
-    else:
-        rare = {}
-        half(e, 1, rare)                              # entry with an odd tile
-        e.raw(f"s_cmp_lt_u32 s{S_J}, s{S_END}")
-        e.raw("s_cbranch_scc0 .Lpf_done_%=")
-        half(e, 0, rare)
-        for p in sorted(rare):
-            rare_lines += rare_path(p, rare[p])
+    iteration = half_r2 if R2 else half
+    iteration(e, 1, rare_lines)                       # entry with an odd tile
+    e.raw(f"s_cmp_lt_u32 s{S_J}, s{S_END}")
+    e.raw("s_cbranch_scc0 .Lpf_done_%=")
+    iteration(e, 0, rare_lines)
     assert len(e.vm) == n_vm, (len(e.vm), n_vm)       # the loads in flight are those the next iteration expects
     e.raw(f"s_cmp_lt_u32 s{S_J}, s{S_END}")
     e.raw("s_cbranch_scc1 .Lpf_loop_%=")
     e.raw("s_branch .Lpf_done_%=")
-    lines = e.lines + rare_lines
-    lines += [
+    lines = e.lines + [
         ".Lpf_done_%=:",
         "s_waitcnt vmcnt(0)",                             # the load registers go back to the compiler
         "s_nop 7", "s_nop 7",                             # ... and so do the accumulators
+        "s_branch .Lpf_out_%=",                           # past the rare paths, which the second file holds
     ]
-    with open(OUT, "w") as f:
-        f.write(f"// generated by gen_prefill_loop.py {D} {LOADER}: do not edit\n")
-        for ln in lines:
-            f.write(f'"{ln}\\n\\t"\n')
+    rare_lines.append(".Lpf_out_%=:")
+    for name, part in ((OUT, lines), (OUT.replace(".inc", "_rare.inc"), rare_lines)):
+        with open(name, "w") as f:
+            f.write(f"// generated by gen_prefill_loop.py {D} {LOADER}: do not edit\n")
+            for ln in part:
+                f.write(f'"{ln}\\n\\t"\n')
     # registers the loop uses beyond its operands (the state tuple is an in/out operand)
     ring = [b + k for b in RING_BUFS for k in range(4)]
     named = set().union(*(regs_of(ln) for ln in lines))     # a head size with one loader pass leaves some unused

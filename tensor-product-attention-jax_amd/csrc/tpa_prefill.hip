@@ -870,6 +870,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
       if constexpr (D == 128) {
         asm volatile(
 #include "gen/prefill_loop_128_dense.inc"
+#include "gen/prefill_loop_128_dense_rare.inc"
             : "+{v[0:15]}"(sa0), "+{v[16:31]}"(sa1), "+{v[32:47]}"(sb0), "+{v[48:63]}"(sb1), "+{v[64:79]}"(nmref[0]),
               "+{v[80:95]}"(o[0][0]), "+{v[96:111]}"(o[0][1]), "+{v[112:127]}"(o[0][NDB > 2 ? 2 : 0]), "+{v[128:143]}"(o[0][NDB > 2 ? 3 : 0]),
               "+{v[176:183]}"(kv_k), "+{v[184:191]}"(kv_v), "+{v[204:219]}"(st16), "+{s[32:47]}"(sc16)
@@ -880,6 +881,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
       } else {
         asm volatile(
 #include "gen/prefill_loop_64_dense.inc"
+#include "gen/prefill_loop_64_dense_rare.inc"
             : "+{v[0:15]}"(sa0), "+{v[16:31]}"(sa1), "+{v[32:47]}"(sb0), "+{v[48:63]}"(sb1), "+{v[64:79]}"(nmref[0]),
               "+{v[80:95]}"(o[0][0]), "+{v[96:111]}"(o[0][1]),
               "+{v[176:183]}"(kv_k), "+{v[184:191]}"(kv_v), "+{v[204:219]}"(st16), "+{s[32:47]}"(sc16)
@@ -955,6 +957,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
       if constexpr (D == 128) {
         asm volatile(
 #include "gen/prefill_loop_128_r2.inc"
+#include "gen/prefill_loop_128_r2_rare.inc"
             : "+{v[0:15]}"(set0), "+{v[16:31]}"(set1), "+{v[32:47]}"(nmref[0]),
               "+{v[48:63]}"(o[0][0]), "+{v[64:79]}"(o[0][1]), "+{v[80:95]}"(o[0][NDB > 2 ? 2 : 0]), "+{v[96:111]}"(o[0][NDB > 2 ? 3 : 0]),
               "+{v[144:159]}"(kv_k), "+{v[160:175]}"(kv_v), "+{v[188:203]}"(st16), "+{s[32:47]}"(sc16)
@@ -967,6 +970,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
         u32x8 kv_v8 = __builtin_shufflevector(kv_v, kv_v, 0, 1, 2, 3, 4, 5, 6, 7);
         asm volatile(
 #include "gen/prefill_loop_64_r2.inc"
+#include "gen/prefill_loop_64_r2_rare.inc"
             : "+{v[0:15]}"(set0), "+{v[16:31]}"(set1), "+{v[32:47]}"(nmref[0]),
               "+{v[48:63]}"(o[0][0]), "+{v[64:79]}"(o[0][1]),
               "+{v[144:151]}"(kv_k8), "+{v[160:167]}"(kv_v8), "+{v[188:203]}"(st16), "+{s[32:47]}"(sc16)
