@@ -232,15 +232,15 @@ struct DecodeLds {
   static constexpr int kReduce = 32 * kRedStride * 2 + 128;  // fp32 O^T + m + l, in uint16 units
   static constexpr int kPerWave = kWave > kReduce ? kWave : kReduce;
   static constexpr size_t kBytes = (size_t)kWaves * kPerWave * sizeof(uint16_t);
-  // with NQ > 1 query rows per workgroup: plus their Q fragments (NQ rows x D/16 steps x 64 lanes x 16 bytes)
-  static constexpr size_t bytes(int nq) { return kBytes + (nq > 1 ? (size_t)nq * (D / 16) * 64 * 16 : 0); }
+  // with several query rows per workgroup: plus their Q fragments (NQ sets x D/16 steps x 64 lanes x 16 bytes)
+  static constexpr size_t bytes(int nq, bool side) { return kBytes + (nq > 1 || side ? (size_t)nq * (D / 16) * 64 * 16 : 0); }
 };
 
 // At head size 64 and from rank 4 on two workgroups fit a compute unit, which the compiler has to be told: at 258 registers
 // instead of 256 rank 8 lost the second one (64 heads, two rows per workgroup: 48 x 4096 keys, eight rows 544 -> 707 us; 4 x 1024
 // rows and keys without K and V 2.42 -> 3.15 ms; 2.10 so, with 204).
 constexpr int min_waves(int d, int rk) { return d == 64 && rk >= 4 ? 2 : 1; }
-template <int D, int RK, bool PAGED, int NQ, Reads READS>
+template <int D, int RK, bool PAGED, int NQ, Reads READS, bool SIDE = false>
 __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(DecodeParams p) {
   constexpr int CPR = D / 8;               // 16-byte chunks per B row
   constexpr int RPI = 64 / CPR;            // B rows per load instruction
@@ -256,18 +256,21 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
   // workgroup id -> (key range x, query row qi): ids are dealt to the 8 XCDs round-robin, and the
   // rows of one query token group read the same cache slice, so they get ids that are 8 apart
   // (same XCD, same L2) and next to each other in launch order (resident together)
-  // A workgroup serves NQ query rows from one pass over its cache blocks (each staged block is
-  // used NQ times); with an odd row count the last group's second row repeats the first and is
-  // not stored.
-  const int nqg = (p.lq + NQ - 1) / NQ;  // groups of NQ query rows
+  // A workgroup serves NQ column sets from one pass over its cache blocks (each staged block is used NQ times).  A set is
+  // the heads of one query row, or (SIDE: 8 or 16 heads) those of 32 / H rows side by side in the 32 columns; rows past the
+  // last one repeat it and are not stored.
+  const int rps = SIDE ? 32 / p.H : 1;            // rows per set
+  const int rpw = NQ * rps;                       // rows per workgroup
+  const int nqg = (p.lq + rpw - 1) / rpw;         // groups of as many query rows
   const int gid = blockIdx.x, grp = gid / (8 * nqg), rem = gid - grp * 8 * nqg;
-  const int qi0 = NQ * (rem >> 3), x = grp * 8 + (rem & 7);
+  const int qi0 = rpw * (rem >> 3), x = grp * 8 + (rem & 7);
   int b, split, S;
   if (!range_of(p, x, b, split, S)) return;  // the grid is rounded up to whole groups of 8 ranges
   const int h0 = blockIdx.y * 32;
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
-  const int hl = min(h0 + i, p.H - 1);  // this lane's head (clamped: lanes past H idle along)
+  const int ci = SIDE ? i / p.H : 0;                           // this lane's row of a set
+  const int hl = SIDE ? i - ci * p.H : min(h0 + i, p.H - 1);  // and its head (clamped: lanes past H idle along)
 
   uint16_t* lds = smem + w * DecodeLds<D>::kPerWave;
   uint16_t* lds_bk = lds;
@@ -278,26 +281,41 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
   const TileAt<D> at(l);
 
   // ---- Qm^T fragments: requested ahead of the cache's first blocks, finished while those are in flight.
-  // With one query row they stay in registers; with NQ rows wave r builds row r's fragments once
-  // and parks them in LDS behind the waves' staging regions (fragment (r, ks) of lane l at
-  // [(r NKS + ks) 64 + l]), from where every wave reads them as it needs them: the registers go to
-  // the NQ accumulator sets instead.
+  // With one query row they stay in registers; with several wave r builds row r's fragments once
+  // and parks them in LDS behind the waves' staging regions (fragment (set, ks) of lane l at
+  // [(set NKS + ks) 64 + l], written by the lanes whose row it is: another row's infinities never
+  // meet theirs), from where every wave reads them: one set into its registers, two as it needs them,
+  // when the registers go to the accumulators instead.
   bf16x8 qf[NQ == 1 ? NKS : 1];
   u32x4* const lds_q = reinterpret_cast<u32x4*>(smem + kWaves * DecodeLds<D>::kPerWave);
-  const int qi_build = NQ == 1 ? qi0 : min(qi0 + w, p.lq - 1);
-  const uint16_t* const qa_row = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qi_build * p.qa.stride_l + hl;
-  const uint16_t* const qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qi_build * p.qb.stride_l;
-  auto build_q = [&](const QRaw<D>& raw) __attribute__((always_inline)) {
-    if constexpr (NQ == 1) {
+  const uint16_t* qa_row;
+  const uint16_t* qb_row;
+  auto q_row = [&](int row) __attribute__((always_inline)) {
+    qa_row = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)row * p.qa.stride_l + hl;
+    qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)row * p.qb.stride_l;
+  };
+  q_row(NQ == 1 && !SIDE ? qi0 : min(qi0 + w, p.lq - 1));
+  auto build_q = [&](QRaw<D> raw) __attribute__((always_inline)) {
+    if constexpr (NQ == 1 && !SIDE) {
       finish_q_fragments<D>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, l, lds, at, qf);
     } else {
-      if (w < NQ) {
+      for (int r = w; r < rpw; r += kWaves) {
         bf16x8 tmp[NKS];
         finish_q_fragments<D>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, l, lds, at, tmp);
+        const int set = SIDE ? r / rps : r;
+        if (!SIDE || ci == r - set * rps) {
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) lds_q[(w * NKS + ks) * 64 + l] = __builtin_bit_cast(u32x4, tmp[ks]);
+          for (int ks = 0; ks < NKS; ++ks) lds_q[(set * NKS + ks) * 64 + l] = __builtin_bit_cast(u32x4, tmp[ks]);
+        }
+        if (!SIDE || r + kWaves >= rpw) break;
+        q_row(min(qi0 + r + kWaves, p.lq - 1));
+        raw = load_q_factors<D>(qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, 0, p.rq, l);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the cache's loads stay in flight
+      if constexpr (NQ == 1) {
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, lds_q[ks * 64 + l]);
+      }
     }
   };
 
@@ -310,9 +328,9 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
   int row_last[NQ], len_b = 0;
 #pragma unroll
   for (int r = 0; r < NQ; ++r) {
-    const int len_r = max(0, min(len_all, min(qi0 + r, p.lq - 1) + p.climit + (p.cbr ? len_all - p.lq_total : 0)));
-    row_last[r] = len_r * RK - 1;
-    len_b = max(len_b, len_r);
+    auto keys_of = [&](int row) { return max(0, min(len_all, min(row, p.lq - 1) + p.climit + (p.cbr ? len_all - p.lq_total : 0))); };
+    row_last[r] = keys_of(qi0 + r * rps + ci) * RK - 1;
+    len_b = max(len_b, keys_of(qi0 + r * rps + rps - 1));  // a row sees no fewer keys than the one before it
   }
   const int blk_begin = part;
   const int blk_end = (len_b * RK + kRowsPerBlock - 1) / kRowsPerBlock;  // 32-row blocks of its cache
@@ -332,7 +350,8 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
 
   // loader lane roles
   const int lb_row = l / CPR, lb_c = l % CPR;             // B tiles: row within the instruction, chunk
-  const int la_row = l >> 2, la_c = min(l & 3, a_chunks - 1);  // A tiles: 16 rows per instruction
+  // A tiles: 16 rows per instruction; 8 or 16 heads with their rows side by side fill the 32 columns by repeating
+  const int la_row = l >> 2, la_c = SIDE ? (l & 3) & (a_chunks - 1) : min(l & 3, a_chunks - 1);
 
   // two register sets: while one block is staged and consumed, two more are in flight (one set
   // with NQ rows, whose accumulators take the room and whose blocks take NQ times as long to
@@ -510,7 +529,7 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
       // split over waves and ranges, and every rescaling factor (here, in the wave merge, in the merge of
       // the key ranges) is an exact power of two
       const float m_new = fmaxf(m[r], __builtin_ceilf(tmax));
-      const float m_use = NQ > 1 && m_new == -INFINITY ? 0.f : m_new;
+      const float m_use = (NQ > 1 || SIDE) && m_new == -INFINITY ? 0.f : m_new;
       if (NQ == 1 && blk == blk_begin) {
         m[r] = m_new;  // nothing to rescale yet
       } else if (__any(m_new > m[r])) {
@@ -578,10 +597,11 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
   float* red_o = reinterpret_cast<float*>(lds);  // [32 heads][RS]
   float* red_m = red_o + 32 * RS;
   float* red_l = red_m + 32;
-  const int nh = min(32, p.H - h0);
 #pragma unroll
   for (int r = 0; r < NQ; ++r) {
-    if (qi0 + r >= p.lq) break;  // uniform: the repeated row of an odd count
+    const int qr = qi0 + r * rps;
+    if (qr >= p.lq) break;  // uniform: a set of repeated rows
+    const int nh = SIDE ? min(32, (p.lq - qr) * p.H) : min(32, p.H - h0);  // columns that are stored: heads, or (row, head)
     const float ltot = halves_sum(lsum[r]);
     __syncthreads();  // the staging (or the previous row's merge) has been read by every wave
 #pragma unroll
@@ -596,7 +616,7 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
     }
     __syncthreads();
 
-    const int64_t pbase = ((int64_t)x * p.lq + qi0 + r) * p.H + h0;
+    const int64_t pbase = ((int64_t)x * p.lq + qr) * p.H + h0;
 #pragma unroll(NQ == 1 ? 4 : 1)
     for (int idx = tid; idx < nh * (D / 4); idx += kWaves * 64) {
       const int hh = idx / (D / 4), d = 4 * (idx % (D / 4));
@@ -973,14 +993,16 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   return p;
 }
 
-template <int D, int RK, bool PAGED, int NQ, Reads READS>
+template <int D, int RK, bool PAGED, int NQ, Reads READS, bool SIDE = false>
 int launch_decode_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
   const DecodeParams p = decode_params<RK>(a, ranges, rows);
-  auto kern = decode_kernel<D, RK, PAGED, NQ, READS>;
+  auto kern = decode_kernel<D, RK, PAGED, NQ, READS, SIDE>;
   static bool configured[kMaxDevices] = {};
-  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), DecodeLds<D>::bytes(NQ)); rc != TPA_OK) return rc;
-  dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * ((a->lq + NQ - 1) / NQ), (a->H + 31) / 32);
-  hipLaunchKernelGGL(kern, grid, dim3(kWaves * 64), DecodeLds<D>::bytes(NQ), stream, p);
+  const size_t lds = DecodeLds<D>::bytes(NQ, SIDE);
+  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
+  const int rpw = NQ * (SIDE ? 32 / a->H : 1);
+  dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * ((a->lq + rpw - 1) / rpw), (a->H + 31) / 32);
+  hipLaunchKernelGGL(kern, grid, dim3(kWaves * 64), lds, stream, p);
   if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
   hipLaunchKernelGGL((decode_merge_kernel<D, uint16_t>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p, static_cast<uint16_t*>(a->o), a->lse, 1.f / (float)RK);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
@@ -1010,6 +1032,11 @@ int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream,
   return launch_decode_f32_t<D, RK, false>(a, ranges, stream, rows);
 }
 
+// 8 and 16 heads leave columns of the matrix instructions to other query rows: 32 / H rows then cost what one does, with the
+// registers of one row (two sets of loads in flight).  Decode and merge, us, two rows of one set of columns each / side by side:
+// 64 x 8192 keys, 16 heads of 128, four rows 166.7 / 124.0, two rows 101.7 / 100.8 (HBM); rank 8, head size 64, four rows 348 / 245; 8
+// heads, rank 4, eight rows 308 / 203; step of 48 paged sequences of 2046 .. 4096 keys, 16 heads of 128, four tokens 91.2 / 75.7.
+// Two sets of rows side by side in one workgroup are slower (158.7 at the first shape): one set of loads in flight.
 // One row group per cache slice: each byte is used once and the loads are marked non-temporal (the whole call 5.1 -> 5.75 TB/s).
 // Several (more query rows than a workgroup serves): the groups' workgroups run side by side on one XCD and the later one is
 // meant to find the slice in its L2, so the loads stay ordinary (four rows at the c4 shape: 1022 MB fetched with non-temporal
@@ -1025,6 +1052,10 @@ int launch_decode_rows(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream
     if constexpr (RK >= 16)
       if (a->H > 32) return launch_decode_t<D, RK, PAGED, 1, Reads::kOrdinary>(a, ranges, stream, rows);
     return launch_decode_t<D, RK, PAGED, 1, Reads::kStreaming>(a, ranges, stream, rows);
+  }
+  if (a->H == 8 || a->H == 16) {
+    if (a->lq <= 32 / a->H) return launch_decode_t<D, RK, PAGED, 1, Reads::kStreaming, true>(a, ranges, stream, rows);
+    return launch_decode_t<D, RK, PAGED, 1, Reads::kOrdinary, true>(a, ranges, stream, rows);
   }
   if (a->lq == 2 && (a->H <= 32 || RK < 4)) return launch_decode_t<D, RK, PAGED, 2, Reads::kStreaming>(a, ranges, stream, rows);
   return launch_decode_t<D, RK, PAGED, 2, Reads::kOrdinary>(a, ranges, stream, rows);
