@@ -32,9 +32,6 @@ constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
 enum class Reads { kOrdinary, kStreaming, kFar };
 constexpr int64_t kFarthestRow = 1 << 25;  // elements between neighbouring rows, at most, for the first two
 constexpr int kMinKeys = kWaves * kRowsPerBlock / 2;  // keys of a range with one block of rank 2 per wave
-// Several query rows make the partials and their merge dearer: ranges of two blocks per wave then (step of 6 sequences of
-// 1022 .. 2048 tokens, four query tokens each: 31.9 us; 33.4 with ranges of one block).
-inline int min_keys(int lq) { return lq >= 2 ? 2 * kMinKeys : kMinKeys; }
 
 
 struct DecodeParams {
@@ -53,7 +50,7 @@ struct DecodeParams {
   int lq_total;
   int S;           // key ranges per batch entry (slots == 0)
   int slots;       // > 0: the ranges are dealt by the batch entries' lengths, this many at most (plan_ranges)
-  int min_keys;    // slots > 0: no range shorter than this while it can be helped
+  float round_keys;  // slots > 0: ranges are this many keys long, or a multiple (a block for each wave); 0: any length
   float qscale;    // sm_scale * log2(e) / (rq * rk)
 };
 
@@ -66,6 +63,9 @@ struct DecodeParams {
 // merge each work the plan out and must arrive at the same one, so nothing in it is left to the compiler: the products
 // and sums are not contracted but where `fmaf` says so, and conversions, quotients and `ceilf` are exact or round once.
 // 48 paged sequences of 2047 .. 4096 tokens (32 heads of 128, rank 2): 67.7 us with equal counts (288 workgroups), 43.4 so.
+// At head size 128 a range is a whole number of rounds of its four waves: one of a round and a bit takes two, and a few more partials
+// to merge (steps, us, any length / whole rounds: 24 x 1024 tokens, 32 heads 23.9 / 23.0, four tokens of 6 x 2048, 16 heads 23.4 / 22.7, 4 x
+// 8192, 32 heads 24.2 / 23.4, 48 x 4096 50.4 / 50.1).  At 64 a round is short and fewer workgroups weigh more (40 x 1024, 16 heads 18.6 / 18.9).
 constexpr int kMaxPlanEntries = 64;
 // What costs time in it is latency, twice per call (here and in the merge): sums over the lanes go through DPP adds (through
 // the LDS permute they were 1 400 cycles), and the search takes four instructions per entry.  With both, append, decode and
@@ -81,14 +81,16 @@ __device__ __forceinline__ int wave_prefix_sum(int x) {  // lane i: sum of lanes
   return add_from<0x143, 0xc>(x);  // row_bcast 31: lane 31 to rows 2 and 3
 }
 struct RangePlan { int S, first; };  // of batch entry `lane`: its number of ranges and the first one's index
-__device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, int min_keys) {
+__device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, float round_keys) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
   const int total = __builtin_amdgcn_readlane(wave_prefix_sum(len), 63);
-  const float shortest = fmaxf((float)total / (float)slots, (float)min_keys);
+  const float shortest = fmaxf((float)total / (float)slots, (float)kMinKeys);
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
-  const float inv = 1.f / fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
+  float length = fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
+  if (round_keys > 0.f) length = ceilf(length / round_keys) * round_keys;
+  const float inv = 1.f / length;
   // eight entries at a time, their chains side by side; an entry without keys counts as one of one key (one range), and so do
   // the lanes past the last entry, which are taken off again
   const uint32_t keys = __float_as_uint((float)max(len, 1));
@@ -117,7 +119,7 @@ __device__ __forceinline__ bool range_of(const DecodeParams& p, int x, int& b, i
     split = x - b * S;
     return x < p.B * S;
   }
-  const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.min_keys);
+  const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.round_keys);
   const int lane = threadIdx.x & 63;
   b = __popcll(__ballot(lane < p.B && plan.first <= x)) - 1;
   S = __builtin_amdgcn_readlane(plan.S, b);
@@ -905,57 +907,76 @@ __global__ __launch_bounds__(kWaves * 64) void decode_f32_kernel(DecodeParams p)
 }
 
 // Merge the key ranges: o = sum_s f_s O_s / (Rk sum_s f_s l_s), f_s = 2^(m_s - max m); lse = ln of the total.
-template <int D, typename TO>
-__global__ __launch_bounds__(D) void decode_merge_kernel(DecodeParams p, TO* o, float* lse, float inv_rk) {
-  const int h = blockIdx.y, H = p.H;
-  const int d = threadIdx.x;
+// What it takes is a few dependent trips to memory, so a thread takes four elements of up to four ranges in one trip and SL groups of
+// threads share the ranges of a (row, head): the launcher takes as many as they need for one trip (above 4 SL ranges, several).
+// One element of 8 or 24 ranges a thread and trip / this, decode and merge, us, 24 ranges: 1 x 1500 keys, 16 heads of 128, four rows
+// 11.5 / 10.6; 63: 1 x 20 000 26.3 / 15.1; 47: 1 x 6000, 32 heads 17.3 / 11.4; 18: 3 x 9000 19.7 / 15.8; 4: 64 x 8192 108.2 / 107.0;
+// dealt by length, with the append: 4 paged sequences of 4096 .. 8192 29.6 / 23.4, 48 of 2048 .. 4096 51.8 / 50.1.
+template <int D, typename TO, int SL>
+__global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, TO* o, float* lse, float inv_rk) {
+  constexpr int LPR = D / 4, SLOTS = 256 / LPR, HB = SLOTS / SL, U = 4;  // lanes per row; (head, group) slots; heads; ranges per trip
+  __shared__ f32x4 red_o[SL > 1 ? 256 : 1];
+  __shared__ float red_m[SLOTS], red_l[SLOTS];
+  const int H = p.H, tid = threadIdx.x, c = tid % LPR, place = tid / LPR, group = place % SL;
+  const int h = blockIdx.y * HB + place / SL, h_ld = min(h, H - 1);
   const int b = blockIdx.x / p.lq, qi = blockIdx.x % p.lq;
   int S = p.S, first = b * S;  // the batch entry's ranges
   if (p.slots > 0) {
-    const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.min_keys);
+    const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.round_keys);
     S = __builtin_amdgcn_readlane(plan.S, b);
     first = __builtin_amdgcn_readlane(plan.first, b);
   }
-  // ranges are taken eight at a time with all their loads in flight together (one round trip to memory), or 24 at a
-  // time where all entries have the same number of more than eight.  Decode and merge by 8 / 16 / 24 / 32, us, one sequence,
-  // 16 heads of 128, 64 keys per range: 9 to 16 ranges 10.6 / 9.8 / 10.4 / 11.0, 17 to 24 11.7 / 11.3 / 10.5 / 11.0, 25 to 32
-  // 12.9 / 11.4 / 12.4 / 11.1, 40 and 48 15.0 / 13.3 / 12.8 / 13.8, 64 17.4 / 14.9 / 14.8 / 14.0; the same order for 32 heads,
-  // four sequences, head size 64, four query rows and fp32.  With ranges dealt by length, where entries of few ranges pay for
-  // the empty places (6 x 4 rows of about 21 ranges), 24 lose: 4.5 us by eight, 5.4 by 24.
-  // A running (max, sum, acc) triple carries across groups
-  float mmax = -INFINITY, acc = 0.f, lacc = 0.f;
-  auto merge = [&](auto group_c) __attribute__((always_inline)) {
-    constexpr int G = decltype(group_c)::value;
-    for (int s0 = 0; s0 < S; s0 += G) {
-      float ms[G], ls[G], os[G];
+  float mmax = -INFINITY, lacc = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = group; s0 < S; s0 += U * SL) {  // a running (max, sum, acc) triple carries across the trips
+    float ms[U], ls[U];
+    f32x4 os[U];
 #pragma unroll
-      for (int q = 0; q < G; ++q) {
-        const int s = min(s0 + q, S - 1);
-        const int64_t idx = ((int64_t)(first + s) * p.lq + qi) * H + h;
-        ms[q] = s0 + q < S ? p.part_m[idx] : -INFINITY;
-        ls[q] = p.part_l[idx];
-        os[q] = p.part_o[idx * D + d];
-      }
-      float gmax = mmax;
-#pragma unroll
-      for (int q = 0; q < G; ++q) gmax = fmaxf(gmax, ms[q]);
-      const float carry = mmax == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mmax - gmax);
-      acc *= carry;
-      lacc *= carry;
-#pragma unroll
-      for (int q = 0; q < G; ++q) {
-        const float f = ms[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[q] - gmax);
-        acc += f * os[q];
-        lacc += f * ls[q];
-      }
-      mmax = gmax;
+    for (int q = 0; q < U; ++q) {
+      const int s = s0 + q * SL;
+      const int64_t idx = ((int64_t)(first + min(s, S - 1)) * p.lq + qi) * H + h_ld;
+      ms[q] = p.part_m[idx];
+      ls[q] = p.part_l[idx];
+      os[q] = *reinterpret_cast<const f32x4*>(p.part_o + idx * D + 4 * c);
+      if (s >= S) ms[q] = -INFINITY;
     }
-  };
-  if (S <= 8 || p.slots > 0) merge(std::integral_constant<int, 8>{});
-  else merge(std::integral_constant<int, 24>{});
+    float gmax = mmax;
+#pragma unroll
+    for (int q = 0; q < U; ++q) gmax = fmaxf(gmax, ms[q]);
+    const float carry = mmax == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mmax - gmax);
+    acc *= carry;
+    lacc *= carry;
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const float f = ms[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[q] - gmax);
+      acc += f * os[q];
+      lacc += f * ls[q];
+    }
+    mmax = gmax;
+  }
+  if constexpr (SL > 1) {
+    red_o[tid] = acc;
+    if (c == 0) { red_m[place] = mmax; red_l[place] = lacc; }
+    __syncthreads();
+    if (group != 0) return;
+    float ms[SL];
+#pragma unroll
+    for (int q = 0; q < SL; ++q) { ms[q] = red_m[place + q]; mmax = fmaxf(mmax, ms[q]); }
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    lacc = 0.f;
+#pragma unroll
+    for (int q = 0; q < SL; ++q) {
+      const float f = ms[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[q] - mmax);
+      acc += f * red_o[tid + q * LPR];
+      lacc += f * red_l[place + q];
+    }
+  }
+  if (h >= H) return;
   // this call's rows are row0 .. row0 + lq - 1 of the lq_total rows of o and lse
-  store_from_f32(o + (((int64_t)b * p.lq_total + p.row0 + qi) * H + h) * D + d, acc * inv_rk / lacc);
-  if (lse && d == 0) lse[((int64_t)b * H + h) * p.lq_total + p.row0 + qi] = (mmax + __builtin_amdgcn_logf(lacc)) * kLn2;
+  TO* const out = o + (((int64_t)b * p.lq_total + p.row0 + qi) * H + h) * D + 4 * c;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) store_from_f32(out + e, acc[e] * inv_rk / lacc);
+  if (lse && c == 0) lse[((int64_t)b * H + h) * p.lq_total + p.row0 + qi] = (mmax + __builtin_amdgcn_logf(lacc)) * kLn2;
 }
 
 size_t workspace_bytes(int B, int lq, int H, int D, int S) {
@@ -981,7 +1002,7 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   p.part_o = ws; p.part_m = ws + no; p.part_l = ws + no + nm;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq;
   p.S = ranges.S; p.slots = ranges.slots;
-  p.min_keys = min_keys(a->lq);
+  p.round_keys = a->dv == 128 ? kWaves * kRowsPerBlock / (float)RK : 0.f;
   p.kvlen = a->kv_lengths;
   p.climit = a->causal ? causal_offset_of(a) + 1 + rows.row0 : a->lk;
   p.cbr = a->causal == TPA_CAUSAL_BOTTOM_RIGHT;
@@ -991,6 +1012,22 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   p.page_shift = page_rows > 0 && (page_rows & (page_rows - 1)) == 0 ? __builtin_ctz(page_rows) : -1;
   p.qscale = a->sm_scale * kLog2e / ((float)a->rq * (float)RK);
   return p;
+}
+
+template <int D, typename TO, int SL>
+int launch_merge_t(const TpaFwdArgs* a, const DecodeParams& p, float inv_rk, hipStream_t stream) {
+  constexpr int HB = 256 / (D / 4) / SL;
+  hipLaunchKernelGGL((decode_merge_kernel<D, TO, SL>), dim3(a->B * a->lq, (a->H + HB - 1) / HB), dim3(256), 0, stream, p, static_cast<TO*>(a->o), a->lse, inv_rk);
+  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+}
+
+template <int D, typename TO>
+int launch_merge(const TpaFwdArgs* a, const DecodeParams& p, float inv_rk, hipStream_t stream) {
+  const int S = p.slots > 0 ? (p.slots + p.B - 1) / p.B : p.S;  // dealt by length: on average
+  if (S <= 4) return launch_merge_t<D, TO, 1>(a, p, inv_rk, stream);
+  if (S <= 8) return launch_merge_t<D, TO, 2>(a, p, inv_rk, stream);
+  if (S <= 16) return launch_merge_t<D, TO, 4>(a, p, inv_rk, stream);
+  return launch_merge_t<D, TO, 8>(a, p, inv_rk, stream);
 }
 
 template <int D, int RK, bool PAGED, int NQ, Reads READS, bool SIDE = false>
@@ -1004,8 +1041,7 @@ int launch_decode_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, R
   dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * ((a->lq + rpw - 1) / rpw), (a->H + 31) / 32);
   hipLaunchKernelGGL(kern, grid, dim3(kWaves * 64), lds, stream, p);
   if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
-  hipLaunchKernelGGL((decode_merge_kernel<D, uint16_t>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p, static_cast<uint16_t*>(a->o), a->lse, 1.f / (float)RK);
-  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+  return launch_merge<D, uint16_t>(a, p, 1.f / (float)RK, stream);
 }
 
 template <int D, int RK, bool PAGED>
@@ -1017,8 +1053,7 @@ int launch_decode_f32_t(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t strea
   dim3 grid((ranges.count(a->B) + 7) / 8 * 8 * a->lq, (a->H + 31) / 32);
   hipLaunchKernelGGL(kern, grid, dim3(kWaves * 64), DecodeF32Lds<D>::kBytes, stream, p);
   if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
-  hipLaunchKernelGGL((decode_merge_kernel<D, float>), dim3(a->B * a->lq, a->H), dim3(D), 0, stream, p, static_cast<float*>(a->o), a->lse, 1.f / (float)RK);
-  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+  return launch_merge<D, float>(a, p, 1.f / (float)RK, stream);
 }
 
 template <int D, int RK>
@@ -1096,13 +1131,18 @@ int default_splits(int B, int lq, int lk, int H, int rows_per_group = 2) {
 // How a launch splits the keys if the caller leaves it to us, with partials for B * default_splits ranges at hand.
 // With lengths per batch entry the ranges are dealt by them; otherwise all entries get one count, which fills the chip
 // at most once: 288 workgroups take two rounds, the second nearly empty (48 x 4096 keys, 32 heads of 128: 6 ranges each 69.5 us, 5 48.6).
+// What some wave has to do is a whole number of blocks, so there are no more ranges than that number needs: the others would only
+// be partials to merge (1 x 20 000 keys, 16 heads of 128: 63 ranges of up to ten blocks per wave 34.3 us, fewer 26.3; 3 x 9000, 32 heads
+// 22.1 / 19.7; five paged sequences dealt by length, 4 x 8192 keys 32.2 / 29.6, 24 x 1024 25.0 / 23.2).
 KeyRanges choose_ranges(const TpaFwdArgs* a, int rows_per_group) {
   const int S = default_splits(a->B, a->lq, a->lk, a->H, rows_per_group);
   const int per_range = (a->lq + rows_per_group - 1) / rows_per_group * ((a->H + 31) / 32);  // workgroups of one range
   if (a->kv_lengths && a->B <= kMaxPlanEntries)
     return KeyRanges{S, std::min(std::max(a->B, 256 / per_range), a->B * S)};
-  const int most = (a->lk + min_keys(a->lq) - 1) / min_keys(a->lq);
-  return KeyRanges{std::max(1, (int)std::min<int64_t>(std::min(S, most), 256 / ((int64_t)a->B * per_range))), 0};
+  const int most = (a->lk + kMinKeys - 1) / kMinKeys;
+  const int n = std::max(1, (int)std::min<int64_t>(std::min(S, most), 256 / ((int64_t)a->B * per_range)));
+  const int64_t blocks = ((int64_t)a->lk * a->rk + kRowsPerBlock - 1) / kRowsPerBlock, rounds = (blocks + kWaves * n - 1) / (kWaves * n);
+  return KeyRanges{(int)((blocks + kWaves * rounds - 1) / (kWaves * rounds)), 0};
 }
 
 }  // namespace
