@@ -36,7 +36,7 @@ namespace tpa {
 namespace {
 
 constexpr int kTK = 64;   // keys per tile
-constexpr int kBQ = 256;  // query rows per workgroup: 8 blocks of 32, one per wave
+constexpr int kBQ = 256;  // query rows per workgroup: 8 blocks of 32, one per wave (or half of them, see wants_four_waves)
 
 enum { LOAD_TPA_R2 = 0, LOAD_TPA_ANY = 1, LOAD_DENSE = 2 };
 
@@ -108,13 +108,12 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int V>
 using IC = std::integral_constant<int, V>;
 
-template <int D, int LOADER, bool SEG, bool SPLIT>
-__global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
+template <int D, int LOADER, bool SEG, bool SPLIT, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
   // row blocks per wave: the per-wave state below is indexed by row block, and one is what fits 256 registers
   // (two per wave on four waves of 512 registers were slower: one wave per SIMD issues too slowly)
   constexpr int RB = 1;
-  constexpr int kNW = 8;  // waves per workgroup
-  constexpr int NT = kNW * 64;
+  constexpr int NT = NW * 64, kRows = 32 * NW;  // query rows per workgroup
   using L = Lds<D>;
   constexpr int KS = L::KS, VS = L::VS;
   constexpr int CPR = D / 8;             // 16-byte chunks per row
@@ -169,7 +168,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
 
   const int tid = threadIdx.x;
   const int w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
-  const int q0 = qblk * kBQ;
+  const int q0 = qblk * kRows;
   // row block r of this wave within the workgroup's eight
   int rblk[RB], wrow0[RB], qrow[RB], qrow_ld[RB];
 #pragma unroll
@@ -205,10 +204,10 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
       // coalesced 16-byte loads (each row is read once, not once per lane pair), then every lane
       // picks up its own row's fragments.  The next rank's loads are in flight meanwhile.
       constexpr int QS = D + 8;                  // row stride in LDS (elements)
-      constexpr int CH = kBQ * CPR / NT;         // 16-byte chunks per thread and rank
-      uint16_t* const qs = smem;                 // [kBQ][QS]
-      uint16_t* const qas = smem + kBQ * QS;     // [kBQ] head factors of this rank
-      static_assert((kBQ * QS + kBQ) * sizeof(uint16_t) <= L::kBytes, "Q staging fits the K/V buffers");
+      constexpr int CH = kRows * CPR / NT;         // 16-byte chunks per thread and rank
+      uint16_t* const qs = smem;                 // [kRows][QS]
+      uint16_t* const qas = smem + kRows * QS;     // [kRows] head factors of this rank
+      static_assert((kRows * QS + kRows) * sizeof(uint16_t) <= L::kBytes, "Q staging fits the K/V buffers");
       const uint16_t* qb_b = p.qb.ptr + b * p.qb.stride_b;
       const uint16_t* qa_b = p.qa.ptr + b * p.qa.stride_b + h;
       u32x4 nxt[CH];
@@ -220,7 +219,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
           const int grow = min(q0 + row, p.lq - 1);
           nxt[q] = *reinterpret_cast<const u32x4*>(qb_b + (int64_t)grow * p.qb.stride_l + r * p.qb.stride_r + 8 * cc);
         }
-        if (tid < kBQ) a_nxt = qa_b[(int64_t)min(q0 + tid, p.lq - 1) * p.qa.stride_l + r * p.qa.stride_r];
+        if (tid < kRows) a_nxt = qa_b[(int64_t)min(q0 + tid, p.lq - 1) * p.qa.stride_l + r * p.qa.stride_r];
       };
       float acc[RB][NKS][8];
 #pragma unroll
@@ -236,7 +235,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
           const int chunk = q * NT + tid, row = chunk / CPR, cc = chunk % CPR;
           *reinterpret_cast<u32x4*>(qs + row * QS + 8 * cc) = nxt[q];
         }
-        if (tid < kBQ) qas[tid] = (uint16_t)a_nxt;
+        if (tid < kRows) qas[tid] = (uint16_t)a_nxt;
         if (r + 1 < p.rq) load_rank(r + 1);
         lds_barrier();
         // a * b[d] for a packed pair (b[d], b[d+1]) is one dot instruction with (a, 0) or (0, a):
@@ -278,12 +277,12 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // causal offset of this batch entry: counted from the end of its keys where the caller aligns the last
   // query with the last key
   const int coff = p.coff + (p.causal == TPA_CAUSAL_BOTTOM_RIGHT ? len_b - p.lq : 0);
-  int kend = p.causal ? min(len_b, min(q0 + kBQ, p.lq) + coff) : len_b;
+  int kend = p.causal ? min(len_b, min(q0 + kRows, p.lq) + coff) : len_b;
   if constexpr (SPLIT) {  // this workgroup's share of the block's tiles
     const int all = kend > 0 ? (kend + kTK - 1) / kTK : 0;
     const int t0 = (int)((int64_t)all * range / p.S), t1 = (int)((int64_t)all * (range + 1) / p.S);
     if (t0 == t1) {
-      if (tid < kBQ && q0 + tid < p.lq) pp.part_ml[(((int64_t)range * p.B + b) * p.lq + q0 + tid) * p.H + h] = float2{-INFINITY, 0.f};
+      if (tid < kRows && q0 + tid < p.lq) pp.part_ml[(((int64_t)range * p.B + b) * p.lq + q0 + tid) * p.H + h] = float2{-INFINITY, 0.f};
       return;
     }
     kpos0 = t0 * kTK;
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     // contiguous run, the tiles inside the run need no segment mask at all.
     int lo, hi, cnt;
     int32_t qmin, qmax;
-    id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kBQ, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem), tid, lo, hi, cnt, qmin, qmax);
+    id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kRows, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem), tid, lo, hi, cnt, qmin, qmax);
     if (hi >= 0) {
       kpos0 = lo / kTK * kTK;
       kend = hi + 1;
@@ -402,7 +401,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
   // into an LDS slot one iteration later, like the head factors; slot j&1 holds the ids of tile j
   // during iteration j.
   constexpr bool has_seg = SEG;  // a kernel of its own: the mask code slows the others down even when skipped
-  constexpr int kSegWave = kNW > 4 ? 4 : 0;
+  constexpr int kSegWave = NW > 4 ? 4 : 0;
   int32_t seg_pending = 0;
   auto issue_seg = [&](int tile) __attribute__((always_inline)) {
     if constexpr (has_seg)
@@ -878,6 +877,17 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
             :
 #include "gen/prefill_loop_128_dense_clobbers.inc"
         );
+      } else if constexpr (NW == 4) {
+        asm volatile(
+#include "gen/prefill_loop_64_dense4w.inc"
+#include "gen/prefill_loop_64_dense4w_rare.inc"
+            : "+{v[0:15]}"(sa0), "+{v[16:31]}"(sa1), "+{v[32:47]}"(sb0), "+{v[48:63]}"(sb1), "+{v[64:79]}"(nmref[0]),
+              "+{v[80:95]}"(o[0][0]), "+{v[96:111]}"(o[0][1]),
+              "+{v[176:183]}"(kv_k), "+{v[184:191]}"(kv_v), "+{v[204:219]}"(st16), "+{s[32:47]}"(sc16)
+            : "{v[144:159]}"(qp0), "{s[48:51]}"(kbr), "{s[52:55]}"(vbr)
+            :
+#include "gen/prefill_loop_64_dense4w_clobbers.inc"
+        );
       } else {
         asm volatile(
 #include "gen/prefill_loop_64_dense.inc"
@@ -1027,7 +1037,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(PrefillParams pp) {
     const float inv = 1.f / ltot;
     constexpr int OS = D + 8;  // row stride (elements)
     uint16_t* const ot = smem + w * 32 * OS;
-    static_assert(kNW * 32 * OS * sizeof(uint16_t) <= L::kBytes, "output staging fits");
+    static_assert(NW * 32 * OS * sizeof(uint16_t) <= L::kBytes, "output staging fits");
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -1102,16 +1112,41 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* part_o,
 // in one group of all, 86 in two.
 inline int dense_pair_groups(int npairs, int nqb) { return pair_groups(npairs, (64 + nqb - 1) / nqb); }
 
-template <int D, int LOADER, bool SEG = false, bool SPLIT = false>
+// Four waves and 128 query rows per workgroup, two workgroups on a compute unit, in place of eight and 256 (dense tiles at head size
+// 64; at 128 the tiles leave room for one).  The two do not wait for each other's barriers, fit documents and the diagonal more
+// closely and fill more compute units where there are few blocks; both stage every tile, which is what long runs of unmasked
+// tiles lose by.  With the reconstruction, us, eight waves / four:
+//   documents, causal: 3 x 1777, 16 heads, of 421 tokens 41.7 / 37.7; 4 x 2500, 64 heads, of 800 233.7 / 202.5; 8 x 1200, 64
+//     heads, of 150 174 / 152; 1 x 16 384, 16 heads, of 1000 138.7 / 111.8, of 4000 211 / 207; 2 x 8192 of 2000 147 / 145; but one
+//     document in every row, which the host cannot see: 4 x 4096 160 / 166, 2 x 9000, 8 heads 146 / 162; without a mask 2 x
+//     9000 of 3000 306 / 303
+//   causal: 1 x 700, 16 heads 21.7 / 18.6; 16 x 512, 16 heads 37.2 / 35.3; 4 x 1600, 64 heads 169 / 155; 1 x 2048, 32 heads 49.5 / 43.8;
+//     8 x 1500, 16 heads 74.7 / 76.0; 3 x 2300, 8 heads 48.6 / 40.9; 2 x 2300, 64 heads 129 / 132; 1 x 8192, 16 heads 153 / 174
+//   no mask: 1 x 600, 8 heads 17.9 / 15.1; 16 x 512, 16 heads 42.5 / 40.6; 4 x 1000, 64 heads 102.5 / 99.5; 1 x 1000, 64 heads (256
+//     workgroups of eight) 37.5 / 39.0; 3 x 1300, 64 heads 142 / 133; 2 x 2000, 16 heads 52.6 / 55.3
+inline bool wants_four_waves(const PrefillParams& p) {
+  const int64_t wgs = (int64_t)p.npairs * p.H;  // of eight waves
+  if (p.kvseg || wgs <= 128) return true;
+  return p.causal ? p.lq <= 2048 || (wgs < 256 && p.lq <= 4096) : p.lq <= 1408 && wgs > 256;
+}
+
+template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8>
 int launch_prefill(const PrefillParams& p, hipStream_t stream) {
-  if constexpr (!SEG && !SPLIT)
+  if constexpr (!SEG && !SPLIT && NW == 8)
     if (p.S > 1) return launch_prefill<D, LOADER, SEG, true>(p, stream);
-  auto kern = prefill_kernel<D, LOADER, SEG, SPLIT>;
+  PrefillParams q = p;
+  if constexpr (D == 64 && LOADER == LOAD_DENSE && !SPLIT && NW == 8) {
+    if (wants_four_waves(p)) {
+      q.nqb = (p.lq + kBQ / 2 - 1) / (kBQ / 2);
+      q.npairs = q.nqb * p.B;
+      return launch_prefill<D, LOADER, SEG, SPLIT, 4>(q, stream);
+    }
+  }
+  auto kern = prefill_kernel<D, LOADER, SEG, SPLIT, NW>;
   constexpr size_t lds_bytes = Lds<D>::kBytes;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds_bytes); rc != TPA_OK) return rc;
   // one workgroup per (query block, batch, head): see the kernel for how ids map to them
-  PrefillParams q = p;
   int64_t n;
   if (LOADER == LOAD_DENSE) {
     q.pair_groups = dense_pair_groups(p.B * p.H, p.nqb);
@@ -1122,7 +1157,7 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
   }
   if (n > 2147483647LL) return TPA_ERR_SHAPE;
   dim3 grid((unsigned)n);
-  hipLaunchKernelGGL(kern, grid, dim3(512), lds_bytes, stream, q);
+  hipLaunchKernelGGL(kern, grid, dim3(NW * 64), lds_bytes, stream, q);
   if constexpr (SPLIT) {
     if (hipGetLastError() != hipSuccess) return TPA_ERR_LAUNCH;
     const int64_t rows = (int64_t)p.B * p.lq * p.H;
