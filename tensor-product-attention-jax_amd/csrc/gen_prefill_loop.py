@@ -45,7 +45,7 @@ The script keeps track of outstanding LDS / memory operations and of the softwar
 of gfx950 (results of matrix, dot and transcendental instructions, lane swaps, vector writes read by
 matrix instructions) and inserts the s_waitcnt / s_nop instructions they need.
 
-usage: gen_prefill_loop.py <D: 128|64> <dense|dense4w|r2> <output.inc>     (dense4w: workgroups of four waves)
+usage: gen_prefill_loop.py <D: 128|64> <dense|dense4w|r2|r24w> <output.inc>     (4w: workgroups of four waves)
 Beside the output it writes <output>_rare.inc (the rare paths; the asm statement includes them behind the loop) and
 <output>_clobbers.inc.
 """
@@ -54,15 +54,15 @@ import sys
 
 D = int(sys.argv[1])
 LOADER = sys.argv[2]
-assert LOADER in ("dense", "dense4w", "r2") and D in (128, 64)
+assert LOADER in ("dense", "dense4w", "r2", "r24w") and D in (128, 64)
 OUT = sys.argv[3]
-R2 = LOADER == "r2"
+R2 = LOADER.startswith("r2")
 
 KTK = 64
 KS, VS = D + 8, D + 32                  # LDS row strides (elements)
 NKS, NDB = D // 16, D // 32
 CPR = D // 8
-TPP = (256 if LOADER == "dense4w" else 512) // CPR  # tokens per loader pass (of the workgroup's threads)
+TPP = (256 if LOADER.endswith("4w") else 512) // CPR  # tokens per loader pass (of the workgroup's threads)
 NPASS = KTK // TPP
 KBUF, VBUF = KTK * KS * 2, KTK * VS * 2  # bytes of one K / V buffer
 NF = 2 * NKS + 4 * NDB                  # matrix instructions per iteration

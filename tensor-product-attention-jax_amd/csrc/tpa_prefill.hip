@@ -975,6 +975,17 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
             :
 #include "gen/prefill_loop_128_r2_clobbers.inc"
         );
+      } else if constexpr (NW == 4) {
+        asm volatile(
+#include "gen/prefill_loop_64_r24w.inc"
+#include "gen/prefill_loop_64_r24w_rare.inc"
+            : "+{v[0:15]}"(set0), "+{v[16:31]}"(set1), "+{v[32:47]}"(nmref[0]),
+              "+{v[48:63]}"(o[0][0]), "+{v[64:79]}"(o[0][1]),
+              "+{v[144:159]}"(kv_k), "+{v[160:175]}"(kv_v), "+{v[188:203]}"(st16), "+{s[32:47]}"(sc16)
+            : "{v[112:127]}"(qp0), "{s[48:51]}"(kbr), "{s[52:55]}"(vbr), "{s[56:59]}"(abr)
+            :
+#include "gen/prefill_loop_64_r24w_clobbers.inc"
+        );
       } else {
         u32x8 kv_k8 = __builtin_shufflevector(kv_k, kv_k, 0, 1, 2, 3, 4, 5, 6, 7);
         u32x8 kv_v8 = __builtin_shufflevector(kv_v, kv_v, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -1112,22 +1123,29 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* part_o,
 // in one group of all, 86 in two.
 inline int dense_pair_groups(int npairs, int nqb) { return pair_groups(npairs, (64 + nqb - 1) / nqb); }
 
-// Four waves and 128 query rows per workgroup, two workgroups on a compute unit, in place of eight and 256 (dense tiles at head size
-// 64; at 128 the tiles leave room for one).  The two do not wait for each other's barriers, fit documents and the diagonal more
-// closely and fill more compute units where there are few blocks; both stage every tile, which is what long runs of unmasked
-// tiles lose by.  With the reconstruction, us, eight waves / four:
+// Four waves and 128 query rows per workgroup, two workgroups on a compute unit, in place of eight and 256 (head size 64; at 128 the
+// tiles leave room for one).  The two do not wait for each other's barriers, fit documents, the diagonal and a last block of rows
+// more closely and fill more compute units where there are few blocks; both stage (or rebuild) every tile, which is what long runs
+// of unmasked tiles lose by.  Where those decide, the two are compared by their rounds of 256 workgroups, a round of four waves as half
+// a round of eight and a tenth (dense tiles, few of them: 2 %) of what they stage twice.  us, eight waves / four, dense tiles
+// with the reconstruction:
 //   documents, causal: 3 x 1777, 16 heads, of 421 tokens 41.7 / 37.7; 4 x 2500, 64 heads, of 800 233.7 / 202.5; 8 x 1200, 64
 //     heads, of 150 174 / 152; 1 x 16 384, 16 heads, of 1000 138.7 / 111.8, of 4000 211 / 207; 2 x 8192 of 2000 147 / 145; but one
 //     document in every row, which the host cannot see: 4 x 4096 160 / 166, 2 x 9000, 8 heads 146 / 162; without a mask 2 x
-//     9000 of 3000 306 / 303
+//     9000 of 3000 306 / 303; rank 2 fused: 1 x 500, 16 heads, of 200 21.2 / 17.1; 2 x 1700, 8 heads, of 150 21.4 / 17.7
 //   causal: 1 x 700, 16 heads 21.7 / 18.6; 16 x 512, 16 heads 37.2 / 35.3; 4 x 1600, 64 heads 169 / 155; 1 x 2048, 32 heads 49.5 / 43.8;
-//     8 x 1500, 16 heads 74.7 / 76.0; 3 x 2300, 8 heads 48.6 / 40.9; 2 x 2300, 64 heads 129 / 132; 1 x 8192, 16 heads 153 / 174
-//   no mask: 1 x 600, 8 heads 17.9 / 15.1; 16 x 512, 16 heads 42.5 / 40.6; 4 x 1000, 64 heads 102.5 / 99.5; 1 x 1000, 64 heads (256
-//     workgroups of eight) 37.5 / 39.0; 3 x 1300, 64 heads 142 / 133; 2 x 2000, 16 heads 52.6 / 55.3
-inline bool wants_four_waves(const PrefillParams& p) {
-  const int64_t wgs = (int64_t)p.npairs * p.H;  // of eight waves
-  if (p.kvseg || wgs <= 128) return true;
-  return p.causal ? p.lq <= 2048 || (wgs < 256 && p.lq <= 4096) : p.lq <= 1408 && wgs > 256;
+//     8 x 1500, 16 heads 74.7 / 76.0; 3 x 2300, 8 heads 48.6 / 40.9; 2 x 2300, 64 heads 129 / 132; 1 x 8192, 16 heads 153 / 174; rank 2
+//     fused: 1 x 256, 8 heads 14.2 / 12.3; 3 x 800, 64 heads 61.9 / 53.3; 16 x 512, 16 heads 34.5 / 34.0
+//   no mask, or many cached keys: 1 x 600, 8 heads 17.9 / 15.1; 3 x 1300, 64 heads 142 / 133; 8 x 600, 64 heads 112.6 / 97.3; 1 x 1000, 64
+//     heads 37.5 / 39.0; 2 x 2000, 16 heads 52.6 / 55.3; rank 2 fused: 8 x 300, 64 heads 59.4 / 46.9; 8 x 700, 64 heads 134 / 145;
+//     16 x 512, 16 heads 37.9 / 41.2; chunks of 300 over 2000, 64 heads 200 / 176, of 512 over 8192 305 / 347
+inline bool wants_four_waves(const PrefillParams& p, bool dense) {
+  if (p.kvseg) return true;
+  const int64_t pairs = (int64_t)p.B * p.H, eight = pairs * ((p.lq + 255) / 256), four = pairs * ((p.lq + 127) / 128);
+  const bool triangle = p.causal && p.lk < 2 * (int64_t)p.lq;  // masked tiles are a good part of all
+  if (triangle && (p.lk <= 2048 || (dense && eight < 256 && p.lk <= 4096))) return true;
+  const double staging = dense && p.lk <= 1408 ? 1.02 : triangle ? 1.2 : 1.1;
+  return staging * (double)((four + 255) / 256) < 2.0 * (double)((eight + 255) / 256);
 }
 
 template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8>
@@ -1135,8 +1153,8 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
   if constexpr (!SEG && !SPLIT && NW == 8)
     if (p.S > 1) return launch_prefill<D, LOADER, SEG, true>(p, stream);
   PrefillParams q = p;
-  if constexpr (D == 64 && LOADER == LOAD_DENSE && !SPLIT && NW == 8) {
-    if (wants_four_waves(p)) {
+  if constexpr (D == 64 && LOADER != LOAD_TPA_ANY && !SPLIT && NW == 8) {
+    if (wants_four_waves(p, LOADER == LOAD_DENSE)) {
       q.nqb = (p.lq + kBQ / 2 - 1) / (kBQ / 2);
       q.npairs = q.nqb * p.B;
       return launch_prefill<D, LOADER, SEG, SPLIT, 4>(q, stream);
