@@ -631,8 +631,11 @@ int launch(const BwdParams& base, hipStream_t stream) {
 //   documents: 3 x 1777, 16 heads, of 421 tokens 129 / 117; 2 x 9000, 8 heads, of 9000 684 / 590; 1 x 20 000, 8 heads, of 4000
 //     609 / 569; 4 x 3000, 16 heads, of 2900 401 / 377; without a mask 2 x 9000, 16 heads, of 3000 1216 / 1136
 //   causal: 16 x 512, 16 heads 163 / 146; 2 x 1300, 64 heads 265 / 252; 8 x 1024, 64 heads 681 / 657; 2 x 2300, 64 heads 560 /
-//     559; 8 x 3000, 16 heads 904 / 908; 1 x 8192, 16 heads 636 / 654
-//   no mask: 16 x 512, 16 heads 180 / 174; 4 x 1000, 64 heads 443 / 449; 4 x 2048, 16 heads 361 / 376
+//     559; 1 x 2600, 64 heads 359 / 351; 8 x 3000, 16 heads 904 / 908; 1 x 8192, 16 heads 636 / 654; few workgroups: 1 x 3000, 8 heads 137.6 /
+//     126.5; 1 x 6000, 8 heads 248 / 235; 1 x 4096, 16 heads 213 / 210.5; 2 x 4000, 16 heads 354 / 360; 1 x 10 000, 8 heads 517 / 522
+//   no mask, where the rounds of 256 workgroups decide (of four waves half a round of eight and 4 %): 8 x 300, 64 heads 197 / 181; 8 x 600
+//     445 / 420; 3 x 1300, 64 heads 544 / 530; 4 x 1000, 64 heads 443 / 449; 3 x 2100, 8 heads 170 / 174.5; 4 x 2048, 16 heads 361 / 376; all in
+//     one round: 1 x 1500, 16 heads 95 / 90; 1 x 4000, 8 heads 189 / 182
 // (64 keys per wave would halve the LDS reads per MFMA, but its 384 stationary registers at D = 128 leave the compiler
 // spilling; the dQ kernel with 4 waves of 64 rows, one wave per SIMD and 512 registers, takes 922 us where 8 waves of 32
 // rows take 401 us.)
@@ -640,7 +643,10 @@ template <int D>
 int launch_both(const BwdParams& p, hipStream_t stream) {
   if constexpr (D == 64) {
     if (p.qseg) return launch<D, 4, 1, true>(p, stream);
-    if (p.causal && p.lq <= 2304 && p.lk <= 2304) return launch<D, 4, 1, false>(p, stream);
+    const int64_t pairs = (int64_t)p.B * p.H;
+    auto rounds = [&](int block) { return (pairs * ((p.lq + block - 1) / block + (p.lk + block - 1) / block) + 255) / 256; };
+    if (p.causal ? (p.lq <= 2816 && p.lk <= 2816) || rounds(256) <= 2 : rounds(256) == 1 || 1.04 * (double)rounds(128) < 2.0 * (double)rounds(256))
+      return launch<D, 4, 1, false>(p, stream);
     return launch<D, 8, 1, false>(p, stream);
   } else {
     return p.qseg ? launch<D, 8, 1, true>(p, stream) : launch<D, 8, 1, false>(p, stream);

@@ -1,6 +1,6 @@
-"""The matrix-core backward at head size 64 works in blocks of 128 rows (documents, or a causal mask of at most
-2304 rows) or 256 (everything else): sizes on either side of the blocks, of the 64-row tiles and of that line, with
-documents that share tiles and, in one case, ids that come back; against the oracle."""
+"""The matrix-core backward at head size 64 works in blocks of 128 rows (documents, a causal mask of at most 2816 rows, few
+workgroups, or fewer rounds of them) or 256 (everything else): sizes on either side of the blocks, of the 64-row tiles
+and of those lines, with documents that share tiles and, in one case, ids that come back; against the oracle."""
 
 import numpy as np
 import pytest
@@ -30,6 +30,10 @@ def _ids(kind, b, t):
         (3, 385, 8, True, None),
         (1, 2304, 8, True, None),
         (1, 2305, 8, True, None),
+        (3, 2817, 8, True, None),    # blocks of 256: 576 workgroups of them
+        (1, 600, 8, False, None),    # one round of blocks of 256
+        (4, 512, 32, False, None),   # blocks of 256: two rounds, as four of half the size
+        (5, 512, 32, False, None),   # three rounds against five
     ],
 )
 def test_backward_at_the_edges_of_blocks(gpu, b, t, h, causal, kind):
