@@ -938,7 +938,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, TO* o
       ms[q] = p.part_m[idx];
       ls[q] = p.part_l[idx];
       os[q] = *reinterpret_cast<const f32x4*>(p.part_o + idx * D + 4 * c);
-      if (s >= S) ms[q] = -INFINITY;
+      if (s >= S) { ms[q] = -INFINITY; os[q] = f32x4{0.f, 0.f, 0.f, 0.f}; ls[q] = 0.f; }  // an infinity of the last range counts once
     }
     float gmax = mmax;
 #pragma unroll

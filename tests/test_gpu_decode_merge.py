@@ -40,3 +40,20 @@ def test_rows_without_keys(gpu, b, lk):
         oi, li = tpa.tpa_decode(*tpa_split(q[i : i + 1], k[i : i + 1, : lengths[i]], v[i : i + 1, : lengths[i]], h), num_splits=1, **args)
         torch.testing.assert_close(o[i : i + 1], oi, rtol=2.0**-7, atol=1e-3)
         torch.testing.assert_close(lse[i : i + 1], li, rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("splits", [0, 6, 9, 24])
+def test_infinity_of_the_last_range(gpu, dt, splits):
+    """A trip repeats the last range where there are no more: an infinity in it counts once and stays one."""
+    from tpa import tpa
+
+    h, d, lk = 16, 128, 1500
+    q, k, v = (to_gpu(x, dt, gpu) for x in make_factors(73, 1, 1, lk, h, d, d, 6, 2, scale_by_rank=True))
+    args = tpa_split(q, k, v, h)
+    base, _ = tpa.tpa_decode(*args, sm_scale=d**-0.5, num_splits=splits, kernel=2)
+    v[0, -1, 0, h] = float("inf")  # token factor of rank 0, its first element
+    o, lse = tpa.tpa_decode(*tpa_split(q, k, v, h), sm_scale=d**-0.5, num_splits=splits, kernel=2)
+    sign = torch.sign(v[0, -1, 0, :h].float())
+    assert torch.equal(o[0, 0, :, 0].float(), sign * float("inf"))
+    assert torch.equal(o[..., 1:], base[..., 1:])
