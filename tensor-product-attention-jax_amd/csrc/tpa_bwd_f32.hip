@@ -252,6 +252,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dq_kernel(BwdF32Params p) {
   const float delta = p.delta[((int64_t)b * p.H + h) * p.lq + qrow_ld];
   int32_t qseg = 0;
   if constexpr (SEG) qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
+  const TileIds<SEG, 1> ids_of_wave({qseg});
 
   f32x16 dq[NDB];
   const float* const kbase = p.k + (int64_t)b * p.lk * hd + (int64_t)h * D;
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dq_kernel(BwdF32Params p) {
     for (int j = 0; j < ntiles; ++j) {
       const bool more = j + 1 < ntiles;
       if (more) issue(j + 1);
-      if (j <= wave_last_tile) compute(fp32, j);
+      if (j <= wave_last_tile && ids_of_wave.look(lds_seg + (j & 1) * kTile, l & (kTile - 1)) != kNoneOfThem) compute(fp32, j);
       if (more) commit(fp32, j + 1);
       __syncthreads();
     }
@@ -363,6 +364,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dkv_kernel(BwdF32Params p) {
   };
   int32_t kseg = 0;
   if constexpr (SEG) kseg = p.kvseg[(int64_t)b * p.lk + key_ld];
+  const TileIds<SEG, 1> ids_of_wave({kseg});
 
   f32x16 dk[NDB], dv[NDB];
   const float* const qbase = p.q + (int64_t)b * p.lq * hd + (int64_t)h * D;
@@ -436,7 +438,9 @@ __global__ __launch_bounds__(NW * 64) void bwd_f32_dkv_kernel(BwdF32Params p) {
     for (int j = first_tile; j < ntiles; ++j) {
       const bool more = j + 1 < ntiles;
       if (more) issue(j + 1);
-      if (j >= wave_first_tile) compute(fp32, j);
+      bool mine = j >= wave_first_tile;
+      if constexpr (SEG) mine = mine && ids_of_wave.look(reinterpret_cast<const int32_t*>(lds_row) + ((j & 1) * 3 + 2) * kTile, l & (kTile - 1)) != kNoneOfThem;
+      if (mine) compute(fp32, j);
       if (more) commit(fp32, j + 1);
       __syncthreads();
     }

@@ -198,6 +198,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   float m_run, lsum;  // running max of row qrow (log2 domain, scale included); this lane's share of sum exp2(x - m_run)
   int32_t qseg = 0;
   if constexpr (SEG) qseg = p.qseg[(int64_t)b * p.lq + qrow_ld];
+  const TileIds<SEG, 1> ids_of_wave({qseg});
 
   f32x16 s[NMB];  // logits, then probabilities, of the tile in flight
   auto logits_softmax = [&](auto fp32, int tile) __attribute__((always_inline)) {
@@ -348,7 +349,9 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
     // middle of it, so the SIMD always has a wave with matrix work and both end the tile together.
     const bool rebuild_first = w < NW / 2;
     for (int j = 0; j < ntiles; ++j) {
-      const bool more = j + 1 < ntiles, mine = j <= wave_last_tile && wrow0 < p.lq;  // waves past the last row only help rebuild
+      const bool more = j + 1 < ntiles;
+      const bool mine = j <= wave_last_tile && wrow0 < p.lq &&  // waves past the last row, or whose documents a tile has not, only help rebuild
+                        ids_of_wave.look(lds_seg + (j & 1) * kTK, l & (kTK - 1)) != kNoneOfThem;
       if (rebuild_first && more) rebuild(fp32, j + 1);
       if (mine) logits_softmax(fp32, j);
       if (!rebuild_first && more) rebuild(fp32, j + 1);
