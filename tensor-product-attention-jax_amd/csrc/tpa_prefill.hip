@@ -1,15 +1,16 @@
 // Flash-style prefill for gfx950: bf16 MFMA contractions, fp32 online softmax.
 //
 // One workgroup = one (batch, head, block of 256 query rows): eight waves (two per SIMD, 256 registers
-// each), a wave owns one block of 32 query rows.
+// each), a wave owns one block of 32 query rows.  At head size 64 it is 128 rows and four waves, two workgroups
+// to a compute unit, where wants_four_waves() says so.
 // Per tile of 64 keys the workgroup rebuilds the head's K and V
 // tile from the rank factors (K = (1/R) sum_r a_r (x) b_r, tpa/tpa.py:364,417) straight out of
 // coalesced 16-byte factor loads and stores it once, as bf16, in LDS.  Each wave then computes
 //     S^T = K Q^T        (v_mfma_f32_32x32x16_bf16, A = K rows from LDS, B = Q kept in registers,
 //                         Q pre-scaled by sm_scale*log2(e) and the accumulator started at minus
 //                         the running reference, so the result is the exponent itself)
-//     online softmax     (each lane holds 32 logits of ONE query row, so the row max and sum
-//                         are in-lane apart from one exchange with lane ^ 32)
+//     online softmax     (each lane holds 32 logits of ONE query row, so the row max, where one is
+//                         taken, and sum are in-lane apart from one exchange with lane ^ 32)
 //     O^T += V^T P^T     (A = V^T read with ds_read_b64_tr_b16 from row-major V, B = P^T, which
 //                         is the S^T accumulator converted in place: no LDS round trip for P)
 // with the deferred normalisation of flash attention (a reference m and a sum l per row), which
