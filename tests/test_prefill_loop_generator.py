@@ -13,6 +13,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "tensor-product-attention-jax_amd", "csrc")
+LOOPS = [(128, "dense"), (64, "dense"), (64, "dense4w"), (128, "r2"), (64, "r2"), (64, "r24w")]  # the ones that are built
 REG = re.compile(r"\b([vs])(?:(\d+)|\[(\d+):(\d+)\])")
 
 
@@ -97,6 +98,17 @@ def test_generated_loop_matches_its_asm_statement(tmp_path, d, loader):
         if ds:
             used |= ds[0] | ds[1]
     assert clob_regs <= used, sorted(clob_regs - used)
+
+
+@pytest.mark.parametrize("d,loader", LOOPS)
+def test_a_nan_does_not_take_the_rare_path(tmp_path, d, loader):
+    """Whatever branches to a rare path does so on an ordered comparison `slack < sum`: false for NaN, true for an overflow."""
+    lines, _ = generate(tmp_path, d, loader)
+    branches = [i for i, ln in enumerate(lines) if ln.startswith("s_cbranch_vccnz .Lpf_rare_")]
+    assert len(branches) == (8 if loader.startswith("r2") else 4)  # two parities, a group per block (rank 2: two)
+    for i in branches:
+        writer = next(ln for ln in reversed(lines[:i]) if (dst_and_src(ln) or (set(),))[0] & {"vcc"})
+        assert re.fullmatch(r"v_cmp_lt_f32 vcc, s64, v\d+", writer), writer
 
 
 def test_generator_takes_no_environment_input():
