@@ -2,7 +2,8 @@
 them their registers (csrc/tpa_prefill.hip), without a GPU: every register an instruction of a loop writes
 is an in/out operand of its asm statement or a listed clobber, every register it reads is an operand or was
 written earlier in the loop, input-only operands are never written, each copy of the iteration passes
-exactly one workgroup barrier, and nothing beyond the 256 registers of a wave is named."""
+exactly one workgroup barrier, and nothing beyond the 256 registers of a wave is named.  The rare paths, which the asm statement
+includes behind the loop, are held to the same rules, each from the place that branches to it."""
 
 import os
 import re
@@ -25,10 +26,14 @@ def regs(text):
     return out
 
 
-def generate(tmp_path, d, loader):
+def read_lines(path):
+    return [ln.strip()[1:].split("\\n")[0] for ln in path.read_text().splitlines() if ln.startswith('"')]
+
+
+def generate(tmp_path, d, loader, generator=os.path.join(CSRC, "gen_prefill_loop.py")):
     out = tmp_path / f"loop_{d}_{loader}.inc"
-    subprocess.run([sys.executable, os.path.join(CSRC, "gen_prefill_loop.py"), str(d), loader, str(out)], check=True, capture_output=True)
-    lines = [ln.strip()[1:].split("\\n")[0] for ln in out.read_text().splitlines() if ln.startswith('"')]
+    subprocess.run([sys.executable, generator, str(d), loader, str(out)], check=True, capture_output=True)
+    lines = read_lines(out)
     clob = re.findall(r'"([^"]+)"', (tmp_path / f"loop_{d}_{loader}_clobbers.inc").read_text())
     return lines, set(clob)
 
@@ -63,8 +68,7 @@ def dst_and_src(line):
     return regs(opnds[0]), set().union(*(regs(o) for o in opnds[1:])) if len(opnds) > 1 else set()
 
 
-@pytest.mark.parametrize("loader", ["dense", "r2"])
-@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("d,loader", LOOPS)
 def test_generated_loop_matches_its_asm_statement(tmp_path, d, loader):
     lines, clob = generate(tmp_path, d, loader)
     inout, inputs = asm_operands(d, loader)
@@ -93,7 +97,7 @@ def test_generated_loop_matches_its_asm_statement(tmp_path, d, loader):
     assert n_mfma == 2 * (2 * (d // 16) + 4 * (d // 32))
     # every clobbered register is really used (a stale clobber would hide a register the compiler could have)
     used = set()
-    for ln in lines:
+    for ln in lines + read_lines(tmp_path / f"loop_{d}_{loader}_rare.inc"):
         ds = dst_and_src(ln)
         if ds:
             used |= ds[0] | ds[1]
@@ -109,6 +113,74 @@ def test_a_nan_does_not_take_the_rare_path(tmp_path, d, loader):
     for i in branches:
         writer = next(ln for ln in reversed(lines[:i]) if (dst_and_src(ln) or (set(),))[0] & {"vcc"})
         assert re.fullmatch(r"v_cmp_lt_f32 vcc, s64, v\d+", writer), writer
+
+
+def rare_paths(lines):
+    """label -> instructions, of the lines of the second file"""
+    assert lines[-1] == ".Lpf_out_%=:"
+    paths, label = {}, None
+    for ln in lines[:-1]:
+        if ln.endswith(":"):
+            label = ln[:-1]
+            assert label.startswith(".Lpf_rare_") and label not in paths
+            paths[label] = []
+        else:
+            paths[label].append(ln)
+    return paths
+
+
+def check_rare_paths(lines, rare, clob, inout, inputs, n_mfma):
+    """the rules of the loop for each rare path, with what is defined where the loop branches to it"""
+    clob_regs = {c for c in clob if REG.fullmatch(c)}
+    paths, defined = rare_paths(rare), set(inout) | set(inputs)
+    entered = []
+    for i, ln in enumerate(lines):
+        if ln.startswith("s_cbranch_vccnz .Lpf_rare_"):
+            label = ln.split()[1]
+            back = label.replace("_rare_", "_cont_")
+            entered.append(label)
+            assert lines[i + 1] == back + ":" and lines.count(back + ":") == 1, "a path returns behind its branch"
+            path, known = paths[label], set(defined)
+            assert path[-1] == "s_branch " + back and not any(x.startswith(("s_cbranch", "s_branch", "s_barrier", "buffer_", "ds_write")) for x in path[:-1])
+            assert sum(x.startswith("v_mfma") for x in path) == n_mfma
+            for x in path:
+                dst, src = dst_and_src(x) or (set(), set())
+                dst, src = ({r for r in rs if not r.startswith("vcc")} for rs in (dst, src))
+                assert all(int(r[1:]) < (256 if r[0] == "v" else 102) for r in dst | src), x
+                assert not dst & inputs, f"`{x}` writes an input-only operand"
+                assert not dst - inout - clob_regs, f"`{x}` writes {sorted(dst - inout - clob_regs)}: neither an in/out operand nor a clobber"
+                assert not src - known, f"`{x}` reads {sorted(src - known)} before anything wrote them"
+                known |= dst
+        defined |= (dst_and_src(ln) or (set(),))[0]
+    assert sorted(entered) == sorted(paths), "each path is entered from one place"
+
+
+@pytest.mark.parametrize("d,loader", LOOPS)
+def test_rare_paths_match_the_asm_statement(tmp_path, d, loader):
+    lines, clob = generate(tmp_path, d, loader)
+    rare = read_lines(tmp_path / f"loop_{d}_{loader}_rare.inc")
+    operands = asm_operands(d, loader)
+    check_rare_paths(lines, rare, clob, *operands, n_mfma=d // 16)
+    inout, inputs = operands
+    unlisted = next(f"v{i}" for i in range(255, 0, -1) if f"v{i}" not in inout | inputs | clob)
+    at = next(i for i, ln in enumerate(rare) if ln.startswith("v_max_f32"))
+    op, dst, src = re.fullmatch(r"(v_max_f32) (v\d+), (.*)", rare[at]).groups()
+    for planted, what in ((f"{op} {unlisted}, {src}", "neither"), (f"{op} {dst}, {unlisted}, {unlisted}", "before anything"),
+                          (f"{op} {sorted(inputs & regs('v[0:255]'))[0]}, {src}", "input-only"), ("s_barrier", None)):
+        with pytest.raises(AssertionError, match=what):
+            check_rare_paths(lines, rare[:at] + [planted] + rare[at:], clob, *operands, n_mfma=d // 16)
+
+
+def test_a_register_of_the_rare_paths_alone_is_a_clobber(tmp_path):
+    """Head size 64 with eight waves has one loader pass and leaves a temporary unused in the loop; a rare path that wrote it would
+    have to say so."""
+    text = open(os.path.join(CSRC, "gen_prefill_loop.py")).read()
+    assert text.count("    addr = set_address(e, t1)\n") == 1
+    planted = text.replace("    addr = set_address(e, t1)\n", '    addr = set_address(e, t1)\n    e.ins("v_mov_b32", f"v{AAK1}", "0")\n')
+    (tmp_path / "gen.py").write_text(planted)
+    lines, clob = generate(tmp_path, 64, "r2", str(tmp_path / "gen.py"))
+    written = {ln.split()[1].rstrip(",") for ln in read_lines(tmp_path / "loop_64_r2_rare.inc") if ln.startswith("v_mov_b32") and ln.endswith(", 0")}
+    assert len(written) == 1 and written <= clob and not any(written & regs(ln) for ln in lines)
 
 
 def test_generator_takes_no_environment_input():
