@@ -377,11 +377,15 @@ def issue_loads(e, is_v):
 
 # ---- softmax
 # There is no row maximum in the loop.  The exponentials are taken against the running reference as it is; what says that the
-# reference must move is the sum of a group of them, which is needed anyway: a sum above 2^8 means that an exponent
-# may have left the range in which nothing is lost.  Up to there no bit depends on the reference (it is a whole number and every factor an exact
-# power of two).  The rare path then computes the group's logits again from K tile j, which stays in LDS until the iteration
-# ends, takes their maximum, moves the reference and repeats the group's exponentials, before any O^T instruction has
-# seen them.  A maximum of 32 logits is 20 vector instructions of the 139 an iteration of the dense loop had.
+# reference must move is the sum of a group of them, which is needed anyway: above 2^8 the row may have outgrown it.  The reference is a
+# whole number, so that all factors that come of it are powers of two; what depends on it is where the fp32 sum of a logit starts, hence
+# its last bits, and now and then the rounding of a probability to bf16.  The rare path scales down what was made with the old
+# reference, the group's packed exponentials included, before any O^T instruction has seen them; only where the sum may have overflowed are the
+# group's logits computed again, from K tile j, which stays in LDS until the iteration ends.
+# A maximum of 32 logits is 20 vector instructions of the 139 an iteration of the dense loop had (4 x 4096 tokens, 16 heads of 128, causal:
+# 287 us with it, 281 so).  In return a move is dearer than behind a maximum, which matters where logits grow along the keys.  With a
+# maximum / every moving group computed again / this, us: the mean row by 55 in the log2 domain 304 / 320 / 299, by 170 309 / 342 /
+# 305, by 1700 303 / 371 / 315; 4 x 800 (rank-2 loop), by 170 44.2 / 49.2 / 43.2.
 def sm_exp_regs(e, s, q, T0, T1, BS, first):
     """exponentials and bf16 packing of logits 4q .. 4q+3 of the 16 in v[s:s+15]; their sum goes to BS (`first`) or onto it"""
     for k in range(4):
@@ -403,21 +407,25 @@ def sm_check(e, BS, name):
     e.raw(f".Lpf_cont_{name}_%=:")
     e.ins("v_add_f32", f"v{LSUM}", f"v{LSUM}", f"v{BS}")
 
-def row_max(e, regs, TA, TB):
-    """maximum of the listed logits of this lane's row, over both lanes that share it, into TA"""
-    regs = list(regs)
-    e.ins("v_max_f32", f"v{TA}", f"v{regs[0]}", f"v{regs[1]}")
-    for k in range(2, len(regs), 2):
-        e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{regs[k]}", f"v{regs[k + 1]}")
+def over_both_lanes(e, TA, TB):
+    """the larger of TA of the two lanes that share a row, into TA"""
     e.ins("v_mov_b32", f"v{TB}", f"v{TA}")
     e.ins("v_permlane32_swap_b32", f"v{TA}", f"v{TB}", ndst=2)
     e.ins("v_max_f32", f"v{TA}", f"v{TA}", f"v{TB}")
 
-def rescale(e, tmax, RD, RAL, sets):
-    """the reference moves up by ceil(row maximum) (a whole number, so every factor is an exact power of
-    two): O and the row sum shrink, the logit registers listed in `sets` move down"""
-    e.ins("v_ceil_f32", f"v{RD}", f"v{tmax}")
-    e.ins("v_max_f32", f"v{RD}", "0", f"v{RD}")               # delta = tmax > 0 ? ceil(tmax) : 0
+def row_max(e, regs, TA, TB):
+    """ceil of the maximum of the listed logits of this lane's row, over both lanes that share it, into TA"""
+    regs = list(regs)
+    e.ins("v_max_f32", f"v{TA}", f"v{regs[0]}", f"v{regs[1]}")
+    for k in range(2, len(regs), 2):
+        e.ins("v_max3_f32", f"v{TA}", f"v{TA}", f"v{regs[k]}", f"v{regs[k + 1]}")
+    over_both_lanes(e, TA, TB)
+    e.ins("v_ceil_f32", f"v{TA}", f"v{TA}")
+
+def rescale(e, up, RD, RAL, logits):
+    """the reference moves up by max(0, `up`) (a whole number, so every factor is an exact power of
+    two): O and the row sum shrink, the listed logits move down"""
+    e.ins("v_max_f32", f"v{RD}", "0", f"v{up}")
     e.ins("v_exp_f32_e64", f"v{RAL}", f"-v{RD}")              # alpha = 2^-delta
     e.ins("v_add_f32", f"v{MREF}", f"v{MREF}", f"v{RD}")
     for k in range(16):
@@ -426,18 +434,52 @@ def rescale(e, tmax, RD, RAL, sets):
     for db in range(NDB):
         for k in range(16):
             e.ins("v_mul_f32", f"v{O(db) + k}", f"v{O(db) + k}", f"v{RAL}")
-    for s in sets:
-        for k in range(16):
-            e.ins("v_sub_f32", f"v{s + k}", f"v{s + k}", f"v{RD}")
+    for r in logits:
+        e.ins("v_sub_f32", f"v{r}", f"v{r}", f"v{RD}")
 
-def rare_path(name, f, frag_load, set_address, temps, again, moved, redo):
-    """A group's sum left the slack behind matrix instruction f (do_softmax() in tpa_prefill.hip moves the reference by
-    the same rule).  `again` = (register, byte offset of its rows in a K buffer) of the blocks whose logits are computed again,
-    `moved` = the logits of later blocks whose accumulation began at the old reference, `redo` = the recorded exponentials that
+def block(s): return list(range(s, s + 16))
+
+def scale_path(name, temps, free, packed, raw, moved):
+    """A group's sum left the slack (do_softmax() in tpa_prefill.hip does the like).  Its exponentials are there, as bf16 in
+    `packed`: the reference moves so that their sum falls below 1, and no further logit of `raw`, complete and not touched yet, lies
+    above it; everything that was made with the old reference shrinks with it, `packed` included.  `moved` = logits whose accumulation
+    began at the old reference.  `temps` = the registers of the group's sum and its two temporaries, `free` = another group's, which holds
+    nothing here.  A sum of 2^126 and more may have lost its group to infinity: the path that computes it again."""
+    e = Stream()
+    e.raw(f".Lpf_rare_{name}_%=:")
+    e.ins("v_cmp_lt_f32", "vcc", "0x7e800000", f"v{temps[0]}")
+    e.raw(f"s_cbranch_vccnz .Lpf_full_{name}_%=")
+    e.nop(20)                        # the matrix instruction in flight: its result and its operand reads
+    sum_, t0, t1 = temps
+    up, alpha, t2 = free
+    e.ins("v_mov_b32", f"v{t0}", f"v{sum_}")
+    over_both_lanes(e, t0, t1)
+    e.ins("v_frexp_exp_i32_f32", f"v{t0}", f"v{t0}")          # sum < 2^t0
+    e.ins("v_cvt_f32_i32", f"v{t0}", f"v{t0}")
+    if raw:
+        row_max(e, raw, t1, t2)
+        e.ins("v_max_f32", f"v{t0}", f"v{t0}", f"v{t1}")
+    rescale(e, t0, up, alpha, raw + moved)
+    e.ins("v_mul_f32", f"v{sum_}", f"v{sum_}", f"v{alpha}")
+    for n, r in enumerate(packed):
+        a, b = ((t0, t1), (t2, up))[n & 1]                    # `up` has been used
+        e.ins("v_lshlrev_b32", f"v{a}", "16", f"v{r}")
+        e.ins("v_and_b32", f"v{b}", "0xffff0000", f"v{r}")
+        e.ins("v_mul_f32", f"v{a}", f"v{a}", f"v{alpha}")
+        e.ins("v_mul_f32", f"v{b}", f"v{b}", f"v{alpha}")
+        e.ins("v_cvt_pk_bf16_f32", f"v{r}", f"v{a}", f"v{b}")
+    e.nop(4)
+    e.raw(f"s_branch .Lpf_cont_{name}_%=")
+    return e.lines
+
+def full_path(name, f, frag_load, set_address, temps, again, whole, moved, redo):
+    """The same for a sum that may have overflowed, behind matrix instruction f.  `again` = (register, byte offset of its rows in a K buffer) of the blocks whose logits are computed again,
+    `whole` = those of a later block that are complete and not touched yet: its maximum counts at once, or a row that grows would
+    come here again for it; `moved` = the logits of blocks whose accumulation began at the old reference, `redo` = the recorded exponentials that
     were issued.  `temps` = the registers of the group's sum and its two temporaries, which `redo` writes anew.  The fragments that the
     loop has read ahead are overwritten here and read again at the end."""
     e = Stream()
-    e.raw(f".Lpf_rare_{name}_%=:")
+    e.raw(f".Lpf_full_{name}_%=:")
     e.raw("s_waitcnt lgkmcnt(0)")
     e.nop(64)                        # matrix instructions in flight: their results and their operand reads
     sum_, t0, t1 = temps
@@ -447,8 +489,9 @@ def rare_path(name, f, frag_load, set_address, temps, again, moved, redo):
         b = RING_BUFS[n % len(RING_BUFS)]
         e.ins("ds_read_b128", vt(b), f"v{addr} offset:{off + kk * 32}")
         e.ins("v_mfma_f32_32x32x16_bf16", vt(s, 16), vt(b), vt(Q(kk)), vt(NMREF, 16) if kk == 0 else vt(s, 16))
-    row_max(e, [s + k for s, _ in again for k in range(16)], t0, t1)
-    rescale(e, t0, sum_, t1, [s for s, _ in again] + moved)
+    logits = [r for s, _ in again for r in block(s)] + whole
+    row_max(e, logits, t0, t1)
+    rescale(e, t0, sum_, t1, logits + moved)
     for it in redo:
         replay(e, it)
     for n in range(f + 1, min(f + LA, NF - 1) + 1):
@@ -500,8 +543,11 @@ def half(e, p, rare):
     for mb in range(2):
         # block 0's check comes before any exponential of block 1, whose logits only move; at block 1's, block 0 is in O
         assert check[0] >= N_QK // 2 and check[0] < N_QK and check[1] == N_QK + 2 * NDB - 1
-        rare += rare_path(f"{p}{mb}", check[mb], lambda e2, n: emit_frag_load(e2, n, p), address, ((BS0, T0A, T1A), (BS1, T0B, T1B))[mb], [(S(p, mb), mb * 32 * KS * 2)],
-                          ([S(p, 1)] if mb == 0 else []) + [S(1 - p, 0), S(1 - p, 1)], sm[mb].items)
+        temps = [(BS0, T0A, T1A), (BS1, T0B, T1B)]
+        whole, moved = block(S(p, 1)) if mb == 0 else [], block(S(1 - p, 0)) + block(S(1 - p, 1))
+        rare += scale_path(f"{p}{mb}", temps[mb], temps[1 - mb], block(S(p, mb))[:8], whole, moved)
+        rare += full_path(f"{p}{mb}", check[mb], lambda e2, n: emit_frag_load(e2, n, p), address, temps[mb], [(S(p, mb), mb * 32 * KS * 2)],
+                          whole, moved, sm[mb].items)
     # the K buffers rotate: next iteration reads what this one wrote beside, and writes the one after
     e.ins("s_mov_b32", f"s{S_KR}", f"s{S_KWB}")
     e.ins("s_add_u32", f"s{S_KWB}", f"s{S_KWB}", f"0x{KBUF:x}")
@@ -648,9 +694,13 @@ def half_r2(e, p, rare):
             replay(e, it)
     for blk, hf, at in checks:
         # the block is one half of K tile j; the other set holds the next block, begun at the old reference
-        rare += rare_path(f"{p}{blk}{hf}", at, lambda e2, n: r2_frag_load(e2, n, p), lambda e2, t: KFA, ((BS0, T0A, T1A), (BS1, T0B, T1B))[hf],
-                          [(SET(blk), blk * 32 * KS * 2)],
-                          [SET(1 - blk)], sm[blk][hf].items)
+        # (complete behind the first O^T instructions); of the block itself the first half of a lane's logits, bf16 by now, lies in
+        # the first four registers and in O behind the second check, the second half is untouched before the first
+        temps = [(BS0, T0A, T1A), (BS1, T0B, T1B)]
+        own, other = block(SET(blk)), block(SET(1 - blk))
+        rare += scale_path(f"{p}{blk}{hf}", temps[hf], temps[1 - hf], own[4 * hf:4 * hf + 4], other if hf else own[8:], [] if hf else other)
+        rare += full_path(f"{p}{blk}{hf}", at, lambda e2, n: r2_frag_load(e2, n, p), lambda e2, t: KFA, temps[hf], [(SET(blk), blk * 32 * KS * 2)],
+                          other if hf else [], [] if hf else other, sm[blk][hf].items)
     # the K buffers rotate: (tile j, tile j+1, free) -> (tile j+1, tile j+2, free)
     e.ins("s_mov_b32", f"s{S_T0}", f"s{S_K0}")
     e.ins("s_mov_b32", f"s{S_K0}", f"s{S_K1}")

@@ -122,7 +122,7 @@ def rare_paths(lines):
     for ln in lines[:-1]:
         if ln.endswith(":"):
             label = ln[:-1]
-            assert label.startswith(".Lpf_rare_") and label not in paths
+            assert label.startswith((".Lpf_rare_", ".Lpf_full_")) and label not in paths
             paths[label] = []
         else:
             paths[label].append(ln)
@@ -140,17 +140,24 @@ def check_rare_paths(lines, rare, clob, inout, inputs, n_mfma):
             back = label.replace("_rare_", "_cont_")
             entered.append(label)
             assert lines[i + 1] == back + ":" and lines.count(back + ":") == 1, "a path returns behind its branch"
-            path, known = paths[label], set(defined)
-            assert path[-1] == "s_branch " + back and not any(x.startswith(("s_cbranch", "s_branch", "s_barrier", "buffer_", "ds_write")) for x in path[:-1])
-            assert sum(x.startswith("v_mfma") for x in path) == n_mfma
-            for x in path:
-                dst, src = dst_and_src(x) or (set(), set())
-                dst, src = ({r for r in rs if not r.startswith("vcc")} for rs in (dst, src))
-                assert all(int(r[1:]) < (256 if r[0] == "v" else 102) for r in dst | src), x
-                assert not dst & inputs, f"`{x}` writes an input-only operand"
-                assert not dst - inout - clob_regs, f"`{x}` writes {sorted(dst - inout - clob_regs)}: neither an in/out operand nor a clobber"
-                assert not src - known, f"`{x}` reads {sorted(src - known)} before anything wrote them"
-                known |= dst
+            full = label.replace("_rare_", "_full_")
+            entered.append(full)
+            for path, matrix in ((paths[label], 0), (paths[full], n_mfma)):
+                # the first goes on to the second where the sum may have overflowed, before it has written anything
+                assert path[-1] == "s_branch " + back and sum(x.startswith("v_mfma") for x in path) == matrix
+                head = [x for x in path[:2] if path is paths[label]]
+                if head:
+                    assert re.fullmatch(r"v_cmp_lt_f32 vcc, 0x7e800000, v\d+", head[0]) and head[1] == "s_cbranch_vccnz " + full
+                assert not any(x.startswith(("s_cbranch", "s_branch", "s_barrier", "buffer_", "ds_write")) for x in path[len(head):-1])
+            for path, known in ((paths[label], set(defined)), (paths[full], set(defined))):
+                for x in path:
+                    dst, src = dst_and_src(x) or (set(), set())
+                    dst, src = ({r for r in rs if not r.startswith("vcc")} for rs in (dst, src))
+                    assert all(int(r[1:]) < (256 if r[0] == "v" else 102) for r in dst | src), x
+                    assert not dst & inputs, f"`{x}` writes an input-only operand"
+                    assert not dst - inout - clob_regs, f"`{x}` writes {sorted(dst - inout - clob_regs)}: neither an in/out operand nor a clobber"
+                    assert not src - known, f"`{x}` reads {sorted(src - known)} before anything wrote them"
+                    known |= dst
         defined |= (dst_and_src(ln) or (set(),))[0]
     assert sorted(entered) == sorted(paths), "each path is entered from one place"
 
@@ -181,6 +188,23 @@ def test_a_register_of_the_rare_paths_alone_is_a_clobber(tmp_path):
     lines, clob = generate(tmp_path, 64, "r2", str(tmp_path / "gen.py"))
     written = {ln.split()[1].rstrip(",") for ln in read_lines(tmp_path / "loop_64_r2_rare.inc") if ln.startswith("v_mov_b32") and ln.endswith(", 0")}
     assert len(written) == 1 and written <= clob and not any(written & regs(ln) for ln in lines)
+
+
+@pytest.mark.parametrize("d,loader", LOOPS)
+def test_a_growing_row_is_not_computed_again(tmp_path, d, loader):
+    """A sum that left the slack without an overflow moves the reference by what is in the registers: no matrix instruction, no
+    operand from LDS, no exponential but the factor's, and with the maximum of the logits of the tile that are complete and still to
+    come (of the second block, of a lane's other eight), or a row that grows would be back for them at the next group."""
+    generate(tmp_path, d, loader)
+    maxima = []
+    for label, path in rare_paths(read_lines(tmp_path / f"loop_{d}_{loader}_rare.inc")).items():
+        if "_rare_" in label:
+            assert not any(ln.startswith(("v_mfma", "ds_")) for ln in path), label
+            assert sum(ln.startswith("v_exp") for ln in path) == 1, label
+            maxima.append(sum(ln.startswith(("v_max_f32", "v_max3_f32")) and ln.count(" v") >= 3 for ln in path))
+    # 2 and more two-operand ones combine lanes and maxima; 8 for 16 logits, 4 for 8
+    want = [2 + 8, 1] * 2 if not loader.startswith("r2") else [2 + 4, 2 + 8] * 4
+    assert [m >= w for m, w in zip(maxima, want)] == [True] * len(want) and len(maxima) == len(want), maxima
 
 
 def test_generator_takes_no_environment_input():
