@@ -1122,7 +1122,16 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* part_o,
 // 112; 80, T = 2048 94 / 78; 136, T = 1024 68 / 57; not causal 40, T = 4096, D = 128 429 / 343, 72 677 / 588, but 104, T = 2048 (of
 // eight and five; seven and six) 248 / 259.  The number of groups is the nearest: with 31 pairs per XCD of 4 blocks, causal, 88 us
 // in one group of all, 86 in two.
-inline int dense_pair_groups(int npairs, int nqb) { return pair_groups(npairs, (64 + nqb - 1) / nqb); }
+// Of workgroups of four waves 64 are resident on an XCD, and two rounds are 128.  With groups of 64 under the causal mask the second group
+// began when the first one's light blocks ended (D = 64, us, groups of 64 / of 128: 4 x 4096, 16 heads 179 / 167.5; 1 x 8192, 16 heads
+// 173.6 / 162; 8 x 1500, 16 heads 70.3 / 67.4; 1 x 3200, 64 heads 126.6 / 110.4; documents of 1000 in 1 x 8192, 16 heads 66.3 / 62.0).  From
+// eight rounds on a late group weighs little and fewer pairs side by side share more (8 x 1024, 64 heads 139.7 / 141.9), without a
+// mask all blocks are alike (8 x 2048, 64 heads 667 / 677).
+inline int dense_pair_groups(int npairs, int nqb, bool four_waves, bool causal) {
+  const bool late_blocks_weigh = causal && (int64_t)((npairs + 7) / 8) * nqb < 512;
+  const int workgroups = four_waves && late_blocks_weigh ? 128 : 64;
+  return pair_groups(npairs, (workgroups + nqb - 1) / nqb);
+}
 
 // Four waves and 128 query rows per workgroup, two workgroups on a compute unit, in place of eight and 256 (head size 64; at 128 the
 // tiles leave room for one).  The two do not wait for each other's barriers, fit documents, the diagonal and a last block of rows
@@ -1168,7 +1177,7 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
   // one workgroup per (query block, batch, head): see the kernel for how ids map to them
   int64_t n;
   if (LOADER == LOAD_DENSE) {
-    q.pair_groups = dense_pair_groups(p.B * p.H, p.nqb);
+    q.pair_groups = dense_pair_groups(p.B * p.H, p.nqb, NW == 4, p.causal != 0);
     n = pair_group_workgroups(p.B * p.H, p.nqb);
   } else {
     q.head_groups = head_groups(p.npairs, p.H);
