@@ -1136,26 +1136,41 @@ inline int dense_pair_groups(int npairs, int nqb, bool four_waves, bool causal) 
 // Four waves and 128 query rows per workgroup, two workgroups on a compute unit, in place of eight and 256 (head size 64; at 128 the
 // tiles leave room for one).  The two do not wait for each other's barriers, fit documents, the diagonal and a last block of rows
 // more closely and fill more compute units where there are few blocks; both stage (or rebuild) every tile, which is what long runs
-// of unmasked tiles lose by.  Where those decide, the two are compared by their rounds of 256 workgroups, a round of four waves as half
-// a round of eight and a tenth (dense tiles, few of them: 2 %) of what they stage twice.  us, eight waves / four, dense tiles
-// with the reconstruction:
-//   documents, causal: 3 x 1777, 16 heads, of 421 tokens 41.7 / 37.7; 4 x 2500, 64 heads, of 800 233.7 / 202.5; 8 x 1200, 64
-//     heads, of 150 174 / 152; 1 x 16 384, 16 heads, of 1000 138.7 / 111.8, of 4000 211 / 207; 2 x 8192 of 2000 147 / 145; but one
-//     document in every row, which the host cannot see: 4 x 4096 160 / 166, 2 x 9000, 8 heads 146 / 162; without a mask 2 x
-//     9000 of 3000 306 / 303; rank 2 fused: 1 x 500, 16 heads, of 200 21.2 / 17.1; 2 x 1700, 8 heads, of 150 21.4 / 17.7
-//   causal: 1 x 700, 16 heads 21.7 / 18.6; 16 x 512, 16 heads 37.2 / 35.3; 4 x 1600, 64 heads 169 / 155; 1 x 2048, 32 heads 49.5 / 43.8;
-//     8 x 1500, 16 heads 74.7 / 76.0; 3 x 2300, 8 heads 48.6 / 40.9; 2 x 2300, 64 heads 129 / 132; 1 x 8192, 16 heads 153 / 174; rank 2
-//     fused: 1 x 256, 8 heads 14.2 / 12.3; 3 x 800, 64 heads 61.9 / 53.3; 16 x 512, 16 heads 34.5 / 34.0
-//   no mask, or many cached keys: 1 x 600, 8 heads 17.9 / 15.1; 3 x 1300, 64 heads 142 / 133; 8 x 600, 64 heads 112.6 / 97.3; 1 x 1000, 64
-//     heads 37.5 / 39.0; 2 x 2000, 16 heads 52.6 / 55.3; rank 2 fused: 8 x 300, 64 heads 59.4 / 46.9; 8 x 700, 64 heads 134 / 145;
-//     16 x 512, 16 heads 37.9 / 41.2; chunks of 300 over 2000, 64 heads 200 / 176, of 512 over 8192 305 / 347
+// of unmasked tiles lose by.  us, eight waves / four, with the reconstruction where the tiles are dense:
+//   Without a mask, or with many cached keys, the two are compared by their rounds of 256 workgroups, a round of four waves as half a round of
+//     eight and a tenth (dense tiles, few of them: 2 %) of what they stage twice.  1 x 600, 8 heads 20.5 / 17.5; 3 x 1300, 64 heads 138 /
+//     131; 8 x 600, 64 heads 123 / 109; 2 x 2000, 16 heads 50.7 / 59.7; rank 2 fused: 8 x 300, 64 heads 59.3 / 46.7; 1 x 300, 64 heads 15.9 /
+//     13.6; 1 x 1000, 64 heads 30.1 / 33.8; 8 x 700, 64 heads 130 / 135; chunks of 300 over 2000, 64 heads 200 / 176, of 512 over 8192 305 / 347
+//   Causal: up to about a round and a half of eight waves the longest block decides, and half of it ends sooner: 1 x 2048, 32 heads 48.0 / 41.5;
+//     3 x 2300, 8 heads 48.6 / 40.4; 1 x 2304, 32 heads 52.8 / 47.2; 1 x 2816, 32 heads 61.1 / 57.5; rank 2 fused: 1 x 700, 16 heads 21.6 / 18.5; 1 x
+//     1800, 32 heads 43.3 / 37.9; 4 x 1024, 16 heads 28.7 / 26.7.  But not where the fused kernel's mapping leaves each XCD one block of all
+//     heads, light or heavy, and more of them than compute units: 1 x 1024, 64 heads 30.0 / 33.6; 2 x 512, 64 heads 20.4 / 22.8.
+//     Beyond, the tiles that all blocks visit decide, of which blocks of 128 rows have fewer (the diagonal, the last block), with 6 % for staging
+//     them twice (rank 2 fused, rebuilding: 13 %): 8 x 1024, 64 heads 148 / 141; 8 x 1500, 16 heads 70.5 / 68.4; 4 x 1600, 64 heads 163 / 146; 1 x
+//     3200, 64 heads 117 / 111; but 3 x 2048, 16 heads 49.2 / 51.4; 4 x 2048 56.4 / 57.6; 2 x 4000 87.3 / 91.9; 4 x 4096 166 / 169; 1 x 8192 153 / 163;
+//     fused 12 x 768, 32 heads 91.9 / 85.6; 16 x 512, 16 heads 36.7 / 34.7.
+//   Segment ids: what the rows hold the host cannot see, and documents are what ids are for.  Causal: 3 x 1777, 16 heads, of 421 tokens 43.4 /
+//     38.4; 4 x 2500, 64 heads, of 800 236 / 202; 1 x 8192, 16 heads, of 1000 70.9 / 62.2; 1 x 16 384, 16 heads, of 1000 136 / 113, of 4000 234 / 216;
+//     one document in every row loses: 4 x 4096, 16 heads 172.5 / 174.5, 2 x 9000, 8 heads 198 / 194, 1 x 8192, 16 heads 153 / 166, 1 x 16 384
+//     549 / 571.  Without a mask 4 x 4096, 16 heads, of 1000 148 / 138, one document 289 / 299; 16 x 512, 16 heads, of 100 43.6 / 40.9, one 44.4 / 46.3; but
+//     in one round of eight waves 2 x 2000, 16 heads, of 300 31.1 / 34.1, one 51.7 / 60.4.
 inline bool wants_four_waves(const PrefillParams& p, bool dense) {
-  if (p.kvseg) return true;
-  const int64_t pairs = (int64_t)p.B * p.H, eight = pairs * ((p.lq + 255) / 256), four = pairs * ((p.lq + 127) / 128);
-  const bool triangle = p.causal && p.lk < 2 * (int64_t)p.lq;  // masked tiles are a good part of all
-  if (triangle && (p.lk <= 2048 || (dense && eight < 256 && p.lk <= 4096))) return true;
-  const double staging = dense && p.lk <= 1408 ? 1.02 : triangle ? 1.2 : 1.1;
-  return staging * (double)((four + 255) / 256) < 2.0 * (double)((eight + 255) / 256);
+  const int64_t pairs = (int64_t)p.B * p.H, blocks = (int64_t)p.B * ((p.lq + 127) / 128);
+  const int64_t eight = pairs * ((p.lq + 255) / 256), four = p.H * blocks;
+  const double staging = dense && p.lk <= 1408 ? 1.02 : 1.1;
+  const bool rounds = staging * (double)((four + 255) / 256) < 2.0 * (double)((eight + 255) / 256);
+  const bool one_block_per_xcd = !dense && blocks == 8 && p.H > 32;  // pair_of_workgroup
+  if (p.kvseg) return p.causal ? !one_block_per_xcd : eight > 256 || rounds;
+  if (!p.causal || p.lk >= 2 * (int64_t)p.lq) return rounds;  // masked tiles are a small part of all
+  if (p.lq > 8192 || p.lk > 8192 || one_block_per_xcd) return false;
+  if (eight <= 352 && p.lk <= (dense ? 4096 : 2048)) return true;
+  const int offset = p.coff + (p.causal == TPA_CAUSAL_BOTTOM_RIGHT ? p.lk - p.lq : 0);
+  auto tiles = [&](int rows) {  // of all blocks of so many query rows
+    int64_t n = 0;
+    for (int q0 = 0; q0 < p.lq; q0 += rows) n += (max(0, min(p.lk, q0 + rows + offset)) + kTK - 1) / kTK;
+    return (double)n;
+  };
+  return (dense ? 1.06 : 1.13) * tiles(128) < 2.0 * tiles(256);
 }
 
 template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8>
