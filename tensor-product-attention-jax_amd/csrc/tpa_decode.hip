@@ -1079,10 +1079,14 @@ int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream,
 // rank 4 on that decides (3 x 9000 keys, 64 heads of 64, rank 4: 24.1 us non-temporal, 22.5 ordinary; rank 2 19.1 / 19.2, paged
 // 52.0 / 54.3), with one row from rank 16 on (48 x 4096 keys, 64 heads of 64: rank 4 94 / 93, rank 8 180 / 179 - 187, paged
 // 140 / 133; 16 380 / 356 and 270 / 250; 32 831 / 700 and 557 / 468; with one block of loads in flight, non-temporal, 798 and 518).
+bool far_rows(const TpaFwdArgs* a) {
+  for (const TpaFactor* f : {&a->ka, &a->kb, &a->va, &a->vb})
+    if (f->stride_r < 0 || f->stride_r > kFarthestRow) return true;
+  return false;
+}
 template <int D, int RK, bool PAGED>
 int launch_decode_rows(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, RowWindow rows) {
-  for (const TpaFactor* f : {&a->ka, &a->kb, &a->va, &a->vb})
-    if (f->stride_r < 0 || f->stride_r > kFarthestRow) return launch_decode_t<D, RK, PAGED, 2, Reads::kFar>(a, ranges, stream, rows);
+  if (far_rows(a)) return launch_decode_t<D, RK, PAGED, 2, Reads::kFar>(a, ranges, stream, rows);
   if (a->lq == 1) {
     if constexpr (RK >= 16)
       if (a->H > 32) return launch_decode_t<D, RK, PAGED, 1, Reads::kOrdinary>(a, ranges, stream, rows);
@@ -1110,23 +1114,35 @@ int launch_decode(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream, Row
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
+// ranges whose partials (at head size 128) the fixed array of tpa_decode_noalloc holds
+int noalloc_room(int B, int lq, int H) { return (int)(TPA_DECODE_NOALLOC_SCRATCH_BYTES / workspace_bytes(B, lq, H, 128, 1)); }
+
 // Key ranges per batch entry that the workspace is sized for.  One workgroup per compute unit is resident (the kernel
 // keeps two blocks of loads in flight in registers), so there are as many as fill 256 of them.  A wave then has at
 // least one block of rank 2; where that would take more partials than four blocks per wave
 // and more than the fixed array of tpa_decode_noalloc holds (at head size 128), it has four.
 // (One sequence of 1500 keys, 16 heads of 128, with the merge: 17.3 us with 6 ranges of four blocks per wave, 14.1 with
 // 12 of two, 12.3 with 24 of one.)
-// The bf16 kernel serves two query rows per workgroup, which is what callers are told to size
-// the workspace for; the fp32 kernel serves one, launches twice the workgroups per range and so
+// The fp32 kernel serves one query row per workgroup, launches at least twice the workgroups per range of the bf16 kernel and so
 // asks for at most as many ranges (and never more workspace).
-int default_splits(int B, int lq, int lk, int H, int rows_per_group = 2) {
+int splits_for(int B, int lq, int lk, int H, int rows_per_group) {
   const int64_t groups = (int64_t)B * ((lq + rows_per_group - 1) / rows_per_group) * ((H + 31) / 32);
   if (groups >= 256) return 1;
   const int want = (int)((256 + groups - 1) / groups);
   const int few = std::min(want, (lk + 4 * kMinKeys - 1) / (4 * kMinKeys));
-  const int room = (int)(TPA_DECODE_NOALLOC_SCRATCH_BYTES / workspace_bytes(B, lq, H, 128, 1));
-  return std::max({1, few, std::min({want, (lk + kMinKeys - 1) / kMinKeys, room})});
+  return std::max({1, few, std::min({want, (lk + kMinKeys - 1) / kMinKeys, noalloc_room(B, lq, H)})});
 }
+// The bf16 kernel, which is what callers are told to size the workspace for, serves two query rows per workgroup, or four where eight
+// heads lie side by side (launch_decode_rows).  Counted as two, these were at most half as many workgroups as compute units: us, 8 heads, so /
+// counted as four: 20 x 8192 keys, head size 64, four rows 29.4 / 23.1, rank 8 78.5 / 62.5; 50 x 4096, 128, four rows 62.1 / 44.9; 3 x 16384,
+// 64, 16 rows 30.8 / 21.2; 6 x 8192 dealt by length 14.8 / 14.4; one sequence is bound by its chain: 1 x 32768, 128, three rows 21.1 / 22.0.  The ranges that this adds
+// are no more than the fixed array holds, so that nothing it took is refused.
+int default_splits(int B, int lq, int lk, int H, int rows_per_group) {
+  const int two = splits_for(B, lq, lk, H, std::min(rows_per_group, 2));
+  if (rows_per_group <= 2) return two;
+  return std::max(two, std::min(splits_for(B, lq, lk, H, rows_per_group), noalloc_room(B, lq, H)));
+}
+int rows_per_workgroup(int H) { return H == 8 ? 4 : 2; }
 
 // How a launch splits the keys if the caller leaves it to us, with partials for B * default_splits ranges at hand.
 // With lengths per batch entry the ranges are dealt by them; otherwise all entries get one count, which fills the chip
@@ -1150,12 +1166,12 @@ KeyRanges choose_ranges(const TpaFwdArgs* a, int rows_per_group) {
 
 extern "C" int32_t tpa_decode_default_splits(int32_t B, int32_t lq, int32_t lk, int32_t H) {
   if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0) return 0;
-  return tpa::default_splits(B, lq, lk, H);
+  return tpa::default_splits(B, lq, lk, H, tpa::rows_per_workgroup(H));
 }
 
 extern "C" size_t tpa_decode_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dv, int32_t num_splits) {
   if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0 || dv <= 0) return 0;
-  const int S = num_splits > 0 ? num_splits : tpa::default_splits(B, lq, lk, H);
+  const int S = num_splits > 0 ? num_splits : tpa::default_splits(B, lq, lk, H, tpa::rows_per_workgroup(H));
   return tpa::workspace_bytes(B, lq, H, dv, S);
 }
 
@@ -1182,9 +1198,10 @@ int tpa_decode_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) { return tpa
 int tpa_decode_mfma_launch_rows(const TpaFwdArgs* a, hipStream_t stream, int row0, int lq_total) {
   using namespace tpa;
   const RowWindow rows{row0, lq_total};
-  const int S = a->num_splits > 0 ? a->num_splits : default_splits(a->B, a->lq, a->lk, a->H);
+  const int rows_each = far_rows(a) ? 2 : rows_per_workgroup(a->H);  // as launch_decode_rows has it
+  const int S = a->num_splits > 0 ? a->num_splits : default_splits(a->B, a->lq, a->lk, a->H, rows_each);
   if (S > 65535 || (int64_t)a->B * S > 2147483647LL) return TPA_ERR_SHAPE;
-  const KeyRanges ranges = a->num_splits > 0 ? KeyRanges{S, 0} : choose_ranges(a, 2);
+  const KeyRanges ranges = a->num_splits > 0 ? KeyRanges{S, 0} : choose_ranges(a, rows_each);
   if (!a->workspace || a->workspace_bytes < workspace_bytes(a->B, a->lq, a->H, a->dv, S)) return TPA_ERR_WORKSPACE;
   if (!aligned16(a->workspace)) return TPA_ERR_ALIGN;
   if (a->dk == 128) {
@@ -1293,7 +1310,7 @@ extern "C" int tpa_decode_noalloc(const TpaFwdArgs* a, void* stream) {
   if (a->q_segment_ids) return TPA_ERR_UNSUPPORTED;
   const bool bf16 = tpa_decode_mfma_supported(a), f32 = !bf16 && tpa_decode_f32_supported(a);
   if (a->kernel == TPA_KERNEL_GENERIC || (!bf16 && !f32)) return TPA_ERR_UNSUPPORTED;  // the split-key kernels only
-  const int S = a->num_splits > 0 ? a->num_splits : default_splits(a->B, a->lq, a->lk, a->H, bf16 ? 2 : 1);
+  const int S = a->num_splits > 0 ? a->num_splits : default_splits(a->B, a->lq, a->lk, a->H, bf16 ? rows_per_workgroup(a->H) : 1);
   if (S > 65535 || (int64_t)a->B * S > 2147483647LL) return TPA_ERR_SHAPE;
   if (workspace_bytes(a->B, a->lq, a->H, a->dv, S) > (size_t)TPA_DECODE_NOALLOC_SCRATCH_BYTES) return TPA_ERR_WORKSPACE;  // partials exceed the fixed array
   void* ptr = nullptr;
