@@ -241,9 +241,11 @@ struct DecodeLds {
 // At head size 64 and from rank 4 on two workgroups fit a compute unit, which the compiler has to be told: at 258 registers
 // instead of 256 rank 8 lost the second one (64 heads, two rows per workgroup: 48 x 4096 keys, eight rows 544 -> 707 us; 4 x 1024
 // rows and keys without K and V 2.42 -> 3.15 ms; 2.10 so, with 204).
-constexpr int min_waves(int d, int rk) { return d == 64 && rk >= 4 ? 2 : 1; }
+// So it is with rows side by side at every rank: 256 to 260 registers at ranks 1 and 2, three of four instances without the second
+// workgroup (us, 16 heads, before / now: 300 x 1000 keys, rank 1, two rows 34.0 / 28.5; 64 x 8192, rank 2, four rows 75.0 / 68.7; 4 x 8192 13.4 / 12.6).
+constexpr int min_waves(int d, int rk, bool side) { return d == 64 && (rk >= 4 || side) ? 2 : 1; }
 template <int D, int RK, bool PAGED, int NQ, Reads READS, bool SIDE = false>
-__global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(DecodeParams p) {
+__global__ __launch_bounds__(kWaves * 64, min_waves(D, RK, SIDE)) void decode_kernel(DecodeParams p) {
   constexpr int CPR = D / 8;               // 16-byte chunks per B row
   constexpr int RPI = 64 / CPR;            // B rows per load instruction
   constexpr int NLB = kRowsPerBlock / RPI; // load instructions per B tile
@@ -283,35 +285,28 @@ __global__ __launch_bounds__(kWaves * 64, min_waves(D, RK)) void decode_kernel(D
   const TileAt<D> at(l);
 
   // ---- Qm^T fragments: requested ahead of the cache's first blocks, finished while those are in flight.
-  // With one query row they stay in registers; with several wave r builds row r's fragments once
+  // With one query row they stay in registers; with several (no more than waves) wave r builds row r's fragments once
   // and parks them in LDS behind the waves' staging regions (fragment (set, ks) of lane l at
   // [(set NKS + ks) 64 + l], written by the lanes whose row it is: another row's infinities never
   // meet theirs), from where every wave reads them: one set into its registers, two as it needs them,
   // when the registers go to the accumulators instead.
+  static_assert(!SIDE || NQ == 1, "rows side by side are one set");
   bf16x8 qf[NQ == 1 ? NKS : 1];
   u32x4* const lds_q = reinterpret_cast<u32x4*>(smem + kWaves * DecodeLds<D>::kPerWave);
-  const uint16_t* qa_row;
-  const uint16_t* qb_row;
-  auto q_row = [&](int row) __attribute__((always_inline)) {
-    qa_row = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)row * p.qa.stride_l + hl;
-    qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)row * p.qb.stride_l;
-  };
-  q_row(NQ == 1 && !SIDE ? qi0 : min(qi0 + w, p.lq - 1));
-  auto build_q = [&](QRaw<D> raw) __attribute__((always_inline)) {
+  const int qi_build = NQ == 1 && !SIDE ? qi0 : min(qi0 + w, p.lq - 1);
+  const uint16_t* const qa_row = static_cast<const uint16_t*>(p.qa.ptr) + b * p.qa.stride_b + (int64_t)qi_build * p.qa.stride_l + hl;
+  const uint16_t* const qb_row = static_cast<const uint16_t*>(p.qb.ptr) + b * p.qb.stride_b + (int64_t)qi_build * p.qb.stride_l;
+  auto build_q = [&](const QRaw<D>& raw) __attribute__((always_inline)) {
     if constexpr (NQ == 1 && !SIDE) {
       finish_q_fragments<D>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, l, lds, at, qf);
     } else {
-      for (int r = w; r < rpw; r += kWaves) {
+      if (w < rpw) {
         bf16x8 tmp[NKS];
         finish_q_fragments<D>(raw, qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, p.rq, p.qscale, l, lds, at, tmp);
-        const int set = SIDE ? r / rps : r;
-        if (!SIDE || ci == r - set * rps) {
+        if (!SIDE || ci == w) {
 #pragma unroll
-          for (int ks = 0; ks < NKS; ++ks) lds_q[(set * NKS + ks) * 64 + l] = __builtin_bit_cast(u32x4, tmp[ks]);
+          for (int ks = 0; ks < NKS; ++ks) lds_q[((SIDE ? 0 : w) * NKS + ks) * 64 + l] = __builtin_bit_cast(u32x4, tmp[ks]);
         }
-        if (!SIDE || r + kWaves >= rpw) break;
-        q_row(min(qi0 + r + kWaves, p.lq - 1));
-        raw = load_q_factors<D>(qa_row, p.qa.stride_r, qb_row, p.qb.stride_r, 0, p.rq, l);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the cache's loads stay in flight
       if constexpr (NQ == 1) {
@@ -1067,10 +1062,10 @@ int launch_decode_f32(const TpaFwdArgs* a, KeyRanges ranges, hipStream_t stream,
   return launch_decode_f32_t<D, RK, false>(a, ranges, stream, rows);
 }
 
-// 8 and 16 heads leave columns of the matrix instructions to other query rows: 32 / H rows then cost what one does, with the
+// 8 and 16 heads leave columns of the matrix instructions to other query rows: 32 / H rows then cost what one does, with about the
 // registers of one row (two sets of loads in flight).  Decode and merge, us, two rows of one set of columns each / side by side:
 // 64 x 8192 keys, 16 heads of 128, four rows 166.7 / 124.0, two rows 101.7 / 100.8 (HBM); rank 8, head size 64, four rows 348 / 245; 8
-// heads, rank 4, eight rows 308 / 203; step of 48 paged sequences of 2046 .. 4096 keys, 16 heads of 128, four tokens 91.2 / 75.7.
+// heads of 64, 300 x 1000 keys, four rows 85.4 / 43.4; 1 x 8192, head size 128, rank 4, eight rows 24.0 / 17.7; step of 48 paged sequences of 2046 .. 4096 keys, 16 heads of 128, four tokens 91.2 / 75.7.
 // Two sets of rows side by side in one workgroup are slower (158.7 at the first shape): one set of loads in flight.
 // One row group per cache slice: each byte is used once and the loads are marked non-temporal (the whole call 5.1 -> 5.75 TB/s).
 // Several (more query rows than a workgroup serves): the groups' workgroups run side by side on one XCD and the later one is
