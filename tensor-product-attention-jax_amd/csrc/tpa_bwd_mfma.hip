@@ -634,20 +634,24 @@ int launch(const BwdParams& base, hipStream_t stream) {
 //     559; 1 x 2600, 64 heads 359 / 351; 8 x 3000, 16 heads 904 / 908; 1 x 8192, 16 heads 636 / 654; few workgroups: 1 x 3000, 8 heads 137.6 /
 //     126.5; 1 x 6000, 8 heads 248 / 235; 1 x 4096, 16 heads 213 / 210.5; 2 x 4000, 16 heads 354 / 360; 1 x 10 000, 8 heads 517 / 522
 //   no mask, where the rounds of 256 workgroups decide (of four waves half a round of eight and 4 %): 8 x 300, 64 heads 197 / 181; 8 x 600
-//     445 / 420; 3 x 1300, 64 heads 544 / 530; 4 x 1000, 64 heads 443 / 449; 3 x 2100, 8 heads 170 / 174.5; 4 x 2048, 16 heads 361 / 376; all in
-//     one round: 1 x 1500, 16 heads 95 / 90; 1 x 4000, 8 heads 189 / 182
+//     468 / 439; 3 x 1300, 64 heads 555 / 542; 2 x 2300, 16 heads 269 / 262; 4 x 1000, 64 heads 443 / 449; 3 x 2100, 8 heads 170 / 174.5; 4 x 2048, 16
+//     heads 361 / 376; all in one round: 1 x 1500, 16 heads 95 / 90; 1 x 4000, 8 heads 189 / 182.  Long blocks lose more by staging and less by a
+//     last round that is not full: 3 x 4809, 16 heads 1349 / 1382, 4 x 5350 2166 / 2238, 1 x 5000 514 / 535, 2 x 4000 610 / 639
 // (64 keys per wave would halve the LDS reads per MFMA, but its 384 stationary registers at D = 128 leave the compiler
 // spilling; the dQ kernel with 4 waves of 64 rows, one wave per SIMD and 512 registers, takes 922 us where 8 waves of 32
 // rows take 401 us.)
+inline bool bwd_wants_four_waves(const BwdParams& p) {
+  if (p.qseg) return true;
+  const int64_t pairs = (int64_t)p.B * p.H;
+  auto rounds = [&](int64_t block) { return (pairs * ((p.lq + block - 1) / block + (p.lk + block - 1) / block) + 255) / 256; };
+  if (p.causal) return (p.lq <= 2816 && p.lk <= 2816) || rounds(256) <= 2;
+  return rounds(256) == 1 || (p.lq <= 2560 && p.lk <= 2560 && 1.04 * (double)rounds(128) < 2.0 * (double)rounds(256));
+}
 template <int D>
 int launch_both(const BwdParams& p, hipStream_t stream) {
   if constexpr (D == 64) {
     if (p.qseg) return launch<D, 4, 1, true>(p, stream);
-    const int64_t pairs = (int64_t)p.B * p.H;
-    auto rounds = [&](int block) { return (pairs * ((p.lq + block - 1) / block + (p.lk + block - 1) / block) + 255) / 256; };
-    if (p.causal ? (p.lq <= 2816 && p.lk <= 2816) || rounds(256) <= 2 : rounds(256) == 1 || 1.04 * (double)rounds(128) < 2.0 * (double)rounds(256))
-      return launch<D, 4, 1, false>(p, stream);
-    return launch<D, 8, 1, false>(p, stream);
+    return bwd_wants_four_waves(p) ? launch<D, 4, 1, false>(p, stream) : launch<D, 8, 1, false>(p, stream);
   } else {
     return p.qseg ? launch<D, 8, 1, true>(p, stream) : launch<D, 8, 1, false>(p, stream);
   }

@@ -1,5 +1,5 @@
-"""Host rules of the prefill launcher (csrc/tpa_prefill.hip), compiled here from its own text, without a GPU: how the workgroups
-over dense tiles are ordered on an XCD, and which calls take workgroups of four waves."""
+"""Host rules of the launchers of the prefill and the backward (csrc/tpa_prefill.hip, tpa_bwd_mfma.hip), compiled here from their own
+text, without a GPU: how the workgroups over dense tiles are ordered on an XCD, and which calls take workgroups of four waves."""
 
 import ctypes
 import os
@@ -32,7 +32,10 @@ def rules(tmp_path_factory):
         + "enum { TPA_CAUSAL_BOTTOM_RIGHT = 2 };\nconstexpr int kTK = 64;\n"
         + "struct PrefillParams { int B, H, lq, lk, causal, coff; const int32_t* kvseg; };\n"
         + "".join(function(n, "tpa_prefill.hip") for n in ("dense_pair_groups", "wants_four_waves"))
+        + "struct BwdParams { int B, H, lq, lk, causal; const int32_t* qseg; };\n"
+        + function("bwd_wants_four_waves", "tpa_bwd_mfma.hip")
         + """
+extern "C" int bwd_four_waves(int B, int lq, int lk, int H, int causal) { return bwd_wants_four_waves({B, H, lq, lk, causal, nullptr}); }
 extern "C" int four_waves(int B, int lq, int lk, int H, int causal, int coff, int ids, int dense) {
   return wants_four_waves({B, H, lq, lk, causal, coff, ids ? &ids : nullptr}, dense);
 }
@@ -112,3 +115,26 @@ def test_the_rule_ends_where_blocks_are_many(rules):
     for causal, coff in ((1, 0), (1, -big // 2), (1, big // 2), (2, 0)):
         rules.four_waves(1, big // 2, big // 2, 1, causal, coff, 0, 1)
         rules.four_waves(1, big // 2, 4096, 1, causal, 0, 0, 1)
+
+
+# the same of training steps
+BACKWARD_PLAIN = {
+    (3, 4809, 16): (1349, 1382), (4, 5350, 16): (2166, 2238), (1, 5000, 16): (513.6, 534.5), (2, 4000, 16): (610, 639), (4, 3000, 16): (722, 756),
+    (2, 3000, 64): (1468, 1509), (1, 10000, 16): (1793, 1827), (4, 2500, 16): (539, 557), (5, 1800, 16): (412, 410), (3, 900, 64): (322, 328),
+    (2, 2300, 16): (268.7, 261.7), (3, 2300, 16): (365, 361.7), (3, 1400, 16): (186.7, 182.6), (3, 1300, 64): (554.6, 542.4), (8, 600, 64): (467.5, 438.8),
+    (16, 300, 16): (112.7, 104.9), (2, 1700, 32): (291.8, 288.7), (7, 1100, 16): (260.3, 246.6), (1, 2100, 64): (421.4, 413.8), (5, 1200, 32): (395.9, 393.0),
+    (1, 1000, 64): (123.1, 124.8), (2, 2000, 16): (192.9, 197.4), (4, 1024, 16): (124.0, 128.8), (4, 2048, 16): (369.4, 377.9), (1, 1500, 16): (95.0, 89.9),
+}
+BACKWARD_CAUSAL = {
+    (1, 2048, 32): (132.3, 129.8), (4, 2048, 16): (244.4, 243.7), (8, 1500, 16): (306.6, 303.6), (8, 1024, 16): (192.7, 174.9), (16, 512, 16): (162.1, 144.9),
+    (4, 1600, 64): (687, 660.6), (2, 2816, 16): (209.5, 208.9), (1, 4096, 8): (171.5, 160.3), (1, 4096, 16): (216.4, 214.0), (2, 3500, 16): (286.3, 292.7),
+    (1, 5000, 16): (295.4, 295.6), (6, 2500, 16): (500.1, 501.0), (5, 1800, 16): (269.6, 261.8), (7, 1100, 16): (188.6, 177.3), (1, 3300, 32): (260.8, 262.9),
+}
+
+
+@pytest.mark.parametrize("table,causal", [(BACKWARD_PLAIN, 0), (BACKWARD_CAUSAL, 1)])
+def test_four_waves_in_the_backward_where_they_were_measured_faster(rules, table, causal):
+    """Within 2 %: the forward and the reconstruction are in both sides."""
+    for (b, t, h), sides in table.items():
+        four = rules.bwd_four_waves(b, t, t, h, causal)
+        assert sides[four] <= 1.02 * min(sides), ((b, t, h), "four" if four else "eight", sides)
