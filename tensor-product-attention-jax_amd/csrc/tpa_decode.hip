@@ -1144,7 +1144,7 @@ int rows_per_workgroup(int H) { return H == 8 ? 4 : 2; }
 // at most once: 288 workgroups take two rounds, the second nearly empty (48 x 4096 keys, 32 heads of 128: 6 ranges each 69.5 us, 5 48.6).
 // What some wave has to do is a whole number of blocks, so there are no more ranges than that number needs: the others would only
 // be partials to merge (1 x 20 000 keys, 16 heads of 128: 63 ranges of up to ten blocks per wave 34.3 us, fewer 26.3; 3 x 9000, 32 heads
-// 22.1 / 19.7; five paged sequences dealt by length, 4 x 8192 keys 32.2 / 29.6, 24 x 1024 25.0 / 23.2).
+// 22.1 / 19.7).
 KeyRanges choose_ranges(const TpaFwdArgs* a, int rows_per_group) {
   const int S = default_splits(a->B, a->lq, a->lk, a->H, rows_per_group);
   const int per_range = (a->lq + rows_per_group - 1) / rows_per_group * ((a->H + 31) / 32);  // workgroups of one range

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
   const int tid = threadIdx.x;
   const int w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
   const int q0 = qblk * kRows;
-  // row block r of this wave within the workgroup's eight
+  // row block r of this wave within the workgroup's (one per wave)
   int rblk[RB], wrow0[RB], qrow[RB], qrow_ld[RB];
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
         }
       }
     } else {
-      // One rank at a time through LDS: the workgroup copies the 256 x D slab qb[q0.., r, :] with
+      // One rank at a time through LDS: the workgroup copies the kRows x D slab qb[q0.., r, :] with
       // coalesced 16-byte loads (each row is read once, not once per lane pair), then every lane
       // picks up its own row's fragments.  The next rank's loads are in flight meanwhile.
       constexpr int QS = D + 8;                  // row stride in LDS (elements)
@@ -376,8 +376,8 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
 
   // Head factors (LOAD_TPA_R2): a thread fetches one value a[matrix][token][rank], matrix = (tid % 256) / 128
   // (0: K of tile kt, 1: V of tile vt), token = (tid / 2) % 64, rank = tid % 2, and parks it in a register
-  // until it is stored into an LDS slot one iteration later.  Waves 4-7 repeat what waves 0-3 do (same
-  // values to the same addresses), so that the eight waves run one instruction stream.
+  // until it is stored into an LDS slot one iteration later.  Where there are eight, waves 4-7 repeat what waves 0-3 do (same
+  // values to the same addresses), so that all run one instruction stream.
   uint32_t a_pending = 0;
   const int a_idx = tid & (4 * kTK - 1);
   const int a_mat = scalar(a_idx / (2 * kTK)), a_tok = (a_idx >> 1) % kTK, a_rank = a_idx & 1;
@@ -1286,14 +1286,15 @@ int tpa_prefill_wants_dense(int64_t lq, int64_t lk, int64_t rk) {
 
 namespace tpa {
 namespace {
-// The same for one call, of which the number of workgroups is known.  Rank 2 below 2048 rows, dense over fused time, no mask /
-// causal / packed documents, 8 to 400 (batch, head) pairs of 257 to 2040 rows each, one to five times as many keys:
+// The same for one call, of which the number of workgroups (of 256 rows) is known.  Rank 2 below 2048 rows, dense over fused time, no
+// mask / causal / packed documents, 8 to 400 (batch, head) pairs of 512 to 2040 rows each (head size 64 with four or eight waves as
+// wants_four_waves has it for either):
 //   at most 64 workgroups: the prologue with its loads and Q is most of the time, and shorter without the factors.  D = 128
-//     0.76 - 1.01 (8 pairs of 512 rows 27 / 23 us); D = 64 0.89 - 1.16, not taken
-//   65 to 256: every compute unit rebuilds for itself and the reconstruction is a launch more.  0.84 - 1.40, from 0.97 on for
-//     most; 128 pairs of 512 rows 22 / 29 us, but 24 pairs of 2040 rows, D = 128 75 / 66
-//   more, from 1000 rows on: 0.77 - 1.07 (48 pairs of 1777, D = 64, documents of 421 tokens 46 / 41 us)
-//   more, of fewer rows: 0.83 - 1.04, with more keys than rows up to 1.32
+//     0.78 - 0.86 (8 pairs of 512 rows 27.4 / 22.5 us); D = 64 0.87 - 0.99, with more keys than rows up to 1.16, not taken
+//   65 to 256: every compute unit rebuilds for itself and the reconstruction is a launch more.  D = 64 0.92 - 1.32 (128 pairs of 512
+//     rows 19.5 / 25.8, but 24 pairs of 2040 40.1 / 37.0), D = 128 0.84 - 1.10 (128 pairs of 512 31.5 / 34.5, but 24 of 2040 66.7 / 58.3)
+//   more, from 1000 rows on: D = 64 0.83 - 0.98 (48 pairs of 1777 49.1 / 43.1, with documents of 421 tokens 39.3 / 38.2), D = 128 0.77 - 0.99
+//   more, of fewer rows: 512 rows 1.01 - 1.07, 700 to 900 0.81 - 0.99, with more keys than rows up to 1.32
 bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   if (tpa_prefill_wants_dense(lq, lk, rk)) return true;
   if (rk != 2 || lq <= kBQ || lk > 5 * lq) return false;
@@ -1344,7 +1345,7 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
   p.npairs = p.nqb * a->B;
   // With a workspace Q (times sm_scale * log2 e), K and V are reconstructed once as dense bf16 and
   // the kernel runs with its plain tile loader: no workgroup rebuilds tiles from the rank factors
-  // (the fused kernel does that once per 256 query rows and head).
+  // (the fused kernel does that once per workgroup's query rows and head).
   const bool usable = a->workspace && !(reinterpret_cast<uintptr_t>(a->workspace) & 255);
   const PrefillRoute route = route_of(a);
   const bool dense = usable && route.dense && a->workspace_bytes >= route.dense;
