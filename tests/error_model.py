@@ -96,7 +96,8 @@ def emulate_bf16_attention(qd, kd, vd, sm_scale, bias=None, q_prescaled=False, f
         o  = bf16( (sum_k P_k V'_k) / l )   lse = (m + log2 l) / log2 e
 
     Because m is a whole number, P has the mantissa of bf16(2^x) whatever m is: the kernels' choice of
-    reference (the first tile's maximum rounded up, moved by whole numbers) changes no bit of P, so this
+    reference (the first tile's maximum rounded up, moved by whole numbers) changes P only where the fp32 sum
+    of a logit, which starts at -m, rounds elsewhere.  So this
     emulation and a kernel differ only by fp32 summation order, the fp32 accuracy of exp2 and rare double
     roundings - a few output elements in a thousand, by one bf16 spacing.
 

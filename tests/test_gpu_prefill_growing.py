@@ -1,10 +1,10 @@
 """Rows whose logits grow along the keys.
 
 The generated loops of the prefill kernel keep one reference per row and move it when the sum of a group of
-exponentials says so; they then compute the group's logits again.  Here the reference has to move in every group a lane can
+exponentials says so; the group is then scaled, or, where its sum overflowed, computed again.  Here the reference has to move in every group a lane can
 own (both 32-key blocks of a tile, both halves of a block, both tile parities), by little and by more than the range of a float
 at once, for some rows of a wave and not for others, in both loops and both head sizes; against the emulation of the
-kernels' rounding points, of which no bit depends on the reference.
+kernels' rounding points, of which only the start of a logit's fp32 sum depends on the reference.
 
 The head factors are powers of two on one rank, so that Q, K and V are exact before their one rounding: a rounding that falls
 the other way would move a logit of a thousand by more than a group's worth."""
