@@ -473,11 +473,11 @@ def scale_path(name, temps, free, packed, raw, moved):
     return e.lines
 
 def full_path(name, f, frag_load, set_address, temps, again, whole, moved, redo):
-    """The same for a sum that may have overflowed, behind matrix instruction f.  `again` = (register, byte offset of its rows in a K buffer) of the blocks whose logits are computed again,
-    `whole` = those of a later block that are complete and not touched yet: its maximum counts at once, or a row that grows would
-    come here again for it; `moved` = the logits of blocks whose accumulation began at the old reference, `redo` = the recorded exponentials that
-    were issued.  `temps` = the registers of the group's sum and its two temporaries, which `redo` writes anew.  The fragments that the
-    loop has read ahead are overwritten here and read again at the end."""
+    """The same for a sum that may have overflowed, behind matrix instruction f.  `again` = (register, byte offset of its rows in a K
+    buffer) of the blocks whose logits are computed again, `whole` = the logits of a later block that are complete and not touched yet,
+    `moved` = those of blocks whose accumulation began at the old reference, `redo` = the recorded exponentials that were issued.  `temps` =
+    the registers of the group's sum and its two temporaries, which `redo` writes anew.  The fragments that the loop has read ahead are
+    overwritten here and read again at the end."""
     e = Stream()
     e.raw(f".Lpf_full_{name}_%=:")
     e.raw("s_waitcnt lgkmcnt(0)")

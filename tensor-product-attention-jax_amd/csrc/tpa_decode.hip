@@ -1128,10 +1128,10 @@ int splits_for(int B, int lq, int lk, int H, int rows_per_group) {
   return std::max({1, few, std::min({want, (lk + kMinKeys - 1) / kMinKeys, noalloc_room(B, lq, H)})});
 }
 // The bf16 kernel, which is what callers are told to size the workspace for, serves two query rows per workgroup, or four where eight
-// heads lie side by side (launch_decode_rows).  Counted as two, these were at most half as many workgroups as compute units: us, 8 heads, so /
-// counted as four: 20 x 8192 keys, head size 64, four rows 29.4 / 23.1, rank 8 78.5 / 62.5; 50 x 4096, 128, four rows 62.1 / 44.9; 3 x 16384,
-// 64, 16 rows 30.8 / 21.2; 6 x 8192 dealt by length 14.8 / 14.4; one sequence is bound by its chain: 1 x 32768, 128, three rows 21.1 / 22.0.  The ranges that this adds
-// are no more than the fixed array holds, so that nothing it took is refused.
+// heads lie side by side (launch_decode_rows).  Counted as two, these were at most half as many workgroups as compute units: us, 8
+// heads, so / counted as four: 20 x 8192 keys, head size 64, four rows 29.4 / 23.1, rank 8 78.5 / 62.5; 50 x 4096, 128, four rows 62.1 /
+// 44.9; 3 x 16384, 64, 16 rows 30.8 / 21.2; 6 x 8192 dealt by length 14.8 / 14.4; one sequence is bound by its chain: 1 x 32768, 128,
+// three rows 21.1 / 22.0.  The ranges that this adds are no more than the fixed array holds, so that nothing it took is refused.
 int default_splits(int B, int lq, int lk, int H, int rows_per_group) {
   const int two = splits_for(B, lq, lk, H, std::min(rows_per_group, 2));
   if (rows_per_group <= 2) return two;
