@@ -100,7 +100,7 @@ struct ReconJob { TpaFactor fa, fb; void* out; int L, R; float scale; };
 // The backward's delta in the same launch (blockIdx.z = 3): delta[b, h, i] = sum_d o * do, NaN products (an empty row's o)
 // skipped; a thread takes the same piece of 8 heads of one row, the sum over d runs across the lanes that share them.
 struct DeltaJob { const void *o, *d_o; float* delta; int lq; };
-struct ReconJobs { ReconJob job[3]; DeltaJob delta; };  // blockIdx.z picks one: several arrays in one launch
+struct ReconJobs { ReconJob job[3]; DeltaJob delta; WindowJob windows[2]; };  // blockIdx.z picks one: several arrays in one launch
 template <typename T>
 __device__ __forceinline__ void delta_h8(const DeltaJob& j, int64_t t, int g, int cc, int cpr, int b, int H, int D) {
   constexpr int N = 16 / sizeof(T);  // elements of a 16-byte piece
@@ -190,6 +190,11 @@ __global__ __launch_bounds__(256) void recon_f32_h8_kernel(ReconJobs jobs, int H
 }
 
 __global__ __launch_bounds__(256) void recon_bf16_h8_kernel(ReconJobs jobs, int H, int D) {
+  if (blockIdx.z == 0) {  // the workgroups that start first
+    __shared__ int32_t red[3 * 256 / 64];
+    if (jobs.windows[0].mine) find_windows<256>(jobs.windows[0], blockIdx.y, blockIdx.x, gridDim.x, red, threadIdx.x);
+    if (jobs.windows[1].mine) find_windows<256>(jobs.windows[1], blockIdx.y, gridDim.x - 1 - blockIdx.x, gridDim.x, red, threadIdx.x);
+  }
   const TpaFactor fa = blockIdx.z == 0 ? jobs.job[0].fa : blockIdx.z == 1 ? jobs.job[1].fa : jobs.job[2].fa;
   const TpaFactor fb = blockIdx.z == 0 ? jobs.job[0].fb : blockIdx.z == 1 ? jobs.job[1].fb : jobs.job[2].fb;
   uint16_t* const out = static_cast<uint16_t*>(blockIdx.z == 0 ? jobs.job[0].out : blockIdx.z == 1 ? jobs.job[1].out : jobs.job[2].out);
@@ -803,12 +808,21 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
   for (const TpaFactor* f : fs) one_launch = one_launch && rows16<T>(*f);
   const int lmax = a->lq > a->lk ? a->lq : a->lk;
   const int64_t blocks = ((int64_t)lmax * cpr * (a->H / 8) + 255) / 256;
+  int32_t *qwin = nullptr, *kwin = nullptr;
   if (one_launch && blocks <= 2147483647LL) {
     ReconJobs jobs{};
     jobs.job[0] = ReconJob{a->qa, a->qb, qd, a->lq, a->rq, 1.f};
     jobs.job[1] = ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
     jobs.job[2] = ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
     jobs.delta = DeltaJob{a->o, a->d_o, delta, a->lq};
+    if (mfma && a->q_segment_ids) {
+      // into the halves of the slots of Q and K that bf16 leaves: H D / 2 words a row there, eight a block taken
+      const int block = dense_bwd_mfma_block(a->B, a->lq, a->lk, a->H, a->dk, a->causal, 1), coff = causal_offset_of(a);
+      qwin = reinterpret_cast<int32_t*>(qd + nq / 2);
+      kwin = reinterpret_cast<int32_t*>(kd + nk / 2);
+      jobs.windows[0] = WindowJob{a->q_segment_ids, a->kv_segment_ids, nullptr, a->lq, a->lk, block, 0, a->causal != 0, coff, qwin, (a->lq + block - 1) / block * 8, 8, 0, 1};
+      jobs.windows[1] = WindowJob{a->kv_segment_ids, a->q_segment_ids, nullptr, a->lk, a->lq, block, 1, a->causal != 0, coff, kwin, (a->lk + block - 1) / block * 8, 8, 0, 1};
+    }
     if constexpr (sizeof(T) == 2) hipLaunchKernelGGL(recon_bf16_h8_kernel, dim3((unsigned)blocks, a->B, 4), dim3(256), 0, stream, jobs, a->H, a->dk);
     else hipLaunchKernelGGL(recon_f32_h8_kernel, dim3((unsigned)blocks, a->B, 4), dim3(256), 0, stream, jobs, a->H, a->dk);
   } else {
@@ -837,7 +851,7 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
   int rc;
   if (mfma) {
     rc = dense_bwd_mfma_launch(qd, kd, vd, a->d_o, a->lse, delta, a->q_segment_ids, a->kv_segment_ids, dqd, dkd, dvd,
-                               a->B, a->lq, a->lk, a->H, a->dk, a->sm_scale, a->causal, causal_offset_of(a), stream);
+                               a->B, a->lq, a->lk, a->H, a->dk, a->sm_scale, a->causal, causal_offset_of(a), qwin, kwin, stream);
   } else if (mfma32) {
     rc = dense_bwd_f32_launch(qd, kd, vd, static_cast<const float*>(a->d_o), a->lse, delta, a->q_segment_ids, a->kv_segment_ids,
                               dqd, dkd, dvd, a->B, a->lq, a->lk, a->H, a->dk, a->sm_scale, a->causal, causal_offset_of(a), stream);
@@ -883,7 +897,7 @@ int mha_bwd_t(const MhaBwdArgs* a, hipStream_t stream, bool mfma) {
                                 a->B, a->lq, a->lk, a->H, a->dk, a->sm_scale, a->causal, 0, stream);
   if (mfma)
     return dense_bwd_mfma_launch(a->q, a->k, a->v, a->d_o, a->lse, delta, nullptr, nullptr, a->dq, a->dk_out, a->dv_out,
-                                 a->B, a->lq, a->lk, a->H, a->dk, a->sm_scale, a->causal, 0, stream);
+                                 a->B, a->lq, a->lk, a->H, a->dk, a->sm_scale, a->causal, 0, nullptr, nullptr, stream);
   const float *qd, *kd, *vd;
   if constexpr (sizeof(T) == sizeof(float)) {
     qd = static_cast<const float*>(a->q); kd = static_cast<const float*>(a->k); vd = static_cast<const float*>(a->v);
@@ -930,7 +944,7 @@ int tpa_recon_dense_bf16(const TpaFactor* fa, const TpaFactor* fb, uint16_t* out
 
 // Q (with its scale), K and V in one launch where every factor is 16-byte aligned and H % 8 == 0;
 // TPA_ERR_UNSUPPORTED otherwise (the caller then reconstructs them one by one).
-int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, hipStream_t stream) {
+int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, const tpa::WindowJob& windows, hipStream_t stream) {
   if (a->B > 65535 || a->H % 8 != 0 || a->dk % 8 != 0 || a->dk != a->dv) return TPA_ERR_UNSUPPORTED;
   const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
   for (const TpaFactor* f : fs)
@@ -942,6 +956,7 @@ int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, ui
   jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale};
   jobs.job[1] = tpa::ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
   jobs.job[2] = tpa::ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
+  jobs.windows[0] = windows;
   hipLaunchKernelGGL(tpa::recon_bf16_h8_kernel, dim3((unsigned)blocks, a->B, 3), dim3(256), 0, stream, jobs, a->H, a->dk);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }

@@ -50,6 +50,7 @@ struct BwdParams {
   int nblk;    // row blocks (dq) or key blocks (dkv) per (batch, head)
   int npairs;  // nblk * B
   int pair_groups;  // groups of (batch, head) pairs of an XCD whose blocks run side by side
+  const int32_t *qwin, *kwin;  // the windows of ids of the blocks of rows and of keys (WindowJob, eight words each), or null
 };
 
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -175,7 +176,11 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int id) {
   int kpos0 = 0, kend = p.causal ? max(1, min(p.lk, min(q0 + kBQ, p.lq) + p.coff)) : p.lk;  // at least one (then fully masked) tile
   if constexpr (SEG) {
     int first, lastk;
-    id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kBQ, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend,
+    if (p.qwin) {
+      const IdWindow* const win = reinterpret_cast<const IdWindow*>(p.qwin + ((int64_t)b * p.nblk + qblk) * 8);
+      first = scalar(win->first);
+      lastk = scalar(win->last);
+    } else id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kBQ, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend,
                   reinterpret_cast<int32_t*>(smem), tid, first, lastk);
     if (lastk >= 0) { kpos0 = first / kTile * kTile; kend = lastk + 1; }
     else kend = min(kend, kTile);  // nothing visible: one fully masked tile
@@ -376,7 +381,11 @@ __device__ __forceinline__ void dkv_block(const BwdParams& p, int id) {
   if constexpr (SEG) {
     int first, lastq;
     const int rbeg = min(tile0 * kTile, p.lq);
-    id_window<NT>(p.kvseg + (int64_t)b * p.lk + k0, min(kBK, p.lk - k0), p.qseg + (int64_t)b * p.lq + rbeg, p.lq - rbeg,
+    if (p.kwin) {
+      const IdWindow* const win = reinterpret_cast<const IdWindow*>(p.kwin + ((int64_t)b * p.nblk + kblk) * 8);
+      first = scalar(win->first);
+      lastq = scalar(win->last);
+    } else id_window<NT>(p.kvseg + (int64_t)b * p.lk + k0, min(kBK, p.lk - k0), p.qseg + (int64_t)b * p.lq + rbeg, p.lq - rbeg,
                   reinterpret_cast<int32_t*>(smem), tid, first, lastq);
     if (lastq >= 0) { tile0 = (rbeg + first) / kTile; lq_r = rbeg + lastq + 1; }
     else lq_r = 0;  // no row can see a key of this block
@@ -669,10 +678,19 @@ int dense_bwd_mfma_supported(int dtype, int dk, int dv, int64_t lq, int64_t lk, 
   return 1;
 }
 
+int dense_bwd_mfma_block(int B, int lq, int lk, int H, int D, int causal, int segments) {
+  tpa::BwdParams p{};
+  static const int32_t some = 0;
+  p.B = B; p.lq = lq; p.lk = lk; p.H = H; p.causal = causal;
+  p.qseg = segments ? &some : nullptr;
+  return D == 64 && tpa::bwd_wants_four_waves(p) ? 128 : 256;
+}
+
 int dense_bwd_mfma_launch(const void* q, const void* k, const void* v, const void* d_o, const float* lse, const float* delta,
                           const int32_t* qseg, const int32_t* kvseg, float* dq, float* dk, float* dv, int B, int lq, int lk,
-                          int H, int D, float sm_scale, int causal, int coff, hipStream_t stream) {
+                          int H, int D, float sm_scale, int causal, int coff, const int32_t* qwin, const int32_t* kwin, hipStream_t stream) {
   tpa::BwdParams p{};
+  p.qwin = qwin; p.kwin = kwin;
   p.q = static_cast<const uint16_t*>(q); p.k = static_cast<const uint16_t*>(k); p.v = static_cast<const uint16_t*>(v);
   p.d_o = static_cast<const uint16_t*>(d_o); p.lse = lse; p.delta = delta; p.qseg = qseg; p.kvseg = kvseg;
   p.dq = dq; p.dk = dk; p.dv = dv; p.B = B; p.lq = lq; p.lk = lk; p.H = H; p.sm_scale = sm_scale; p.causal = causal; p.coff = causal ? coff : 0;

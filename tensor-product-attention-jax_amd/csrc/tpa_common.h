@@ -173,6 +173,49 @@ __device__ __forceinline__ void id_window(const int32_t* mine, int n_mine, const
   id_window<NT>(mine, n_mine, other, n_other, red, tid, first, last, cnt, smin, smax);
 }
 
+// The windows of all blocks of `block` rows (keys) of a call, found by the launch that reconstructs the dense arrays: once per batch
+// entry and block where the attention kernels found them once per head too, each on its way to its first tile.  us, found by the
+// attention kernels / here: training step of 3 x 1777 tokens, 16 heads of 64, documents of 421 115.5 / 110.3; 2 x 13 505 of 284 527 /
+// 492; 14 x 569 of 129, rank 8 157.5 / 153.3; 1 x 20 000, 32 heads of 128, of 1000 1806 / 1743; forward alone 2 x 13 505 124 / 113, 14 x 569
+// 42.2 / 38.8, 5 x 9865, 16 heads of 128, of 477 472 / 458.
+struct IdWindow { int32_t first, last, count, least, most; };  // what id_window finds
+struct WindowJob {
+  const int32_t *mine, *other;  // ids [B, n_mine], [B, n_other]; mine = null: no such job
+  const int32_t* other_len;     // [B] elements of `other`, or null (= n_other)
+  int n_mine, n_other, block;
+  int keys;                     // 0: blocks of rows that look for keys, 1: the other way round
+  int causal, coff;             // as the attention kernels have them
+  int32_t* out;                 // an IdWindow per batch entry, block and copy; strides in int32
+  int64_t stride_b, stride_block, stride_copy;
+  int copies;
+};
+// The elements of `other` that the mask leaves a block: [begin, begin + n)
+__device__ __forceinline__ void window_range(const WindowJob& j, int b, int x0, int& begin, int& n) {
+  begin = 0;
+  const int len = j.other_len ? max(0, min(j.other_len[b], j.n_other)) : j.n_other;
+  if (!j.causal) { n = len; return; }
+  if (j.keys) {  // rows from the tile of 64 on that holds the first one
+    begin = min(max(x0 - j.coff, 0) / 64 * 64, len);
+    n = len - begin;
+  } else {
+    const int coff = j.coff + (j.causal == TPA_CAUSAL_BOTTOM_RIGHT ? len - j.n_mine : 0);
+    n = max(0, min(len, min(x0 + j.block, j.n_mine) + coff));
+  }
+}
+// workgroup `at` of `of` workgroups of NT threads that share out the blocks of batch entry b; red: 3 ints of LDS per wave
+template <int NT>
+__device__ __forceinline__ void find_windows(const WindowJob& j, int b, int at, int of, int32_t* red, int tid) {
+  for (int blk = at; blk < (j.n_mine + j.block - 1) / j.block; blk += of) {
+    const int x0 = blk * j.block;
+    int begin, n;
+    window_range(j, b, x0, begin, n);
+    IdWindow w;
+    id_window<NT>(j.mine + (int64_t)b * j.n_mine + x0, min(j.block, j.n_mine - x0), j.other + (int64_t)b * j.n_other + begin, n, red, tid,
+                  w.first, w.last, w.count, w.least, w.most);
+    for (int c = tid; c < j.copies; c += NT) *reinterpret_cast<IdWindow*>(j.out + b * j.stride_b + blk * j.stride_block + c * j.stride_copy) = w;
+  }
+}
+
 // Segment ids inside the window.  A workgroup visits every tile that one of its rows needs, a wave owns 32 of them and often a
 // single document, so a wave looks at each tile's 64 ids itself: a tile without an id in the range of its own rows is left out, and
 // one that holds nothing but the one id of all of them needs no mask.  Both are exact for any order of the ids.
@@ -316,7 +359,9 @@ int mha_bwd_launch(const MhaBwdArgs* a, hipStream_t stream, int mfma);
 int dense_bwd_mfma_supported(int dtype, int dk, int dv, int64_t lq, int64_t lk, int64_t H, float sm_scale, const void* bias);
 int dense_bwd_mfma_launch(const void* q, const void* k, const void* v, const void* d_o, const float* lse, const float* delta,
                           const int32_t* qseg, const int32_t* kvseg, float* dq, float* dk, float* dv, int B, int lq, int lk,
-                          int H, int D, float sm_scale, int causal, int causal_offset, hipStream_t stream);
+                          int H, int D, float sm_scale, int causal, int causal_offset, const int32_t* qwin, const int32_t* kwin, hipStream_t stream);
+// rows (keys) per workgroup of that launch
+int dense_bwd_mfma_block(int B, int lq, int lk, int H, int D, int causal, int segments);
 int dense_bwd_f32_supported(int dtype, int dk, int dv, int64_t lq, int64_t lk, const void* bias);
 int dense_bwd_f32_launch(const float* q, const float* k, const float* v, const float* d_o, const float* lse, const float* delta,
                          const int32_t* qseg, const int32_t* kvseg, float* dq, float* dk, float* dv, int B, int lq, int lk,
@@ -330,4 +375,5 @@ size_t tpa_prefill_call_bytes(const TpaFwdArgs* a);
 // dense bf16 X[B, L, H, D] = (scale/R) sum_r a_r (x) b_r from bf16 factors
 int tpa_recon_dense_bf16(const TpaFactor* fa, const TpaFactor* fb, uint16_t* out, int B, int L, int H, int D, int R, float scale, hipStream_t stream);
 // dense Q (times q_scale), K, V of a forward call in one launch; TPA_ERR_UNSUPPORTED where the vectorised kernel does not apply
-int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, hipStream_t stream);
+// (and the windows of packed documents, see WindowJob)
+int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, const tpa::WindowJob& windows, hipStream_t stream);

@@ -62,6 +62,9 @@ struct PrefillParams {
   int S;
   float* part_o;
   float2* part_ml;  // [S][B, lq, H]
+  // dense loader with segment ids: 1 = the id window of a workgroup is an IdWindow in its first row of the output (written by the launch
+  // that reconstructed Q, K, V, read before any of this workgroup's own results are written; no other workgroup writes that row of this head)
+  int windows;
 };
 
 // LDS: three buffers of a K tile (tile j is read while tile j+1 is already there for waves that run
@@ -310,7 +313,10 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
     // contiguous run, the tiles inside the run need no segment mask at all.
     int lo, hi, cnt;
     int32_t qmin, qmax;
-    id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kRows, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem), tid, lo, hi, cnt, qmin, qmax);
+    if (LOADER == LOAD_DENSE && pp.windows) {
+      const IdWindow* const win = reinterpret_cast<const IdWindow*>(p.o + (((int64_t)b * p.lq + q0) * p.H + h) * D);
+      lo = scalar(win->first); hi = scalar(win->last); cnt = scalar(win->count); qmin = scalar(win->least); qmax = scalar(win->most);
+    } else id_window<NT>(p.qseg + (int64_t)b * p.lq + q0, min(kRows, p.lq - q0), p.kvseg + (int64_t)b * p.lk, kend, reinterpret_cast<int32_t*>(smem), tid, lo, hi, cnt, qmin, qmax);
     if (hi >= 0) {
       kpos0 = lo / kTK * kTK;
       kend = hi + 1;
@@ -1366,7 +1372,14 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
     uint16_t* kd = static_cast<uint16_t*>(a->workspace);
     uint16_t* vd = kd + kv_slot / 2;
     uint16_t* qd = vd + kv_slot / 2;
-    int rc = tpa_recon_dense_qkv_bf16(a, qd, kd, vd, a->sm_scale * kLog2e, stream);
+    WindowJob windows{};
+    if (p.kvseg) {
+      const int rows = a->dk == 64 && wants_four_waves(p, true) ? kBQ / 2 : kBQ;  // as launch_prefill has it
+      windows = WindowJob{p.qseg, p.kvseg, p.kvlen, a->lq, a->lk, rows, 0, a->causal, p.coff, reinterpret_cast<int32_t*>(p.o),
+                          a->lq * hd / 2, rows * hd / 2, a->dk / 2, a->H};
+    }
+    int rc = tpa_recon_dense_qkv_bf16(a, qd, kd, vd, a->sm_scale * kLog2e, windows, stream);
+    p.windows = p.kvseg && rc == TPA_OK;
     if (rc == TPA_ERR_UNSUPPORTED) {
       rc = tpa_recon_dense_bf16(&a->ka, &a->kb, kd, a->B, a->lk, a->H, a->dk, a->rk, 1.f, stream);
       if (rc == TPA_OK) rc = tpa_recon_dense_bf16(&a->va, &a->vb, vd, a->B, a->lk, a->H, a->dv, a->rk, 1.f, stream);
