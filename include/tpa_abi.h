@@ -369,6 +369,11 @@ int tpa_decode_noalloc(const TpaFwdArgs* args, void* stream);
 /* Bytes of workspace tpa_decode needs for this problem (num_splits = 0: the default choice). */
 size_t tpa_decode_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dv, int32_t num_splits);
 
+/* Bytes of workspace with which tpa_decode has every key range that it has a use for in this very call: its sizes, rank, element type
+   and num_splits.  At least tpa_decode_workspace_bytes(...), which is what it needs; 0 if the sizes are not positive.
+   `workspace` and `workspace_bytes` of the arguments are not looked at. */
+size_t tpa_decode_call_workspace_bytes(const TpaFwdArgs* args);
+
 /* Number of key ranges per batch entry that tpa_decode_workspace_bytes sizes the workspace for when
    num_splits == 0.  An upper bound on what the kernels use: with kv_lengths (B <= 64) up to B times as many
    ranges are dealt to the entries by their lengths; otherwise every entry gets as many as fill the chip once. */

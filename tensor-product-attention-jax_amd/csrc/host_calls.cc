@@ -31,7 +31,7 @@ using at::Tensor;
 // ------------------------------------------------------------------------------------------------ the C ABI, by name
 #define TPA_CALLS(X)                                                                                             \
   X(tpa_fwd) X(tpa_decode) X(tpa_cache_append) X(tpa_bwd) X(tpa_strerror) X(tpa_fwd_call_workspace_bytes) \
-  X(tpa_decode_workspace_bytes) X(tpa_cache_append_workspace_bytes) X(tpa_bwd_workspace_bytes)
+  X(tpa_decode_call_workspace_bytes) X(tpa_cache_append_workspace_bytes) X(tpa_bwd_workspace_bytes)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
   TPA_CALLS(X)
@@ -326,7 +326,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Tensor kvlen = lengths(tensor_or_none(args[6]), a.B);
     a.kv_lengths = ids_ptr(kvlen);
     const auto options = at::TensorOptions().device(device);
-    if (!ws.defined()) ws = bytes_on(device, std::max<size_t>(lib.tpa_decode_workspace_bytes(a.B, a.lq, a.lk, a.H, a.dv, a.num_splits), 16));
+    if (!ws.defined()) ws = bytes_on(device, std::max<size_t>(lib.tpa_decode_call_workspace_bytes(&a), 16));
     r.first = at::empty({a.B, a.lq, a.H, a.dv}, options.dtype(t[0].scalar_type()));
     r.second = at::empty({a.B, a.H, a.lq}, options.dtype(at::kFloat));
     a.workspace = ws.data_ptr();

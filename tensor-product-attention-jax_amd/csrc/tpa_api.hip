@@ -157,7 +157,12 @@ size_t tpa_fwd_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int
 size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk) {
   const size_t base = tpa_fwd_workspace_bytes(B, lq, lk, H, dk, dv, rq, rk);
   if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0 || rk <= 0 || dk != dv || (dk != 64 && dk != 128)) return base;
-  const size_t best = tpa_prefill_best_bytes(B, lq, lk, H, dk, rk);
+  size_t best = tpa_prefill_best_bytes(B, lq, lk, H, dk, rk);
+  if (lq <= 16 && lk >= 1024)
+    for (int dtype : {TPA_DTYPE_BF16, TPA_DTYPE_F32}) {
+      const size_t decode = tpa_decode_rank_bytes(B, lq, lk, H, dv, rk, dtype);
+      if (decode > best) best = decode;
+    }
   return best > base ? best : base;
 }
 
@@ -168,7 +173,7 @@ size_t tpa_fwd_call_workspace_bytes(const TpaFwdArgs* a) {
     return tpa_decode_mfma_supported(&w) || tpa_decode_f32_supported(&w) ? nomat_bytes(a, w) : 0;
   }
   if (is_decode(a) && (tpa_decode_mfma_supported(a) || tpa_decode_f32_supported(a)))
-    return tpa_decode_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->num_splits);
+    return tpa_decode_call_workspace_bytes(a);
   return tpa_prefill_mfma_supported(a) ? tpa_prefill_call_bytes(a) : 0;
 }
 

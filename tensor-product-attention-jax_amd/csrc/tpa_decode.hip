@@ -32,6 +32,13 @@ constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
 enum class Reads { kOrdinary, kStreaming, kFar };
 constexpr int64_t kFarthestRow = 1 << 25;  // elements between neighbouring rows, at most, for the first two
 constexpr int kMinKeys = kWaves * kRowsPerBlock / 2;  // keys of a range with one block of rank 2 per wave
+// The same of the call's rank, from rank 4 on.  Not at rank 4 of bf16 rows of 64 with one set of columns per workgroup: two of these blocks
+// cost no more than the partials of twice the ranges (us, one block / two: 1 x 700, 64 heads 10.5 / 10.2, 16 x 1500, 8 heads, two rows 11.7 /
+// 11.4, but with two sets 10.7 / 11.4).
+inline int least_keys(int dtype, int lq, int H, int D, int rk) {
+  if (rk <= 2 || (dtype == TPA_DTYPE_BF16 && D == 64 && rk == 4 && (lq == 1 || H == 8 || H == 16))) return kMinKeys;
+  return kWaves * kRowsPerBlock / rk;
+}
 
 
 struct DecodeParams {
@@ -51,6 +58,7 @@ struct DecodeParams {
   int S;           // key ranges per batch entry (slots == 0)
   int slots;       // > 0: the ranges are dealt by the batch entries' lengths, this many at most (plan_ranges)
   float round_keys;  // slots > 0: ranges are this many keys long, or a multiple (a block for each wave); 0: any length
+  float min_keys;    // slots > 0: and no shorter than this
   float qscale;    // sm_scale * log2(e) / (rq * rk)
 };
 
@@ -81,12 +89,12 @@ __device__ __forceinline__ int wave_prefix_sum(int x) {  // lane i: sum of lanes
   return add_from<0x143, 0xc>(x);  // row_bcast 31: lane 31 to rows 2 and 3
 }
 struct RangePlan { int S, first; };  // of batch entry `lane`: its number of ranges and the first one's index
-__device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, float round_keys) {
+__device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, int lk, int slots, float round_keys, float min_keys) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
   const int total = __builtin_amdgcn_readlane(wave_prefix_sum(len), 63);
-  const float shortest = fmaxf((float)total / (float)slots, (float)kMinKeys);
+  const float shortest = fmaxf((float)total / (float)slots, min_keys);
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
   float length = fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
   if (round_keys > 0.f) length = ceilf(length / round_keys) * round_keys;
@@ -119,7 +127,7 @@ __device__ __forceinline__ bool range_of(const DecodeParams& p, int x, int& b, i
     split = x - b * S;
     return x < p.B * S;
   }
-  const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.round_keys);
+  const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.round_keys, p.min_keys);
   const int lane = threadIdx.x & 63;
   b = __popcll(__ballot(lane < p.B && plan.first <= x)) - 1;
   S = __builtin_amdgcn_readlane(plan.S, b);
@@ -917,7 +925,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, TO* o
   const int b = blockIdx.x / p.lq, qi = blockIdx.x % p.lq;
   int S = p.S, first = b * S;  // the batch entry's ranges
   if (p.slots > 0) {
-    const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.round_keys);
+    const RangePlan plan = plan_ranges(p.kvlen, p.B, p.lk, p.slots, p.round_keys, p.min_keys);
     S = __builtin_amdgcn_readlane(plan.S, b);
     first = __builtin_amdgcn_readlane(plan.first, b);
   }
@@ -998,6 +1006,7 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq;
   p.S = ranges.S; p.slots = ranges.slots;
   p.round_keys = a->dv == 128 ? kWaves * kRowsPerBlock / (float)RK : 0.f;
+  p.min_keys = (float)least_keys(a->dtype, a->lq, a->H, a->dv, RK);
   p.kvlen = a->kv_lengths;
   p.climit = a->causal ? causal_offset_of(a) + 1 + rows.row0 : a->lk;
   p.cbr = a->causal == TPA_CAUSAL_BOTTOM_RIGHT;
@@ -1139,18 +1148,39 @@ int default_splits(int B, int lq, int lk, int H, int rows_per_group) {
 }
 int rows_per_workgroup(int H) { return H == 8 ? 4 : 2; }
 
-// How a launch splits the keys if the caller leaves it to us, with partials for B * default_splits ranges at hand.
+// From rank 4 on a block holds fewer keys than those counts, which go by the sizes alone, have in mind: with them a wave of a short cache
+// has RK / 2 blocks to walk, one after the other, while compute units are idle.  So with the room for their partials there are as many
+// ranges as leave one block per wave, within the fixed array's size.  us, by the sizes alone / so: rank 8, head size 128, 1 x 700 keys, 16
+// heads 15.2 / 10.8, 32 heads 16.2 / 11.6, 3 x 920 16.1 / 11.6, 2 x 3000 17.3 / 15.1, 32 heads, four rows 23.2 / 21.8; rank 4, 1 x 700 12.5 /
+// 10.5, 2 x 3000, 32 heads 14.6 / 13.0; fp32, 2 x 2000, 8 heads of 64, rank 8 32.0 / 21.9, 3 x 900, 32 heads of 128 56.3 / 36.8.  (Rank 2, 1 x 670,
+// 32 heads, two rows: 13.4, with twice the ranges 13.8.)
+int splits_by_rank(int B, int lq, int lk, int H, int D, int rk, int dtype, int rows_per_group) {
+  const int by_size = default_splits(B, lq, lk, H, rows_per_group);
+  const int64_t groups = (int64_t)B * ((lq + rows_per_group - 1) / rows_per_group) * ((H + 31) / 32);
+  const int keys = rk <= kRowsPerBlock && (rk & (rk - 1)) == 0 ? least_keys(dtype, lq, H, D, rk) : kMinKeys;  // of a rank that the kernels take
+  if (keys >= kMinKeys || groups >= 256) return by_size;
+  const int want = (int)((256 + groups - 1) / groups);
+  return std::max(by_size, std::min({want, (lk + keys - 1) / keys, noalloc_room(B, lq, H)}));
+}
+// and within the room that the call brings
+int splits_of_call(const TpaFwdArgs* a, int rows_per_group) {
+  const size_t room = a->workspace_bytes / workspace_bytes(a->B, a->lq, a->H, a->dv, 1);
+  return std::max(default_splits(a->B, a->lq, a->lk, a->H, rows_per_group),
+                  (int)std::min<size_t>(room, splits_by_rank(a->B, a->lq, a->lk, a->H, a->dv, a->rk, a->dtype, rows_per_group)));
+}
+
+// How a launch splits the keys if the caller leaves it to us, with partials for B * splits_of_call ranges at hand.
 // With lengths per batch entry the ranges are dealt by them; otherwise all entries get one count, which fills the chip
 // at most once: 288 workgroups take two rounds, the second nearly empty (48 x 4096 keys, 32 heads of 128: 6 ranges each 69.5 us, 5 48.6).
 // What some wave has to do is a whole number of blocks, so there are no more ranges than that number needs: the others would only
 // be partials to merge (1 x 20 000 keys, 16 heads of 128: 63 ranges of up to ten blocks per wave 34.3 us, fewer 26.3; 3 x 9000, 32 heads
 // 22.1 / 19.7).
 KeyRanges choose_ranges(const TpaFwdArgs* a, int rows_per_group) {
-  const int S = default_splits(a->B, a->lq, a->lk, a->H, rows_per_group);
+  const int S = splits_of_call(a, rows_per_group);
   const int per_range = (a->lq + rows_per_group - 1) / rows_per_group * ((a->H + 31) / 32);  // workgroups of one range
   if (a->kv_lengths && a->B <= kMaxPlanEntries)
     return KeyRanges{S, std::min(std::max(a->B, 256 / per_range), a->B * S)};
-  const int most = (a->lk + kMinKeys - 1) / kMinKeys;
+  const int keys = least_keys(a->dtype, a->lq, a->H, a->dv, a->rk), most = (a->lk + keys - 1) / keys;
   const int n = std::max(1, (int)std::min<int64_t>(std::min(S, most), 256 / ((int64_t)a->B * per_range)));
   const int64_t blocks = ((int64_t)a->lk * a->rk + kRowsPerBlock - 1) / kRowsPerBlock, rounds = (blocks + kWaves * n - 1) / (kWaves * n);
   return KeyRanges{(int)((blocks + kWaves * rounds - 1) / (kWaves * rounds)), 0};
@@ -1168,6 +1198,16 @@ extern "C" size_t tpa_decode_workspace_bytes(int32_t B, int32_t lq, int32_t lk, 
   if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0 || dv <= 0) return 0;
   const int S = num_splits > 0 ? num_splits : tpa::default_splits(B, lq, lk, H, tpa::rows_per_workgroup(H));
   return tpa::workspace_bytes(B, lq, H, dv, S);
+}
+
+size_t tpa_decode_rank_bytes(int B, int lq, int lk, int H, int dv, int rk, int dtype) {
+  return tpa::workspace_bytes(B, lq, H, dv, tpa::splits_by_rank(B, lq, lk, H, dv, rk, dtype, dtype == TPA_DTYPE_BF16 ? tpa::rows_per_workgroup(H) : 1));
+}
+
+extern "C" size_t tpa_decode_call_workspace_bytes(const TpaFwdArgs* a) {
+  if (!a || a->B <= 0 || a->lq <= 0 || a->lk <= 0 || a->H <= 0 || a->dv <= 0 || a->rk <= 0) return 0;
+  const size_t base = tpa_decode_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->num_splits);
+  return a->num_splits > 0 ? base : std::max(base, tpa_decode_rank_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->rk, a->dtype));
 }
 
 int tpa_decode_mfma_supported(const TpaFwdArgs* a) {

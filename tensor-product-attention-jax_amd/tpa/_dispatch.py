@@ -251,6 +251,8 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
         lib.tpa_fwd_workspace_bytes.argtypes = [ctypes.c_int32] * 8
         lib.tpa_fwd_best_workspace_bytes.restype = ctypes.c_size_t
         lib.tpa_fwd_best_workspace_bytes.argtypes = [ctypes.c_int32] * 8
+        lib.tpa_decode_call_workspace_bytes.restype = ctypes.c_size_t
+        lib.tpa_decode_call_workspace_bytes.argtypes = [ctypes.POINTER(TpaFwdArgs)]
         lib.tpa_fwd_call_workspace_bytes.restype = ctypes.c_size_t
         lib.tpa_fwd_call_workspace_bytes.argtypes = [ctypes.POINTER(TpaFwdArgs)]
         lib.tpa_fwd_nomat_workspace_bytes.restype = ctypes.c_size_t
