@@ -158,6 +158,7 @@ size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H
   const size_t base = tpa_fwd_workspace_bytes(B, lq, lk, H, dk, dv, rq, rk);
   if (B <= 0 || lq <= 0 || lk <= 0 || H <= 0 || rk <= 0 || dk != dv || (dk != 64 && dk != 128)) return base;
   size_t best = tpa_prefill_best_bytes(B, lq, lk, H, dk, rk);
+  if (const size_t f32 = tpa_prefill_f32_dense_bytes(B, lq, lk, H, dk, rk); f32 > best) best = f32;
   if (lq <= 16 && lk >= 1024)
     for (int dtype : {TPA_DTYPE_BF16, TPA_DTYPE_F32}) {
       const size_t decode = tpa_decode_rank_bytes(B, lq, lk, H, dv, rk, dtype);
@@ -174,7 +175,7 @@ size_t tpa_fwd_call_workspace_bytes(const TpaFwdArgs* a) {
   }
   if (is_decode(a) && (tpa_decode_mfma_supported(a) || tpa_decode_f32_supported(a)))
     return tpa_decode_call_workspace_bytes(a);
-  return tpa_prefill_mfma_supported(a) ? tpa_prefill_call_bytes(a) : 0;
+  return tpa_prefill_mfma_supported(a) ? tpa_prefill_call_bytes(a) : tpa_prefill_f32_supported(a) ? tpa_prefill_f32_call_bytes(a) : 0;
 }
 
 int tpa_decode(const TpaFwdArgs* a, void* stream) {

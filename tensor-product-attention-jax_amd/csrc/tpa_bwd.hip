@@ -961,6 +961,21 @@ int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, ui
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
+int tpa_recon_dense_qkv_f32(const TpaFwdArgs* a, float* qd, float* kd, float* vd, float q_scale, hipStream_t stream) {
+  const int cpr = a->dk / 4, lmax = a->lq > a->lk ? a->lq : a->lk;
+  const int64_t blocks = ((int64_t)lmax * cpr * (a->H / 8) + 255) / 256;
+  if (a->B > 65535 || a->H % 8 != 0 || a->dk != a->dv || (cpr != 16 && cpr != 32) || blocks > 2147483647LL) return TPA_ERR_UNSUPPORTED;
+  const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
+  for (const TpaFactor* f : fs)
+    if (!tpa::rows16<float>(*f)) return TPA_ERR_UNSUPPORTED;
+  tpa::ReconJobs jobs{};
+  jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale};
+  jobs.job[1] = tpa::ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
+  jobs.job[2] = tpa::ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
+  hipLaunchKernelGGL(tpa::recon_f32_h8_kernel, dim3((unsigned)blocks, a->B, 3), dim3(256), 0, stream, jobs, a->H, a->dk);
+  return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
+}
+
 size_t tpa_bwd_workspace_size(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t dk, int64_t dv) {
   using tpa::align256;
   const size_t nq = (size_t)(B * lq * H * dk), nk = (size_t)(B * lk * H * dk), nv = (size_t)(B * lk * H * dv), nd = (size_t)(B * H * lq);

@@ -340,6 +340,11 @@ int mha_prefill_mfma_supported(const MhaFwdArgs* a);
 int mha_prefill_mfma_launch(const MhaFwdArgs* a, hipStream_t stream);
 int tpa_prefill_f32_supported(const TpaFwdArgs* a);
 int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream);
+// bytes of workspace with which that runs on dense fp32 Q, K and V (0: it would not)
+size_t tpa_prefill_f32_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk);
+size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a);
+// dense fp32 Q (times q_scale), K, V of a forward call in one launch; TPA_ERR_UNSUPPORTED where the vectorised kernel does not apply
+int tpa_recon_dense_qkv_f32(const TpaFwdArgs* a, float* qd, float* kd, float* vd, float q_scale, hipStream_t stream);
 int mha_prefill_f32_supported(const MhaFwdArgs* a);
 int mha_prefill_f32_launch(const MhaFwdArgs* a, hipStream_t stream);
 int tpa_nomat_pairs_supported(const TpaFwdArgs* a);

@@ -34,7 +34,7 @@ struct F32Params {
   float* o;
   float* lse;
   int B, lq, lk, H, rq, rk;
-  float sm_scale;
+  float q_scale;  // of the sum over Q's ranks: sm_scale log2(e) / rq, or 1 for a dense Q that has it already
   int causal, coff, nqb, npairs, groups;  // coff: with causal, row i sees keys <= i + coff; groups: see pair_of_workgroup
 };
 
@@ -60,9 +60,9 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
 
   struct Fac { const float* ptr; int64_t stride_b, stride_l, stride_r; };
   auto fac = [](const TpaFactor& f) { return Fac{static_cast<const float*>(f.ptr), f.stride_b, f.stride_l, f.stride_r}; };
-  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; float* o; float* lse; int B, lq, lk, H, rq, rk; float sm_scale; int causal, coff, nqb, npairs, groups; } const p = {
+  struct { Fac qa, qb, ka, kb, va, vb; const int32_t* qseg; const int32_t* kvseg; const int32_t* kvlen; float* o; float* lse; int B, lq, lk, H, rq, rk; float q_scale; int causal, coff, nqb, npairs, groups; } const p = {
       fac(pp.qa), fac(pp.qb), fac(pp.ka), fac(pp.kb), fac(pp.va), fac(pp.vb), pp.qseg, pp.kvseg, pp.kvlen, pp.o, pp.lse,
-      pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk, pp.sm_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.groups};
+      pp.B, pp.lq, pp.lk, pp.H, pp.rq, pp.rk, pp.q_scale, pp.causal, pp.causal ? pp.coff : 0, pp.nqb, pp.npairs, pp.groups};
 
   extern __shared__ __attribute__((aligned(16))) float smem_f32[];
   uint16_t* const planes = reinterpret_cast<uint16_t*>(smem_f32);  // [2][K h, m, l; V h, m, l]
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(F32Params pp) {
   auto load_q = [&](auto fp32) __attribute__((always_inline)) {
     const float* const qb = p.qb.ptr + b * p.qb.stride_b + (int64_t)qrow_ld * p.qb.stride_l + (dense ? (int64_t)h * D : 0) + 8 * g;
     const float* const qa = dense ? nullptr : p.qa.ptr + b * p.qa.stride_b + (int64_t)qrow_ld * p.qa.stride_l + h;
-    const float scale = p.sm_scale * kLog2e / (float)p.rq;
+    const float scale = p.q_scale;
     float top = 0.f;
     constexpr int NH = NKS < 4 ? NKS : 4;  // steps at a time
 #pragma unroll
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(SplitLdsF32<D>::NW * 64, 1) void prefill_f32_split_
         for (int u = 0; u < G; ++u)
           if (r0 + u < p.rq) acc += a[u] * bv[u];
       }
-      acc *= p.sm_scale * kLog2e / (float)p.rq;
+      acc *= p.q_scale;
       top = largest(top, acc);
       const Pair3 x = whole ? halves_of_pair(acc[0], acc[1]) : split_pair(acc[0], acc[1]), y = whole ? halves_of_pair(acc[2], acc[3]) : split_pair(acc[2], acc[3]);
       uint16_t* const at = lds_q + row * SplitLdsF32<D>::QS + 4 * cc;
@@ -854,6 +854,37 @@ int tpa_prefill_f32_supported(const TpaFwdArgs* a) {
   return 1;
 }
 
+namespace tpa {
+namespace {
+int64_t dense_slot(int64_t floats) { return (floats + 63) / 64 * 64; }
+// Whether K and V (and Q) as dense fp32 arrays, formed once by a launch of their own, beat rebuilding every tile from the factors in
+// each workgroup: the rebuild grows with the rank and the blocks of rows that repeat it, the launch with the keys alone.  us, fused / dense,
+// causal, 8 heads of 64 | 4 x 64 heads of 64 | 2 x 16 heads of 128:
+//   rank 8: 40 rows over 300 keys 27.2 / 19.9 | 58.5 / 49.1 | 67.7 / 42.2; 200 x 200 19.6 / 19.0 | 60.3 / 46.8 | 49.9 / 30.5; 300 x 3000 183 / 76 | 1064 /
+//     647 | 886 / 304; 700 x 700 50.0 / 28.6 | 329 / 175 | 272 / 124; but 17 x 300 27.2 / 19.5 | 31.2 / 36.4 | 66.9 / 36.4
+//   rank 4: 40 x 300 19.5 / 18.8 | 39.0 / 47.9 | 45.9 / 39.4; 200 x 200 14.9 / 18.5 | 38.5 / 47.1 | 34.3 / 29.2; 40 x 2000 80 / 53 | 151 / 161 | 215 / 120; 300 x
+//     300 19.4 / 19.0 | 87 / 76 | 47.3 / 40.9; 700 x 700 30.7 / 27.3 | 208 / 171 | 171 / 123
+//   rank 3: 300 x 300 16.9 / 19.5 | 82 / 77 | 42.9 / 40.8; 100 x 1000 33.5 / 33.3 | 133 / 140 | 101 / 71; 700 x 700 27.3 / 26.7 | 190 / 170 | 156 / 123
+//   rank 2: 700 x 700 23.7 / 26.9 | 176 / 173 | 139 / 124; 1500 x 1500 42.1 / 42.4 | 592 / 571 | 275 / 244, no mask 79 / 72 | 950 / 921 | 287 / 252; 4000 x 4000
+//     202 / 176 | - | 796 / 742; 300 x 3000 70 / 75 | 586 / 615 | 411 / 298; 4 x 32 heads of 128 700 x 700 178 / 161, 4000 x 4000 3206 / 3138
+//   rank 1: never (700 x 700 20.2 / 26.7 | 167 / 175 | 123 / 124)
+bool f32_dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
+  const int64_t pairs = B * H;
+  if (rk < 2 || lq <= 16) return false;
+  if (rk == 2) return pairs <= 128 && lq >= (D == 128 ? 700 : 1500) && lk <= 5 * lq;  // beyond, 2 % for three arrays of O's size
+  if (lq <= 32 && pairs > 64) return false;
+  if (rk >= 8 || D == 128) return true;
+  return pairs > 64 ? lq > 256 : lk * rk >= 2800;
+}
+}  // namespace
+}  // namespace tpa
+
+size_t tpa_prefill_f32_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
+  if (H % 8 != 0 || !tpa::f32_dense_pays(B, lq, lk, H, D, rk)) return 0;
+  return (size_t)(tpa::dense_slot(B * lq * H * D) + 2 * tpa::dense_slot(B * lk * H * D)) * 4;
+}
+size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a) { return tpa_prefill_f32_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->rk); }
+
 int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
   using namespace tpa;
   F32Params p{};
@@ -861,7 +892,24 @@ int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
   p.qseg = a->q_segment_ids; p.kvseg = a->kv_segment_ids; p.kvlen = a->kv_lengths;
   p.o = static_cast<float*>(a->o); p.lse = a->lse;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq; p.rk = a->rk;
-  p.sm_scale = a->sm_scale; p.causal = a->causal; p.coff = causal_offset_of(a);
+  p.q_scale = a->sm_scale * kLog2e / (float)a->rq; p.causal = a->causal; p.coff = causal_offset_of(a);
+  if (const size_t need = tpa_prefill_f32_call_bytes(a); need && a->workspace && !(reinterpret_cast<uintptr_t>(a->workspace) & 255) && a->workspace_bytes >= need) {
+    const int64_t hd = (int64_t)a->H * a->dk;
+    float* const kd = static_cast<float*>(a->workspace);
+    float* const vd = kd + dense_slot(a->B * a->lk * hd);
+    float* const qd = vd + dense_slot(a->B * a->lk * hd);
+    const int rc = tpa_recon_dense_qkv_f32(a, qd, kd, vd, a->sm_scale * kLog2e, stream);
+    if (rc == TPA_OK) {
+      p.qa = p.ka = p.va = TpaFactor{nullptr, 0, 0, 0};
+      p.qb = TpaFactor{qd, a->lq * hd, hd, 0};
+      p.kb = TpaFactor{kd, a->lk * hd, hd, 0};
+      p.vb = TpaFactor{vd, a->lk * hd, hd, 0};
+      p.rq = p.rk = 1;
+      p.q_scale = 1.f;
+    } else if (rc != TPA_ERR_UNSUPPORTED) {
+      return rc;
+    }
+  }
   return launch_any(p, a->dk, stream);
 }
 
@@ -883,6 +931,6 @@ int mha_prefill_f32_launch(const MhaFwdArgs* a, hipStream_t stream) {
   p.qa = p.ka = p.va = TpaFactor{nullptr, 0, 0, 0};
   p.o = static_cast<float*>(a->o); p.lse = a->lse;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = 1; p.rk = 1;
-  p.sm_scale = a->sm_scale; p.causal = a->causal ? TPA_CAUSAL_TOP_LEFT : TPA_CAUSAL_NONE;
+  p.q_scale = a->sm_scale * kLog2e; p.causal = a->causal ? TPA_CAUSAL_TOP_LEFT : TPA_CAUSAL_NONE;
   return launch_any(p, a->dk, stream);
 }
