@@ -96,7 +96,10 @@ __device__ __forceinline__ float dpp_add(float v) {
 // (token, 16-byte piece of D, group of 8 heads) and reads, per rank, one 16-byte piece of b and
 // the 8 head factors as one 16-byte piece of a - 64 multiply-adds per two loads.  Pieces are the
 // fastest thread index, so the 16 threads of a (token, head group) store whole rows of D.
-struct ReconJob { TpaFactor fa, fb; void* out; int L, R; float scale; };
+// Of the L tokens of a batch entry that lie in `out`, the first `n` are made, and where `lengths` is given no more than lengths[b]: the
+// loops over the dense tiles read no key beyond.  A chunk over caches of 8192 tokens, half to wholly full, 4 sequences of 32 heads of
+// 128, rank 4, us with all keys made / without: 128 rows 234 / 215, 512 rows 312 / 306; rank 8, 512 rows 328 / 320.
+struct ReconJob { TpaFactor fa, fb; void* out; int L, R; float scale; int n; const int32_t* lengths; };
 // The backward's delta in the same launch (blockIdx.z = 3): delta[b, h, i] = sum_d o * do, NaN products (an empty row's o)
 // skipped; a thread takes the same piece of 8 heads of one row, the sum over d runs across the lanes that share them.
 struct DeltaJob { const void *o, *d_o; float* delta; int lq; };
@@ -152,6 +155,8 @@ __device__ __forceinline__ void piece_of(int cpr, int hg, int64_t& t, int& g, in
   }
 }
 
+__device__ __forceinline__ int tokens_of(int n, const int32_t* lengths, int b) { return lengths ? min(n, lengths[b]) : n; }
+
 // fp32 factors -> dense fp32, in the same way: a thread owns 4 elements of D for 8 heads of a token
 __global__ __launch_bounds__(256) void recon_f32_h8_kernel(ReconJobs jobs, int H, int D) {
   const int cpr = D / 4, hg = H / 8;
@@ -161,7 +166,7 @@ __global__ __launch_bounds__(256) void recon_f32_h8_kernel(ReconJobs jobs, int H
   const int b = blockIdx.y;
   if (blockIdx.z == 3) return delta_h8<float>(jobs.delta, t, g, cc, cpr, b, H, D);
   const ReconJob job = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
-  if (t >= job.L) return;
+  if (t >= tokens_of(job.n, job.lengths, b)) return;
   const float* ap = static_cast<const float*>(job.fa.ptr) + b * job.fa.stride_b + t * job.fa.stride_l + 8 * g;
   const float* bp = static_cast<const float*>(job.fb.ptr) + b * job.fb.stride_b + t * job.fb.stride_l + 4 * cc;
   f32x4 acc[8];
@@ -201,13 +206,15 @@ __global__ __launch_bounds__(256) void recon_bf16_h8_kernel(ReconJobs jobs, int 
   const int L = blockIdx.z == 0 ? jobs.job[0].L : blockIdx.z == 1 ? jobs.job[1].L : jobs.job[2].L;
   const int R = blockIdx.z == 0 ? jobs.job[0].R : blockIdx.z == 1 ? jobs.job[1].R : jobs.job[2].R;
   const float scale = blockIdx.z == 0 ? jobs.job[0].scale : blockIdx.z == 1 ? jobs.job[1].scale : jobs.job[2].scale;
+  const int n = blockIdx.z == 0 ? jobs.job[0].n : blockIdx.z == 1 ? jobs.job[1].n : jobs.job[2].n;
+  const int32_t* const lengths = blockIdx.z == 0 ? jobs.job[0].lengths : blockIdx.z == 1 ? jobs.job[1].lengths : jobs.job[2].lengths;
   const int cpr = D / 8, hg = H / 8;
   int cc, g;
   int64_t t;
   piece_of(cpr, hg, t, g, cc);
   const int b = blockIdx.y;
   if (blockIdx.z == 3) return delta_h8<uint16_t>(jobs.delta, t, g, cc, cpr, b, H, D);
-  if (t >= L) return;
+  if (t >= tokens_of(n, lengths, b)) return;
   const uint16_t* ap = static_cast<const uint16_t*>(fa.ptr) + b * fa.stride_b + t * fa.stride_l + 8 * g;
   const uint16_t* bp = static_cast<const uint16_t*>(fb.ptr) + b * fb.stride_b + t * fb.stride_l + 8 * cc;
   float acc[8][8];
@@ -811,9 +818,9 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
   int32_t *qwin = nullptr, *kwin = nullptr;
   if (one_launch && blocks <= 2147483647LL) {
     ReconJobs jobs{};
-    jobs.job[0] = ReconJob{a->qa, a->qb, qd, a->lq, a->rq, 1.f};
-    jobs.job[1] = ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
-    jobs.job[2] = ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
+    jobs.job[0] = ReconJob{a->qa, a->qb, qd, a->lq, a->rq, 1.f, a->lq, nullptr};
+    jobs.job[1] = ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f, a->lk, nullptr};
+    jobs.job[2] = ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f, a->lk, nullptr};
     jobs.delta = DeltaJob{a->o, a->d_o, delta, a->lq};
     if (mfma && a->q_segment_ids) {
       // into the halves of the slots of Q and K that bf16 leaves: H D / 2 words a row there, eight a block taken
@@ -931,7 +938,7 @@ int tpa_recon_dense_bf16(const TpaFactor* fa, const TpaFactor* fb, uint16_t* out
   const int64_t threads = (int64_t)L * (D / 8) * (H / 8);
   if (vec_a && (threads + 255) / 256 <= 2147483647LL) {
     tpa::ReconJobs jobs{};
-    jobs.job[0] = tpa::ReconJob{*fa, *fb, out, L, R, scale};
+    jobs.job[0] = tpa::ReconJob{*fa, *fb, out, L, R, scale, L, nullptr};
     hipLaunchKernelGGL(tpa::recon_bf16_h8_kernel, dim3((unsigned)((threads + 255) / 256), B, 1), dim3(256), 0, stream, jobs, H, D);
   } else if (vec)
     hipLaunchKernelGGL(tpa::recon_bf16_kernel, dim3((L + tpa::kReconTokens - 1) / tpa::kReconTokens, B), dim3(256), 0, stream, *fa, *fb, out, L, H, D, R, scale);
@@ -952,10 +959,11 @@ int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, ui
   const int lmax = a->lq > a->lk ? a->lq : a->lk;
   const int64_t blocks = ((int64_t)lmax * (a->dk / 8) * (a->H / 8) + 255) / 256;
   if (blocks > 2147483647LL) return TPA_ERR_UNSUPPORTED;
+  const int keys = tpa::keys_in_reach(a);
   tpa::ReconJobs jobs{};
-  jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale};
-  jobs.job[1] = tpa::ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
-  jobs.job[2] = tpa::ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
+  jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale, a->lq, nullptr};
+  jobs.job[1] = tpa::ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f, keys, a->kv_lengths};
+  jobs.job[2] = tpa::ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f, keys, a->kv_lengths};
   jobs.windows[0] = windows;
   hipLaunchKernelGGL(tpa::recon_bf16_h8_kernel, dim3((unsigned)blocks, a->B, 3), dim3(256), 0, stream, jobs, a->H, a->dk);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
@@ -968,10 +976,11 @@ int tpa_recon_dense_qkv_f32(const TpaFwdArgs* a, float* qd, float* kd, float* vd
   const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
   for (const TpaFactor* f : fs)
     if (!tpa::rows16<float>(*f)) return TPA_ERR_UNSUPPORTED;
+  const int keys = tpa::keys_in_reach(a);
   tpa::ReconJobs jobs{};
-  jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale};
-  jobs.job[1] = tpa::ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f};
-  jobs.job[2] = tpa::ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f};
+  jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale, a->lq, nullptr};
+  jobs.job[1] = tpa::ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f, keys, a->kv_lengths};
+  jobs.job[2] = tpa::ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f, keys, a->kv_lengths};
   hipLaunchKernelGGL(tpa::recon_f32_h8_kernel, dim3((unsigned)blocks, a->B, 3), dim3(256), 0, stream, jobs, a->H, a->dk);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }

@@ -308,6 +308,12 @@ inline int causal_offset_of(const TpaFwdArgs* a) {
   if (a->causal == TPA_CAUSAL_BOTTOM_RIGHT) return clamp_causal_offset(a->causal_offset, -a->lq - a->lk, a->lq + a->lk);
   return clamp_causal_offset(a->causal_offset, -a->lq, a->lk);
 }
+// keys from here on are behind every query's mask, whatever the lengths of the batch entries
+inline int keys_in_reach(const TpaFwdArgs* a) {
+  if (a->causal != TPA_CAUSAL_TOP_LEFT) return a->lk;
+  const int end = a->lq + causal_offset_of(a);
+  return end < 0 ? 0 : end < a->lk ? end : a->lk;
+}
 // the backward takes no kv_lengths, so bottom-right alignment is the fixed offset lk - lq
 inline int causal_offset_of(const TpaBwdArgs* a) {
   if (!a->causal) return 0;
