@@ -951,11 +951,16 @@ int tpa_recon_dense_bf16(const TpaFactor* fa, const TpaFactor* fb, uint16_t* out
 
 // Q (with its scale), K and V in one launch where every factor is 16-byte aligned and H % 8 == 0;
 // TPA_ERR_UNSUPPORTED otherwise (the caller then reconstructs them one by one).
-int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, const tpa::WindowJob& windows, hipStream_t stream) {
-  if (a->B > 65535 || a->H % 8 != 0 || a->dk % 8 != 0 || a->dk != a->dv) return TPA_ERR_UNSUPPORTED;
+bool tpa_recon_dense_qkv_takes(const TpaFwdArgs* a) {
+  if (a->B > 65535 || a->H % 8 != 0 || a->dk % 8 != 0 || a->dk != a->dv) return false;
   const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
   for (const TpaFactor* f : fs)
-    if ((reinterpret_cast<uintptr_t>(f->ptr) & 15) || f->stride_b % 8 != 0 || f->stride_l % 8 != 0 || f->stride_r % 8 != 0) return TPA_ERR_UNSUPPORTED;
+    if ((reinterpret_cast<uintptr_t>(f->ptr) & 15) || f->stride_b % 8 != 0 || f->stride_l % 8 != 0 || f->stride_r % 8 != 0) return false;
+  return true;
+}
+
+int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, const tpa::WindowJob& windows, hipStream_t stream) {
+  if (!tpa_recon_dense_qkv_takes(a)) return TPA_ERR_UNSUPPORTED;
   const int lmax = a->lq > a->lk ? a->lq : a->lk;
   const int64_t blocks = ((int64_t)lmax * (a->dk / 8) * (a->H / 8) + 255) / 256;
   if (blocks > 2147483647LL) return TPA_ERR_UNSUPPORTED;

@@ -388,4 +388,6 @@ size_t tpa_prefill_call_bytes(const TpaFwdArgs* a);
 int tpa_recon_dense_bf16(const TpaFactor* fa, const TpaFactor* fb, uint16_t* out, int B, int L, int H, int D, int R, float scale, hipStream_t stream);
 // dense Q (times q_scale), K, V of a forward call in one launch; TPA_ERR_UNSUPPORTED where the vectorised kernel does not apply
 // (and the windows of packed documents, see WindowJob)
+// whether the bf16 launch below takes these factors (whole groups of 8 heads, 16-byte rows)
+bool tpa_recon_dense_qkv_takes(const TpaFwdArgs* a);
 int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, uint16_t* vd, float q_scale, const tpa::WindowJob& windows, hipStream_t stream);

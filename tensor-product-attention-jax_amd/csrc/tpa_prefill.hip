@@ -1292,6 +1292,19 @@ int tpa_prefill_wants_dense(int64_t lq, int64_t lk, int64_t rk) {
 
 namespace tpa {
 namespace {
+// One block of query rows over fewer than 1024 keys, any rank but 2: the rebuild that the fused kernel does for every tile of 64 keys,
+// against a launch more and the trip of the dense arrays through memory.  Fitted to 500 shapes of 17 to 256 rows, 8 to 1024 (batch,
+// head) pairs, ranks 1, 3, 4 and 8 (us, within 5 of each): a tile costs 0.55 + 0.36 R more where it is rebuilt at head size 64, 0.55 + 0.57 R
+// at 128 (there rank 8 more than that, its loop waits for every rank's loads), for every round of workgroups a compute unit takes - at 64 two of them share
+// one, so that pairs beyond 256 add 0.7 of a round.  Fused / dense, us: rank 4, 1 x 250 rows, 8 heads of 64 17.3 / 12.1; 2 x 130 over 900, 32 heads of 128
+// 73.7 / 42.1; 12 x 200, 32 heads of 128 57.8 / 42.9; 8 x 200, 64 heads of 64 27.7 / 34.3 (stays fused); 4 x 40, 64 heads of 64 9.6 / 10.8 (stays);
+// rank 8, 1 x 130 over 900, 16 heads of 128 188 / 34; rank 1, 1 x 130 over 900, 8 heads of 64 31.2 / 20.2; 8 x 250, 32 heads of 128 22.6 / 32.2 (stays).
+bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
+  if (lk >= 1024 || H % 8 != 0) return false;  // beyond that the rule above has spoken; other head counts take three launches
+  const double pairs = (double)(B * H), tiles = (double)((lk + kTK - 1) / kTK), mb = pairs * (double)((lq + 2 * lk) * D) * 2e-6;
+  if (D == 64) return (pairs > 366 ? pairs / 366 : 1.0) * tiles * (0.55 + 0.36 * rk) > 4.5 + 0.28 * mb;
+  return (double)((B * H + 255) / 256) * tiles * (0.55 + 0.57 * rk) > 2.0 + 0.21 * mb;
+}
 // The same for one call, of which the number of workgroups (of 256 rows) is known.  Rank 2 below 2048 rows, dense over fused time, no
 // mask / causal / packed documents, 8 to 400 (batch, head) pairs of 512 to 2040 rows each (head size 64 with four or eight waves as
 // wants_four_waves has it for either):
@@ -1303,7 +1316,8 @@ namespace {
 //   more, of fewer rows: 512 rows 1.01 - 1.07, 700 to 900 0.81 - 0.99, with more keys than rows up to 1.32
 bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   if (tpa_prefill_wants_dense(lq, lk, rk)) return true;
-  if (rk != 2 || lq <= kBQ || lk > 5 * lq) return false;
+  if (rk != 2) return one_block_pays(B, lq, lk, H, D, rk);
+  if (lq <= kBQ || lk > 5 * lq) return false;
   const int64_t wgs = B * H * ((lq + kBQ - 1) / kBQ);
   return wgs <= 64 ? D == 128 : wgs > 256 && lq >= 1000;
 }
@@ -1327,7 +1341,9 @@ struct PrefillRoute {
 };
 PrefillRoute route_of(const TpaFwdArgs* a) {
   const int tiles = (int)(((int64_t)a->lk + kTK - 1) / kTK);  // a caller's count beyond that only adds empty ranges
-  return {dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
+  // one block of rows is made dense for the time of one launch, so only where the factors allow that
+  const bool pays = dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) && (tpa_prefill_wants_dense(a->lq, a->lk, a->rk) || a->rk == 2 || tpa_recon_dense_qkv_takes(a));
+  return {pays ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
           a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0)};
 }
 
