@@ -1221,13 +1221,26 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
 // and the partial results at 4 TB/s; the launch takes its rounds of 256 average workgroups, or the heaviest workgroup.
 // Measured, us without / with ranges: a chunk of 331 tokens over 2258 keys, 16 heads of 128: 97 / 73; 608 over 11433, 8
 // heads of 64: 182 / 76; one sequence of 4096 tokens, 8 heads of 64, causal: 70 / 47.
-int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, bool causal) {
+// Fewer than 24 tiles: of 2 and more blocks 512 to 1400 rows gain at most 8 % and lose up to twofold.  One block, where the ranges
+// find compute units that have nothing to do: a tile of the rank-2 rebuild is 2.0 us (1.1 at D = 64), one of dense arrays 1.55 (0.65),
+// a second range 9.5 and its partial results.  140 rows over 1160 keys, us without / with: rank 2, 8 heads of 128 44.4 / 29.6, 2 x 32 heads of 128
+// 45.1 / 39.5, 8 heads of 64 25.7 / 21.9; rank 4, 8 heads of 128 35.6 / 26.7; 4 x 16 heads of 64 26.2 / 26.2 (one range), rank 4 29.7 / 31.3 (one).
+int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk, bool causal) {
   const int64_t blocks = (lq + kBQ - 1) / kBQ, wgs = blocks * B * H;
   const double per_tile = D == 128 ? 1.7 : 1.3, per_wg = 7.0, most = (double)((lk + kTK - 1) / kTK);
   // tiles of an average block: under the causal mask the first one sees (lk - lq + 256) keys, the last one all
   const double least = lk > lq ? (double)(lk - lq) / kTK : 0.0, avg = causal ? 0.5 * (least + most) + 2.0 : most;
-  if (most < 24) return 1;  // a block's own tiles take 40 us at most: little to win over the merge
   int best = 1;
+  if (most < 24) {  // a block's own tiles take 40 us at most: little to win over the merge, but where one block has them all
+    if (blocks > 1) return 1;
+    const double tile = rk == 2 ? (D == 128 ? 2.0 : 1.1) : (D == 128 ? 1.55 : 0.65);
+    double gain = 1.5;
+    for (int S = 2; S <= 8 && wgs * S <= 256; ++S) {
+      const double us = tile * (double)((int64_t)most - ((int64_t)most + S - 1) / S) - 9.5 - (double)S * B * lq * H * D * 8.0 / 4e6;
+      if (us > gain) { best = S; gain = us; }
+    }
+    return best;
+  }
   double best_us = 0.0;
   for (int S = 1; S <= 16 && wgs * S <= 1024 && (S == 1 || most >= 2 * S); ++S) {
     const double heaviest = per_wg + per_tile * (double)(((int64_t)most + S - 1) / S), all = (double)((wgs * S + 255) / 256) * (per_wg + per_tile * avg / S);
@@ -1326,7 +1339,7 @@ bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t
 
 size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   const size_t dense = tpa::dense_pays(B, lq, lk, H, D, rk) ? tpa_prefill_dense_bytes(B, lq, lk, H, D) : 0;
-  const int s0 = tpa::choose_splits(B, lq, lk, H, D, false), s1 = tpa::choose_splits(B, lq, lk, H, D, true);
+  const int s0 = tpa::choose_splits(B, lq, lk, H, D, rk, false), s1 = tpa::choose_splits(B, lq, lk, H, D, rk, true);
   return dense + tpa::split_bytes(B, lq, H, D, s0 > s1 ? s0 : s1);
 }
 
@@ -1344,7 +1357,7 @@ PrefillRoute route_of(const TpaFwdArgs* a) {
   // one block of rows is made dense for the time of one launch, so only where the factors allow that
   const bool pays = dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) && (tpa_prefill_wants_dense(a->lq, a->lk, a->rk) || a->rk == 2 || tpa_recon_dense_qkv_takes(a));
   return {pays ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
-          a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->causal != 0)};
+          a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->rk, a->causal != 0)};
 }
 
 }  // namespace

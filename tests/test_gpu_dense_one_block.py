@@ -33,6 +33,7 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
     fake = d.TpaFactor(256, 8, 8, 8)
     call = _forward_call(B=B, H=H, D=D, lq=lq, lk=lk, rk=rk, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake)
     call.kernel = d.KERNEL_MFMA
+    call.num_splits = 1
     need = lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call))
     slot = lambda n: (2 * n + 255) // 256 * 256
     assert need == (slot(B * lq * H * D) + 2 * slot(B * lk * H * D) if dense else 0)
