@@ -4,9 +4,9 @@
 // prefill kernels read.  The reference has no such step (its tests draw the factors at random,
 // tpa/tpa_test.py:86-91); the arithmetic follows arXiv 2501.06425, section 3.
 //
-// bf16, three kernels by the number of new tokens: 256 x 256 or 128 x 128 tiles for a large prefill chunk, 64 x 64 tiles
-// below that, and for a decode step and other few tokens a kernel whose workgroups own 16 columns
-// and split the contraction over their waves.  All of them compute with v_mfma_f32_*_bf16, stage the
+// bf16, three kernels by the number of new tokens: tiles of 256 x 256 or 128 x 128 whose quarters belong to four waves for a large
+// prefill chunk, tiles of 64 x 64 or 64 x 128 whose contraction is dealt to four waves for an ordinary one, and for a decode
+// step and other few tokens a kernel whose workgroups own 16 columns and split the contraction over their waves.  All of them compute with v_mfma_f32_*_bf16, stage the
 // fp32 results in LDS, and finish whole 16-byte chunks of eight columns: a chunk lies inside one rank
 // row of one factor (H and D are multiples of 8), so the rotation partners (2j, 2j+1) are inside it.
 // Any other dtype / shape: one thread per chunk of eight columns, fp32 arithmetic.
@@ -30,10 +30,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 template <int V>
 using IC = std::integral_constant<int, V>;
-
-constexpr int kBM = 64, kBN = 64, kBK = 64;
-constexpr int kXS = kBK + 8;   // LDS row stride of the x / W tiles (elements): 16-byte reads of 32 rows are conflict free
-constexpr int kCS = kBN + 4;   // LDS row stride of the staged fp32 tile
 
 struct AppendParams {
   const void* x;
@@ -128,95 +124,6 @@ __device__ __forceinline__ bool tile_of_workgroup(int id, int ntm, int ntn, int&
   return t < (int)((tiles * (xcd + 1) + 7) / 8);
 }
 inline unsigned tile_workgroups(int ntm, int ntn) { return (unsigned)(((int64_t)ntm * ntn + 7) / 8 * 8); }
-
-// ---- bf16, 64 x 64 tiles: four waves, one 32 x 32 block each; x and W tiles of 64 x 64 double buffered in LDS,
-// the next tiles in registers while the current ones are multiplied.  One tile on a compute unit waits for its loads (0.6 us a
-// step for 0.06 us of matrix work), so KS groups of four waves deal the steps among themselves, each with buffers of its own, and
-// their sums meet in LDS: d_model 4096, 600 tokens x 1600 columns 38 -> 20 us, 1000 x 1600 with two groups 39 -> 28.  With four
-// groups the LDS is what bounds a step (192 KB, 0.7 of 1 us); loads two steps ahead change nothing.
-constexpr int kTileStage = (kBM + kBN) * kXS;
-template <int KS>
-__global__ __launch_bounds__(256 * KS) void append_mfma_kernel(AppendParams p, int ntm, int ntn) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t tile_mem[];  // [KS][2][x | W][64][kXS]
-  const int grp = KS > 1 ? scalar(threadIdx.x >> 8) : 0;
-  uint16_t* const mem = tile_mem + grp * 2 * kTileStage;
-  const int tid = threadIdx.x & 255, w = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
-  int tm, tn;
-  if (!tile_of_workgroup(blockIdx.x, ntm, ntn, tm, tn)) return;
-  const int m0 = tm * kBM, n0 = tn * kBN;
-  const int wm = w >> 1, wn = w & 1;       // this wave's 32 x 32 block of the tile
-
-  // loader: a 64 x 64 tile is 512 chunks of 16 bytes, two per thread (rows past the end read as zero)
-  constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
-  const __amdgpu_buffer_rsrc_t x_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.x) + (int64_t)m0 * p.K), 0, min(kBM, p.M - m0) * p.K * 2, kRsrcFlags);
-  const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.w) + (int64_t)n0 * p.K), 0, min(kBN, p.N - n0) * p.K * 2, kRsrcFlags);
-  const int lrow = tid >> 3, lc = tid & 7, voff = (lrow * p.K + 8 * lc) * 2;
-  const int nk = p.K / kBK, steps = (nk + KS - 1) / KS, mine = (nk - grp + KS - 1) / KS;  // this group takes steps grp, grp + KS, ..
-  u32x4 xr[2], wr[2];
-  auto load = [&](int kt) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int at = (32 * q * p.K + (grp + KS * kt) * kBK) * 2;
-      xr[q] = __builtin_amdgcn_raw_buffer_load_b128(x_rs, voff, at, 0);
-      wr[q] = __builtin_amdgcn_raw_buffer_load_b128(w_rs, voff, at, 0);
-    }
-  };
-  auto stage = [&](int buf) {
-    uint16_t* const xs = mem + buf * kTileStage + lrow * kXS + 8 * lc;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      *reinterpret_cast<u32x4*>(xs + 32 * q * kXS) = xr[q];
-      *reinterpret_cast<u32x4*>(xs + (kBM + 32 * q) * kXS) = wr[q];
-    }
-  };
-  f32x16 acc;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  if (mine > 0) { load(0); stage(0); }
-  __syncthreads();
-  for (int kt = 0; kt < steps; ++kt) {
-    if (kt + 1 < mine) load(kt + 1);
-    if (kt < mine) {
-      const uint16_t* xb = mem + (kt & 1) * kTileStage + (32 * wm + i) * kXS + 8 * g;
-      const uint16_t* wb = mem + (kt & 1) * kTileStage + (kBM + 32 * wn + i) * kXS + 8 * g;
-#pragma unroll
-      for (int ks = 0; ks < kBK / 16; ++ks) {
-        // A = 32 tokens x 16, B = 16 x 32 output columns (rows of W): acc[v] = y[token 8(v/4) + 4g + v%4][column i]
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(xb + 16 * ks);
-        const bf16x8 bq = *reinterpret_cast<const bf16x8*>(wb + 16 * ks);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bq, acc, 0, 0, 0);
-      }
-    }
-    if (kt + 1 < mine) stage((kt + 1) & 1);
-    __syncthreads();
-  }
-  // ---- stage the fp32 tiles (each reuses its group's buffers, which every wave has finished reading) and add them
-  constexpr int kGroupFloats = 2 * kTileStage / 2;
-  float* const all = reinterpret_cast<float*>(tile_mem);
-  static_assert(kGroupFloats >= kBM * kCS, "the staged tile fits a group's buffers");
-#pragma unroll
-  for (int v = 0; v < 16; ++v) all[grp * kGroupFloats + (32 * wm + 8 * (v >> 2) + 4 * g + (v & 3)) * kCS + 32 * wn + i] = acc[v];
-  __syncthreads();
-  for (int c = threadIdx.x; c < kBM * kBN / 8; c += 256 * KS) {
-    const int row = c >> 3, cc = c & 7;
-    const int m = m0 + row, c0 = n0 + 8 * cc;
-    if (m >= p.M || c0 >= p.N) continue;
-    float y[8] = {};
-#pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      const float* const src = all + k * kGroupFloats + row * kCS + 8 * cc;
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) { y[j] += lo[j]; y[4 + j] += hi[j]; }
-    }
-    bool rotate; int j0, pos;
-    uint16_t* dst = chunk_destination<uint16_t>(p, m, c0, rotate, j0, pos);
-    if (!dst) continue;
-    if (rotate) rotate_chunk(p, y, pos, j0);
-    store_chunk(dst, y);
-  }
-  write_new_lengths(p);
-}
 
 // ---- bf16, many new tokens (a prefill chunk): 256 tokens x 256 columns of y per workgroup, four waves
 // (one per SIMD, 512 registers each: the 256 accumulators sit in AGPRs).  A wave owns 128 tokens x 128
@@ -480,6 +387,188 @@ __global__ __launch_bounds__(256 * KS) void append_gemm_kernel(AppendParams p) {
   }
 }
 
+// ---- bf16, tiles of 64 tokens x 32 CB columns whose contraction is dealt to the four waves: each multiplies the whole tile by 16 of
+// the 64 k of a stage, so that every byte of a stage is read from LDS once (a wave that owns a quarter of the tile reads half of
+// both operands), and the four parts are added up at the end.  Stages go from memory straight to LDS, into a ring of NS, one barrier
+// for each: behind it everyone's share of the next stage has landed and the slot of this one, whose fragments are in
+// registers by then, takes the loads of the stage NS further on.  Loads, fragment reads and matrix instructions take turns - a wave that
+// has filled the queue of loads stands still, with its matrix unit.
+// What bounds it: bytes into the compute unit, of which the L2 delivers 115 to 135 a ns where nothing else is done, 108 with a
+// barrier and a read of each; the ring takes in 16 KB in 0.2 us (0.26 with all units at it) and 24 KB in 0.27, for 0.05 and 0.1 of matrix
+// work.  Two stages per barrier, deeper rings: the same.  d_model 4096, us with waves that own quarters and stage through
+// registers (two or four groups of them sharing the contraction) / now: 300 tokens x 1600 columns 19.2 / 15.3, 600 x 1600 20.9 / 16.9, 693 x 1600
+// 28.4 / 22.4, 844 x 2240 30.5 / 24.8; d_model 8192: 269 x 2560 32.3 / 24.0, 1160 x 1280 55 / 39.  (128 x 128 tiles in this way: 2048 x 1600
+// alone 38.2 / 34.8, but the attention behind it, which the power limit holds, takes 9 us more: 268 / 276 together.)
+template <int CB>
+struct StreamTile {
+  static constexpr int TB = 2, NS = 4;
+  static constexpr int kM = 32 * TB, kN = 32 * CB;    // tokens, columns per workgroup
+  static constexpr int kStage = (kM + kN) * 128;      // bytes of a stage: 64 k of the rows of x, then of W
+  static constexpr int kPass = 64;                    // columns of the tile that are added up at a time
+  static constexpr int kPS = kPass + 4;               // row stride (floats) of a wave's part of them
+  static constexpr int kPart = kM * kPS;
+  static constexpr int kBuffers = NS * kStage > 16 * kPart ? NS * kStage : 16 * kPart;
+  static constexpr size_t kLds = kBuffers + kM * 5 * sizeof(int32_t);
+};
+template <int CB>
+__global__ __launch_bounds__(256) void append_stream_kernel(AppendParams p) {
+  using Tile = StreamTile<CB>;
+  constexpr int TB = Tile::TB, NS = Tile::NS;
+  constexpr int kTM = Tile::kM, kTN = Tile::kN, NL = TB + CB;  // NL: loads and fragments of a wave per stage
+  extern __shared__ __attribute__((aligned(1024))) unsigned char stream_mem[];
+  int32_t* const table = reinterpret_cast<int32_t*>(stream_mem + Tile::kBuffers);  // [5][kTM]: pos, b, i, cache row coordinates
+  const int tid = threadIdx.x, w = scalar(tid >> 6), l = tid & 63, i = l & 31, g = l >> 5;
+  const int ntn = (p.N + kTN - 1) / kTN, ntm = (p.M + kTM - 1) / kTM;
+  int tm, tn;
+  if (!tile_of_workgroup(blockIdx.x, ntm, ntn, tm, tn)) return;
+  const int m0 = tm * kTM, n0 = tn * kTN;
+
+  // A load instruction brings 8 rows x 64 k straight to LDS, 16 bytes a lane in lane order: the lane of chunk c of row r fetches
+  // chunk c ^ (r / 2 & 7), so that reads of one chunk of 16 rows in a row meet no bank twice.  (Rows past the end read as zeros.)
+  typedef uint32_t Resource __attribute__((ext_vector_type(4)));
+  auto resource = [&](const void* base, int rows) __attribute__((always_inline)) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(base);
+    return Resource{(uint32_t)scalar((int)(uint32_t)at), (uint32_t)scalar((int)((uint32_t)(at >> 32) & 0xffff)), (uint32_t)scalar(rows * p.K * 2), 0x00020000u};
+  };
+  const Resource x_rs = resource(static_cast<const uint16_t*>(p.x) + (int64_t)m0 * p.K, min(kTM, p.M - m0));
+  const Resource w_rs = resource(static_cast<const uint16_t*>(p.w) + (int64_t)n0 * p.K, min(kTN, p.N - n0));
+  const int voff = ((l >> 3) * p.K + 8 * ((l & 7) ^ (4 * (w & 1) + (l >> 4)))) * 2;
+  const int nk = p.K / 64;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)stream_mem;
+  auto load = [&](auto j_c, int kt, int slot) __attribute__((always_inline)) {  // (stages past the last repeat it: loaded, never used)
+    constexpr int j = decltype(j_c)::value;
+    const int row = 8 * (4 * j + w - (j < TB ? 0 : 4 * TB));
+    const int soff = scalar((row * p.K + 64 * min(kt, nk - 1)) * 2);
+    const uint32_t to = (uint32_t)scalar((int)(lds0 + slot * Tile::kStage + 1024 * (4 * j + w)));
+    const Resource rs = j < TB ? x_rs : w_rs;
+    const int at = voff;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to), "v"(at), "s"(rs), "s"(soff) : "memory");
+  };
+  for (int c = 0; c < NS; ++c) static_for<NL>([&](auto j) __attribute__((always_inline)) { load(j, c, c); });
+
+  if (tid < kTM) {  // what the end needs to know about a token (one per thread)
+    const int m = min(m0 + tid, p.M - 1);
+    const int b = m / p.n, ii = m % p.n;
+    const int base_len = p.kvlen ? max(0, min(p.kvlen[b], p.cache_len)) : 0;
+    int pos = p.positions ? p.positions[(int64_t)b * p.n + ii] : base_len + ii;
+    pos = max(0, min(pos, p.rope_len - 1));
+    const int t = base_len + ii;
+    int ra = b, rb = t;
+    if (t >= p.cache_len) { ra = 0; rb = -1; }  // dropped
+    else if (p.page_table) { ra = p.page_table[(int64_t)b * p.pages_per_seq + t / p.page_size]; rb = t % p.page_size; }
+    table[tid] = pos; table[kTM + tid] = b; table[2 * kTM + tid] = ii; table[3 * kTM + tid] = ra; table[4 * kTM + tid] = rb;
+  }
+  if (blockIdx.x == 0) write_new_lengths(p);
+
+  f32x16 acc[CB][TB];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[cb][tb][v] = 0.f;
+  bf16x8 frag[2][NL];  // TB of x, CB of W
+  const unsigned char* const mine = stream_mem + i * 128 + (((2 * w + g) ^ (i >> 1 & 7)) * 16);
+  auto read = [&](auto set_c, auto j_c, int slot) __attribute__((always_inline)) {
+    constexpr int j = decltype(j_c)::value;
+    frag[decltype(set_c)::value][j] = *reinterpret_cast<const bf16x8*>(mine + slot * Tile::kStage + 4096 * j);
+  };
+  // acc[cb][tb][v] = part of y[token 32 tb + i][column 32 cb + 8 (v / 4) + 4 g + v % 4]
+  int slot = 0;
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * NL) : "memory");
+  static_for<NL>([&](auto j) __attribute__((always_inline)) { read(IC<0>{}, j, 0); });
+  auto step = [&](int kt, auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+    const int next = slot + 1 == NS ? 0 : slot + 1;
+    // this wave's loads of the next stage have landed and its fragments of this one are here; behind the barrier, everyone's
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * NL) : "memory");
+    constexpr int MF = TB * CB;
+    static_for<MF>([&](auto n_c) __attribute__((always_inline)) {
+      constexpr int n = decltype(n_c)::value;
+      constexpr int cb = n / TB, tb = n % TB;
+      acc[cb][tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[set][TB + cb], frag[set][tb], acc[cb][tb], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<2 * NL>([&](auto e_c) __attribute__((always_inline)) {
+        constexpr int e = decltype(e_c)::value;
+        if constexpr (e * MF / (2 * NL) == n) {
+          if constexpr (e % 2 == 1) read(IC<1 - set>{}, IC<e / 2>{}, next);
+          else load(IC<e / 2>{}, kt + NS, slot);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      });
+    });
+    slot = next;
+  };
+  int kt = 0;
+  for (; kt + 1 < nk; kt += 2) { step(kt, IC<0>{}); step(kt + 1, IC<1>{}); }
+  if (kt < nk) step(kt, IC<0>{});
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // nothing is on its way to the buffers any more, and nobody reads them
+
+  // ---- the four parts of a piece of the tile meet in LDS, and each thread finishes two chunks of eight columns
+  constexpr int kPass = Tile::kPass, kPS = Tile::kPS, kCpr = kPass / 8;
+  float* const parts = reinterpret_cast<float*>(stream_mem);
+  const int cc = tid % kCpr, row0 = tid / kCpr, half_d = p.D / 2;
+  static_for<kTN / kPass>([&](auto pass_c) __attribute__((always_inline)) {
+    constexpr int pass = decltype(pass_c)::value;
+#pragma unroll
+    for (int cq = 0; cq < kPass / 32; ++cq)
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int vq = 0; vq < 4; ++vq) {
+          const f32x16& t = acc[pass * (kPass / 32) + cq][tb];
+          *reinterpret_cast<f32x4*>(parts + w * Tile::kPart + (32 * tb + i) * kPS + 32 * cq + 8 * vq + 4 * g) = f32x4{t[4 * vq], t[4 * vq + 1], t[4 * vq + 2], t[4 * vq + 3]};
+        }
+    const int c0 = n0 + kPass * pass + 8 * cc;
+    int f = 0;
+#pragma unroll
+    for (int k = 1; k < 6; ++k) f += c0 >= p.seg[k];
+    const int width = (f & 1) ? p.D : p.H;
+    const int local = c0 - p.seg[f], r = local / width, e = local % width;
+    const bool rotate = f == 1 || f == 3;
+    auto pick = [&](auto get) __attribute__((always_inline)) {
+      return f == 0 ? get(p.qa) : f == 1 ? get(p.qb) : f == 2 ? get(p.ka) : f == 3 ? get(p.kb) : f == 4 ? get(p.va) : get(p.vb);
+    };
+    uint16_t* const base = static_cast<uint16_t*>(const_cast<void*>(pick([](const TpaFactor& t) { return t.ptr; }))) +
+                           (int64_t)r * pick([](const TpaFactor& t) { return t.stride_r; }) + e;
+    const int64_t sb = pick([](const TpaFactor& t) { return t.stride_b; }), sl = pick([](const TpaFactor& t) { return t.stride_l; });
+    typedef f32x4 Angles __attribute__((aligned(4)));  // the tables may start at any element
+    int64_t off[2];
+    f32x4 c4[2], s4[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int tl = row0 + u * (256 / kCpr);
+      const int32_t* const place = table + (f < 2 ? kTM : 3 * kTM) + tl;
+      const int ra = place[0], rb = place[kTM];
+      off[u] = c0 < p.N && m0 + tl < p.M && rb >= 0 ? ra * sb + rb * sl : -1;
+      const int64_t at = rotate && c0 < p.N ? (int64_t)table[tl] * half_d + (e >> 1) : 0;
+      c4[u] = *reinterpret_cast<const Angles*>(p.cosv + at);
+      s4[u] = *reinterpret_cast<const Angles*>(p.sinv + at);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float* const src = parts + (row0 + u * (256 / kCpr)) * kPS + 8 * cc;
+      f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+      for (int ww = 1; ww < 4; ++ww) {
+        lo += *reinterpret_cast<const f32x4*>(src + ww * Tile::kPart);
+        hi += *reinterpret_cast<const f32x4*>(src + ww * Tile::kPart + 4);
+      }
+      float y[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float a0 = y[2 * j], b0 = y[2 * j + 1];
+        const float ya = a0 * c4[u][j] - b0 * s4[u][j], yb = b0 * c4[u][j] + a0 * s4[u][j];
+        y[2 * j] = rotate ? ya : a0;
+        y[2 * j + 1] = rotate ? yb : b0;
+      }
+      if (off[u] >= 0) store_chunk(base + off[u], y);
+    }
+    __syncthreads();
+  });
+}
+
 // ---- bf16, few tokens (a decode step): the call is one read of W, and tiles of 64 columns would leave most of the chip idle.
 // A workgroup owns 16 columns, up to 64 tokens and all of k: each of its eight waves takes an eighth of the chunks of 64 k, stages
 // its own chunk (16 rows of W and the tokens' rows, whole cache lines in 16-byte pieces, kept in flight in registers several
@@ -655,10 +744,10 @@ __global__ __launch_bounds__(256) void append_generic_kernel(AppendParams p) {
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 // The tiles of 256 x 256 and 128 x 128 read the rotation tables four angles at a time, and take what is more than one round of
-// the 64 x 64 tiles with their contraction in two groups (512 of them).  d_model 4096, us of 64 x 64 / 128 x 128: 1200 tokens x
-// 1600 columns (475) 29.9 / 37.2, 416 x 4608 (504) 33 / 38, 1536 x 1440 (552) 39.6 / 37.4, 600 x 4096 (640) 42.8 / 37.2.
+// the 64 x 64 tiles with two of them on a compute unit (512).  d_model 4096, us of 64 x 64 or 64 x 128 / 128 x 128: 844 tokens x
+// 2240 columns (490) 24.8 / 31.3, 2482 x 720 (468) 23.9 / 31.4, 1536 x 1440 (552) 38.3 / 36.4, 600 x 4096 (640) 37.7 / 35.5.
 bool gemm_tiles_pay(const AppendParams& p, const TpaAppendArgs* a) {
-  const int64_t tiles = (int64_t)((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
+  const int64_t tiles = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64);
   return tiles > 512 && tiles < (1 << 28) && p.K < (1 << 22) && p.D % 8 == 0 && aligned16(a->rope_cos) && aligned16(a->rope_sin);
 }
 
@@ -674,14 +763,14 @@ int launch_gemm(const AppendParams& p, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
-template <int KS>
-int launch_tiles(const AppendParams& p, hipStream_t s) {
-  const int ntm = (p.M + kBM - 1) / kBM, ntn = (p.N + kBN - 1) / kBN;
-  constexpr size_t lds = (size_t)KS * 2 * kTileStage * sizeof(uint16_t);
-  auto kern = append_mfma_kernel<KS>;
+template <int CB>
+int launch_stream(const AppendParams& p, hipStream_t s) {
+  using Tile = StreamTile<CB>;
+  const int ntn = (p.N + Tile::kN - 1) / Tile::kN, ntm = (p.M + Tile::kM - 1) / Tile::kM;
+  auto kern = append_stream_kernel<CB>;
   static bool configured[kMaxDevices] = {};
-  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds); rc != TPA_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(tile_workgroups(ntm, ntn)), dim3(256 * KS), lds, s, p, ntm, ntn);
+  if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), Tile::kLds); rc != TPA_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(tile_workgroups(ntm, ntn)), dim3(256), Tile::kLds, s, p);
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
@@ -693,17 +782,15 @@ int rows_cost(const AppendParams& p, int mb) {
   const int64_t per_xcd = (int64_t)(((p.N + 15) / 16 + 7) / 8) * ((p.M + 16 * mb - 1) / (16 * mb));
   return (int)std::min<int64_t>((per_xcd + 31) / 32 * (32 + 16 * mb), 1 << 20);
 }
-// Blocks of 16 tokens per workgroup if the few-token kernel serves the call, 0 if the tiles do: their time is nearly the same from
-// one tile to 256, and less of it is proportional to d_model than of the few tokens'.  us of this kernel / 64 x 64 tiles: d_model
-// 256, 100 tokens x 1440 columns (cost 128) 6.6 / 6.3, 48 x 1440 (64) 6.0 / 6.3; 512, 150 x 1440 (128) 7.0 / 7.2, 200 x 1440 (192)
-// 9.2 / 7.2; 1024, 150 x 1440 7.8 / 8.8, 200 x 1440 10.4 / 8.9; 2048, 10.1 / 12.0 and 12.6 / 12.1; 4096, 14.6 / 18.8 and 19.1 / 19.0;
-// 8192, 23.5 / 35.0 and 32.6 / 35.2; 4096 with more than 400 workgroups of 64 tokens: 600 x 720 20.6 / 19.7, 300 x 1600 24.5 / 19.1.
+// Blocks of 16 tokens per workgroup if the few-token kernel serves the call, 0 if the tiles do, whose time is nearly the same from
+// one tile to 100: 12 us at d_model 4096.  us of this kernel / 64 x 64 tiles by cost: d_model 4096, 160 tokens x 720 columns (cost 64)
+// 8.3 / 12.2, 128 x 1600 (96) 10.8 / 11.9, 80 x 2240 (128) 13.7 / 12.3, 160 x 1440 (128) 14.0 / 12.0, 128 x 2560 (192) 19.6 / 11.9; 2048, 128 x 1600
+// 7.7 / 8.7, 32 x 5120 (128) 11.0 / 8.4; 8192, 128 x 1600 17.2 / 24.4, 146 x 1440 (128) 20.6 / 25.8, 192 x 1600 (192) 30.5 / 24.5.
 int few_tokens(const AppendParams& p) {
-  if ((int64_t)((p.N + 15) / 16) * ((p.M + 63) / 64) > 400) return 0;
   int mb = 4;
   for (int n : {2, 1})
     if (rows_cost(p, n) < rows_cost(p, mb)) mb = n;
-  return (int64_t)rows_cost(p, mb) * (p.K + 320) <= (int64_t)208 * p.K ? mb : 0;
+  return rows_cost(p, mb) <= (p.K >= 8192 ? 128 : 96) ? mb : 0;
 }
 
 template <int MB>
@@ -762,7 +849,7 @@ extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
   p.N = p.seg[6];
 
   hipStream_t s = static_cast<hipStream_t>(stream);
-  bool mfma = a->kernel != TPA_KERNEL_GENERIC && a->dtype == TPA_DTYPE_BF16 && a->d_model % kBK == 0 && aligned16(a->x) && aligned16(a->w);
+  bool mfma = a->kernel != TPA_KERNEL_GENERIC && a->dtype == TPA_DTYPE_BF16 && a->d_model % 64 == 0 && aligned16(a->x) && aligned16(a->w);
   for (const TpaFactor* f : fs) mfma = mfma && chunk_ok(*f);
   if (a->kernel == TPA_KERNEL_MFMA && !mfma) return TPA_ERR_UNSUPPORTED;
   mfma = mfma && p.K < (1 << 24);  // up to 64 rows are read with offsets of 32 bits
@@ -785,9 +872,12 @@ extern "C" int tpa_cache_append(const TpaAppendArgs* a, void* stream) {
                                                                                             : launch_gemm<2, 1>(p, s);
     if (rc != TPA_OK) return rc;
   } else if (mfma) {
-    const int64_t ntm = (p.M + kBM - 1) / kBM, tiles = ntm * ((p.N + kBN - 1) / kBN);
+    // One round of 64 x 128 tiles where the 64 x 64 ones would share compute units, us of the latter / the former: d_model 8192, 1160
+    // tokens x 1280 columns (380 and 190 of them) 56 / 39, 4096, 844 x 2240 (490, 252) 29.5 / 25.1, 693 x 1600 (275, 143) 25.4 / 22.3; 2048, 1124 x
+    // 1280 (360, 180) 15.3 / 15.2; 1024 9.8 / 10.3.
+    const int64_t ntm = (p.M + 63) / 64, tiles = ntm * ((p.N + 63) / 64), wide = ntm * ((p.N + 127) / 128);
     if (ntm > 65535 || tiles > 2147483640) return TPA_ERR_SHAPE;
-    const int rc = tiles <= 256 ? launch_tiles<4>(p, s) : tiles <= 512 ? launch_tiles<2>(p, s) : launch_tiles<1>(p, s);
+    const int rc = tiles > 256 && wide <= 256 && p.K >= 2048 && p.K < (1 << 22) ? launch_stream<4>(p, s) : launch_stream<2>(p, s);
     if (rc != TPA_OK) return rc;
   } else {
     const int64_t chunks = (int64_t)p.M * (p.N / 8);
