@@ -65,6 +65,7 @@ struct PrefillParams {
   // dense loader with segment ids: 1 = the id window of a workgroup is an IdWindow in its first row of the output (written by the launch
   // that reconstructed Q, K, V, read before any of this workgroup's own results are written; no other workgroup writes that row of this head)
   int windows;
+  int by_length;  // 1: batch entries of different lengths go longest first (LongestFirst)
 };
 
 // LDS: three buffers of a K tile (tile j is read while tile j+1 is already there for waves that run
@@ -112,6 +113,32 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int V>
 using IC = std::integral_constant<int, V>;
 
+// Batch entries by their lengths, longest first (equal ones in their order): lane = batch entry, B <= 64.  A launch of several workgroups
+// per compute unit ends with the last of them, so the long ones start first; every workgroup works the order out, as the lengths are known on the
+// device only.
+constexpr int kMostOrdered = 64;
+struct LongestFirst {
+  int len, B;
+  __device__ __forceinline__ LongestFirst(const int32_t* kvlen, int B, int lk) : B(B) {
+    const int lane = threadIdx.x & 63;
+    len = max(0, min(kvlen[min(lane, B - 1)], lk));
+  }
+  // whether an order is worth anything: the lengths differ by more than an eighth of the longest
+  __device__ __forceinline__ bool differ() const {
+    const int longest = wave_max(len), shortest = wave_min(len);
+    return scalar(longest - shortest > longest >> 3);
+  }
+  __device__ __forceinline__ int entry(int at) const {
+    const int lane = threadIdx.x & 63;
+    int ahead = 0;
+    for (int e = 0; e < B; ++e) {
+      const int other = __builtin_amdgcn_readlane(len, e);
+      ahead += other > len || (other == len && e < lane);
+    }
+    return scalar(__builtin_ctzll(__ballot(lane < B && ahead == at)));
+  }
+};
+
 template <int D, int LOADER, bool SEG, bool SPLIT, int NW>
 __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
   // row blocks per wave: the per-wave state below is indexed by row block, and one is what fits 256 registers
@@ -157,11 +184,28 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
     qblk = p.nqb - 1 - rank;
     b = bh / p.H;
     h = bh % p.H;
+    if constexpr (!SEG)
+      if (pp.by_length) b = LongestFirst(p.kvlen, p.B, p.lk).entry(b);
   } else {
+    // Where the lengths differ, all heads of an entry on one XCD, or of the same entries in every round, would leave the XCDs of the short
+    // ones idle: the heads then go in eight groups, one per XCD, and an entry's blocks side by side.
     int pair;
-    if (!pair_of_workgroup(id, p.npairs, p.H, p.B, p.head_groups, pair, h)) return;
-    qblk = p.nqb - 1 - pair / p.B;
-    b = pair % p.B;
+    bool differ = false;
+    if constexpr (!SEG)
+      if (pp.by_length) {
+        const LongestFirst order(p.kvlen, p.B, p.lk);
+        differ = order.differ();
+        if (differ) {
+          if (!pair_of_workgroup(id, p.npairs, p.H, p.B, 8, pair, h)) return;
+          qblk = p.nqb - 1 - pair % p.nqb;
+          b = order.entry(pair / p.nqb);
+        }
+      }
+    if (!differ) {
+      if (!pair_of_workgroup(id, p.npairs, p.H, p.B, p.head_groups, pair, h)) return;
+      qblk = p.nqb - 1 - pair / p.B;
+      b = pair % p.B;
+    }
   }
 
   int range = 0;
@@ -1179,6 +1223,18 @@ inline bool wants_four_waves(const PrefillParams& p, bool dense) {
   return (dense ? 1.06 : 1.13) * tiles(128) < 2.0 * tiles(256);
 }
 
+// Batch entries of different lengths, longest first, where a launch is more than a round of workgroups and a half; in one round there is
+// nothing to order, and an XCD that meets every entry has more factors to fetch.  Over a cache of at least twice the rows: with fewer keys a
+// causal block's place weighs as much as the length.  us before / now, mean of four sets of lengths from half of the cache on (all equal), rank 2: 9 x
+// 512 rows over 8192, 16 heads of 128 (288 workgroups) 327 / 334, 5 x 512, 32 heads (320) 342 / 341, 2 x 1500, 32 heads (384) 355 / 347 (422 / 423),
+// 3 x 500 over 4000, 64 heads of 64 (384) 129 / 124 (148 / 151); one set, 512 workgroups and more: 8 x 512 over 8192, 32 heads of 128 458 / 391 (523 /
+// 525), 4 x 1024 451 / 405 (506 / 508), 4 x 512, 64 heads of 64 272 / 233 (329 / 326), 8 x 300 over 4000 254 / 226 (282 / 285); rank 4, dense tiles: 16 x
+// 300 over 4000, 32 heads of 128 648 / 628 (732 / 734).  Ranges do not count as rounds: 7 x 1000 over 9000, 8 heads of 128, 224 blocks in two
+// each 241 / 249.  (The grid covers eight groups of heads as well: they are npairs * H workgroups.)
+bool longest_first_pays(const PrefillParams& p) {
+  return p.kvlen && p.B > 1 && p.B <= kMostOrdered && p.H % 8 == 0 && p.lk >= 2 * (int64_t)p.lq && (int64_t)p.npairs * p.H >= 384 * p.S;
+}
+
 template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8>
 int launch_prefill(const PrefillParams& p, hipStream_t stream) {
   if constexpr (!SEG && !SPLIT && NW == 8)
@@ -1197,6 +1253,7 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds_bytes); rc != TPA_OK) return rc;
   // one workgroup per (query block, batch, head): see the kernel for how ids map to them
   int64_t n;
+  q.by_length = !SEG && longest_first_pays(p);
   if (LOADER == LOAD_DENSE) {
     q.pair_groups = dense_pair_groups(p.B * p.H, p.nqb, NW == 4, p.causal != 0);
     n = pair_group_workgroups(p.B * p.H, p.nqb);
