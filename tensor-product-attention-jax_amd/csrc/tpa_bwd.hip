@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256) void project_kernel(const float* dx, TpaFactor
 // All arrays that this kernel takes in one launch (blockIdx.z): at short lengths a launch of its own leaves each of them
 // waiting for the one before.  The gradients are written in the type the caller wants them in (rounded once, from the fp32 sums).
 struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R, D; };
-struct ProjectJobs { ProjectJob job[3]; };
+struct ProjectJobs { ProjectJob job[3]; int first[3], ranks; };  // array i: blockIdx.z = first[i] on, `ranks` ranks for each
 template <typename T>
 using Four = std::conditional_t<sizeof(T) == 2, u32x2, f32x4>;  // four values as they lie in memory
 __device__ __forceinline__ f32x4 as_f32(const u32x2& x) { return f32x4{bf16lo_to_f32(x[0]), bf16hi_to_f32(x[0]), bf16lo_to_f32(x[1]), bf16hi_to_f32(x[1])}; }
@@ -626,7 +626,9 @@ __device__ __forceinline__ float swap_add(float x, float y) {
 }
 template <typename T, typename TO>
 __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H) {
-  const ProjectJob j = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
+  const int z = blockIdx.z, job = (z >= jobs.first[1]) + (z >= jobs.first[2]);
+  const ProjectJob j = job == 0 ? jobs.job[0] : job == 1 ? jobs.job[1] : jobs.job[2];
+  const int r0 = (z - (job == 0 ? jobs.first[0] : job == 1 ? jobs.first[1] : jobs.first[2])) * jobs.ranks;
   const TpaFactor &fa = j.fa, &fb = j.fb;
   const TpaGrad &ga = j.ga, &gb = j.gb;
   const int L = j.L, R = j.R, D = j.D;
@@ -668,10 +670,11 @@ __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H
     next[2] = *reinterpret_cast<const Four<T>*>(b);
     next[3] = *reinterpret_cast<const Four<T>*>(b + dh);
   };
-  request(0);
-  for (int r = 0; r < R; ++r) {
+  request(r0);
+  const int r1 = min(R, r0 + jobs.ranks);
+  for (int r = r0; r < r1; ++r) {
     const f32x4 al = as_f32(next[0]), ah = as_f32(next[1]), bl = as_f32(next[2]), bh = as_f32(next[3]);
-    if (r + 1 < R) request(r + 1);
+    if (r + 1 < r1) request(r + 1);
     float af[8], bf[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) { af[j] = al[j]; af[4 + j] = ah[j]; bf[j] = bl[j]; bf[4 + j] = bh[j]; }
@@ -745,6 +748,22 @@ bool projects_by_h8(const ProjectJob& j, int H) {
          al16(j.dx) && rows16<T>(j.fa) && rows16<T>(j.fb) && rows16<TO>(ga) && rows16<TO>(gb);
 }
 
+// Ranks that a workgroup of the launch takes.  One after the other they are a chain of 0.6 us each that a short call has too few workgroups
+// to hide, so there they are dealt to workgroups of their own, which read dx again, as long as these are no more than 400.  us, all ranks / so,
+// by workgroups of one array: ranks 16, 8, 8: 11 of them (335 tokens, 8 heads of 64) 14.9 / 6.5, 63 17.1 / 12.5 (four ranks each, 504 workgroups
+// 11.7), 99 19.0 / 15.8 (four each 19.0), 250 23.4 / 25.8; 6, 2, 2: 34 7.2 / 5.3, 54 7.8 / 7.2, fp32 64 8.6 / 7.0; 6, 4, 4: 175 13.1 / 13.5.
+int ranks_per_workgroup(const ProjectJobs& jobs, unsigned n, int64_t blocks) {
+  int most = 0;
+  for (unsigned i = 0; i < n; ++i) most = std::max(most, jobs.job[i].R);
+  for (int k = std::min(most / 2, 16); k > 1; --k) {
+    const int ranks = (most + k - 1) / k;
+    int64_t parts = 0;
+    for (unsigned i = 0; i < n; ++i) parts += (jobs.job[i].R + ranks - 1) / ranks;
+    if (blocks * parts <= 400) return ranks;
+  }
+  return most;
+}
+
 template <typename T, typename TO>
 void launch_project(const ProjectJobs& jobs, int B, int H, hipStream_t stream) {
   ProjectJobs h8{};
@@ -766,7 +785,14 @@ void launch_project(const ProjectJobs& jobs, int B, int H, hipStream_t stream) {
     else
       hipLaunchKernelGGL((project_kernel<T, TO, false>), dim3(j.L, B), dim3(256), 0, stream, j.dx, j.fa, j.fb, j.ga, j.gb, j.L, H, j.D, j.R, dsh, nsh);
   }
-  if (n) hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, n), dim3(256), 0, stream, h8, H);
+  if (!n) return;
+  h8.ranks = ranks_per_workgroup(h8, n, blocks * B);
+  unsigned parts = 0;
+  for (unsigned i = 0; i < 3; ++i) {
+    h8.first[i] = i < n ? (int)parts : INT32_MAX;
+    if (i < n) parts += (h8.job[i].R + h8.ranks - 1) / h8.ranks;
+  }
+  hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, parts), dim3(256), 0, stream, h8, H);
 }
 
 template <typename T, int DMAX>
