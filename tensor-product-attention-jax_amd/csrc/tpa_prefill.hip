@@ -65,7 +65,6 @@ struct PrefillParams {
   // dense loader with segment ids: 1 = the id window of a workgroup is an IdWindow in its first row of the output (written by the launch
   // that reconstructed Q, K, V, read before any of this workgroup's own results are written; no other workgroup writes that row of this head)
   int windows;
-  int by_length;  // 1: batch entries of different lengths go longest first (LongestFirst)
 };
 
 // LDS: three buffers of a K tile (tile j is read while tile j+1 is already there for waves that run
@@ -139,7 +138,9 @@ struct LongestFirst {
   }
 };
 
-template <int D, int LOADER, bool SEG, bool SPLIT, int NW>
+// ORDER: batch entries of different lengths go longest first (an instance of its own: as a branch it cost every call 0.25 us, 1 x 500 tokens,
+// 8 heads of 64 15.9 / 16.2)
+template <int D, int LOADER, bool SEG, bool SPLIT, int NW, bool ORDER>
 __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
   // row blocks per wave: the per-wave state below is indexed by row block, and one is what fits 256 registers
   // (two per wave on four waves of 512 registers were slower: one wave per SIMD issues too slowly)
@@ -184,23 +185,21 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(PrefillParams pp) {
     qblk = p.nqb - 1 - rank;
     b = bh / p.H;
     h = bh % p.H;
-    if constexpr (!SEG)
-      if (pp.by_length) b = LongestFirst(p.kvlen, p.B, p.lk).entry(b);
+    if constexpr (ORDER) b = LongestFirst(p.kvlen, p.B, p.lk).entry(b);
   } else {
     // Where the lengths differ, all heads of an entry on one XCD, or of the same entries in every round, would leave the XCDs of the short
     // ones idle: the heads then go in eight groups, one per XCD, and an entry's blocks side by side.
     int pair;
     bool differ = false;
-    if constexpr (!SEG)
-      if (pp.by_length) {
-        const LongestFirst order(p.kvlen, p.B, p.lk);
-        differ = order.differ();
-        if (differ) {
-          if (!pair_of_workgroup(id, p.npairs, p.H, p.B, 8, pair, h)) return;
-          qblk = p.nqb - 1 - pair % p.nqb;
-          b = order.entry(pair / p.nqb);
-        }
+    if constexpr (ORDER) {
+      const LongestFirst order(p.kvlen, p.B, p.lk);
+      differ = order.differ();
+      if (differ) {
+        if (!pair_of_workgroup(id, p.npairs, p.H, p.B, 8, pair, h)) return;
+        qblk = p.nqb - 1 - pair % p.nqb;
+        b = order.entry(pair / p.nqb);
       }
+    }
     if (!differ) {
       if (!pair_of_workgroup(id, p.npairs, p.H, p.B, p.head_groups, pair, h)) return;
       qblk = p.nqb - 1 - pair / p.B;
@@ -1230,30 +1229,32 @@ inline bool wants_four_waves(const PrefillParams& p, bool dense) {
 // 3 x 500 over 4000, 64 heads of 64 (384) 129 / 124 (148 / 151); one set, 512 workgroups and more: 8 x 512 over 8192, 32 heads of 128 458 / 391 (523 /
 // 525), 4 x 1024 451 / 405 (506 / 508), 4 x 512, 64 heads of 64 272 / 233 (329 / 326), 8 x 300 over 4000 254 / 226 (282 / 285); rank 4, dense tiles: 16 x
 // 300 over 4000, 32 heads of 128 648 / 628 (732 / 734).  Ranges do not count as rounds: 7 x 1000 over 9000, 8 heads of 128, 224 blocks in two
-// each 241 / 249.  (The grid covers eight groups of heads as well: they are npairs * H workgroups.)
-bool longest_first_pays(const PrefillParams& p) {
-  return p.kvlen && p.B > 1 && p.B <= kMostOrdered && p.H % 8 == 0 && p.lk >= 2 * (int64_t)p.lq && (int64_t)p.npairs * p.H >= 384 * p.S;
+// each 241 / 249.  Dense tiles of an XCD belong to a head of every entry anyway; they gain with up to two blocks of rows, and with four 8 x 1024
+// over 4096, 32 heads of 128 take 470 / 474 (551 / 564).  (The grid covers eight groups of heads as well: they are npairs * H workgroups.)
+bool longest_first_pays(const PrefillParams& p, bool dense) {
+  return p.kvlen && (!dense || p.lq <= 2 * kBQ) && p.B > 1 && p.B <= kMostOrdered && p.H % 8 == 0 && p.lk >= 2 * (int64_t)p.lq && (int64_t)p.npairs * p.H >= 384 * p.S;
 }
 
-template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8>
+template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8, bool ORDER = false>
 int launch_prefill(const PrefillParams& p, hipStream_t stream) {
-  if constexpr (!SEG && !SPLIT && NW == 8)
+  if constexpr (!SEG && !SPLIT && NW == 8 && !ORDER)
     if (p.S > 1) return launch_prefill<D, LOADER, SEG, true>(p, stream);
   PrefillParams q = p;
-  if constexpr (D == 64 && LOADER != LOAD_TPA_ANY && !SPLIT && NW == 8) {
+  if constexpr (D == 64 && LOADER != LOAD_TPA_ANY && !SPLIT && NW == 8 && !ORDER) {
     if (wants_four_waves(p, LOADER == LOAD_DENSE)) {
       q.nqb = (p.lq + kBQ / 2 - 1) / (kBQ / 2);
       q.npairs = q.nqb * p.B;
       return launch_prefill<D, LOADER, SEG, SPLIT, 4>(q, stream);
     }
   }
-  auto kern = prefill_kernel<D, LOADER, SEG, SPLIT, NW>;
+  if constexpr (!SEG && !ORDER)
+    if (longest_first_pays(p, LOADER == LOAD_DENSE)) return launch_prefill<D, LOADER, SEG, SPLIT, NW, true>(p, stream);
+  auto kern = prefill_kernel<D, LOADER, SEG, SPLIT, NW, ORDER>;
   constexpr size_t lds_bytes = Lds<D>::kBytes;
   static bool configured[kMaxDevices] = {};
   if (int rc = raise_lds_limit(configured, reinterpret_cast<const void*>(kern), lds_bytes); rc != TPA_OK) return rc;
   // one workgroup per (query block, batch, head): see the kernel for how ids map to them
   int64_t n;
-  q.by_length = !SEG && longest_first_pays(p);
   if (LOADER == LOAD_DENSE) {
     q.pair_groups = dense_pair_groups(p.B * p.H, p.nqb, NW == 4, p.causal != 0);
     n = pair_group_workgroups(p.B * p.H, p.nqb);
