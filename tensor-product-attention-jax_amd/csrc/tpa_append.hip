@@ -129,8 +129,7 @@ inline unsigned tile_workgroups(int ntm, int ntn) { return (unsigned)(((int64_t)
 // (one per SIMD, 512 registers each: the 256 accumulators sit in AGPRs).  A wave owns 128 tokens x 128
 // columns = 4 x 4 blocks of v_mfma_f32_32x32x16_bf16, computed transposed (A = rows of W, B = tokens), so
 // that a lane ends up with runs of four consecutive columns of one token.  A k step reads 8 fragments for
-// 16 MFMAs (the 64 x 64 tiles above read 2 for 1; eight waves of 64 x 128 read
-// 6 for 8 and measured the same time as this form).  x and W tiles of 256 rows x 64 k are double buffered
+// 16 MFMAs (eight waves of 64 x 128 read 6 for 8 and measured the same time as this form).  x and W tiles of 256 rows x 64 k are double buffered
 // in LDS (row stride 72 elements), raw buffer loads over the tile's rows only (rows past the end read as
 // zeros and are never stored).
 // One wave per SIMD has nobody to hide behind, so the order inside an iteration is fixed by hand:
@@ -578,8 +577,7 @@ __global__ __launch_bounds__(256) void append_stream_kernel(AppendParams p) {
 // behind the first one's way from HBM; hence the tokens are dealt to more workgroups while there are idle ones.
 // (Until now operands were read as fragments, half a cache line per row, and the contraction was split over workgroups with
 // a second kernel to add the parts.  d_model 4096, us before / now: 1 token x 1600 columns 10.9 / 7.2, 24 x 1440 11.6 / 7.6,
-// 48 x 1600 13.5 / 9.5, 64 x 4096 23.5 / 15.3; above 64 tokens against 64 x 64 tiles of one group: 128 x 1600 38 /
-// 13.6.)
+// 48 x 1600 13.5 / 9.5, 64 x 4096 23.5 / 15.3.)
 template <int MB>
 struct RowsTile {
   static constexpr int kTok = 16 * MB;
