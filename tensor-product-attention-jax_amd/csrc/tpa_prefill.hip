@@ -1376,6 +1376,14 @@ bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int
   if (D == 64) return (pairs > 366 ? pairs / 366 : 1.0) * tiles * (0.55 + 0.36 * rk) > 4.5 + 0.28 * mb;
   return (double)((B * H + 255) / 256) * tiles * (0.55 + 0.57 * rk) > 2.0 + 0.21 * mb;
 }
+// Rank 2 at head size 128: the fused kernel's Q, summed rank by rank through LDS, takes longer than the launch that makes dense arrays, as long as
+// these are few.  us, fused / dense, rank 6 of Q, by (batch, head) pairs: 8, 64 rows over 64 keys 14.2 / 10.4, 200 x 600 25.9 / 22.9; 32, 200 x 200 20.6 /
+// 17.7, 200 x 600 31.1 / 28.8, 40 x 900 26.9 / 28.8; 64, 130 x 130 18.6 / 16.6, 250 x 250 21.1 / 21.2; 128, 64 x 64 14.4 / 13.1, 130 x 130 18.7 / 19.5.
+// (16, 250 x 1000 31.8 / 31.7: from twelve tiles on the walk counts, not Q.  Head size 64: 0.82 - 1.15 with no such line.)
+constexpr int kSlowQ = 6;  // ranks of Q from which that holds
+bool one_block_of_rank_2_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D) {
+  return D == 128 && H % 8 == 0 && lq <= kBQ && lk <= 12 * kTK && B * H * (lq + 2 * lk) <= 40000;
+}
 // The same for one call, of which the number of workgroups (of 256 rows) is known.  Rank 2 below 2048 rows, dense over fused time, no
 // mask / causal / packed documents, 8 to 400 (batch, head) pairs of 512 to 2040 rows each (head size 64 with four or eight waves as
 // wants_four_waves has it for either):
@@ -1388,7 +1396,8 @@ bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int
 bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   if (tpa_prefill_wants_dense(lq, lk, rk)) return true;
   if (rk != 2) return one_block_pays(B, lq, lk, H, D, rk);
-  if (lq <= kBQ || lk > 5 * lq) return false;
+  if (lq <= kBQ) return one_block_of_rank_2_pays(B, lq, lk, H, D);
+  if (lk > 5 * lq) return false;
   const int64_t wgs = B * H * ((lq + kBQ - 1) / kBQ);
   return wgs <= 64 ? D == 128 : wgs > 256 && lq >= 1000;
 }
@@ -1413,7 +1422,7 @@ struct PrefillRoute {
 PrefillRoute route_of(const TpaFwdArgs* a) {
   const int tiles = (int)(((int64_t)a->lk + kTK - 1) / kTK);  // a caller's count beyond that only adds empty ranges
   // one block of rows is made dense for the time of one launch, so only where the factors allow that
-  const bool pays = dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) && (tpa_prefill_wants_dense(a->lq, a->lk, a->rk) || a->rk == 2 || tpa_recon_dense_qkv_takes(a));
+  const bool pays = dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) && (tpa_prefill_wants_dense(a->lq, a->lk, a->rk) || (a->rk == 2 && a->lq > kBQ) || (tpa_recon_dense_qkv_takes(a) && (a->rk != 2 || a->rq >= kSlowQ)));
   return {pays ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
           a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->rk, a->causal != 0)};
 }
