@@ -883,16 +883,46 @@ size_t tpa_prefill_f32_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H,
   if (H % 8 != 0 || !tpa::f32_dense_pays(B, lq, lk, H, D, rk)) return 0;
   return (size_t)(tpa::dense_slot(B * lq * H * D) + 2 * tpa::dense_slot(B * lk * H * D)) * 4;
 }
-size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a) { return tpa_prefill_f32_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->rk); }
 
-int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
-  using namespace tpa;
+namespace tpa {
+namespace {
+F32Params params_of(const TpaFwdArgs* a) {  // on the factors as they are
   F32Params p{};
   p.qa = a->qa; p.qb = a->qb; p.ka = a->ka; p.kb = a->kb; p.va = a->va; p.vb = a->vb;
   p.qseg = a->q_segment_ids; p.kvseg = a->kv_segment_ids; p.kvlen = a->kv_lengths;
   p.o = static_cast<float*>(a->o); p.lse = a->lse;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq; p.rk = a->rk;
   p.q_scale = a->sm_scale * kLog2e / (float)a->rq; p.causal = a->causal; p.coff = causal_offset_of(a);
+  return p;
+}
+// and with Q (the scale in it), K and V as dense arrays of H * D floats a row
+F32Params dense_params_of(const TpaFwdArgs* a, const float* qd, const float* kd, const float* vd) {
+  F32Params p = params_of(a);
+  const int64_t hd = (int64_t)a->H * a->dk;
+  p.qa = p.ka = p.va = TpaFactor{nullptr, 0, 0, 0};
+  p.qb = TpaFactor{qd, a->lq * hd, hd, 0};
+  p.kb = TpaFactor{kd, a->lk * hd, hd, 0};
+  p.vb = TpaFactor{vd, a->lk * hd, hd, 0};
+  p.rq = p.rk = 1;
+  p.q_scale = 1.f;
+  return p;
+}
+}  // namespace
+}  // namespace tpa
+
+size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a) {
+  using namespace tpa;
+  const size_t need = tpa_prefill_f32_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->rk);
+  // Rows of H * D floats reach the 2 GiB of the kernel of 32 rows before those of the factors do: a call that would fall from it to 256
+  // rows stays on the factors (64 rows over 140 000 keys, 32 heads of 128, rank 4: 128 workgroups that share out the keys against 32 with
+  // two of eight waves at work, and 4.6 GB).
+  if (need && rows_per_workgroup(params_of(a), a->dk) == 32 && !split_supported(dense_params_of(a, nullptr, nullptr, nullptr))) return 0;
+  return need;
+}
+
+int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
+  using namespace tpa;
+  F32Params p = params_of(a);
   if (const size_t need = tpa_prefill_f32_call_bytes(a); need && a->workspace && !(reinterpret_cast<uintptr_t>(a->workspace) & 255) && a->workspace_bytes >= need) {
     const int64_t hd = (int64_t)a->H * a->dk;
     float* const kd = static_cast<float*>(a->workspace);
@@ -900,12 +930,7 @@ int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
     float* const qd = vd + dense_slot(a->B * a->lk * hd);
     const int rc = tpa_recon_dense_qkv_f32(a, qd, kd, vd, a->sm_scale * kLog2e, stream);
     if (rc == TPA_OK) {
-      p.qa = p.ka = p.va = TpaFactor{nullptr, 0, 0, 0};
-      p.qb = TpaFactor{qd, a->lq * hd, hd, 0};
-      p.kb = TpaFactor{kd, a->lk * hd, hd, 0};
-      p.vb = TpaFactor{vd, a->lk * hd, hd, 0};
-      p.rq = p.rk = 1;
-      p.q_scale = 1.f;
+      p = dense_params_of(a, qd, kd, vd);
     } else if (rc != TPA_ERR_UNSUPPORTED) {
       return rc;
     }

@@ -34,6 +34,11 @@ from test_abi import _forward_call
         (1, 8, 64, 40, 699, 4, False),
         (1, 8, 64, 40, 700, 4, True),
         (1, 5, 64, 400, 700, 8, False),      # heads in no groups of eight
+        (1, 32, 128, 64, 131071, 4, True),   # the last dense entry below 2 GiB, which the kernel of 32 rows can address
+        (1, 32, 128, 64, 131072, 4, False),
+        (1, 32, 128, 64, 140000, 4, False),
+        (2, 64, 64, 17, 131072, 8, False),
+        (9, 32, 128, 64, 140000, 4, True),   # 576 workgroups of 32 rows: on the factors 256 rows too
     ],
 )
 def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
