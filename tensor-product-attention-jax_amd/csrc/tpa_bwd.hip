@@ -1000,13 +1000,21 @@ int tpa_recon_dense_qkv_bf16(const TpaFwdArgs* a, uint16_t* qd, uint16_t* kd, ui
   return hipGetLastError() == hipSuccess ? TPA_OK : TPA_ERR_LAUNCH;
 }
 
-int tpa_recon_dense_qkv_f32(const TpaFwdArgs* a, float* qd, float* kd, float* vd, float q_scale, hipStream_t stream) {
-  const int cpr = a->dk / 4, lmax = a->lq > a->lk ? a->lq : a->lk;
-  const int64_t blocks = ((int64_t)lmax * cpr * (a->H / 8) + 255) / 256;
-  if (a->B > 65535 || a->H % 8 != 0 || a->dk != a->dv || (cpr != 16 && cpr != 32) || blocks > 2147483647LL) return TPA_ERR_UNSUPPORTED;
+namespace {
+int64_t recon_f32_blocks(const TpaFwdArgs* a) { return ((int64_t)(a->lq > a->lk ? a->lq : a->lk) * (a->dk / 4) * (a->H / 8) + 255) / 256; }
+}  // namespace
+
+bool tpa_recon_dense_qkv_f32_takes(const TpaFwdArgs* a) {
+  if (a->B > 65535 || a->H % 8 != 0 || a->dk != a->dv || (a->dk != 64 && a->dk != 128) || recon_f32_blocks(a) > 2147483647LL) return false;
   const TpaFactor* fs[6] = {&a->qa, &a->qb, &a->ka, &a->kb, &a->va, &a->vb};
   for (const TpaFactor* f : fs)
-    if (!tpa::rows16<float>(*f)) return TPA_ERR_UNSUPPORTED;
+    if (!tpa::rows16<float>(*f)) return false;
+  return true;
+}
+
+int tpa_recon_dense_qkv_f32(const TpaFwdArgs* a, float* qd, float* kd, float* vd, float q_scale, hipStream_t stream) {
+  if (!tpa_recon_dense_qkv_f32_takes(a)) return TPA_ERR_UNSUPPORTED;
+  const int64_t blocks = recon_f32_blocks(a);
   const int keys = tpa::keys_in_reach(a);
   tpa::ReconJobs jobs{};
   jobs.job[0] = tpa::ReconJob{a->qa, a->qb, qd, a->lq, a->rq, q_scale, a->lq, nullptr};

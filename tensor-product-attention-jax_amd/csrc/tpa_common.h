@@ -350,6 +350,8 @@ int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream);
 size_t tpa_prefill_f32_dense_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk);
 size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a);
 // dense fp32 Q (times q_scale), K, V of a forward call in one launch; TPA_ERR_UNSUPPORTED where the vectorised kernel does not apply
+// (whole groups of 8 heads of 64 or 128, 16-byte rows)
+bool tpa_recon_dense_qkv_f32_takes(const TpaFwdArgs* a);
 int tpa_recon_dense_qkv_f32(const TpaFwdArgs* a, float* qd, float* kd, float* vd, float q_scale, hipStream_t stream);
 int mha_prefill_f32_supported(const MhaFwdArgs* a);
 int mha_prefill_f32_launch(const MhaFwdArgs* a, hipStream_t stream);

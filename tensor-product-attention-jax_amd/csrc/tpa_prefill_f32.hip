@@ -912,6 +912,7 @@ F32Params dense_params_of(const TpaFwdArgs* a, const float* qd, const float* kd,
 
 size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a) {
   using namespace tpa;
+  if (!tpa_recon_dense_qkv_f32_takes(a)) return 0;
   const size_t need = tpa_prefill_f32_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->rk);
   // Rows of H * D floats reach the 2 GiB of the kernel of 32 rows before those of the factors do: a call that would fall from it to 256
   // rows stays on the factors (64 rows over 140 000 keys, 32 heads of 128, rank 4: 128 workgroups that share out the keys against 32 with
@@ -928,12 +929,8 @@ int tpa_prefill_f32_launch(const TpaFwdArgs* a, hipStream_t stream) {
     float* const kd = static_cast<float*>(a->workspace);
     float* const vd = kd + dense_slot(a->B * a->lk * hd);
     float* const qd = vd + dense_slot(a->B * a->lk * hd);
-    const int rc = tpa_recon_dense_qkv_f32(a, qd, kd, vd, a->sm_scale * kLog2e, stream);
-    if (rc == TPA_OK) {
-      p = dense_params_of(a, qd, kd, vd);
-    } else if (rc != TPA_ERR_UNSUPPORTED) {
-      return rc;
-    }
+    if (const int rc = tpa_recon_dense_qkv_f32(a, qd, kd, vd, a->sm_scale * kLog2e, stream); rc != TPA_OK) return rc;
+    p = dense_params_of(a, qd, kd, vd);
   }
   return launch_any(p, a->dk, stream);
 }

@@ -56,6 +56,22 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
     assert need <= lib.tpa_fwd_best_workspace_bytes(B, lq, lk, H, D, D, 6, rk)
 
 
+@pytest.mark.parametrize("name", ["qa", "qb", "ka", "kb", "va", "vb"])
+def test_rows_that_the_launch_refuses_ask_for_nothing(name):
+    """Rows of factors that start between 16 bytes, and more batch entries than the launch has room for: such a call runs on the factors."""
+    from tpa import _dispatch as d
+
+    lib = d.load_library()
+    fake = d.TpaFactor(256, 8, 8, 8)
+    factors = dict(qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake)
+    make = lambda B=1, **f: _forward_call(B=B, H=8, D=128, lq=300, lk=3000, rk=8, dtype=d.TPA_DTYPE_F32, **{**factors, **f})
+    room = lambda call: lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call))
+    assert room(make()) > 0
+    assert room(make(**{name: d.TpaFactor(256, 8, 9, 8)})) == 0
+    assert room(make(**{name: d.TpaFactor(260, 8, 8, 8)})) == 0
+    assert room(make(B=65536)) == 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["concatenated", "split", "ranks first"])
 @pytest.mark.parametrize("mask", ["none", "causal", "offset", "bottom right", "lengths", "packed", "ids in no order", "no common id"])
