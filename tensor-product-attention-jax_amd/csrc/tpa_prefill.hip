@@ -28,6 +28,7 @@
 // The dense flash baseline (tpa/mha.py:23-37) is the same kernel with a plain K/V loader.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1283,7 +1284,9 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
 // find compute units that have nothing to do: a tile of the rank-2 rebuild is 2.0 us (1.1 at D = 64), one of dense arrays 1.55 (0.65),
 // a second range 9.5 and its partial results.  140 rows over 1160 keys, us without / with: rank 2, 8 heads of 128 44.4 / 29.6, 2 x 32 heads of 128
 // 45.1 / 39.5, 8 heads of 64 25.7 / 21.9; rank 4, 8 heads of 128 35.6 / 26.7; 4 x 16 heads of 64 26.2 / 26.2 (one range), rank 4 29.7 / 31.3 (one).
-int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk, bool causal) {
+// (What counts there is the `reach` of the mask, not the length of the cache: 33 rows over 861 keys from the first one on, 2 x 16 heads of 64, rank 2:
+// eight ranges, all but one empty, 11.7, one 6.7.)
+int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk, bool causal, int64_t reach, bool dense) {
   const int64_t blocks = (lq + kBQ - 1) / kBQ, wgs = blocks * B * H;
   const double per_tile = D == 128 ? 1.7 : 1.3, per_wg = 7.0, most = (double)((lk + kTK - 1) / kTK);
   // tiles of an average block: under the causal mask the first one sees (lk - lq + 256) keys, the last one all
@@ -1291,10 +1294,11 @@ int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64
   int best = 1;
   if (most < 24) {  // a block's own tiles take 40 us at most: little to win over the merge, but where one block has them all
     if (blocks > 1) return 1;
-    const double tile = rk == 2 ? (D == 128 ? 2.0 : 1.1) : (D == 128 ? 1.55 : 0.65);
+    const double tile = rk == 2 && !dense ? (D == 128 ? 2.0 : 1.1) : (D == 128 ? 1.55 : 0.65);
+    const int64_t tiles = (reach + kTK - 1) / kTK;
     double gain = 1.5;
     for (int S = 2; S <= 8 && wgs * S <= 256; ++S) {
-      const double us = tile * (double)((int64_t)most - ((int64_t)most + S - 1) / S) - 9.5 - (double)S * B * lq * H * D * 8.0 / 4e6;
+      const double us = tile * (double)(tiles - (tiles + S - 1) / S) - 9.5 - (double)S * B * lq * H * D * 8.0 / 4e6;
       if (us > gain) { best = S; gain = us; }
     }
     return best;
@@ -1370,9 +1374,12 @@ namespace {
 // one, so that pairs beyond 256 add 0.7 of a round.  Fused / dense, us: rank 4, 1 x 250 rows, 8 heads of 64 17.3 / 12.1; 2 x 130 over 900, 32 heads of 128
 // 73.7 / 42.1; 12 x 200, 32 heads of 128 57.8 / 42.9; 8 x 200, 64 heads of 64 27.7 / 34.3 (stays fused); 4 x 40, 64 heads of 64 9.6 / 10.8 (stays);
 // rank 8, 1 x 130 over 900, 16 heads of 128 188 / 34; rank 1, 1 x 130 over 900, 8 heads of 64 31.2 / 20.2; 8 x 250, 32 heads of 128 22.6 / 32.2 (stays).
-bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
+// Of the keys, `made` are made dense and `met` are met by the rows: what the mask hides is neither, and a block of documents
+// meets about as many keys as it has rows, and two tiles.  47 rows over 882 keys from the first one on, 11 x 16 heads of 128, rank 3 10.4 / 14.1; 95 over
+// 867 in documents of 100, 4 x 64 heads of 64, rank 3 11.8 / 20.9 (both stay fused).
+bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk, int64_t made, int64_t met) {
   if (lk >= 1024 || H % 8 != 0) return false;  // beyond that the rule above has spoken; other head counts take three launches
-  const double pairs = (double)(B * H), tiles = (double)((lk + kTK - 1) / kTK), mb = pairs * (double)((lq + 2 * lk) * D) * 2e-6;
+  const double pairs = (double)(B * H), tiles = (double)((met + kTK - 1) / kTK), mb = pairs * (double)((lq + 2 * made) * D) * 2e-6;
   if (D == 64) return (pairs > 366 ? pairs / 366 : 1.0) * tiles * (0.55 + 0.36 * rk) > 4.5 + 0.28 * mb;
   return (double)((B * H + 255) / 256) * tiles * (0.55 + 0.57 * rk) > 2.0 + 0.21 * mb;
 }
@@ -1395,7 +1402,7 @@ bool one_block_of_rank_2_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int6
 //   more, of fewer rows: 512 rows 1.01 - 1.07, 700 to 900 0.81 - 0.99, with more keys than rows up to 1.32
 bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   if (tpa_prefill_wants_dense(lq, lk, rk)) return true;
-  if (rk != 2) return one_block_pays(B, lq, lk, H, D, rk);
+  if (rk != 2) return one_block_pays(B, lq, lk, H, D, rk, lk, lk);
   if (lq <= kBQ) return one_block_of_rank_2_pays(B, lq, lk, H, D);
   if (lk > 5 * lq) return false;
   const int64_t wgs = B * H * ((lq + kBQ - 1) / kBQ);
@@ -1406,7 +1413,7 @@ bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t
 
 size_t tpa_prefill_best_bytes(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   const size_t dense = tpa::dense_pays(B, lq, lk, H, D, rk) ? tpa_prefill_dense_bytes(B, lq, lk, H, D) : 0;
-  const int s0 = tpa::choose_splits(B, lq, lk, H, D, rk, false), s1 = tpa::choose_splits(B, lq, lk, H, D, rk, true);
+  const int s0 = tpa::choose_splits(B, lq, lk, H, D, rk, false, lk, false), s1 = tpa::choose_splits(B, lq, lk, H, D, rk, true, lk, false);
   return dense + tpa::split_bytes(B, lq, H, D, s0 > s1 ? s0 : s1);
 }
 
@@ -1419,12 +1426,27 @@ struct PrefillRoute {
   size_t dense;
   int S;
 };
-PrefillRoute route_of(const TpaFwdArgs* a) {
+// One block of rows is made dense for the time of one launch, so only where the factors allow that and the keys that this call's mask and
+// documents leave are enough.
+bool one_block_of_call_pays(const TpaFwdArgs* a) {
+  if (!tpa_recon_dense_qkv_takes(a)) return false;
+  if (a->rk == 2) return a->rq >= kSlowQ;
+  const int64_t made = keys_in_reach(a), met = a->kv_segment_ids ? std::min<int64_t>(made, ((int64_t)a->lq + 3 * kTK - 1) / kTK * kTK) : made;
+  return one_block_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk, made, met);
+}
+int splits_of_call(const TpaFwdArgs* a, bool dense) {
+  if (a->kv_segment_ids) return 1;
   const int tiles = (int)(((int64_t)a->lk + kTK - 1) / kTK);  // a caller's count beyond that only adds empty ranges
-  // one block of rows is made dense for the time of one launch, so only where the factors allow that
-  const bool pays = dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) && (tpa_prefill_wants_dense(a->lq, a->lk, a->rk) || (a->rk == 2 && a->lq > kBQ) || (tpa_recon_dense_qkv_takes(a) && (a->rk != 2 || a->rq >= kSlowQ)));
-  return {pays ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0,
-          a->kv_segment_ids ? 1 : a->num_splits > 0 ? (a->num_splits < tiles ? a->num_splits : tiles) : choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->rk, a->causal != 0)};
+  if (a->num_splits > 0) return std::min(a->num_splits, tiles);
+  const bool causal = a->causal != 0;
+  return std::min(choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->rk, causal, a->lk, false),  // of which the room by sizes alone takes account
+                  choose_splits(a->B, a->lq, a->lk, a->H, a->dk, a->rk, causal, keys_in_reach(a), dense));
+}
+PrefillRoute route_of(const TpaFwdArgs* a) {
+  const bool pays = dense_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rk) &&
+                    (tpa_prefill_wants_dense(a->lq, a->lk, a->rk) || (a->rk == 2 && a->lq > kBQ) || one_block_of_call_pays(a));
+  const size_t dense = pays ? tpa_prefill_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk) : 0;
+  return {dense, splits_of_call(a, dense != 0)};
 }
 
 }  // namespace

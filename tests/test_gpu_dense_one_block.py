@@ -42,6 +42,29 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
     assert lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call)) == 0
 
 
+@pytest.mark.parametrize(
+    "B,H,D,lq,lk,rk,mask,dense",
+    [
+        (11, 16, 128, 47, 882, 3, dict(), True),
+        (11, 16, 128, 47, 882, 3, dict(causal=1), False),                       # one tile in reach of 14
+        (11, 16, 128, 47, 882, 3, dict(causal=1, causal_offset=835), True),
+        (11, 16, 128, 47, 882, 3, dict(causal=1, causal_offset=-47), False),    # none
+        (4, 64, 64, 95, 867, 3, dict(), True),
+        (4, 64, 64, 95, 867, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),   # documents: four tiles met, 14 made
+        (1, 8, 64, 250, 900, 4, dict(q_segment_ids=256, kv_segment_ids=256), True),
+        (1, 16, 128, 33, 1100, 4, dict(causal=1), True),                        # as long as that the lengths decide
+    ],
+)
+def test_keys_that_no_row_meets_do_not_count(B, H, D, lq, lk, rk, mask, dense):
+    from tpa import _dispatch as d
+
+    lib = d.load_library()
+    fake = d.TpaFactor(256, 8, 8, 8)
+    call = _forward_call(B=B, H=H, D=D, lq=lq, lk=lk, rk=rk, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, num_splits=1, **mask)
+    slot = lambda n: (2 * n + 255) // 256 * 256
+    assert lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call)) == (slot(B * lq * H * D) + 2 * slot(B * lk * H * D) if dense else 0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["concatenated", "split", "ranks first", "head factors apart"])
 @pytest.mark.parametrize("mask", ["none", "causal", "offset", "bottom right", "lengths", "packed", "ids in no order", "no common id"])

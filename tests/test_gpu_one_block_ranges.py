@@ -38,6 +38,32 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, ranges):
     assert need[0] <= lib.tpa_fwd_best_workspace_bytes(B, lq, lk, H, D, D, 6, rk)
 
 
+@pytest.mark.parametrize(
+    "lq,lk,rk,mask,ranges",
+    [
+        (100, 1400, 2, dict(causal=1), 1),                        # two tiles are in reach
+        (100, 1400, 4, dict(causal=1), 1),
+        (100, 1400, 2, dict(causal=1, causal_offset=1300), 8),
+        (100, 1400, 2, dict(causal=1, causal_offset=700), 7),     # 13 tiles, two for each
+        (100, 1400, 2, dict(causal=1, causal_offset=-50), 1),
+        (100, 1400, 2, dict(causal=2), 8),
+        (100, 1400, 2, dict(), 8),
+        (64, 512, 2, dict(), 1),                                  # dense tiles, of which eight are not worth it
+    ],
+)
+def test_keys_behind_the_mask_ask_for_no_ranges(lq, lk, rk, mask, ranges):
+    from tpa import _dispatch as d
+
+    lib = d.load_library()
+    fake = d.TpaFactor(256, 8, 8, 8)
+    need = []
+    for splits in (0, 1):
+        call = _forward_call(B=1, H=8, D=128, lq=lq, lk=lk, rk=rk, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, num_splits=splits, **mask)
+        need.append(lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call)))
+    assert need[0] - need[1] == (ranges * lq * 8 * (128 + 2) * 4 if ranges > 1 else 0)
+    assert need[0] <= lib.tpa_fwd_best_workspace_bytes(1, lq, lk, 8, 128, 128, 6, rk)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mask", ["none", "top left", "bottom right", "lengths"])
 @pytest.mark.parametrize("b,h,d,lq,lk,rk", [(5, 1, 128, 140, 1160, 2), (5, 1, 64, 256, 900, 2), (2, 8, 128, 17, 520, 2), (1, 8, 128, 100, 1400, 4)])
