@@ -43,6 +43,29 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
 
 
 @pytest.mark.parametrize(
+    "B,H,D,lq,lk,rq,rk,dense",
+    [
+        (5, 32, 128, 125, 125, 6, 4, True),
+        (5, 32, 128, 125, 125, 5, 4, False),  # Q of few ranks is soon summed
+        (10, 8, 128, 217, 458, 6, 1, True),
+        (10, 8, 128, 217, 458, 2, 1, False),
+        (10, 8, 128, 217, 458, 2, 4, True),
+        (1, 8, 64, 250, 250, 2, 4, True),     # at head size 64 it does not matter
+        (1, 8, 128, 200, 600, 6, 2, True),
+        (1, 8, 128, 200, 600, 5, 2, False),
+    ],
+)
+def test_ranks_of_q(B, H, D, lq, lk, rq, rk, dense):
+    from tpa import _dispatch as d
+
+    lib = d.load_library()
+    fake = d.TpaFactor(256, 8, 8, 8)
+    call = _forward_call(B=B, H=H, D=D, lq=lq, lk=lk, rk=rk, rq=rq, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, num_splits=1)
+    slot = lambda n: (2 * n + 255) // 256 * 256
+    assert lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call)) == (slot(B * lq * H * D) + 2 * slot(B * lk * H * D) if dense else 0)
+
+
+@pytest.mark.parametrize(
     "B,H,D,lq,lk,rk,mask,dense",
     [
         (11, 16, 128, 47, 882, 3, dict(), True),
