@@ -56,6 +56,37 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
     assert need <= lib.tpa_fwd_best_workspace_bytes(B, lq, lk, H, D, D, 6, rk)
 
 
+@pytest.mark.parametrize(
+    "B,H,D,lq,lk,rq,rk,call,dense",
+    [
+        (4, 16, 128, 100, 100, 6, 3, dict(causal=1), False),    # 32 rows: one step of four waves
+        (4, 16, 128, 100, 100, 6, 8, dict(causal=1), True),
+        (2, 16, 128, 200, 200, 6, 4, dict(causal=1), True),     # two
+        (12, 32, 128, 40, 40, 2, 3, dict(causal=1), False),     # 256 rows, Q of two ranks
+        (12, 32, 128, 40, 40, 16, 3, dict(causal=1), True),
+        (2, 64, 64, 307, 307, 2, 4, dict(), False),
+        (2, 64, 64, 307, 307, 16, 4, dict(), True),
+        (4, 32, 128, 135, 135, 2, 3, dict(), False),            # 128 rows
+        (4, 32, 128, 135, 135, 16, 3, dict(), True),
+        (4, 32, 128, 256, 1000, 2, 3, dict(causal=2), True),
+        (4, 32, 128, 256, 1000, 2, 3, dict(causal=1), False),   # a quarter of the keys in reach
+        (1, 16, 128, 40, 1500, 6, 3, dict(causal=1), False),    # the same of 32 rows
+        (1, 16, 128, 40, 1500, 6, 3, dict(causal=1, causal_offset=1460), True),
+        (1, 16, 128, 40, 1500, 6, 3, dict(causal=1, causal_offset=-40), False),
+        (45, 40, 128, 100, 317, 4, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),  # documents: 228 of 317 keys
+        (1, 8, 128, 65537, 65537, 6, 3, dict(causal=1), True),  # more blocks than are looked at
+    ],
+)
+def test_calls_that_would_not_win_by_it(B, H, D, lq, lk, rq, rk, call, dense):
+    from tpa import _dispatch as d
+
+    lib = d.load_library()
+    fake = d.TpaFactor(256, 8, 8, 8)
+    call = _forward_call(B=B, H=H, D=D, lq=lq, lk=lk, rq=rq, rk=rk, dtype=d.TPA_DTYPE_F32, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, **call)
+    slot = lambda n: (n + 63) // 64 * 256
+    assert lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call)) == (slot(B * lq * H * D) + 2 * slot(B * lk * H * D) if dense else 0)
+
+
 @pytest.mark.parametrize("name", ["qa", "qb", "ka", "kb", "va", "vb"])
 def test_rows_that_the_launch_refuses_ask_for_nothing(name):
     """Rows of factors that start between 16 bytes, and more batch entries than the launch has room for: such a call runs on the factors."""
