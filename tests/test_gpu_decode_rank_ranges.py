@@ -27,10 +27,15 @@ def _call(b, lq, lk, h, d, rk, bf16=True, splits=0):
         (1, 1, 705, 16, 128, 8, True, 45),
         (1, 1, 700, 16, 128, 4, True, 22),
         (1, 1, 700, 16, 128, 2, True, 11),    # as by the sizes alone
-        (1, 1, 700, 64, 64, 4, True, 11),     # short blocks
+        (1, 1, 700, 64, 64, 4, True, 22),     # one set of columns
         (1, 2, 700, 64, 64, 4, True, 22),     # two sets of columns
         (1, 1, 700, 64, 64, 8, True, 44),
         (1, 1, 700, 16, 64, 4, False, 22),
+        (1, 1, 2016, 16, 64, 4, True, 63),    # as many as that pays for, in blocks of eight keys
+        (1, 1, 2500, 16, 64, 4, True, 64),
+        (1, 2, 8000, 32, 64, 4, True, 125),   # by the sizes alone
+        (1, 1, 7724, 8, 64, 8, True, 128),
+        (1, 1, 7724, 8, 64, 8, False, 256),
         (4, 1, 9000, 32, 128, 8, True, 64),   # a workgroup per compute unit
         (300, 1, 9000, 32, 128, 8, True, 1),
         (1, 1, 100000, 128, 128, 32, True, 64),
@@ -47,6 +52,20 @@ def test_room_for_a_block_per_wave(b, lq, lk, h, d, rk, bf16, ranges):
     assert lib.tpa_decode_call_workspace_bytes(ctypes.byref(_call(b, lq, lk, h, d, rk, bf16, 3))) == lib.tpa_decode_workspace_bytes(b, lq, lk, h, d, 3)
     if lq <= 16 and lk >= 1024:
         assert need <= lib.tpa_fwd_best_workspace_bytes(b, lq, lk, h, d, d, 6, rk)
+
+
+@pytest.mark.parametrize("b,lq,lk,h,d,rk,bf16,ranges", [(2, 4, 1519, 64, 64, 4, True, 24), (2, 4, 1519, 64, 128, 4, True, 31), (2, 4, 1519, 64, 64, 8, True, 31),
+                                                        (2, 4, 1519, 64, 64, 4, False, 24), (65, 1, 1519, 32, 64, 4, True, 4)])
+def test_room_where_the_ranges_are_dealt_by_the_lengths(b, lq, lk, h, d, rk, bf16, ranges):
+    """bf16, head size 64, rank 4: two blocks per wave, as by the sizes alone; the others as without lengths, within the fixed array."""
+    from tpa import _dispatch as disp
+
+    lib = disp.load_library()
+    call = _call(b, lq, lk, h, d, rk, bf16)
+    call.kv_lengths = 256
+    need = lib.tpa_decode_call_workspace_bytes(ctypes.byref(call))
+    assert need == b * lq * h * (d + 2) * 4 * ranges
+    assert lib.tpa_decode_workspace_bytes(b, lq, lk, h, d, 0) <= need <= lib.tpa_fwd_best_workspace_bytes(b, lq, lk, h, d, d, 6, rk)
 
 
 @pytest.mark.gpu
