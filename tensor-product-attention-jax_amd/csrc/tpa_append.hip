@@ -783,12 +783,14 @@ int rows_cost(const AppendParams& p, int mb) {
 // Blocks of 16 tokens per workgroup if the few-token kernel serves the call, 0 if the tiles do, whose time is nearly the same from
 // one tile to 100: 12 us at d_model 4096.  us of this kernel / 64 x 64 tiles by cost: d_model 4096, 160 tokens x 720 columns (cost 64)
 // 8.3 / 12.2, 128 x 1600 (96) 10.8 / 11.9, 80 x 2240 (128) 13.7 / 12.3, 160 x 1440 (128) 14.0 / 12.0, 128 x 2560 (192) 19.6 / 11.9; 2048, 128 x 1600
-// 7.7 / 8.7, 32 x 5120 (128) 11.0 / 8.4; 8192, 128 x 1600 17.2 / 24.4, 146 x 1440 (128) 20.6 / 25.8, 192 x 1600 (192) 30.5 / 24.5.
+// 7.7 / 8.7, 32 x 5120 (128) 11.0 / 8.4; 8192, 128 x 1600 17.2 / 24.4, 146 x 1440 (128) 20.6 / 25.8, 192 x 1600 (192) 30.5 / 24.5.  Cost 128 changes
+// sides between 4096 and 5120, where 150 x 1440 takes 15.1 / 17.1 (6144 17.6 / 21.0, 7168 19.4 / 22.8; 3072, 88 x 2560 11.4 / 9.9); from 2048 down to 256
+// it is 0.2 - 0.6 slower here, cost 96 between 1.3 faster and the same.
 int few_tokens(const AppendParams& p) {
   int mb = 4;
   for (int n : {2, 1})
     if (rows_cost(p, n) < rows_cost(p, mb)) mb = n;
-  return rows_cost(p, mb) <= (p.K >= 8192 ? 128 : 96) ? mb : 0;
+  return rows_cost(p, mb) <= (p.K >= 5120 ? 128 : 96) ? mb : 0;
 }
 
 template <int MB>

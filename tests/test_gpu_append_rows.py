@@ -33,6 +33,19 @@ def test_append_few_tokens(gpu, b, n, dm, h, d, rq, rk):
     check_append(gpu, torch.bfloat16, 2, b, n, dm, h, d, rq, rk, False)
 
 
+@pytest.mark.parametrize(
+    "b,n,dm,h,d,rq,rk",
+    [
+        (2, 75, 5120, 16, 128, 6, 2),  # two rounds of blocks of 32: from here on they are the faster side
+        (2, 75, 5056, 16, 128, 6, 2),  # and below tiles of 64 x 64
+        (2, 80, 4096, 8, 64, 6, 2),    # one round
+        (3, 64, 5120, 32, 128, 6, 2),  # three rounds: tiles
+    ],
+)
+def test_append_at_the_line_to_the_tiles(gpu, b, n, dm, h, d, rq, rk):
+    check_append(gpu, torch.bfloat16, 2, b, n, dm, h, d, rq, rk, False)
+
+
 def test_results_are_the_roundings_of_exact_sums(gpu):
     """Results of a long contraction that are not the bf16 rounding of the exact sum.  An fp32 sum that is off by e rounds to the
     wrong side for a share of about 2 e / spacing of the results; with the chunks of 64 summed one by one that is 1.7e-4 here, with one
