@@ -752,6 +752,9 @@ bool projects_by_h8(const ProjectJob& j, int H) {
 // to hide, so there they are dealt to workgroups of their own, which read dx again, as long as these are no more than 400.  us, all ranks / so,
 // by workgroups of one array: ranks 16, 8, 8: 11 of them (335 tokens, 8 heads of 64) 14.9 / 6.5, 63 17.1 / 12.5 (four ranks each, 504 workgroups
 // 11.7), 99 19.0 / 15.8 (four each 19.0), 250 23.4 / 25.8; 6, 2, 2: 34 7.2 / 5.3, 54 7.8 / 7.2, fp32 64 8.6 / 7.0; 6, 4, 4: 175 13.1 / 13.5.
+// What they read again has to be little against the links of the chain that they save, 25 workgroups for each.  Whole backward: ranks 6, 4, 4, 3 x 156
+// tokens, 32 heads of 64 29.9 / 34.2 in parts of two; 4, 3, 3, 208 tokens, 64 heads 26.8 / 32.3, 3 x 264, 16 heads 30.8 / 34.1 (all ranks again, in 207
+// calls that were dealt 19 were slower for it by more than 2 %, now 3).
 int ranks_per_workgroup(const ProjectJobs& jobs, unsigned n, int64_t blocks) {
   int most = 0;
   for (unsigned i = 0; i < n; ++i) most = std::max(most, jobs.job[i].R);
@@ -759,7 +762,7 @@ int ranks_per_workgroup(const ProjectJobs& jobs, unsigned n, int64_t blocks) {
     const int ranks = (most + k - 1) / k;
     int64_t parts = 0;
     for (unsigned i = 0; i < n; ++i) parts += (jobs.job[i].R + ranks - 1) / ranks;
-    if (blocks * parts <= 400) return ranks;
+    if (blocks * parts <= 400 && blocks * (parts - n) <= 25 * (most - ranks)) return ranks;
   }
   return most;
 }
