@@ -1494,13 +1494,14 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
     uint16_t* vd = kd + kv_slot / 2;
     uint16_t* qd = vd + kv_slot / 2;
     WindowJob windows{};
-    if (p.kvseg) {
+    const bool ahead = p.kvseg && windows_ahead_pay(a->H, a->lq, a->lk);
+    if (ahead) {
       const int rows = a->dk == 64 && wants_four_waves(p, true) ? kBQ / 2 : kBQ;  // as launch_prefill has it
       windows = WindowJob{p.qseg, p.kvseg, p.kvlen, a->lq, a->lk, rows, 0, a->causal, p.coff, reinterpret_cast<int32_t*>(p.o),
                           a->lq * hd / 2, rows * hd / 2, a->dk / 2, a->H};
     }
     int rc = tpa_recon_dense_qkv_bf16(a, qd, kd, vd, a->sm_scale * kLog2e, windows, stream);
-    p.windows = p.kvseg && rc == TPA_OK;
+    p.windows = ahead && rc == TPA_OK;
     if (rc == TPA_ERR_UNSUPPORTED) {
       rc = tpa_recon_dense_bf16(&a->ka, &a->kb, kd, a->B, a->lk, a->H, a->dk, a->rk, 1.f, stream);
       if (rc == TPA_OK) rc = tpa_recon_dense_bf16(&a->va, &a->vb, vd, a->B, a->lk, a->H, a->dv, a->rk, 1.f, stream);
