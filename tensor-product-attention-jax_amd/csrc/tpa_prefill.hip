@@ -113,10 +113,10 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int V>
 using IC = std::integral_constant<int, V>;
 
-// Batch entries by their lengths, longest first (equal ones in their order): lane = batch entry, B <= 64.  A launch of several workgroups
+// Batch entries by their lengths, longest first (equal ones in their order): lane = batch entry, B <= 64 (kMostOrdered are worth it).  A launch of several workgroups
 // per compute unit ends with the last of them, so the long ones start first; every workgroup works the order out, as the lengths are known on the
 // device only.
-constexpr int kMostOrdered = 64;
+constexpr int kMostOrdered = 32;
 struct LongestFirst {
   int len, B;
   __device__ __forceinline__ LongestFirst(const int32_t* kvlen, int B, int lk) : B(B) {
@@ -1231,9 +1231,14 @@ inline bool wants_four_waves(const PrefillParams& p, bool dense) {
 // 525), 4 x 1024 451 / 405 (506 / 508), 4 x 512, 64 heads of 64 272 / 233 (329 / 326), 8 x 300 over 4000 254 / 226 (282 / 285); rank 4, dense tiles: 16 x
 // 300 over 4000, 32 heads of 128 648 / 628 (732 / 734).  Ranges do not count as rounds: 7 x 1000 over 9000, 8 heads of 128, 224 blocks in two
 // each 241 / 249.  Dense tiles of an XCD belong to a head of every entry anyway; they gain with up to two blocks of rows, and with four 8 x 1024
-// over 4096, 32 heads of 128 take 470 / 474 (551 / 564).  (The grid covers eight groups of heads as well: they are npairs * H workgroups.)
+// over 4096, 32 heads of 128 take 470 / 474 (551 / 564).
+// The order costs every workgroup the lengths and their comparison before its first load, which short walks do not get back, nor those of many
+// entries, whose lengths level out by themselves: 44 x 47 rows over 113, 16 heads of 64, rank 4 24.9 / 34.4; 48 x 27 over 200, 64 heads 72 / 88; 25 x 103 over 406, 32
+// heads of 128 87 / 95; 40 x 633 over 1808, 8 heads of 64 106 / 122; 33 x 159 over 2036 96 / 103.  Up to 32 entries over 2048 keys and more: mean of 88 shapes, half to
+// all of the cache, 0.95 (fused) and 0.96 (dense) of the time without the order, 0.83 - 1.05; all lengths equal 0.99 and 1.00 (67 shapes, 0.94 - 1.03).  Shorter
+// caches 1.015 fused and 0.99 dense, more entries 1.07 and 1.00.  (The grid covers eight groups of heads as well: they are npairs * H workgroups.)
 bool longest_first_pays(const PrefillParams& p, bool dense) {
-  return p.kvlen && (!dense || p.lq <= 2 * kBQ) && p.B > 1 && p.B <= kMostOrdered && p.H % 8 == 0 && p.lk >= 2 * (int64_t)p.lq && (int64_t)p.npairs * p.H >= 384 * p.S;
+  return p.kvlen && (!dense || p.lq <= 2 * kBQ) && p.B > 1 && p.B <= kMostOrdered && p.H % 8 == 0 && p.lk >= std::max<int64_t>(2048, 2 * (int64_t)p.lq) && (int64_t)p.npairs * p.H >= 384 * p.S;
 }
 
 template <int D, int LOADER, bool SEG = false, bool SPLIT = false, int NW = 8, bool ORDER = false>

@@ -10,14 +10,23 @@ import torch
 @pytest.mark.parametrize(
     "b,h,d,lq,lk,rk,lengths",
     [
-        (4, 48, 64, 300, 700, 2, [300, 64, 700, 600]),             # 384 workgroups, the fewest; two blocks
-        (3, 64, 128, 300, 700, 2, [0, 700, 1]),                    # no key, one key
-        (7, 32, 128, 260, 900, 2, [800, 900, 790, 900, 900, 800, 801]),  # alike: the order of equal lengths
-        (5, 32, 64, 513, 1100, 2, [300, 1100, 300, 900, 1100]),    # equal ones among them, three blocks
-        (6, 40, 128, 260, 600, 4, [65, 600, 300, 0, 600, 1]),      # dense tiles
-        (6, 32, 128, 300, 4000, 2, [1500, 4000, 64, 0, 3000, 3001]),  # the keys in ranges
-        (64, 8, 64, 17, 200, 2, [3 * i + 1 for i in range(64)]),   # as many as are ordered
-        (65, 8, 64, 17, 200, 8, [3 * i + 1 for i in range(65)]),   # and one more
+        (4, 48, 64, 300, 700, 2, [300, 64, 700, 600]),             # too short to be ordered
+        (3, 64, 128, 300, 700, 2, [0, 700, 1]),
+        (7, 32, 128, 260, 900, 2, [800, 900, 790, 900, 900, 800, 801]),
+        (5, 32, 64, 513, 1100, 2, [300, 1100, 300, 900, 1100]),
+        (6, 40, 128, 260, 600, 4, [65, 600, 300, 0, 600, 1]),
+        (6, 32, 128, 300, 4000, 2, [1500, 4000, 64, 0, 3000, 3001]),  # the fewest workgroups, the keys in ranges
+        (64, 8, 64, 17, 200, 2, [3 * i + 1 for i in range(64)]),
+        (65, 8, 64, 17, 200, 8, [3 * i + 1 for i in range(65)]),
+        (4, 48, 64, 300, 2047, 2, [300, 64, 2047, 1600]),          # one key below the line, and at it
+        (4, 48, 64, 300, 2048, 2, [300, 64, 2048, 1600]),
+        (3, 64, 128, 300, 2100, 2, [0, 2100, 1]),                  # no key, one key
+        (7, 32, 128, 260, 2200, 2, [2000, 2200, 1990, 2200, 2200, 2000, 2001]),  # alike: the order of equal lengths
+        (5, 32, 64, 513, 2300, 2, [300, 2300, 300, 1900, 2300]),   # equal ones among them, three blocks
+        (6, 40, 128, 260, 2600, 4, [65, 2600, 300, 0, 2600, 1]),   # dense tiles
+        (7, 64, 64, 260, 2500, 8, [65, 2500, 300, 0, 2500, 1, 64]),
+        (32, 16, 64, 17, 2100, 2, [65 * i + 1 for i in range(32)]),  # as many as are ordered
+        (33, 16, 64, 17, 2100, 2, [65 * i + 1 for i in range(33)]),  # and one more
     ],
 )
 def test_entries_are_what_they_are_alone(gpu, b, h, d, lq, lk, rk, lengths, causal):
