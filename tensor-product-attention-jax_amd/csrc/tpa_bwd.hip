@@ -752,9 +752,10 @@ bool projects_by_h8(const ProjectJob& j, int H) {
 // to hide, so there they are dealt to workgroups of their own, which read dx again, as long as these are no more than 400.  us, all ranks / so,
 // by workgroups of one array: ranks 16, 8, 8: 11 of them (335 tokens, 8 heads of 64) 14.9 / 6.5, 63 17.1 / 12.5 (four ranks each, 504 workgroups
 // 11.7), 99 19.0 / 15.8 (four each 19.0), 250 23.4 / 25.8; 6, 2, 2: 34 7.2 / 5.3, 54 7.8 / 7.2, fp32 64 8.6 / 7.0; 6, 4, 4: 175 13.1 / 13.5.
-// What they read again has to be little against the links of the chain that they save, 25 workgroups for each.  Whole backward: ranks 6, 4, 4, 3 x 156
-// tokens, 32 heads of 64 29.9 / 34.2 in parts of two; 4, 3, 3, 208 tokens, 64 heads 26.8 / 32.3, 3 x 264, 16 heads 30.8 / 34.1 (all ranks again, in 207
-// calls that were dealt 19 were slower for it by more than 2 %, now 3).
+// That holds where the parts of a token find its dx in the L2 of their XCD: workgroups go to the XCDs in turn, so a part has a multiple of eight of them (the
+// last ones past every array).  Without that, whole backward, all ranks / parts of two: ranks 6, 4, 4, 3 x 156 tokens, 32 heads of 64 (60 workgroups)
+// 29.9 / 34.2, 2 x 218 (56) 30.4 / 28.1; 4, 3, 3, 208 tokens, 64 heads (52) 26.8 / 32.3, 2 x 112 (56) 27.0 / 26.0; 6, 2, 2, 3 x 130, 64 heads (99) 31.5 /
+// 32.3, 16 x 164, 8 heads (96) 29.6 / 27.4.
 int ranks_per_workgroup(const ProjectJobs& jobs, unsigned n, int64_t blocks) {
   int most = 0;
   for (unsigned i = 0; i < n; ++i) most = std::max(most, jobs.job[i].R);
@@ -762,7 +763,7 @@ int ranks_per_workgroup(const ProjectJobs& jobs, unsigned n, int64_t blocks) {
     const int ranks = (most + k - 1) / k;
     int64_t parts = 0;
     for (unsigned i = 0; i < n; ++i) parts += (jobs.job[i].R + ranks - 1) / ranks;
-    if (blocks * parts <= 400 && blocks * (parts - n) <= 25 * (most - ranks)) return ranks;
+    if (blocks * parts <= 400) return ranks;
   }
   return most;
 }
@@ -795,6 +796,7 @@ void launch_project(const ProjectJobs& jobs, int B, int H, hipStream_t stream) {
     h8.first[i] = i < n ? (int)parts : INT32_MAX;
     if (i < n) parts += (h8.job[i].R + h8.ranks - 1) / h8.ranks;
   }
+  if (parts > n) blocks = (blocks + 7) / 8 * 8;
   hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, parts), dim3(256), 0, stream, h8, H);
 }
 

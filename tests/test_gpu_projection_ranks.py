@@ -25,9 +25,9 @@ pytestmark = pytest.mark.gpu
         (1, 700, 300, 16, 64, 16, 8),  # 400 workgroups or fewer only with eight ranks each
         (1, 1600, 1600, 8, 64, 16, 8),
         (1, 96, 64, 8, 256, 5, 2),    # the other kernel
-        (1, 400, 400, 16, 64, 6, 4),  # two ranks each, 25 workgroups more for every one saved
-        (1, 416, 400, 16, 64, 6, 4),  # one more: all of them
-        (1, 400, 401, 16, 64, 4, 3),
+        (1, 400, 400, 16, 64, 6, 4),  # two ranks each, 25 workgroups in 32
+        (3, 300, 17, 16, 64, 6, 4),   # 19 in 24, one of them with keys
+        (1, 512, 400, 8, 128, 4, 3),  # 32
     ],
 )
 def test_gradients_of_every_rank(gpu, dt, tol, b, lq, lk, h, d, rq, rk):
