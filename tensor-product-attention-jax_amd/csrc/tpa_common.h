@@ -178,10 +178,11 @@ __device__ __forceinline__ void id_window(const int32_t* mine, int n_mine, const
 // attention kernels / here: training step of 3 x 1777 tokens, 16 heads of 64, documents of 421 115.5 / 110.3; 2 x 13 505 of 284 527 /
 // 492; 14 x 569 of 129, rank 8 157.5 / 153.3; 1 x 20 000, 32 heads of 128, of 1000 1806 / 1743; forward alone 2 x 13 505 124 / 113, 14 x 569
 // 42.2 / 38.8, 5 x 9865, 16 heads of 128, of 477 472 / 458.
-// Of short calls of few heads the attention kernels find them in less time than that launch takes longer: us, here / by them, 1 x 58 tokens, 8 heads of
-// 64, backward 16.6 / 15.7, 2 x 323 25.8 / 24.9, 7 x 179, rank 4, forward 13.9 / 13.2; 16 heads, 1 x 130, backward 22.2 / 21.3.  By tokens times
-// heads, mean over 470 shapes: below 2048 0.98 forward and 0.975 backward of the time without, to 4096 1.01 and 0.995, from there on 1.01 - 1.09.
-inline bool windows_ahead_pay(int H, int lq, int lk) { return (int64_t)H * (lq > lk ? lq : lk) >= 4096; }
+// In short calls of few heads the attention kernels find them in less time than that launch takes longer: us, here / by them, 1 x 58 tokens, 8 heads of
+// 64, backward 16.6 / 15.7, 2 x 323 25.8 / 24.9; 1 x 82, rank 8, forward 11.9 / 11.5.  By (batch, head) pairs times tokens, mean of the time by them over the
+// time here, 700 shapes: forward to 2048 0.98, to 4096 0.99, to 8192 1.02, to 65 536 1.016, beyond 1.05; backward to 4096 0.975, to 8192 0.99, to 16 384
+// 1.01, to 65 536 1.02, beyond 1.03.  `least`: of the forward's and of the backward's.
+inline bool windows_ahead_pay(int B, int H, int lq, int lk, int64_t least) { return (int64_t)B * H * (lq > lk ? lq : lk) >= least; }
 struct IdWindow { int32_t first, last, count, least, most; };  // what id_window finds
 struct WindowJob {
   const int32_t *mine, *other;  // ids [B, n_mine], [B, n_other]; mine = null: no such job

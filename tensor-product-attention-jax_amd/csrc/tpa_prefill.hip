@@ -1499,7 +1499,7 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
     uint16_t* vd = kd + kv_slot / 2;
     uint16_t* qd = vd + kv_slot / 2;
     WindowJob windows{};
-    const bool ahead = p.kvseg && windows_ahead_pay(a->H, a->lq, a->lk);
+    const bool ahead = p.kvseg && windows_ahead_pay(a->B, a->H, a->lq, a->lk, 4096);
     if (ahead) {
       const int rows = a->dk == 64 && wants_four_waves(p, true) ? kBQ / 2 : kBQ;  // as launch_prefill has it
       windows = WindowJob{p.qseg, p.kvseg, p.kvlen, a->lq, a->lk, rows, 0, a->causal, p.coff, reinterpret_cast<int32_t*>(p.o),
