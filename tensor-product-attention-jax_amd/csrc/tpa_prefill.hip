@@ -1379,23 +1379,34 @@ namespace {
 // one, so that pairs beyond 256 add 0.7 of a round.  Fused / dense, us: rank 4, 1 x 250 rows, 8 heads of 64 17.3 / 12.1; 2 x 130 over 900, 32 heads of 128
 // 73.7 / 42.1; 12 x 200, 32 heads of 128 57.8 / 42.9; 8 x 200, 64 heads of 64 27.7 / 34.3 (stays fused); 4 x 40, 64 heads of 64 9.6 / 10.8 (stays);
 // rank 8, 1 x 130 over 900, 16 heads of 128 188 / 34; rank 1, 1 x 130 over 900, 8 heads of 64 31.2 / 20.2; 8 x 250, 32 heads of 128 22.6 / 32.2 (stays).
-// Of the keys, `made` are made dense and `met` are met by the rows: what the mask hides is neither, and a block of documents
-// meets about as many keys as it has rows, and two tiles.  47 rows over 882 keys from the first one on, 11 x 16 heads of 128, rank 3 10.4 / 14.1; 95 over
-// 867 in documents of 100, 4 x 64 heads of 64, rank 3 11.8 / 20.9 (both stay fused).
-// At head size 128 the fused kernel sums Q rank by rank through LDS, and of fewer ranks than those shapes had (six) it takes less of its time: rank 2 of Q, 5 x
-// 32 heads, 125 x 125, rank 4 16.2 / 19.7; 10 x 8 heads, 217 x 458, rank 1 26.3 / 31.9; 7 x 40, 128 x 128, rank 4 28.9 / 32.6.  (Of 1100 further shapes
-// with 2 to 16 ranks of Q the lines took 48 to the slower side by more than 2 %, and take 9 now.)
-constexpr int kSlowQ = 6;
-bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rq, int64_t rk, int64_t made, int64_t met) {
+bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   if (lk >= 1024 || H % 8 != 0) return false;  // beyond that the rule above has spoken; other head counts take three launches
-  const double pairs = (double)(B * H), tiles = (double)((met + kTK - 1) / kTK), mb = pairs * (double)((lq + 2 * made) * D) * 2e-6;
+  const double pairs = (double)(B * H), tiles = (double)((lk + kTK - 1) / kTK), mb = pairs * (double)((lq + 2 * lk) * D) * 2e-6;
   if (D == 64) return (pairs > 366 ? pairs / 366 : 1.0) * tiles * (0.55 + 0.36 * rk) > 4.5 + 0.28 * mb;
-  return (double)((B * H + 255) / 256) * tiles * (0.55 + 0.57 * rk) > (rq < kSlowQ ? 4.5 : 2.0) + 0.21 * mb;
+  return (double)((B * H + 255) / 256) * tiles * (0.55 + 0.57 * rk) > 2.0 + 0.21 * mb;
+}
+// The same for one call, whose mask and ranks of Q are known, in us.  What the mask hides is neither made dense nor met, and a block of documents meets about
+// as many keys as it has rows, and two tiles; the fused kernel sums Q rank by rank, which the dense launch does in passing.  Fitted to 1400 shapes of 17 to 256
+// rows, ranks 1 to 8 (1, 2, 4, 6, 16 of Q), within 1.1 us for the half of them.  The line above alone took 48 of 917 to the slower side by more than 2 %,
+// with this 15, at the same gain over all (1.24).  Fused / dense: 47 rows over 882 keys from the first one on, 11 x 16 heads of 128, ranks 2, 3 10.4 / 14.1; 95 over
+// 867 in documents of 100, 4 x 64 heads of 64, 2, 3 11.8 / 20.9; 227 x 227, 2 x 32 of 128, 2, 1 14.6 / 18.3; 102 x 172, 9 x 16, 2, 3 18.4 / 21.5 (all stay
+// fused); 59 over 127 from the first on, 2 x 32 of 128, 16, 3 24.1 / 12.8; 79 x 79, 4 x 8, 4, 3 15.5 / 12.0.
+double one_block_saves_us(const TpaFwdArgs* a) {
+  const int64_t pairs = (int64_t)a->B * a->H, made = keys_in_reach(a);
+  if (!made) return 0.0;  // the rows end before Q is needed
+  const int64_t tiles = ((a->kv_segment_ids ? std::min<int64_t>(made, a->lq + 2 * kTK) : made) + kTK - 1) / kTK;
+  const double mb = (double)(pairs * (a->lq + 2 * made) * a->dk) * 2e-6;
+  if (a->dk == 64) {
+    const double rounds = pairs > 366 ? (double)pairs / 366 : 1.0;
+    return rounds * ((double)tiles * (0.21 + 0.30 * a->rk) + 0.41 * a->rq) - 2.9 - 0.13 * mb;
+  }
+  return (double)((pairs + 255) / 256) * ((double)tiles * (0.12 + 0.54 * a->rk) + 0.86 * a->rq) - 3.5 - 0.22 * mb;
 }
 // Rank 2 at head size 128: the fused kernel's Q, summed rank by rank through LDS, takes longer than the launch that makes dense arrays, as long as
 // these are few.  us, fused / dense, rank 6 of Q, by (batch, head) pairs: 8, 64 rows over 64 keys 14.2 / 10.4, 200 x 600 25.9 / 22.9; 32, 200 x 200 20.6 /
 // 17.7, 200 x 600 31.1 / 28.8, 40 x 900 26.9 / 28.8; 64, 130 x 130 18.6 / 16.6, 250 x 250 21.1 / 21.2; 128, 64 x 64 14.4 / 13.1, 130 x 130 18.7 / 19.5.
 // (16, 250 x 1000 31.8 / 31.7: from twelve tiles on the walk counts, not Q.  Head size 64: 0.82 - 1.15 with no such line.)
+constexpr int kSlowQ = 6;  // ranks of Q from which that holds
 bool one_block_of_rank_2_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D) {
   return D == 128 && H % 8 == 0 && lq <= kBQ && lk <= 12 * kTK && B * H * (lq + 2 * lk) <= 40000;
 }
@@ -1410,7 +1421,7 @@ bool one_block_of_rank_2_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int6
 //   more, of fewer rows: 512 rows 1.01 - 1.07, 700 to 900 0.81 - 0.99, with more keys than rows up to 1.32
 bool dense_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk) {
   if (tpa_prefill_wants_dense(lq, lk, rk)) return true;
-  if (rk != 2) return one_block_pays(B, lq, lk, H, D, kSlowQ, rk, lk, lk);  // (of any rank of Q)
+  if (rk != 2) return one_block_pays(B, lq, lk, H, D, rk);
   if (lq <= kBQ) return one_block_of_rank_2_pays(B, lq, lk, H, D);
   if (lk > 5 * lq) return false;
   const int64_t wgs = B * H * ((lq + kBQ - 1) / kBQ);
@@ -1434,13 +1445,9 @@ struct PrefillRoute {
   size_t dense;
   int S;
 };
-// One block of rows is made dense for the time of one launch, so only where the factors allow that and the keys that this call's mask and
-// documents leave are enough.
+// One block of rows is made dense for the time of one launch, so only where the factors allow that and this very call saves by it.
 bool one_block_of_call_pays(const TpaFwdArgs* a) {
-  if (!tpa_recon_dense_qkv_takes(a)) return false;
-  if (a->rk == 2) return a->rq >= kSlowQ;
-  const int64_t made = keys_in_reach(a), met = a->kv_segment_ids ? std::min<int64_t>(made, ((int64_t)a->lq + 3 * kTK - 1) / kTK * kTK) : made;
-  return one_block_pays(a->B, a->lq, a->lk, a->H, a->dk, a->rq, a->rk, made, met);
+  return tpa_recon_dense_qkv_takes(a) && (a->rk == 2 ? a->rq >= kSlowQ : one_block_saves_us(a) > 0.5);
 }
 int splits_of_call(const TpaFwdArgs* a, bool dense) {
   if (a->kv_segment_ids) return 1;

@@ -46,11 +46,12 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
     "B,H,D,lq,lk,rq,rk,dense",
     [
         (5, 32, 128, 125, 125, 6, 4, True),
-        (5, 32, 128, 125, 125, 5, 4, False),  # Q of few ranks is soon summed
+        (5, 32, 128, 125, 125, 2, 4, False),  # Q of few ranks is soon summed
         (10, 8, 128, 217, 458, 6, 1, True),
         (10, 8, 128, 217, 458, 2, 1, False),
         (10, 8, 128, 217, 458, 2, 4, True),
-        (1, 8, 64, 250, 250, 2, 4, True),     # at head size 64 it does not matter
+        (4, 8, 128, 79, 79, 4, 3, True),
+        (1, 8, 64, 250, 250, 2, 4, True),
         (1, 8, 128, 200, 600, 6, 2, True),
         (1, 8, 128, 200, 600, 5, 2, False),
     ],
@@ -66,24 +67,25 @@ def test_ranks_of_q(B, H, D, lq, lk, rq, rk, dense):
 
 
 @pytest.mark.parametrize(
-    "B,H,D,lq,lk,rk,mask,dense",
+    "B,H,D,lq,lk,rq,rk,mask,dense",
     [
-        (11, 16, 128, 47, 882, 3, dict(), True),
-        (11, 16, 128, 47, 882, 3, dict(causal=1), False),                       # one tile in reach of 14
-        (11, 16, 128, 47, 882, 3, dict(causal=1, causal_offset=835), True),
-        (11, 16, 128, 47, 882, 3, dict(causal=1, causal_offset=-47), False),    # none
-        (4, 64, 64, 95, 867, 3, dict(), True),
-        (4, 64, 64, 95, 867, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),   # documents: four tiles met, 14 made
-        (1, 8, 64, 250, 900, 4, dict(q_segment_ids=256, kv_segment_ids=256), True),
-        (1, 16, 128, 33, 1100, 4, dict(causal=1), True),                        # as long as that the lengths decide
+        (11, 16, 128, 47, 882, 2, 3, dict(), True),
+        (11, 16, 128, 47, 882, 2, 3, dict(causal=1), False),                       # one tile in reach of 14
+        (11, 16, 128, 47, 882, 16, 3, dict(causal=1), True),                       # but many ranks of Q
+        (11, 16, 128, 47, 882, 2, 3, dict(causal=1, causal_offset=835), True),
+        (11, 16, 128, 47, 882, 16, 3, dict(causal=1, causal_offset=-47), False),   # none
+        (4, 64, 64, 95, 867, 2, 3, dict(), True),
+        (4, 64, 64, 95, 867, 2, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),   # documents: four tiles met, 14 made
+        (1, 8, 64, 250, 900, 6, 4, dict(q_segment_ids=256, kv_segment_ids=256), True),
+        (1, 16, 128, 33, 1100, 6, 4, dict(causal=1), True),                        # as long as that the lengths decide
     ],
 )
-def test_keys_that_no_row_meets_do_not_count(B, H, D, lq, lk, rk, mask, dense):
+def test_keys_that_no_row_meets_do_not_count(B, H, D, lq, lk, rq, rk, mask, dense):
     from tpa import _dispatch as d
 
     lib = d.load_library()
     fake = d.TpaFactor(256, 8, 8, 8)
-    call = _forward_call(B=B, H=H, D=D, lq=lq, lk=lk, rk=rk, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, num_splits=1, **mask)
+    call = _forward_call(B=B, H=H, D=D, lq=lq, lk=lk, rq=rq, rk=rk, qa=fake, qb=fake, ka=fake, kb=fake, va=fake, vb=fake, num_splits=1, **mask)
     slot = lambda n: (2 * n + 255) // 256 * 256
     assert lib.tpa_fwd_call_workspace_bytes(ctypes.byref(call)) == (slot(B * lq * H * D) + 2 * slot(B * lk * H * D) if dense else 0)
 
