@@ -915,14 +915,14 @@ namespace tpa {
 namespace {
 // The same for one call, whose kernel, mask and ranks of Q are known: the us that dense arrays save there, from rank 3 on.  Against them
 // stand the launch and the trip of the arrays through memory, 0.3 us a MB; for them, every tile that a workgroup does not rebuild, as many as the longest
-// walk of a block has or the 256 compute units' share of all - in the kernel of 32 rows steps of its waves, 32 keys each - and, in the others, Q,
-// which they sum rank by rank.  Fitted to 1400 shapes of 17 to 2000 rows, ranks 3 to 16 (and 2, 6, 16 of Q), within 1.7 us (32 rows) and 3 (256) for the
-// half of them.  The line above alone took 56 of 1032 to the slower side by more than 2 %, with this 16, at the same gain over all (1.24).
-// fused / dense: 105 x 105, 3 x 16 heads of 128, rank 3 19.2 / 23.2; 100 x 100, 4 x 16, rank 3 19.6 / 24.8; 40 x 40, 12 x 32, rank 3 30.2 / 38.5;
-// 33 x 1000, 2 x 16 heads of 64, rank 3 32.6 / 41.4; 307 x 307, 2 x 64 of 64, rank 4 47.5 / 56.4; 100 x 317 in documents of 161, 45 x 40 of 128, rank 3
-// 381 / 463 (all stay fused); 200 x 200, 2 x 16 of 128, rank 4 34.3 / 29.2; 256 x 1000, 4 x 32 of 128, rank 4 249 / 190.
+// walk of a block has or the rounds of average ones - in the kernel of 32 rows steps of its waves, 32 keys each, the first of which hides a part - and, in the
+// others, Q, which they sum rank by rank.  Rank 3 costs less than its share.  Fitted to 2000 shapes of 17 to 2000 rows, ranks 3 to 16 (and 2, 4, 6, 16 of Q),
+// within 1.3 us (32 rows) and 3.4 (256) for the half of them.  The line above alone took 100 of 1500 to the slower side by more than 2 %, with this 28, at the
+// same gain over all (1.27).  fused / dense: 105 x 105, 3 x 16 heads of 128, rank 3 19.2 / 23.2; 100 x 100, 4 x 16, rank 3 19.6 / 24.8; 40 x 40, 12 x 32, rank 3 30.2 /
+// 38.5; 33 x 1000, 2 x 16 heads of 64, rank 3 32.6 / 41.4; 307 x 307, 2 x 64 of 64, rank 4 47.5 / 56.4; 100 x 317 in documents of 161, 45 x 40 of 128, rank 3
+// 381 / 463 (all stay fused); 200 x 200, 2 x 16 of 128, rank 4 34.3 / 29.2; 25 x 25, 2 x 8, rank 4 of Q, 3 20.2 / 17.5; 256 x 1000, 4 x 32, rank 4 249 / 190.
 double dense_saves_us(const TpaFwdArgs* a, int rows) {
-  const int64_t D = a->dk, pairs = (int64_t)a->B * a->H, reach = keys_in_reach(a), nblk = ((int64_t)a->lq + rows - 1) / rows;
+  const int64_t D = a->dk, pairs = (int64_t)a->B * a->H, reach = keys_in_reach(a), nblk = ((int64_t)a->lq + rows - 1) / rows, wgs = nblk * pairs;
   if (nblk > 256) return 1e9;  // K and V of so many blocks are not made in vain
   const int64_t behind = a->causal ? causal_offset_of(a) + (a->causal == TPA_CAUSAL_BOTTOM_RIGHT ? a->lk - a->lq : 0) : a->lk;  // row i meets keys up to i + this
   const int64_t step = rows == 32 ? 32 * (D == 64 ? SplitLdsF32<64>::NW : SplitLdsF32<128>::NW) : 64;
@@ -932,12 +932,12 @@ double dense_saves_us(const TpaFwdArgs* a, int rows) {
     longest = std::max(longest, steps);
     all += steps;
   }
-  double walk = std::max((double)longest, (double)(all * pairs) / 256.);
+  const double rounds = (double)((wgs + 255) / 256), rank = a->rk == 3 ? 2.4 : a->rk, mb = (double)(pairs * (a->lq + 2 * reach) * D) * 4e-6;
+  double walk = std::max((double)longest, rows == 32 ? (double)all / nblk * rounds : (double)(all * pairs) / 256.);
   if (a->kv_segment_ids && a->lk > a->lq && reach > 0) walk *= std::min(1., (double)(a->lq + 128) / (double)reach);  // documents: about as many keys as rows
-  const double rebuilt = walk * a->rk, q = (double)((nblk * pairs + 255) / 256) * a->rq, mb = (double)(pairs * (a->lq + 2 * reach) * D) * 4e-6;
-  if (rows == 32) return (D == 64 ? 0.97 * rebuilt - 5.3 : 1.67 * rebuilt - 4.7) - 0.3 * mb;
-  if (rows == 128 && D == 128) return 2.3 * (rebuilt - walk) + 2.1 * q - 20. - 0.3 * mb;
-  return (D == 64 ? 0.73 * rebuilt + 1.14 * q - 10.8 : 1.465 * rebuilt + 1.41 * q - 6.) - 0.3 * mb;
+  if (rows == 32) return (D == 64 ? (0.82 * walk - 0.15) * rank : (1.65 * walk - 0.21) * rank) - 3.6 - 0.3 * mb;
+  if (rows == 128 && D == 128) return 2.4 * walk * rank + 1.9 * rounds * a->rq - 26.5 - 0.3 * mb;
+  return (D == 64 ? 0.70 * walk * rank + 0.87 * rounds * a->rq - 11. : 1.43 * walk * rank + 1.22 * rounds * a->rq - 5.) - 0.3 * mb;
 }
 }  // namespace
 }  // namespace tpa
@@ -948,7 +948,7 @@ size_t tpa_prefill_f32_call_bytes(const TpaFwdArgs* a) {
   const size_t need = tpa_prefill_f32_dense_bytes(a->B, a->lq, a->lk, a->H, a->dk, a->rk);
   if (!need) return 0;
   const int rows = rows_per_workgroup(params_of(a), a->dk);
-  if (a->rk > 2 && dense_saves_us(a, rows) < 1.) return 0;
+  if (a->rk > 2 && dense_saves_us(a, rows) < 0.5) return 0;
   // Rows of H * D floats reach the 2 GiB of the kernel of 32 rows before those of the factors do: a call that would fall from it to 256
   // rows stays on the factors (64 rows over 140 000 keys, 32 heads of 128, rank 4: 128 workgroups that share out the keys against 32 with
   // two of eight waves at work, and 4.6 GB).
