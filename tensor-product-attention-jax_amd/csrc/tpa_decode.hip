@@ -1358,6 +1358,6 @@ extern "C" int tpa_decode_noalloc(const TpaFwdArgs* a, void* stream) {
   // the decode kernel of the same call, so nothing of the previous call's contents has to be cleared
   TpaFwdArgs b = *a;
   b.workspace = ptr;
-  b.workspace_bytes = TPA_DECODE_NOALLOC_SCRATCH_BYTES;
+  b.workspace_bytes = workspace_bytes(a->B, a->lq, a->H, a->dv, S);  // as many ranges as tpa_decode has with what it needs
   return bf16 ? tpa_decode_mfma_launch(&b, static_cast<hipStream_t>(stream)) : tpa_decode_f32_launch(&b, static_cast<hipStream_t>(stream));
 }

@@ -92,6 +92,13 @@ def test_noalloc_decode_other_instances(gpu):
     _both(gpu, lib, 5, 1, 1, 300, 8, 64, 2, 2, torch.float32)
 
 
+@pytest.mark.parametrize("b,lq,lk,h,d,rk", [(1, 1, 700, 16, 128, 8), (2, 2, 3000, 32, 64, 4), (3, 1, 920, 8, 64, 16), (2, 4, 2000, 64, 128, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_noalloc_decode_of_high_ranks(gpu, b, lq, lk, h, d, rk, dtype):
+    """Ranks for which more key ranges than the sizes ask for would fit the array: as many as tpa_decode has with the workspace that it needs."""
+    _both(gpu, _d.load_library(), 6, b, lq, lk, h, d, 3, rk, dtype)
+
+
 def test_noalloc_decode_refuses_what_does_not_fit(gpu):
     lib = _d.load_library()
     b, lq, lk, h, d, rq, rk = 64, 8, 8192, 32, 128, 6, 2  # partials of 8 query rows: beyond the fixed array
