@@ -161,7 +161,7 @@ size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H
   if (const size_t f32 = tpa_prefill_f32_dense_bytes(B, lq, lk, H, dk, rk); f32 > best) best = f32;
   if (lq <= 16 && lk >= 1024)
     for (int dtype : {TPA_DTYPE_BF16, TPA_DTYPE_F32}) {
-      const size_t decode = tpa_decode_rank_bytes(B, lq, lk, H, dv, rk, dtype, false);
+      const size_t decode = tpa_decode_rank_bytes(B, lq, lk, H, dv, rk, dtype);
       if (decode > best) best = decode;
     }
   return best > base ? best : base;

@@ -362,8 +362,7 @@ int mha_prefill_f32_supported(const MhaFwdArgs* a);
 int mha_prefill_f32_launch(const MhaFwdArgs* a, hipStream_t stream);
 int tpa_nomat_pairs_supported(const TpaFwdArgs* a);
 int tpa_nomat_pairs_launch(const TpaFwdArgs* a, hipStream_t stream);
-// of the partials of as many key ranges as the rank has a use for; dealt: by the lengths of the batch entries, for which it never has more
-size_t tpa_decode_rank_bytes(int B, int lq, int lk, int H, int dv, int rk, int dtype, bool dealt);
+size_t tpa_decode_rank_bytes(int B, int lq, int lk, int H, int dv, int rk, int dtype);  // of the partials of as many key ranges as the rank has a use for
 int tpa_decode_mfma_supported(const TpaFwdArgs* a);
 int tpa_decode_mfma_launch(const TpaFwdArgs* a, hipStream_t stream);
 int tpa_decode_f32_supported(const TpaFwdArgs* a);

@@ -32,12 +32,8 @@ constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit data format
 enum class Reads { kOrdinary, kStreaming, kFar };
 constexpr int64_t kFarthestRow = 1 << 25;  // elements between neighbouring rows, at most, for the first two
 constexpr int kMinKeys = kWaves * kRowsPerBlock / 2;  // keys of a range with one block of rank 2 per wave
-// The same of the call's rank, from rank 4 on.  In bf16 at head size 64 and rank 4 the ranges of fewer keys than two blocks that lengths deal out are
-// no whole rounds of blocks, and are left as they were: us, two blocks / one, lengths from half on: 28 x 317, 32 heads, two rows 12.7 / 13.9; 2 x 1519, 64
-// heads, four rows 12.7 / 14.1; 4 x 1500, 64 heads 10.8 / 11.7.
-inline int least_keys(int dtype, int D, int rk, bool dealt) {
-  return rk <= 2 || (dtype == TPA_DTYPE_BF16 && D == 64 && rk == 4 && dealt) ? kMinKeys : kWaves * kRowsPerBlock / rk;
-}
+// The same of the call's rank, from rank 4 on
+inline int least_keys(int rk) { return rk <= 2 ? kMinKeys : kWaves * kRowsPerBlock / rk; }
 // Ranges up to which that counts: beyond, in bf16 at head size 64, the partials of twice the ranges cost more than a second block.  us, by the sizes
 // alone / by rank: rank 4, 16 to 63 ranges 1 x 700, 64 heads 8.7 / 8.1, 4 x 1000, 16 heads, two rows 9.7 / 8.6, 2 x 1500, 8 heads 8.6 / 8.3; more 1 x 8000, 32
 // heads, two rows 13.3 / 15.2, 1 x 8000, 8 heads 10.5 / 12.0; rank 8, over 127 1 x 7724, 8 heads 12.9 / 13.9, 1 x 8812, two rows 14.7 / 15.7.
@@ -97,7 +93,10 @@ __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, in
   const int lane = threadIdx.x & 63;
   const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
   const int total = __builtin_amdgcn_readlane(wave_prefix_sum(len), 63);
-  const float shortest = fmaxf((float)total / (float)slots, min_keys);
+  float shortest = fmaxf((float)total / (float)slots, min_keys);
+  // From rank 4 on short ranges are whole rounds of blocks (a power of two of keys): in between, a wave has as many blocks and there are more partials.  us, any
+  // length / so, head size 64, rank 4, lengths from half on: 28 x 317 keys, 32 heads, two rows 13.9 / 12.6; 2 x 1519, 64 heads, four rows 14.1 / 12.6.
+  if (shortest < (float)kMinKeys) shortest = ceilf(shortest / min_keys) * min_keys;
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
   float length = fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
   if (round_keys > 0.f) length = ceilf(length / round_keys) * round_keys;
@@ -1009,7 +1008,7 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq;
   p.S = ranges.S; p.slots = ranges.slots;
   p.round_keys = a->dv == 128 ? kWaves * kRowsPerBlock / (float)RK : 0.f;
-  p.min_keys = (float)least_keys(a->dtype, a->dv, RK, true);
+  p.min_keys = (float)least_keys(RK);
   p.kvlen = a->kv_lengths;
   p.climit = a->causal ? causal_offset_of(a) + 1 + rows.row0 : a->lk;
   p.cbr = a->causal == TPA_CAUSAL_BOTTOM_RIGHT;
@@ -1157,20 +1156,19 @@ int rows_per_workgroup(int H) { return H == 8 ? 4 : 2; }
 // heads 15.2 / 10.8, 32 heads 16.2 / 11.6, 3 x 920 16.1 / 11.6, 2 x 3000 17.3 / 15.1, 32 heads, four rows 23.2 / 21.8; rank 4, 1 x 700 12.5 /
 // 10.5, 2 x 3000, 32 heads 14.6 / 13.0; fp32, 2 x 2000, 8 heads of 64, rank 8 32.0 / 21.9, 3 x 900, 32 heads of 128 56.3 / 36.8.  (Rank 2, 1 x 670,
 // 32 heads, two rows: 13.4, with twice the ranges 13.8.)
-int splits_by_rank(int B, int lq, int lk, int H, int D, int rk, int dtype, int rows_per_group, bool dealt) {
+int splits_by_rank(int B, int lq, int lk, int H, int D, int rk, int dtype, int rows_per_group) {
   const int by_size = default_splits(B, lq, lk, H, rows_per_group);
   const int64_t groups = (int64_t)B * ((lq + rows_per_group - 1) / rows_per_group) * ((H + 31) / 32);
-  const int keys = rk <= kRowsPerBlock && (rk & (rk - 1)) == 0 ? least_keys(dtype, D, rk, dealt) : kMinKeys;  // of a rank that the kernels take
+  const int keys = rk <= kRowsPerBlock && (rk & (rk - 1)) == 0 ? least_keys(rk) : kMinKeys;  // of a rank that the kernels take
   if (keys >= kMinKeys || groups >= 256) return by_size;
   const int want = (int)((256 + groups - 1) / groups);
   return std::max(by_size, std::min({want, (lk + keys - 1) / keys, noalloc_room(B, lq, H), most_by_rank(dtype, D, rk)}));
 }
-bool ranges_are_dealt(const TpaFwdArgs* a) { return a->kv_lengths && a->B <= kMaxPlanEntries; }
 // and within the room that the call brings
 int splits_of_call(const TpaFwdArgs* a, int rows_per_group) {
   const size_t room = a->workspace_bytes / workspace_bytes(a->B, a->lq, a->H, a->dv, 1);
   return std::max(default_splits(a->B, a->lq, a->lk, a->H, rows_per_group),
-                  (int)std::min<size_t>(room, splits_by_rank(a->B, a->lq, a->lk, a->H, a->dv, a->rk, a->dtype, rows_per_group, ranges_are_dealt(a))));
+                  (int)std::min<size_t>(room, splits_by_rank(a->B, a->lq, a->lk, a->H, a->dv, a->rk, a->dtype, rows_per_group)));
 }
 
 // How a launch splits the keys if the caller leaves it to us, with partials for B * splits_of_call ranges at hand.
@@ -1182,9 +1180,9 @@ int splits_of_call(const TpaFwdArgs* a, int rows_per_group) {
 KeyRanges choose_ranges(const TpaFwdArgs* a, int rows_per_group) {
   const int S = splits_of_call(a, rows_per_group);
   const int per_range = (a->lq + rows_per_group - 1) / rows_per_group * ((a->H + 31) / 32);  // workgroups of one range
-  if (ranges_are_dealt(a))
+  if (a->kv_lengths && a->B <= kMaxPlanEntries)
     return KeyRanges{S, std::min(std::max(a->B, 256 / per_range), a->B * S)};
-  const int keys = least_keys(a->dtype, a->dv, a->rk, false), most = (a->lk + keys - 1) / keys;
+  const int keys = least_keys(a->rk), most = (a->lk + keys - 1) / keys;
   const int n = std::max(1, (int)std::min<int64_t>(std::min(S, most), 256 / ((int64_t)a->B * per_range)));
   const int64_t blocks = ((int64_t)a->lk * a->rk + kRowsPerBlock - 1) / kRowsPerBlock, rounds = (blocks + kWaves * n - 1) / (kWaves * n);
   return KeyRanges{(int)((blocks + kWaves * rounds - 1) / (kWaves * rounds)), 0};
@@ -1204,14 +1202,14 @@ extern "C" size_t tpa_decode_workspace_bytes(int32_t B, int32_t lq, int32_t lk, 
   return tpa::workspace_bytes(B, lq, H, dv, S);
 }
 
-size_t tpa_decode_rank_bytes(int B, int lq, int lk, int H, int dv, int rk, int dtype, bool dealt) {
-  return tpa::workspace_bytes(B, lq, H, dv, tpa::splits_by_rank(B, lq, lk, H, dv, rk, dtype, dtype == TPA_DTYPE_BF16 ? tpa::rows_per_workgroup(H) : 1, dealt));
+size_t tpa_decode_rank_bytes(int B, int lq, int lk, int H, int dv, int rk, int dtype) {
+  return tpa::workspace_bytes(B, lq, H, dv, tpa::splits_by_rank(B, lq, lk, H, dv, rk, dtype, dtype == TPA_DTYPE_BF16 ? tpa::rows_per_workgroup(H) : 1));
 }
 
 extern "C" size_t tpa_decode_call_workspace_bytes(const TpaFwdArgs* a) {
   if (!a || a->B <= 0 || a->lq <= 0 || a->lk <= 0 || a->H <= 0 || a->dv <= 0 || a->rk <= 0) return 0;
   const size_t base = tpa_decode_workspace_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->num_splits);
-  return a->num_splits > 0 ? base : std::max(base, tpa_decode_rank_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->rk, a->dtype, tpa::ranges_are_dealt(a)));
+  return a->num_splits > 0 ? base : std::max(base, tpa_decode_rank_bytes(a->B, a->lq, a->lk, a->H, a->dv, a->rk, a->dtype));
 }
 
 int tpa_decode_mfma_supported(const TpaFwdArgs* a) {

@@ -54,18 +54,27 @@ def test_room_for_a_block_per_wave(b, lq, lk, h, d, rk, bf16, ranges):
         assert need <= lib.tpa_fwd_best_workspace_bytes(b, lq, lk, h, d, d, 6, rk)
 
 
-@pytest.mark.parametrize("b,lq,lk,h,d,rk,bf16,ranges", [(2, 4, 1519, 64, 64, 4, True, 24), (2, 4, 1519, 64, 128, 4, True, 31), (2, 4, 1519, 64, 64, 8, True, 31),
-                                                        (2, 4, 1519, 64, 64, 4, False, 24), (65, 1, 1519, 32, 64, 4, True, 4)])
-def test_room_where_the_ranges_are_dealt_by_the_lengths(b, lq, lk, h, d, rk, bf16, ranges):
-    """bf16, head size 64, rank 4: two blocks per wave, as by the sizes alone; the others as without lengths, within the fixed array."""
-    from tpa import _dispatch as disp
+@pytest.mark.gpu
+@pytest.mark.parametrize("h,d,rk", [(16, 64, 4), (32, 64, 8), (8, 128, 4), (64, 64, 16), (32, 128, 32)])
+@pytest.mark.parametrize("lengths", [[317, 200, 158, 250] * 7, [1519, 760], [32, 33, 64, 65, 31, 1, 0, 1000], [128 * 32], [16 * i + 1 for i in range(64)]])
+def test_short_ranges_are_whole_rounds(gpu, lengths, h, d, rk):
+    """Lengths of which the ranges' share lies at, below and between rounds of blocks: every entry is what it is alone."""
+    from tpa import tpa
 
-    lib = disp.load_library()
-    call = _call(b, lq, lk, h, d, rk, bf16)
-    call.kv_lengths = 256
-    need = lib.tpa_decode_call_workspace_bytes(ctypes.byref(call))
-    assert need == b * lq * h * (d + 2) * 4 * ranges
-    assert lib.tpa_decode_workspace_bytes(b, lq, lk, h, d, 0) <= need <= lib.tpa_fwd_best_workspace_bytes(b, lq, lk, h, d, d, 6, rk)
+    gen = torch.Generator(device="cpu").manual_seed(len(lengths))
+    b, lk, lq = len(lengths), max(lengths), 2
+    make = lambda n, r, x: (torch.randn((b, n, r, x), generator=gen) / r**0.5).to(gpu, torch.bfloat16)
+    args = [make(n, r, x) for n, r in ((lq, 6), (lk, rk), (lk, rk)) for x in (h, d)]
+    kw = dict(sm_scale=d**-0.5, kernel=2)
+    o, lse = tpa.tpa_decode(*args, kv_lengths=torch.tensor(lengths, dtype=torch.int32, device=gpu), **kw)
+    for i in sorted({0, b // 2, b - 1, lengths.index(max(lengths)), lengths.index(min(lengths))}):
+        if not lengths[i]:
+            assert o[i].isnan().all() and lse[i].isneginf().all()
+            continue
+        want, want_lse = tpa.tpa_decode(*(x[i : i + 1, : (lengths[i] if n > 1 else lq)] for n, x in enumerate(args)), num_splits=1, **kw)
+        got, want = o[i].float(), want[0].float()
+        assert ((got - want).abs() <= 2**-7 * want.abs() + 2**-12 * want.abs().amax(-1, keepdim=True)).all()
+        assert torch.allclose(lse[i], want_lse[0], atol=1e-5, rtol=0)
 
 
 @pytest.mark.gpu
