@@ -914,13 +914,13 @@ F32Params dense_params_of(const TpaFwdArgs* a, const float* qd, const float* kd,
 namespace tpa {
 namespace {
 // The same for one call, whose kernel, mask and ranks of Q are known: the us that dense arrays save there, from rank 3 on.  Against them
-// stand the launch and the trip of the arrays through memory, 0.3 us a MB; for them, every tile that a workgroup does not rebuild, as many as the longest
+// stand the launch and the trip of K and V through memory, 0.2 us a MB; for them, every tile that a workgroup does not rebuild, as many as the longest
 // walk of a block has or the rounds of average ones - in the kernel of 32 rows steps of its waves, 32 keys each, the first of which hides a part - and, in the
 // others, Q, which they sum rank by rank.  Rank 3 costs less than its share.  Fitted to 2000 shapes of 17 to 2000 rows, ranks 3 to 16 (and 2, 4, 6, 16 of Q),
-// within 1.3 us (32 rows) and 3.4 (256) for the half of them.  The line above alone took 100 of 1500 to the slower side by more than 2 %, with this 28, at the
-// same gain over all (1.27).  fused / dense: 105 x 105, 3 x 16 heads of 128, rank 3 19.2 / 23.2; 100 x 100, 4 x 16, rank 3 19.6 / 24.8; 40 x 40, 12 x 32, rank 3 30.2 /
-// 38.5; 33 x 1000, 2 x 16 heads of 64, rank 3 32.6 / 41.4; 307 x 307, 2 x 64 of 64, rank 4 47.5 / 56.4; 100 x 317 in documents of 161, 45 x 40 of 128, rank 3
-// 381 / 463 (all stay fused); 200 x 200, 2 x 16 of 128, rank 4 34.3 / 29.2; 25 x 25, 2 x 8, rank 4 of Q, 3 20.2 / 17.5; 256 x 1000, 4 x 32, rank 4 249 / 190.
+// within 1.2 us (32 rows) and 3 (256) for the half of them.  The line above alone took 100 of 1500 to the slower side by more than 2 %, with this 34, at the
+// same gain over all (1.275).  fused / dense: 105 x 105, 3 x 16 heads of 128, rank 3 19.2 / 23.2; 100 x 100, 4 x 16, rank 3 19.6 / 24.8; 40 x 40, 12 x 32, rank 3 30.2 /
+// 38.5; 307 x 307, 2 x 64 of 64, rank 4 47.5 / 56.4; 100 x 317 in documents of 161, 45 x 40 of 128, rank 3 381 / 463 (all stay fused); 33 x 1000, 2 x 16 heads of 64,
+// rank 3 32.6 / 41.4 (does not); 25 x 25, 2 x 8, rank 4 of Q, 3 20.2 / 17.5; 200 x 200, 2 x 16 of 128, rank 4 34.3 / 29.2; 256 x 256, 8 x 32, rank 4 86.6 / 72.6; 256 x 1000, 4 x 32, rank 4 249 / 190.
 double dense_saves_us(const TpaFwdArgs* a, int rows) {
   const int64_t D = a->dk, pairs = (int64_t)a->B * a->H, reach = keys_in_reach(a), nblk = ((int64_t)a->lq + rows - 1) / rows, wgs = nblk * pairs;
   if (nblk > 256) return 1e9;  // K and V of so many blocks are not made in vain
@@ -932,12 +932,14 @@ double dense_saves_us(const TpaFwdArgs* a, int rows) {
     longest = std::max(longest, steps);
     all += steps;
   }
-  const double rounds = (double)((wgs + 255) / 256), rank = a->rk == 3 ? 2.4 : a->rk, mb = (double)(pairs * (a->lq + 2 * reach) * D) * 4e-6;
-  double walk = std::max((double)longest, rows == 32 ? (double)all / nblk * rounds : (double)(all * pairs) / 256.);
+  const double rounds = (double)((wgs + 255) / 256), rank = a->rk == 3 ? 2.7 : a->rk, mb = (double)(2 * pairs * reach * D) * 4e-6;
+  double walk = std::max((double)longest, (double)all / nblk * rounds);
   if (a->kv_segment_ids && a->lk > a->lq && reach > 0) walk *= std::min(1., (double)(a->lq + 128) / (double)reach);  // documents: about as many keys as rows
-  if (rows == 32) return (D == 64 ? (0.82 * walk - 0.15) * rank : (1.65 * walk - 0.21) * rank) - 3.6 - 0.3 * mb;
-  if (rows == 128 && D == 128) return 2.4 * walk * rank + 1.9 * rounds * a->rq - 26.5 - 0.3 * mb;
-  return (D == 64 ? 0.70 * walk * rank + 0.87 * rounds * a->rq - 11. : 1.43 * walk * rank + 1.22 * rounds * a->rq - 5.) - 0.3 * mb;
+  if (rows == 32)
+    return D == 64 ? (0.94 * walk - 0.30) * rank - 2.2 * wgs / 256 - 2.8 - 0.23 * mb : (1.63 * walk - 0.26) * rank - 3.3 * wgs / 256 - 2.2 - 0.24 * mb;
+  if (rows == 128 && D == 128) return walk * (2.56 * rank - 2.8) + rounds * (2. * a->rq) - 25. - 0.05 * mb;
+  return D == 64 ? walk * (0.69 * rank - 0.68) + rounds * (0.98 * a->rq - 3.6) - 8. - 0.16 * mb
+                 : walk * (1.33 * rank - 1.2) + rounds * (1.63 * a->rq - 9.4) + 4.6 - 0.24 * mb;
 }
 }  // namespace
 }  // namespace tpa

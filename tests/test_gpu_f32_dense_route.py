@@ -70,9 +70,9 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, dense):
         (4, 32, 128, 135, 135, 16, 3, dict(), True),
         (4, 32, 128, 256, 1000, 2, 3, dict(causal=2), True),
         (4, 32, 128, 256, 1000, 2, 3, dict(causal=1), False),   # a quarter of the keys in reach
-        (1, 16, 128, 40, 1500, 6, 3, dict(causal=1), False),    # the same of 32 rows
-        (1, 16, 128, 40, 1500, 6, 3, dict(causal=1, causal_offset=1460), True),
-        (1, 16, 128, 40, 1500, 6, 3, dict(causal=1, causal_offset=-40), False),
+        (4, 16, 128, 40, 1500, 6, 3, dict(causal=1), False),    # the same of 32 rows
+        (4, 16, 128, 40, 1500, 6, 3, dict(causal=1, causal_offset=1460), True),
+        (4, 16, 128, 40, 1500, 6, 3, dict(causal=1, causal_offset=-40), False),
         (45, 40, 128, 100, 317, 4, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),  # documents: 228 of 317 keys
         (1, 8, 128, 65537, 65537, 6, 3, dict(causal=1), True),  # more blocks than are looked at
     ],
