@@ -141,8 +141,8 @@ __device__ __forceinline__ void delta_h8(const DeltaJob& j, int64_t t, int g, in
 
 // This thread's token t, group g of 8 heads and piece cc of D: shifts where the counts are powers of two (three divisions of 64 bits
 // are a microsecond before the first load: 1340 tokens x 16 heads x 128 with the delta 10.6 us, with shifts and its sums by DPP 7.8)
-__device__ __forceinline__ void piece_of(int cpr, int hg, int64_t& t, int& g, int& cc) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void piece_of(int cpr, int hg, int64_t& t, int& g, int& cc, int blk) {
+  const int64_t idx = (int64_t)blk * 256 + threadIdx.x;
   if (((cpr & (cpr - 1)) | (hg & (hg - 1))) == 0) {
     const int s = __builtin_ctz(cpr);
     cc = (int)idx & (cpr - 1);
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void recon_f32_h8_kernel(ReconJobs jobs, int H
   const int cpr = D / 4, hg = H / 8;
   int cc, g;
   int64_t t;
-  piece_of(cpr, hg, t, g, cc);
+  piece_of(cpr, hg, t, g, cc, blockIdx.x);
   const int b = blockIdx.y;
   if (blockIdx.z == 3) return delta_h8<float>(jobs.delta, t, g, cc, cpr, b, H, D);
   const ReconJob job = blockIdx.z == 0 ? jobs.job[0] : blockIdx.z == 1 ? jobs.job[1] : jobs.job[2];
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void recon_bf16_h8_kernel(ReconJobs jobs, int 
   const int cpr = D / 8, hg = H / 8;
   int cc, g;
   int64_t t;
-  piece_of(cpr, hg, t, g, cc);
+  piece_of(cpr, hg, t, g, cc, blockIdx.x);
   const int b = blockIdx.y;
   if (blockIdx.z == 3) return delta_h8<uint16_t>(jobs.delta, t, g, cc, cpr, b, H, D);
   if (t >= tokens_of(n, lengths, b)) return;
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256) void project_kernel(const float* dx, TpaFactor
 // All arrays that this kernel takes in one launch (blockIdx.z): at short lengths a launch of its own leaves each of them
 // waiting for the one before.  The gradients are written in the type the caller wants them in (rounded once, from the fp32 sums).
 struct ProjectJob { const float* dx; TpaFactor fa, fb; TpaGrad ga, gb; int L, R, D; };
-struct ProjectJobs { ProjectJob job[3]; int first[3], ranks; };  // array i: blockIdx.z = first[i] on, `ranks` ranks for each
+struct ProjectJobs { ProjectJob job[3]; int first[3], ranks, blocks, B; };  // array i: blockIdx.z = first[i] on, `ranks` ranks for each; blocks > 0: batch entries of so many workgroups, one after the other in blockIdx.x
 template <typename T>
 using Four = std::conditional_t<sizeof(T) == 2, u32x2, f32x4>;  // four values as they lie in memory
 __device__ __forceinline__ f32x4 as_f32(const u32x2& x) { return f32x4{bf16lo_to_f32(x[0]), bf16hi_to_f32(x[0]), bf16lo_to_f32(x[1]), bf16hi_to_f32(x[1])}; }
@@ -635,11 +635,16 @@ __global__ __launch_bounds__(256) void project_h8_kernel(ProjectJobs jobs, int H
   const int cpr = D / 8, hgs = H / 8, tt = cpr * hgs;  // threads per token
   int cc, hg;
   int64_t tok;
-  piece_of(cpr, hgs, tok, hg, cc);
+  int blk = blockIdx.x, b = blockIdx.y;
+  if (jobs.blocks > 0) {
+    b = blk / jobs.blocks;
+    blk -= b * jobs.blocks;
+    if (b >= jobs.B) return;
+  }
+  piece_of(cpr, hgs, tok, hg, cc, blk);
   const bool live = tok < L;
-  if ((int64_t)blockIdx.x * (256 >> __builtin_ctz(tt)) >= L) return;  // a whole workgroup past the end of a shorter array
+  if ((int64_t)blk * (256 >> __builtin_ctz(tt)) >= L) return;  // a whole workgroup past the end of a shorter array
   const int64_t t = live ? tok : L - 1;  // lanes past the end idle along: the reductions need whole waves
-  const int b = blockIdx.y;
   const int dh = D / 2;  // a thread's eight columns: 4 cc .. 4 cc + 3 and the same in the upper half of the row
   const float* xp = j.dx + (((int64_t)b * L + t) * H + 8 * hg) * D + 4 * cc;
   const T* ap = static_cast<const T*>(fa.ptr) + b * fa.stride_b + t * fa.stride_l + 8 * hg;
@@ -753,7 +758,7 @@ bool projects_by_h8(const ProjectJob& j, int H) {
 // by workgroups of one array: ranks 16, 8, 8: 11 of them (335 tokens, 8 heads of 64) 14.9 / 6.5, 63 17.1 / 12.5 (four ranks each, 504 workgroups
 // 11.7), 99 19.0 / 15.8 (four each 19.0), 250 23.4 / 25.8; 6, 2, 2: 34 7.2 / 5.3, 54 7.8 / 7.2, fp32 64 8.6 / 7.0; 6, 4, 4: 175 13.1 / 13.5.
 // That holds where the parts of a token find its dx in the L2 of their XCD: workgroups go to the XCDs in turn, so a part has a multiple of eight of them (the
-// last ones past every array).  Without that, whole backward, all ranks / parts of two: ranks 6, 4, 4, 3 x 156 tokens, 32 heads of 64 (60 workgroups)
+// last ones past every array), those of all batch entries side by side.  Without that, whole backward, all ranks / parts of two: ranks 6, 4, 4, 3 x 156 tokens, 32 heads of 64 (60 workgroups)
 // 29.9 / 34.2, 2 x 218 (56) 30.4 / 28.1; 4, 3, 3, 208 tokens, 64 heads (52) 26.8 / 32.3, 2 x 112 (56) 27.0 / 26.0; 6, 2, 2, 3 x 130, 64 heads (99) 31.5 /
 // 32.3, 16 x 164, 8 heads (96) 29.6 / 27.4.
 int ranks_per_workgroup(const ProjectJobs& jobs, unsigned n, int64_t blocks) {
@@ -796,8 +801,13 @@ void launch_project(const ProjectJobs& jobs, int B, int H, hipStream_t stream) {
     h8.first[i] = i < n ? (int)parts : INT32_MAX;
     if (i < n) parts += (h8.job[i].R + h8.ranks - 1) / h8.ranks;
   }
-  if (parts > n) blocks = (blocks + 7) / 8 * 8;
-  hipLaunchKernelGGL((project_h8_kernel<T, TO>), dim3((unsigned)blocks, B, parts), dim3(256), 0, stream, h8, H);
+  dim3 grid((unsigned)blocks, B, parts);
+  if (parts > n) {
+    h8.blocks = (int)blocks;
+    h8.B = B;
+    grid = dim3((unsigned)((blocks * B + 7) / 8 * 8), 1, parts);
+  }
+  hipLaunchKernelGGL((project_h8_kernel<T, TO>), grid, dim3(256), 0, stream, h8, H);
 }
 
 template <typename T, int DMAX>
