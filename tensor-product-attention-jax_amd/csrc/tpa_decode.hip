@@ -93,10 +93,7 @@ __device__ __forceinline__ RangePlan plan_ranges(const int32_t* kvlen, int B, in
   const int lane = threadIdx.x & 63;
   const int len = lane < B ? max(0, min(kvlen[lane], lk)) : 0;
   const int total = __builtin_amdgcn_readlane(wave_prefix_sum(len), 63);
-  float shortest = fmaxf((float)total / (float)slots, min_keys);
-  // From rank 4 on short ranges are whole rounds of blocks (a power of two of keys): in between, a wave has as many blocks and there are more partials.  us, any
-  // length / so, head size 64, rank 4, lengths from half on: 28 x 317 keys, 32 heads, two rows 13.9 / 12.6; 2 x 1519, 64 heads, four rows 14.1 / 12.6.
-  if (shortest < (float)kMinKeys) shortest = ceilf(shortest / min_keys) * min_keys;
+  const float shortest = fmaxf((float)total / (float)slots, min_keys);
   const float longest = slots > B ? fmaxf((float)total / (float)(slots - B) + 1.f, shortest) : (float)lk;
   float length = fmaf((longest - shortest) * (float)lane, 1.f / 63.f, shortest);
   if (round_keys > 0.f) length = ceilf(length / round_keys) * round_keys;
@@ -1007,7 +1004,9 @@ DecodeParams decode_params(const TpaFwdArgs* a, KeyRanges ranges, RowWindow rows
   p.part_o = ws; p.part_m = ws + no; p.part_l = ws + no + nm;
   p.B = a->B; p.lq = a->lq; p.lk = a->lk; p.H = a->H; p.rq = a->rq;
   p.S = ranges.S; p.slots = ranges.slots;
-  p.round_keys = a->dv == 128 ? kWaves * kRowsPerBlock / (float)RK : 0.f;
+  // (Rank 2 at head size 64 has any length.  Rank 4 there, us, any length / whole rounds, lengths from half on: 28 x 317 keys, 32 heads, two rows 13.9 / 12.6;
+  // 2 x 1519, 64 heads, four rows 14.1 / 12.6; mean of 1092 shapes 1.00 of the time by the sizes alone / 0.98.)
+  p.round_keys = a->dv == 128 || RK > 2 ? kWaves * kRowsPerBlock / (float)RK : 0.f;
   p.min_keys = (float)least_keys(RK);
   p.kvlen = a->kv_lengths;
   p.climit = a->causal ? causal_offset_of(a) + 1 + rows.row0 : a->lk;
