@@ -863,7 +863,7 @@ int tpa_bwd_t(const TpaBwdArgs* a, hipStream_t stream, bool mfma) {
     jobs.job[1] = ReconJob{a->ka, a->kb, kd, a->lk, a->rk, 1.f, a->lk, nullptr};
     jobs.job[2] = ReconJob{a->va, a->vb, vd, a->lk, a->rk, 1.f, a->lk, nullptr};
     jobs.delta = DeltaJob{a->o, a->d_o, delta, a->lq};
-    if (mfma && a->q_segment_ids && windows_ahead_pay(a->B, a->H, a->lq, a->lk, 8192)) {
+    if (mfma && a->q_segment_ids && windows_ahead_pay(a->B, a->H, a->lq, a->lk, a->rk >= 16 ? 512 : 8192)) {
       // into the halves of the slots of Q and K that bf16 leaves: H D / 2 words a row there, eight a block taken
       const int block = dense_bwd_mfma_block(a->B, a->lq, a->lk, a->H, a->dk, a->causal, 1), coff = causal_offset_of(a);
       qwin = reinterpret_cast<int32_t*>(qd + nq / 2);

@@ -181,7 +181,9 @@ __device__ __forceinline__ void id_window(const int32_t* mine, int n_mine, const
 // In short calls of few heads the attention kernels find them in less time than that launch takes longer: us, here / by them, 1 x 58 tokens, 8 heads of
 // 64, backward 16.6 / 15.7, 2 x 323 25.8 / 24.9; 1 x 82, rank 8, forward 11.9 / 11.5.  By (batch, head) pairs times tokens, mean of the time by them over the
 // time here, 700 shapes: forward to 2048 0.98, to 4096 0.99, to 8192 1.02, to 65 536 1.016, beyond 1.05; backward to 4096 0.975, to 8192 0.99, to 16 384
-// 1.01, to 65 536 1.02, beyond 1.03.  `least`: of the forward's and of the backward's.
+// 1.01, to 65 536 1.02, beyond 1.03.  `least`: of the forward's and of the backward's;
+// from rank 16 on the workgroups of Q, which find them, have done before K and V are made (3 x 40 heads of 128, 24 tokens, forward 12.9 / 14.0; mean of 106 shapes
+// below 8192 1.045, of 55 backward 1.015).
 inline bool windows_ahead_pay(int B, int H, int lq, int lk, int64_t least) { return (int64_t)B * H * (lq > lk ? lq : lk) >= least; }
 struct IdWindow { int32_t first, last, count, least, most; };  // what id_window finds
 struct WindowJob {

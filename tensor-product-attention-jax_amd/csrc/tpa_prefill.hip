@@ -1286,11 +1286,13 @@ int launch_prefill(const PrefillParams& p, hipStream_t stream) {
 // Measured, us without / with ranges: a chunk of 331 tokens over 2258 keys, 16 heads of 128: 97 / 73; 608 over 11433, 8
 // heads of 64: 182 / 76; one sequence of 4096 tokens, 8 heads of 64, causal: 70 / 47.
 // Fewer than 24 tiles: of 2 and more blocks 512 to 1400 rows gain at most 8 % and lose up to twofold.  One block, where the ranges
-// find compute units that have nothing to do: a tile of the rank-2 rebuild is 2.0 us (1.1 at D = 64), one of dense arrays 1.55 (0.65),
+// find compute units that have nothing to do: a tile of the rank-2 rebuild is 2.0 us (1.1 at D = 64), one of dense arrays 1.75 in rank 2 (110 shapes of 380 to 768 keys,
+// 1.066 of one range's speed, 1.10 with the best count for each), of other ranks 1.55 (0.65),
 // a second range 9.5 and its partial results.  140 rows over 1160 keys, us without / with: rank 2, 8 heads of 128 44.4 / 29.6, 2 x 32 heads of 128
 // 45.1 / 39.5, 8 heads of 64 25.7 / 21.9; rank 4, 8 heads of 128 35.6 / 26.7; 4 x 16 heads of 64 26.2 / 26.2 (one range), rank 4 29.7 / 31.3 (one).
 // (What counts there is the `reach` of the mask, not the length of the cache: 33 rows over 861 keys from the first one on, 2 x 16 heads of 64, rank 2:
-// eight ranges, all but one empty, 11.7, one 6.7.)
+// eight ranges, all but one empty, 11.7, one 6.7.  And the tiles of the route: 217 over 437, 4 x 8 heads of 128, dense 23.7, in two ranges 28.9; 85 over 612, 2 x 8 24.2, in
+// five 22.8.)
 int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64_t rk, bool causal, int64_t reach, bool dense) {
   const int64_t blocks = (lq + kBQ - 1) / kBQ, wgs = blocks * B * H;
   const double per_tile = D == 128 ? 1.7 : 1.3, per_wg = 7.0, most = (double)((lk + kTK - 1) / kTK);
@@ -1299,7 +1301,7 @@ int choose_splits(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int64
   int best = 1;
   if (most < 24) {  // a block's own tiles take 40 us at most: little to win over the merge, but where one block has them all
     if (blocks > 1) return 1;
-    const double tile = rk == 2 && !dense ? (D == 128 ? 2.0 : 1.1) : (D == 128 ? 1.55 : 0.65);
+    const double tile = rk == 2 ? (D == 128 ? (dense ? 1.75 : 2.0) : 1.1) : (D == 128 ? 1.55 : 0.65);
     const int64_t tiles = (reach + kTK - 1) / kTK;
     double gain = 1.5;
     for (int S = 2; S <= 8 && wgs * S <= 256; ++S) {
@@ -1385,8 +1387,8 @@ bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int
   if (D == 64) return (pairs > 366 ? pairs / 366 : 1.0) * tiles * (0.55 + 0.36 * rk) > 4.5 + 0.28 * mb;
   return (double)((B * H + 255) / 256) * tiles * (0.55 + 0.57 * rk) > 2.0 + 0.21 * mb;
 }
-// The same for one call, whose mask and ranks of Q are known, in us.  What the mask hides is neither made dense nor met, and a block of documents meets about
-// as many keys as it has rows, and two tiles; the fused kernel sums Q rank by rank, which the dense launch does in passing.  Fitted to 1400 shapes of 17 to 256
+// The same for one call, whose mask and ranks of Q are known, in us.  What the mask hides is neither made dense nor met, and a block of documents, whose lengths
+// the host does not know, meets between as many keys as it has rows, with two tiles, and all: half way; the fused kernel sums Q rank by rank, which the dense launch does in passing.  Fitted to 1400 shapes of 17 to 256
 // rows, ranks 1 to 8 (1, 2, 4, 6, 16 of Q), within 1.1 us for the half of them.  The line above alone took 48 of 917 to the slower side by more than 2 %,
 // with this 15, at the same gain over all (1.24).  Fused / dense: 47 rows over 882 keys from the first one on, 11 x 16 heads of 128, ranks 2, 3 10.4 / 14.1; 95 over
 // 867 in documents of 100, 4 x 64 heads of 64, 2, 3 11.8 / 20.9; 227 x 227, 2 x 32 of 128, 2, 1 14.6 / 18.3; 102 x 172, 9 x 16, 2, 3 18.4 / 21.5 (all stay
@@ -1394,7 +1396,7 @@ bool one_block_pays(int64_t B, int64_t lq, int64_t lk, int64_t H, int64_t D, int
 double one_block_saves_us(const TpaFwdArgs* a) {
   const int64_t pairs = (int64_t)a->B * a->H, made = keys_in_reach(a);
   if (!made) return 0.0;  // the rows end before Q is needed
-  const int64_t tiles = ((a->kv_segment_ids ? std::min<int64_t>(made, a->lq + 2 * kTK) : made) + kTK - 1) / kTK;
+  const int64_t met = a->kv_segment_ids ? (made + std::min<int64_t>(made, a->lq + 2 * kTK)) / 2 : made, tiles = (met + kTK - 1) / kTK;
   const double mb = (double)(pairs * (a->lq + 2 * made) * a->dk) * 2e-6;
   if (a->dk == 64) {
     const double rounds = pairs > 366 ? (double)pairs / 366 : 1.0;
@@ -1506,7 +1508,7 @@ int tpa_prefill_mfma_launch(const TpaFwdArgs* a, hipStream_t stream) {
     uint16_t* vd = kd + kv_slot / 2;
     uint16_t* qd = vd + kv_slot / 2;
     WindowJob windows{};
-    const bool ahead = p.kvseg && windows_ahead_pay(a->B, a->H, a->lq, a->lk, 4096);
+    const bool ahead = p.kvseg && windows_ahead_pay(a->B, a->H, a->lq, a->lk, a->rk >= 16 ? 0 : 4096);
     if (ahead) {
       const int rows = a->dk == 64 && wants_four_waves(p, true) ? kBQ / 2 : kBQ;  // as launch_prefill has it
       windows = WindowJob{p.qseg, p.kvseg, p.kvlen, a->lq, a->lk, rows, 0, a->causal, p.coff, reinterpret_cast<int32_t*>(p.o),

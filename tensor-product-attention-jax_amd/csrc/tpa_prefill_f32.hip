@@ -934,7 +934,8 @@ double dense_saves_us(const TpaFwdArgs* a, int rows) {
   }
   const double rounds = (double)((wgs + 255) / 256), rank = a->rk == 3 ? 2.7 : a->rk, mb = (double)(2 * pairs * reach * D) * 4e-6;
   double walk = std::max((double)longest, (double)all / nblk * rounds);
-  if (a->kv_segment_ids && a->lk > a->lq && reach > 0) walk *= std::min(1., (double)(a->lq + 128) / (double)reach);  // documents: about as many keys as rows
+  // documents, whose lengths the host does not know, meet between as many keys as there are rows and all: half way
+  if (a->kv_segment_ids && a->lk > a->lq && reach > 0) walk *= 0.5 + 0.5 * std::min(1., (double)(a->lq + 128) / (double)reach);
   if (rows == 32)
     return D == 64 ? (0.94 * walk - 0.30) * rank - 2.2 * wgs / 256 - 2.8 - 0.23 * mb : (1.63 * walk - 0.26) * rank - 3.3 * wgs / 256 - 2.2 - 0.24 * mb;
   if (rows == 128 && D == 128) return walk * (2.56 * rank - 2.8) + rounds * (2. * a->rq) - 25. - 0.05 * mb;

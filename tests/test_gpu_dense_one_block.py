@@ -75,7 +75,7 @@ def test_ranks_of_q(B, H, D, lq, lk, rq, rk, dense):
         (11, 16, 128, 47, 882, 2, 3, dict(causal=1, causal_offset=835), True),
         (11, 16, 128, 47, 882, 16, 3, dict(causal=1, causal_offset=-47), False),   # none
         (4, 64, 64, 95, 867, 2, 3, dict(), True),
-        (4, 64, 64, 95, 867, 2, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),   # documents: four tiles met, 14 made
+        (4, 64, 64, 95, 867, 2, 3, dict(q_segment_ids=256, kv_segment_ids=256), False),   # documents: nine of 14 tiles met
         (1, 8, 64, 250, 900, 6, 4, dict(q_segment_ids=256, kv_segment_ids=256), True),
         (1, 16, 128, 33, 1100, 6, 4, dict(causal=1), True),                        # as long as that the lengths decide
     ],

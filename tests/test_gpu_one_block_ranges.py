@@ -48,7 +48,7 @@ def test_which_calls_ask_for_it(B, H, D, lq, lk, rk, ranges):
         (100, 1400, 2, dict(causal=1, causal_offset=-50), 1),
         (100, 1400, 2, dict(causal=2), 8),
         (100, 1400, 2, dict(), 8),
-        (64, 512, 2, dict(), 1),                                  # dense tiles, of which eight are not worth it
+        (64, 448, 2, dict(), 1),                                  # dense tiles, of which seven are not worth it
     ],
 )
 def test_keys_behind_the_mask_ask_for_no_ranges(lq, lk, rk, mask, ranges):
