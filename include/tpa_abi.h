@@ -305,7 +305,9 @@ const char* tpa_strerror(int code);
  * sm_scale * log2 e), K and V are reconstructed into it once and the prefill kernel runs its loop over
  * dense tiles.  Without a workspace the same problems run on the fused prefill kernel, which rebuilds
  * K / V tiles from the rank factors inside its loop.  The two routes round at the same points (Q, K, V,
- * the probabilities and the output to bf16 once each) but are not bit-identical.
+ * the probabilities and the output to bf16 once each) but are not bit-identical.  fp32 calls have the same
+ * two routes (dense fp32 arrays) where tpa_fwd_call_workspace_bytes asks for the room; they differ in the order
+ * of fp32 sums.
  */
 int tpa_fwd(const TpaFwdArgs* args, void* stream);
 
@@ -318,15 +320,18 @@ int tpa_fwd(const TpaFwdArgs* args, void* stream);
 size_t tpa_fwd_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk);
 
 /*
- * Bytes of optional workspace (256-byte aligned) that leave tpa_fwd every route it has for this problem: at least
- * tpa_fwd_workspace_bytes(...), plus room for the partial results of key ranges where the blocks of 256 query rows
- * alone would leave the chip partly idle (bf16, no segment ids), and for dense Q, K and V of calls of rank 2 below 2048
- * query rows where these pay.
+ * Bytes of optional workspace (256-byte aligned) that leave tpa_fwd every route it has for a problem of these sizes, whatever
+ * its element type, mask and strides: at least tpa_fwd_workspace_bytes(...), room for dense Q, K and V where these can pay, and
+ * behind them for the partial results of key ranges where the blocks of 256 query rows alone would leave the chip partly
+ * idle (bf16, no segment ids); for few query rows the partials of every key range that a decode of this rank has a use for.
+ * The element type is not an argument, so dense arrays are counted as fp32 where an fp32 call of these sizes could use them: a bf16 call
+ * then uses half of it or less (4 x 4096 tokens, 16 heads of 128, rank 2: 403 MB, of which a bf16 call uses 201).  Callers who hold
+ * one element type, or the call itself, ask tpa_fwd_call_workspace_bytes, which names what that call uses.
  */
 size_t tpa_fwd_best_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dk, int32_t dv, int32_t rq, int32_t rk);
 
 /*
- * Bytes of workspace (256-byte aligned) that tpa_fwd would use for this very call: its sizes, mask, segment ids, strides,
+ * Bytes of workspace (256-byte aligned) that tpa_fwd would use for this very call: its sizes, element type, mask, segment ids, strides,
  * alignment, kernel, num_splits and nomat; 0 if none, or if tpa_fwd would refuse the call.  `workspace` and
  * `workspace_bytes` of the arguments are not looked at.  Never more than tpa_fwd_best_workspace_bytes(...) unless
  * num_splits or nomat is set.
@@ -353,7 +358,8 @@ int tpa_decode(const TpaFwdArgs* args, void* stream);
 /*
  * tpa_decode without a caller workspace.  No counterpart in the reference: it exists for callers
  * that cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc).  Same arguments, kernels and results as tpa_decode, but args->workspace
+ * that forbid hipMalloc).  Same arguments, kernels and results as tpa_decode with a workspace of
+ * tpa_decode_workspace_bytes(...), but args->workspace
  * and args->workspace_bytes are ignored: the split partials go to a fixed device array of
  * TPA_DECODE_NOALLOC_SCRATCH_BYTES inside the library, one copy per GPU, held until the process
  * ends.  Problems whose partials (tpa_decode_workspace_bytes) exceed that size return
@@ -366,7 +372,8 @@ int tpa_decode(const TpaFwdArgs* args, void* stream);
 #define TPA_DECODE_NOALLOC_SCRATCH_BYTES (8u << 20)
 int tpa_decode_noalloc(const TpaFwdArgs* args, void* stream);
 
-/* Bytes of workspace tpa_decode needs for this problem (num_splits = 0: the default choice). */
+/* Bytes of workspace tpa_decode needs for this problem (num_splits = 0: the default choice, by the sizes alone).  With more, up to
+   tpa_decode_call_workspace_bytes(...), a decode of rank 4 and more has further key ranges and is faster over short caches. */
 size_t tpa_decode_workspace_bytes(int32_t B, int32_t lq, int32_t lk, int32_t H, int32_t dv, int32_t num_splits);
 
 /* Bytes of workspace with which tpa_decode has every key range that it has a use for in this very call: its sizes, rank, element type

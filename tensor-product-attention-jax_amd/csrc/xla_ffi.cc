@@ -121,7 +121,8 @@ ffi::Error TpaFwdSegImpl(hipStream_t stream, ffi::AnyBuffer q, ffi::AnyBuffer k,
   return rc == TPA_OK ? ffi::Error::Success() : fail(rc);
 }
 
-// workspace: an extra u8 result of tpa_decode_workspace_bytes(...) bytes, allocated by XLA
+// workspace: an extra u8 result of tpa_decode_workspace_bytes(...) bytes or more, allocated by XLA; what it has beyond that, up to
+// tpa_decode_call_workspace_bytes(...), gives calls of rank 4 and more further key ranges
 ffi::Error TpaDecodeImpl(hipStream_t stream, ffi::AnyBuffer q, ffi::AnyBuffer k, ffi::AnyBuffer v,
                          ffi::Result<ffi::AnyBuffer> o, ffi::Result<ffi::AnyBuffer> lse,
                          ffi::Result<ffi::AnyBuffer> workspace, int32_t num_heads, float sm_scale) {

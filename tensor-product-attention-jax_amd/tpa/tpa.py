@@ -245,6 +245,9 @@ def cache_append_workspace_bytes(b: int, n: int, d_model: int, h: int, d: int, r
 
 
 def decode_workspace_bytes(b: int, lq: int, lk: int, h: int, dv: int, num_splits: int = 0) -> int:
+    """What `tpa_decode` needs, by the sizes alone.  A larger `workspace` is used too: from rank 4 on, up to
+    `tpa_decode_call_workspace_bytes` of the C ABI, it gives short caches further key ranges - as many as a call
+    without `workspace` has."""
     return int(_d.load_library().tpa_decode_workspace_bytes(b, lq, lk, h, dv, num_splits))
 
 

@@ -18,15 +18,15 @@ pytestmark = pytest.mark.gpu
         (1, 1, 4096, 32, 128, 6, 2),   # blocks of 16 tokens, 15 of them past the end
         (17, 1, 192, 8, 64, 2, 1),     # three chunks of k: five waves have none; a second block of one token
         (11, 3, 1088, 32, 128, 6, 2),  # 17 chunks; 33 tokens x 100 column blocks: blocks of 32
-        (13, 5, 64, 32, 128, 6, 2),    # one chunk of k: tiles
+        (13, 5, 64, 32, 128, 6, 2),    # one chunk of k: seven waves have none
         (13, 5, 1024, 32, 128, 6, 2),  # 65 tokens: two blocks of 64, the last of one token
         (1, 20, 576, 64, 64, 16, 8),   # 256 column blocks, nine chunks: one wave has two; blocks of 32
         (3, 5, 2048, 32, 128, 16, 8),  # 15 tokens x 320 column blocks, two rounds of blocks of 16
         (3, 30, 2112, 8, 64, 1, 1),    # 33 chunks; 216 columns: the last block owns 8 of its 16
         (2, 83, 512, 64, 64, 16, 8),   # 166 tokens x 256 column blocks, 768 workgroups: tiles
         (3, 71, 512, 64, 64, 16, 8),   # 213 tokens, 1024: tiles
-        (4, 63, 512, 32, 128, 6, 2),   # 252 tokens x 100 column blocks, 400 of 64 tokens: tiles at this d_model
-        (4, 63, 4096, 32, 128, 6, 2),  # 400 workgroups, the most it serves
+        (4, 63, 512, 32, 128, 6, 2),   # 252 tokens x 100 column blocks, two rounds of blocks of 64 tokens: tiles
+        (4, 63, 4096, 32, 128, 6, 2),  # the same, 64 chunks
     ],
 )
 def test_append_few_tokens(gpu, b, n, dm, h, d, rq, rk):
